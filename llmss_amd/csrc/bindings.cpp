@@ -147,6 +147,16 @@ void launch_selective_scan(const void* x, int64_t ldx, const void* dt, int64_t l
                            const void* Cm, int64_t ldb, const void* A, const void* D, const void* z, int64_t ldz,
                            void* state, const void* cu, const void* ctx, const void* sslots, void* out, int64_t ldo, int B,
                            int inner, int N, int all_single, int dtype, hipStream_t st);
+bool linear_step_ok(int dim, int vdim);
+void launch_linear_step(int mode, const void* q, const void* k, const void* v, int64_t ldq, int64_t ldk, int64_t ldv,
+                        const void* dt, int64_t lddt, const void* decay, const void* dt_bias, const void* skip, void* S,
+                        const void* cu, const void* ctx, const void* sslots, void* out, int B, int H, int G, int dim, int vdim,
+                        int silu, int dtype, hipStream_t st);
+bool linear_chunk_ok(int dim, int vdim);
+void launch_linear_chunk(int mode, const void* q, const void* k, const void* v, int64_t ldq, int64_t ldk, int64_t ldv,
+                         const void* dt, int64_t lddt, const void* decay, const void* dt_bias, const void* skip, void* S,
+                         const void* cu, const void* ctx, const void* sslots, void* out, int B, int H, int G, int dim, int vdim,
+                         int silu, hipStream_t st);
 bool delta_step_ok(int dim, int vdim);
 void launch_delta_step(const void* q, const void* k, const void* v, int64_t ldq, int64_t ldk, int64_t ldv, const void* a,
                        const void* b, int64_t ldab, const void* A_log, const void* dt_bias, void* S, const void* cu,
@@ -496,6 +506,22 @@ PYBIND11_MODULE(_C, m) {
                              int all_single, int dtype, uintptr_t st) {
     launch_selective_scan(CP(x), ldx, CP(dt), ldt, CP(dtb), CP(Bm), CP(Cm), ldb, CP(A), CP(D), CP(z), ldz, P(state), CP(cu),
                           CP(ctx), CP(ss), P(out), ldo, B, inner, N, all_single, dtype, S(st));
+  });
+  m.def("linear_step_ok", &linear_step_ok);
+  m.def("linear_chunk_ok", &linear_chunk_ok);
+  m.def("linear_step", [](int mode, uintptr_t q, uintptr_t k, uintptr_t v, int64_t ldq, int64_t ldk, int64_t ldv, uintptr_t dt,
+                          int64_t lddt, uintptr_t decay, uintptr_t dtb, uintptr_t skip, uintptr_t Sp, uintptr_t cu,
+                          uintptr_t ctx, uintptr_t ss, uintptr_t out, int B, int H, int G, int dim, int vdim, int silu,
+                          int dtype, uintptr_t st) {
+    launch_linear_step(mode, CP(q), CP(k), CP(v), ldq, ldk, ldv, CP(dt), lddt, CP(decay), CP(dtb), CP(skip), P(Sp), CP(cu),
+                       CP(ctx), CP(ss), P(out), B, H, G, dim, vdim, silu, dtype, S(st));
+  });
+  m.def("linear_chunk", [](int mode, uintptr_t q, uintptr_t k, uintptr_t v, int64_t ldq, int64_t ldk, int64_t ldv, uintptr_t dt,
+                           int64_t lddt, uintptr_t decay, uintptr_t dtb, uintptr_t skip, uintptr_t Sp, uintptr_t cu,
+                           uintptr_t ctx, uintptr_t ss, uintptr_t out, int B, int H, int G, int dim, int vdim, int silu,
+                           uintptr_t st) {
+    launch_linear_chunk(mode, CP(q), CP(k), CP(v), ldq, ldk, ldv, CP(dt), lddt, CP(decay), CP(dtb), CP(skip), P(Sp), CP(cu),
+                        CP(ctx), CP(ss), P(out), B, H, G, dim, vdim, silu, S(st));
   });
   m.def("delta_step_ok", &delta_step_ok);
   m.def("delta_chunk_ok", &delta_chunk_ok);

@@ -304,7 +304,9 @@ class DecayMixer:
         proj = ops.linear_f(h, W.proj, dt)
         o = ops.decay_recurrence(proj[:, c["q"]:c["q"] + nqk], proj[:, c["k"]:c["k"] + nqk],
                                  proj[:, c["v"]:c["v"] + nv], W.decay, caches[i][2]["S"], cu, inp.ctx_lens,
-                                 inp.state_slots, spec.heads, spec.dim, spec.vdim, True)
+                                 inp.state_slots, spec.heads, spec.dim, spec.vdim, True,
+                                 max_qlen=1 if inp.kind == "decode" else max(1, inp.max_seqlen),
+                                 num_decode=0 if inp.kind == "decode" else inp.num_decode)
         y = ops.gated_group_norm(o, proj[:, c["g"]:c["g"] + nv], W.norm, model.cfg.norm_eps, "sigmoid", 1.0,
                                  out_dtype=dt)
         return ops.linear_f(y, W.o, dt)
@@ -401,7 +403,9 @@ class SSDMixer:
                               inp.state_slots, False, True, dt, bias=W.conv_b)
         y = ops.ssd_recurrence(xbc[:, :inner], xbc[:, inner:inner + gn], xbc[:, inner + gn:],
                                proj[:, c["dt"]:c["dt"] + spec.heads], W.A_log, W.dt_bias, W.D, st["S"], cu,
-                               inp.ctx_lens, inp.state_slots, spec.heads, spec.groups, spec.state, spec.vdim)
+                               inp.ctx_lens, inp.state_slots, spec.heads, spec.groups, spec.state, spec.vdim,
+                               max_qlen=1 if inp.kind == "decode" else max(1, inp.max_seqlen),
+                               num_decode=0 if inp.kind == "decode" else inp.num_decode)
         y = ops.gated_group_norm(y, proj[:, c["z"]:c["z"] + inner], W.norm, model.cfg.norm_eps, "silu", 1.0,
                                  out_dtype=dt, groups=spec.norm_groups, gate_first=True)
         return ops.linear_f(y, W.o, dt)

@@ -1312,11 +1312,50 @@ def _rec_common(q, k, v, state, cu, ctx_lens, state_slots, heads, kv_heads, dim,
     return T, B, torch.empty(T, heads * vdim, dtype=torch.float32, device=q.device)
 
 
-def decay_recurrence(q, k, v, decay, state, cu, ctx_lens, state_slots, heads, dim, vdim, silu_in=True):
+# smallest portion (rows of the step's longest one) that the chunked form takes, by mode. A chunk costs about as much as the walk
+# of so many tokens when 64 sequences fill the chip (ssd 117 us, the walk of 4 139 us; decay 95 us, the walk of 8 63, of 16 101
+# us); a single sequence is faster chunk by chunk from 8 rows on (17 against 47 us).
+LINEAR_CHUNK_MIN = {0: 12, 2: 4}
+
+
+def _linear_forms(mode, q, k, v, dt, args, state, cu, ctx_lens, state_slots, out, heads, groups, dim, vdim, silu, max_qlen,
+                  num_decode):
+    """The sequences of a step that the two fast forms of a linear recurrence take: the ``num_decode`` leading single-row ones
+    (all when ``max_qlen`` is 1), then, on bf16 rows, the portions chunk by chunk. ``args``: addresses of decay / A_log, dt_bias
+    and D. Returns the first sequence left for the token-by-token walk."""
+    B, L, st = cu.numel() - 1, lib(), _stream()
+    nd = B if max_qlen == 1 else int(num_decode)
+    _check(0 <= nd <= B and (nd < B or q.shape[0] == B), "num_decode outside the step")
+    dt_ptr, lddt = (dt.data_ptr(), dt.stride(0)) if dt is not None else (0, 0)
+    if not (L.linear_step_ok(dim, vdim) and state.data_ptr() % 16 == 0 and (dt is None or dt.dtype == q.dtype)):
+        nd = 0
+    qkv = (q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), k.stride(0), v.stride(0))
+
+    def seqs(b):
+        return (state.data_ptr(), cu.data_ptr() + 4 * b, ctx_lens.data_ptr() + 4 * b, state_slots.data_ptr() + 4 * b,
+                out.data_ptr())
+    if nd:
+        L.linear_step(mode, *qkv, dt_ptr, lddt, *args, *seqs(0), nd, heads, groups, dim, vdim, int(silu), _dt(q, "q"), st)
+    if nd < B and max_qlen >= LINEAR_CHUNK_MIN[mode] and q.dtype == torch.bfloat16 and L.linear_chunk_ok(dim, vdim) and \
+            (dt is None or dt.dtype == q.dtype) and not any(p % 16 for p in qkv[:2]) and not any(x % 8 for x in qkv[3:5]):
+        L.linear_chunk(mode, *qkv, dt_ptr, lddt, *args, *seqs(nd), B - nd, heads, groups, dim, vdim, int(silu), st)
+        return B
+    return nd
+
+
+def decay_recurrence(q, k, v, decay, state, cu, ctx_lens, state_slots, heads, dim, vdim, silu_in=True, max_qlen=0, num_decode=0):
+    """``max_qlen`` (rows of the longest portion, 0: unknown) and ``num_decode`` (leading single-row sequences) choose the form:
+    see _linear_forms."""
     T, B, out = _rec_common(q, k, v, state, cu, ctx_lens, state_slots, heads, heads, dim, vdim)
     _f32c(decay, "decay")
     _check(decay.numel() == heads, "decay [heads]")
-    if T and silu_in and T > B:
+    if not T:
+        return out
+    first = _linear_forms(0, q, k, v, None, (decay.data_ptr(), 0, 0), state, cu, ctx_lens, state_slots, out, heads, heads, dim,
+                          vdim, bool(silu_in), max_qlen, num_decode)
+    if first == B:
+        return out
+    if silu_in and T - first > B - first:
         # portions: every workgroup of a head stages the head's whole q and k, so the activation is applied once
         # beforehand (fp32 rows) instead of in each of them
         nqk, nv = heads * dim, heads * vdim
@@ -1325,11 +1364,10 @@ def decay_recurrence(q, k, v, decay, state, cu, ctx_lens, state_slots, heads, di
             lib().silu_f32(src.data_ptr(), src.stride(0), act.data_ptr() + 4 * off, act.stride(0), T, n, _dt(src, "q"),
                            _stream())
         q, k, v, silu_in = act[:, :nqk], act[:, nqk:2 * nqk], act[:, 2 * nqk:], False
-    if T:
-        lib().recurrence(0, q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), k.stride(0), v.stride(0), 0, 0, 0, 0,
-                         decay.data_ptr(), 0, state.data_ptr(), cu.data_ptr(), ctx_lens.data_ptr(),
-                         state_slots.data_ptr(), out.data_ptr(), heads * vdim, B, heads, heads, dim, vdim,
-                         int(bool(silu_in)), 0, _dt(q, "q"), 0, 0, 0, 0, _stream())
+    lib().recurrence(0, q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), k.stride(0), v.stride(0), 0, 0, 0, 0,
+                     decay.data_ptr(), 0, state.data_ptr(), cu.data_ptr() + 4 * first, ctx_lens.data_ptr() + 4 * first,
+                     state_slots.data_ptr() + 4 * first, out.data_ptr(), heads * vdim, B - first, heads, heads, dim, vdim,
+                     int(bool(silu_in)), 0, _dt(q, "q"), 0, 0, 0, 0, _stream())
     return out
 
 
@@ -1803,20 +1841,26 @@ def pool_window_attn(q, k_cache, v_cache, kp_cache, vp_cache, block_tables, cu, 
     return out
 
 
-def ssd_recurrence(x, Bm, Cm, dt, A_log, dt_bias, D, state, cu, ctx_lens, state_slots, heads, groups, N, vdim):
-    """The state-space scan on the matrix-state recurrence kernel: keys = B, queries = C (one per group), values = x."""
+def ssd_recurrence(x, Bm, Cm, dt, A_log, dt_bias, D, state, cu, ctx_lens, state_slots, heads, groups, N, vdim, max_qlen=0,
+                   num_decode=0):
+    """The state-space scan on the matrix-state recurrences' kernels: keys = B, queries = C (one per group), values = x.
+    ``max_qlen`` / ``num_decode`` as for decay_recurrence."""
     T, B, out = _rec_common(Cm, Bm, x, state, cu, ctx_lens, state_slots, heads, groups, N, vdim)
     for t, nm in ((A_log, "A_log"), (dt_bias, "dt_bias"), (D, "D")):
         _f32c(t, nm)
         _check(t.numel() == heads, f"{nm} [heads]")
     _rows(dt, "dt", heads)
     _check(dt.shape[0] == T, "dt rows")
-    if T:
+    if not T:
+        return out
+    first = _linear_forms(2, Cm, Bm, x, dt, (A_log.data_ptr(), dt_bias.data_ptr(), D.data_ptr()), state, cu, ctx_lens,
+                          state_slots, out, heads, groups, N, vdim, False, max_qlen, num_decode)
+    if first < B:
         lib().recurrence(2, Cm.data_ptr(), Bm.data_ptr(), x.data_ptr(), Cm.stride(0), Bm.stride(0), x.stride(0),
                          dt.data_ptr(), dt.stride(0), 0, 0, A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(),
-                         cu.data_ptr(), ctx_lens.data_ptr(), state_slots.data_ptr(), out.data_ptr(), heads * vdim, B,
-                         heads, groups, N, vdim, 0, 0, _dt(x, "x"), _dt(dt, "dt"), D.data_ptr(), 0, 0,
-                         _stream())
+                         cu.data_ptr() + 4 * first, ctx_lens.data_ptr() + 4 * first, state_slots.data_ptr() + 4 * first,
+                         out.data_ptr(), heads * vdim, B - first, heads, groups, N, vdim, 0, 0, _dt(x, "x"), _dt(dt, "dt"),
+                         D.data_ptr(), 0, 0, _stream())
     return out
 
 

@@ -762,7 +762,7 @@ def glu_act(gu, F_: int, act: str):
 
 
 def decay_recurrence(q, k, v, decay, state, cu, ctx_lens, state_slots, heads: int, dim: int, vdim: int,
-                     silu_in: bool = True):
+                     silu_in: bool = True, max_qlen: int = 0, num_decode: int = 0):
     """Per head S <- decay_h S + k v^T, o = S^T q over each sequence's rows, S fp32 [slots, heads, dim, vdim]
     carried in the sequence's slot (zero when the portion starts at position 0). Returns fp32 [T, heads * vdim]."""
     T = q.shape[0]
@@ -1137,7 +1137,7 @@ def pool_window_attn(q, k_cache, v_cache, kp_cache, vp_cache, block_tables, cu, 
 
 
 def ssd_recurrence(x, Bm, Cm, dt, A_log, dt_bias, D, state, cu, ctx_lens, state_slots, heads: int, groups: int,
-                   N: int, vdim: int):
+                   N: int, vdim: int, max_qlen: int = 0, num_decode: int = 0):
     """Per head h (group g = h // (heads / groups)) over each sequence's rows: d = softplus(dt + dt_bias_h);
     S <- exp(-exp(A_log_h) d) S + d B_g x_h^T; y = S^T C_g + D_h x_h, S fp32 [slots, heads, N, vdim] carried in the
     sequence's slot (zero when the portion starts at position 0). x [T, heads * vdim], Bm / Cm [T, groups * N], dt [T,
