@@ -161,12 +161,18 @@ bool delta_step_ok(int dim, int vdim);
 void launch_delta_step(const void* q, const void* k, const void* v, int64_t ldq, int64_t ldk, int64_t ldv, const void* a,
                        const void* b, int64_t ldab, const void* A_log, const void* dt_bias, void* S, const void* cu,
                        const void* ctx, const void* sslots, const void* gate, int64_t ldg, const void* w, float eps,
-                       float scale, void* y, int64_t ldy, int B, int H, int G, int dim, int vdim, int dt, hipStream_t st);
+                       float scale, void* y, int64_t ldy, int B, int H, int G, int dim, int vdim, int dq, int dt,
+                       hipStream_t st);
 bool delta_chunk_ok(int dim, int vdim);
 void launch_delta_chunk(const void* q, const void* k, const void* v, int64_t ldq, int64_t ldk, int64_t ldv, const void* a,
                         const void* b, int64_t ldab, const void* A_log, const void* dt_bias, void* S, const void* cu,
                         const void* ctx, const void* sslots, void* out, void* work, void* aux, int T_, int B, int max_qlen,
                         int H, int G, int dim, int vdim, hipStream_t st);
+bool delta_chunk32_ok(int dim, int vdim);
+void launch_delta_chunk32(const void* q, const void* k, const void* v, int64_t ldq, int64_t ldk, int64_t ldv, const void* a,
+                          const void* b, int64_t ldab, const void* A_log, const void* dt_bias, void* S, const void* cu,
+                          const void* ctx, const void* sslots, void* out, void* work, void* aux, int T_, int B, int max_qlen,
+                          int H, int G, int dim, int vdim, int dp, hipStream_t st);
 bool mlstm_step_ok(int dim, int vdim);
 void launch_mlstm_step(const void* q, const void* k, const void* v, int64_t ldq, int64_t ldk, int64_t ldv, const void* zi,
                        const void* zf, int64_t ldz, const void* bi, const void* bf, float cap, void* S, void* n, void* m,
@@ -528,9 +534,10 @@ PYBIND11_MODULE(_C, m) {
   m.def("delta_step", [](uintptr_t q, uintptr_t k, uintptr_t v, int64_t ldq, int64_t ldk, int64_t ldv, uintptr_t a,
                          uintptr_t b, int64_t ldab, uintptr_t A_log, uintptr_t dtb, uintptr_t Sp, uintptr_t cu,
                          uintptr_t ctx, uintptr_t ss, uintptr_t gate, int64_t ldg, uintptr_t w, float eps, float scale,
-                         uintptr_t y, int64_t ldy, int B, int H, int G, int dim, int vdim, int dt, uintptr_t st) {
+                         uintptr_t y, int64_t ldy, int B, int H, int G, int dim, int vdim, int dq, int dt,
+                         uintptr_t st) {
     launch_delta_step(CP(q), CP(k), CP(v), ldq, ldk, ldv, CP(a), CP(b), ldab, CP(A_log), CP(dtb), P(Sp), CP(cu), CP(ctx),
-                      CP(ss), CP(gate), ldg, CP(w), eps, scale, P(y), ldy, B, H, G, dim, vdim, dt, S(st));
+                      CP(ss), CP(gate), ldg, CP(w), eps, scale, P(y), ldy, B, H, G, dim, vdim, dq, dt, S(st));
   });
   m.def("delta_chunk", [](uintptr_t q, uintptr_t k, uintptr_t v, int64_t ldq, int64_t ldk, int64_t ldv, uintptr_t a,
                           uintptr_t b, int64_t ldab, uintptr_t A_log, uintptr_t dtb, uintptr_t Sp, uintptr_t cu,
@@ -538,6 +545,14 @@ PYBIND11_MODULE(_C, m) {
                           int max_qlen, int H, int G, int dim, int vdim, uintptr_t st) {
     launch_delta_chunk(CP(q), CP(k), CP(v), ldq, ldk, ldv, CP(a), CP(b), ldab, CP(A_log), CP(dtb), P(Sp), CP(cu), CP(ctx),
                        CP(ss), P(out), P(work), P(aux), T, B, max_qlen, H, G, dim, vdim, S(st));
+  });
+  m.def("delta_chunk32_ok", &delta_chunk32_ok);
+  m.def("delta_chunk32", [](uintptr_t q, uintptr_t k, uintptr_t v, int64_t ldq, int64_t ldk, int64_t ldv, uintptr_t a,
+                            uintptr_t b, int64_t ldab, uintptr_t A_log, uintptr_t dtb, uintptr_t Sp, uintptr_t cu,
+                            uintptr_t ctx, uintptr_t ss, uintptr_t out, uintptr_t work, uintptr_t aux, int T, int B,
+                            int max_qlen, int H, int G, int dim, int vdim, int dp, uintptr_t st) {
+    launch_delta_chunk32(CP(q), CP(k), CP(v), ldq, ldk, ldv, CP(a), CP(b), ldab, CP(A_log), CP(dtb), P(Sp), CP(cu), CP(ctx),
+                         CP(ss), P(out), P(work), P(aux), T, B, max_qlen, H, G, dim, vdim, dp, S(st));
   });
   m.def("mlstm_step_ok", &mlstm_step_ok);
   m.def("mlstm_chunk_ok", &mlstm_chunk_ok);

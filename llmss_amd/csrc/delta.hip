@@ -41,8 +41,10 @@ struct DeltaStepArgs {
   int H, G, dim, vdim;
 };
 
-// U: state rows per thread; a thread holds U rows x 4 columns of the state
-template <typename T, int U>
+// Bound by the state's bytes, read and written once. fp32 rows (TQ) beside bf16 projections, 64 sequences x 16 heads of 128 x
+// 128: 29 us against the walk's 117.
+// U: state rows per thread; a thread holds U rows x 4 columns of the state. TQ: storage of q, k, v; T: of everything else
+template <typename TQ, typename T, int U>
 __global__ __launch_bounds__(512) void delta_step_kernel(DeltaStepArgs A) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   __shared__ float red[32];
@@ -72,11 +74,11 @@ __global__ __launch_bounds__(512) void delta_step_kernel(DeltaStepArgs A) {
   const float za = El<T>::ld((const T*)A.a + (int64_t)t * A.ldab + h) + A.dt_bias[h];
   const float beta = 1.0f / (1.0f + expf(-zb));
   const float g = expf(-expf(A.A_log[h]) * (za > 20.f ? za : log1pf(expf(za))));
-  const T* qr = (const T*)A.q + (int64_t)t * A.ldq + (int64_t)gq * dim;
-  const T* kr = (const T*)A.k + (int64_t)t * A.ldk + (int64_t)gq * dim;
+  const TQ* qr = (const TQ*)A.q + (int64_t)t * A.ldq + (int64_t)gq * dim;
+  const TQ* kr = (const TQ*)A.k + (int64_t)t * A.ldk + (int64_t)gq * dim;
   float qq = 0.f, kk = 0.f, kq = 0.f;
   for (int d = tid; d < dim; d += nthr) {
-    const float qd = El<T>::ld(qr + d), kd = El<T>::ld(kr + d);
+    const float qd = El<TQ>::ld(qr + d), kd = El<TQ>::ld(kr + d);
     qs[d] = qd;
     ks[d] = kd;
     qq = fmaf(qd, qd, qq);
@@ -109,7 +111,7 @@ __global__ __launch_bounds__(512) void delta_step_kernel(DeltaStepArgs A) {
       a += pk[r * vdim + c];
       o += pq[r * vdim + c];
     }
-    const float v = El<T>::ld((const T*)A.v + (int64_t)t * A.ldv + (int64_t)h * vdim + c);
+    const float v = El<TQ>::ld((const TQ*)A.v + (int64_t)t * A.ldv + (int64_t)h * vdim + c);
     const float u = beta * (v - g * kn * a);
     us[c] = u;
     o = g * qn * o + kq * kn * qn * u;
@@ -151,7 +153,7 @@ bool delta_step_ok(int dim, int vdim) { return delta_step_threads(dim, vdim) > 0
 void launch_delta_step(const void* q, const void* k, const void* v, int64_t ldq, int64_t ldk, int64_t ldv, const void* a,
                        const void* b, int64_t ldab, const void* A_log, const void* dt_bias, void* S, const void* cu,
                        const void* ctx, const void* sslots, const void* gate, int64_t ldg, const void* w, float eps,
-                       float scale, void* y, int64_t ldy, int B, int H, int G, int dim, int vdim, int dt, hipStream_t st) {
+                       float scale, void* y, int64_t ldy, int B, int H, int G, int dim, int vdim, int dq, int dt, hipStream_t st) {
   if (B == 0) return;
   const int th = delta_step_threads(dim, vdim);
   if (!th || B > 65535 || G < 1 || H % G) throw std::runtime_error("delta_step: shape");
@@ -161,11 +163,17 @@ void launch_delta_step(const void* q, const void* k, const void* v, int64_t ldq,
   const int RG = th / (vdim / 4), U = (dim + RG - 1) / RG;
   const size_t lds = ((size_t)2 * dim + 4 + vdim + (size_t)2 * RG * vdim) * 4;
   dim3 g(H, B);
-  DISPATCH_T(dt, T, {
-    if (U <= 4) delta_step_kernel<T, 4><<<g, th, lds, st>>>(A);
-    else if (U <= 8) delta_step_kernel<T, 8><<<g, th, lds, st>>>(A);
-    else delta_step_kernel<T, 16><<<g, th, lds, st>>>(A);
-  });
+  if (dq == 0 && dt != 0) throw std::runtime_error("delta_step: 16-bit rows beside 32-bit projections");
+#define LAUNCH_DS(TQ_, T_)                                                       \
+  do {                                                                           \
+    if (U <= 4) delta_step_kernel<TQ_, T_, 4><<<g, th, lds, st>>>(A);            \
+    else if (U <= 8) delta_step_kernel<TQ_, T_, 8><<<g, th, lds, st>>>(A);       \
+    else delta_step_kernel<TQ_, T_, 16><<<g, th, lds, st>>>(A);                  \
+  } while (0)
+  if (dq == 0) LAUNCH_DS(bf16_t, bf16_t);
+  else if (dt == 0) LAUNCH_DS(float, bf16_t);
+  else LAUNCH_DS(float, float);
+#undef LAUNCH_DS
   HIP_CHECK_LAUNCH();
 }
 
@@ -198,6 +206,51 @@ __device__ __forceinline__ void split2(float x, bf16_t& hi, bf16_t& lo) {
 
 constexpr int prep_kq_bytes(int kt) {  // K and Q rows, or P (value, remainder) and the fp32 inverse
   return 2 * 64 * (16 * kt + 8) * 2 > 2 * 64 * 72 * 2 + 64 * 68 * 4 ? 2 * 64 * (16 * kt + 8) * 2 : 2 * 64 * 72 * 2 + 64 * 68 * 4;
+}
+
+// (I + L)^-1 of a 64 x 64 matrix in LDS (4 waves; the blocks of X above the diagonal hold zeros already)
+__device__ __forceinline__ void lower_inverse(const float* Ls, float* Xs, const int LDL, int w, int li, int g) {
+  // wave w its 16 x 16 diagonal block by substitution, a column per lane (four copies of each)
+  {
+    float x[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) x[t] = t == li ? 1.0f : 0.f;
+#pragma unroll
+    for (int t = 1; t < 16; ++t) {
+      const float* lr = &Ls[(16 * w + t) * LDL + 16 * w];
+      float acc = 0.f, acc2 = 0.f;
+#pragma unroll
+      for (int s = 0; s < t; ++s) {
+        if (s & 1) acc2 = fmaf(lr[s], x[s], acc2);
+        else acc = fmaf(lr[s], x[s], acc);
+      }
+      x[t] -= acc + acc2;
+    }
+#pragma unroll
+    for (int t = 0; t < 16; ++t)
+      if ((t >> 2) == g) Xs[(16 * w + t) * LDL + 16 * w + li] = x[t];
+  }
+  // the blocks below, a diagonal at a time: X_ij = -X_ii sum_{j <= m < i} L_im X_mj
+#pragma unroll
+  for (int lev = 1; lev < 4; ++lev) {
+    __syncthreads();
+    const int bi = w + lev, bj = w;
+    if (bi < 4) {
+      f32x4 z = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f};
+      for (int m = bj; m < bi; ++m) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          z = __builtin_amdgcn_mfma_f32_16x16x4f32(Ls[(16 * bi + li) * LDL + 16 * m + 4 * g + i],
+                                                   Xs[(16 * m + 4 * g + i) * LDL + 16 * bj + li], z, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)  // (the accumulator's rows 4 g + i are the second operand as they stand)
+        o = __builtin_amdgcn_mfma_f32_16x16x4f32(Xs[(16 * bi + li) * LDL + 16 * bi + 4 * g + i], z[i], o, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) Xs[(16 * bi + 4 * g + i) * LDL + 16 * bj + li] = -o[i];
+    }
+  }
+  __syncthreads();
 }
 
 // Workgroup (chunk of a portion, head, sequence), 4 waves
@@ -299,47 +352,7 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(DeltaChunkArgs A) {
     }
   }
   __syncthreads();
-  // (I + L)^-1: wave w its 16 x 16 diagonal block by substitution, a column per lane (four copies of each)
-  {
-    float x[16];
-#pragma unroll
-    for (int t = 0; t < 16; ++t) x[t] = t == li ? 1.0f : 0.f;
-#pragma unroll
-    for (int t = 1; t < 16; ++t) {
-      const float* lr = &Ls[(16 * w + t) * LDL + 16 * w];
-      float acc = 0.f, acc2 = 0.f;
-#pragma unroll
-      for (int s = 0; s < t; ++s) {
-        if (s & 1) acc2 = fmaf(lr[s], x[s], acc2);
-        else acc = fmaf(lr[s], x[s], acc);
-      }
-      x[t] -= acc + acc2;
-    }
-#pragma unroll
-    for (int t = 0; t < 16; ++t)
-      if ((t >> 2) == g) Xs[(16 * w + t) * LDL + 16 * w + li] = x[t];
-  }
-  // the blocks below, a diagonal at a time: X_ij = -X_ii sum_{j <= m < i} L_im X_mj
-#pragma unroll
-  for (int lev = 1; lev < 4; ++lev) {
-    __syncthreads();
-    const int bi = w + lev, bj = w;
-    if (bi < 4) {
-      f32x4 z = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f};
-      for (int m = bj; m < bi; ++m) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          z = __builtin_amdgcn_mfma_f32_16x16x4f32(Ls[(16 * bi + li) * LDL + 16 * m + 4 * g + i],
-                                                   Xs[(16 * m + 4 * g + i) * LDL + 16 * bj + li], z, 0, 0, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)  // (the accumulator's rows 4 g + i are the second operand as they stand)
-        o = __builtin_amdgcn_mfma_f32_16x16x4f32(Xs[(16 * bi + li) * LDL + 16 * bi + 4 * g + i], z[i], o, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) Xs[(16 * bi + 4 * g + i) * LDL + 16 * bj + li] = -o[i];
-    }
-  }
-  __syncthreads();
+  lower_inverse(Ls, Xs, LDL, w, li, g);
   const int64_t row = (int64_t)(t0 + j0) * H + h;
   for (int e = tid; e < C * 8; e += 256) {
     const int r = e >> 3, s0 = (e & 7) * 8;
@@ -604,5 +617,388 @@ void launch_delta_chunk(const void* q, const void* k, const void* v, int64_t ldq
   else if (dim <= 128) LAUNCH_DC(8);
   else LAUNCH_DC(16);
 #undef LAUNCH_DC
+  HIP_CHECK_LAUNCH();
+}
+
+// ------------------------------------------------------------------------------------------------ portions of fp32 rows
+// The same two kernels for rows in 32 bits (a convolution's fp32 results), every product on the fp32 matrix instructions, the
+// sums of log decays in 64 bits, X and P held in 32. Bound by the chain of chunks: 8 sequences x 16
+// heads of 128 x 128 are one workgroup per CU (wave per SIMD), each 16 dependent chunks of 464 matrix instructions of 32 cycles.
+// 8 x 1024 tokens: 408 us with the norm, 1615 us token by token; one sequence of 2048: 440 and 3130 us.
+struct DeltaChunk32Args {
+  const float* q;
+  const float* k;
+  const float* v;
+  int64_t ldq, ldk, ldv;
+  const void* a;
+  const void* b;
+  int64_t ldab;
+  const float* A_log;
+  const float* dt_bias;
+  float* S;
+  const int* cu;
+  const int* ctx;
+  const int* sslots;
+  float* out;  // [T, H * vdim]
+  float* X;    // [2][T, H, 64]: X, P; row t of its chunk
+  int64_t mat;
+  f32x4* aux;  // as above
+  int H, G, dim, vdim;
+};
+
+__device__ __forceinline__ f32x4 ldv4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+
+constexpr int prep32_kq_bytes(int kt) {  // K and Q rows, or P and the inverse
+  return 2 * 64 * (16 * kt + 4) * 4 > 2 * 64 * 68 * 4 ? 2 * 64 * (16 * kt + 4) * 4 : 2 * 64 * 68 * 4;
+}
+
+// acc += A B^T over the keys: A's rows at ap (this lane's, from column 4 g on), B's at bp, in up to four chains (shorter ones
+// round less)
+template <int KT>
+__device__ __forceinline__ f32x4 dot32(const float* ap, const float* bp) {
+  constexpr int N = KT < 4 ? 2 : 4;
+  f32x4 c[N];
+#pragma unroll
+  for (int n = 0; n < N; ++n) c[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kt = 0; kt < KT; kt += N) {
+    f32x4 x[N], y[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) x[n] = ldv4(ap + 16 * (kt + n)), y[n] = ldv4(bp + 16 * (kt + n));
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int n = 0; n < N; ++n) c[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[n][i], y[n][i], c[n], 0, 0, 0);
+  }
+  return N == 4 ? (c[0] + c[1]) + (c[N - 2] + c[N - 1]) : c[0] + c[1];
+}
+// A S: the state's tiles are the second operand as they stand
+template <int KT>
+__device__ __forceinline__ f32x4 dot32s(const float* ap, const f32x4* S) {
+  constexpr int N = KT < 4 ? 2 : 4;
+  f32x4 c[N];
+#pragma unroll
+  for (int n = 0; n < N; ++n) c[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kt = 0; kt < KT; kt += N) {
+    f32x4 x[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) x[n] = ldv4(ap + 16 * (kt + n));
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int n = 0; n < N; ++n) c[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[n][i], S[kt + n][i], c[n], 0, 0, 0);
+  }
+  return N == 4 ? (c[0] + c[1]) + (c[N - 2] + c[N - 1]) : c[0] + c[1];
+}
+
+// Workgroup (chunk of a portion, head, sequence), 4 waves. TP: storage of a and b
+template <int KT, typename TP>
+__global__ __launch_bounds__(256) void delta_prep32_kernel(DeltaChunk32Args A) {
+  constexpr int C = 64, DKP = 16 * KT, LDK = DKP + 4, LDL = 64 + 4;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  float* Ks = reinterpret_cast<float*>(smem);
+  float* Qs = Ks + C * LDK;
+  float* Ps = reinterpret_cast<float*>(smem);  // once the rows' products are taken
+  float* Xs = Ps + C * LDL;
+  float* Ls = reinterpret_cast<float*>(smem + prep32_kq_bytes(KT));
+  double* bs = reinterpret_cast<double*>(Ls + C * LDL);  // [64] sum of the log decays
+  float* be = reinterpret_cast<float*>(bs + C);          // [64] write strength
+  float* nk = be + C;                                    // [64] 1 / |k|
+  float* nq = nk + C;                                    // [64] dim^-1/2 / |q|
+  const int b = blockIdx.z, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, g = lane >> 4;
+  const int t0 = A.cu[b], qlen = A.cu[b + 1] - t0, j0 = blockIdx.x * C;
+  if (j0 >= qlen || A.sslots[b] < 0 || A.ctx[b] <= 0) return;
+  const int nt = min(C, qlen - j0), dim = A.dim, H = A.H, gq = h / (H / A.G);
+  constexpr int CHK = DKP / 4, NK = C * CHK / 256;
+  static_assert((C * CHK) % 256 == 0, "whole 16-byte pieces per thread");
+#pragma unroll
+  for (int j = 0; j < NK; ++j) {
+    const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 4;
+    const bool in = r < nt && d < dim;
+    const int64_t tt = t0 + j0 + r;
+    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+    *reinterpret_cast<f32x4*>(&Ks[r * LDK + d]) = in ? ldv4(A.k + tt * A.ldk + (int64_t)gq * dim + d) : z;
+    *reinterpret_cast<f32x4*>(&Qs[r * LDK + d]) = in ? ldv4(A.q + tt * A.ldq + (int64_t)gq * dim + d) : z;
+  }
+  if (w == 0) {  // the tokens' decays and write strengths
+    const bool in = lane < nt;
+    const int64_t tt = (int64_t)(t0 + j0 + min(lane, nt - 1)) * A.ldab + h;
+    const float z = El<TP>::ld((const TP*)A.a + tt) + A.dt_bias[h];
+    // (a decay of zero: a sum this low vanishes over a single token, and differences of equal sums stay zero)
+    double F = in ? fmax((double)(-expf(A.A_log[h]) * (z > 20.f ? z : log1pf(expf(z)))), -1e8) : 0.0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double x = __shfl_up(F, o, 64);
+      if (lane >= o) F += x;
+    }
+    bs[lane] = F;
+    be[lane] = in ? 1.0f / (1.0f + expf(-El<TP>::ld((const TP*)A.b + tt))) : 0.f;
+  }
+  __syncthreads();
+  {  // norms: four neighbouring lanes per row
+    const int r = tid >> 2, part = tid & 3;
+    float kk = 0.f, qq = 0.f;
+    for (int d = part * 4; d < DKP; d += 16) {
+      const f32x4 x = ldv4(&Ks[r * LDK + d]), y = ldv4(&Qs[r * LDK + d]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        kk = fmaf(x[i], x[i], kk);
+        qq = fmaf(y[i], y[i], qq);
+      }
+    }
+    kk += __shfl_xor(kk, 1, 64);
+    kk += __shfl_xor(kk, 2, 64);
+    qq += __shfl_xor(qq, 1, 64);
+    qq += __shfl_xor(qq, 2, 64);
+    if (part == 0) {
+      nk[r] = 1.0f / sqrtf(kk + 1e-6f);
+      nq[r] = 1.0f / (sqrtf(qq + 1e-6f) * sqrtf((float)dim));
+    }
+  }
+  // wave w: the products of its 16 tokens (rows) with the keys of the blocks up to its own (columns)
+  f32x4 pk[4], pq[4];
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct) {
+    pk[ct] = pq[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (ct > w || 16 * w >= nt) continue;
+    const float* kb = &Ks[(16 * ct + li) * LDK + 4 * g];
+    pk[ct] = dot32<KT>(&Ks[(16 * w + li) * LDK + 4 * g], kb);
+    pq[ct] = dot32<KT>(&Qs[(16 * w + li) * LDK + 4 * g], kb);
+  }
+  __syncthreads();  // every wave has read its rows; the norms are written
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct) {
+    const int s = 16 * ct + li;
+    const double bsv = bs[s];
+    const float nks = nk[s];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = 16 * w + 4 * g + i;
+      const float e = s <= t ? expf((float)(bs[t] - bsv)) * nks : 0.f;
+      Ls[t * LDL + s] = s < t ? e * be[t] * nk[t] * pk[ct][i] : 0.f;
+      Ps[t * LDL + s] = s <= t ? e * nq[t] * pq[ct][i] : 0.f;
+      if (ct > w) Xs[t * LDL + s] = 0.f;  // the blocks of the inverse above the diagonal
+    }
+  }
+  __syncthreads();
+  lower_inverse(Ls, Xs, LDL, w, li, g);
+  const int64_t row = (int64_t)(t0 + j0) * H + h;
+  for (int e = tid; e < C * 16; e += 256) {
+    const int r = e >> 4, s0 = (e & 15) * 4;
+    if (r >= nt) continue;
+    f32x4 x = ldv4(&Xs[r * LDL + s0]);
+    const f32x4 y = ldv4(&be[s0]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] *= y[i];
+    float* dst = A.X + (row + (int64_t)r * H) * 64 + s0;
+    *reinterpret_cast<f32x4*>(dst) = x;
+    *reinterpret_cast<f32x4*>(dst + A.mat) = ldv4(&Ps[r * LDL + s0]);
+  }
+  if (tid < nt) {
+    const double bc = bs[C - 1];
+    const float e = expf((float)bs[tid]);
+    A.aux[row + (int64_t)tid * H] = f32x4{e * nk[tid], e * nq[tid], expf((float)(bc - bs[tid])) * nk[tid], expf((float)bc)};
+  }
+}
+
+// Workgroup (head, block of 64 value columns, sequence), 4 waves, the portion's chunks in order; layouts as in delta_chunk: a
+// register of an accumulator tile is the second operand of a 16x16x4 instruction over its rows 4 g + i, and the first operand's
+// matching numbers are four neighbours of a row in LDS. Blocks of 16 tokens past the portion's end are skipped.
+template <int KT>
+__global__ __launch_bounds__(256) void delta_chunk32_kernel(DeltaChunk32Args A) {
+  constexpr int C = 64, DKP = 16 * KT, LDK = DKP + 4, LDP = 64 + 4;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  float* Qs = reinterpret_cast<float*>(smem);
+  float* Ks = Qs + C * LDK;
+  float* Ms = Ks + C * LDK;                                // [2][64][LDP]: X, P
+  f32x4* ax = reinterpret_cast<f32x4*>(Ms + 2 * C * LDP);  // [64]
+  const int h = blockIdx.x, b = gridDim.z - 1 - blockIdx.z;
+  const int dim = A.dim, vdim = A.vdim, H = A.H, gq = h / (H / A.G);
+  const int t0 = A.cu[b], qlen = A.cu[b + 1] - t0, slot = A.sslots[b], ctx = A.ctx[b];
+  if (qlen <= 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, g = lane >> 4;
+  const int col = blockIdx.y * 64 + 16 * w + li, colc = min(col, vdim - 1);
+  float* outp = A.out + (int64_t)t0 * H * vdim + (int64_t)h * vdim + col;
+  if (slot < 0 || ctx <= 0) {
+    if (g == 0 && col < vdim)
+      for (int j = 0; j < qlen; ++j) outp[(int64_t)j * H * vdim] = 0.f;
+    return;
+  }
+  const bool cont = ctx > qlen;  // continues an earlier portion
+  f32x4 S[KT];
+  float* sp = A.S + (((int64_t)slot * H + h) * dim) * (int64_t)vdim;
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 16 * kt + 4 * g + i;
+      S[kt][i] = (cont && r < dim && col < vdim) ? sp[(int64_t)r * vdim + col] : 0.f;
+    }
+  constexpr int CHK = DKP / 4, NK = C * CHK / 256;
+  f32x4 rq[NK], rk[NK], rm[8];
+  float rv[16];
+  f32x4 ra = {0.f, 0.f, 0.f, 0.f};
+  const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+  auto fetch = [&](int j0) {
+#pragma unroll
+    for (int j = 0; j < NK; ++j) {
+      const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 4;
+      const bool in = j0 + r < qlen && d < dim;
+      const int64_t tt = t0 + j0 + r;
+      rq[j] = in ? ldv4(A.q + tt * A.ldq + (int64_t)gq * dim + d) : zero4;
+      rk[j] = in ? ldv4(A.k + tt * A.ldk + (int64_t)gq * dim + d) : zero4;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int c = tid + 256 * (j & 3), r = c >> 4, s0 = (c & 15) * 4;
+      rm[j] = j0 + r < qlen ? ldv4(A.X + (j >> 2) * A.mat + ((int64_t)(t0 + j0 + r) * H + h) * 64 + s0) : zero4;
+    }
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {  // token 16 (j / 4) + 4 g + j % 4 at this lane's column
+      const int r = j0 + 16 * (j >> 2) + 4 * g + (j & 3);
+      rv[j] = A.v[(int64_t)(t0 + min(r, qlen - 1)) * A.ldv + (int64_t)h * vdim + colc];
+      if (r >= qlen) rv[j] = 0.f;
+    }
+    if (w == 0) ra = A.aux[(int64_t)(t0 + min(j0 + lane, qlen - 1)) * H + h];
+  };
+  fetch(0);
+  for (int j0 = 0; j0 < qlen; j0 += C) {
+    const int nt = min(C, qlen - j0), nb = (nt + 15) >> 4;
+    __syncthreads();  // the previous chunk's readers are done
+#pragma unroll
+    for (int j = 0; j < NK; ++j) {
+      const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 4;
+      *reinterpret_cast<f32x4*>(&Qs[r * LDK + d]) = rq[j];
+      *reinterpret_cast<f32x4*>(&Ks[r * LDK + d]) = rk[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int c = tid + 256 * (j & 3);
+      *reinterpret_cast<f32x4*>(&Ms[(j >> 2) * C * LDP + (c >> 4) * LDP + (c & 15) * 4]) = rm[j];
+    }
+    if (w == 0) ax[lane] = ra;
+    f32x4 u[4], o[4], U[4];  // u: first V, then V - e^b K S_0
+#pragma unroll
+    for (int j = 0; j < 16; ++j) u[j >> 2][j & 3] = rv[j];
+    __syncthreads();
+    if (j0 + C < qlen) fetch(j0 + C);
+    const float a_all = ax[0][3];
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      o[rt] = U[rt] = zero4;
+      if (rt >= nb) continue;
+      const f32x4 ksv = dot32s<KT>(&Ks[(16 * rt + li) * LDK + 4 * g], S);
+      o[rt] = dot32s<KT>(&Qs[(16 * rt + li) * LDK + 4 * g], S);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f32x4 x = ax[16 * rt + 4 * g + i];
+        u[rt][i] = fmaf(-x[0], ksv[i], u[rt][i]);
+        o[rt][i] *= x[1];
+      }
+    }
+    // U = X u, O += P U
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      if (rt >= nb) continue;
+#pragma unroll
+      for (int m = 0; m <= rt; ++m) {
+        const f32x4 x = ldv4(&Ms[(16 * rt + li) * LDP + 16 * m + 4 * g]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) U[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], u[m][i], U[rt], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      if (rt >= nb) continue;
+      f32x4 in = zero4;
+#pragma unroll
+      for (int m = 0; m <= rt; ++m) {
+        const f32x4 x = ldv4(&Ms[C * LDP + (16 * rt + li) * LDP + 16 * m + 4 * g]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) in = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], U[m][i], in, 0, 0, 0);
+      }
+      o[rt] += in;
+    }
+    // the state: e^(b_C) S_0 + K^T (w U)
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[kt][i] *= a_all;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      if (m >= nb) continue;
+      f32x4 wu;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) wu[i] = U[m][i] * ax[16 * m + 4 * g + i][2];
+#pragma unroll
+      for (int k0 = 0; k0 < KT; k0 += 2) {
+        f32x4 x[2];
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          const float* p = &Ks[(16 * m + 4 * g) * LDK + 16 * (k0 + n) + li];
+          x[n] = f32x4{p[0], p[LDK], p[2 * LDK], p[3 * LDK]};
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int n = 0; n < 2; ++n) S[k0 + n] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[n][i], wu[i], S[k0 + n], 0, 0, 0);
+      }
+    }
+    if (col < vdim) {
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int t = 16 * rt + 4 * g + i;
+          if (t < nt) outp[(int64_t)(j0 + t) * H * vdim] = o[rt][i];
+        }
+    }
+  }
+  if (col < vdim) {
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 16 * kt + 4 * g + i;
+        if (r < dim) sp[(int64_t)r * vdim + col] = S[kt][i];
+      }
+  }
+}
+
+// (above 128 the chunk's rows and matrices do not fit in LDS)
+bool delta_chunk32_ok(int dim, int vdim) { return dim % 4 == 0 && dim >= 4 && dim <= 128 && vdim >= 1; }
+
+// q, k, v fp32, a and b in storage type dp; max_qlen: rows of the longest portion; work: fp32 [2][T, H, 64]; aux: fp32 [T, H, 4]
+void launch_delta_chunk32(const void* q, const void* k, const void* v, int64_t ldq, int64_t ldk, int64_t ldv, const void* a,
+                          const void* b, int64_t ldab, const void* A_log, const void* dt_bias, void* S, const void* cu,
+                          const void* ctx, const void* sslots, void* out, void* work, void* aux, int T_, int B, int max_qlen,
+                          int H, int G, int dim, int vdim, int dp, hipStream_t st) {
+  if (B == 0 || max_qlen <= 0) return;
+  if (!delta_chunk32_ok(dim, vdim) || B > 65535 || H > 65535 || G < 1 || H % G) throw std::runtime_error("delta_chunk32: shape");
+  if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)work | (uintptr_t)aux) & 15 || (ldq | ldk) & 3)
+    throw std::runtime_error("delta_chunk32: rows must be 16-byte aligned");
+  DeltaChunk32Args A{(const float*)q, (const float*)k, (const float*)v, ldq, ldk, ldv, a, b, ldab, (const float*)A_log,
+                     (const float*)dt_bias, (float*)S, (const int*)cu, (const int*)ctx, (const int*)sslots, (float*)out,
+                     (float*)work, (int64_t)T_ * H * 64, (f32x4*)aux, H, G, dim, vdim};
+  dim3 g1((max_qlen + 63) / 64, H, B), g2(H, (vdim + 63) / 64, B);
+  auto lds1 = [](int kt) { return (size_t)prep32_kq_bytes(kt) + (size_t)4 * (64 * 68 + 3 * 64) + 8 * 64; };
+  auto lds2 = [](int kt) { return (size_t)4 * (2 * 64 * (16 * kt + 4) + 2 * 64 * 68) + (size_t)16 * 64; };
+#define LAUNCH_DC32(KT_)                                                                                             \
+  do {                                                                                                               \
+    static bool once = [] {                                                                                          \
+      for (const void* f : {(const void*)delta_prep32_kernel<KT_, bf16_t>, (const void*)delta_prep32_kernel<KT_, float>, \
+                            (const void*)delta_chunk32_kernel<KT_>})                                                 \
+        (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                        \
+      return true;                                                                                                   \
+    }();                                                                                                             \
+    (void)once;                                                                                                      \
+    DISPATCH_T(dp, TP, (delta_prep32_kernel<KT_, TP><<<g1, 256, lds1(KT_), st>>>(A)));                               \
+    delta_chunk32_kernel<KT_><<<g2, 256, lds2(KT_), st>>>(A);                                                        \
+  } while (0)
+  if (dim <= 32) LAUNCH_DC32(2);
+  else if (dim <= 64) LAUNCH_DC32(4);
+  else LAUNCH_DC32(8);
+#undef LAUNCH_DC32
   HIP_CHECK_LAUNCH();
 }

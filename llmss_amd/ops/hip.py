@@ -1403,14 +1403,17 @@ def delta_recurrence(q, k, v, a, b_, A_log, dt_bias, state, cu, ctx_lens, state_
     return out
 
 
+# smallest portion (rows of the step's longest one) of fp32 rows that the chunked form takes: 64 sequences of 16 heads 128 x 128
+# take 121 us chunk by chunk whatever their portions up to 16 rows, 107 us token by token with 4 rows and 140 us with 8
+DELTA32_CHUNK_MIN = 6
 _DELTA_MFMA = os.environ.get("LLMSS_DELTA_MFMA", "1") != "0"  # 0: portions token by token (A/B runs)
 
 
 def delta_mix(q, k, v, a, b_, A_log, dt_bias, state, cu, ctx_lens, state_slots, heads, kv_heads, dim, vdim, gate, w, eps,
               scale, out, max_qlen=0, num_decode=0):
     """The ``num_decode`` leading single-row sequences (all of them when ``max_qlen`` is 1) take one fused launch; portions of
-    bf16 rows the chunked form on the matrix cores, everything else the token-by-token walk, then the per-head norm and
-    gate."""
+    bf16 rows (and longer ones of fp32 rows) the chunked form on the matrix cores, everything else the token-by-token walk,
+    then the per-head norm and gate."""
     N = heads * vdim
     _rows(gate, "gate", N)
     _rows(out, "out", N)
@@ -1422,14 +1425,18 @@ def delta_mix(q, k, v, a, b_, A_log, dt_bias, state, cu, ctx_lens, state_slots, 
     L, st, dt, es = lib(), _stream(), _dt(out, "out"), out.element_size()
     nd = B if max_qlen == 1 else int(num_decode)
     _check(0 <= nd <= B and (nd < B or T == B), "num_decode outside the step")
-    same = q.dtype == k.dtype == v.dtype == a.dtype == out.dtype
-    if not (same and L.delta_step_ok(dim, vdim) and state.data_ptr() % 16 == 0):
+    rows = q.dtype == k.dtype == v.dtype
+    same = rows and q.dtype == a.dtype == out.dtype
+    wide = rows and q.dtype == torch.float32  # rows in 32 bits beside projections of either type
+    if not (a.dtype == out.dtype and (same or wide) and L.delta_step_ok(dim, vdim) and state.data_ptr() % 16 == 0):
         nd = 0
     qkv = (q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), k.stride(0), v.stride(0))
     ab = (a.data_ptr(), b_.data_ptr(), a.stride(0), A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr())
     o = None
-    if nd < B and not (same and q.dtype == torch.bfloat16 and max_qlen > 0 and _DELTA_MFMA and L.delta_chunk_ok(dim, vdim)
-                       and not any(p % 16 for p in qkv[:2]) and not any(x % 8 for x in qkv[3:5])):
+    wide = wide and L.delta_chunk32_ok(dim, vdim) and max_qlen >= DELTA32_CHUNK_MIN
+    chunk = (wide or same and q.dtype == torch.bfloat16 and max_qlen > 0 and L.delta_chunk_ok(dim, vdim)) and _DELTA_MFMA \
+        and not any(p % 16 for p in qkv[:2]) and not any(x * q.element_size() % 16 for x in qkv[3:5])
+    if nd < B and not chunk:
         o = delta_recurrence(q, k, v, a, b_, A_log, dt_bias, state, cu, ctx_lens, state_slots, heads, kv_heads, dim, vdim, nd)
     else:
         _, _, o = _rec_common(q, k, v, state, cu, ctx_lens, state_slots, heads, kv_heads, dim, vdim)
@@ -1437,13 +1444,16 @@ def delta_mix(q, k, v, a, b_, A_log, dt_bias, state, cu, ctx_lens, state_slots, 
         if nd < B:
             work = torch.empty(4, T, heads, 64, dtype=torch.bfloat16, device=q.device)
             aux = torch.empty(T, heads, 4, dtype=torch.float32, device=q.device)
-            L.delta_chunk(*qkv, *ab, cu.data_ptr() + 4 * nd, ctx_lens.data_ptr() + 4 * nd, state_slots.data_ptr() + 4 * nd,
-                          o.data_ptr(), work.data_ptr(), aux.data_ptr(), T, B - nd, int(max_qlen), heads, kv_heads, dim,
-                          vdim, st)
+            args = (*qkv, *ab, cu.data_ptr() + 4 * nd, ctx_lens.data_ptr() + 4 * nd, state_slots.data_ptr() + 4 * nd,
+                    o.data_ptr(), work.data_ptr(), aux.data_ptr(), T, B - nd, int(max_qlen), heads, kv_heads, dim, vdim)
+            if wide:
+                L.delta_chunk32(*args, _dt(a, "a"), st)
+            else:
+                L.delta_chunk(*args, st)
     if nd:
         L.delta_step(*qkv, *ab, cu.data_ptr(), ctx_lens.data_ptr(), state_slots.data_ptr(), gate.data_ptr(), gate.stride(0),
                      w.data_ptr(), float(eps), float(scale), out.data_ptr(), out.stride(0), nd, heads, kv_heads, dim, vdim,
-                     dt, st)
+                     _dt(q, "q"), dt, st)
     if nd < B:  # the portions' rows: nd .. T - 1 (single-row sequences come first)
         L.gated_group_norm(o.data_ptr() + 4 * nd * N, N, gate.data_ptr() + es * nd * gate.stride(0), gate.stride(0),
                            w.data_ptr(), float(eps), 1, float(scale), out.data_ptr() + es * nd * out.stride(0),
