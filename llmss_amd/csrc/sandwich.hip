@@ -349,6 +349,148 @@ __global__ __launch_bounds__(512) void token_side_add_kernel(SandwichArgs p, Sid
   norm_out<T, V>(xs, ss2, p, t, red);
 }
 
+// The token input for bf16 weights, 16 rows per workgroup on the matrix cores (the kernel above reads both small matrices from L2
+// for every row: 2 GB per prompt step
+// of 8192 rows at width 2048, 189 us; 52 us here, of which 27 are the bytes of x and h: a workgroup is a chain of two products and
+// two norms of 25 us, so below 1024 rows, where the chip is not filled twice, the kernel above is the faster one: 13 us at 64 rows,
+// 26 on both at 1006). Wave w takes an eighth of the width. First product:
+// the fp32 rows enter as three bf16 numbers that add up to them exactly, the weights are exact, the waves' sums meet in LDS.
+// Second: the weights' rows are the first operand, so that a lane holds four neighbouring columns of one row - 16-byte accesses
+// of x, 8-byte ones of h - and the projected row, then the new x, stay in registers between the norms.
+// DT: 16-number blocks of d; NT: 16-column blocks per wave, at least W / 128.
+template <int DT, int NT>
+__global__ __launch_bounds__(512, NT <= 16 ? 4 : 2) void token_side_rows_kernel(SandwichArgs p, SideArgs s, int T_) {
+  constexpr int D = 16 * DT, LDG = D + 4;
+  __shared__ __attribute__((aligned(16))) float part[8 * 16 * D];
+  __shared__ __attribute__((aligned(16))) float gs[16 * LDG];
+  __shared__ float red[2][8 * 16];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, g = lane >> 4;
+  const int t0 = blockIdx.x * 16, W = p.W, span = W >> 3, c0 = w * span;
+  const int t = min(t0 + li, T_ - 1);  // this lane's row, as first operand and in the results
+  const bf16_t* wg = (const bf16_t*)s.wg;
+  const bf16_t* wp = (const bf16_t*)s.wp;
+  float* xr = p.x + (int64_t)t * W;
+  auto split = [](const float* v, s16x8& h, s16x8& m, s16x8& l) {  // cut off, not rounded: 8 bits each
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float a = __uint_as_float(__float_as_uint(v[i]) & 0xffff0000u), b = v[i] - a;
+      const float c = __uint_as_float(__float_as_uint(b) & 0xffff0000u);
+      h[i] = (short)(__float_as_uint(a) >> 16);
+      m[i] = (short)(__float_as_uint(c) >> 16);
+      l[i] = (short)(__float_as_uint(b - c) >> 16);
+    }
+  };
+  f32x4 acc[DT];
+#pragma unroll
+  for (int k = 0; k < DT; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int k = c0 + 8 * g; k < c0 + span; k += 32) {
+    float v[8];
+    ldv<float, 4>(xr + k, v);
+    ldv<float, 4>(xr + k + 4, v + 4);
+    s16x8 b[DT], h, m, l;
+#pragma unroll
+    for (int j = 0; j < DT; ++j) b[j] = *reinterpret_cast<const s16x8*>(wg + (int64_t)(16 * j + li) * W + k);
+    split(v, h, m, l);
+#pragma unroll
+    for (int j = 0; j < DT; ++j) {
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l, b[j], acc[j], 0, 0, 0);
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(m, b[j], acc[j], 0, 0, 0);
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h, b[j], acc[j], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < DT; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) part[(w * 16 + 4 * g + i) * D + 16 * j + li] = acc[j][i];
+  __syncthreads();
+  for (int e = tid; e < 16 * D; e += 512) {
+    const int r = e / D, j = e - r * D;
+    float a = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a += part[(k * 16 + r) * D + j];
+    int64_t id = s.ids[min(t0 + r, T_ - 1)];
+    id = id < 0 ? 0 : (id >= s.vocab ? s.vocab - 1 : id);
+    gs[r * LDG + j] = gelu_tanh_f(a) * bf2f(((const bf16_t*)s.table)[id * s.ldt + s.col0 + j]);
+  }
+  __syncthreads();
+  f32x4 y[NT];
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct) y[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < DT / 2; ++k) {
+    float v[8];
+    s16x8 h, m, l;
+    ldv<float, 4>(&gs[li * LDG + 32 * k + 8 * g], v);
+    ldv<float, 4>(&gs[li * LDG + 32 * k + 8 * g + 4], v + 4);
+    split(v, h, m, l);
+#pragma unroll
+    for (int ct = 0; ct < NT; ++ct) {
+      // (blocks past the wave's columns take its last one again; their sums are dropped below)
+      const s16x8 a = *reinterpret_cast<const s16x8*>(wp + (int64_t)(c0 + min(16 * ct, span - 16) + li) * D + 32 * k + 8 * g);
+      y[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, l, y[ct], 0, 0, 0);
+      y[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, m, y[ct], 0, 0, 0);
+      y[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, h, y[ct], 0, 0, 0);
+    }
+  }
+  auto row_inv = [&](float ss, float* r8) {  // 1 / root mean square of the lane's row
+    ss += __shfl_xor(ss, 16, 64);
+    ss += __shfl_xor(ss, 32, 64);
+    if (g == 0) r8[w * 16 + li] = ss;
+    __syncthreads();
+    float a = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a += r8[k * 16 + li];
+    return 1.0f / sqrtf(a / (float)W + p.eps);
+  };
+  float ss = 0.f;
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct) {
+    if (16 * ct >= span) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ss = fmaf(y[ct][i], y[ct][i], ss);
+  }
+  const float inv = row_inv(ss, red[0]);
+  const bool in = t0 + li < T_;
+  const float* ar = p.add ? p.add + (int64_t)t * W : nullptr;
+  ss = 0.f;
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct) {
+    if (16 * ct >= span) continue;
+    const int c = c0 + 16 * ct + 4 * g;
+    float xv[4], wn[4];
+    ldv<float, 4>(xr + c, xv);
+    ldv<float, 4>(s.wn + c, wn);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) xv[i] = fmaf(y[ct][i] * inv, wn[i], xv[i]);
+    if (ar) {
+      float a[4];
+      ldv<float, 4>(ar + c, a);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xv[i] += a[i];
+    }
+    if (in) stv<float, 4>(xr + c, xv);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      y[ct][i] = xv[i];
+      ss = fmaf(xv[i], xv[i], ss);
+    }
+  }
+  if (!p.wnext) return;
+  const float inv2 = row_inv(ss, red[1]);
+  bf16_t* hr = (bf16_t*)p.h + (int64_t)t * p.ldh;
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct) {
+    if (16 * ct >= span) continue;
+    const int c = c0 + 16 * ct + 4 * g;
+    float wn[4], o[4];
+    ldv<float, 4>(p.wnext + c, wn);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = y[ct][i] * inv2 * wn[i];
+    if (in) stv<bf16_t, 4>(hr + c, o);
+  }
+}
+
 void launch_token_side_add(void* x, const void* ids, const void* table, int64_t ldt, int vocab, int col0, int d,
                            const void* wg, const void* wp, const void* wn, const void* add, const void* wnext, void* h,
                            int64_t ldh, float eps, int T_, int W, int dt, hipStream_t st) {
@@ -361,6 +503,19 @@ void launch_token_side_add(void* x, const void* ids, const void* table, int64_t 
   const int es = dt == 0 ? 2 : 4;
   const bool vec = W % 4 == 0 && al16(x) && al16(wn) && al16(add) && al16(wnext) && ((uintptr_t)wg % (4 * es)) == 0 &&
                    (!h || (((uintptr_t)h % (4 * es)) == 0 && ldh % 4 == 0));
+  if (dt == 0 && vec && T_ >= 1024 && (d == 32 || d == 64) && W % 256 == 0 && W <= 4096 && al16(wg) && al16(wp)) {
+#define LAUNCH_SIDE(DT_)                                                                              \
+  do {                                                                                                \
+    if (W <= 1024) token_side_rows_kernel<DT_, 8><<<(T_ + 15) / 16, 512, 0, st>>>(p, s, T_);          \
+    else if (W <= 2048) token_side_rows_kernel<DT_, 16><<<(T_ + 15) / 16, 512, 0, st>>>(p, s, T_);    \
+    else token_side_rows_kernel<DT_, 32><<<(T_ + 15) / 16, 512, 0, st>>>(p, s, T_);                   \
+  } while (0)
+    if (d == 32) LAUNCH_SIDE(2);
+    else LAUNCH_SIDE(4);
+#undef LAUNCH_SIDE
+    HIP_CHECK_LAUNCH();
+    return;
+  }
   DISPATCH_T(dt, T, {
     if (vec) token_side_add_kernel<T, 4><<<T_, 512, lds, st>>>(p, s);
     else token_side_add_kernel<T, 1><<<T_, 512, lds, st>>>(p, s);
