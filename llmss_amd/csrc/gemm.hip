@@ -1653,11 +1653,94 @@ bool gemm_tuned_get(int M, int N, int K, bool glu, int kind, int* nt_hint, int* 
   return true;
 }
 
+// Plan of a bf16 product that carries no hint and no tuned plan: prompt and mixed steps of any size, models run without the
+// autotuner. Leaves the hints at 0 where the older static rules below are still the better ones.
+//
+// M <= 64: the K-split-wave decode kernel (gemm_dec.hip) on column tiles of 16 - 64, the width that makes the waves of 256
+// workgroups times the tile's width smallest, ties to the wider. Over 13 shapes of 1024 - 32000 columns (bench shapes of the
+// 1024, 1600, 2048 and 4096 wide models) this is 0.4 - 3 % above the best plan found at M <= 20 and 1.5 (M <= 16) and 1.2
+// (M = 20) times faster than the streaming / 64 x 64 plans: 4096 x 4096 at one row 13.6 -> 9.6 us, 22016 x 4096 44 -> 35 us. From 33 rows on
+// narrow products read X too often for their weights and keep the 64 x 64 tiles: below 3072 columns (2048 x 4096 at 64 rows:
+// 12.2 against 14.7 us), and where 16-column tiles would walk a long K (4096 x 11008: 27.8 against 35.7 us); very wide ones (SwiGLU,
+// LM heads) take one wave of 64 x 96 or 64 x 128 tiles (22016 x 4096 at 64 rows: 53 -> 39 us).
+//
+// M > 64: the cheapest of six tiles by a cost model. A wave of the chip takes (k-steps of 64) x us per step + 5 us, an unfilled
+// second workgroup per CU counts for less, a K split adds its slabs' write and read at 4.5 TB/s and a launch, and nothing
+// beats the operands' bytes at 4 TB/s. Steps measured at M = 80 - 6000 over the shapes above; the choice is 2.7 % above the
+// best of 60 plans on average, and 1.5 times faster than 128 x 128 tiles below 192 tiles of 256 x 256 (4096 x 4096: M = 500 56
+// -> 29, M = 1000 93 -> 45, M = 1536 135 -> 66 us; 4096 x 11008 at M = 1000: 197 -> 100 us).
+struct TileCost {
+  int tsel;      // tile | depth code << 4 (| 512: interleaved ring)
+  int bm, bn, per_cu;
+  double step;   // us per 64 of k with the chip full
+  double alone;  // the same with one of two workgroups per CU
+};
+static constexpr TileCost kTileCost[] = {
+    {4, 256, 256, 1, 1.45, 1.45},           {9 | 16, 256, 128, 1, 1.02, 1.02},        {12 | 16 | 512, 128, 256, 1, 1.06, 1.06},
+    {8 | 32 | 512, 128, 128, 1, 0.70, 0.70}, {11 | 32 | 512, 64, 128, 1, 0.41, 0.41}, {11 | 16, 64, 128, 2, 0.64, 0.44},
+};
+// slabs: the consumer sums split-K slabs itself and so gets the product in 32 bits. Where the older rules split K that stays so:
+// only split plans are looked at, their slabs costing a write and a read and no launch.
+static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t ws_bytes, int* nt_hint, int* split) {
+  if (N % 8 || K % 16) return;
+  if (slabs) {
+    int t = 0, s = 0;
+    if (M <= 16) gemm_stream_plan(M, N, K, &t, &s);
+    else gemm_tiled_plan(M, N, K, &t, &s, glu);
+    slabs = s > 1 && (int64_t)s * M * N * 4 <= ws_bytes;
+  }
+  if (M <= 64) {
+    if (M > 32 && N > 16384 && !slabs) {
+      const int t96 = (N + 95) / 96;
+      *nt_hint = (t96 <= 256 ? 15 | 32 : 11 | 32) << 8;
+      *split = 1;
+      return;
+    }
+    int best = 0, width = 0, sp = 1;
+    for (int s = slabs ? 2 : 1; s <= (slabs ? 4 : 1); s *= 2) {
+      if (s > 1 && K / s < 256) break;
+      for (int code = 4; code >= 1; --code) {  // 64, 48, 32, 16 columns
+        const int bn = 16 * code;
+        if (glu && bn % 32) continue;
+        const int cost = ((N + bn - 1) / bn * s + 255) / 256 * bn * (4 / s);
+        if (!best || cost < best) best = cost, width = bn, sp = s;
+      }
+    }
+    if (!best || (M > 32 && (N < 3072 || (width == 16 && K > 4096)))) return;
+    *nt_hint = (width / 16 | 32 | 1024) << 8;
+    *split = sp;
+    return;
+  }
+  const int nk = (K + 63) / 64;
+  const double bytes = 2.0 * N * K + 2.0 * M * K + 2.0 * M * (glu ? N / 2 : N);
+  double best = 0;
+  for (const TileCost& c : kTileCost) {
+    for (int s : {1, 2, 3, 4, 6, 8}) {
+      if (s == 1 && slabs) continue;
+      if (s > 1 && (c.tsel == 4 || K / s < 256 || (int64_t)s * M * N * 4 > ws_bytes)) break;
+      const int per = (nk + s - 1) / s;
+      const int64_t wgs = (int64_t)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * s, slots = 256 * c.per_cu;
+      const int64_t rest = wgs % slots;
+      double t = (double)(wgs / slots) * (per * c.step + 5.0);
+      if (rest) t += per * (rest <= 256 ? c.alone : c.step) + 5.0;
+      t = std::max(t, bytes / 4.0e6);
+      if (s > 1) t += (slabs ? 0.0 : 4.0) + 8.0 * s * M * N / 4.5e6;
+      if (best == 0 || t < best) {
+        best = t;
+        *nt_hint = (K % 64 ? c.tsel & ~512 : c.tsel) << 8;
+        *split = s;
+      }
+    }
+  }
+}
+
 int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_fp8, const void* w_scale,
                 const void* bias, void* y, int64_t ldy, int M, int N, int K, int act, bool glu, void* workspace,
                 int64_t ws_bytes, int nt_hint, int split_hint, bool partial_out, hipStream_t st) {
   if (M == 0 || N == 0) return 0;
-  if (nt_hint == 0 && split_hint == 0) gemm_tuned_get(M, N, K, glu, w_fp8 ? 1 : 0, &nt_hint, &split_hint);
+  if (nt_hint == 0 && split_hint == 0 && !gemm_tuned_get(M, N, K, glu, w_fp8 ? 1 : 0, &nt_hint, &split_hint) && !w_fp8 &&
+      ldx % 8 == 0 && ldw % 8 == 0 && !(((uintptr_t)x | (uintptr_t)w) & 15))
+    gemm_static_plan(M, N, K, glu, partial_out && !glu && act == 0, ws_bytes, &nt_hint, &split_hint);
   if (!y && (!partial_out || gemm_partial_slabs(M, N, K, w_fp8, glu, act, nt_hint, split_hint, ws_bytes) == 0))
     throw std::runtime_error("gemm: this configuration writes the output, but no output buffer was given");
   if (K % 16) throw std::runtime_error("gemm: K must be a multiple of 16");
@@ -2009,7 +2092,8 @@ int launch_tiled(const bf16_t* X, int64_t ldx, const void* W, int64_t ldw, const
 int gemm_partial_slabs(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint,
                        int64_t ws_bytes) {
   if (M == 0 || N == 0 || glu || act != 0) return 0;
-  if (nt_hint == 0 && split_hint == 0) gemm_tuned_get(M, N, K, glu, w_fp8 ? 1 : 0, &nt_hint, &split_hint);
+  if (nt_hint == 0 && split_hint == 0 && !gemm_tuned_get(M, N, K, glu, w_fp8 ? 1 : 0, &nt_hint, &split_hint) && !w_fp8)
+    gemm_static_plan(M, N, K, glu, true, ws_bytes, &nt_hint, &split_hint);
   const int tiled_hint = nt_hint >> 8;
   const bool stream = (nt_hint & 0xff) || (!tiled_hint && (M <= 16 || (w_fp8 && M > 128)));
   int s;
@@ -2095,7 +2179,10 @@ int launch_gemm_qkv_args(const void* x, int64_t ldx, const void* w, int64_t ldw,
 }
 
 void gemm_plan(int M, int N, int K, bool w_fp8, int* nt, int* splitk) {
-  if (gemm_tuned_get(M, N, K, false, w_fp8 ? 1 : 0, nt, splitk)) {
+  *nt = *splitk = 0;
+  const bool tuned = gemm_tuned_get(M, N, K, false, w_fp8 ? 1 : 0, nt, splitk);
+  if (!tuned && !w_fp8) gemm_static_plan(M, N, K, false, true, 64 << 20, nt, splitk);
+  if (tuned || *nt) {
     if ((*nt >> 8) & kDecHint) {
       *splitk = ((*nt >> 8) & 256) ? 1 : dec_split(M, N, K, *splitk, INT64_MAX);
     } else if ((*nt >> 8) & (128 | 256)) {

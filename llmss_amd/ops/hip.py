@@ -886,17 +886,6 @@ def _mfma_ok(x, w, out_dtype) -> bool:
             and x.data_ptr() % 16 == 0 and (x.stride(0) * 2) % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-def prompt_plan(M: int, N: int, K: int):
-    """(nt_hint, split) of a prompt's product that is too narrow to fill the chip with 256 x 256 tiles: 128 x 256 tiles, K split
-    until there are about as many workgroups as compute units. (0, 0): the GEMM's own plan."""
-    if M < 2048 or -(-M // 256) * -(-N // 256) >= 192 or N < 128 or lib().gemm_tuned_get(M, N, K, False, 0) is not None:
-        return 0, 0
-    split = 1
-    while split < 4 and -(-M // 128) * -(-N // 256) * split * 2 <= 288 and K // (2 * split) >= 512:
-        split *= 2
-    return (12 | 16 | (512 if K % 64 == 0 else 0)) << 8, split
-
-
 def linear_f(x, w, out_dtype, bias=None, act="none"):
     """act(x [M, K] . w [N, K]^T + bias) -> [M, N] in ``out_dtype`` with fp32 accumulation: the MFMA GEMM where it applies
     (bias and activation in its epilogue), else the tile GEMM or the strided VALU GEMM (fp32 storage, fp32 output, odd
@@ -911,8 +900,7 @@ def linear_f(x, w, out_dtype, bias=None, act="none"):
     if M == 0:
         return torch.empty(0, N, dtype=out_dtype, device=x.device)
     if _mfma_ok(x, w, out_dtype):
-        nt, split = prompt_plan(M, N, K)
-        return linear(x, w, bias, act, nt_hint=nt, split_hint=split)
+        return linear(x, w, bias, act)
     y = torch.empty(M, N, dtype=out_dtype, device=x.device)
     gemm_any(x, w, y, M, N, K, 1, 0, x.stride(0), 0, K, 1, 0, N, bias)
     return y if act in ("none", None) else act_fn(y, act)
