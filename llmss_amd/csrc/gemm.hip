@@ -23,6 +23,7 @@
 // Split-K partial slabs never leave a call unless gemm_partial_slabs() says so (one source of
 // truth shared with the Python wrapper).
 #include "common.h"
+#include "gemm_quad.h"
 
 #include <mutex>
 #include <unordered_map>
@@ -688,7 +689,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_tiled_kernel(const bf16_t* __res
 }
 
 // -------------------------------------------------------------------------------------------
-// W8A8 big-tile GEMM (fp8 prefill, M >= ~1024; bf16 prompt batches take gemm_pp_kernel below):
+// W8A8 big-tile GEMM (fp8 prefill, M >= ~1024; bf16 prompt batches take gemm_quad.hip or gemm_pp_kernel below):
 // 256x256 tile of 128-element fp8 K-tiles, 8 waves (2 x 4), each wave 128x64 = 8x4 accumulators on the
 // MX-fp8 16x16x128 MFMA. LDS = 2 buffers x {A rows 0-127, A rows 128-255, B rows 0-127, B rows 128-255}
 // of 16 KiB = 128 KiB -> one workgroup per CU.
@@ -882,7 +883,7 @@ __global__ __launch_bounds__(512, 1) void gemm_big_kernel(const void* __restrict
 }
 
 // -------------------------------------------------------------------------------------------
-// Ping-pong prefill GEMM (bf16, M >= ~1024): the shipped bf16 big-tile kernel (profiles/r5_gemm_pp).
+// Ping-pong prefill GEMM (bf16, M >= ~1024) for what gemm_quad.hip does not take: K off 64, N off 8, outputs off 16 bytes.
 // 256x256x64 tile, 8 waves = two groups of 4 (waves 0-3 / 4-7; one wave of each group per SIMD). Waves
 // 4-7 pass one extra barrier before the K-loop, so on every SIMD one wave's compute segment runs beside
 // its partner's load segment (guide "The 256^2 8-phase template", MI355X_MICROARCH "Two waves per SIMD").
@@ -910,14 +911,6 @@ __device__ __forceinline__ void pp_barrier() {
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
 }
-
-struct PpGroup {
-  const int* meta = nullptr;
-  const int* order = nullptr;
-  int E = 0, maxt = 0, top = 1;
-  int64_t sB = 0;         // elements between the experts' weights
-  float* Yf = nullptr;    // GRP 2
-};
 
 template <bool KTAIL, int GRP = 0>
 __global__ __launch_bounds__(512, 1) void gemm_pp_kernel(const bf16_t* __restrict__ A, int64_t lda,
@@ -1992,7 +1985,10 @@ int launch_tiled(const bf16_t* X, int64_t ldx, const void* W, int64_t ldw, const
   if ((tsel == 2 || tsel == 6) && ns > 4) ns = 4;
   if (f8 && tsel == 4) tsel = 1;
   if (tsel == 4) {
-    if (K & 63)
+    if (gemm_quad_ok(N, K, ldx, ldw, 256, Y, ldy, 2, g != 0))
+      launch_gemm_quad(0, X, ldx, (const bf16_t*)W, ldw, B, Y, ldy, M, N, K, act, g, g_big_group_m,
+                       tiles_of(M, N, 256, 256), PpGroup{}, st);
+    else if (K & 63)
       gemm_pp_kernel<true><<<tiles_of(M, N, 256, 256), 512, 0, st>>>(X, ldx, (const bf16_t*)W, ldw, B, Y, ldy, M, N, K,
                                                                      act, g, g_big_group_m, zero_page(), PpGroup{});
     else
@@ -2219,6 +2215,13 @@ void launch_moe_pp(int mode, const void* A, int64_t lda, const void* W, const vo
   const char* z = K & 63 ? zero_page() : nullptr;
   const int glu = mode == 3;
   if (glu && N % 32) throw std::runtime_error("moe_pp: gate and up in groups of 16 rows");
+  if (gemm_quad_ok(N, K, lda, K, mode == 2 ? 256 : (int64_t)maxt * 256 / std::max(top, 1) + 1, C, glu ? N / 2 : N,
+                   mode == 2 ? 4 : 2, glu != 0)) {
+    if (mode < 1 || mode > 3) throw std::runtime_error("moe_pp: mode");
+    launch_gemm_quad(mode == 2 ? 2 : 1, (const bf16_t*)A, lda, (const bf16_t*)W, K, nullptr, (bf16_t*)C, glu ? N / 2 : N, 0, N, K,
+                     glu ? 0 : act, glu, 1, (unsigned)nwg, gr, st);
+    return;
+  }
 #define LAUNCH_PPG(KT_, G_)                                                                                         \
   gemm_pp_kernel<KT_, G_><<<(unsigned)nwg, 512, 0, st>>>((const bf16_t*)A, lda, (const bf16_t*)W, K, nullptr, (bf16_t*)C, \
                                                          glu ? N / 2 : N, 0, N, K, glu ? 0 : act, glu, 1, z, gr)

@@ -1,0 +1,273 @@
+// Prompt GEMM (bf16, K % 64 == 0): Y[M, N] = epilogue(X[M, K] . W[N, K]^T) on 256 x 256 tiles by FOUR waves, a wave per SIMD with a
+// 128 x 128 part of the tile.
+//
+// Bound by the matrix units' power: with loads and epilogue taken out, 64 of k take a wave of 256 tiles 1.27 us, far over the 0.85 us of
+// the issue rate at 2.4 GHz, and 1.5 us as it stands. Per 64 of k a wave reads (128 + 128) x 64 for 128 products, half of what
+// eight waves read together, and the reads are free behind them. What costs is the loads and the epilogue:
+// - a step's loads are issued 1.5 (X) and 1 (W) steps before the barrier that waits for them, by count. With a step's distance of less than
+//   one (two buffers) it took 1.63 - 1.84 us; a ring of four 32-k buffers, with more distance but rows of 64 bytes, 1.6 - 1.75 us.
+// - 42 us a tile with stores of 64 bytes a row straight from the accumulators, 20 us through LDS with the activations' code
+//   unrolled (36 KB of it), 6 - 8 us as written below.
+// Against the ping-pong kernel of 8 waves (weights not in the caches, us): 8192 x 12288 x 4096 794 -> 715, 8192 x 4096 x 4096 232 -> 206,
+// 8192 x 4096 x 11008 540 -> 530, 8192 x 11264 x 2048 379 -> 330; SwiGLU 8192 x 22016 x 4096 1237 (1195 TFLOP/s).
+//
+// GRP: grouped expert products over moe.hip's list of 256-row tiles, as in the ping-pong kernel: 1 - rows of X gathered through
+// order[] / top, activation or gating in the epilogue; 2 - rows in expert order, fp32 output. GLU: W's rows are gate and up in
+// alternating groups of 16.
+#include "gemm_quad.h"
+
+template <int GRP, bool GLU>
+__global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restrict__ X, int64_t ldx,
+                                                           const bf16_t* __restrict__ W, int64_t ldw,
+                                                           const bf16_t* __restrict__ bias, bf16_t* __restrict__ Y,
+                                                           int64_t ldy, int M, int N, int K, int act, int group_m, PpGroup gr) {
+  // a ring of five buffers, each 64 of k (128 bytes, a line) of 256 rows: X of step 0, W of step 0, X of step 1, ...
+  constexpr int BUF = 32768, NB = 5, QA = 6;
+  __shared__ __attribute__((aligned(16))) char smem[NB * BUF];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, g = lane >> 4;
+  const int wr = w >> 1, wc = w & 1;
+  const int ntn = (N + 255) / 256, ntm = (M + 255) / 256;
+  int m0, n0;
+  if constexpr (GRP != 0) {
+    const int nt = gr.meta[0];
+    if ((int)blockIdx.x >= nt * ntn) return;
+    const int id = xcd_remap(blockIdx.x, nt * ntn), ty = id / ntn;
+    const int e = gr.meta[1 + (gr.E + 1) + ty];
+    n0 = (id - ty * ntn) * 256;
+    m0 = gr.meta[1 + (gr.E + 1) + gr.maxt + ty];
+    M = gr.meta[1 + e + 1];
+    W += (int64_t)e * gr.sB;
+  } else {
+    const int tile = xcd_remap(blockIdx.x, ntn * ntm);
+    const int grp = tile / (group_m * ntn), gidx = tile - grp * (group_m * ntn);
+    const int gm = min(group_m, ntm - grp * group_m);
+    m0 = (grp * group_m + gidx % gm) * 256, n0 = (gidx / gm) * 256;
+  }
+  const int nk = K >> 6;
+  const uint64_t xbytes = (uint64_t)(M - m0) * (uint64_t)ldx * 2, wbytes = (uint64_t)(N - n0) * (uint64_t)ldw * 2;
+  const auto rx = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char*>(reinterpret_cast<const char*>(X) + (GRP == 1 ? 0 : (int64_t)m0 * ldx * 2)), (short)0,
+      (int)(GRP == 1 || xbytes > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)xbytes), 0x00020000);
+  const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(W) + (int64_t)n0 * ldw * 2),
+                                                    (short)0, (int)(wbytes > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)wbytes),
+                                                    0x00020000);
+  // chunk c of row r lies at place c ^ key(r) of the row: the eight rows that a fragment read's eight lanes take fall on eight
+  // different 16-byte columns of the banks
+  auto xkey = [](int r) { return r & 7; };
+  auto wkey = [](int r) { return GLU ? r & 7 : (r & 3) | ((r >> 3) & 1) << 2; };
+  uint32_t vx[8], vw[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int row = (i * 4 + w) * 8 + (lane >> 3);
+    int xr = row;
+    if constexpr (GRP == 1) xr = gr.order[min(m0 + row, M - 1)] / gr.top;
+    vx[i] = (uint32_t)xr * (uint32_t)(ldx * 2) + (uint32_t)(((lane & 7) ^ xkey(row)) << 4);
+    vw[i] = (uint32_t)row * (uint32_t)(ldw * 2) + (uint32_t)(((lane & 7) ^ wkey(row)) << 4);
+  }
+  // eight rows (1 KB) of step T_ of X or W into buffer B_
+#define Q_LOADX(I_, T_, B_)                                                                                           \
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (LDS_AS void*)(smem + (B_) + ((I_) * 4 + w) * 1024), 16, vx[I_], (uint32_t)((T_) * 128), 0, 0)
+#define Q_LOADW(I_, T_, B_)                                                                                           \
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (LDS_AS void*)(smem + (B_) + ((I_) * 4 + w) * 1024), 16, vw[I_], (uint32_t)((T_) * 128), 0, 0)
+  const int wrow = GLU ? li : 8 * (li >> 2) + (li & 3);
+  const int xo = (wr * 128 + li) * 128 + ((g ^ xkey(li)) << 4);
+  const int wo = (wc * 128 + wrow) * 128 + ((g ^ wkey(wrow)) << 4);
+#define Q_X(P_, T_) (*reinterpret_cast<const s16x8*>(smem + (P_) + (T_) * 2048))
+#define Q_W(P_, T_) (*reinterpret_cast<const s16x8*>(smem + (P_) + (GLU ? (T_) * 2048 : ((T_) >> 1) * 4096 + ((T_) & 1) * 512)))
+  f32x4 acc[8][8];  // [W tile][X tile]
+#pragma unroll
+  for (int a = 0; a < 8; ++a)
+#pragma unroll
+    for (int b = 0; b < 8; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  s16x8 w0[8], x0[8], w1[8], x1[8];
+  // In place by the instruction's own operands: left to itself the compiler, with every accumulation register taken, rotates the
+  // accumulators through the file by 272 moves per 64 of k. A quarter of them lives in the vector file, so that both have room.
+#define Q_MFMA(W_, X_, NT_, MT_)                                                                                          \
+  do {                                                                                                                    \
+    if ((NT_) < QA)                                                                                                       \
+      asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[NT_][MT_]) : "v"(W_[NT_]), "v"(X_[MT_]));                  \
+    else                                                                                                                  \
+      asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[NT_][MT_]) : "v"(W_[NT_]), "v"(X_[MT_]));                  \
+  } while (0)
+#pragma unroll
+  for (int l = 0; l < 5; ++l) {
+    const int t = min(l >> 1, nk - 1);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (l & 1) Q_LOADW(i, t, l * BUF);
+      else Q_LOADX(i, t, l * BUF);
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x4F78);  // vmcnt(24): the first step has landed
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    w0[q] = Q_W(BUF + wo, q);
+    x0[q] = Q_X(xo, q);
+  }
+  // One copy of the body: with separate last steps the compiler moves every accumulator between register files. The last steps
+  // load the last one again, and the very last reads fragments that nobody uses.
+  int cx = 0;  // buffer of this step's X; its W lies in the next one
+#pragma unroll 1
+  for (int t = 0; t < nk; ++t) {
+    const int cw = cx == 4 * BUF ? 0 : cx + BUF;
+    const int nx = cw == 4 * BUF ? 0 : cw + BUF;
+    const int nw = nx == 4 * BUF ? 0 : nx + BUF;
+    const int xa = cx + (xo ^ 64), wa = cw + (wo ^ 64), xb = nx + xo, wb = nw + wo;
+    const int tw = min(t + 2, nk - 1), tx = min(t + 3, nk - 1);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      if (q < 8) {
+        w1[q] = Q_W(wa, q);
+        x1[q] = Q_X(xa, q);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) Q_MFMA(w0, x0, q >> 1, (q & 1) * 4 + e);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0078);  // vmcnt(8) lgkmcnt(0): this step is read, this wave's part of the next has landed
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      if (q < 8) {
+        w0[q] = Q_W(wb, q);
+        x0[q] = Q_X(xb, q);
+        Q_LOADW(q, tw, cx);
+      } else {
+        Q_LOADX(q - 8, tx, cw);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) Q_MFMA(w1, x1, q >> 1, (q & 1) * 4 + e);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    cx = nx;
+  }
+#undef Q_MFMA
+#undef Q_X
+#undef Q_W
+#undef Q_LOADX
+#undef Q_LOADW
+  __builtin_amdgcn_s_waitcnt(0x0070);                    // no load of this wave is on its way into LDS any more,
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");     // the last products are written, which the compiler does not see,
+  __builtin_amdgcn_s_barrier();                          // and all waves are there
+  __builtin_amdgcn_sched_barrier(0);
+  // Out through LDS, 64 columns of the wave's 128 rows at a time as fp32: stored from the accumulators' own layout (16 rows of 64
+  // bytes an instruction) the stores alone took 42 us a tile. A lane holds, of row 16 mt + li, eight neighbouring columns in tiles
+  // 2 p and 2 p + 1 (GLU: four gates and their four ups).
+  char* img = smem + w * BUF;
+  auto flush = [&](int c0) {  // the image is columns c0 .. c0 + 63 of the output
+    if constexpr (GRP == 2) {
+      const int n = c0 + 4 * li;
+#pragma unroll 4
+      for (int i = 0; i < 32; ++i) {
+        const int r = 4 * i + g, m = m0 + wr * 128 + r;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(img + r * 256 + ((li ^ (r & 15)) << 4));
+        if (m < M && n < N) *reinterpret_cast<f32x4*>(gr.Yf + (int64_t)m * ldy + n) = v;
+      }
+    } else {
+      const int j = lane & 7, n = c0 + 8 * j, nmax = GLU ? N / 2 : N;
+      float bl[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (!GLU && bias && n < nmax) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) bl[i] = bf2f(bias[n + i]);
+      }
+      auto row = [&](int i, float (&v)[8]) {
+        const int r = 8 * i + (lane >> 3);
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(img + r * 256 + (((2 * j) ^ (r & 15)) << 4));
+        const f32x4 hi = *reinterpret_cast<const f32x4*>(img + r * 256 + (((2 * j + 1) ^ (r & 15)) << 4));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] = lo[e] + bl[e];
+          v[4 + e] = hi[e] + bl[4 + e];
+        }
+      };
+      auto out = [&](int i, const float (&v)[8]) {
+        const int m = m0 + wr * 128 + 8 * i + (lane >> 3);
+        u16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = f2bf(v[e]);
+        if (m < M && n < nmax) *reinterpret_cast<u16x8*>(Y + (int64_t)m * ldy + n) = o;
+      };
+      float v[8];
+      if (GLU || act == 0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          row(i, v);
+          out(i, v);
+        }
+      } else {  // (one copy of the functions' code: unrolled it does not fit the instruction cache)
+#pragma unroll 1
+        for (int i = 0; i < 16; ++i) {
+          row(i, v);
+#pragma unroll 1
+          for (int h = 0; h < 2; ++h) {
+            f32x4 u = h ? f32x4{v[4], v[5], v[6], v[7]} : f32x4{v[0], v[1], v[2], v[3]};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) u[e] = apply_act(u[e], act);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              if (h) v[4 + e] = u[e];
+              else v[e] = u[e];
+            }
+          }
+          out(i, v);
+        }
+      }
+    }
+  };
+  auto put = [&](int p, const f32x4 (&lo)[8], const f32x4 (&hi)[8]) {
+    if constexpr (GLU) {
+      const int n = n0 + wc * 128 + 32 * p + 4 * g;
+      float bg[4], bu[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        bg[i] = bias && n < N ? bf2f(bias[n + i]) : 0.f;
+        bu[i] = bias && n < N ? bf2f(bias[n + 16 + i]) : 0.f;
+      }
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt) {
+        f32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = silu(lo[mt][i] + bg[i]) * (hi[mt][i] + bu[i]);
+        *reinterpret_cast<f32x4*>(img + (16 * mt + li) * 256 + (((4 * p + g) ^ li) << 4)) = v;
+      }
+    } else {
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt) {
+        char* row = img + (16 * mt + li) * 256;
+        const int c = 8 * (p & 1) + 2 * g;
+        *reinterpret_cast<f32x4*>(row + ((c ^ li) << 4)) = lo[mt];
+        *reinterpret_cast<f32x4*>(row + (((c + 1) ^ li) << 4)) = hi[mt];
+      }
+    }
+  };
+  put(0, acc[0], acc[1]);
+  put(1, acc[2], acc[3]);
+  if constexpr (!GLU) flush(n0 + wc * 128);
+  put(2, acc[4], acc[5]);
+  put(3, acc[6], acc[7]);
+  flush(GLU ? n0 / 2 + wc * 64 : n0 + wc * 128 + 64);
+}
+
+// rows: of X that one descriptor covers; es: bytes of an output element
+bool gemm_quad_ok(int N, int K, int64_t ldx, int64_t ldw, int64_t rows, const void* Y, int64_t ldy, int es, bool glu) {
+  return K % 64 == 0 && K >= 64 && (uint64_t)rows * (uint64_t)ldx * 2 < (1ull << 31) && (uint64_t)256 * (uint64_t)ldw * 2 < (1ull << 31) &&
+         ldx % 8 == 0 && ldw % 8 == 0 && N % (glu ? 32 : 8) == 0 && ((uintptr_t)Y & 15) == 0 && ldy * es % 16 == 0;
+}
+
+void launch_gemm_quad(int grp, const bf16_t* X, int64_t ldx, const bf16_t* W, int64_t ldw, const bf16_t* bias, bf16_t* Y,
+                      int64_t ldy, int M, int N, int K, int act, int glu, int group_m, unsigned nwg, const PpGroup& gr,
+                      hipStream_t st) {
+#define LAUNCH_Q(G_, U_) gemm_quad_kernel<G_, U_><<<nwg, 256, 0, st>>>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, act, group_m, gr)
+  if (grp == 2) LAUNCH_Q(2, false);
+  else if (grp == 1 && glu) LAUNCH_Q(1, true);
+  else if (grp == 1) LAUNCH_Q(1, false);
+  else if (glu) LAUNCH_Q(0, true);
+  else LAUNCH_Q(0, false);
+#undef LAUNCH_Q
+  HIP_CHECK_LAUNCH();
+}
