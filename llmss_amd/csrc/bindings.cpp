@@ -90,6 +90,9 @@ void launch_moe_gate_up_tile(const void* h, int64_t ldh, const void* wg, const v
                              float alpha, int tile_rows, const void* pw, int silu, int ilv, hipStream_t st);
 void launch_moe_pp(int mode, const void* A, int64_t lda, const void* W, const void* meta, const void* order, void* C, int E,
                    int maxt, int top, int N, int K, int act, hipStream_t st);
+bool moe_pp_glu_ok(int64_t ldh, int maxt, int top, int F, int K);
+void launch_moe_pp_glu(const void* h, int64_t ldh, const void* Wg, const void* Wu, const void* meta, const void* order, void* act,
+                       int E, int maxt, int top, int F, int K, float limit, float alpha, const void* pw, int silu, hipStream_t st);
 void launch_moe_down_tile(const void* act, const void* wd, const void* meta, void* y, int E, int maxt, int N, int F,
                           int tile_rows, hipStream_t st);
 void launch_latent_norm_cache(const void* src, int64_t ld, int off, const void* w, float eps, void* cache,
@@ -414,6 +417,11 @@ PYBIND11_MODULE(_C, m) {
   m.def("moe_pp", [](int mode, uintptr_t A, int64_t lda, uintptr_t W, uintptr_t meta, uintptr_t order, uintptr_t C, int E,
                      int maxt, int top, int N, int K, int act, uintptr_t st) {
     launch_moe_pp(mode, CP(A), lda, CP(W), CP(meta), CP(order), P(C), E, maxt, top, N, K, act, S(st));
+  });
+  m.def("moe_pp_glu_ok", &moe_pp_glu_ok);
+  m.def("moe_pp_glu", [](uintptr_t h, int64_t ldh, uintptr_t Wg, uintptr_t Wu, uintptr_t meta, uintptr_t order, uintptr_t act,
+                         int E, int maxt, int top, int F, int K, float limit, float alpha, uintptr_t pw, int silu, uintptr_t st) {
+    launch_moe_pp_glu(CP(h), ldh, CP(Wg), CP(Wu), CP(meta), CP(order), P(act), E, maxt, top, F, K, limit, alpha, CP(pw), silu, S(st));
   });
   m.def("moe_down_tile", [](uintptr_t act, uintptr_t wd, uintptr_t meta, uintptr_t y, int E, int maxt, int N, int F,
                             int tile_rows, uintptr_t st) {

@@ -2237,3 +2237,24 @@ void launch_moe_pp(int mode, const void* A, int64_t lda, const void* W, const vo
 #undef LAUNCH_PPG
   HIP_CHECK_LAUNCH();
 }
+
+// Whether moe_pp_glu takes a layer with gate and up matrices [E, F, K] of their own: h [rows, K] with row stride ldh.
+bool moe_pp_glu_ok(int64_t ldh, int maxt, int top, int F, int K) {
+  return gemm_quad_ok(2 * F, K, ldh, K, (int64_t)maxt * 256 / std::max(top, 1) + 1, nullptr, F, 2, true) && F % 16 == 0;
+}
+
+// act [pairs, F] = glu(pw h Wg_e^T, pw h Wu_e^T) in bf16 over a tile list of 256 rows per tile
+void launch_moe_pp_glu(const void* h, int64_t ldh, const void* Wg, const void* Wu, const void* meta, const void* order, void* act,
+                       int E, int maxt, int top, int F, int K, float limit, float alpha, const void* pw, int silu, hipStream_t st) {
+  if (maxt <= 0) return;
+  if (!moe_pp_glu_ok(ldh, maxt, top, F, K) || (((uintptr_t)h | (uintptr_t)Wg | (uintptr_t)Wu | (uintptr_t)act) & 15))
+    throw std::runtime_error("moe_pp_glu: K % 64, F % 16, rows of 16-byte alignment");
+  const int64_t nwg = (int64_t)maxt * ((2 * F + 255) / 256);
+  if (nwg > 0x7fffffff) throw std::runtime_error("moe_pp_glu: grid too large");
+  PpGroup gr;
+  gr.meta = (const int*)meta, gr.order = (const int*)order, gr.E = E, gr.maxt = maxt, gr.top = top;
+  gr.sB = (int64_t)F * K;
+  gr.Wu = (const bf16_t*)Wu, gr.pw = (const float*)pw, gr.limit = limit, gr.alpha = alpha, gr.silu = silu;
+  launch_gemm_quad(3, (const bf16_t*)h, ldh, (const bf16_t*)Wg, K, nullptr, (bf16_t*)act, F, 0, 2 * F, K, 0, 1, 1, (unsigned)nwg, gr,
+                   st);
+}

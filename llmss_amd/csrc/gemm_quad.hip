@@ -12,9 +12,11 @@
 // 8192 x 4096 x 11008 540 -> 530, 8192 x 11264 x 2048 379 -> 330; SwiGLU 8192 x 22016 x 4096 1237 (1195 TFLOP/s).
 //
 // GRP: grouped expert products over moe.hip's list of 256-row tiles, as in the ping-pong kernel: 1 - rows of X gathered through
-// order[] / top, activation or gating in the epilogue; 2 - rows in expert order, fp32 output. GLU: W's rows are gate and up in
-// alternating groups of 16.
+// order[] / top, activation or gating in the epilogue; 2 - rows in expert order, fp32 output; 3 - as 1 with GLU over two
+// matrices, gate and up, the products scaled by the pair's weight first. GLU: W's rows are gate and up in alternating groups of 16.
 #include "gemm_quad.h"
+
+#include <type_traits>
 
 template <int GRP, bool GLU>
 __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restrict__ X, int64_t ldx,
@@ -23,6 +25,7 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
                                                            int64_t ldy, int M, int N, int K, int act, int group_m, PpGroup gr) {
   // a ring of five buffers, each 64 of k (128 bytes, a line) of 256 rows: X of step 0, W of step 0, X of step 1, ...
   constexpr int BUF = 32768, NB = 5, QA = 6;
+  constexpr bool GATHER = GRP == 1 || GRP == 3;
   __shared__ __attribute__((aligned(16))) char smem[NB * BUF];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -38,6 +41,8 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
     n0 = (id - ty * ntn) * 256;
     m0 = gr.meta[1 + (gr.E + 1) + gr.maxt + ty];
     M = gr.meta[1 + e + 1];
+    // (rows 16 .. 31 of every 32 of a tile are up rows: a load takes eight rows, so a wave's loads are all of one matrix)
+    if (GRP == 3 && (w & 2)) W = gr.Wu;
     W += (int64_t)e * gr.sB;
   } else {
     const int tile = xcd_remap(blockIdx.x, ntn * ntm);
@@ -46,11 +51,11 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
     m0 = (grp * group_m + gidx % gm) * 256, n0 = (gidx / gm) * 256;
   }
   const int nk = K >> 6;
-  const uint64_t xbytes = (uint64_t)(M - m0) * (uint64_t)ldx * 2, wbytes = (uint64_t)(N - n0) * (uint64_t)ldw * 2;
+  const uint64_t xbytes = (uint64_t)(M - m0) * (uint64_t)ldx * 2, wbytes = (uint64_t)(GRP == 3 ? (N - n0) / 2 : N - n0) * (uint64_t)ldw * 2;
   const auto rx = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<char*>(reinterpret_cast<const char*>(X) + (GRP == 1 ? 0 : (int64_t)m0 * ldx * 2)), (short)0,
-      (int)(GRP == 1 || xbytes > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)xbytes), 0x00020000);
-  const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(W) + (int64_t)n0 * ldw * 2),
+      const_cast<char*>(reinterpret_cast<const char*>(X) + (GATHER ? 0 : (int64_t)m0 * ldx * 2)), (short)0,
+      (int)(GATHER || xbytes > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)xbytes), 0x00020000);
+  const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(W) + (int64_t)(GRP == 3 ? n0 / 2 : n0) * ldw * 2),
                                                     (short)0, (int)(wbytes > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)wbytes),
                                                     0x00020000);
   // chunk c of row r lies at place c ^ key(r) of the row: the eight rows that a fragment read's eight lanes take fall on eight
@@ -62,9 +67,10 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
   for (int i = 0; i < 8; ++i) {
     const int row = (i * 4 + w) * 8 + (lane >> 3);
     int xr = row;
-    if constexpr (GRP == 1) xr = gr.order[min(m0 + row, M - 1)] / gr.top;
+    if constexpr (GATHER) xr = gr.order[min(m0 + row, M - 1)] / gr.top;
     vx[i] = (uint32_t)xr * (uint32_t)(ldx * 2) + (uint32_t)(((lane & 7) ^ xkey(row)) << 4);
-    vw[i] = (uint32_t)row * (uint32_t)(ldw * 2) + (uint32_t)(((lane & 7) ^ wkey(row)) << 4);
+    const int wrw = GRP == 3 ? (row >> 5) * 16 + (row & 15) : row;
+    vw[i] = (uint32_t)wrw * (uint32_t)(ldw * 2) + (uint32_t)(((lane & 7) ^ wkey(row)) << 4);
   }
   // eight rows (1 KB) of step T_ of X or W into buffer B_
 #define Q_LOADX(I_, T_, B_)                                                                                           \
@@ -192,33 +198,40 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
         for (int e = 0; e < 8; ++e) o[e] = f2bf(v[e]);
         if (m < M && n < nmax) *reinterpret_cast<u16x8*>(Y + (int64_t)m * ldy + n) = o;
       };
-      float v[8];
-      if (GLU || act == 0) {
+      auto some = [&](auto kind) {
+#pragma unroll 2
+        for (int i = 0; i < 16; ++i) {
+          float v[8];
+          row(i, v);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = apply_act(v[e], kind());
+          out(i, v);
+        }
+      };
+      // (a loop for each function: with the choice inside, the unrolled code does not fit the instruction cache)
+      if (GLU || act == ACT_NONE) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
+          float v[8];
           row(i, v);
           out(i, v);
         }
-      } else {  // (one copy of the functions' code: unrolled it does not fit the instruction cache)
-#pragma unroll 1
-        for (int i = 0; i < 16; ++i) {
-          row(i, v);
-#pragma unroll 1
-          for (int h = 0; h < 2; ++h) {
-            f32x4 u = h ? f32x4{v[4], v[5], v[6], v[7]} : f32x4{v[0], v[1], v[2], v[3]};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) u[e] = apply_act(u[e], act);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              if (h) v[4 + e] = u[e];
-              else v[e] = u[e];
-            }
-          }
-          out(i, v);
-        }
+      } else if (act == ACT_GELU_TANH) {
+        some(std::integral_constant<int, ACT_GELU_TANH>());
+      } else if (act == ACT_GELU) {
+        some(std::integral_constant<int, ACT_GELU>());
+      } else if (act == ACT_RELU) {
+        some(std::integral_constant<int, ACT_RELU>());
+      } else {
+        some(std::integral_constant<int, ACT_RELU2>());
       }
     }
   };
+  float sw[8];
+  if constexpr (GRP == 3) {
+#pragma unroll
+    for (int mt = 0; mt < 8; ++mt) sw[mt] = gr.pw ? gr.pw[gr.order[min(m0 + wr * 128 + 16 * mt + li, M - 1)]] : 1.f;
+  }
   auto put = [&](int p, const f32x4 (&lo)[8], const f32x4 (&hi)[8]) {
     if constexpr (GLU) {
       const int n = n0 + wc * 128 + 32 * p + 4 * g;
@@ -232,7 +245,10 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
       for (int mt = 0; mt < 8; ++mt) {
         f32x4 v;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = silu(lo[mt][i] + bg[i]) * (hi[mt][i] + bu[i]);
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (GRP == 3) v[i] = glu_clamped_t(lo[mt][i] * sw[mt], hi[mt][i] * sw[mt], gr.limit, gr.alpha, gr.silu);
+          else v[i] = silu(lo[mt][i] + bg[i]) * (hi[mt][i] + bu[i]);
+        }
         *reinterpret_cast<f32x4*>(img + (16 * mt + li) * 256 + (((4 * p + g) ^ li) << 4)) = v;
       }
     } else {
@@ -264,6 +280,7 @@ void launch_gemm_quad(int grp, const bf16_t* X, int64_t ldx, const bf16_t* W, in
                       hipStream_t st) {
 #define LAUNCH_Q(G_, U_) gemm_quad_kernel<G_, U_><<<nwg, 256, 0, st>>>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, act, group_m, gr)
   if (grp == 2) LAUNCH_Q(2, false);
+  else if (grp == 3) LAUNCH_Q(3, true);
   else if (grp == 1 && glu) LAUNCH_Q(1, true);
   else if (grp == 1) LAUNCH_Q(1, false);
   else if (glu) LAUNCH_Q(0, true);

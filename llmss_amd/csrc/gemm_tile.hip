@@ -14,6 +14,7 @@
 // gelu(up), the error-function form) and DOWN (grouped: A = the activation rows,
 // fp32 output). The tile list and offsets are those moe_group writes (moe.hip).
 #include "anytype.h"
+#include "gemm_quad.h"
 
 #define GT_BK 64
 #define GT_LD 72  // bf16 per LDS row: 144 bytes, keeps ds_read_b128 rows 16-byte aligned and spreads the banks
@@ -37,13 +38,6 @@ struct GemmTileArgs {
   int ilv;          // GATE_UP: one weight matrix, gate and up rows in alternating groups of 16 (B the first gate row, B2 the first up row)
   const bf16_t* bias;  // PLAIN: [N] or null
 };
-
-__device__ __forceinline__ float glu_clamped_t(float g, float u, float limit, float alpha, int silu) {
-  if (silu) return g / (1.f + expf(-g)) * u;
-  g = fminf(g, limit);
-  u = fminf(fmaxf(u, -limit), limit);
-  return g / (1.f + expf(-alpha * g)) * (u + 1.f);
-}
 
 // 8 consecutive k of one row (zero beyond the row / k range)
 __device__ __forceinline__ u16x8 gt_load(const bf16_t* row, int k, int K, bool vec) {

@@ -1098,6 +1098,11 @@ def moe_router(h, router, corr, top, normalize=True, score="sigmoid", bias=None,
 
 
 _MOE_PP = os.environ.get("LLMSS_MOE_PP", "1") != "0"  # 0: grouped products on the tile kernel at every size (A/B runs)
+# (token, expert) pairs per expert from which the 256-row tiles are the faster ones, with gate and up in two matrices and else. All products
+# of a layer together, 32 experts of 2048 x 768, 16 of 1024 x 512 and 8 of 4096 x 2048, in us: interleaved, 128 pairs 161 -> 113, 62 -> 55,
+# 186 -> 163; no gate, 128 pairs 145 -> 105, 100 -> 72, 230 -> 174, 64 pairs 75 -> 105, 35 -> 68, 118 -> 164; two matrices, 128 pairs
+# 163 -> 124, 64 -> 68, 188 -> 178, 256 pairs 208 -> 206, 74 -> 71, 288 -> 183, 1024 pairs 605 -> 449, 166 -> 138, 739 -> 511.
+MOE_PP_ROWS_TWO, MOE_PP_ROWS = 256, 128
 
 
 def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=True, act="glu_clamp",
@@ -1133,10 +1138,14 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     P = T * top
     # rows per tile of the grouped GEMMs: 128 where the experts get enough rows to fill big tiles (bf16 only)
     rows = 128 if h.dtype == torch.bfloat16 and P >= 128 * E else 64
-    # ungated experts with still more rows each: the dense GEMMs' 256x256 ping-pong kernel
-    # (gated ones with their gate and up rows interleaved, the activation in the epilogue)
-    pp = (gate is None and h.dtype == torch.bfloat16 and P >= 384 * E and min(F, N) >= 256 and F % 8 == 0 and K % 8 == 0
-          and h.stride(0) % 8 == 0 and not weight_input and h.data_ptr() % 16 == 0 and _MOE_PP)
+    # experts with still more rows each: the dense GEMMs' 256 x 256 tiles; gate and up in one matrix (interleaved) or in two
+    pp = (h.dtype == torch.bfloat16 and P >= (MOE_PP_ROWS if gate is None else MOE_PP_ROWS_TWO) * E and min(F, N) >= 256 and F % 8 == 0 and K % 8 == 0
+          and h.stride(0) % 8 == 0 and h.data_ptr() % 16 == 0 and _MOE_PP)
+    if gate is not None:
+        pp = pp and lib().moe_pp_glu_ok(h.stride(0), -(-P // 256) + min(E, P), top, F, K) and \
+            not (gate.data_ptr() | up.data_ptr() | down.data_ptr()) & 15
+    elif weight_input:
+        pp = False
     if pp:
         rows = 256
     maxt = -(-P // rows) + min(E, P)
@@ -1154,8 +1163,12 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     st = _stream()
     L.moe_group(idx.data_ptr(), P, E, maxt, meta.data_ptr(), order.data_ptr(), place.data_ptr(), rows, st)
     if pp:
-        L.moe_pp(3 if interleaved else 1, h.data_ptr(), h.stride(0), up.data_ptr(), meta.data_ptr(), order.data_ptr(),
-                 act_.data_ptr(), E, maxt, top, UF, K, 0 if interleaved else _ACT["gelu"], st)
+        if gate is not None:
+            L.moe_pp_glu(h.data_ptr(), h.stride(0), gate.data_ptr(), up.data_ptr(), meta.data_ptr(), order.data_ptr(),
+                         act_.data_ptr(), E, maxt, top, F, K, float(limit), float(alpha), pw, silu, st)
+        else:
+            L.moe_pp(3 if interleaved else 1, h.data_ptr(), h.stride(0), up.data_ptr(), meta.data_ptr(), order.data_ptr(),
+                     act_.data_ptr(), E, maxt, top, UF, K, 0 if interleaved else _ACT["gelu"], st)
         L.moe_pp(2, act_.data_ptr(), F, down.data_ptr(), meta.data_ptr(), order.data_ptr(), y.data_ptr(), E, maxt, 1, N, F,
                  0, st)
     elif h.dtype == torch.bfloat16:  # matrix cores (csrc/gemm_tile.hip)
