@@ -349,11 +349,101 @@ __global__ __launch_bounds__(512) void token_side_add_kernel(SandwichArgs p, Sid
   norm_out<T, V>(xs, ss2, p, t, red);
 }
 
+// The token input of a few bf16 rows, up to 2048 wide (NW: at least W / 256): the kernel above with everything that a row needs asked for
+// at the start - a wave its gate rows, a thread the projection's rows of its four columns - since a decode step is nothing but the
+// chain of its loads: 24 -> 15 us for 33 rows
+// of 2048 in a decode step. A CU holds one workgroup: up to 256 rows (12.6 us), at 1006 it takes 43 us and the kernel above 26.
+template <int D, int NW>
+__global__ __launch_bounds__(512) void token_side_row_kernel(SandwichArgs p, SideArgs s) {
+  constexpr int R = D / 8;  // gate rows of a wave
+  __shared__ __attribute__((aligned(16))) float xs[NW * 256];
+  __shared__ __attribute__((aligned(16))) float gs[D];
+  __shared__ float red[32];
+  const int t = blockIdx.x, W = p.W, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, c = threadIdx.x * 4;
+  const bool live = c < W;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  float* xr = p.x + (int64_t)t * W;
+  f32x4 xv = live ? *reinterpret_cast<const f32x4*>(xr + c) : zero;
+  int64_t id = s.ids[t];
+  u16x4 wg[R][NW];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int k = 0; k < NW; ++k)
+      if (k * 256 < W) wg[r][k] = *reinterpret_cast<const u16x4*>((const bf16_t*)s.wg + (int64_t)(wv * R + r) * W + k * 256 + lane * 4);
+  u16x8 wp[4][D / 8];
+  auto load_wp = [&]() {
+    if (live) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < D / 8; ++j) wp[i][j] = *reinterpret_cast<const u16x8*>((const bf16_t*)s.wp + (int64_t)(c + i) * D + 8 * j);
+    }
+  };
+  if constexpr (D == 32) load_wp();  // (the deeper form's registers hold one of the two at a time)
+  const f32x4 wn = live ? *reinterpret_cast<const f32x4*>(s.wn + c) : zero;
+  const f32x4 wx = live && p.wnext ? *reinterpret_cast<const f32x4*>(p.wnext + c) : zero;
+  const f32x4 ad = live && p.add ? *reinterpret_cast<const f32x4*>(p.add + (int64_t)t * W + c) : zero;
+  id = id < 0 ? 0 : (id >= s.vocab ? s.vocab - 1 : id);
+  const float er = lane < R ? bf2f(((const bf16_t*)s.table)[id * s.ldt + s.col0 + wv * R + lane]) : 0.f;
+  if (live) *reinterpret_cast<f32x4*>(xs + c) = xv;
+  __syncthreads();
+  float a[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) a[r] = 0.f;
+#pragma unroll
+  for (int k = 0; k < NW; ++k)
+    if (k * 256 < W) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(xs + k * 256 + lane * 4);
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[r] = fmaf(bf2f(wg[r][k][i]), v[i], a[r]);
+    }
+  if constexpr (D != 32) load_wp();
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    a[r] = warp_sum(a[r]);
+    if (lane == r) gs[wv * R + r] = gelu_tanh_f(a[r]) * er;
+  }
+  __syncthreads();
+  f32x4 y = zero;
+  if (live) {
+#pragma unroll
+    for (int j = 0; j < D / 8; ++j) {
+      const f32x4 g0 = *reinterpret_cast<const f32x4*>(gs + 8 * j), g1 = *reinterpret_cast<const f32x4*>(gs + 8 * j + 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          y[i] = fmaf(bf2f(wp[i][j][e]), g0[e], y[i]);
+          y[i] = fmaf(bf2f(wp[i][j][4 + e]), g1[e], y[i]);
+        }
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ss = fmaf(y[i], y[i], ss);
+  const float inv = 1.0f / sqrtf(block_sum(ss, red) / (float)W + p.eps);
+  float ss2 = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    xv[i] = fmaf(y[i] * inv, wn[i], xv[i]);
+    if (p.add) xv[i] += ad[i];
+    ss2 = fmaf(xv[i], xv[i], ss2);
+  }
+  if (live) *reinterpret_cast<f32x4*>(xr + c) = xv;
+  if (!p.wnext) return;
+  const float invx = 1.0f / sqrtf(block_sum(ss2, red) / (float)W + p.eps);
+  if (live)
+    *reinterpret_cast<u16x4*>((bf16_t*)p.h + (int64_t)t * p.ldh + c) =
+        u16x4{f2bf(xv[0] * invx * wx[0]), f2bf(xv[1] * invx * wx[1]), f2bf(xv[2] * invx * wx[2]), f2bf(xv[3] * invx * wx[3])};
+}
+
 // The token input for bf16 weights, 16 rows per workgroup on the matrix cores (the kernel above reads both small matrices from L2
 // for every row: 2 GB per prompt step
 // of 8192 rows at width 2048, 189 us; 52 us here, of which 27 are the bytes of x and h: a workgroup is a chain of two products and
-// two norms of 25 us, so below 1024 rows, where the chip is not filled twice, the kernel above is the faster one: 13 us at 64 rows,
-// 26 on both at 1006). Wave w takes an eighth of the width. First product:
+// two norms of 25 us, so below 1024 rows, where the chip is not filled twice, the kernels above are the faster ones). Wave w takes an eighth of the width. First product:
 // the fp32 rows enter as three bf16 numbers that add up to them exactly, the weights are exact, the waves' sums meet in LDS.
 // Second: the weights' rows are the first operand, so that a lane holds four neighbouring columns of one row - 16-byte accesses
 // of x, 8-byte ones of h - and the projected row, then the new x, stay in registers between the norms.
@@ -513,6 +603,14 @@ void launch_token_side_add(void* x, const void* ids, const void* table, int64_t 
     if (d == 32) LAUNCH_SIDE(2);
     else LAUNCH_SIDE(4);
 #undef LAUNCH_SIDE
+    HIP_CHECK_LAUNCH();
+    return;
+  }
+  if (dt == 0 && vec && T_ <= 256 && (d == 32 || d == 64) && W % 256 == 0 && W <= 2048 && al16(wp)) {
+    if (d == 32 && W <= 1024) token_side_row_kernel<32, 4><<<T_, 512, 0, st>>>(p, s);
+    else if (d == 32) token_side_row_kernel<32, 8><<<T_, 512, 0, st>>>(p, s);
+    else if (W <= 1024) token_side_row_kernel<64, 4><<<T_, 512, 0, st>>>(p, s);
+    else token_side_row_kernel<64, 8><<<T_, 512, 0, st>>>(p, s);
     HIP_CHECK_LAUNCH();
     return;
   }

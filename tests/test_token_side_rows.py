@@ -7,7 +7,10 @@ from llmss_amd import ops
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("T,W,d,add,nxt", [(1024, 256, 32, False, True), (1025, 1024, 32, True, True), (1039, 2048, 64, True, False),
+# (below 1024 rows, and up to 2048 wide: a row per workgroup with its weights in registers)
+@pytest.mark.parametrize("T,W,d,add,nxt", [(1, 256, 64, True, True), (3, 1024, 32, False, True), (33, 1280, 32, True, False),
+                                           (2, 2048, 64, True, True), (5, 2048, 32, False, True), (2, 1024, 64, False, True),
+                                           (2, 2304, 32, False, True), (1024, 256, 32, False, True), (1025, 1024, 32, True, True), (1039, 2048, 64, True, False),
                                            (1040, 2304, 32, False, True), (1100, 4096, 64, True, True), (1024, 4352, 32, False, True),
                                            (1023, 2048, 32, True, True), (1030, 2000, 32, False, True)])
 def test_token_side_rows(T, W, d, add, nxt):
