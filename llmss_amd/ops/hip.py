@@ -1103,6 +1103,8 @@ _MOE_PP = os.environ.get("LLMSS_MOE_PP", "1") != "0"  # 0: grouped products on t
 # 186 -> 163; no gate, 128 pairs 145 -> 105, 100 -> 72, 230 -> 174, 64 pairs 75 -> 105, 35 -> 68, 118 -> 164; two matrices, 128 pairs
 # 163 -> 124, 64 -> 68, 188 -> 178, 256 pairs 208 -> 206, 74 -> 71, 288 -> 183, 1024 pairs 605 -> 449, 166 -> 138, 739 -> 511.
 MOE_PP_ROWS_TWO, MOE_PP_ROWS = 256, 128
+# And up to which those of 16 rows are: the same three layers gain 1.05 - 1.4 at 4 pairs, 1.0 - 1.5 at 8, 0.8 - 1.3 at 16, 0.65 - 1.1 at 24.
+MOE_DEC_ROWS = 8
 
 
 def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=True, act="glu_clamp",
@@ -1139,15 +1141,21 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     # rows per tile of the grouped GEMMs: 128 where the experts get enough rows to fill big tiles (bf16 only)
     rows = 128 if h.dtype == torch.bfloat16 and P >= 128 * E else 64
     # experts with still more rows each: the dense GEMMs' 256 x 256 tiles; gate and up in one matrix (interleaved) or in two
-    pp = (h.dtype == torch.bfloat16 and P >= (MOE_PP_ROWS if gate is None else MOE_PP_ROWS_TWO) * E and min(F, N) >= 256 and F % 8 == 0 and K % 8 == 0
-          and h.stride(0) % 8 == 0 and h.data_ptr() % 16 == 0 and _MOE_PP)
+    pp = (h.dtype == torch.bfloat16 and P >= (MOE_PP_ROWS if gate is None else MOE_PP_ROWS_TWO) * E
+          and min(F, N) >= 256 and F % 8 == 0 and K % 8 == 0 and h.stride(0) % 8 == 0 and h.data_ptr() % 16 == 0 and _MOE_PP)
     if gate is not None:
         pp = pp and lib().moe_pp_glu_ok(h.stride(0), -(-P // 256) + min(E, P), top, F, K) and \
             not (gate.data_ptr() | up.data_ptr() | down.data_ptr()) & 15
     elif weight_input:
         pp = False
+    # and those with a few rows each: weights straight into the matrix instructions' operands
+    aligned = h.data_ptr() | up.data_ptr() | down.data_ptr() | (0 if gate is None else gate.data_ptr())
+    dec = (h.dtype == torch.bfloat16 and P <= MOE_DEC_ROWS * E and K % 32 == 0 and F % 32 == 0 and h.stride(0) % 8 == 0
+           and not aligned & 15 and not pp)
     if pp:
         rows = 256
+    if dec:
+        rows = 16
     maxt = -(-P // rows) + min(E, P)
     _check(maxt <= 65535, "too many (token, expert) pairs in one step")
     dev = h.device
@@ -1171,6 +1179,12 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
                      act_.data_ptr(), E, maxt, top, UF, K, 0 if interleaved else _ACT["gelu"], st)
         L.moe_pp(2, act_.data_ptr(), F, down.data_ptr(), meta.data_ptr(), order.data_ptr(), y.data_ptr(), E, maxt, 1, N, F,
                  0, st)
+    elif dec:
+        L.moe_dec(1 if act == "gelu" else 0, h.data_ptr(), h.stride(0), up.data_ptr() if gate is None else gate.data_ptr(),
+                  0 if gate is None else up.data_ptr(), meta.data_ptr(), order.data_ptr(), act_.data_ptr(), E, maxt, top, F, K,
+                  float(limit), float(alpha), pw, silu, st)
+        L.moe_dec(2, act_.data_ptr(), F, down.data_ptr(), 0, meta.data_ptr(), order.data_ptr(), y.data_ptr(), E, maxt, 1, N, F,
+                  0.0, 0.0, 0, 0, st)
     elif h.dtype == torch.bfloat16:  # matrix cores (csrc/gemm_tile.hip)
         L.moe_gate_up_tile(h.data_ptr(), h.stride(0), up.data_ptr() if interleaved else _ptr(gate), up.data_ptr(),
                            meta.data_ptr(), order.data_ptr(), act_.data_ptr(), E, maxt, top, F, K, float(limit), float(alpha),
