@@ -586,6 +586,55 @@ __global__ __launch_bounds__(256) void gated_group_norm_kernel(const float* __re
     El<T>::st(dst + i, row[i] * inv * El<T>::ld(wr + i) * gate_of(i));
 }
 
+// The same for groups of more than 512 and up to 4096 columns: four an access, a group's numbers in registers between the sum of squares
+// and the result (NC times 1024 columns), the gate evaluated once. 8192 rows of 4096, bf16: 106 -> 47 us (5.7 TB/s).
+template <typename T, int NC>
+__global__ __launch_bounds__(256) void gated_group_norm_rows_kernel(const float* __restrict__ o, int64_t ldo,
+                                                                    const T* __restrict__ gate, int64_t ldg,
+                                                                    const T* __restrict__ w, float eps, int act, float c,
+                                                                    T* __restrict__ out, int64_t ldout, int n, int wfull,
+                                                                    int first, const float* __restrict__ den,
+                                                                    const f32x4* __restrict__ gates, float qs) {
+  __shared__ float red[32];
+  const int t = blockIdx.x, g = blockIdx.y;
+  const float* row = o + (int64_t)t * ldo + (int64_t)g * n;
+  const T* gr = gate + (int64_t)t * ldg + (int64_t)g * n;
+  const T* wr = wfull ? w + (int64_t)g * n : w;
+  f32x4 u[NC], a[NC], wv[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int col = 4 * (threadIdx.x + 256 * i);
+    u[i] = a[i] = wv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (col < n) u[i] = ld4(row + col), a[i] = ld4(gr + col), wv[i] = ld4(wr + col);
+  }
+  float pre = 1.0f;
+  if (den) {
+    const int64_t e = (int64_t)t * gridDim.y + g;
+    pre = qs / (fmaxf(fabsf(qs * den[e]), expf(-gates[e][2])) + 1e-6f);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NC; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float sg = 1.0f / (1.0f + expf(-a[i][e]));
+      a[i][e] = act ? a[i][e] * sg : sg;
+      const float v = (first ? u[i][e] * a[i][e] : u[i][e]) * pre;
+      ss = fmaf(v, v, ss);
+    }
+  ss = block_sum(ss, red);
+  const float inv = pre * c / sqrtf(ss / (float)n + eps);
+  T* dst = out + (int64_t)t * ldout + (int64_t)g * n;
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int col = 4 * (threadIdx.x + 256 * i);
+    f32x4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = u[i][e] * inv * wv[i][e] * a[i][e];
+    if (col < n) st4(dst + col, r);
+  }
+}
+
 // The same, the gate after the norm, for groups of 8 to 512 columns that are a power of two: L = n / 8 neighbouring lanes share
 // a group, eight columns each in 16-byte accesses; the numbers stay in registers between the sum of squares and the result.
 template <typename T>
@@ -646,6 +695,21 @@ void launch_gated_group_norm(const void* o, int64_t ldo, const void* gate, int64
     DISPATCH_T(dt, T, (gated_group_norm_vec_kernel<T><<<gv, 256, 0, st>>>(
         (const float*)o, ldo, (const T*)gate, ldg, (const T*)w, eps, act, c, (T*)out, ldout, n, wfull,
         (const float*)den, (const f32x4*)gates, qs, groups, T_)));
+    HIP_CHECK_LAUNCH();
+    return;
+  }
+  if (n > 512 && n <= 4096 && n % 4 == 0 && ldo % 4 == 0 && ldg % 4 == 0 && ldout % 4 == 0 && al(o, 16) && al(gate, 4 * es) &&
+      al(w, 4 * es) && al(out, 4 * es)) {
+#define LAUNCH_GGN(NC_)                                                                                                       \
+  gated_group_norm_rows_kernel<T, NC_><<<dim3(T_, groups), 256, 0, st>>>((const float*)o, ldo, (const T*)gate, ldg, (const T*)w, \
+                                                                         eps, act, c, (T*)out, ldout, n, wfull, first,        \
+                                                                         (const float*)den, (const f32x4*)gates, qs)
+    DISPATCH_T(dt, T, {
+      if (n <= 1024) LAUNCH_GGN(1);
+      else if (n <= 2048) LAUNCH_GGN(2);
+      else LAUNCH_GGN(4);
+    });
+#undef LAUNCH_GGN
     HIP_CHECK_LAUNCH();
     return;
   }

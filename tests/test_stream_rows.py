@@ -55,3 +55,25 @@ def test_glu_act(T, F, act, dtype):
     # two units of the product where the tanh form is taken, for 1 + tanh near -1
     lim = (8 + 4 * z.abs()) * 2.0 ** -24 * want.abs() + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0.0) + 2 * 2.0 ** -24 * (a * u).abs() * (act == "gelu_tanh") + 1e-36
     assert ((got - want).abs() <= lim).all()
+
+
+# groups on both sides of 512 and 4096 and at the edges of 1024 and 2048; the gate before the norm and after
+@pytest.mark.parametrize("T,groups,n", [(3, 2, 516), (2, 1, 1024), (1, 3, 1028), (2, 1, 2048), (3, 1, 2052), (2, 2, 4096), (2, 1, 4100),
+                                        (2, 1, 770)])
+@pytest.mark.parametrize("act,first", [("silu", True), ("silu", False), ("sigmoid", False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_gated_group_norm(T, groups, n, act, first, dtype):
+    from llmss_amd.ops import hip
+    g = torch.Generator().manual_seed(n + T)
+    o = torch.randn(T, groups * n, generator=g).cuda() * 3
+    gate = torch.randn(T, groups * n + 4, generator=g).to(dtype).cuda()[:, 4:]
+    w = (1 + 0.1 * torch.randn(groups * n, generator=g)).to(dtype).cuda()
+    got = hip.gated_group_norm(o, gate, w, 1e-5, act, 0.9, out_dtype=dtype, groups=groups, gate_first=first).double()
+    z = gate.double()
+    a = torch.sigmoid(z) * (z if act == "silu" else 1)
+    u = (o.double() * a if first else o.double()).view(T, groups, n)
+    want = (0.9 * u / torch.sqrt(u.pow(2).mean(-1, keepdim=True) + 1e-5)).view(T, -1) * w.double() * (1 if first else a)
+    # the gate's exponential and quotient (8 + |z| units), the norm (sum of squares in any order: n / 2 units at most of ss, in practice
+    # steps of 16 and a tree of 8), 8 products; bf16 results one rounding
+    lim = (32 + 2 * z.abs()) * 2.0 ** -24 * want.abs() + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0.0) + 1e-30
+    assert ((got - want).abs() <= lim).all()
