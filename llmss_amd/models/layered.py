@@ -740,7 +740,8 @@ class LayeredLM:
                 self.tap(i - 1, x.sum(0))
             if canon:
                 tail = self.canon_tail[i] if cfg.canon_taps > 1 else None
-                h = ops.causal_conv(h, L.canon, tail, cu, inp.ctx_lens, inp.state_slots, True, False, dt)
+                h = ops.causal_conv(h, L.canon, tail, cu, inp.ctx_lens, inp.state_slots, True, False, dt,
+                                    single=inp.kind == "decode")
             y, prev = MIXERS[spec.mixer.kind].forward(self, i, L.mix, spec.mixer, h, inp, cu, kv_caches), L.hc1
             if spec.mlp is not None:
                 h = ops.stream_add_norm(x, y, prev.mix, prev.outw, c, L.hc2.inw, L.norm2, eps, rms, dt)
@@ -787,7 +788,8 @@ class LayeredLM:
                 if canon is None:
                     return x.to(dt)
                 tail = self.canon_tail[nsub * i + k] if cfg.canon_taps > 1 else None
-                return ops.causal_conv(x, canon, tail, cu, inp.ctx_lens, inp.state_slots, True, False, dt)
+                return ops.causal_conv(x, canon, tail, cu, inp.ctx_lens, inp.state_slots, True, False, dt,
+                                       single=inp.kind == "decode")
             y = MIXERS[spec.mixer.kind].forward(self, i, Lw.mix, spec.mixer, read(Lw.canon1, 0), inp, cu, kv_caches)
             last = spec.mlp is None
             x = ops.resid_norm_add(hist, n, y, Lw.norm1, eps, Lw.dwa if last and dwa else None)
