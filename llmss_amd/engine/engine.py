@@ -830,13 +830,10 @@ class LLMEngine:
         modes = self._decode_modes()
         # warm-up passes (lazy allocations, first launches). Native RCCL: with real collectives, so each
         # algorithm's lazy peer connection happens here and not inside the capture. torch's RCCL process
-        # group: collectives suspended - its watchdog thread would otherwise still track the warm-up's work
-        # items when the capture starts, and a watchdog query of their end events (recorded on the
-        # communicator's stream, which the captured collectives pull into the capture) aborts the process
-        torch_pg = self.tp.is_real and self.tp.comm is None and not self.tp.host_staged
+        # group: collectives suspended, and those issued before (this engine's agreements, earlier steps) waited for below
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(s), (self.tp.suspended() if torch_pg else contextlib.nullcontext()):
+        with torch.cuda.stream(s), (self.tp.suspended() if self.tp.torch_pg else contextlib.nullcontext()):
             for b in reversed(self.buckets):
                 for d in modes:
                     for _ in range(2):
@@ -846,6 +843,7 @@ class LLMEngine:
         # settle the caching allocator's pending cross-stream events (freed side-stream blocks) outside the
         # capture, so no allocation during capture queries an event
         torch.cuda.empty_cache()
+        self.tp.settle()
         # thread-local capture: the RCCL communicator's watchdog thread keeps querying the events of earlier
         # collectives; under the default global capture mode such a query from another thread aborts the
         # process ("operation not permitted when stream is capturing")
@@ -932,6 +930,7 @@ class LLMEngine:
             torch.cuda.synchronize()
 
         def capture_all(triples):
+            self.tp.settle()  # the warm-up's collectives and the agreement on it
             for b, d, name in triples:
                 with self._schedule(b, name):
                     g = torch.cuda.CUDAGraph()

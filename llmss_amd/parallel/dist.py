@@ -113,6 +113,25 @@ class TPGroup:
         return st
 
     @property
+    def torch_pg(self) -> bool:
+        """Collectives go through torch's nccl process group, whose watchdog thread tracks every eager one."""
+        return self.is_real and self.comm is None and not self.host_staged
+
+    def settle(self):
+        """Return once torch's watchdog thread tracks no collective of this process any more (torch process-group mode;
+        nothing to do otherwise). To be called right before a graph capture with collectives inside: the watchdog queries
+        the end events of the collectives on its list every 100 ms, those of finished ones too until its next pass, and a
+        query of an event of the communicator's stream while the capture holds that stream ends the process
+        (hipErrorCapturedEvent raised in the watchdog thread). Captured collectives are not put on the list."""
+        if not self.torch_pg:
+            return
+        torch.cuda.synchronize()
+        groups = [self.group, dist.group.WORLD]
+        for i, g in enumerate(groups):
+            if g is not None and g not in groups[:i] and dist.get_backend(g) == "nccl":
+                g._wait_for_pending_works()
+
+    @property
     def backend(self) -> str:
         """'rccl-native' | 'nccl' (torch's RCCL process group) | 'gloo' | 'local' | 'fake'."""
         if self.fake:

@@ -1,5 +1,7 @@
 """End-to-end model/engine checks on the GPU: HIP forward vs the CPU fp32 reference forward,
 HIP-graph decode vs eager decode, and continuous batching determinism."""
+import gc
+
 import pytest
 import torch
 
@@ -9,6 +11,19 @@ from llmss_amd.models.decoder import DecoderLM, StepInput
 from llmss_amd.models.weights import random_weights
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def nccl_world():
+    """A one-member torch nccl process group for this file's tests; destroyed with its watchdog thread after the last of them."""
+    import torch.distributed as dist
+
+    assert not dist.is_initialized()
+    dist.init_process_group("nccl", store=dist.HashStore(), rank=0, world_size=1, device_id=torch.device("cuda", 0))
+    yield
+    gc.collect()  # graphs that hold captured collectives go before their communicator
+    torch.cuda.synchronize()
+    dist.destroy_process_group()
 
 
 def _to_gpu(w):
@@ -123,20 +138,14 @@ def test_engine_graph_vs_eager_and_batching():
     assert a == b
 
 
-def test_tp_allreduce_overlap_streams():
+def test_tp_allreduce_overlap_streams(nccl_world):
     """Row-chunked all-reduce on the comm stream (RCCL) overlapped with the next chunk's GEMMs must give
     the same hidden states as one all-reduce. A one-member RCCL group makes the collective the
     identity, so the multi-stream path runs for real on a single GPU."""
-    import os
-
     import torch.distributed as dist
 
     from llmss_amd.parallel.dist import TPGroup
 
-    if not dist.is_initialized():
-        os.environ.setdefault("MASTER_ADDR", "127.0.0.1")
-        os.environ.setdefault("MASTER_PORT", "29533")
-        dist.init_process_group("nccl", rank=0, world_size=1, device_id=torch.device("cuda", 0))
     tp = TPGroup(0, 2, group=dist.group.WORLD)  # rank-0 shard of a TP=2 plan, "real" communicator
     assert tp.is_real
     for fam, par in (("tiny-llama", False), ("tiny-gptj", True)):
@@ -161,22 +170,15 @@ def test_tp_allreduce_overlap_streams():
         assert err < 5e-2, err
 
 
-def test_rccl_collectives_inside_decode_graphs():
+def test_rccl_collectives_inside_decode_graphs(nccl_world):
     """Capture smoke test (torch process-group mode, LLMSS_COMM=torch): the TP decode step with its
     all-reduces + all-gather through torch's RCCL process group captures into HIP graphs and replays ==
     eager. The communicator has ONE member, so its in-place all-reduces move no data and need not leave a
     node in the graph: this proves capture works, not that a multi-rank collective is in the graph (that is
     measured by bench.py's comm probe on the driver's multi-GPU node)."""
-    import os
-
     import torch.distributed as dist
 
     from llmss_amd.parallel.dist import TPGroup
-
-    if not dist.is_initialized():
-        os.environ.setdefault("MASTER_ADDR", "127.0.0.1")
-        os.environ.setdefault("MASTER_PORT", "29533")
-        dist.init_process_group("nccl", rank=0, world_size=1, device_id=torch.device("cuda", 0))
 
     class OneMemberTP(TPGroup):  # TP=2 shard plan over a 1-rank communicator (collectives run, sum = identity)
         def all_gather_last_dim(self, t):
@@ -198,26 +200,19 @@ def test_rccl_collectives_inside_decode_graphs():
     assert e_eager.generate(prompts, sp) == out_g
 
 
-@pytest.mark.skip(reason="aborted the test process once in eight runs of the GPU tests: torch's process-group watchdog "
-                         "queried an event 'last recorded in a capturing stream' (hipErrorCapturedEvent) while this "
-                         "loop captured collectives; no cause shown in this package's code, so the loop stays off the "
-                         "GPU (the engine's own captures with collectives are covered by the tests around this one)")
-def test_graph_capture_while_rccl_watchdog_polls():
+@pytest.mark.skip(reason="captures a collective right behind eager ones without the wait for the process group's watchdog that "
+                         "the engine's captures have (TPGroup.settle): the watchdog may query an event of the stream that the "
+                         "capture holds (hipErrorCapturedEvent), which ended the test process in one of eight runs")
+def test_graph_capture_while_rccl_watchdog_polls(nccl_world):
     """Capture smoke regression (torch process-group mode): with the RCCL process group's watchdog thread
     tracking earlier collectives, a capture in torch's default (global) mode aborted the process when the
     watchdog queried an event mid-capture ("operation not permitted when stream is capturing"). Engine and
     autotuner capture thread-locally. One member: the captured in-place all-reduce is empty (HIP warns
     "The CUDA Graph is empty"); the test is about the watchdog, not the collective."""
-    import os
-
     import torch.distributed as dist
 
     from llmss_amd.ops import autotune as A
 
-    if not dist.is_initialized():
-        os.environ.setdefault("MASTER_ADDR", "127.0.0.1")
-        os.environ.setdefault("MASTER_PORT", "29533")
-        dist.init_process_group("nccl", rank=0, world_size=1, device_id=torch.device("cuda", 0))
     t = torch.ones(1 << 16, device="cuda")
     for i in range(60):
         for _ in range(4):  # eager collectives: work items the watchdog polls
@@ -228,16 +223,9 @@ def test_graph_capture_while_rccl_watchdog_polls():
 
 
 def _one_member_tp():
-    import os
-
     import torch.distributed as dist
 
     from llmss_amd.parallel.dist import TPGroup
-
-    if not dist.is_initialized():
-        os.environ.setdefault("MASTER_ADDR", "127.0.0.1")
-        os.environ.setdefault("MASTER_PORT", "29533")
-        dist.init_process_group("nccl", rank=0, world_size=1, device_id=torch.device("cuda", 0))
 
     class OneMemberTP(TPGroup):  # TP=2 shard plan over a 1-rank communicator (collectives run, sum = identity)
         def all_gather_last_dim(self, t):
@@ -249,7 +237,7 @@ def _one_member_tp():
 
 
 @pytest.mark.parametrize("fam", ["tiny-llama", "tiny-gptj"])
-def test_decode_microbatch_overlap(fam):
+def test_decode_microbatch_overlap(fam, nccl_world):
     """Two-micro-batch decode (each half's RCCL all-reduces on the comm stream while the other half
     computes) == the single-batch decode step, for sequential (Llama) and parallel (GPT-J) blocks."""
     tp = _one_member_tp()
@@ -281,7 +269,7 @@ def test_decode_microbatch_overlap(fam):
 
 
 @pytest.mark.parametrize("fam", ["tiny-llama", "tiny-gptj"])
-def test_prefill_microbatch_overlap(fam):
+def test_prefill_microbatch_overlap(fam, nccl_world):
     """Prefill split into two micro-batches at a sequence boundary (each half's RCCL all-reduces on the comm
     stream while the other half computes) == the single prefill step: hidden states and the paged KV."""
     tp = _one_member_tp()
@@ -309,7 +297,7 @@ def test_prefill_microbatch_overlap(fam):
         assert (ka.float() - kb.float()).abs().max().item() < 5e-2 and (va.float() - vb.float()).abs().max() < 5e-2
 
 
-def test_decode_microbatch_overlap_in_graphs():
+def test_decode_microbatch_overlap_in_graphs(nccl_world):
     """The micro-batch decode schedule (two streams, event joins, RCCL) captures into HIP graphs and
     replays exactly like eager; also with the modelled-comm fake group used by bench --sim-comm."""
     from llmss_amd.parallel.dist import TPGroup
