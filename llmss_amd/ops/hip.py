@@ -1140,18 +1140,17 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     P = T * top
     # rows per tile of the grouped GEMMs: 128 where the experts get enough rows to fill big tiles (bf16 only)
     rows = 128 if h.dtype == torch.bfloat16 and P >= 128 * E else 64
+    # (both forms below load the weights in pieces of 16 bytes; the tile kernel takes any place)
+    aligned = not (h.data_ptr() | up.data_ptr() | down.data_ptr() | _ptr(gate)) & 15 and h.stride(0) % 8 == 0
     # experts with still more rows each: the dense GEMMs' 256 x 256 tiles; gate and up in one matrix (interleaved) or in two
     pp = (h.dtype == torch.bfloat16 and P >= (MOE_PP_ROWS if gate is None else MOE_PP_ROWS_TWO) * E
-          and min(F, N) >= 256 and F % 8 == 0 and K % 8 == 0 and h.stride(0) % 8 == 0 and h.data_ptr() % 16 == 0 and _MOE_PP)
+          and min(F, N) >= 256 and F % 8 == 0 and K % 8 == 0 and aligned and _MOE_PP)
     if gate is not None:
-        pp = pp and lib().moe_pp_glu_ok(h.stride(0), -(-P // 256) + min(E, P), top, F, K) and \
-            not (gate.data_ptr() | up.data_ptr() | down.data_ptr()) & 15
+        pp = pp and lib().moe_pp_glu_ok(h.stride(0), -(-P // 256) + min(E, P), top, F, K)
     elif weight_input:
         pp = False
     # and those with a few rows each: weights straight into the matrix instructions' operands
-    aligned = h.data_ptr() | up.data_ptr() | down.data_ptr() | (0 if gate is None else gate.data_ptr())
-    dec = (h.dtype == torch.bfloat16 and P <= MOE_DEC_ROWS * E and K % 32 == 0 and F % 32 == 0 and h.stride(0) % 8 == 0
-           and not aligned & 15 and not pp)
+    dec = h.dtype == torch.bfloat16 and P <= MOE_DEC_ROWS * E and K % 32 == 0 and F % 32 == 0 and aligned and not pp
     if pp:
         rows = 256
     if dec:
