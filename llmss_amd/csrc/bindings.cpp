@@ -57,8 +57,8 @@ int launch_gemm_f8f8(const void* xq, int64_t ldx, const void* xs, const void* wq
                      int depth, int split, void* workspace, int64_t ws_bytes, hipStream_t st, bool partial_out,
                      bool ilv, void* mxq, void* mxs, const void* asc);
 int gemm_f8f8_partial_slabs(int M, int N, int K, bool glu, int act, int tile, int split, int64_t ws_bytes);
-int gemm_partial_slabs(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint,
-                       int64_t ws_bytes);
+int gemm_partial_slabs(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint, int64_t ws_bytes,
+                       const void* x, int64_t ldx, const void* w, int64_t ldw);
 void attn_decode_set_unroll(int u);
 void launch_comm_model(void* buf, int channels, int64_t nbytes, double us, hipStream_t st);
 int64_t comm_model_slice(int channels, int64_t nbytes);
@@ -361,7 +361,12 @@ PYBIND11_MODULE(_C, m) {
      pybind11::arg("st"), pybind11::arg("partial_out") = false, pybind11::arg("ilv") = false,
      pybind11::arg("mxq") = 0, pybind11::arg("mxs") = 0, pybind11::arg("asc") = 0);
   m.def("gemm_f8f8_partial_slabs", &gemm_f8f8_partial_slabs);
-  m.def("gemm_partial_slabs", &gemm_partial_slabs);
+  m.def("gemm_partial_slabs", [](int M, int N, int K, bool fp8, bool glu, int act, int nt_hint, int split_hint, int64_t ws_bytes,
+                                 uintptr_t x, int64_t ldx, uintptr_t w, int64_t ldw) {
+    return gemm_partial_slabs(M, N, K, fp8, glu, act, nt_hint, split_hint, ws_bytes, CP(x), ldx, CP(w), ldw);
+  }, pybind11::arg(), pybind11::arg(), pybind11::arg(), pybind11::arg(), pybind11::arg(), pybind11::arg(), pybind11::arg(),
+     pybind11::arg(), pybind11::arg(), pybind11::arg("x") = 0, pybind11::arg("ldx") = 0, pybind11::arg("w") = 0,
+     pybind11::arg("ldw") = 0);
   m.def("attn_decode_set_unroll", &attn_decode_set_unroll);
   m.def("comm_model", [](uintptr_t buf, int channels, int64_t nbytes, double us, uintptr_t st) {
     launch_comm_model(P(buf), channels, nbytes, us, S(st));

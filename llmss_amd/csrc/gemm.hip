@@ -1607,8 +1607,6 @@ int launch_tiled(const bf16_t* X, int64_t ldx, const void* W, int64_t ldw, const
                  int M, int N, int K, int act, int g, int tsel, int split_hint, void* workspace, int64_t ws_bytes,
                  bool partial_out, hipStream_t st, const float* wscale = nullptr, const QkvEpi* qe = nullptr);
 
-int gemm_partial_slabs(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint,
-                       int64_t ws_bytes);
 void gemm_tiled_plan(int M, int N, int K, int* tsel_io, int* split_io, bool glu);
 void gemm_stream_plan(int M, int N, int K, int* nt_out, int* splitk_out);
 
@@ -1727,14 +1725,28 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
   }
 }
 
+// Operands that every tile of gemm_static_plan takes: rows of 16-byte alignment, 256 of them within a descriptor of 31 bits
+// (strides below 4.2 M numbers). Anything else keeps the older rules.
+static bool gemm_static_takes(const void* x, int64_t ldx, const void* w, int64_t ldw) {
+  return ldx % 8 == 0 && ldw % 8 == 0 && !(((uintptr_t)x | (uintptr_t)w) & 15) && std::max(ldx, ldw) < (1 << 22);
+}
+
+// The plan of a product: its hints, else a tuned plan, else the static one where it applies. Hints of 0 remain where the older
+// rules choose.
+static void gemm_default_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int64_t ws_bytes, bool takes, int* nt_hint,
+                              int* split) {
+  if (*nt_hint || *split || gemm_tuned_get(M, N, K, glu, w_fp8 ? 1 : 0, nt_hint, split)) return;
+  if (!w_fp8 && takes) gemm_static_plan(M, N, K, glu, slabs, ws_bytes, nt_hint, split);
+}
+static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint, int64_t ws_bytes);
+
 int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_fp8, const void* w_scale,
                 const void* bias, void* y, int64_t ldy, int M, int N, int K, int act, bool glu, void* workspace,
                 int64_t ws_bytes, int nt_hint, int split_hint, bool partial_out, hipStream_t st) {
   if (M == 0 || N == 0) return 0;
-  if (nt_hint == 0 && split_hint == 0 && !gemm_tuned_get(M, N, K, glu, w_fp8 ? 1 : 0, &nt_hint, &split_hint) && !w_fp8 &&
-      ldx % 8 == 0 && ldw % 8 == 0 && !(((uintptr_t)x | (uintptr_t)w) & 15))
-    gemm_static_plan(M, N, K, glu, partial_out && !glu && act == 0, ws_bytes, &nt_hint, &split_hint);
-  if (!y && (!partial_out || gemm_partial_slabs(M, N, K, w_fp8, glu, act, nt_hint, split_hint, ws_bytes) == 0))
+  gemm_default_plan(M, N, K, w_fp8, glu, partial_out && !glu && act == 0, ws_bytes, gemm_static_takes(x, ldx, w, ldw), &nt_hint,
+                    &split_hint);
+  if (!y && (!partial_out || slabs_of_plan(M, N, K, w_fp8, glu, act, nt_hint, split_hint, ws_bytes) == 0))
     throw std::runtime_error("gemm: this configuration writes the output, but no output buffer was given");
   if (K % 16) throw std::runtime_error("gemm: K must be a multiple of 16");
   if (glu && (N % 32)) throw std::runtime_error("gemm: glu needs N % 32 == 0");
@@ -2084,12 +2096,18 @@ int launch_tiled(const bf16_t* X, int64_t ldx, const void* W, int64_t ldw, const
 
 // Number of fp32 partial slabs launch_gemm(..., partial_out=true) leaves for these hints, or 0 if
 // that call writes the finished output (stream-K, fp8 prefill panels, act / glu epilogues, no
-// split). The Python wrapper allocates Y exactly when this returns 0 - one source of truth.
-int gemm_partial_slabs(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint,
-                       int64_t ws_bytes) {
+// split). The Python wrapper allocates Y exactly when this returns 0 - one source of truth: the operands are asked for because the plan
+// depends on their strides and places (0: strides and places that any plan takes).
+int gemm_partial_slabs(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint, int64_t ws_bytes,
+                       const void* x, int64_t ldx, const void* w, int64_t ldw) {
   if (M == 0 || N == 0 || glu || act != 0) return 0;
-  if (nt_hint == 0 && split_hint == 0 && !gemm_tuned_get(M, N, K, glu, w_fp8 ? 1 : 0, &nt_hint, &split_hint) && !w_fp8)
-    gemm_static_plan(M, N, K, glu, true, ws_bytes, &nt_hint, &split_hint);
+  gemm_default_plan(M, N, K, w_fp8, glu, true, ws_bytes, gemm_static_takes(x, ldx, w, ldw), &nt_hint, &split_hint);
+  return slabs_of_plan(M, N, K, w_fp8, glu, act, nt_hint, split_hint, ws_bytes);
+}
+
+// The same once the hints are those that the launch runs with
+static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint, int64_t ws_bytes) {
+  if (M == 0 || N == 0 || glu || act != 0) return 0;
   const int tiled_hint = nt_hint >> 8;
   const bool stream = (nt_hint & 0xff) || (!tiled_hint && (M <= 16 || (w_fp8 && M > 128)));
   int s;

@@ -645,7 +645,7 @@ def linear(x, w, bias=None, act="none", glu=False, w_scale=None, out=None, nt_hi
     partial_ok = partial_ok and not glu and act in ("none", None) and out is None
     y = out if out is not None else (None if partial_ok else torch.empty(M, nout, dtype=x.dtype, device=x.device))
     if partial_ok and lib().gemm_partial_slabs(M, N, K, fp8, False, 0, int(nt_hint), int(split_hint),
-                                               ws.numel() * 4) == 0:
+                                               ws.numel() * 4, x.data_ptr(), x.stride(0), w.data_ptr(), K) == 0:
         y = torch.empty(M, nout, dtype=x.dtype, device=x.device)  # this call finishes its output itself
     if y is not None:
         _bf16_rows(y, "out", nout)
