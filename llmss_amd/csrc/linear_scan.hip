@@ -118,7 +118,7 @@ __global__ __launch_bounds__(256) void linear_step_kernel(LinearArgs A) {
 }
 
 static int linear_step_rows(int dim, int vdim) {  // state rows per thread (0: the shape does not fit)
-  if (vdim % 4 || vdim < 4 || vdim > 1024 || dim < 1) return 0;
+  if (vdim % 4 || vdim < 4 || vdim > 1024 || dim < 1 || dim > 512) return 0;  // (512: the walk's largest; 8 KB of LDS here)
   const int RG = 256 / (vdim / 4), U = (dim + RG - 1) / RG;
   return U <= 32 ? U : 0;
 }

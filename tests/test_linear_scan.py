@@ -115,3 +115,14 @@ def test_padded_rows_leave_states_alone():
         y = ops.decay_recurrence(x, x, x, torch.full((heads,), 0.9, device="cuda"), S, cu, ctx, slots, heads, dim, vdim, True,
                                  max_qlen=n)
         assert not y[n:].any() and torch.equal(S[0], S0[0]) and torch.equal(S[2], S0[2]) and not torch.equal(S[1], S0[1])
+
+
+def test_step_form_takes_what_fits():
+    """Key dimensions up to the walk's largest, so that its launch never asks for more LDS than a workgroup gets by default."""
+    from llmss_amd.ops import hip
+    L = hip.lib()
+    for vdim in (4, 8, 64, 1024):
+        for dim in (1, 8, 31, 32, 512, 513, 4096, 7700, 8192):
+            if L.linear_step_ok(dim, vdim):
+                assert dim <= 512 and 4 * (2 * dim + 4 + 256 // (vdim // 4) * vdim) <= 64 << 10
+    assert L.linear_step_ok(512, 4) and L.linear_step_ok(128, 128)
