@@ -1335,10 +1335,10 @@ LINEAR_CHUNK_MIN = {0: 12, 2: 4}
 def _linear_forms(mode, q, k, v, dt, args, state, cu, ctx_lens, state_slots, out, heads, groups, dim, vdim, silu, max_qlen,
                   num_decode):
     """The sequences of a step that the two fast forms of a linear recurrence take: the ``num_decode`` leading single-row ones
-    (all when ``max_qlen`` is 1), then, on bf16 rows, the portions chunk by chunk. ``args``: addresses of decay / A_log, dt_bias
+    (all when ``max_qlen`` is 1 and none is empty), then, on bf16 rows, the portions chunk by chunk. ``args``: addresses of decay / A_log, dt_bias
     and D. Returns the first sequence left for the token-by-token walk."""
     B, L, st = cu.numel() - 1, lib(), _stream()
-    nd = B if max_qlen == 1 else int(num_decode)
+    nd = B if max_qlen == 1 and q.shape[0] == B else int(num_decode)  # (fewer rows: some portions are empty)
     _check(0 <= nd <= B and (nd < B or q.shape[0] == B), "num_decode outside the step")
     dt_ptr, lddt = (dt.data_ptr(), dt.stride(0)) if dt is not None else (0, 0)
     if not (L.linear_step_ok(dim, vdim) and state.data_ptr() % 16 == 0 and (dt is None or dt.dtype == q.dtype)):

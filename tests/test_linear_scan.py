@@ -126,3 +126,29 @@ def test_step_form_takes_what_fits():
             if L.linear_step_ok(dim, vdim):
                 assert dim <= 512 and 4 * (2 * dim + 4 + 256 // (vdim // 4) * vdim) <= 64 << 10
     assert L.linear_step_ok(512, 4) and L.linear_step_ok(128, 128)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,nd", [([1, 0, 1], 0), ([0], 0), ([1, 1, 0, 70, 0], 2)])
+@pytest.mark.parametrize("mode", [0, 2])
+def test_empty_portions(mode, lens, nd):
+    """A sequence without rows changes nothing, its own state among it."""
+    heads, dim, vdim, B, T = 2, 64, 64, len(lens), sum(lens)
+    S0 = torch.randn(B, heads, dim, vdim, device="cuda")
+    x = torch.randn(T, heads * dim, device="cuda").bfloat16()
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    w = [torch.full((heads,), 0.5, device="cuda") for _ in range(3)]
+
+    def step(lens, slots, S, **form):
+        cu, ctx = i32([0] + lens).cumsum(0).to(torch.int32), i32([n + 3 for n in lens])
+        if mode == 0:
+            return ops.decay_recurrence(x, x, x, w[0], S, cu, ctx, i32(slots), heads, dim, vdim, True, **form)
+        return ops.ssd_recurrence(x, x, x, x[:, :heads], *w, S, cu, ctx, i32(slots), heads, heads, dim, vdim, **form)
+    S = S0.clone()
+    y = step(lens, list(range(B)), S, max_qlen=max(1, max(lens)), num_decode=nd)
+    kept = [b for b in range(B) if lens[b]]
+    S1 = S0.clone()
+    want = step([lens[b] for b in kept], kept, S1) if kept else x[:, :0].float()
+    assert y.shape[0] == T and (not T or rel(y, want.double().cpu()) < REL)
+    for b in range(B):
+        assert torch.equal(S[b], S0[b]) if not lens[b] else rel(S[b], S1[b].double().cpu()) < REL
