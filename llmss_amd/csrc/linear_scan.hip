@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "anytype.h"
+#include "chunk_rows.h"
 
 struct LinearArgs {
   const void* q;  // [T, ldq]: head group's query at q + (h / rep) * dim
@@ -184,8 +185,57 @@ __device__ __forceinline__ s16x8 lin_cat(const s16x4& a, const s16x4& b) {
   return s16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
 }
 
+// A value that is infinite or NaN makes, by zeros of the scores times it, the tokens before it in its block of 16 NaN as well, which a walk
+// token by token does not. Their results once more, by such a walk from the portion's start: a wave for its 16 columns from col0 on, those
+// in `lanes` (a column has four), which the state tells: it has taken the value. Written for the rare case; in the chunks' loop a
+// branch for it cost 200 -> 244 us (8 x 1024 tokens, 64 heads 128 x 64).
+template <int MODE>
+__device__ __forceinline__ void linear_mend(const LinearArgs& A, int h, int b, int col0, uint64_t lanes, int lane) {
+  const int t0 = A.cu[b], qlen = A.cu[b + 1] - t0, dim = A.dim, vdim = A.vdim, gq = h / (A.H / A.G);
+  const bool cont = A.ctx[b] > qlen;
+  const float* sp = A.S + (((int64_t)A.sslots[b] * A.H + h) * dim) * (int64_t)vdim;
+  const uint64_t cols = lanes | lanes >> 16 | lanes >> 32 | lanes >> 48;
+  for (int c = 0; c < 16; ++c) {
+    const int col = col0 + c;
+    if (!(cols >> c & 1) || col >= vdim) continue;
+    auto value = [&](int t) {
+      const float x = bf2f(((const bf16_t*)A.v)[(int64_t)(t0 + t) * A.ldv + (int64_t)h * vdim + col]);
+      return MODE == 0 && A.silu ? lin_silu<bf16_t>(x) : x;
+    };
+    int bad = qlen;
+    for (int t = lane; t < qlen; t += 64)
+      if (!(fabsf(value(t)) <= FLT_MAX)) bad = min(bad, t);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) bad = min(bad, __shfl_xor(bad, o, 64));
+    if (bad % 16 == 0 || bad == qlen) continue;
+    float S[4];  // rows lane, lane + 64, ...
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[i] = cont && lane + 64 * i < dim ? sp[(int64_t)(lane + 64 * i) * vdim + col] : 0.f;
+    for (int t = 0; t < bad; ++t) {
+      const int64_t tt = t0 + t;
+      float a = A.decay[h], e = 1.f, acc = 0.f;
+      if (MODE == 2) {
+        e = lin_softplus(bf2f(((const bf16_t*)A.dt)[tt * A.lddt + h]) + A.dt_bias[h]);
+        a = expf(-expf(a) * e);
+      }
+      const float x = value(t);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (lane + 64 * i < dim) {
+          const int64_t d = (int64_t)gq * dim + lane + 64 * i;
+          const float k = bf2f(((const bf16_t*)A.k)[tt * A.ldk + d]), q = bf2f(((const bf16_t*)A.q)[tt * A.ldq + d]);
+          S[i] = fmaf(a, S[i], e * (A.silu ? lin_silu<bf16_t>(k) : k) * x);
+          acc = fmaf(S[i], A.silu ? lin_silu<bf16_t>(q) : q, acc);
+        }
+      acc = warp_sum(acc);
+      if (MODE == 2 && A.skip) acc = fmaf(A.skip[h], x, acc);
+      if (t >= (bad & ~15) && lane == 0) A.out[(tt * A.H + h) * vdim + col] = acc;
+    }
+  }
+}
+
 // Bound by the chain of chunks: a prompt step of 8 sequences has one (decay) or two (ssd) workgroups per CU, each 16 dependent
-// chunks. 8 x 1024 tokens: ssd, 64 heads 128 x 64, 2160 us token by token, 310 us with fp32 instructions throughout, 195 us here
+// chunks. 8 x 1024 tokens: ssd, 64 heads 128 x 64, 2160 us token by token, 310 us with fp32 instructions throughout, 208 us here
 // (no workgroup exchanges anything inside a chunk but the scores); decay, 16 heads 128 x 128, 1230 us with its activation pass,
 // 290 us here.
 //
@@ -273,7 +323,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
   const float dskip = MODE == 2 && A.skip ? A.skip[h] : 0.f;
   const float dec = A.decay[h];
   // the log factor of a token; a factor of zero (or nearly so) becomes one that vanishes over a single token
-  const double lg0 = MODE == 0 ? fmax(log((double)fabsf(dec)), -1e4) : 0.0;
+  const double lg0 = MODE == 0 ? at_least(log((double)fabsf(dec)), -1e4) : 0.0;
   const bool alt = MODE == 0 && dec < 0.f;  // a negative factor: the sign alternates with the distance
   const float ea = MODE == 2 ? expf(dec) : 0.f, dtb = MODE == 2 ? A.dt_bias[h] : 0.f;
   fetch(0);
@@ -298,7 +348,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
       float e = in ? 1.0f : 0.f;
       if (MODE == 2) {
         e = in ? lin_softplus(rd + dtb) : 0.f;
-        F = in ? fmax((double)(-ea * e), -1e8) : 0.0;
+        F = in ? at_least((double)(-ea * e), -1e8) : 0.0;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
           const double x = __shfl_up(F, o, 64);
@@ -488,6 +538,12 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
         }
     }
   }
+  float z = 0.f;
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) z = fmaf(S[kt][i], 0.f, z);
+  if (__any(z != z)) linear_mend<MODE>(A, h, b, blockIdx.y * 64 + 16 * w, __ballot(z != z), lane);
   if (col < vdim) {
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt)
