@@ -16,6 +16,7 @@
 //                 X, P) enters as value + remainder, two bf16 numbers, and sums and the state itself stay fp32. The inverse is
 //                 taken in fp32: 16 x 16 diagonal blocks by substitution, the blocks below by fp32 matrix instructions.
 #include "anytype.h"
+#include "chunk_rows.h"
 
 // ------------------------------------------------------------------------------------------------ single rows
 struct DeltaStepArgs {
@@ -243,6 +244,8 @@ __device__ __forceinline__ void lower_inverse(const float* Ls, float* Xs, const 
           z = __builtin_amdgcn_mfma_f32_16x16x4f32(Ls[(16 * bi + li) * LDL + 16 * m + 4 * g + i],
                                                    Xs[(16 * m + 4 * g + i) * LDL + 16 * bj + li], z, 0, 0, 0);
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) z[i] = fabsf(z[i]) <= FLT_MAX ? z[i] : 0.f;  // (rows that are NaN in any case: not into those above)
 #pragma unroll
       for (int i = 0; i < 4; ++i)  // (the accumulator's rows 4 g + i are the second operand as they stand)
         o = __builtin_amdgcn_mfma_f32_16x16x4f32(Xs[(16 * bi + li) * LDL + 16 * bi + 4 * g + i], z[i], o, 0, 0, 0);
@@ -726,7 +729,7 @@ __global__ __launch_bounds__(256) void delta_prep32_kernel(DeltaChunk32Args A) {
     const int64_t tt = (int64_t)(t0 + j0 + min(lane, nt - 1)) * A.ldab + h;
     const float z = El<TP>::ld((const TP*)A.a + tt) + A.dt_bias[h];
     // (a decay of zero: a sum this low vanishes over a single token, and differences of equal sums stay zero)
-    double F = in ? fmax((double)(-expf(A.A_log[h]) * (z > 20.f ? z : log1pf(expf(z)))), -1e8) : 0.0;
+    double F = in ? at_least((double)(-expf(A.A_log[h]) * (z > 20.f ? z : log1pf(expf(z)))), -1e8) : 0.0;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const double x = __shfl_up(F, o, 64);
@@ -790,7 +793,7 @@ __global__ __launch_bounds__(256) void delta_prep32_kernel(DeltaChunk32Args A) {
     f32x4 x = ldv4(&Xs[r * LDL + s0]);
     const f32x4 y = ldv4(&be[s0]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] *= y[i];
+    for (int i = 0; i < 4; ++i) x[i] = s0 + i <= r ? x[i] * y[i] : 0.f;  // (no later token's NaN in an earlier row)
     float* dst = A.X + (row + (int64_t)r * H) * 64 + s0;
     *reinterpret_cast<f32x4*>(dst) = x;
     *reinterpret_cast<f32x4*>(dst + A.mat) = ldv4(&Ps[r * LDL + s0]);
@@ -806,7 +809,7 @@ __global__ __launch_bounds__(256) void delta_prep32_kernel(DeltaChunk32Args A) {
 // register of an accumulator tile is the second operand of a 16x16x4 instruction over its rows 4 g + i, and the first operand's
 // matching numbers are four neighbours of a row in LDS. Blocks of 16 tokens past the portion's end are skipped.
 template <int KT>
-__global__ __launch_bounds__(256) void delta_chunk32_kernel(DeltaChunk32Args A) {
+__global__ __launch_bounds__(256, KT <= 2 ? 2 : 1) void delta_chunk32_kernel(DeltaChunk32Args A) {
   constexpr int C = 64, DKP = 16 * KT, LDK = DKP + 4, LDP = 64 + 4;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   float* Qs = reinterpret_cast<float*>(smem);
@@ -897,6 +900,7 @@ __global__ __launch_bounds__(256) void delta_chunk32_kernel(DeltaChunk32Args A) 
         o[rt][i] *= x[1];
       }
     }
+    int bad = contain(u, o, g);
     // U = X u, O += P U
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
@@ -908,6 +912,7 @@ __global__ __launch_bounds__(256) void delta_chunk32_kernel(DeltaChunk32Args A) 
         for (int i = 0; i < 4; ++i) U[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], u[m][i], U[rt], 0, 0, 0);
       }
     }
+    bad = min(bad, contain(U, o, g));
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
       if (rt >= nb) continue;
@@ -921,10 +926,11 @@ __global__ __launch_bounds__(256) void delta_chunk32_kernel(DeltaChunk32Args A) 
       o[rt] += in;
     }
     // the state: e^(b_C) S_0 + K^T (w U)
+    const float keep = bad < C ? __uint_as_float(0x7fc00000u) : a_all;
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) S[kt][i] *= a_all;
+      for (int i = 0; i < 4; ++i) S[kt][i] *= keep;
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       if (m >= nb) continue;

@@ -64,3 +64,47 @@ def test_linear(mode, dim, vdim, t, place, value):
     same(y.view(T, heads, vdim), o, 1e-5)  # the bound of the finite cases: fp32 sums over at most 256 terms and 64 tokens
     for b in range(B):
         same(S[b], states[b], 1e-5)
+
+
+@pytest.mark.parametrize("dim,vdim", [(32, 36), (128, 64)])
+@pytest.mark.parametrize("t", [3, 16, 47, 79, 129, 133])
+@pytest.mark.parametrize("place,value", [("v", NAN), ("v", INF), ("k", NAN), ("k", INF), ("q", NAN), ("q", -INF), ("a", NAN), ("a", INF),
+                                         ("a", -INF), ("b", NAN), ("b", INF), ("b", -INF), ("S", INF)])
+def test_delta_rows32(dim, vdim, t, place, value):
+    heads = 2
+    gen = torch.Generator().manual_seed(t)
+    T, B = sum(LENS), len(LENS)
+    q, k, v = (torch.randn(T, heads, n, generator=gen) for n in (dim, dim, vdim))
+    a, b_, S0 = torch.randn(T, heads, generator=gen), torch.randn(T, heads, generator=gen), torch.randn(B, heads, dim, vdim, generator=gen)
+    if place == "S":
+        S0[0, 0, 2, 5] = value
+    else:
+        {"v": v, "k": k, "q": q, "a": a.view(T, heads, 1), "b": b_.view(T, heads, 1)}[place][t, 1, -1] = value
+    gate, w = torch.randn(T, heads * vdim, generator=gen), 1 + 0.1 * torch.randn(vdim, generator=gen)
+    A_log, bias = torch.randn(heads, generator=gen) - 1, torch.randn(heads, generator=gen)
+    unit = lambda x: x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6)  # noqa: E731
+    Q, K, V = unit(q.double()) * dim ** -0.5, unit(k.double()), v.double()
+    g = torch.exp(-torch.exp(A_log.double()) * torch.nn.functional.softplus(a.double() + bias.double()))
+    beta = torch.sigmoid(b_.double())
+    o, states, r = torch.zeros_like(V), [], 0
+    for b, n in enumerate(LENS):
+        S = S0[b].double()
+        for _ in range(n):
+            S = S * g[r, :, None, None]
+            u = beta[r, :, None] * (V[r] - (S * K[r, :, :, None]).sum(1))
+            S = S + K[r, :, :, None] * u[:, None]
+            o[r] = (S * Q[r, :, :, None]).sum(1)
+            r += 1
+        states.append(S)
+    z = gate.double().view(T, heads, vdim)
+    want = 0.7 * o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-6) * w.double() * z * torch.sigmoid(z)
+    c = lambda x: x.cuda()  # noqa: E731
+    S, cu, out = c(S0), prefix(LENS), torch.empty(T, heads * vdim, device="cuda")
+    rows = [c(x).flatten(1) for x in (q, k, v)]
+    ab = c(torch.cat([a, b_], 1))
+    ops.delta_mix(*rows, ab[:, :heads], ab[:, heads:], c(A_log), c(bias), S, c(cu), c(cu.diff() + 7), torch.arange(B, dtype=torch.int32, device="cuda"),
+                  heads, heads, dim, vdim, c(gate), c(w), 1e-6, 0.7, out, max_qlen=max(LENS), num_decode=0)
+    # the bound of the finite cases: fp32 sums over up to 128 terms, then substitution over 64 tokens
+    same(out.view(T, heads, vdim), want, 2e-5)
+    for b in range(B):
+        same(S[b], states[b], 2e-5)
