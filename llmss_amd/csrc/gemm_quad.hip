@@ -262,11 +262,21 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
       }
     }
   };
+  // the image passes numbers between the lanes of this wave: its writes before the reads, and those before the next writes
+  auto turn = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
   put(0, acc[0], acc[1]);
   put(1, acc[2], acc[3]);
-  if constexpr (!GLU) flush(n0 + wc * 128);
+  if constexpr (!GLU) {
+    turn();
+    flush(n0 + wc * 128);
+    turn();
+  }
   put(2, acc[4], acc[5]);
   put(3, acc[6], acc[7]);
+  turn();
   flush(GLU ? n0 / 2 + wc * 64 : n0 + wc * 128 + 64);
 }
 
