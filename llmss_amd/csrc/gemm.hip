@@ -883,7 +883,8 @@ __global__ __launch_bounds__(512, 1) void gemm_big_kernel(const void* __restrict
 }
 
 // -------------------------------------------------------------------------------------------
-// Ping-pong prefill GEMM (bf16, M >= ~1024) for what gemm_quad.hip does not take: K off 64, N off 8, outputs off 16 bytes.
+// Ping-pong prefill GEMM (bf16, M >= ~1024) for what gemm_quad.hip does not take: K off 64 (Llama-2-7B's TP=8 down projection,
+// K = 1376), N off 8 (GLU 32), rows over more than 31 bits of bytes (256 of them; gathered ones: all).
 // 256x256x64 tile, 8 waves = two groups of 4 (waves 0-3 / 4-7; one wave of each group per SIMD). Waves
 // 4-7 pass one extra barrier before the K-loop, so on every SIMD one wave's compute segment runs beside
 // its partner's load segment (guide "The 256^2 8-phase template", MI355X_MICROARCH "Two waves per SIMD").
@@ -912,7 +913,7 @@ __device__ __forceinline__ void pp_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <bool KTAIL, int GRP = 0>
+template <int GRP>
 __global__ __launch_bounds__(512, 1) void gemm_pp_kernel(const bf16_t* __restrict__ A, int64_t lda,
                                                          const bf16_t* __restrict__ B, int64_t ldb,
                                                          const bf16_t* __restrict__ bias, bf16_t* __restrict__ Y,
@@ -967,7 +968,7 @@ __global__ __launch_bounds__(512, 1) void gemm_pp_kernel(const bf16_t* __restric
     soff[2][i] = (int64_t)bc1 * ldb * 2 + gc * 16;
   }
   auto stage = [&](int t, int h, char* buf) {
-    const bool last = KTAIL && t == nk - 1;  // wave-uniform; KTAIL: K % 64 != 0 (Llama-2-7B TP=8 down, K = 1376)
+    const bool last = t == nk - 1;  // wave-uniform
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const char* p = src[h] + soff[h][i] + (int64_t)t * 128;
@@ -2000,12 +2001,9 @@ int launch_tiled(const bf16_t* X, int64_t ldx, const void* W, int64_t ldw, const
     if (gemm_quad_ok(N, K, ldx, ldw, 256, Y, ldy, 2, g != 0))
       launch_gemm_quad(0, X, ldx, (const bf16_t*)W, ldw, B, Y, ldy, M, N, K, act, g, g_big_group_m,
                        tiles_of(M, N, 256, 256), PpGroup{}, st);
-    else if (K & 63)
-      gemm_pp_kernel<true><<<tiles_of(M, N, 256, 256), 512, 0, st>>>(X, ldx, (const bf16_t*)W, ldw, B, Y, ldy, M, N, K,
-                                                                     act, g, g_big_group_m, zero_page(), PpGroup{});
     else
-      gemm_pp_kernel<false><<<tiles_of(M, N, 256, 256), 512, 0, st>>>(X, ldx, (const bf16_t*)W, ldw, B, Y, ldy, M, N, K,
-                                                                      act, g, g_big_group_m, nullptr, PpGroup{});
+      gemm_pp_kernel<0><<<tiles_of(M, N, 256, 256), 512, 0, st>>>(X, ldx, (const bf16_t*)W, ldw, B, Y, ldy, M, N, K, act, g,
+                                                                  g_big_group_m, K & 63 ? zero_page() : nullptr, PpGroup{});
     HIP_CHECK_LAUNCH();
     return 0;
   }
@@ -2217,7 +2215,7 @@ void gemm_plan(int M, int N, int K, bool w_fp8, int* nt, int* splitk) {
   }
 }
 
-// Grouped expert products on the ping-pong kernel, over a tile list of 256 rows per tile (moe_group): C = act(A[order / top]
+// Grouped expert products on 256 x 256 tiles (gemm_quad.hip, else the ping-pong kernel), over a tile list of 256 rows per tile (moe_group): C = act(A[order / top]
 // W_e^T) in bf16 (mode 1), C = A W_e^T in fp32 (mode 2), or C [rows, N / 2] = silu(gate) * up in bf16 with W's rows gate and up
 // in alternating groups of 16 (mode 3). A [rows, K] with row stride lda, W [E, N, K].
 void launch_moe_pp(int mode, const void* A, int64_t lda, const void* W, const void* meta, const void* order, void* C, int E,
@@ -2240,18 +2238,12 @@ void launch_moe_pp(int mode, const void* A, int64_t lda, const void* W, const vo
                      glu ? 0 : act, glu, 1, (unsigned)nwg, gr, st);
     return;
   }
-#define LAUNCH_PPG(KT_, G_)                                                                                         \
-  gemm_pp_kernel<KT_, G_><<<(unsigned)nwg, 512, 0, st>>>((const bf16_t*)A, lda, (const bf16_t*)W, K, nullptr, (bf16_t*)C, \
-                                                         glu ? N / 2 : N, 0, N, K, glu ? 0 : act, glu, 1, z, gr)
-  if (mode == 1 || mode == 3) {
-    if (K & 63) LAUNCH_PPG(true, 1);
-    else LAUNCH_PPG(false, 1);
-  } else if (mode == 2) {
-    if (K & 63) LAUNCH_PPG(true, 2);
-    else LAUNCH_PPG(false, 2);
-  } else {
-    throw std::runtime_error("moe_pp: mode");
-  }
+#define LAUNCH_PPG(G_)                                                                                              \
+  gemm_pp_kernel<G_><<<(unsigned)nwg, 512, 0, st>>>((const bf16_t*)A, lda, (const bf16_t*)W, K, nullptr, (bf16_t*)C, \
+                                                    glu ? N / 2 : N, 0, N, K, glu ? 0 : act, glu, 1, z, gr)
+  if (mode == 1 || mode == 3) LAUNCH_PPG(1);
+  else if (mode == 2) LAUNCH_PPG(2);
+  else throw std::runtime_error("moe_pp: mode");
 #undef LAUNCH_PPG
   HIP_CHECK_LAUNCH();
 }
