@@ -1648,13 +1648,15 @@ bool gemm_tuned_get(int M, int N, int K, bool glu, int kind, int* nt_hint, int* 
 // Plan of a bf16 product that carries no hint and no tuned plan: prompt and mixed steps of any size, models run without the
 // autotuner. Leaves the hints at 0 where the older static rules below are still the better ones.
 //
-// M <= 64: the K-split-wave decode kernel (gemm_dec.hip) on column tiles of 16 - 64, the width that makes the waves of 256
-// workgroups times the tile's width smallest, ties to the wider. Over 13 shapes of 1024 - 32000 columns (bench shapes of the
-// 1024, 1600, 2048 and 4096 wide models) this is 0.4 - 3 % above the best plan found at M <= 20 and 1.5 (M <= 16) and 1.2
-// (M = 20) times faster than the streaming / 64 x 64 plans: 4096 x 4096 at one row 13.6 -> 9.6 us, 22016 x 4096 44 -> 35 us. From 33 rows on
-// narrow products read X too often for their weights and keep the 64 x 64 tiles: below 3072 columns (2048 x 4096 at 64 rows:
-// 12.2 against 14.7 us), and where 16-column tiles would walk a long K (4096 x 11008: 27.8 against 35.7 us); very wide ones (SwiGLU,
-// LM heads) take one wave of 64 x 96 or 64 x 128 tiles (22016 x 4096 at 64 rows: 53 -> 39 us).
+// M <= 64: the K-split-wave decode kernel (gemm_dec.hip) on column tiles of 16 - 64 where a cost model expects it to be 1.25 times
+// faster than the older rules. A wave of 256 workgroups takes the bytes that one asks for - its weights, and X once more for every tile,
+// which is what narrow products with a long K pay for - at what a CU gets, or all their weights at what the chip gets, whichever is
+// longer. The older rules are priced likewise. Constants fitted over random shapes of 256 - 32000 columns and K of 256 - 16000
+// (13 % off on average, the width chosen 0 - 0.5 % above the best one). 987 others take 0.60 (up to 16 rows), 0.81 (32) and 0.88 (64)
+// of the older rules' time, one of them more than 5 % longer (8 %): 4096 x 4096 at one row 13.6 -> 9.6 us, 22016 x 4096 44 -> 35 us;
+// 512 x 11168 SwiGLU at 32 rows (14.0 against 35.6 us) and 18368 x 816 at 17 (13.8, 21.3) stay. From 33 rows on products below
+// 3072 columns keep the 64 x 64 tiles (2048 x 4096 at 64 rows: 12.2 against 14.7 us), and SwiGLU and LM heads of more than 16384 columns
+// take one wave of 64 x 96 or 64 x 128 tiles (22016 x 4096 at 64 rows: 53 -> 39 us).
 //
 // M > 64: the cheapest of six tiles by a cost model. A wave of the chip takes (k-steps of 64) x us per step + 5 us, an unfilled
 // second workgroup per CU counts for less, a K split adds its slabs' write and read at 4.5 TB/s and a launch, and nothing
@@ -1671,6 +1673,13 @@ static constexpr TileCost kTileCost[] = {
     {4, 256, 256, 1, 1.45, 1.45},           {9 | 16, 256, 128, 1, 1.02, 1.02},        {12 | 16 | 512, 128, 256, 1, 1.06, 1.06},
     {8 | 32 | 512, 128, 128, 1, 0.70, 0.70}, {11 | 32 | 512, 64, 128, 1, 0.41, 0.41}, {11 | 16, 64, 128, 2, 0.64, 0.44},
 };
+struct DecCost {
+  double start, cu, x, wave, chip;  // us; bytes per us and CU; a row of X against one of W; us per wave of workgroups; bytes per us
+};
+static constexpr DecCost kDecCost[] = {  // up to 16, 32, 64 rows
+    {2.5, 37.5e3, 0.72, 1.17, 4.58e6}, {1.1, 36.9e3, 0.70, 2.68, 3.90e6}, {1.3, 31.5e3, 0.53, 3.07, 3.61e6}};
+static int tile_dims(int tsel, int* bm, int* bn);
+static int tiles_of(int M, int N, int bm, int bn);
 // slabs: the consumer sums split-K slabs itself and so gets the product in 32 bits. Where the older rules split K that stays so:
 // only split plans are looked at, their slabs costing a write and a read and no launch.
 static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t ws_bytes, int* nt_hint, int* split) {
@@ -1688,21 +1697,43 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
       *split = 1;
       return;
     }
-    int best = 0, width = 0, sp = 1;
+    if (M > 32 && N < 3072) return;
+    const double bytes = 2.0 * N * K, slab = 8.0 * M * N / 2.5e6;
+    double older;
+    if (M <= 16) {
+      int nt, s;
+      gemm_stream_plan(M, N, K, &nt, &s);
+      older = 2.0 + std::max(((K + 255) / 256 + s - 1) / s * 2.17 * nt, bytes / 3.03e6) + (s > 1 && !slabs ? 2.9 : 0.0);
+    } else {
+      int t = 0, s = 0, bm, bn;
+      gemm_tiled_plan(M, N, K, &t, &s, glu);
+      tile_dims(t & 15, &bm, &bn);
+      const double step = (t & 15) == 4 ? 1.45 : (bn == 64 ? 0.334 : 0.45);
+      older = 4.8 + std::max(((K + 63) / 64 + s - 1) / s * step, bytes / 4.16e6) + (s > 1 ? s * slab + (slabs ? 0.0 : 1.0) : 0.0);
+    }
+    const DecCost& c = kDecCost[M <= 16 ? 0 : M <= 32 ? 1 : 2];
+    double best = 0;
+    int width = 0, sp = 1;
     for (int s = slabs ? 2 : 1; s <= (slabs ? 4 : 1); s *= 2) {
-      if (s > 1 && K / s < 256) break;
-      for (int code = 4; code >= 1; --code) {  // 64, 48, 32, 16 columns
-        const int bn = 16 * code;
+      if (s > 1 && (K / s < 256 || (int64_t)s * M * N * 4 > ws_bytes)) break;
+      for (int bn = 64; bn >= 16; bn -= 16) {
         if (glu && bn % 32) continue;
-        const int cost = ((N + bn - 1) / bn * s + 255) / 256 * bn * (4 / s);
-        if (!best || cost < best) best = cost, width = bn, sp = s;
+        const int wgs = (N + bn - 1) / bn * s;
+        const double one = (double)K / s * (bn + c.x * M) * 2 / c.cu + c.wave, read = (double)K / s * bn * 2 / c.chip;
+        const double t = c.start + wgs / 256 * std::max(one, 256 * read) + (wgs % 256 ? std::max(one, wgs % 256 * read) : 0.0) +
+                         (s > 1 ? s * slab : 0.0);
+        if (!width || t < best) best = t, width = bn, sp = s;
       }
     }
-    if (!best || (M > 32 && (N < 3072 || (width == 16 && K > 4096)))) return;
+    if (!width || best * 1.25 > older) return;
     *nt_hint = (width / 16 | 32 | 1024) << 8;
     *split = sp;
     return;
   }
+  // two rows of 64 x 64 tiles, two to three workgroups per CU: the older rule's one launch of them is the faster one until K is long
+  // (22016 x 2656 at 80 rows: 42.7 against 47.4 us; x 4096: 53.6 and 54.4; 16640 x 5120: 57.5 and 52.9)
+  const int t64 = tiles_of(M, N, 64, 64);
+  if (glu && M <= 128 && t64 > 512 && t64 <= 768 && K < 3900) return;
   const int nk = (K + 63) / 64;
   const double bytes = 2.0 * N * K + 2.0 * M * K + 2.0 * M * (glu ? N / 2 : N);
   double best = 0;
