@@ -47,7 +47,7 @@ int launch_gemm_qkv_args(const void* x, int64_t ldx, const void* w, int64_t ldw,
 int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_fp8, const void* w_scale,
                 const void* bias, void* y, int64_t ldy, int M, int N, int K, int act, bool glu, void* workspace,
                 int64_t ws_bytes, int nt_hint, int split_hint, bool partial_out, hipStream_t st);
-void gemm_plan(int M, int N, int K, bool w_fp8, int* nt, int* splitk);
+void gemm_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int* nt, int* splitk);
 void gemm_tuned_set(int M, int N, int K, bool glu, int kind, int nt_hint, int split);
 void gemm_tuned_clear();
 void gemm_reserve_streamk(int n);
@@ -339,11 +339,12 @@ PYBIND11_MODULE(_C, m) {
      pybind11::arg("pos"), pybind11::arg("cos_t"), pybind11::arg("sin_t"), pybind11::arg("kc"), pybind11::arg("vc"),
      pybind11::arg("slot"), pybind11::arg("nh"), pybind11::arg("nkv"), pybind11::arg("D"), pybind11::arg("rot"),
      pybind11::arg("bs"), pybind11::arg("style"), pybind11::arg("do_rope"), pybind11::arg("st"));
-  m.def("gemm_plan", [](int M, int N, int K, bool fp8) {
+  m.def("gemm_plan", [](int M, int N, int K, bool fp8, bool glu, bool slabs) {
     int nt, s;
-    gemm_plan(M, N, K, fp8, &nt, &s);
+    gemm_plan(M, N, K, fp8, glu, slabs, &nt, &s);
     return py::make_tuple(nt, s);
-  });
+  }, pybind11::arg(), pybind11::arg(), pybind11::arg(), pybind11::arg(), pybind11::arg("glu") = false,
+     pybind11::arg("slabs") = true);
   m.def("gemm_tuned_set", &gemm_tuned_set);
   m.def("gemm_tuned_clear", &gemm_tuned_clear);
   m.def("gemm_reserve_streamk", &gemm_reserve_streamk);

@@ -1648,15 +1648,18 @@ bool gemm_tuned_get(int M, int N, int K, bool glu, int kind, int* nt_hint, int* 
 // Plan of a bf16 product that carries no hint and no tuned plan: prompt and mixed steps of any size, models run without the
 // autotuner. Leaves the hints at 0 where the older static rules below are still the better ones.
 //
-// M <= 64: the K-split-wave decode kernel (gemm_dec.hip) on column tiles of 16 - 64 where a cost model expects it to be 1.25 times
-// faster than the older rules. A wave of 256 workgroups takes the bytes that one asks for - its weights, and X once more for every tile,
-// which is what narrow products with a long K pay for - at what a CU gets, or all their weights at what the chip gets, whichever is
-// longer. The older rules are priced likewise. Constants fitted over random shapes of 256 - 32000 columns and K of 256 - 16000
-// (13 % off on average, the width chosen 0 - 0.5 % above the best one). 987 others take 0.60 (up to 16 rows), 0.81 (32) and 0.88 (64)
-// of the older rules' time, one of them more than 5 % longer (8 %): 4096 x 4096 at one row 13.6 -> 9.6 us, 22016 x 4096 44 -> 35 us;
-// 512 x 11168 SwiGLU at 32 rows (14.0 against 35.6 us) and 18368 x 816 at 17 (13.8, 21.3) stay. From 33 rows on products below
-// 3072 columns keep the 64 x 64 tiles (2048 x 4096 at 64 rows: 12.2 against 14.7 us), and SwiGLU and LM heads of more than 16384 columns
-// take one wave of 64 x 96 or 64 x 128 tiles (22016 x 4096 at 64 rows: 53 -> 39 us).
+// M <= 64: the K-split-wave decode kernel (gemm_dec.hip) on column tiles of 16 - 64, or, for 33 - 64 rows and more than 8192 columns,
+// tiles of 64 x 96 and 64 x 128, where a cost model expects the cheapest to be 1.15 times faster than the older rules (1.25 up to 16 rows).
+// A wave of 256 workgroups takes the bytes that one asks for - its weights, and X once more for every tile, which is what narrow
+// products with a long K pay for - at what a CU gets, or all their weights at what the chip gets, whichever is longer. The older
+// rules are priced likewise. Constants fitted over 1030 random shapes of 256 - 70000 columns and K of 256 - 16000 (9 - 13 % off on
+// average, the choice 1.6 - 2.7 % above the best of all). Against the older rules: 0.68 of their time up to 16 rows, 0.84 to 32,
+// 0.88 to 64: 4096 x 4096 at one row 13.6 -> 9.6 us, 32000 x 4096 at 23 rows 62 -> 48, 22016 x 4096 at 24 rows 46 -> 35 us; 512 x 11168
+// SwiGLU at 32 rows (14.0 against 35.6 us) and 18368 x 816 at 17 (13.8, 21.3) stay. From 33 rows on products below 3072 columns keep
+// the 64 x 64 tiles (2048 x 4096 at 64 rows: 12.2 against 14.7 us). Tiles of 96 columns are for one wave of them (22016 x 4096 SwiGLU at
+// 64 rows: 53 -> 39 us); one of the two taken for every product of more than 16384 columns lost to the older rules where a second wave
+// is nearly empty and where K is short (43776 x 8160 SwiGLU at 33 rows 182 -> 223 us on 128 columns, 178 on 96; 35616 x 384 at 45
+// rows 10.0 -> 13.9).
 //
 // M > 64: the cheapest of six tiles by a cost model. A wave of the chip takes (k-steps of 64) x us per step + 5 us, an unfilled
 // second workgroup per CU counts for less, a K split adds its slabs' write and read at 4.5 TB/s and a launch, and nothing
@@ -1677,7 +1680,21 @@ struct DecCost {
   double start, cu, x, wave, chip;  // us; bytes per us and CU; a row of X against one of W; us per wave of workgroups; bytes per us
 };
 static constexpr DecCost kDecCost[] = {  // up to 16, 32, 64 rows
-    {2.5, 37.5e3, 0.72, 1.17, 4.58e6}, {1.1, 36.9e3, 0.70, 2.68, 3.90e6}, {1.3, 31.5e3, 0.53, 3.07, 3.61e6}};
+    {2.5, 37.5e3, 0.72, 1.17, 4.58e6}, {1.33, 34.1e3, 0.404, 2.61, 6.28e6}, {1.33, 29.8e3, 0.382, 3.06, 4.54e6}};
+struct OlderCost {  // of 17 - 64 rows: us per 64 of k on tiles of 64, 128 and 256 columns; bytes per us; the same of slabs; us for their sum
+  double s64, s128, s256, chip, slab, sum;
+};
+static constexpr OlderCost kOlderCost[] = {  // up to 32, 64 rows
+    {0.334, 0.2, 1.74, 5.37e6, 2.05e6, 0.98}, {0.364, 1.04, 2.33, 4.47e6, 2.86e6, 1.07}};
+struct WideCost {  // the 64-row tiles of wide products, as DecCost but for us per 64 of k
+  int tsel, bn;
+  double start, step, wave, chip;
+};
+static constexpr WideCost kWideCost[] = {{15 | 32, 96, 3.43, 0.511, 1.17, 6.19e6}, {11 | 32, 128, 0.02, 0.587, 5.44, 5.40e6}};
+// waves of 256 workgroups: one of them takes `one` us, its share of the chip's rate `read`
+static double waves_us(int wgs, double one, double read) {
+  return wgs / 256 * std::max(one, 256 * read) + (wgs % 256 ? std::max(one, wgs % 256 * read) : 0.0);
+}
 static int tile_dims(int tsel, int* bm, int* bn);
 static int tiles_of(int M, int N, int bm, int bn);
 // slabs: the consumer sums split-K slabs itself and so gets the product in 32 bits. Where the older rules split K that stays so:
@@ -1691,12 +1708,6 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
     slabs = s > 1 && (int64_t)s * M * N * 4 <= ws_bytes;
   }
   if (M <= 64) {
-    if (M > 32 && N > 16384 && !slabs) {
-      const int t96 = (N + 95) / 96;
-      *nt_hint = (t96 <= 256 ? 15 | 32 : 11 | 32) << 8;
-      *split = 1;
-      return;
-    }
     if (M > 32 && N < 3072) return;
     const double bytes = 2.0 * N * K, slab = 8.0 * M * N / 2.5e6;
     double older;
@@ -1705,28 +1716,34 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
       gemm_stream_plan(M, N, K, &nt, &s);
       older = 2.0 + std::max(((K + 255) / 256 + s - 1) / s * 2.17 * nt, bytes / 3.03e6) + (s > 1 && !slabs ? 2.9 : 0.0);
     } else {
+      const OlderCost& c = kOlderCost[M > 32];
       int t = 0, s = 0, bm, bn;
       gemm_tiled_plan(M, N, K, &t, &s, glu);
       tile_dims(t & 15, &bm, &bn);
-      const double step = (t & 15) == 4 ? 1.45 : (bn == 64 ? 0.334 : 0.45);
-      older = 4.8 + std::max(((K + 63) / 64 + s - 1) / s * step, bytes / 4.16e6) + (s > 1 ? s * slab + (slabs ? 0.0 : 1.0) : 0.0);
+      const double step = (t & 15) == 4 ? c.s256 : (bn == 64 ? c.s64 : c.s128);
+      older = 4.71 + std::max(((K + 63) / 64 + s - 1) / s * step, bytes / c.chip);
+      if (s > 1) older += s * 8.0 * M * N / c.slab + (slabs ? 0.0 : c.sum);
     }
     const DecCost& c = kDecCost[M <= 16 ? 0 : M <= 32 ? 1 : 2];
     double best = 0;
-    int width = 0, sp = 1;
+    int code = 0, sp = 1;
     for (int s = slabs ? 2 : 1; s <= (slabs ? 4 : 1); s *= 2) {
       if (s > 1 && (K / s < 256 || (int64_t)s * M * N * 4 > ws_bytes)) break;
       for (int bn = 64; bn >= 16; bn -= 16) {
         if (glu && bn % 32) continue;
-        const int wgs = (N + bn - 1) / bn * s;
         const double one = (double)K / s * (bn + c.x * M) * 2 / c.cu + c.wave, read = (double)K / s * bn * 2 / c.chip;
-        const double t = c.start + wgs / 256 * std::max(one, 256 * read) + (wgs % 256 ? std::max(one, wgs % 256 * read) : 0.0) +
-                         (s > 1 ? s * slab : 0.0);
-        if (!width || t < best) best = t, width = bn, sp = s;
+        const double t = c.start + waves_us((N + bn - 1) / bn * s, one, read) + (s > 1 ? s * slab : 0.0);
+        if (!code || t < best) best = t, code = bn / 16 | 32 | 1024, sp = s;
       }
     }
-    if (!width || best * 1.25 > older) return;
-    *nt_hint = (width / 16 | 32 | 1024) << 8;
+    if (M > 32 && N > 8192 && !slabs) {
+      for (const WideCost& w : kWideCost) {
+        const double t = w.start + waves_us((N + w.bn - 1) / w.bn, (K + 63) / 64 * w.step + w.wave, 2.0 * K * w.bn / w.chip);
+        if (t < best) best = t, code = w.tsel;
+      }
+    }
+    if (!code || best * (M <= 16 ? 1.25 : 1.15) > older) return;
+    *nt_hint = code << 8;
     *split = sp;
     return;
   }
@@ -2221,10 +2238,11 @@ int launch_gemm_qkv_args(const void* x, int64_t ldx, const void* w, int64_t ldw,
   return launch_gemm_qkv(x, ldx, w, ldw, bias, y, ldy, M, N, K, workspace, ws_bytes, nt_hint, split_hint, qe, st);
 }
 
-void gemm_plan(int M, int N, int K, bool w_fp8, int* nt, int* splitk) {
+// The plan of a product without hints. slabs: of one whose consumer sums split-K slabs itself
+void gemm_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int* nt, int* splitk) {
   *nt = *splitk = 0;
-  const bool tuned = gemm_tuned_get(M, N, K, false, w_fp8 ? 1 : 0, nt, splitk);
-  if (!tuned && !w_fp8) gemm_static_plan(M, N, K, false, true, 64 << 20, nt, splitk);
+  const bool tuned = gemm_tuned_get(M, N, K, glu, w_fp8 ? 1 : 0, nt, splitk);
+  if (!tuned && !w_fp8) gemm_static_plan(M, N, K, glu, slabs && !glu, 64 << 20, nt, splitk);
   if (tuned || *nt) {
     if ((*nt >> 8) & kDecHint) {
       *splitk = ((*nt >> 8) & 256) ? 1 : dec_split(M, N, K, *splitk, INT64_MAX);
@@ -2232,7 +2250,7 @@ void gemm_plan(int M, int N, int K, bool w_fp8, int* nt, int* splitk) {
       *splitk = 1;  // stream-K / split-K combine finish their tiles in-kernel: no partial slabs for the consumer
     } else if (*nt >> 8) {  // tiled hint: the split the kernel will really use
       int tsel = *nt >> 8;
-      gemm_tiled_plan(M, N, K, &tsel, splitk, false);
+      gemm_tiled_plan(M, N, K, &tsel, splitk, glu);
     }
     return;
   }
@@ -2240,7 +2258,7 @@ void gemm_plan(int M, int N, int K, bool w_fp8, int* nt, int* splitk) {
     gemm_stream_plan(std::min(M, 128), N, K, nt, splitk);
   } else {
     int tsel = 0, s = 0;
-    gemm_tiled_plan(M, N, K, &tsel, &s, false);
+    gemm_tiled_plan(M, N, K, &tsel, &s, glu);
     *nt = tsel << 8;
     *splitk = s;
   }
