@@ -1326,10 +1326,42 @@ def _rec_common(q, k, v, state, cu, ctx_lens, state_slots, heads, kv_heads, dim,
     return T, B, torch.empty(T, heads * vdim, dtype=torch.float32, device=q.device)
 
 
-# smallest portion (rows of the step's longest one) that the chunked form takes, by mode. A chunk costs about as much as the walk
-# of so many tokens when 64 sequences fill the chip (ssd 117 us, the walk of 4 139 us; decay 95 us, the walk of 8 63, of 16 101
-# us); a single sequence is faster chunk by chunk from 8 rows on (17 against 47 us).
-LINEAR_CHUNK_MIN = {0: 12, 2: 4}
+# What the sequences of a step cost in the three forms of a matrix-state recurrence, in us, fitted over 950 random steps of each kind
+# (1 - 170 sequences, up to 400 rows, 2 - 64 heads of 16 - 256 x 16 - 128, a third of them behind 1 - 70 single rows; 7 - 15 % off on
+# average, the choice 1 % above the best form). Chunk by chunk: a start, a part that grows with the state's 16-row tiles and one for
+# each 16 rows, for the longest portion and again for all workgroups at 256 at a time. Token by token: a start, the rows of the longest
+# portion, and the numbers of all rows and states; key dimensions above 128 cost more. Single rows apart: a launch and their states.
+# Chunks at every size from a few rows on took up to 4 times the walk where many sequences fill the chip with short portions or narrow
+# values (53 of up to 14 rows, decay, 32 heads 128 x 64: 82 -> 152 us; 59 of up to 7, delta, 32 heads 128 x 32: 71 -> 217), single rows
+# always apart 1.14 times on average over fp32 rows (one beside a portion of two, decay, 16 heads 128 x 128: 13.4 -> 19.3 us). With this
+# choice: 0.55 (decay), 0.28 (ssd) and 0.51 (delta) of the walk's time.
+_REC_COST = {  # (start, part, by tiles, 16 rows, by tiles, workgroups), (start, row, above 128, rows' numbers, columns beside, states', above 128), (launch, numbers)
+    "decay": ((4.22, 0.0, 1.13, 0.628, 0.25, 1.09), (10.4, 0.711, 1.98, 0.198, 14.7, 1.23, 2.63), (3.75, 1.06)),
+    "ssd": ((3.51, 0.718, 0.915, 0.771, 0.103, 0.784), (8.23, 1.52, 1.34, 0.341, 0.0, 1.97, 2.82), (5.48, 0.862)),
+    "delta": ((13.7, 0.35, 0.965, 0.842, 0.291, 1.63), (10.6, 1.37, 1.5, 0.562, 0.0, 2.84, 1.2), (6.99, 1.09)),
+}
+
+
+def _rec_plan(kind, nd, B, T, longest, heads, dim, vdim, step, chunk):
+    """(leading single-row sequences of ``nd`` to take in a launch of their own: all or none, whether the others go chunk by chunk) for
+    B sequences of T rows; ``step`` and ``chunk``: whether those forms take the step at all."""
+    if nd == B:
+        return (nd if step else 0), False
+    (c0, c1, c2, c3, c4, c5), (w0, w1, w2, w3, w4, w5, w6), (s0, s1) = _REC_COST[kind]
+    tiles = 2 if dim <= 32 else 4 if dim <= 64 else 8 if dim <= 128 else 16
+    wide = (w2, w6) if dim > 128 else (1, 1)
+    once, rows16, wgs = c1 + c2 * tiles, c3 + c4 * tiles, heads * -(-vdim // 64) / 256
+
+    def form(b, t):
+        walk = w0 + longest * w1 * wide[0] + 1e-6 * heads * dim * (w3 * t * (vdim + w4) + w5 * b * vdim) * wide[1]
+        us = c0 + once + longest / 16 * rows16 + c5 * wgs * (b * once + t / 16 * rows16)
+        return (us, True) if chunk and us < walk else (walk, False)
+    us, chunks = form(B, T)
+    if step and nd:
+        rest, rest_chunks = form(B - nd, T - nd)
+        if rest + s0 + s1 * 1e-6 * nd * heads * dim * vdim < us:
+            return nd, rest_chunks
+    return 0, chunks
 
 
 def _linear_forms(mode, q, k, v, dt, args, state, cu, ctx_lens, state_slots, out, heads, groups, dim, vdim, silu, max_qlen,
@@ -1341,17 +1373,19 @@ def _linear_forms(mode, q, k, v, dt, args, state, cu, ctx_lens, state_slots, out
     nd = B if max_qlen == 1 and q.shape[0] == B else int(num_decode)  # (fewer rows: some portions are empty)
     _check(0 <= nd <= B and (nd < B or q.shape[0] == B), "num_decode outside the step")
     dt_ptr, lddt = (dt.data_ptr(), dt.stride(0)) if dt is not None else (0, 0)
-    if not (L.linear_step_ok(dim, vdim) and state.data_ptr() % 16 == 0 and (dt is None or dt.dtype == q.dtype)):
-        nd = 0
+    same = dt is None or dt.dtype == q.dtype
     qkv = (q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), k.stride(0), v.stride(0))
+    nd, chunk = _rec_plan("decay" if mode == 0 else "ssd", nd, B, q.shape[0], max_qlen, heads, dim, vdim,
+                          same and state.data_ptr() % 16 == 0 and L.linear_step_ok(dim, vdim),
+                          same and max_qlen > 1 and q.dtype == torch.bfloat16 and L.linear_chunk_ok(dim, vdim)
+                          and not any(p % 16 for p in qkv[:2]) and not any(x % 8 for x in qkv[3:5]))
 
     def seqs(b):
         return (state.data_ptr(), cu.data_ptr() + 4 * b, ctx_lens.data_ptr() + 4 * b, state_slots.data_ptr() + 4 * b,
                 out.data_ptr())
     if nd:
         L.linear_step(mode, *qkv, dt_ptr, lddt, *args, *seqs(0), nd, heads, groups, dim, vdim, int(silu), _dt(q, "q"), st)
-    if nd < B and max_qlen >= LINEAR_CHUNK_MIN[mode] and q.dtype == torch.bfloat16 and L.linear_chunk_ok(dim, vdim) and \
-            (dt is None or dt.dtype == q.dtype) and not any(p % 16 for p in qkv[:2]) and not any(x % 8 for x in qkv[3:5]):
+    if chunk:
         L.linear_chunk(mode, *qkv, dt_ptr, lddt, *args, *seqs(nd), B - nd, heads, groups, dim, vdim, int(silu), st)
         return B
     return nd
@@ -1417,9 +1451,6 @@ def delta_recurrence(q, k, v, a, b_, A_log, dt_bias, state, cu, ctx_lens, state_
     return out
 
 
-# smallest portion (rows of the step's longest one) of fp32 rows that the chunked form takes: 64 sequences of 16 heads 128 x 128
-# take 121 us chunk by chunk whatever their portions up to 16 rows, 107 us token by token with 4 rows and 140 us with 8
-DELTA32_CHUNK_MIN = 6
 _DELTA_MFMA = os.environ.get("LLMSS_DELTA_MFMA", "1") != "0"  # 0: portions token by token (A/B runs)
 
 
@@ -1442,14 +1473,17 @@ def delta_mix(q, k, v, a, b_, A_log, dt_bias, state, cu, ctx_lens, state_slots, 
     rows = q.dtype == k.dtype == v.dtype
     same = rows and q.dtype == a.dtype == out.dtype
     wide = rows and q.dtype == torch.float32  # rows in 32 bits beside projections of either type
-    if not (a.dtype == out.dtype and (same or wide) and L.delta_step_ok(dim, vdim) and state.data_ptr() % 16 == 0):
-        nd = 0
     qkv = (q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), k.stride(0), v.stride(0))
     ab = (a.data_ptr(), b_.data_ptr(), a.stride(0), A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr())
     o = None
-    wide = wide and L.delta_chunk32_ok(dim, vdim) and max_qlen >= DELTA32_CHUNK_MIN
-    chunk = (wide or same and q.dtype == torch.bfloat16 and max_qlen > 0 and L.delta_chunk_ok(dim, vdim)) and _DELTA_MFMA \
-        and not any(p % 16 for p in qkv[:2]) and not any(x * q.element_size() % 16 for x in qkv[3:5])
+    step = a.dtype == out.dtype and (same or wide) and L.delta_step_ok(dim, vdim) and state.data_ptr() % 16 == 0
+    chunk = max_qlen > 0 and _DELTA_MFMA and not any(p % 16 for p in qkv[:2]) \
+        and not any(x * q.element_size() % 16 for x in qkv[3:5])
+    if wide:
+        nd, chunk = _rec_plan("delta", nd, B, T, max_qlen, heads, dim, vdim, step, chunk and max_qlen > 1 and L.delta_chunk32_ok(dim, vdim))
+    else:
+        nd = nd if step else 0
+        chunk = chunk and same and q.dtype == torch.bfloat16 and L.delta_chunk_ok(dim, vdim)
     if nd < B and not chunk:
         o = delta_recurrence(q, k, v, a, b_, A_log, dt_bias, state, cu, ctx_lens, state_slots, heads, kv_heads, dim, vdim, nd)
     else:
