@@ -1649,12 +1649,14 @@ bool gemm_tuned_get(int M, int N, int K, bool glu, int kind, int* nt_hint, int* 
 // autotuner. Leaves the hints at 0 where the older static rules below are still the better ones.
 //
 // M <= 64: the K-split-wave decode kernel (gemm_dec.hip) on column tiles of 16 - 64, or, for 33 - 64 rows and more than 8192 columns,
-// tiles of 64 x 96 and 64 x 128, where a cost model expects the cheapest to be 1.15 times faster than the older rules (1.25 up to 16 rows).
+// tiles of 64 x 96 and 64 x 128, where a cost model expects the cheapest to be 1.15 times faster than the older rules (1.25 up to 16 rows; or
+// just faster, from 17 rows on, where those need a second launch for their split sums and K is at most 5120, so that X in every tile
+// costs little).
 // A wave of 256 workgroups takes the bytes that one asks for - its weights, and X once more for every tile, which is what narrow
 // products with a long K pay for - at what a CU gets, or all their weights at what the chip gets, whichever is longer. The older
-// rules are priced likewise. Constants fitted over 1030 random shapes of 256 - 70000 columns and K of 256 - 16000 (9 - 13 % off on
-// average, the choice 1.6 - 2.7 % above the best of all). Against the older rules: 0.68 of their time up to 16 rows, 0.84 to 32,
-// 0.88 to 64: 4096 x 4096 at one row 13.6 -> 9.6 us, 32000 x 4096 at 23 rows 62 -> 48, 22016 x 4096 at 24 rows 46 -> 35 us; 512 x 11168
+// rules are priced likewise. Constants fitted over 1600 random shapes of 256 - 70000 columns and K of 256 - 16000 (11 - 12 % off on
+// average, the choice 1.5 - 2.7 % above the best of all). Against the older rules: 0.68 of their time up to 16 rows, 0.84 to 32,
+// 0.92 to 64: 4096 x 4096 at one row 13.6 -> 9.6 us, 32000 x 4096 at 23 rows 62 -> 48, 22016 x 4096 at 24 rows 46 -> 35 us; 512 x 11168
 // SwiGLU at 32 rows (14.0 against 35.6 us) and 18368 x 816 at 17 (13.8, 21.3) stay. From 33 rows on products below 3072 columns keep
 // the 64 x 64 tiles (2048 x 4096 at 64 rows: 12.2 against 14.7 us). Tiles of 96 columns are for one wave of them (22016 x 4096 SwiGLU at
 // 64 rows: 53 -> 39 us); one of the two taken for every product of more than 16384 columns lost to the older rules where a second wave
@@ -1677,10 +1679,11 @@ static constexpr TileCost kTileCost[] = {
     {8 | 32 | 512, 128, 128, 1, 0.70, 0.70}, {11 | 32 | 512, 64, 128, 1, 0.41, 0.41}, {11 | 16, 64, 128, 2, 0.64, 0.44},
 };
 struct DecCost {
-  double start, cu, x, wave, chip;  // us; bytes per us and CU; a row of X against one of W; us per wave of workgroups; bytes per us
+  // us; bytes per us and CU; a row of X against one of W; us per wave of workgroups; bytes per us; what a CU gets more beside idle ones
+  double start, cu, x, wave, chip, spare;
 };
 static constexpr DecCost kDecCost[] = {  // up to 16, 32, 64 rows
-    {2.5, 37.5e3, 0.72, 1.17, 4.58e6}, {1.33, 34.1e3, 0.404, 2.61, 6.28e6}, {1.33, 29.8e3, 0.382, 3.06, 4.54e6}};
+    {2.5, 37.5e3, 0.72, 1.17, 4.58e6, 0}, {1.66, 30.4e3, 0.382, 2.37, 10.1e6, 0.231}, {1.74, 24.7e3, 0.313, 2.75, 5.32e6, 0.242}};
 struct OlderCost {  // of 17 - 64 rows: us per 64 of k on tiles of 64, 128 and 256 columns; bytes per us; the same of slabs; us for their sum
   double s64, s128, s256, chip, slab, sum;
 };
@@ -1691,9 +1694,11 @@ struct WideCost {  // the 64-row tiles of wide products, as DecCost but for us p
   double start, step, wave, chip;
 };
 static constexpr WideCost kWideCost[] = {{15 | 32, 96, 3.43, 0.511, 1.17, 6.19e6}, {11 | 32, 128, 0.02, 0.587, 5.44, 5.40e6}};
-// waves of 256 workgroups: one of them takes `one` us, its share of the chip's rate `read`
-static double waves_us(int wgs, double one, double read) {
-  return wgs / 256 * std::max(one, 256 * read) + (wgs % 256 ? std::max(one, wgs % 256 * read) : 0.0);
+// waves of 256 workgroups: each takes `us` of its workgroups, and at least `read` for each of them, its share of the chip's rate
+template <typename F>
+static double waves_us(int wgs, double read, F us) {
+  const int rest = wgs % 256;
+  return (wgs >= 256 ? wgs / 256 * std::max(us(256), 256 * read) : 0.0) + (rest ? std::max(us(rest), rest * read) : 0.0);
 }
 static int tile_dims(int tsel, int* bm, int* bn);
 static int tiles_of(int M, int N, int bm, int bn);
@@ -1710,7 +1715,7 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
   if (M <= 64) {
     if (M > 32 && N < 3072) return;
     const double bytes = 2.0 * N * K, slab = 8.0 * M * N / 2.5e6;
-    double older;
+    double older, faster = M <= 16 ? 1.25 : 1.15;
     if (M <= 16) {
       int nt, s;
       gemm_stream_plan(M, N, K, &nt, &s);
@@ -1723,6 +1728,7 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
       const double step = (t & 15) == 4 ? c.s256 : (bn == 64 ? c.s64 : c.s128);
       older = 4.71 + std::max(((K + 63) / 64 + s - 1) / s * step, bytes / c.chip);
       if (s > 1) older += s * 8.0 * M * N / c.slab + (slabs ? 0.0 : c.sum);
+      if (s > 1 && !slabs && K <= 5120) faster = 1.0;  // (else two launches, the second waiting for the first)
     }
     const DecCost& c = kDecCost[M <= 16 ? 0 : M <= 32 ? 1 : 2];
     double best = 0;
@@ -1731,18 +1737,21 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
       if (s > 1 && (K / s < 256 || (int64_t)s * M * N * 4 > ws_bytes)) break;
       for (int bn = 64; bn >= 16; bn -= 16) {
         if (glu && bn % 32) continue;
-        const double one = (double)K / s * (bn + c.x * M) * 2 / c.cu + c.wave, read = (double)K / s * bn * 2 / c.chip;
-        const double t = c.start + waves_us((N + bn - 1) / bn * s, one, read) + (s > 1 ? s * slab : 0.0);
+        const double t = c.start + (s > 1 ? s * slab : 0.0) +
+                         waves_us((N + bn - 1) / bn * s, (double)K / s * bn * 2 / c.chip, [&](int n) {
+                           return (double)K / s * (bn + c.x * M) * 2 / (c.cu * (1 + c.spare * (256 - n) / 256)) + c.wave;
+                         });
         if (!code || t < best) best = t, code = bn / 16 | 32 | 1024, sp = s;
       }
     }
     if (M > 32 && N > 8192 && !slabs) {
       for (const WideCost& w : kWideCost) {
-        const double t = w.start + waves_us((N + w.bn - 1) / w.bn, (K + 63) / 64 * w.step + w.wave, 2.0 * K * w.bn / w.chip);
+        const double t = w.start + waves_us((N + w.bn - 1) / w.bn, 2.0 * K * w.bn / w.chip,
+                                            [&](int) { return (K + 63) / 64 * w.step + w.wave; });
         if (t < best) best = t, code = w.tsel;
       }
     }
-    if (!code || best * (M <= 16 ? 1.25 : 1.15) > older) return;
+    if (!code || best * faster > older) return;
     *nt_hint = code << 8;
     *split = sp;
     return;

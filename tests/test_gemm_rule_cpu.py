@@ -11,7 +11,7 @@ DEC = 1024  # the hint bit of the decode kernel
     (20, 23200, 1136, False),  # 18.4 against 52.2: slabs of a wide product
     (64, 23200, 1136, False),  # 21.9, 65.1
     (17, 24992, 288, False),  # 8.6, 22.7
-    (17, 10560, 7776, True),  # 37.9, 37.7 on 48 columns and K in two (55.1 on 16 columns)
+    (17, 10560, 7776, False),  # 37.5, 55.1
     (48, 20672, 2272, False),  # 32.0, 41.8
     (1, 4096, 4096, True),  # 13.6, 9.6
     (1, 1600, 6400, True),
