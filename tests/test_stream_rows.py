@@ -38,7 +38,8 @@ def test_stream_add_norm(S, T, W, rms, dtype, out):
     assert ((h.double() - want).abs() <= e).all()
 
 
-@pytest.mark.parametrize("T,F", [(1, 8), (3, 2040), (2, 2048), (5, 2056), (2, 5632), (3, 100), (2, 7)])
+@pytest.mark.parametrize("T,F", [(1, 8), (3, 2040), (2, 2048), (5, 2056), (2, 5632), (3, 100), (2, 7),
+                                 (4096, 256), (4097, 264), (514, 2040), (512, 2048), (511, 2056), (187, 5632), (8192, 200)])
 @pytest.mark.parametrize("act", ["gelu_tanh", "silu"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_glu_act(T, F, act, dtype):
