@@ -1,9 +1,11 @@
 // Prompt GEMM (bf16, K % 64 == 0): Y[M, N] = epilogue(X[M, K] . W[N, K]^T) on 256 x 256 tiles by FOUR waves, a wave per SIMD with a
 // 128 x 128 part of the tile.
 //
-// Bound by the matrix units' power: with loads and epilogue taken out, 64 of k take a wave of 256 tiles 1.27 us, far over the 0.85 us of
-// the issue rate at 2.4 GHz, and 1.5 us as it stands. Per 64 of k a wave reads (128 + 128) x 64 for 128 products, half of what
-// eight waves read together, and the reads are free behind them. What costs is the loads and the epilogue:
+// Bound by the matrix units at the clock that the chip holds under them: over 8192 x 12288 x 4096 it is 1.43 - 1.93 GHz (GRBM_GUI_ACTIVE
+// over the launch's time; 2.4 nominal) and the matrix units are busy for 67 - 73 % of the cycles (SQ_VALU_MFMA_BUSY_CYCLES). With loads
+// and epilogue taken out, 64 of k take a wave of 256 tiles 1.27 us (0.85 us of issue at 2.4 GHz), and 1.5 us as it stands. Per 64
+// of k a wave reads (128 + 128) x 64 for 128 products, half of what eight waves read together, and the reads are free behind them. What
+// costs is the loads and the epilogue:
 // - a step's loads are issued 1.5 (X) and 1 (W) steps before the barrier that waits for them, by count. With a step's distance of less than
 //   one (two buffers) it took 1.63 - 1.84 us; a ring of four 32-k buffers, with more distance but rows of 64 bytes, 1.6 - 1.75 us.
 // - 42 us a tile with stores of 64 bytes a row straight from the accumulators, 20 us through LDS with the activations' code
