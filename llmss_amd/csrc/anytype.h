@@ -21,6 +21,28 @@ struct El<bf16_t> {
   static __device__ __forceinline__ void st(bf16_t* p, float v) { *p = f2bf(v); }
 };
 
+// Four neighbouring numbers of a row, at a multiple of four
+template <typename T>
+__device__ __forceinline__ f32x4 ld4(const T* p) {
+  if constexpr (sizeof(T) == 4) return *reinterpret_cast<const f32x4*>(p);
+  const u16x4 q = *reinterpret_cast<const u16x4*>(p);
+  return f32x4{bf2f(q[0]), bf2f(q[1]), bf2f(q[2]), bf2f(q[3])};
+}
+template <typename T>
+__device__ __forceinline__ void st4(T* p, f32x4 v) {
+  if constexpr (sizeof(T) == 4) *reinterpret_cast<f32x4*>(p) = v;
+  else *reinterpret_cast<u16x4*>(p) = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
+}
+
+// x as the sum of three bf16 numbers (cut off, not rounded: 8 bits each, 24 together, nothing left over), into place j of each
+__device__ __forceinline__ void split3(float x, int j, s16x8& h, s16x8& m, s16x8& l) {
+  const float a = __uint_as_float(__float_as_uint(x) & 0xffff0000u), y = x - a;
+  const float b = __uint_as_float(__float_as_uint(y) & 0xffff0000u), z = y - b;
+  h[j] = (short)(__float_as_uint(a) >> 16);
+  m[j] = (short)(__float_as_uint(b) >> 16);
+  l[j] = (short)(__float_as_uint(z) >> 16);
+}
+
 // dtype codes shared with the Python launchers: 0 = bf16, 1 = fp32
 #define DISPATCH_T(code, T, ...)                    \
   do {                                              \

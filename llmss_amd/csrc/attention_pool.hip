@@ -45,18 +45,6 @@ __global__ __launch_bounds__(256) void rope_pairs_cache_kernel(const T* __restri
     for (int i = threadIdx.x; i < nv; i += blockDim.x) vc[slot * nv + i] = row[off_v + i];
 }
 
-template <typename T>
-__device__ __forceinline__ f32x4 rope_ld4(const T* p) {
-  if constexpr (sizeof(T) == 4) return *reinterpret_cast<const f32x4*>(p);
-  const u16x4 q = *reinterpret_cast<const u16x4*>(p);
-  return f32x4{bf2f(q[0]), bf2f(q[1]), bf2f(q[2]), bf2f(q[3])};
-}
-template <typename T>
-__device__ __forceinline__ void rope_st4(T* p, f32x4 v) {
-  if constexpr (sizeof(T) == 4) *reinterpret_cast<f32x4*>(p) = v;
-  else *reinterpret_cast<u16x4*>(p) = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
-}
-
 // The same four numbers (two pairs) an access; in steps of few rows a row is spread over gridDim.y workgroups, so that a thread has one
 // access to wait for. 8192 rows of 2048 + 2 x 1024, bf16: 55 -> 28 us, 33 rows 10 -> 5 us.
 template <typename T>
@@ -74,20 +62,20 @@ __global__ __launch_bounds__(256) void rope_pairs_vec_kernel(const T* __restrict
   for (int e = (blockIdx.y * 256 + threadIdx.x) * 4; e < nq + nk + nv; e += gridDim.y * 1024) {
     if (e >= nq + nk) {
       const int i = e - nq - nk;
-      if (slot >= 0) rope_st4(vc + slot * nv + i, rope_ld4(row + off_v + i));
+      if (slot >= 0) st4(vc + slot * nv + i, ld4(row + off_v + i));
       continue;
     }
     const bool isq = e < nq;
     const int i = isq ? e : e - nq;
     const int d = i % dim;
-    f32x4 v = rope_ld4(row + (isq ? off_q : off_k) + i);
+    f32x4 v = ld4(row + (isq ? off_q : off_k) + i);
     if (d < rdims) {
       const f32x4 a = *reinterpret_cast<const f32x4*>(ang + d);
       v = f32x4{fmaf(v[0], a[0], -v[1] * a[1]), fmaf(v[1], a[0], v[0] * a[1]), fmaf(v[2], a[2], -v[3] * a[3]),
                 fmaf(v[3], a[2], v[2] * a[3])};
     }
     if (isq) *reinterpret_cast<f32x4*>(qout + (int64_t)t * nq + i) = v;
-    else if (slot >= 0) rope_st4(kc + slot * nk + i, v);
+    else if (slot >= 0) st4(kc + slot * nk + i, v);
   }
 }
 

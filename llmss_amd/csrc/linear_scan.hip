@@ -163,19 +163,9 @@ void launch_linear_step(int mode, const void* q, const void* k, const void* v, i
 }
 
 // ------------------------------------------------------------------------------------------------ portions
-__device__ __forceinline__ f32x4 lin_ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
-
-// x as the sum of three bf16 numbers (cut off, not rounded: 8 bits each, 24 together, nothing left over)
-struct Split3 {
+struct Split3 {  // eight numbers, each the sum of three
   s16x8 h, m, l;
 };
-__device__ __forceinline__ void lin_split3(float x, int j, Split3& r) {
-  const float h = __uint_as_float(__float_as_uint(x) & 0xffff0000u), y = x - h;
-  const float m = __uint_as_float(__float_as_uint(y) & 0xffff0000u), z = y - m;
-  r.h[j] = (short)(__float_as_uint(h) >> 16);
-  r.m[j] = (short)(__float_as_uint(m) >> 16);
-  r.l[j] = (short)(__float_as_uint(z) >> 16);
-}
 __device__ __forceinline__ f32x4 lin_mfma3(const s16x8& a, const Split3& b, f32x4 c) {
   c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b.l, c, 0, 0, 0);
   c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b.m, c, 0, 0, 0);
@@ -390,7 +380,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
       } else {
         f32x4 a[KT];
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) a[kt] = lin_ld4(&Qs[(16 * w + li) * LDK + 16 * kt + 4 * g]);
+        for (int kt = 0; kt < KT; ++kt) a[kt] = ld4(&Qs[(16 * w + li) * LDK + 16 * kt + 4 * g]);
 #pragma unroll
         for (int ct = 0; ct < 4; ++ct) {
           if (ct > w) continue;
@@ -401,7 +391,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
           for (int kt = 0; kt < KT; kt += NCH) {
             f32x4 x[NCH];
 #pragma unroll
-            for (int n = 0; n < NCH; ++n) x[n] = lin_ld4(&Ks[(16 * ct + li) * LDK + 16 * (kt + n) + 4 * g]);
+            for (int n = 0; n < NCH; ++n) x[n] = ld4(&Ks[(16 * ct + li) * LDK + 16 * (kt + n) + 4 * g]);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -434,7 +424,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
       for (int ks = 0; ks < KT / 2; ++ks) {
         Split3 x;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) lin_split3(S[2 * ks + (j >> 2)][j & 3], j, x);
+        for (int j = 0; j < 8; ++j) split3(S[2 * ks + (j >> 2)][j & 3], j, x.h, x.m, x.l);
 #pragma unroll
         for (int rt = 0; rt < 4; ++rt) {
           if (rt >= nb) continue;
@@ -453,7 +443,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
         for (int kt = 0; kt < KT; kt += NCH) {
           f32x4 x[NCH];
 #pragma unroll
-          for (int n = 0; n < NCH; ++n) x[n] = lin_ld4(&Qs[(16 * rt + li) * LDK + 16 * (kt + n) + 4 * g]);
+          for (int n = 0; n < NCH; ++n) x[n] = ld4(&Qs[(16 * rt + li) * LDK + 16 * (kt + n) + 4 * g]);
 #pragma unroll
           for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -466,7 +456,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
     f32x4 vw[4];
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
-      const f32x4 g4 = lin_ld4(&gt[16 * rt + 4 * g]), w4 = lin_ld4(&ws[16 * rt + 4 * g]);
+      const f32x4 g4 = ld4(&gt[16 * rt + 4 * g]), w4 = ld4(&ws[16 * rt + 4 * g]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         o[rt][i] *= g4[i];
@@ -485,7 +475,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
         if (2 * ks >= nb) continue;
         Split3 x;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) lin_split3(vw[2 * ks + (j >> 2)][j & 3], j, x);
+        for (int j = 0; j < 8; ++j) split3(vw[2 * ks + (j >> 2)][j & 3], j, x.h, x.m, x.l);
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) {
           const bf16_t* p = &Ks[(32 * ks + 4 * g + (li >> 2)) * LDK + 16 * kt + 4 * (li & 3)];
@@ -522,7 +512,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
       f32x4 in = {0.f, 0.f, 0.f, 0.f};  // the chunk's own part, summed apart from the state's
 #pragma unroll
       for (int m = 0; m <= rt; ++m) {
-        const f32x4 a = lin_ld4(&Ps[(16 * rt + li) * LDP + 16 * m + 4 * g]);
+        const f32x4 a = ld4(&Ps[(16 * rt + li) * LDP + 16 * m + 4 * g]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) in = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], v[m][i], in, 0, 0, 0);
       }

@@ -53,24 +53,6 @@ struct ResidArgs {
   int H;
 };
 
-template <typename T>
-__device__ __forceinline__ f32x4 ld4(const T* p);
-template <>
-__device__ __forceinline__ f32x4 ld4<float>(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
-template <>
-__device__ __forceinline__ f32x4 ld4<bf16_t>(const bf16_t* p) {
-  const u16x4 v = *reinterpret_cast<const u16x4*>(p);
-  return f32x4{bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3])};
-}
-template <typename T>
-__device__ __forceinline__ void st4(T* p, f32x4 v);
-template <>
-__device__ __forceinline__ void st4<float>(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
-template <>
-__device__ __forceinline__ void st4<bf16_t>(bf16_t* p, f32x4 v) {
-  *reinterpret_cast<u16x4*>(p) = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
-}
-
 template <typename T, int V>  // V = elements per lane and access: 4 (vector) or 1
 __global__ __launch_bounds__(256) void resid_add_norm_kernel(ResidArgs p) {
   __shared__ float red[16];

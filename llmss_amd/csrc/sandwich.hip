@@ -460,15 +460,9 @@ __global__ __launch_bounds__(512, NT <= 16 ? 4 : 2) void token_side_rows_kernel(
   const bf16_t* wg = (const bf16_t*)s.wg;
   const bf16_t* wp = (const bf16_t*)s.wp;
   float* xr = p.x + (int64_t)t * W;
-  auto split = [](const float* v, s16x8& h, s16x8& m, s16x8& l) {  // cut off, not rounded: 8 bits each
+  auto split = [](const float* v, s16x8& h, s16x8& m, s16x8& l) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float a = __uint_as_float(__float_as_uint(v[i]) & 0xffff0000u), b = v[i] - a;
-      const float c = __uint_as_float(__float_as_uint(b) & 0xffff0000u);
-      h[i] = (short)(__float_as_uint(a) >> 16);
-      m[i] = (short)(__float_as_uint(c) >> 16);
-      l[i] = (short)(__float_as_uint(b - c) >> 16);
-    }
+    for (int i = 0; i < 8; ++i) split3(v[i], i, h, m, l);
   };
   f32x4 acc[DT];
 #pragma unroll

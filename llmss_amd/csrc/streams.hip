@@ -108,19 +108,6 @@ __global__ __launch_bounds__(256) void stream_add_norm_kernel(float* __restrict_
     El<TH>::st(h + (int64_t)t * ldh + col, (u_s[col] - mean) * inv * El<T>::ld(w + col));
 }
 
-// Four neighbouring numbers of a row
-template <typename T>
-__device__ __forceinline__ f32x4 ld4(const T* p) {
-  if constexpr (sizeof(T) == 4) return *reinterpret_cast<const f32x4*>(p);
-  const u16x4 q = *reinterpret_cast<const u16x4*>(p);
-  return f32x4{bf2f(q[0]), bf2f(q[1]), bf2f(q[2]), bf2f(q[3])};
-}
-template <typename T>
-__device__ __forceinline__ void st4(T* p, f32x4 v) {
-  if constexpr (sizeof(T) == 4) *reinterpret_cast<f32x4*>(p) = v;
-  else *reinterpret_cast<u16x4*>(p) = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
-}
-
 // The same for up to four streams of rows of up to 4096: a thread keeps NC times four columns of every stream in registers, all
 // loads are issued before the first is used, and nothing passes through LDS but the two sums. The kernel above, with a load of four
 // bytes waited for at a time, is bound by latency: 8192 rows of 2048, two streams, bf16: 136 -> 59 us (5.7 TB/s).
