@@ -18,7 +18,7 @@ __device__ __forceinline__ int contain(f32x4 (&u)[4], f32x4 (&o)[4], int g) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) z = fmaf(u[r][i], 0.f, z);
   int bad = 64;
-  if (__any(z != z)) {
+  if (__builtin_expect(__any(z != z), 0)) {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll

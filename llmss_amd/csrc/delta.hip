@@ -961,12 +961,14 @@ __global__ __launch_bounds__(256, KT <= 2 ? 2 : 1) void delta_chunk32_kernel(Del
         }
     }
   }
+  int r0 = 4 * g;
+  asm volatile("" : "+v"(r0));  // (the rows anew: which of them the state has would be kept in spilled registers through the loop)
   if (col < vdim) {
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r = 16 * kt + 4 * g + i;
+        const int r = r0 + 16 * kt + i;
         if (r < dim) sp[(int64_t)r * vdim + col] = S[kt][i];
       }
   }

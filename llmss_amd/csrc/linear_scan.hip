@@ -533,13 +533,19 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
   for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) z = fmaf(S[kt][i], 0.f, z);
-  if (__any(z != z)) linear_mend<MODE>(A, h, b, blockIdx.y * 64 + 16 * w, __ballot(z != z), lane);
+  if (__builtin_expect(__any(z != z), 0)) {
+    linear_mend<MODE>(A, h, b, blockIdx.y * 64 + 16 * w, __ballot(z != z), lane);
+    // (its loads and stores end here: left open, each store of the state below waits for the one before it, on the usual path too)
+    __builtin_amdgcn_s_waitcnt(0x0070);
+  }
+  int r0 = 4 * g;
+  asm volatile("" : "+v"(r0));  // (the rows anew: those of the state's loads, kept in scratch through the loop, cost a wait for each store)
   if (col < vdim) {
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r = 16 * kt + 4 * g + i;
+        const int r = r0 + 16 * kt + i;
         if (r < dim) sp[(int64_t)r * vdim + col] = S[kt][i];
       }
   }
