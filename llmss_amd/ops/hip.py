@@ -1326,19 +1326,19 @@ def _rec_common(q, k, v, state, cu, ctx_lens, state_slots, heads, kv_heads, dim,
     return T, B, torch.empty(T, heads * vdim, dtype=torch.float32, device=q.device)
 
 
-# What the sequences of a step cost in the three forms of a matrix-state recurrence, in us, fitted over 950 random steps of each kind
-# (1 - 170 sequences, up to 400 rows, 2 - 64 heads of 16 - 256 x 16 - 128, a third of them behind 1 - 70 single rows; 7 - 15 % off on
+# What the sequences of a step cost in the three forms of a matrix-state recurrence, in us, fitted over 670 random steps of each kind
+# (1 - 170 sequences, up to 400 rows, 2 - 64 heads of 16 - 256 x 16 - 128, a third of them behind 1 - 70 single rows; 6 - 15 % off on
 # average, the choice 1 % above the best form). Chunk by chunk: a start, a part that grows with the state's 16-row tiles and one for
 # each 16 rows, for the longest portion and again for all workgroups at 256 at a time. Token by token: a start, the rows of the longest
 # portion, and the numbers of all rows and states; key dimensions above 128 cost more. Single rows apart: a launch and their states.
 # Chunks at every size from a few rows on took up to 4 times the walk where many sequences fill the chip with short portions or narrow
 # values (53 of up to 14 rows, decay, 32 heads 128 x 64: 82 -> 152 us; 59 of up to 7, delta, 32 heads 128 x 32: 71 -> 217), single rows
 # always apart 1.14 times on average over fp32 rows (one beside a portion of two, decay, 16 heads 128 x 128: 13.4 -> 19.3 us). With this
-# choice: 0.55 (decay), 0.28 (ssd) and 0.51 (delta) of the walk's time.
+# choice: 0.52 (decay), 0.26 (ssd) and 0.52 (delta) of the walk's time.
 _REC_COST = {  # (start, part, by tiles, 16 rows, by tiles, workgroups), (start, row, above 128, rows' numbers, columns beside, states', above 128), (launch, numbers)
-    "decay": ((4.22, 0.0, 1.13, 0.628, 0.25, 1.09), (10.4, 0.711, 1.98, 0.198, 14.7, 1.23, 2.63), (3.75, 1.06)),
-    "ssd": ((3.51, 0.718, 0.915, 0.771, 0.103, 0.784), (8.23, 1.52, 1.34, 0.341, 0.0, 1.97, 2.82), (5.48, 0.862)),
-    "delta": ((13.7, 0.35, 0.965, 0.842, 0.291, 1.63), (10.6, 1.37, 1.5, 0.562, 0.0, 2.84, 1.2), (6.99, 1.09)),
+    "decay": ((3.52, 0.688, 0.82, 0.599, 0.265, 1.05), (10.3, 0.714, 2.06, 0.2, 14.7, 1.21, 2.67), (3.76, 1.09)),
+    "ssd": ((1.65, 1.83, 0.816, 0.809, 0.11, 0.57), (7.9, 1.52, 1.33, 0.333, 0.449, 2.19, 2.64), (5.27, 0.976)),
+    "delta": ((13.5, 0.47, 0.861, 0.939, 0.27, 1.67), (10.4, 1.37, 1.5, 0.552, 4.3, 2.79, 1.2), (7.19, 0.836)),
 }
 
 

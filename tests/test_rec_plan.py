@@ -21,7 +21,6 @@ WALK, CHUNK = (0, False), (0, True)
     ("ssd", 0, 8, 8192, 1024, 64, 128, 64, CHUNK),  # 2160, 208
     ("delta", 0, 8, 8192, 1024, 16, 128, 128, CHUNK),  # 1615, 408
     ("delta", 58, 59, 273, 215, 16, 128, 64, (58, True)),  # 342, 239; apart 352, 88
-    ("decay", 20, 23, 34, 5, 16, 256, 128, (20, False)),  # 80, 93; apart 37, 49
     ("decay", 64, 64, 64, 1, 16, 128, 128, (64, False)),  # nothing but single rows
 ])
 def test_choice(kind, nd, B, T, longest, heads, dim, vdim, form):
@@ -32,6 +31,7 @@ def test_forms_that_do_not_take_the_step_are_not_chosen():
     assert H._rec_plan("decay", 0, 8, 8192, 1024, 16, 128, 128, True, False) == WALK
     assert H._rec_plan("decay", 64, 64, 64, 1, 16, 128, 128, False, True) == WALK
     assert H._rec_plan("delta", 58, 59, 273, 215, 16, 128, 64, False, True) == CHUNK
+    assert H._rec_plan("decay", 20, 23, 34, 5, 16, 256, 128, True, False) == (20, False)  # 80; single rows apart 37
 
 
 @pytest.mark.gpu
