@@ -225,9 +225,9 @@ __device__ __forceinline__ void linear_mend(const LinearArgs& A, int h, int b, i
 }
 
 // Bound by the chain of chunks: a prompt step of 8 sequences has one (decay) or two (ssd) workgroups per CU, each 16 dependent
-// chunks. 8 x 1024 tokens: ssd, 64 heads 128 x 64, 2160 us token by token, 310 us with fp32 instructions throughout, 208 us here
+// chunks. 8 x 1024 tokens: ssd, 64 heads 128 x 64, 2160 us token by token, 310 us with fp32 instructions throughout, 182 us here
 // (no workgroup exchanges anything inside a chunk but the scores); decay, 16 heads 128 x 128, 1230 us with its activation pass,
-// 298 us here.
+// 293 us here.
 //
 // Workgroup (head, block of 64 value columns, sequence), 4 waves, the portion's chunks in order. A wave owns 16 value columns:
 // its part of the state lives in registers in the accumulator layout (lane (li, g): column li, rows 16 tile + 4 g + i), and so do
