@@ -1401,10 +1401,11 @@ __global__ __launch_bounds__(256) void gemm_f8f8_kernel(const unsigned char* __r
 
 // decode GEMM (csrc/gemm_dec.hip): hint tile bit 1024 (nt_hint bit 18), tile bits = the BN code, depth bits = ring
 // depth code (2 / 3 / 4 / 4 stages per wave), split_hint = K split over the grid (fp32 slabs for the consumer)
-void launch_gemm_dec(int code, int depth, const bf16_t* X, int64_t ldx, const bf16_t* W, int64_t ldw,
+void launch_gemm_dec(int code, int depth, const bf16_t* X, int64_t ldx, const void* W, int64_t ldw, const float* wscale,
                      const bf16_t* bias, bf16_t* Y, int64_t ldy, float* part, int M, int N, int K, int act, int glu,
                      int split, hipStream_t st, const QkvEpi* qe, int* cnt);
 bool gemm_dec_bn(int code, int* bn);
+bool gemm_dec_f8_ok(int code, int M);
 // the decode GEMM's in-launch combine (hint bit 256 with a split) fits the workspace: [tile][split][64 * bn] fp32
 static bool dec_combine_fits(int N, int tsel, int s, int64_t ws_bytes) {
   int bn;
@@ -1783,10 +1784,52 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
   }
 }
 
+// The same for fp8 weights and up to 32 rows: the decode kernel, priced as above (constants fitted over 420 random shapes of 512 - 60000
+// columns and K of 256 - 16000: 5 - 7 % off on average, its choice of columns and split 0.3 % above the best), instead of the
+// streaming kernel (up to 16 rows) and the 64 x 64 tiles. 0.72 of their time on average: us at 23 rows, 12288 x 4096 24.8 -> 13.7,
+// 22016 x 4096 SwiGLU 39.0 -> 27.6, slabs of 4096 x 11008 18.4 -> 12.6 and of 4096 x 4096 10.0 -> 6.7; at one row 16.1 -> 12.3,
+// 26.3 -> 23.3, 14.3 -> 10.7, 7.2 -> 5.7. The older rules stay where they are faster: many waves of a short K (53344 x 256 at one row
+// 6.7 against 13.6, 57056 x 576 SwiGLU 12.3 and 19.4), and SwiGLU of few columns and a long K, which they split (1856 x 12240 at 15 rows 18.3
+// and 23.6; but 1888 x 6528 at 13 rows 0.63 the other way, where the line lies between).
+struct DecF8Cost {  // as DecCost; slab: bytes of split sums written and read per us, sum: us of their launch
+  double start, cu, x, wave, chip, spare, slab, sum;
+};
+static constexpr DecF8Cost kDecF8Cost[] = {{1.82, 22.3e3, 0.644, 2.05, 4.99e6, 0.415, 100e6, 1.63},
+                                           {1.98, 20.1e3, 0.582, 1.93, 4.38e6, 0.376, 3.94e6, 1.94}};
+static void gemm_static_plan_f8(int M, int N, int K, bool glu, bool slabs, int64_t ws_bytes, int* nt_hint, int* split) {
+  if (M > 32 || N % 8 || K % 16) return;
+  if ((N > 16384 && K < 1024) || (N > 8192 && K < 512) || (glu && N <= 2816 && K >= 6000)) return;
+  if (slabs) {
+    int t = 0, s = 0;
+    if (M <= 16) gemm_stream_plan(M, N, K, &t, &s);
+    else gemm_tiled_plan(M, N, K, &t, &s, glu);
+    slabs = s > 1 && (int64_t)s * M * N * 4 <= ws_bytes;
+  }
+  const DecF8Cost& c = kDecF8Cost[M > 16];
+  const int k = (K + 127) / 128 * 128;
+  double best = 0;
+  int code = 0, sp = 1;
+  for (int s = slabs ? 2 : 1; s <= (glu ? 1 : 8); s *= 2) {
+    if (s > 1 && (K / s < 512 || (int64_t)s * M * N * 4 > ws_bytes)) break;
+    for (int bn = 64; bn >= 16; bn -= 16) {
+      if (glu && bn % 32) continue;
+      const double kk = (double)k / s;
+      double t = c.start + waves_us((N + bn - 1) / bn * s, kk * bn / c.chip, [&](int n) {
+                   return kk * (bn + c.x * M) / (c.cu * (1 + c.spare * (256 - n) / 256)) + c.wave;
+                 });
+      if (s > 1) t += s * 4.0 * M * N / c.slab + (slabs ? 0.0 : c.sum);
+      if (!code || t < best) best = t, code = bn / 16 | 32 | kDecHint, sp = s;
+    }
+  }
+  if (!code) return;
+  *nt_hint = code << 8;
+  *split = sp;
+}
+
 // Operands that every tile of gemm_static_plan takes: rows of 16-byte alignment, 256 of them within a descriptor of 31 bits
 // (strides below 4.2 M numbers). Anything else keeps the older rules.
-static bool gemm_static_takes(const void* x, int64_t ldx, const void* w, int64_t ldw) {
-  return ldx % 8 == 0 && ldw % 8 == 0 && !(((uintptr_t)x | (uintptr_t)w) & 15) && std::max(ldx, ldw) < (1 << 22);
+static bool gemm_static_takes(bool w_fp8, const void* x, int64_t ldx, const void* w, int64_t ldw) {
+  return ldx % 8 == 0 && ldw % (w_fp8 ? 16 : 8) == 0 && !(((uintptr_t)x | (uintptr_t)w) & 15) && std::max(ldx, ldw) < (1 << 22);
 }
 
 // The plan of a product: its hints, else a tuned plan, else the static one where it applies. Hints of 0 remain where the older
@@ -1794,7 +1837,7 @@ static bool gemm_static_takes(const void* x, int64_t ldx, const void* w, int64_t
 static void gemm_default_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int64_t ws_bytes, bool takes, int* nt_hint,
                               int* split) {
   if (*nt_hint || *split || gemm_tuned_get(M, N, K, glu, w_fp8 ? 1 : 0, nt_hint, split)) return;
-  if (!w_fp8 && takes) gemm_static_plan(M, N, K, glu, slabs, ws_bytes, nt_hint, split);
+  if (takes) (w_fp8 ? gemm_static_plan_f8 : gemm_static_plan)(M, N, K, glu, slabs, ws_bytes, nt_hint, split);
 }
 static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint, int64_t ws_bytes);
 
@@ -1802,7 +1845,7 @@ int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_f
                 const void* bias, void* y, int64_t ldy, int M, int N, int K, int act, bool glu, void* workspace,
                 int64_t ws_bytes, int nt_hint, int split_hint, bool partial_out, hipStream_t st) {
   if (M == 0 || N == 0) return 0;
-  gemm_default_plan(M, N, K, w_fp8, glu, partial_out && !glu && act == 0, ws_bytes, gemm_static_takes(x, ldx, w, ldw), &nt_hint,
+  gemm_default_plan(M, N, K, w_fp8, glu, partial_out && !glu && act == 0, ws_bytes, gemm_static_takes(w_fp8, x, ldx, w, ldw), &nt_hint,
                     &split_hint);
   if (!y && (!partial_out || slabs_of_plan(M, N, K, w_fp8, glu, act, nt_hint, split_hint, ws_bytes) == 0))
     throw std::runtime_error("gemm: this configuration writes the output, but no output buffer was given");
@@ -2018,21 +2061,20 @@ int launch_tiled(const bf16_t* X, int64_t ldx, const void* W, int64_t ldw, const
   const int tsel_raw = tsel;
   int s = split_hint;
   const bool f8 = wscale != nullptr;  // fp8-e4m3 weights (W8A16): half the weight bytes of a decode step
-  if (tsel & kDecHint) {  // K split over the waves (gemm_dec.hip), M <= 64, bf16 weights
-    if (f8) throw std::runtime_error("gemm_dec: bf16 weights only");
+  if (tsel & kDecHint) {  // K split over the waves (gemm_dec.hip), M <= 64
     s = dec_split(M, N, K, split_hint, ws_bytes);
     if (s > 1 && Y && dec_combine_fits(N, tsel, s, ws_bytes)) {  // split-K combined in the launch: finished Y
       int bn;
       gemm_dec_bn(tsel & 15, &bn);
       static constexpr int kDecDepthC[4] = {2, 3, 4, 4};
-      launch_gemm_dec(tsel & 15, kDecDepthC[(tsel >> 4) & 3], X, ldx, (const bf16_t*)W, ldw, B, Y, ldy,
+      launch_gemm_dec(tsel & 15, kDecDepthC[(tsel >> 4) & 3], X, ldx, W, ldw, wscale, B, Y, ldy,
                       (float*)workspace, M, N, K, act, g, s, st, qe, sk_counters((N + bn - 1) / bn));
       return 0;
     }
     if (qe && s > 1) throw std::runtime_error("gemm_dec: the QKV epilogue needs an unsplit or in-launch-combined plan");
     static constexpr int kDecDepth[4] = {2, 3, 4, 4};
     float* part = s > 1 ? (float*)workspace : nullptr;
-    launch_gemm_dec(tsel & 15, kDecDepth[(tsel >> 4) & 3], X, ldx, (const bf16_t*)W, ldw, B, Y, ldy, part, M, N, K,
+    launch_gemm_dec(tsel & 15, kDecDepth[(tsel >> 4) & 3], X, ldx, W, ldw, wscale, B, Y, ldy, part, M, N, K,
                     s > 1 ? 0 : act, s > 1 ? 0 : g, s, st, qe, nullptr);
     if (s > 1 && partial_out && !g && act == 0) return s;
     if (s > 1) {
@@ -2156,7 +2198,7 @@ int launch_tiled(const bf16_t* X, int64_t ldx, const void* W, int64_t ldw, const
 int gemm_partial_slabs(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint, int64_t ws_bytes,
                        const void* x, int64_t ldx, const void* w, int64_t ldw) {
   if (M == 0 || N == 0 || glu || act != 0) return 0;
-  gemm_default_plan(M, N, K, w_fp8, glu, true, ws_bytes, gemm_static_takes(x, ldx, w, ldw), &nt_hint, &split_hint);
+  gemm_default_plan(M, N, K, w_fp8, glu, true, ws_bytes, gemm_static_takes(w_fp8, x, ldx, w, ldw), &nt_hint, &split_hint);
   return slabs_of_plan(M, N, K, w_fp8, glu, act, nt_hint, split_hint, ws_bytes);
 }
 
@@ -2174,7 +2216,7 @@ static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int
   } else {
     int tsel = tiled_hint;
     if (tsel & kDecHint) {
-      if (w_fp8) return 0;  // rejected at launch
+      if (w_fp8 && !gemm_dec_f8_ok(tsel & 15, M)) return 0;  // rejected at launch
       s = dec_split(M, N, K, split_hint, ws_bytes);
       if (dec_combine_fits(N, tsel, s, ws_bytes)) return 0;  // combined in the launch
       return s > 1 ? s : 0;
@@ -2251,7 +2293,7 @@ int launch_gemm_qkv_args(const void* x, int64_t ldx, const void* w, int64_t ldw,
 void gemm_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int* nt, int* splitk) {
   *nt = *splitk = 0;
   const bool tuned = gemm_tuned_get(M, N, K, glu, w_fp8 ? 1 : 0, nt, splitk);
-  if (!tuned && !w_fp8) gemm_static_plan(M, N, K, glu, slabs && !glu, 64 << 20, nt, splitk);
+  if (!tuned) (w_fp8 ? gemm_static_plan_f8 : gemm_static_plan)(M, N, K, glu, slabs && !glu, 64 << 20, nt, splitk);
   if (tuned || *nt) {
     if ((*nt >> 8) & kDecHint) {
       *splitk = ((*nt >> 8) & 256) ? 1 : dec_split(M, N, K, *splitk, INT64_MAX);

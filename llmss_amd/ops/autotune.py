@@ -50,6 +50,8 @@ def candidates(M: int, N: int, K: int, glu: bool, fp8: bool) -> List[Tuple[int, 
     if fp8:  # tiled kernel with fp8 weight tiles (no stream-K / big-tile variants)
         if M > 16:
             out += [((t | d) << 8, s) for t, d in ((3, 16), (3, 32), (2, 16), (2, 32)) for s in splits]
+        if M <= 32:  # K split over the waves of a workgroup (hint bit 1024, csrc/gemm_dec.hip)
+            out += [((code | 32 | 1024) << 8, s) for code in (1, 2, 3, 4) for s in splits if s == 1 or K // s >= 256]
         if M >= 32:  # W8A8: per-token fp8 activations on the MX-fp8 matrix cores (ops/hip.py W8A8_FLAG)
             from .hip import W8A8_FLAG
 

@@ -431,6 +431,48 @@ def test_gemm_dec_k_tail_reads_nothing_past_the_operands(code):
         close(y, R.linear(x.float(), w.float(), None), 2e-2)
 
 
+@pytest.mark.parametrize("code,M,N,K,split", [(1, 1, 96, 16, 1), (1, 16, 200, 128 * 5, 2), (2, 5, 1376, 1600, 3), (2, 17, 4096, 1376, 1),
+                                              (3, 32, 200, 128 * 9 + 112, 4), (4, 23, 2752, 4096, 1), (4, 32, 640, 128 * 3 + 16, 2)])
+def test_gemm_dec_fp8(code, M, N, K, split):
+    """The decode GEMM over e4m3 weights against the dequantised product in fp32: 16 / 32-row variants, ragged N, partial last
+    k-steps, slices without k-steps, strided rows of x; GELU, SwiGLU and slabs. Weights are exact in bf16, so what
+    is off is the order of fp32 sums and the output's rounding (2^-9). A NaN weight stays in its own column: the bytes
+    past a row's end are the next row's."""
+    torch.manual_seed(0)
+    x = rnd(M, K + 24)[:, :K]
+    q, sc = H.quant_fp8_rows(rnd(N, K, scale=K ** -0.5))
+    w = q.view(torch.float8_e4m3fn).float() * sc[:, None]
+    b = rnd(N, scale=0.1)
+    hint, bn = (code | 32 | 1024) << 8, DEC_BN[code]
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
+    close(H.linear(x, q, b, act="gelu_tanh", w_scale=sc, nt_hint=hint, split_hint=split, out=y),
+          R.linear(x.float(), w, b.float(), act="gelu_tanh"), 2e-2)
+    if N % 32 == 0 and (bn % 32 == 0 or min(split, -(-K // 64)) > 1):
+        close(H.linear(x, q, None, glu=True, w_scale=sc, nt_hint=hint, split_hint=split), R.linear(x.float(), w, None, glu=True), 2e-2)
+    H._GEMM_WS.get(64 << 20, x.device).fill_(float("nan"))
+    p = H.linear(x, q, b, w_scale=sc, nt_hint=hint, split_hint=split, partial_ok=True)
+    if isinstance(p, H.PartialSum):
+        p = p.buf[:p.S * M * N].view(p.S, M, N).sum(0) + b.float()
+    close(p, R.linear(x.float(), w, b.float()), 2e-2)
+    q[1::2, 0] = 0x7F
+    y = H.linear(x, q, None, w_scale=sc, nt_hint=hint, split_hint=split)
+    assert torch.isfinite(y[:, 0::2]).all() and torch.isnan(y[:, 1::2]).all()
+
+
+@pytest.mark.parametrize("M,N,K,glu", [(1, 4096, 4096, False), (16, 12288, 4096, False), (23, 22016, 4096, True), (32, 4096, 11008, False),
+                                       (33, 4096, 4096, False), (3, 1856, 12240, True), (2, 53344, 256, False), (9, 328, 528, False)])
+def test_fp8_products_of_few_rows_by_any_plan(M, N, K, glu):
+    """What the plan of an fp8 product chooses on both sides of its lines, against the dequantised product."""
+    torch.manual_seed(0)
+    x = rnd(M, K)
+    q, sc = H.quant_fp8_rows(rnd(N, K, scale=K ** -0.5))
+    ref = R.linear(x.float(), q.view(torch.float8_e4m3fn).float() * sc[:, None], None, glu=glu)
+    close(H.linear(x, q, None, glu=glu, w_scale=sc), ref, 2e-2)
+    if not glu:
+        p = H.linear(x, q, None, w_scale=sc, partial_ok=True)
+        close(p.buf[:p.S * M * N].view(p.S, M, N).sum(0) if isinstance(p, H.PartialSum) else p, ref, 2e-2)
+
+
 @pytest.mark.parametrize("code", [1, 2, 4, 5])
 @pytest.mark.parametrize("split", [1, 2, 3])
 @pytest.mark.parametrize("style,D,rot,nh,nkv", [("none", 64, 0, 25, 25), ("gptj", 256, 64, 4, 4), ("neox", 64, 64, 8, 1)])

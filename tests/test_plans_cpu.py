@@ -106,3 +106,18 @@ def test_prompt_batch_plans_take_the_ping_pong_kernel(M, N, K):
 
     nt, split = H.lib().gemm_plan(M, N, K, False)
     assert (nt >> 8) & 15 == 4 and split == 1, (hex(nt), split)
+
+
+@pytest.mark.parametrize("M,N,K,glu,slabs,dec", [
+    (1, 12288, 4096, False, False, True), (32, 22016, 4096, True, False, True), (33, 22016, 4096, True, False, False),
+    (23, 4096, 11008, False, True, True), (16, 53344, 256, False, False, False), (16, 16384, 1008, False, False, True),
+    (15, 1856, 12240, True, False, False), (13, 2848, 6528, True, False, True)])
+def test_fp8_products_of_few_rows_take_the_decode_kernel(M, N, K, glu, slabs, dec):
+    """Up to 32 rows of fp8 weights: gemm_dec.hip (hint bit 1024), split where the consumer sums slabs that the older plan left
+    too; many waves of a short K and SwiGLU of few columns with a long K keep the older kernels."""
+    from llmss_amd.ops import hip as H
+
+    nt, split = H.lib().gemm_plan(M, N, K, True, glu, slabs)
+    assert bool((nt >> 8) & 1024) == dec, (hex(nt), split)
+    if dec:
+        assert (split > 1) == slabs and ((nt >> 8) & 15) <= 4
