@@ -24,7 +24,10 @@ __device__ __forceinline__ float dpp_f(float x) {
 }
 template <int LPT>
 __device__ __forceinline__ float token_sum(float s) {
-  if constexpr (LPT >= 16) {  // row_ror:8,4,2,1 inside each 16-lane row
+  if constexpr (LPT == 4) {
+    s += dpp_f<0x4e>(s);   // quad_perm [2,3,0,1]
+    s += dpp_f<0xb1>(s);   // quad_perm [1,0,3,2]
+  } else if constexpr (LPT >= 16) {  // row_ror:8,4,2,1 inside each 16-lane row
     s += dpp_f<0x128>(s);
     s += dpp_f<0x124>(s);
     s += dpp_f<0x122>(s);
@@ -42,15 +45,23 @@ __device__ __forceinline__ float token_sum(float s) {
 }
 
 // KV8: the paged cache holds fp8 rows (D e4m3 bytes + fp32 scale at byte D, 16-B tail; reference.py
-// kv_rows_quant): each lane loads 8 bytes per token instead of 16 and the row scales multiply the score
-// (K) and the probability (V) instead of every element.
+// kv_rows_quant); the row scales multiply the score (K) and the probability (V) instead of every element.
+// Groups of one or two heads: 16 bytes a lane, so D / 16 lanes own a token, and the running maximum moves once for
+// UNROLL tokens. 8 bytes a lane, a rescaled accumulator per token and a division per row's address made about 120
+// vector instructions a wave for 4 tokens' K and V (1.1 KB), this about 55. Rows of D + 16 bytes share their 128-byte lines with
+// their neighbours, which other waves read: no non-temporal hint, that fetches a shared line again. 23 sequences of 32 heads to
+// 1777 positions (298 MB): 76 us and 5 for the sum of three partitions -> 61 in one (4.9 TB/s), 64 of 192 positions 28.9 -> 26.5,
+// one of 1777 16.3 -> 11.0. Larger groups keep 8 bytes: their accumulators would not fit beside the rows in flight.
+constexpr int decode_elems(int GB, bool KV8) { return KV8 && GB <= 2 ? 16 : 8; }  // dims a lane holds of a token's row
+
 template <int D, int GB, int UNROLL, bool PIPE = false, bool KV8 = false>
-__global__ __launch_bounds__(256, GB == 1 ? 8 : 1) void attn_decode_kernel(
+__global__ __launch_bounds__(256, (decode_elems(GB, KV8) == 16 ? (GB == 1 ? 4 : 2) : GB == 1 ? 8 : 1)) void attn_decode_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, void* __restrict__ kcv, void* __restrict__ vcv,
     const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ ctx_lens, bf16_t* __restrict__ out,
     int64_t out_stride, float* __restrict__ part_o, float* __restrict__ part_ml, int nh, int nkv, int G, int ngroups,
-    int block_size, int part_size, float scale_log2) {
-  constexpr int LPT = D / 8;
+    int block_size, int block_shift, int part_size, float scale_log2) {
+  constexpr int E = decode_elems(GB, KV8);
+  constexpr int LPT = D / E;
   constexpr int TPW = 64 / LPT;
   constexpr int RB = KV8 ? D + 16 : D;  // cache row, in cache elements (bytes for fp8 rows)
   bf16_t* __restrict__ kc = (bf16_t*)kcv;
@@ -66,31 +77,34 @@ __global__ __launch_bounds__(256, GB == 1 ? 8 : 1) void attn_decode_kernel(
   const int nvalid = min(GB, G - grp * GB);
 
   // q (pre-scaled into the log2 domain)
-  float qv[GB][8];
+  float qv[GB][E];
 #pragma unroll
   for (int h = 0; h < GB; ++h) {
     if (h < nvalid) {
-      u16x8 a = *reinterpret_cast<const u16x8*>(q + b * q_stride + (int64_t)(h0 + h) * D + sub * 8);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) qv[h][j] = bf2f(a[j]) * scale_log2;
+      for (int i = 0; i < E; i += 8) {
+        u16x8 a = *reinterpret_cast<const u16x8*>(q + b * q_stride + (int64_t)(h0 + h) * D + sub * E + i);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) qv[h][i + j] = bf2f(a[j]) * scale_log2;
+      }
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) qv[h][j] = 0.f;
+      for (int j = 0; j < E; ++j) qv[h][j] = 0.f;
     }
   }
-  float m[GB], l[GB], acc[GB][8];
+  float m[GB], l[GB], acc[GB][E];
 #pragma unroll
   for (int h = 0; h < GB; ++h) {
     m[h] = kNegBig; l[h] = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[h][j] = 0.f;
+    for (int j = 0; j < E; ++j) acc[h][j] = 0.f;
   }
 
   const int ctx = min(ctx_lens[b], bt_stride * block_size);  // never index past the block table
   const int start = split * part_size;
   const int end = min(ctx, start + part_size);
   const int* bt = block_tables + (int64_t)b * bt_stride;
-  const int64_t head_off = (int64_t)kvh * block_size * RB + sub * 8;
+  const int64_t head_off = (int64_t)kvh * block_size * RB + sub * E;
   const int64_t page_stride = (int64_t)nkv * block_size * RB;
   constexpr int STEP = 4 * TPW;  // tokens per workgroup-iteration
   const int lend = end;
@@ -110,14 +124,15 @@ __global__ __launch_bounds__(256, GB == 1 ? 8 : 1) void attn_decode_kernel(
     __syncthreads();
   }
   auto kv_addr = [&](int t) -> int64_t {
-    const int pi = t / block_size;
+    const int pi = block_shift >= 0 ? t >> block_shift : t / block_size;  // (a division costs as much as a token's products)
     const int page = lds_pages ? s_pages[pi - pg0] : bt[pi];
-    return page * page_stride + head_off + (int64_t)(t % block_size) * RB;
+    return page * page_stride + head_off + (t - pi * block_size) * RB;
   };
-  // a token's K / V registers: bf16 rows 16 B per lane; fp8 rows 8 B per lane + the row's two scales
+  // a token's K / V registers: bf16 rows 16 B per lane; fp8 rows E bytes per lane + the row's two scales
+  typedef unsigned u32xe __attribute__((ext_vector_type(E / 4)));
   struct KVRegs {
     u16x8 k[UNROLL], v[UNROLL];
-    u32x2 k8[UNROLL], v8[UNROLL];
+    u32xe k8[UNROLL], v8[UNROLL];
     float ks[UNROLL], vs[UNROLL];
   };
   auto load_tokens = [&](int tb, KVRegs& r) {
@@ -125,12 +140,17 @@ __global__ __launch_bounds__(256, GB == 1 ? 8 : 1) void attn_decode_kernel(
     for (int u = 0; u < UNROLL; ++u) {
       const int t = tb + u * STEP;
       const int64_t a = kv_addr(t < lend ? t : start);
-      // read once per step: non-temporal (guide 'nt-weights'; +10-15% on streamed reads)
-      if constexpr (KV8) {
-        r.k8[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(kc8 + a));
-        r.v8[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(vc8 + a));
-        r.ks[u] = *reinterpret_cast<const float*>(kc8 + a - sub * 8 + D);
-        r.vs[u] = *reinterpret_cast<const float*>(vc8 + a - sub * 8 + D);
+      // read once per step: non-temporal (guide 'nt-weights'; +10-15% on streamed reads), but for the rows of 16 bytes a lane
+      if constexpr (E == 16) {
+        r.k8[u] = *reinterpret_cast<const u32xe*>(kc8 + a);
+        r.v8[u] = *reinterpret_cast<const u32xe*>(vc8 + a);
+        r.ks[u] = *reinterpret_cast<const float*>(kc8 + a - sub * E + D);
+        r.vs[u] = *reinterpret_cast<const float*>(vc8 + a - sub * E + D);
+      } else if constexpr (KV8) {
+        r.k8[u] = __builtin_nontemporal_load(reinterpret_cast<const u32xe*>(kc8 + a));
+        r.v8[u] = __builtin_nontemporal_load(reinterpret_cast<const u32xe*>(vc8 + a));
+        r.ks[u] = *reinterpret_cast<const float*>(kc8 + a - sub * E + D);
+        r.vs[u] = *reinterpret_cast<const float*>(vc8 + a - sub * E + D);
       } else {
         r.k[u] = __builtin_nontemporal_load(reinterpret_cast<const u16x8*>(kc + a));
         r.v[u] = __builtin_nontemporal_load(reinterpret_cast<const u16x8*>(vc + a));
@@ -138,38 +158,81 @@ __global__ __launch_bounds__(256, GB == 1 ? 8 : 1) void attn_decode_kernel(
     }
   };
   auto consume = [&](int tb, const KVRegs& r) {
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      const bool ok = tb + u * STEP < lend;
-      float kf[8], vf[8], ks = 1.f, vs = 1.f;
-      if constexpr (KV8) {
-        const f32x2 k0 = __builtin_amdgcn_cvt_pk_f32_fp8(r.k8[u][0], false), k1 = __builtin_amdgcn_cvt_pk_f32_fp8(r.k8[u][0], true);
-        const f32x2 k2 = __builtin_amdgcn_cvt_pk_f32_fp8(r.k8[u][1], false), k3 = __builtin_amdgcn_cvt_pk_f32_fp8(r.k8[u][1], true);
-        const f32x2 v0 = __builtin_amdgcn_cvt_pk_f32_fp8(r.v8[u][0], false), v1 = __builtin_amdgcn_cvt_pk_f32_fp8(r.v8[u][0], true);
-        const f32x2 v2 = __builtin_amdgcn_cvt_pk_f32_fp8(r.v8[u][1], false), v3 = __builtin_amdgcn_cvt_pk_f32_fp8(r.v8[u][1], true);
-        kf[0] = k0[0]; kf[1] = k0[1]; kf[2] = k1[0]; kf[3] = k1[1]; kf[4] = k2[0]; kf[5] = k2[1]; kf[6] = k3[0]; kf[7] = k3[1];
-        vf[0] = v0[0]; vf[1] = v0[1]; vf[2] = v1[0]; vf[3] = v1[1]; vf[4] = v2[0]; vf[5] = v2[1]; vf[6] = v3[0]; vf[7] = v3[1];
-        ks = r.ks[u];
-        vs = r.vs[u];
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) { kf[j] = bf2f(r.k[u][j]); vf[j] = bf2f(r.v[u][j]); }
-      }
+    if constexpr (E == 16) {
 #pragma unroll
       for (int h = 0; h < GB; ++h) {
-        float s = 0.f;
+        float s[UNROLL], mn = m[h];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) s = fmaf(qv[h][j], kf[j], s);
-        s = token_sum<LPT>(s);
-        if constexpr (KV8) s *= ks;
-        if (ok) {
-          const float mn = fmaxf(m[h], s);
-          const float alpha = exp2f(m[h] - mn), p = exp2f(s - mn);
-          l[h] = l[h] * alpha + p;
-          const float pv = KV8 ? p * vs : p;
+        for (int u = 0; u < UNROLL; ++u) {
+          float d0 = 0.f, d1 = 0.f;  // (two chains)
 #pragma unroll
-          for (int j = 0; j < 8; ++j) acc[h][j] = fmaf(acc[h][j], alpha, pv * vf[j]);
-          m[h] = mn;
+          for (int j = 0; j < 4; ++j) {
+            const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8(r.k8[u][j], false), c = __builtin_amdgcn_cvt_pk_f32_fp8(r.k8[u][j], true);
+            d0 = fmaf(qv[h][4 * j], a[0], d0);
+            d1 = fmaf(qv[h][4 * j + 1], a[1], d1);
+            d0 = fmaf(qv[h][4 * j + 2], c[0], d0);
+            d1 = fmaf(qv[h][4 * j + 3], c[1], d1);
+          }
+          s[u] = token_sum<LPT>(d0 + d1) * r.ks[u];
+          if (tb + u * STEP >= lend) s[u] = kNegBig;
+          mn = fmaxf(mn, s[u]);
+        }
+        const float alpha = exp2f(m[h] - mn);
+        m[h] = mn;
+        l[h] *= alpha;
+#pragma unroll
+        for (int j = 0; j < E; ++j) acc[h][j] *= alpha;
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+          const bool ok = tb + u * STEP < lend;
+          const float p = ok ? exp2f(s[u] - mn) : 0.f;
+          l[h] += p;
+          const float pv = ok ? p * r.vs[u] : 0.f;  // (tokens past the end read a token of this range)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8(r.v8[u][j], false), c = __builtin_amdgcn_cvt_pk_f32_fp8(r.v8[u][j], true);
+            acc[h][4 * j] = fmaf(pv, a[0], acc[h][4 * j]);
+            acc[h][4 * j + 1] = fmaf(pv, a[1], acc[h][4 * j + 1]);
+            acc[h][4 * j + 2] = fmaf(pv, c[0], acc[h][4 * j + 2]);
+            acc[h][4 * j + 3] = fmaf(pv, c[1], acc[h][4 * j + 3]);
+          }
+        }
+      }
+      return;
+    } else {
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        const bool ok = tb + u * STEP < lend;
+        float kf[8], vf[8], ks = 1.f, vs = 1.f;
+        if constexpr (KV8) {
+          const f32x2 k0 = __builtin_amdgcn_cvt_pk_f32_fp8(r.k8[u][0], false), k1 = __builtin_amdgcn_cvt_pk_f32_fp8(r.k8[u][0], true);
+          const f32x2 k2 = __builtin_amdgcn_cvt_pk_f32_fp8(r.k8[u][1], false), k3 = __builtin_amdgcn_cvt_pk_f32_fp8(r.k8[u][1], true);
+          const f32x2 v0 = __builtin_amdgcn_cvt_pk_f32_fp8(r.v8[u][0], false), v1 = __builtin_amdgcn_cvt_pk_f32_fp8(r.v8[u][0], true);
+          const f32x2 v2 = __builtin_amdgcn_cvt_pk_f32_fp8(r.v8[u][1], false), v3 = __builtin_amdgcn_cvt_pk_f32_fp8(r.v8[u][1], true);
+          kf[0] = k0[0]; kf[1] = k0[1]; kf[2] = k1[0]; kf[3] = k1[1]; kf[4] = k2[0]; kf[5] = k2[1]; kf[6] = k3[0]; kf[7] = k3[1];
+          vf[0] = v0[0]; vf[1] = v0[1]; vf[2] = v1[0]; vf[3] = v1[1]; vf[4] = v2[0]; vf[5] = v2[1]; vf[6] = v3[0]; vf[7] = v3[1];
+          ks = r.ks[u];
+          vs = r.vs[u];
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) { kf[j] = bf2f(r.k[u][j]); vf[j] = bf2f(r.v[u][j]); }
+        }
+#pragma unroll
+        for (int h = 0; h < GB; ++h) {
+          float s = 0.f;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) s = fmaf(qv[h][j], kf[j], s);
+          s = token_sum<LPT>(s);
+          if constexpr (KV8) s *= ks;
+          if (ok) {
+            const float mn = fmaxf(m[h], s);
+            const float alpha = exp2f(m[h] - mn), p = exp2f(s - mn);
+            l[h] = l[h] * alpha + p;
+            const float pv = KV8 ? p * vs : p;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[h][j] = fmaf(acc[h][j], alpha, pv * vf[j]);
+            m[h] = mn;
+          }
         }
       }
     }
@@ -206,7 +269,7 @@ __global__ __launch_bounds__(256, GB == 1 ? 8 : 1) void attn_decode_kernel(
       const float a = exp2f(m[h] - mn), c = exp2f(mo - mn);
       l[h] = l[h] * a + lo * c;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
+      for (int j = 0; j < E; ++j) {
         const float ao = __shfl_xor(acc[h][j], o, 64);
         acc[h][j] = acc[h][j] * a + ao * c;
       }
@@ -220,7 +283,7 @@ __global__ __launch_bounds__(256, GB == 1 ? 8 : 1) void attn_decode_kernel(
 #pragma unroll
     for (int h = 0; h < GB; ++h) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s_acc[w][h][sub * 8 + j] = acc[h][j];
+      for (int j = 0; j < E; ++j) s_acc[w][h][sub * E + j] = acc[h][j];
       if (sub == 0) { s_ml[w][h][0] = m[h]; s_ml[w][h][1] = l[h]; }
     }
   }
@@ -299,9 +362,10 @@ static void launch_decode_t(const bf16_t* q, int64_t qs, bf16_t* kc, bf16_t* vc,
   const int ngroups = (G + GB - 1) / GB;
   dim3 grid(B, nkv * ngroups, nsplit);
   const float sl2 = scale * kLog2e;
+  const int bshift = bs > 0 && (bs & (bs - 1)) == 0 ? __builtin_ctz(bs) : -1;
 #define AD(U_, PIPE_, KV8_)                                                                                      \
   attn_decode_kernel<D, GB, U_, PIPE_, KV8_><<<grid, 256, 0, st>>>(q, qs, kc, vc, bt, bts, cl, out, os, po, pml, nh, \
-                                                                  nkv, G, ngroups, bs, psize, sl2)
+                                                                  nkv, G, ngroups, bs, bshift, psize, sl2)
   if (kv8) {
     switch (g_decode_unroll) {
       case 2: AD(2, false, true); break;

@@ -333,8 +333,15 @@ def decode_splits(B: int, nkv: int, max_ctx: int, block_size: int) -> tuple:
     """(num_splits, partition_size): ~8 workgroups per CU (2048), partitions >= 256 tokens.
 
     Measured (bench/attn_bench.py): with few (sequence, kv-head) pairs - GQA / TP-sharded kv heads -
-    each workgroup otherwise walks the whole context serially and the KV stream drops to 2-3 TB/s."""
+    each workgroup otherwise walks the whole context serially and the KV stream drops to 2-3 TB/s.
+
+    From 640 (sequence, kv-head) pairs on and up to 2048 positions: one partition, no sum behind it. 2.5 workgroups per CU are
+    in flight at once, and the start and end of each cost more than a fuller chip gives (us, three or four partitions and
+    one: 23 sequences of 32 heads to 1777 positions in fp8 67 and 61, 31 to 513 in bf16 41 and 38; at 4000 positions 48 of 8 heads
+    in bf16 would lose 13 %). A partition's pages stay within what the kernel stages (256)."""
     wgs = max(1, B * nkv)
+    if wgs >= 640 and max_ctx <= min(2048, 256 * block_size):
+        return 1, math.ceil(max_ctx / block_size) * block_size
     want = max(1, math.ceil(2048 / wgs))
     nsplit = max(1, min(want, math.ceil(max_ctx / 256)))
     psize = math.ceil(max_ctx / nsplit)

@@ -91,6 +91,34 @@ def test_rope_cache_writes_fp8_rows(style, D, rot, nh, nkv):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bs", [16, 24])
+@pytest.mark.parametrize("D,nh,nkv,ctx", [(128, 32, 32, [1, 31, 32, 33, 65, 300]), (64, 10, 5, [1, 63, 64, 65, 129, 200]),
+                                          (256, 4, 4, [1, 15, 16, 17, 33, 100]), (128, 32, 32, [97, 2] * 10)])
+def test_decode_attention_fp8_rows_at_the_edges_of_its_tiles(D, nh, nkv, ctx, bs):
+    """Groups of one and two heads (16 bytes a lane: 8, 16 and 4 tokens a wave): contexts around a workgroup's tokens, pages of a size
+    that is no power of two, one partition and several, and positions behind a context's end that hold NaN and are not read into
+    the result. Values are e4m3 times a scale on both sides: what is off is the output's rounding (2^-9) and fp32 sums."""
+    from llmss_amd.ops import hip as H
+    from llmss_amd.ops import reference as R
+
+    torch.manual_seed(1)
+    B, maxctx = len(ctx), max(ctx)
+    maxb = -(-maxctx // bs)
+    nb = B * maxb
+    kc, vc = _caches(nb, nkv, bs, D)
+    bt = torch.randperm(nb, device=dev).view(B, maxb).to(torch.int32)
+    q = torch.randn(B, (nh + 2 * nkv) * D, device=dev).to(torch.bfloat16)
+    ctxt = torch.tensor(ctx, device=dev, dtype=torch.int32)
+    ref = R.attn_decode(q.float().cpu(), kc.cpu(), vc.cpu(), bt.cpu(), ctxt.cpu(), nh, nkv, D, D ** -0.5)
+    for b, n in enumerate(ctx):
+        for pos in range(n, maxb * bs):
+            kc[bt[b, pos // bs].item(), :, pos % bs, :D] = vc[bt[b, pos // bs].item(), :, pos % bs, :D] = 0x7F
+    for splits in (None, (1, maxb * bs), (-(-maxb // 2), 2 * bs)):
+        got = H.attn_decode(q, kc, vc, bt, ctxt, nh, nkv, D, D ** -0.5, maxctx, splits=splits)
+        torch.testing.assert_close(got.float().cpu(), ref.float(), rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D,nh,nkv", [(128, 32, 32), (128, 32, 8), (64, 25, 25), (256, 16, 16), (128, 8, 1)])
 def test_decode_attention_fp8_rows(D, nh, nkv):
     from llmss_amd.ops import hip as H
