@@ -237,6 +237,10 @@ void launch_sink_attn_mfma(const void* q, const void* kc, const void* vc, const 
                            int64_t rows, const void* vcs, int direct, hipStream_t st);
 void launch_attn_finish(const void* po, const void* pml, int nsplit, int64_t row0, int64_t rows, int sink,
                         const void* sinks, const void* vcs, void* y, int H, int vdim, int dt, hipStream_t st);
+bool mix_attn_ok(int H, int G, int dim, int vdim, int bs, int maxb, float cap);
+void launch_mix_attn(const void* q, const void* kc, const void* vc, const void* bt, int maxb, const void* cu, const void* ctx,
+                     const void* talk, float c, void* y, int64_t ldy, int B, int max_qlen, int H, int G, int dim, int vdim, int bs,
+                     float scale, float cap, hipStream_t st);
 void launch_talk_mix(const void* O, const void* talk, float c, void* y, int64_t ldy, int T_, int H, int G, int vdim,
                      int dt, hipStream_t st);
 
@@ -633,6 +637,13 @@ PYBIND11_MODULE(_C, m) {
   m.def("attn_finish", [](uintptr_t po, uintptr_t pml, int nsplit, int64_t row0, int64_t rows, int sink, uintptr_t sinks,
                           uintptr_t vcs, uintptr_t y, int H, int vdim, int dt, uintptr_t st) {
     launch_attn_finish(CP(po), CP(pml), nsplit, row0, rows, sink, CP(sinks), CP(vcs), P(y), H, vdim, dt, S(st));
+  });
+  m.def("mix_attn_ok", &mix_attn_ok);
+  m.def("mix_attn", [](uintptr_t q, uintptr_t kc, uintptr_t vc, uintptr_t bt, int maxb, uintptr_t cu, uintptr_t ctx, uintptr_t talk,
+                       float c, uintptr_t y, int64_t ldy, int B, int max_qlen, int H, int G, int dim, int vdim, int bs, float scale,
+                       float cap, uintptr_t st) {
+    launch_mix_attn(CP(q), CP(kc), CP(vc), CP(bt), maxb, CP(cu), CP(ctx), CP(talk), c, P(y), ldy, B, max_qlen, H, G, dim, vdim, bs,
+                    scale, cap, S(st));
   });
   m.def("talk_mix", [](uintptr_t O, uintptr_t talk, float c, uintptr_t y, int64_t ldy, int T, int H, int G, int vdim,
                        int dt, uintptr_t st) { launch_talk_mix(CP(O), CP(talk), c, P(y), ldy, T, H, G, vdim, dt, S(st)); });

@@ -1590,16 +1590,60 @@ def sink_attn(q, k_cache, v_cache, block_tables, cu, ctx_lens, heads, kv_heads, 
     return out
 
 
+def _mix_in_one(n: int, rows: int, kv_heads: int, vdim: int, longest: int) -> bool:
+    """Whether ``n`` sequences of at most ``rows`` rows and ``longest`` keys take csrc/attention_mix.hip, one workgroup per 16 rows. The
+    general kernel has kv_heads * column chunks (256 wide) times as many, each as long: while they fit the chip (two per CU) it is as fast
+    or faster, and far slower beyond that. Short contexts are a matter of launches: one instead of two (us, 16 heads: one row
+    behind 32 keys 20 and 11, behind 512 43 and 62; 64 rows behind 256 46 and 36, behind 1024 118 and 119)."""
+    if rows == 1:
+        return longest <= (192 if n < 32 else 512)
+    return longest <= 256 or n * -(-rows // 16) * kv_heads * -(-kv_heads * vdim // 256) > 512
+
+
 def sink_attn_mix(q, k_cache, v_cache, block_tables, cu, ctx_lens, talk, c, heads, kv_heads, dim, vdim, scale, softcap,
                   out, max_qlen=0, num_decode=0, max_ctx=0):
-    """Sink attention, head mixing and the branch scale, written to ``out`` [T, heads * vdim]: sink_attn (weighted
-    sums of every head over all value groups when ``talk`` is given) followed by talk_mix. (A two-pass form for steps
-    of single rows - scores of every head first, then mixed weights against each head's own group, so that keys and
-    values are each read once - was measured at twice the time of the matrix-core kernel at 64 rows x 1024 keys:
-    too few workgroups without a split over keys. It is not kept.)"""
-    O = sink_attn(q, k_cache, v_cache, block_tables, cu, ctx_lens, heads, kv_heads, dim, vdim, scale, softcap,
-                  talk is not None, max_qlen=max_qlen, num_decode=num_decode)
-    return talk_mix(O, talk, c, heads, kv_heads, vdim, out=out)
+    """Sink attention, head mixing and the branch scale, written to ``out`` [T, heads * vdim]: one kernel that mixes the heads' weights
+    before they meet the values (csrc/attention_mix.hip) where it is built for the shape and faster, else sink_attn (weighted
+    sums of every head over all value groups when ``talk`` is given) followed by talk_mix. ``max_ctx``: an upper bound of every context
+    length (0: what the block tables hold)."""
+    B, T, maxb, bs = cu.numel() - 1, q.shape[0], block_tables.shape[1], k_cache.shape[1]
+    nd = B if max_qlen == 1 else int(num_decode)
+    cap = float(softcap or 0.0)
+    parts = [(first, n, ql) for first, n, ql in ((0, nd, 1), (nd, B - nd, int(max_qlen))) if n > 0]
+    built = (talk is not None and max_qlen > 0 and k_cache.dtype == torch.bfloat16 == out.dtype and _SINK_MFMA
+             and lib().mix_attn_ok(heads, kv_heads, dim, vdim, bs, maxb, cap) and out.stride(0) % 4 == 0
+             and not (k_cache.data_ptr() % 16 or v_cache.data_ptr() % 16 or q.data_ptr() % 16 or out.data_ptr() % 8) and 0 <= nd <= B)
+    longest = min(int(max_ctx) or maxb * bs, maxb * bs)
+    one = [built and _mix_in_one(n, ql, kv_heads, vdim, longest) for _, n, ql in parts]
+    if not any(one):
+        O = sink_attn(q, k_cache, v_cache, block_tables, cu, ctx_lens, heads, kv_heads, dim, vdim, scale, softcap,
+                      talk is not None, max_qlen=max_qlen, num_decode=num_decode)
+        return talk_mix(O, talk, c, heads, kv_heads, vdim, out=out)
+    _rows(q, "q", heads * dim, torch.float32)
+    _check(q.is_contiguous(), "q contiguous")
+    _i32(cu, "cu")
+    _i32(ctx_lens, "ctx_lens", B)
+    _i32(block_tables, "block_tables")
+    _check(block_tables.dim() == 2 and block_tables.shape[0] >= B, "block tables [B, blocks]")
+    _check(k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.dtype == v_cache.dtype
+           and k_cache.dim() == 3 and k_cache.shape[2] == kv_heads * dim and v_cache.shape[2] == kv_heads * vdim
+           and k_cache.shape[:2] == v_cache.shape[:2], "k / v cache [blocks, block_size, kv_heads * dim | vdim]")
+    _f32c(talk, "talk")
+    _check(talk.numel() == heads * heads, "talk [heads, heads]")
+    _check(tuple(out.shape) == (T, heads * vdim) and out.stride(1) == 1, "out [T, heads * vdim]")
+    for (first, n, ql), single_pass in zip(parts, one):
+        if single_pass:
+            lib().mix_attn(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr() + 4 * first * maxb, maxb,
+                           cu.data_ptr() + 4 * first, ctx_lens.data_ptr() + 4 * first, talk.data_ptr(), float(c), out.data_ptr(),
+                           out.stride(0), n, ql, heads, kv_heads, dim, vdim, bs, float(scale), cap, _stream())
+        else:  # rows of this part alone: the single ones stand first
+            r = slice(0, n) if ql == 1 and first == 0 else slice(nd, T)
+            O = torch.empty(T, heads, kv_heads * vdim, dtype=torch.float32, device=q.device)
+            lib().sink_attn_mfma(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr() + 4 * first * maxb,
+                                 maxb, cu.data_ptr() + 4 * first, ctx_lens.data_ptr() + 4 * first, O.data_ptr(), n, ql, heads,
+                                 kv_heads, dim, vdim, bs, float(scale), cap, 1, 1, 0, 1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 0, 0, _stream())
+            talk_mix(O[r], talk, c, heads, kv_heads, vdim, out=out[r])
+    return out
 
 
 def talk_mix(O, talk, c, heads, kv_heads, vdim, out=None, out_dtype=None):

@@ -261,9 +261,10 @@ def test_rotation_bias_and_cache_write(device, dtype, H, G, d, dv, rot):
     assert float(pg.kc.view(-1, nk).float().cpu()[[s for s in range(pg.kc.shape[0] * bs) if s not in slots.tolist()]].min()) == 9.0
 
 
-def attention_case(device, dtype, H, G, d, dv, lens, cuts, scale, cap, talk, bs=16, boost=None, shift=0.0, seed=0):
+def attention_case(device, dtype, H, G, d, dv, lens, cuts, scale, cap, talk, bs=16, boost=None, shift=0.0, seed=0, mix=False):
     """Run sink_attn + talk_mix over portions and compare every row with the oracle. ``boost`` = (sequence, key
-    position, factor): that key and the last query are scaled so that its score stands out."""
+    position, factor): that key and the last query are scaled so that its score stands out. ``mix``: as the one op
+    sink_attn_mix, into a view of a wider buffer."""
     pg = Paged(lens, G, d, dv, bs, device, dtype, seed)
     data = []
     for i, n in enumerate(lens):
@@ -287,9 +288,15 @@ def attention_case(device, dtype, H, G, d, dv, lens, cuts, scale, cap, talk, bs=
             pg.vc.view(-1, G * dv)[sl] = data[s][2][p0:p0 + n].reshape(n, -1).to(dtype).to(device)
         cu, ctx, _ = meta(step, [0] * len(lens), device)
         q = torch.cat([data[s][0][p0:p0 + n] for s, p0, n in step]).reshape(-1, H * d).float().to(device)
-        O = ops.sink_attn(q, pg.kc, pg.vc, pg.bt(seqs, device), cu, ctx, H, G, d, dv, scale, cap, talk,
-                          max_qlen=max(n for _, _, n in step), num_decode=nd)
-        y = ops.talk_mix(O, tk.float().to(device).contiguous() if talk else None, 0.8, H, G, dv,
+        longest, bt = max(n for _, _, n in step), pg.bt(seqs, device)
+        if mix:
+            wide = torch.full((len(q), H * dv + 8), 7.0, dtype=dtype, device=device)
+            ops.sink_attn_mix(q, pg.kc, pg.vc, bt, cu, ctx, tk.float().to(device).contiguous(), 0.8, H, G, d, dv, scale, cap,
+                              wide[:, :H * dv], max_qlen=longest, num_decode=0 if longest == 1 else nd, max_ctx=pg.maxb * bs)
+            assert (wide[:, H * dv:] == 7.0).all()
+        else:
+            O = ops.sink_attn(q, pg.kc, pg.vc, bt, cu, ctx, H, G, d, dv, scale, cap, talk, max_qlen=longest, num_decode=nd)
+        y = wide[:, :H * dv].float().cpu() if mix else ops.talk_mix(O, tk.float().to(device).contiguous() if talk else None, 0.8, H, G, dv,
                          out_dtype=torch.float32).cpu()
         r = 0
         for s, p0, n in step:
@@ -312,6 +319,53 @@ def test_sink_attention_portions_decoding_and_batches(device, dtype, H, G, d, dv
     attention_case(device, dtype, H, G, d, dv, [70, 1, 33], [[16, 1, 15, 2, 1, 1, 30, 3, 1], [1], [2, 31]],
                    d ** -0.5, 30.0, talk)
     attention_case(device, dtype, H, G, d, dv, [150, 90], [[65, 64, 1, 20], [3, 87]], d ** -0.5, 0.0, talk, seed=7)
+
+
+@pytest.mark.parametrize("device,dtype", RUNS)
+@pytest.mark.parametrize("H,G,d,dv,cap,bs", [(8, 2, 64, 128, 30.0, 16), (8, 2, 128, 128, 60.0, 24), (16, 4, 128, 128, 30.0, 16),
+                                             (16, 4, 64, 128, 5.0, 8), (16, 4, 128, 128, 61.0, 16), (16, 4, 128, 128, 0.0, 16),
+                                             (16, 4, 128, 64, 30.0, 16)])
+def test_heads_mixed_before_the_values_at_the_edges_of_the_tiles(device, dtype, H, G, d, dv, cap, bs):
+    """Attention, head mixing and the scale in one op, over portions and single rows: rows around a workgroup's 16, keys around a tile's
+    16 and 32, pages of any size, shapes and caps on both sides of what the one-kernel form takes."""
+    attention_case(device, dtype, H, G, d, dv, [70, 1, 33, 17], [[16, 1, 15, 2, 1, 1, 30, 3, 1], [1], [2, 31], [17]], d ** -0.5, cap,
+                   True, bs=bs, mix=True)
+    attention_case(device, dtype, H, G, d, dv, [150, 96, 31], [[65, 64, 1, 20], [32, 64], [31]], 2 * d ** -0.5, cap, True, bs=bs,
+                   seed=7, mix=True)
+    if (H, d, cap) == (16, 128, 30.0) and device != "cpu":  # prompts longer than what a short context is
+        attention_case(device, dtype, H, G, d, dv, [560, 530], [[560], [530]], d ** -0.5, cap, True, bs=bs, seed=8, mix=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nd,n,prefix,one", [(3, 520, 0, (False, True)), (3, 40, 400, (False, False)), (40, 40, 100, (True, True)),
+                                             (40, 400, 0, (True, False)), (0, 520, 96, (True,))])
+def test_single_rows_and_portions_choose_their_form_of_mixing_alone(nd, n, prefix, one):
+    """A step of single rows and two portions, each part in one kernel or in two by its own sizes; a padded row without keys."""
+    from llmss_amd.ops import hip as H
+
+    device, H_, G, d, dv, bs = "cuda", 16, 4, 128, 128, 16
+    lens = [1 + 7 * i % (n + prefix) for i in range(nd)] + [n + prefix, n + prefix - 3]
+    if nd:
+        lens[1] = 0
+    rows = [1] * nd + [n, n - 3]
+    maxb = -(-max(lens) // bs)
+    gen = torch.Generator(device=device).manual_seed(5)
+    kc, vc = (torch.randn(len(lens) * maxb, bs, G * w, generator=gen, device=device).to(torch.bfloat16) for w in (d, dv))
+    bt = torch.randperm(len(lens) * maxb, generator=gen, device=device).view(-1, maxb).to(torch.int32)
+    q = torch.randn(sum(rows), H_ * d, generator=gen, device=device)
+    talk = torch.eye(H_, device=device) + 0.2 * torch.randn(H_, H_, generator=gen, device=device)
+    cu = torch.tensor([0] + rows, device=device).cumsum(0).to(torch.int32)
+    ctx = i32(lens, device)
+    parts = [(k, r) for k, r in ((nd, 1), (2, n)) if k]
+    assert tuple(H._mix_in_one(k, r, G, dv, maxb * bs) for k, r in parts) == one
+    out = torch.full((len(q), H_ * dv), float("nan"), dtype=torch.bfloat16, device=device)
+    H.sink_attn_mix(q, kc, vc, bt, cu, ctx, talk, 0.8, H_, G, d, dv, d ** -0.5, 30.0, out, max_qlen=n, num_decode=nd)
+    O = H.sink_attn(q, kc, vc, bt, cu, ctx, H_, G, d, dv, d ** -0.5, 30.0, True)  # vector kernel, fp32 weights
+    want = H.talk_mix(O, talk, 0.8, H_, G, dv, out_dtype=torch.float32)
+    # weights rounded to bf16 (2^-9 each) against fp32 ones, and the output's rounding
+    torch.testing.assert_close(out.float(), want, rtol=2e-2, atol=2e-2 * float(want.abs().max()))
+    if nd:
+        assert (out[1] == 0).all()
 
 
 @pytest.mark.parametrize("device,dtype", RUNS)
