@@ -651,14 +651,14 @@ struct DeltaChunk32Args {
 
 __device__ __forceinline__ f32x4 ldv4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
-constexpr int prep32_kq_bytes(int kt) {  // K and Q rows, or P and the inverse
-  return 2 * 64 * (16 * kt + 4) * 4 > 2 * 64 * 68 * 4 ? 2 * 64 * (16 * kt + 4) * 4 : 2 * 64 * 68 * 4;
+constexpr int prep32_k_bytes(int kt) {  // K rows, or P and the inverse
+  return 64 * (16 * kt + 4) * 4 > 2 * 64 * 68 * 4 ? 64 * (16 * kt + 4) * 4 : 2 * 64 * 68 * 4;
 }
 
-// acc += A B^T over the keys: A's rows at ap (this lane's, from column 4 g on), B's at bp, in up to four chains (shorter ones
-// round less)
+// acc += A B^T over the keys: A's row in registers (columns 16 kt + 4 g on), B's at bp (this lane's, from column 4 g on), in up to four
+// chains (shorter ones round less)
 template <int KT>
-__device__ __forceinline__ f32x4 dot32(const float* ap, const float* bp) {
+__device__ __forceinline__ f32x4 dot32(const f32x4* a, const float* bp) {
   constexpr int N = KT < 4 ? 2 : 4;
   f32x4 c[N];
 #pragma unroll
@@ -667,7 +667,7 @@ __device__ __forceinline__ f32x4 dot32(const float* ap, const float* bp) {
   for (int kt = 0; kt < KT; kt += N) {
     f32x4 x[N], y[N];
 #pragma unroll
-    for (int n = 0; n < N; ++n) x[n] = ldv4(ap + 16 * (kt + n)), y[n] = ldv4(bp + 16 * (kt + n));
+    for (int n = 0; n < N; ++n) x[n] = a[kt + n], y[n] = ldv4(bp + 16 * (kt + n));
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -695,16 +695,17 @@ __device__ __forceinline__ f32x4 dot32s(const float* ap, const f32x4* S) {
   return N == 4 ? (c[0] + c[1]) + (c[N - 2] + c[N - 1]) : c[0] + c[1];
 }
 
-// Workgroup (chunk of a portion, head, sequence), 4 waves. TP: storage of a and b
+// Workgroup (chunk of a portion, head, sequence), 4 waves. TP: storage of a and b. Bound by its chain of stages (rows, sums, products,
+// 64 steps of substitution), so by how many workgroups a CU holds: the queries stay in the registers of the wave whose rows they
+// are, and 54 KB of LDS let three in where keys and queries in LDS (86 KB) left room for one.
 template <int KT, typename TP>
-__global__ __launch_bounds__(256) void delta_prep32_kernel(DeltaChunk32Args A) {
+__global__ __launch_bounds__(256, 3) void delta_prep32_kernel(DeltaChunk32Args A) {
   constexpr int C = 64, DKP = 16 * KT, LDK = DKP + 4, LDL = 64 + 4;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   float* Ks = reinterpret_cast<float*>(smem);
-  float* Qs = Ks + C * LDK;
   float* Ps = reinterpret_cast<float*>(smem);  // once the rows' products are taken
   float* Xs = Ps + C * LDL;
-  float* Ls = reinterpret_cast<float*>(smem + prep32_kq_bytes(KT));
+  float* Ls = reinterpret_cast<float*>(smem + prep32_k_bytes(KT));
   double* bs = reinterpret_cast<double*>(Ls + C * LDL);  // [64] sum of the log decays
   float* be = reinterpret_cast<float*>(bs + C);          // [64] write strength
   float* nk = be + C;                                    // [64] 1 / |k|
@@ -720,9 +721,15 @@ __global__ __launch_bounds__(256) void delta_prep32_kernel(DeltaChunk32Args A) {
     const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 4;
     const bool in = r < nt && d < dim;
     const int64_t tt = t0 + j0 + r;
-    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-    *reinterpret_cast<f32x4*>(&Ks[r * LDK + d]) = in ? ldv4(A.k + tt * A.ldk + (int64_t)gq * dim + d) : z;
-    *reinterpret_cast<f32x4*>(&Qs[r * LDK + d]) = in ? ldv4(A.q + tt * A.ldq + (int64_t)gq * dim + d) : z;
+    *reinterpret_cast<f32x4*>(&Ks[r * LDK + d]) = in ? ldv4(A.k + tt * A.ldk + (int64_t)gq * dim + d) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  f32x4 q[KT];  // row 16 w + li, columns 16 kt + 4 g on
+  {
+    const int r = 16 * w + li;
+    const float* qp = A.q + (int64_t)(t0 + j0 + min(r, nt - 1)) * A.ldq + (int64_t)gq * dim;
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+      q[kt] = r < nt && 16 * kt + 4 * g < dim ? ldv4(qp + 16 * kt + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   if (w == 0) {  // the tokens' decays and write strengths
     const bool in = lane < nt;
@@ -743,31 +750,31 @@ __global__ __launch_bounds__(256) void delta_prep32_kernel(DeltaChunk32Args A) {
     const int r = tid >> 2, part = tid & 3;
     float kk = 0.f, qq = 0.f;
     for (int d = part * 4; d < DKP; d += 16) {
-      const f32x4 x = ldv4(&Ks[r * LDK + d]), y = ldv4(&Qs[r * LDK + d]);
+      const f32x4 x = ldv4(&Ks[r * LDK + d]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        kk = fmaf(x[i], x[i], kk);
-        qq = fmaf(y[i], y[i], qq);
-      }
+      for (int i = 0; i < 4; ++i) kk = fmaf(x[i], x[i], kk);
     }
     kk += __shfl_xor(kk, 1, 64);
     kk += __shfl_xor(kk, 2, 64);
-    qq += __shfl_xor(qq, 1, 64);
-    qq += __shfl_xor(qq, 2, 64);
-    if (part == 0) {
-      nk[r] = 1.0f / sqrtf(kk + 1e-6f);
-      nq[r] = 1.0f / (sqrtf(qq + 1e-6f) * sqrtf((float)dim));
-    }
+    if (part == 0) nk[r] = 1.0f / sqrtf(kk + 1e-6f);
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) qq = fmaf(q[kt][i], q[kt][i], qq);
+    qq = xor32_sum(xor16_sum(qq));
+    if (g == 0) nq[16 * w + li] = 1.0f / (sqrtf(qq + 1e-6f) * sqrtf((float)dim));
   }
   // wave w: the products of its 16 tokens (rows) with the keys of the blocks up to its own (columns)
-  f32x4 pk[4], pq[4];
+  f32x4 pk[4], pq[4], ka[KT];
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) ka[kt] = ldv4(&Ks[(16 * w + li) * LDK + 16 * kt + 4 * g]);
 #pragma unroll
   for (int ct = 0; ct < 4; ++ct) {
     pk[ct] = pq[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (ct > w || 16 * w >= nt) continue;
     const float* kb = &Ks[(16 * ct + li) * LDK + 4 * g];
-    pk[ct] = dot32<KT>(&Ks[(16 * w + li) * LDK + 4 * g], kb);
-    pq[ct] = dot32<KT>(&Qs[(16 * w + li) * LDK + 4 * g], kb);
+    pk[ct] = dot32<KT>(ka, kb);
+    pq[ct] = dot32<KT>(q, kb);
   }
   __syncthreads();  // every wave has read its rows; the norms are written
 #pragma unroll
@@ -990,7 +997,7 @@ void launch_delta_chunk32(const void* q, const void* k, const void* v, int64_t l
                      (const float*)dt_bias, (float*)S, (const int*)cu, (const int*)ctx, (const int*)sslots, (float*)out,
                      (float*)work, (int64_t)T_ * H * 64, (f32x4*)aux, H, G, dim, vdim};
   dim3 g1((max_qlen + 63) / 64, H, B), g2(H, (vdim + 63) / 64, B);
-  auto lds1 = [](int kt) { return (size_t)prep32_kq_bytes(kt) + (size_t)4 * (64 * 68 + 3 * 64) + 8 * 64; };
+  auto lds1 = [](int kt) { return (size_t)prep32_k_bytes(kt) + (size_t)4 * (64 * 68 + 3 * 64) + 8 * 64; };
   auto lds2 = [](int kt) { return (size_t)4 * (2 * 64 * (16 * kt + 4) + 2 * 64 * 68) + (size_t)16 * 64; };
 #define LAUNCH_DC32(KT_)                                                                                             \
   do {                                                                                                               \
