@@ -1841,12 +1841,72 @@ static void gemm_default_plan(int M, int N, int K, bool w_fp8, bool glu, bool sl
 }
 static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint, int64_t ws_bytes);
 
+// Where to cut a product of 256 x 256 tiles whose last wave is mostly empty in two launches: the tiles of whole waves, and the rows or
+// columns left over, which smaller tiles spread over the chip. Waves cost what gemm_static_plan has measured, but one that is at most
+// 0.8 full only 0.78 of it (0.6 - 0.94 over eleven shapes: the clock rises as tiles end); up to 64 rows left over read all weights at
+// 4.5 TB/s behind 8 us. us, one launch and two: 1773 x 12288 x 4096 172 -> 151 (predicted 174 and 155), SwiGLU x 22016 280 -> 266,
+// 8261 x 2048 x 2048 91 -> 61, 8261 x 6400 x 2048 190 -> 174, 3999 x 22016 x 4096 570 -> 551. Left whole, as predicted: 8192 x 5120 x 2048
+// (2.5 waves) 141 and 143, 8192 x 9472 x 2048 (4.6) 255 and 255, 5000 x 12288 x 4096 (3.75) 359 and 357.
+struct GemmCut {
+  int rows, cols;  // of the first launch; 0: not cut
+  int hint;        // plan of the second (0: the plan of its size)
+};
+static GemmCut gemm_cut(int M, int N, int K, bool glu) {
+  const int ntm = (M + 255) / 256, ntn = (N + 255) / 256, nk = (K + 63) / 64;
+  auto tiles_us = [&](const TileCost& c, int m, int n) {
+    const int slots = 256 * c.per_cu, wgs = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn), rest = wgs % slots;
+    double t = wgs / slots * (nk * c.step + 5.0);
+    if (rest) t += (nk * (rest <= 256 ? c.alone : c.step) + 5.0) * (rest * 5 <= slots * 4 ? 0.78 : 1.0);
+    return std::max(t, (2.0 * n * K + 2.0 * m * K + 2.0 * m * (glu ? n / 2 : n)) / 4.0e6);
+  };
+  GemmCut cut{0, 0, 0};
+  double best = 0.97 * tiles_us(kTileCost[0], M, N);
+  auto consider = [&](int rows, int cols) {
+    if (rows <= 0 || cols <= 0 || (rows >= M && cols >= N)) return;
+    const int last = (rows < M ? rows / 256 * ntn : ntm * (cols / 256)) % 256;
+    if (last && last < 218) return;  // whole waves, the last of them at least 0.85 full
+    const int m = rows < M ? M - rows : M, n = cols < N ? N - cols : N;
+    double rest = 8.0 + 2.0 * n * K / 4.5e6;
+    int hint = 0;
+    for (const TileCost& c : kTileCost) {
+      if (m <= 64) break;
+      const double t = tiles_us(c, m, n);
+      if (!hint || t < rest) rest = t, hint = c.tsel << 8;
+    }
+    const double t = tiles_us(kTileCost[0], std::min(rows, M), std::min(cols, N)) + rest;
+    if (t < best) best = t, cut = GemmCut{rows < M ? rows : 0, cols < N ? cols : 0, hint};
+  };
+  const int waves = (int)std::min<int64_t>((int64_t)ntm * ntn / 256, 64);
+  for (int w = 1; w <= waves; ++w) {
+    consider(256 * w / ntn * 256, N);
+    consider(M, 256 * w / ntm * 256);
+  }
+  consider((ntm - 1) * 256, N);
+  return cut;
+}
+
 int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_fp8, const void* w_scale,
                 const void* bias, void* y, int64_t ldy, int M, int N, int K, int act, bool glu, void* workspace,
                 int64_t ws_bytes, int nt_hint, int split_hint, bool partial_out, hipStream_t st) {
   if (M == 0 || N == 0) return 0;
+  int tuned_nt, tuned_split;
+  const bool free_plan = !nt_hint && !split_hint && !w_fp8 && !gemm_tuned_get(M, N, K, glu, 0, &tuned_nt, &tuned_split);
   gemm_default_plan(M, N, K, w_fp8, glu, partial_out && !glu && act == 0, ws_bytes, gemm_static_takes(w_fp8, x, ldx, w, ldw), &nt_hint,
                     &split_hint);
+  if (free_plan && nt_hint == 4 << 8 && y && !(glu && N % 32) && gemm_quad_ok(N, K, ldx, ldw, 256, y, ldy, 2, glu)) {
+    const GemmCut cut = gemm_cut(M, N, K, glu);
+    if (cut.rows) {
+      launch_gemm(x, ldx, w, ldw, false, nullptr, bias, y, ldy, cut.rows, N, K, act, glu, workspace, ws_bytes, 4 << 8, 1, false, st);
+      return launch_gemm((const bf16_t*)x + cut.rows * ldx, ldx, w, ldw, false, nullptr, bias, (bf16_t*)y + cut.rows * ldy, ldy,
+                         M - cut.rows, N, K, act, glu, workspace, ws_bytes, cut.hint, cut.hint ? 1 : 0, false, st);
+    }
+    if (cut.cols) {
+      launch_gemm(x, ldx, w, ldw, false, nullptr, bias, y, ldy, M, cut.cols, K, act, glu, workspace, ws_bytes, 4 << 8, 1, false, st);
+      return launch_gemm(x, ldx, (const bf16_t*)w + cut.cols * ldw, ldw, false, nullptr, bias ? (const bf16_t*)bias + cut.cols : nullptr,
+                         (bf16_t*)y + (glu ? cut.cols / 2 : cut.cols), ldy, M, N - cut.cols, K, act, glu, workspace, ws_bytes, cut.hint,
+                         cut.hint ? 1 : 0, false, st);
+    }
+  }
   if (!y && (!partial_out || slabs_of_plan(M, N, K, w_fp8, glu, act, nt_hint, split_hint, ws_bytes) == 0))
     throw std::runtime_error("gemm: this configuration writes the output, but no output buffer was given");
   if (K % 16) throw std::runtime_error("gemm: K must be a multiple of 16");
@@ -2287,6 +2347,12 @@ int launch_gemm_qkv_args(const void* x, int64_t ldx, const void* w, int64_t ldw,
   const QkvEpi qe{(const int64_t*)pos, (const float*)cos_t, (const float*)sin_t, (bf16_t*)kc, (bf16_t*)vc,
                   (const int64_t*)slot, nh, nkv, D, rot, block_size, style, do_rope ? 1 : 0};
   return launch_gemm_qkv(x, ldx, w, ldw, bias, y, ldy, M, N, K, workspace, ws_bytes, nt_hint, split_hint, qe, st);
+}
+
+void gemm_cut_of(int M, int N, int K, bool glu, int* rows, int* cols) {
+  const GemmCut c = gemm_cut(M, N, K, glu);
+  *rows = c.rows;
+  *cols = c.cols;
 }
 
 // The plan of a product without hints. slabs: of one whose consumer sums split-K slabs itself

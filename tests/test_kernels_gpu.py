@@ -350,6 +350,25 @@ def test_gemm_mid_k_tail_reads_nothing_past_the_operands(tile):
         close(y, R.linear(x.float(), w.float(), None), 2e-2)
 
 
+@pytest.mark.parametrize("M,N,K,glu,act", [(1773, 12288, 256, False, "none"), (1773, 22016, 1024, True, "none"), (8261, 2048, 512, False, "gelu_tanh"),
+                                           (8193, 2048, 1024, False, "relu"), (8261, 6400, 1024, False, "none"), (8261, 2048, 1024, True, "none"),
+                                           (8256, 2056, 2048, False, "none")])
+def test_products_cut_in_two_launches(M, N, K, glu, act):
+    """Products of 256 x 256 tiles whose last wave is nearly empty: whole waves and what is left over, by rows or columns, with bias
+    and activation on either side, into strided rows; what lies around the output stays as it is."""
+    torch.manual_seed(0)
+    x, w, b = rnd(M, K + 8)[:, :K], rnd(N, K, scale=K ** -0.5), rnd(N, scale=0.1)
+    n = N // 2 if glu else N
+    wide = torch.full((M + 2, n + 16), 7.0, dtype=torch.bfloat16, device=dev)
+    y = wide[1:M + 1, 8:n + 8]
+    H.linear(x, w, b, act=act, glu=glu, out=y)
+    ref = R.linear(x.float(), w.float(), b.float(), act=act, glu=glu)
+    assert any(H.lib().gemm_cut(M, N, K, glu))
+    close(y, ref, 2e-2)
+    wide[1:M + 1, 8:n + 8] = 7.0
+    assert (wide == 7.0).all()
+
+
 DEC_BN = {1: 16, 2: 32, 3: 48, 4: 64, 5: 96}  # csrc/gemm_dec.hip tile codes (hint bit 1024 of the tile bits)
 
 

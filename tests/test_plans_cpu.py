@@ -121,3 +121,16 @@ def test_fp8_products_of_few_rows_take_the_decode_kernel(M, N, K, glu, slabs, de
     assert bool((nt >> 8) & 1024) == dec, (hex(nt), split)
     if dec:
         assert (split > 1) == slabs and ((nt >> 8) & 15) <= 4
+
+
+@pytest.mark.parametrize("M,N,K,glu,cut", [(8192, 12288, 4096, False, None), (8192, 5120, 2048, False, None), (5000, 12288, 4096, False, None),
+                                           (8261, 2048, 2048, False, "rows"), (1773, 12288, 4096, False, "any"), (3999, 22016, 4096, True, "any"),
+                                           (2500, 6144, 2048, False, None)])
+def test_products_are_cut_where_the_last_wave_of_tiles_is_nearly_empty(M, N, K, glu, cut):
+    """Whole waves of 256 x 256 tiles in one launch and the rest in another: never for products that fill their waves, at multiples
+    of a tile, by rows or by columns but not both."""
+    from llmss_amd.ops import hip as H
+
+    rows, cols = H.lib().gemm_cut(M, N, K, glu)
+    assert not (rows and cols) and rows % 256 == 0 and cols % 256 == 0 and rows < M and cols < N
+    assert bool(rows or cols) == (cut is not None) and (cut != "rows" or rows == 8192)
