@@ -13,6 +13,8 @@
 // Splits > 1 write unnormalised partials that attn_decode_reduce_kernel combines.
 #include "common.h"
 
+#include <type_traits>
+
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNegBig = -1.0e30f;
 
@@ -123,9 +125,9 @@ __global__ __launch_bounds__(256, (decode_elems(GB, KV8) == 16 ? (GB == 1 ? 4 : 
     for (int i = threadIdx.x; i < npg; i += blockDim.x) s_pages[i] = bt[pg0 + i];
     __syncthreads();
   }
-  auto kv_addr = [&](int t) -> int64_t {
+  auto kv_addr = [&](int t, auto staged) -> int64_t {
     const int pi = block_shift >= 0 ? t >> block_shift : t / block_size;  // (a division costs as much as a token's products)
-    const int page = lds_pages ? s_pages[pi - pg0] : bt[pi];
+    const int page = decltype(staged)::value ? s_pages[pi - pg0] : bt[pi];
     return page * page_stride + head_off + (t - pi * block_size) * RB;
   };
   // a token's K / V registers: bf16 rows 16 B per lane; fp8 rows E bytes per lane + the row's two scales
@@ -135,11 +137,11 @@ __global__ __launch_bounds__(256, (decode_elems(GB, KV8) == 16 ? (GB == 1 ? 4 : 
     u32xe k8[UNROLL], v8[UNROLL];
     float ks[UNROLL], vs[UNROLL];
   };
-  auto load_tokens = [&](int tb, KVRegs& r) {
+  auto load_tokens = [&](int tb, KVRegs& r, auto staged) {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       const int t = tb + u * STEP;
-      const int64_t a = kv_addr(t < lend ? t : start);
+      const int64_t a = kv_addr(t < lend ? t : start, staged);
       // read once per step: non-temporal (guide 'nt-weights'; +10-15% on streamed reads), but for the rows of 16 bytes a lane
       if constexpr (E == 16) {
         r.k8[u] = *reinterpret_cast<const u32xe*>(kc8 + a);
@@ -237,27 +239,33 @@ __global__ __launch_bounds__(256, (decode_elems(GB, KV8) == 16 ? (GB == 1 ? 4 : 
       }
     }
   };
-  if constexpr (PIPE) {
-    // two register sets: the loads of the next UNROLL tokens per slot are in flight while the
-    // current ones are consumed (the compiler's counted vmcnt waits only for the set it reads)
-    constexpr int CH = STEP * UNROLL;
-    KVRegs A, Bq;
-    int tb = start + w * TPW + slot;
-    if (start < lend) load_tokens(tb, A);
-    for (; tb - slot - w * TPW < lend; tb += 2 * CH) {
-      load_tokens(tb + CH, Bq);
-      consume(tb, A);
-      if (tb + CH - slot - w * TPW >= lend) break;
-      load_tokens(tb + 2 * CH, A);
-      consume(tb + CH, Bq);
+  auto walk = [&](auto staged) {
+    if constexpr (PIPE) {
+      // two register sets: the loads of the next UNROLL tokens per slot are in flight while the
+      // current ones are consumed (the compiler's counted vmcnt waits only for the set it reads)
+      constexpr int CH = STEP * UNROLL;
+      KVRegs A, Bq;
+      int tb = start + w * TPW + slot;
+      if (start < lend) load_tokens(tb, A, staged);
+      for (; tb - slot - w * TPW < lend; tb += 2 * CH) {
+        load_tokens(tb + CH, Bq, staged);
+        consume(tb, A);
+        if (tb + CH - slot - w * TPW >= lend) break;
+        load_tokens(tb + 2 * CH, A, staged);
+        consume(tb + CH, Bq);
+      }
+    } else {
+      for (int tb = start + w * TPW + slot; tb < lend; tb += STEP * UNROLL) {
+        KVRegs R;
+        load_tokens(tb, R, staged);
+        consume(tb, R);
+      }
     }
-  } else {
-    for (int tb = start + w * TPW + slot; tb < lend; tb += STEP * UNROLL) {
-      KVRegs R;
-      load_tokens(tb, R);
-      consume(tb, R);
-    }
-  }
+  };
+  // a loop for each place of the page ids: with the choice inside, the load of an id that only one side makes has every token wait
+  // until all rows asked for before are there, and nothing stays in flight
+  if (lds_pages) walk(std::true_type{});
+  else walk(std::false_type{});
 
   // merge token slots inside the wave
 #pragma unroll

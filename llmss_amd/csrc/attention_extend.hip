@@ -24,9 +24,15 @@
 // sequence's visible range and leaves the unnormalised O, running maximum and sum in the decode kernel's partial
 // buffers ([token, head, split]); attn_decode_reduce_kernel (attention_decode.hip) joins them. A decode step whose
 // sequences are few but long then fills the chip instead of one workgroup walking each sequence.
+// NS groups of 16 slots a wave: a fragment of keys or values read from LDS feeds the products of all of them. With one group LDS
+// reads take as long as the matrix instructions (32 KB a wave and 64 keys of 128). Tiles that every row of a group sees whole skip
+// the mask. Portions of 950 and 823 rows behind prefixes of as many, 32 heads of 128: 135 -> 94 us (413
+// TFLOP/s), 111 with one group.
 // SAME: keys and values are one tensor (latent attention, where both are the cached latent row and nkv = 1): the
 // tile is loaded and staged once and serves both products.
 #include "common.h"
+
+#include <type_traits>
 
 constexpr float kLog2eX = 1.4426950408889634f;
 
@@ -36,13 +42,13 @@ constexpr float kLog2eX = 1.4426950408889634f;
 // absmax / 448 scale and clamped conversion) for the W8A8 o-projection that consumes them, which then skips its own
 // quantisation launch. Only when a workgroup holds every head of its rows: one kv head (nkv = 1) whose whole query
 // group fits the slots of a wave (GE = G, a power of two <= 16) - Llama-2-70B at TP=8 (8 query heads per rank).
-template <int D, bool KV8, bool SAME = false>
-__global__ __launch_bounds__(256) void attn_extend_kernel(
+template <int D, bool KV8, bool SAME, int NS>
+__global__ __launch_bounds__(256, NS) void attn_extend_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ kcv, const void* __restrict__ vcv,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ cu_q, const int* __restrict__ ctx_lens,
     bf16_t* __restrict__ out, int64_t out_stride, int nh, int nkv, int GE, int bs, float scale_log2,
     unsigned char* __restrict__ q8, float* __restrict__ s8, int window, int nsplit, int split_keys,
-    float* __restrict__ part_o, float* __restrict__ part_ml) {
+    float* __restrict__ part_o, float* __restrict__ part_ml, int bshift) {
   static_assert(!(SAME && KV8), "a shared key/value tile is staged from bf16 rows");
   constexpr int BKV = 64;
   constexpr int LD = D + 16;  // padded LDS row (elements): conflict-free b128 rows and tr_b16 columns
@@ -51,7 +57,7 @@ __global__ __launch_bounds__(256) void attn_extend_kernel(
   bf16_t* const Vs = SAME ? Ks : Vs_;
 
   const int G = nh / nkv;
-  const int rows_per_wg = 64 / GE;
+  const int rows_per_wg = 64 * NS / GE;
   int bx = blockIdx.x, by = blockIdx.y, b = blockIdx.z;
   if (nsplit <= 1) causal_block_order(bx, by, b);  // (with a key split x counts the splits of one row)
   const int kvh = by / (G / GE);
@@ -63,35 +69,42 @@ __global__ __launch_bounds__(256) void attn_extend_kernel(
   const int p0 = ctx - qlen;  // position of the chunk's first token
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int li = lane & 15, g = lane >> 4;
-  const int slot = w * 16 + li;
-  const int row = r0 + slot / GE, h = h0 + slot % GE;
-  const bool valid = slot < rows_per_wg * GE && row < qlen;
-  const int qpos = p0 + (valid ? row : 0);  // causal limit of this lane's slot
-
-  s16x8 qf[D / 32];
-  {
-    const bf16_t* qp = q + (int64_t)(t0 + (valid ? row : 0)) * q_stride + (int64_t)(valid ? h : h0) * D + 8 * g;
+  int row[NS], h[NS], qpos[NS], slot[NS];
+  bool valid[NS];
+  s16x8 qf[NS][D / 32];
+  f32x4 o[NS][D / 16];
+  float m[NS], lsum[NS];
+  // positions that the rows of a group span, the same in every lane
+  int grp_lo[NS], grp_hi[NS], grp_klo[NS];
 #pragma unroll
-    for (int ks = 0; ks < D / 32; ++ks) qf[ks] = *reinterpret_cast<const s16x8*>(qp + 32 * ks);
+  for (int n = 0; n < NS; ++n) {
+    const int s0 = (w * NS + n) * 16;
+    slot[n] = s0 + li;
+    row[n] = r0 + slot[n] / GE, h[n] = h0 + slot[n] % GE;
+    valid[n] = slot[n] < rows_per_wg * GE && row[n] < qlen;
+    qpos[n] = p0 + (valid[n] ? row[n] : 0);  // causal limit of this lane's slot
+    grp_lo[n] = p0 + min(qlen - 1, r0 + s0 / GE);
+    grp_hi[n] = p0 + min(qlen - 1, r0 + (s0 + 15) / GE);
+    grp_klo[n] = window > 0 ? grp_lo[n] - window + 1 : 0;
+    const bf16_t* qp = q + (int64_t)(t0 + (valid[n] ? row[n] : 0)) * q_stride + (int64_t)(valid[n] ? h[n] : h0) * D + 8 * g;
+#pragma unroll
+    for (int ks = 0; ks < D / 32; ++ks) qf[n][ks] = *reinterpret_cast<const s16x8*>(qp + 32 * ks);
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) o[n][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    m[n] = -1.0e30f, lsum[n] = 0.f;
   }
-  f32x4 o[D / 16];
-#pragma unroll
-  for (int i = 0; i < D / 16; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -1.0e30f, lsum = 0.f;
 
   // keys needed by this workgroup: [0, last valid row's position]
   const int r_last = min(qlen, r0 + rows_per_wg) - 1;
   const int kv_end = p0 + r_last + 1;
-  // this wave's slots: rows r0 + (16w)/GE .. r0 + (16w+15)/GE
-  const int wave_qhi = p0 + min(qlen - 1, r0 + (16 * w + 15) / GE);
-  // first key any row of the workgroup / of this wave may see (tile-aligned start of the key loop)
+  const int wave_qhi = grp_hi[NS - 1], wave_klo = grp_klo[0];
+  // first key any row of the workgroup may see (tile-aligned start of the key loop)
   int kv_begin = window > 0 ? max(0, p0 + r0 - window + 1) / BKV * BKV : 0;
   int kv_stop = kv_end;  // end of the key loop (kv_end stays the causal bound of the rows)
   if (nsplit > 1) {
     kv_begin += blockIdx.x * split_keys;
     kv_stop = min(kv_end, kv_begin + split_keys);
   }
-  const int wave_klo = window > 0 ? p0 + min(qlen - 1, r0 + (16 * w) / GE) - window + 1 : 0;
   const int* bt = block_tables + (int64_t)b * max_blocks;
   constexpr int CH = D / 8;
   constexpr int RB = KV8 ? D + 16 : D;         // cache row (elements of the cache dtype)
@@ -117,14 +130,19 @@ __global__ __launch_bounds__(256) void attn_extend_kernel(
   u16x8 kr[NCH], vr[NCH];
   u32x2 kr8[NCH], vr8[NCH];
   float ksr[NCH], vsr[NCH];
-  auto load_tile = [&](int kv0) {
+  // where a key's row lies. staged: the page ids are in LDS; a choice made here, with a load of an id on one side only, would have
+  // every row wait until the rows asked for before it are there
+  auto row_of = [&](int key, auto staged) {
+    const int pi = bshift >= 0 ? key >> bshift : key / bs;
+    const int blk = decltype(staged)::value ? s_pages[pi] : bt[pi];
+    return ((int64_t)blk * nkv + kvh) * head_stride + (key - pi * bs) * RB;
+  };
+  auto load_tile = [&](int kv0, auto staged) {
 #pragma unroll
     for (int j = 0; j < NCH; ++j) {
       const int c = threadIdx.x + j * 256;
       const int r = c / CH, ch = c % CH;
-      const int key = min(kv0 + r, kv_end - 1);
-      const int blk = lds_pages ? s_pages[key / bs] : bt[key / bs];
-      const int64_t rowoff = ((int64_t)blk * nkv + kvh) * head_stride + (int64_t)(key % bs) * RB;
+      const int64_t rowoff = row_of(min(kv0 + r, kv_end - 1), staged);
       if constexpr (KV8) {
         kr8[j] = *reinterpret_cast<const u32x2*>(kc8 + rowoff + ch * 8);
         vr8[j] = *reinterpret_cast<const u32x2*>(vc8 + rowoff + ch * 8);
@@ -162,13 +180,11 @@ __global__ __launch_bounds__(256) void attn_extend_kernel(
   };
   // D = 256: the register set would cost the kernel its occupancy - staged chunk by chunk instead
   constexpr bool PIPE = D <= 128;
-  auto stage_direct = [&](int kv0) {
+  auto stage_direct = [&](int kv0, auto staged) {
 #pragma unroll
     for (int c = threadIdx.x; c < BKV * CH; c += 256) {
       const int r = c / CH, ch = c % CH;
-      const int key = min(kv0 + r, kv_end - 1);
-      const int blk = lds_pages ? s_pages[key / bs] : bt[key / bs];
-      const int64_t rowoff = ((int64_t)blk * nkv + kvh) * head_stride + (int64_t)(key % bs) * RB;
+      const int64_t rowoff = row_of(min(kv0 + r, kv_end - 1), staged);
       if constexpr (KV8) {
         kr8[0] = *reinterpret_cast<const u32x2*>(kc8 + rowoff + ch * 8);
         vr8[0] = *reinterpret_cast<const u32x2*>(vc8 + rowoff + ch * 8);
@@ -193,125 +209,151 @@ __global__ __launch_bounds__(256) void attn_extend_kernel(
       }
     }
   };
-  if constexpr (PIPE) {
-    if (kv_stop > kv_begin) load_tile(kv_begin);
-  }
-  for (int kv0 = kv_begin; kv0 < kv_stop; kv0 += BKV) {
-    __syncthreads();  // every wave is done reading the previous tile
-    if constexpr (PIPE) store_tile();
-    else stage_direct(kv0);
-    __syncthreads();
+  auto walk = [&](auto staged) {
     if constexpr (PIPE) {
-      if (kv0 + BKV < kv_stop) load_tile(kv0 + BKV);
+      if (kv_stop > kv_begin) load_tile(kv_begin, staged);
     }
-    if (kv0 > wave_qhi) continue;  // whole tile in this wave's causal future (barriers stay uniform)
-    if (kv0 + BKV <= wave_klo) continue;  // whole tile older than this wave's windows
+    for (int kv0 = kv_begin; kv0 < kv_stop; kv0 += BKV) {
+      __syncthreads();  // every wave is done reading the previous tile
+      if constexpr (PIPE) store_tile();
+      else stage_direct(kv0, staged);
+      __syncthreads();
+      if constexpr (PIPE) {
+        if (kv0 + BKV < kv_stop) load_tile(kv0 + BKV, staged);
+      }
+      if (kv0 > wave_qhi) continue;  // whole tile in this wave's causal future (barriers stay uniform)
+      if (kv0 + BKV <= wave_klo) continue;  // whole tile older than this wave's windows
 
-    f32x4 s[4];
+      f32x4 s[NS][4];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
-      s[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int kt = 0; kt < 4; ++kt) {
 #pragma unroll
-      for (int ks = 0; ks < D / 32; ++ks) {
-        const s16x8 kf = *reinterpret_cast<const s16x8*>(&Ks[(kt * 16 + li) * LD + 32 * ks + 8 * g]);
-        s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], s[kt], 0, 0, 0);
+        for (int n = 0; n < NS; ++n) s[n][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < D / 32; ++ks) {
+          const s16x8 kf = *reinterpret_cast<const s16x8*>(&Ks[(kt * 16 + li) * LD + 32 * ks + 8 * g]);
+#pragma unroll
+          for (int n = 0; n < NS; ++n) s[n][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[n][ks], s[n][kt], 0, 0, 0);
+        }
       }
-    }
-    // S^T C layout: lane (li, g) holds slot li's scores for keys kv0 + 16kt + 4g + i
-    float mx = m;
+      // S^T C layout: lane (li, g) holds slot li's scores for keys kv0 + 16kt + 4g + i
+      s16x8 pf[NS][2];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
+      for (int n = 0; n < NS; ++n) {
+        float mx = m[n];
+        const bool whole = kv0 + BKV - 1 <= grp_lo[n] && kv0 + BKV <= kv_end && (window <= 0 || kv0 > grp_hi[n] - window);
+        if (whole) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int key = kv0 + kt * 16 + 4 * g + i;
-        float v = s[kt][i] * scale_log2;
-        v = (key <= qpos && key < kv_end && (window <= 0 || key > qpos - window)) ? v : -1.0e30f;
-        s[kt][i] = v;
-        mx = fmaxf(mx, v);
+          for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              s[n][kt][i] *= scale_log2;
+              mx = fmaxf(mx, s[n][kt][i]);
+            }
+        } else {
+#pragma unroll
+          for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int key = kv0 + kt * 16 + 4 * g + i;
+              float v = s[n][kt][i] * scale_log2;
+              v = (key <= qpos[n] && key < kv_end && (window <= 0 || key > qpos[n] - window)) ? v : -1.0e30f;
+              s[n][kt][i] = v;
+              mx = fmaxf(mx, v);
+            }
+        }
+        mx = xor32_max(xor16_max(mx));
+        const float alpha = __builtin_amdgcn_exp2f(m[n] - mx);
+        m[n] = mx;
+        float ps = 0.f;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float p = __builtin_amdgcn_exp2f(s[n][kt][i] - mx);
+            // a masked key adds nothing, also while a slot has seen no visible key yet (mx still at its floor)
+            if (!whole) p = s[n][kt][i] > -1.0e29f ? p : 0.f;
+            const bf16_t pb = f2bf(p);
+            ps += bf2f(pb);
+            pf[n][kt >> 1][(kt & 1) * 4 + i] = (short)pb;
+          }
+        ps = xor32_sum(xor16_sum(ps));
+        lsum[n] = lsum[n] * alpha + ps;
+#pragma unroll
+        for (int i = 0; i < D / 16; ++i) o[n][i] *= alpha;
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float alpha = exp2f(m - mx);
-    m = mx;
-    float ps = 0.f;
-    s16x8 pf[2];
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        // a masked key adds nothing, also while a slot has seen no visible key yet (mx still at its floor)
-        const float p = s[kt][i] > -1.0e29f ? exp2f(s[kt][i] - mx) : 0.f;
-        const bf16_t pb = f2bf(p);
-        ps += bf2f(pb);
-        pf[kt >> 1][(kt & 1) * 4 + i] = (short)pb;
-      }
-    ps += __shfl_xor(ps, 16, 64);
-    ps += __shfl_xor(ps, 32, 64);
-    lsum = lsum * alpha + ps;
-#pragma unroll
-    for (int i = 0; i < D / 16; ++i) o[i] *= alpha;
 
-    const int tq = li >> 2, tp = li & 3;
+      const int tq = li >> 2, tp = li & 3;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
+      for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt) {
-        const bf16_t* a0 = &Vs[(32 * ks + 4 * g + tq) * LD + dt * 16 + 4 * tp];
-        const bf16_t* a1 = a0 + 16 * LD;
-        const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(a0));
-        const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(a1));
-        const s16x8 vf = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[ks], o[dt], 0, 0, 0);
+        for (int dt = 0; dt < D / 16; ++dt) {
+          const bf16_t* a0 = &Vs[(32 * ks + 4 * g + tq) * LD + dt * 16 + 4 * tp];
+          const bf16_t* a1 = a0 + 16 * LD;
+          const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(a0));
+          const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(a1));
+          const s16x8 vf = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+#pragma unroll
+          for (int n = 0; n < NS; ++n) o[n][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[n][ks], o[n][dt], 0, 0, 0);
+        }
       }
     }
-  }
+  };
+  if (lds_pages) walk(std::true_type{});
+  else walk(std::false_type{});
   if (nsplit > 1) {  // kernel argument: uniform
-    if (valid) {
-      const int64_t pi = ((int64_t)(t0 + row) * nh + h) * nsplit + blockIdx.x;
 #pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4*>(part_o + pi * D + dt * 16 + 4 * g) = o[dt];
+    for (int n = 0; n < NS; ++n) {
+      if (!valid[n]) continue;
+      const int64_t pi = ((int64_t)(t0 + row[n]) * nh + h[n]) * nsplit + blockIdx.x;
+#pragma unroll
+      for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4*>(part_o + pi * D + dt * 16 + 4 * g) = o[n][dt];
       if (g == 0) {
-        part_ml[pi * 2] = m;
-        part_ml[pi * 2 + 1] = lsum;
+        part_ml[pi * 2] = m[n];
+        part_ml[pi * 2 + 1] = lsum[n];
       }
     }
     return;
   }
-  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-  u16x4 res[D / 16];
+  u16x4 res[NS][D / 16];
+#pragma unroll
+  for (int n = 0; n < NS; ++n) {
+    const float inv = lsum[n] > 0.f ? 1.f / lsum[n] : 0.f;
+#pragma unroll
+    for (int dt = 0; dt < D / 16; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) res[n][dt][i] = f2bf(o[n][dt][i] * inv);
+    if (valid[n]) {
+      bf16_t* op = out + (int64_t)(t0 + row[n]) * out_stride + (int64_t)h[n] * D + 4 * g;
+#pragma unroll
+      for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<u16x4*>(op + dt * 16) = res[n][dt];
+    }
+  }
+  if (NS > 1 || q8 == nullptr) return;  // kernel argument: uniform (and the host's choice of NS)
+  // a row's slots are GE consecutive lanes of one wave (GE | 16): reduce over them and over the 4 lane groups
   float amax = 0.f;
 #pragma unroll
   for (int dt = 0; dt < D / 16; ++dt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      res[dt][i] = f2bf(o[dt][i] * inv);
-      amax = fmaxf(amax, fabsf(bf2f(res[dt][i])));
-    }
-  if (valid) {
-    bf16_t* op = out + (int64_t)(t0 + row) * out_stride + (int64_t)h * D + 4 * g;
-#pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<u16x4*>(op + dt * 16) = res[dt];
-  }
-  if (q8 == nullptr) return;  // kernel argument: uniform
-  // a row's slots are GE consecutive lanes of one wave (GE | 16): reduce over them and over the 4 lane groups
-  if (!valid) amax = 0.f;
+    for (int i = 0; i < 4; ++i) amax = fmaxf(amax, fabsf(bf2f(res[0][dt][i])));
+  if (!valid[0]) amax = 0.f;
   for (int off = 1; off < GE; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
   amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
   amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-  if (!valid) return;
+  if (!valid[0]) return;
   const float sc = amax > 0.f ? amax / 448.f : 1.f;
   const float rs = 1.f / sc;
-  const int64_t qrow = (int64_t)(t0 + row) * (nh * D);
-  if (slot % GE == 0 && g == 0) s8[t0 + row] = sc;
+  const int64_t qrow = (int64_t)(t0 + row[0]) * (nh * D);
+  if (slot[0] % GE == 0 && g == 0) s8[t0 + row[0]] = sc;
 #pragma unroll
   for (int dt = 0; dt < D / 16; ++dt) {
     float f[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) f[i] = fminf(fmaxf(bf2f(res[dt][i]) * rs, -448.f), 448.f);
+    for (int i = 0; i < 4; ++i) f[i] = fminf(fmaxf(bf2f(res[0][dt][i]) * rs, -448.f), 448.f);
     unsigned v = 0;
     v = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], v, false);
     v = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], v, true);
-    *reinterpret_cast<unsigned*>(q8 + qrow + (int64_t)h * D + dt * 16 + 4 * g) = v;
+    *reinterpret_cast<unsigned*>(q8 + qrow + (int64_t)h[0] * D + dt * 16 + 4 * g) = v;
   }
 }
 
@@ -338,7 +380,12 @@ void launch_attn_extend(const void* q, int64_t q_stride, const void* k_cache, co
   if ((Q8 != nullptr) != (S8 != nullptr)) throw std::runtime_error("attn_extend: fp8 twin needs both q8 and s8");
   if (Q8 && !(nkv == 1 && GE == G && G <= 16 && (G & (G - 1)) == 0))
     throw std::runtime_error("attn_extend: the fp8 twin needs one kv head and a power-of-two query group <= 16");
-  const int rows = 64 / GE;
+  // Two groups of slots a wave from 320 workgroups of them on (us, 32 heads of 128, one group and two: 2 portions of 950 behind as many,
+  // 512 workgroups, 111 and 94; 1 of 1500, 384, 162 and 135; 2 of 600, 320, 70 and 60; 1 of 1000, 256, 68 and 86; 25 heads of 64, 2 of 700,
+  // 300, 36 and 47). Heads of 256 would leave a wave per SIMD: 7 x 1433 rows of 16 heads 289 and 410. The twin's rows need a wave.
+  const int64_t wgs = (int64_t)((max_qlen + 128 / GE - 1) / (128 / GE)) * nkv * (G / GE) * B;
+  const bool two = D <= 128 && nsplit <= 1 && !Q8 && max_qlen > 64 / GE && wgs >= 320;
+  const int rows = (two ? 128 : 64) / GE;
   dim3 grid((max_qlen + rows - 1) / rows, nkv * (G / GE), B);
   if (nsplit > 1) {
     if (max_qlen != 1 || split_keys <= 0 || split_keys % 64 || !part_o || !part_ml || Q8)
@@ -357,19 +404,22 @@ void launch_attn_extend(const void* q, int64_t q_stride, const void* k_cache, co
   auto CL = (const int*)ctx_lens;
   auto O = (bf16_t*)out;
   const float sl = scale * kLog2eX;
+  const int bshift = bs > 0 && (bs & (bs - 1)) == 0 ? __builtin_ctz(bs) : -1;
   const bool same = !kv8 && k_cache == v_cache && nkv == 1;
   if (window < 0) throw std::runtime_error("attn_extend: negative window");
+#define LXN(D_, KV8_, SAME_, NS_)                                                                                      \
+  attn_extend_kernel<D_, KV8_, SAME_, NS_><<<grid, 256, 0, st>>>(Q, q_stride, K, V, BT, max_blocks, CU, CL, O, out_stride, nh, nkv, \
+                                                                 GE, bs, sl, Q8, S8, window, nsplit, split_keys, PO, PML, bshift)
 #define LX(D_)                                                                                                   \
   do {                                                                                                           \
-    if (kv8)                                                                                                     \
-      attn_extend_kernel<D_, true><<<grid, 256, 0, st>>>(Q, q_stride, K, V, BT, max_blocks, CU, CL, O, out_stride, nh, \
-                                                         nkv, GE, bs, sl, Q8, S8, window, nsplit, split_keys, PO, PML);                       \
-    else if (same)                                                                                               \
-      attn_extend_kernel<D_, false, true><<<grid, 256, 0, st>>>(Q, q_stride, K, V, BT, max_blocks, CU, CL, O,          \
-                                                                out_stride, nh, nkv, GE, bs, sl, Q8, S8, window, nsplit, split_keys, PO, PML); \
-    else                                                                                                         \
-      attn_extend_kernel<D_, false><<<grid, 256, 0, st>>>(Q, q_stride, K, V, BT, max_blocks, CU, CL, O, out_stride,   \
-                                                          nh, nkv, GE, bs, sl, Q8, S8, window, nsplit, split_keys, PO, PML);                  \
+    if (D_ <= 128 && two) {                                                                                      \
+      constexpr int D = D_ <= 128 ? D_ : 64; /* (no such kernel for heads of 256) */                              \
+      if (kv8) LXN(D, true, false, 2);                                                                           \
+      else if (same) LXN(D, false, true, 2);                                                                     \
+      else LXN(D, false, false, 2);                                                                              \
+    } else if (kv8) LXN(D_, true, false, 1);                                                                     \
+    else if (same) LXN(D_, false, true, 1);                                                                      \
+    else LXN(D_, false, false, 1);                                                                               \
   } while (0)
   switch (D) {
     case 64: LX(64); break;
@@ -378,6 +428,7 @@ void launch_attn_extend(const void* q, int64_t q_stride, const void* k_cache, co
     default: throw std::runtime_error("attn_extend: head_dim must be 64, 128 or 256");
   }
 #undef LX
+#undef LXN
   HIP_CHECK_LAUNCH();
   if (nsplit > 1) {
     // B single-token rows: token index = sequence index only when cu_q is 0, 1, .., B (the caller's contract)
