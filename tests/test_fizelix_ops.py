@@ -107,6 +107,43 @@ def test_sandwich_add_norm(device, dtype, W):
     close(got, oracle.rms(x + add, eps) * nn, dtype, "norm after it")
 
 
+@gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,W", [(3, 4), (5, 1020), (2, 1024), (4, 1028), (3, 2048), (6, 2052), (2, 4096), (513, 2052), (3, 4100)])
+@pytest.mark.parametrize("what", ["plain", "gated", "experts", "pair", "normed pair", "none"])
+def test_sandwich_add_norm_at_the_widths_of_its_kernels(dtype, T, W, what):
+    """Rows around what a workgroup's registers hold and around the number of rows that keeps the general kernel; every kind of y:
+    rows, gated rows, expert rows of one to six choices with shared ones, pairs; with and without addend and next norm."""
+    from llmss_amd.ops import hip as H
+
+    dev = lambda t, dt=torch.float32: t.to(device="cuda", dtype=dt).contiguous()
+    x, add = rnd(T, W, seed=1), rnd(T, W, seed=2)
+    wp, wn, rb = (1 + 0.1 * rnd(W, seed=k) for k in (3, 4, 5))
+    rms = lambda t: t / torch.sqrt(t.pow(2).mean(-1, keepdim=True) + 1e-5)
+    for k, (use_add, use_next) in enumerate(((False, True), (True, True), (True, False))):
+        y, r = rnd(T, W, seed=6 + k, dtype=dtype), rnd(T, W, seed=16 + k, dtype=dtype)
+        arg, gate = dev(y, dtype), None
+        if what == "gated":
+            gate, y = dev(r, dtype), y * torch.sigmoid(r + rb)
+        elif what == "experts":
+            top = (1, 4, 6)[k]
+            ey, wts, sw = rnd(T * top, W, seed=26 + k), rnd(T, top, seed=36 + k), rnd(T, seed=46 + k)
+            place = torch.randperm(T * top, generator=torch.Generator().manual_seed(k))
+            arg = H.MoEPending(dev(ey), place.to("cuda", torch.int32), dev(wts), dev(r, dtype), shared_w=dev(sw) if k else None)
+            y = (wts[..., None] * ey[place].view(T, top, W)).sum(1) + (sw[:, None] if k else 1) * r
+        elif what == "pair":
+            arg, y = ops.PairPending(arg, dev(r, dtype), None, None, (0.3, -1.7)), 0.3 * y - 1.7 * r
+        elif what == "normed pair":
+            arg, y = ops.PairPending(arg, dev(r, dtype), dev(wn), dev(rb)), 0.5 * (rms(y) * wn + rms(r) * rb)
+        xs = dev(x)
+        got = H.sandwich_add_norm(xs, None if what == "none" else arg, gate, dev(rb) if gate is not None else None,
+                                  None if what == "none" else dev(wp), 1e-5, dev(add) if use_add else None, dev(wn) if use_next else None, dtype)
+        want = x + (0 if what == "none" else rms(y) * wp) + (add if use_add else 0)
+        close(xs, want, torch.float32, "residual")
+        if use_next:
+            close(got, rms(want) * wn, dtype, "next input")
+
+
 @pytest.mark.parametrize("device,dtype", RUNS)
 @pytest.mark.parametrize("W,d,part", [(48, 6, 2), (50, 1, 0), (264, 19, 1)])
 def test_token_side_add(device, dtype, W, d, part):
