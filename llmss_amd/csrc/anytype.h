@@ -34,6 +34,21 @@ __device__ __forceinline__ void st4(T* p, f32x4 v) {
   else *reinterpret_cast<u16x4*>(p) = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
 }
 
+// Four columns of a product whose K was split: the sum of `slabs` fp32 slabs `stride` apart, eight loads in flight, added in their order
+__device__ __forceinline__ f32x4 slab_sum(const float* p, int slabs, int64_t stride) {
+  f32x4 a = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < slabs; s0 += 8) {
+    f32x4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const f32x4*>(p + min(s0 + j, slabs - 1) * stride);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[i] += s0 + j < slabs ? v[j][i] : 0.f;
+  }
+  return a;
+}
+
 // x as the sum of three bf16 numbers (cut off, not rounded: 8 bits each, 24 together, nothing left over), into place j of each
 __device__ __forceinline__ void split3(float x, int j, s16x8& h, s16x8& m, s16x8& l) {
   const float a = __uint_as_float(__float_as_uint(x) & 0xffff0000u), y = x - a;

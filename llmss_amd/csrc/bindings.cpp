@@ -132,7 +132,7 @@ void launch_embed_streams(const void* ids, const void* positions, const void* ta
                           int T_, int W, int vocab, int npos, int dt, hipStream_t st);
 void launch_stream_add_norm(void* x, const void* y, int64_t ldy, const void* mix, const void* outw, float c,
                             const void* inw, const void* w, float eps, int rms, void* h, int64_t ldh, int S, int T_,
-                            int W, int dt, int h_f32, hipStream_t st);
+                            int W, int dt, int h_f32, int slabs, hipStream_t st);
 void launch_causal_conv(const void* in, int64_t ldi, const void* w, void* state, const void* cu, const void* ctx,
                         const void* sslots, void* out, int64_t ldo, int T_, int B, int C, int taps, int res, int silu,
                         int di, int dw, int dout, const void* bias, int single, hipStream_t st);
@@ -199,7 +199,7 @@ void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const void* e
                               int top, const void* shared_, int64_t lds_, const void* r, int64_t ldr, const void* rb,
                               const void* wpost, const void* add, const void* wnext, void* h, int64_t ldh, float eps,
                               int groups, const void* ident, int64_t ldi, const void* y2, int64_t ldy2, const void* wl,
-                              const void* wr, float cl, float cr, int64_t lda, const void* sw, int T_, int W, int dt,
+                              const void* wr, float cl, float cr, int64_t lda, const void* sw, int slabs, int T_, int W, int dt,
                               hipStream_t st);
 void launch_token_side_add(void* x, const void* ids, const void* table, int64_t ldt, int vocab, int col0, int d,
                            const void* wg, const void* wp, const void* wn, const void* add, const void* wnext, void* h,
@@ -503,9 +503,9 @@ PYBIND11_MODULE(_C, m) {
   });
   m.def("stream_add_norm", [](uintptr_t x, uintptr_t y, int64_t ldy, uintptr_t mix, uintptr_t outw, float c,
                               uintptr_t inw, uintptr_t w, float eps, int rms, uintptr_t h, int64_t ldh, int Sn, int T,
-                              int W, int dt, int h_f32, uintptr_t st) {
+                              int W, int dt, int h_f32, int slabs, uintptr_t st) {
     launch_stream_add_norm(P(x), CP(y), ldy, CP(mix), CP(outw), c, CP(inw), CP(w), eps, rms, P(h), ldh, Sn, T, W, dt,
-                           h_f32, S(st));
+                           h_f32, slabs, S(st));
   });
   m.def("causal_conv", [](uintptr_t in, int64_t ldi, uintptr_t w, uintptr_t state, uintptr_t cu, uintptr_t ctx,
                           uintptr_t ss, uintptr_t out, int64_t ldo, int T, int B, int C, int taps, int res, int silu,
@@ -683,11 +683,11 @@ PYBIND11_MODULE(_C, m) {
                                 int top, uintptr_t sh, int64_t lds_, uintptr_t r, int64_t ldr, uintptr_t rb,
                                 uintptr_t wpost, uintptr_t add, uintptr_t wnext, uintptr_t h, int64_t ldh, float eps,
                                 int groups, uintptr_t ident, int64_t ldi, uintptr_t y2, int64_t ldy2, uintptr_t wl,
-                                uintptr_t wr, float cl, float cr, int64_t lda, uintptr_t sw, int T, int W, int dt,
-                                uintptr_t st) {
+                                uintptr_t wr, float cl, float cr, int64_t lda, uintptr_t sw, int slabs, int T, int W,
+                                int dt, uintptr_t st) {
     launch_sandwich_add_norm(P(x), CP(y), ldy, CP(ey), CP(place), CP(wts), top, CP(sh), lds_, CP(r), ldr, CP(rb),
                              CP(wpost), CP(add), CP(wnext), P(h), ldh, eps, groups, CP(ident), ldi, CP(y2), ldy2,
-                             CP(wl), CP(wr), cl, cr, lda, CP(sw), T, W, dt, S(st));
+                             CP(wl), CP(wr), cl, cr, lda, CP(sw), slabs, T, W, dt, S(st));
   });
   m.def("token_side_add", [](uintptr_t x, uintptr_t ids, uintptr_t table, int64_t ldt, int vocab, int col0, int d,
                              uintptr_t wg, uintptr_t wp, uintptr_t wn, uintptr_t add, uintptr_t wnext, uintptr_t h,

@@ -49,6 +49,7 @@ struct SandwichArgs {
   float cl, cr;
   int64_t lda;      // row stride of add (0: one row for all)
   const float* sw;  // [T] or null
+  int slabs;        // > 0: y is the fp32 slabs [slabs][T][W] of a product whose K was split (sandwich_rows_kernel alone)
 };
 
 template <typename T, int V>
@@ -272,6 +273,8 @@ __global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p) {
       } else {
         EACH(for (int e = 0; e < 4; ++e) v[i][e] = fmaf(p.cl, v[i][e], p.cr * y2[i][e]))
       }
+    } else if (p.slabs) {
+      EACH(v[i] = slab_sum((const float*)p.y + (int64_t)t * W + col[i], p.slabs, (int64_t)gridDim.x * W))
     } else if (p.y) {
       EACH(v[i] = ld4((const T*)p.y + (int64_t)t * p.ldy + col[i]))
     } else {
@@ -320,14 +323,14 @@ void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const void* e
                               int top, const void* shared_, int64_t lds_, const void* r, int64_t ldr, const void* rb,
                               const void* wpost, const void* add, const void* wnext, void* h, int64_t ldh, float eps,
                               int groups, const void* ident, int64_t ldi, const void* y2, int64_t ldy2, const void* wl,
-                              const void* wr, float cl, float cr, int64_t lda, const void* sw, int T_, int W, int dt,
+                              const void* wr, float cl, float cr, int64_t lda, const void* sw, int slabs, int T_, int W, int dt,
                               hipStream_t st) {
   if (T_ == 0) return;
   if (groups < 1 || W % groups) throw std::runtime_error("sandwich_add_norm: the norm's parts must divide the row");
   if (((size_t)W + groups) * 4 > 64 * 1024) throw std::runtime_error("sandwich_add_norm: rows wider than 16384");
   SandwichArgs p{(float*)x, y, ldy, (const float*)ey, (const int*)place, (const float*)wts, top, shared_, lds_, r, ldr,
                  (const float*)rb, (const float*)wpost, (const float*)add, (const float*)wnext, h, ldh, eps, W, groups, ident, ldi, y2, ldy2,
-                 (const float*)wl, (const float*)wr, cl, cr, lda, (const float*)sw};
+                 (const float*)wl, (const float*)wr, cl, cr, lda, (const float*)sw, slabs};
   const int es = dt == 0 ? 2 : 4;
   const auto alv = [&](const void* q, int64_t ld) { return !q || (((uintptr_t)q % (4 * es)) == 0 && ld % 4 == 0); };
   const bool vec = W % 4 == 0 && al16(x) && al16(ey) && al16(rb) && al16(wpost) && al16(add) && al16(wnext) &&
@@ -337,6 +340,7 @@ void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const void* e
   const int th = T_ <= 512 && W > 1024 ? 512 : 256;  // few rows: more waves to a row
   // (identity experts and norms in parts keep the general kernel)
   const bool rows = vec && groups == 1 && !ident && (W <= 2048 || (W <= 4096 && T_ <= 512));
+  if (slabs < 0 || (slabs && (!rows || !y || y2 || !al16(y)))) throw std::runtime_error("sandwich_add_norm: slabs of rows that fit the registers only");
   DISPATCH_T(dt, T, {
     if (rows && W <= 2048) sandwich_rows_kernel<T, 1><<<T_, W > 1024 ? 512 : 256, 0, st>>>(p);
     else if (rows) sandwich_rows_kernel<T, 2><<<T_, 512, 0, st>>>(p);

@@ -111,11 +111,12 @@ __global__ __launch_bounds__(256) void stream_add_norm_kernel(float* __restrict_
 // The same for up to four streams of rows of up to 4096: a thread keeps NC times four columns of every stream in registers, all
 // loads are issued before the first is used, and nothing passes through LDS but the two sums. The kernel above, with a load of four
 // bytes waited for at a time, is bound by latency: 8192 rows of 2048, two streams, bf16: 136 -> 59 us (5.7 TB/s).
+// slabs > 0: y is the fp32 slabs [slabs][T][W] of a product whose K was split, summed here instead of in a launch of their own.
 template <typename T, typename TH, int S, int NC>
 __global__ __launch_bounds__(256) void stream_rows_kernel(float* __restrict__ x, const T* __restrict__ y, int64_t ldy,
                                                           const float* __restrict__ mix, const float* __restrict__ outw, float c,
                                                           const float* __restrict__ inw, const T* __restrict__ w, float eps,
-                                                          int rms, TH* __restrict__ h, int64_t ldh, int T_, int W) {
+                                                          int rms, TH* __restrict__ h, int64_t ldh, int T_, int W, int slabs) {
   __shared__ float red[32];
   const int t = blockIdx.x;
   f32x4 xs[S][NC], yv[NC], wv[NC];
@@ -128,7 +129,8 @@ __global__ __launch_bounds__(256) void stream_rows_kernel(float* __restrict__ x,
     if (col < W) {
 #pragma unroll
       for (int s = 0; s < S; ++s) xs[s][i] = ld4(x + ((int64_t)s * T_ + t) * W + col);
-      if (y) yv[i] = ld4(y + (int64_t)t * ldy + col);
+      if (slabs) yv[i] = slab_sum((const float*)y + (int64_t)t * W + col, slabs, (int64_t)T_ * W);
+      else if (y) yv[i] = ld4(y + (int64_t)t * ldy + col);
       if (w) wv[i] = ld4(w + col);
     }
   }
@@ -190,15 +192,15 @@ __global__ __launch_bounds__(256) void stream_rows_kernel(float* __restrict__ x,
 
 template <typename T, typename TH, int S>
 void launch_stream_rows(float* x, const T* y, int64_t ldy, const float* mix, const float* outw, float c, const float* inw,
-                        const T* w, float eps, int rms, TH* h, int64_t ldh, int T_, int W, hipStream_t st) {
-  if (W <= 1024) stream_rows_kernel<T, TH, S, 1><<<T_, 256, 0, st>>>(x, y, ldy, mix, outw, c, inw, w, eps, rms, h, ldh, T_, W);
-  else if (W <= 2048) stream_rows_kernel<T, TH, S, 2><<<T_, 256, 0, st>>>(x, y, ldy, mix, outw, c, inw, w, eps, rms, h, ldh, T_, W);
-  else stream_rows_kernel<T, TH, S, 4><<<T_, 256, 0, st>>>(x, y, ldy, mix, outw, c, inw, w, eps, rms, h, ldh, T_, W);
+                        const T* w, float eps, int rms, TH* h, int64_t ldh, int T_, int W, int slabs, hipStream_t st) {
+  if (W <= 1024) stream_rows_kernel<T, TH, S, 1><<<T_, 256, 0, st>>>(x, y, ldy, mix, outw, c, inw, w, eps, rms, h, ldh, T_, W, slabs);
+  else if (W <= 2048) stream_rows_kernel<T, TH, S, 2><<<T_, 256, 0, st>>>(x, y, ldy, mix, outw, c, inw, w, eps, rms, h, ldh, T_, W, slabs);
+  else stream_rows_kernel<T, TH, S, 4><<<T_, 256, 0, st>>>(x, y, ldy, mix, outw, c, inw, w, eps, rms, h, ldh, T_, W, slabs);
 }
 
 void launch_stream_add_norm(void* x, const void* y, int64_t ldy, const void* mix, const void* outw, float c,
                             const void* inw, const void* w, float eps, int rms, void* h, int64_t ldh, int S, int T_,
-                            int W, int dt, int h_f32, hipStream_t st) {
+                            int W, int dt, int h_f32, int slabs, hipStream_t st) {
   if (T_ == 0) return;
   if (S < 1 || S > MAX_STREAMS) throw std::runtime_error("stream_add_norm: 1 to 8 streams");
   const size_t lds = (size_t)(W + 32) * 4;
@@ -207,9 +209,10 @@ void launch_stream_add_norm(void* x, const void* y, int64_t ldy, const void* mix
   const int es = dt == 0 ? 2 : 4, eh = h_f32 ? 4 : es;
   const bool rows4 = S <= 4 && W % 4 == 0 && W <= 4096 && ldy % 4 == 0 && ldh % 4 == 0 && !((uintptr_t)x & 15) &&
                      !(((uintptr_t)y | (uintptr_t)w) & (4 * es - 1)) && !((uintptr_t)h & (4 * eh - 1));
+  if (slabs < 0 || (slabs && (!y || !rows4 || ((uintptr_t)y & 15)))) throw std::runtime_error("stream_add_norm: slabs of rows of four only");
 #define LAUNCH_SR(TH_, S_)                                                                                           \
   launch_stream_rows<T, TH_, S_>((float*)x, (const T*)y, ldy, (const float*)mix, (const float*)outw, c, (const float*)inw, \
-                                 (const T*)w, eps, rms, (TH_*)h, ldh, T_, W, st)
+                                 (const T*)w, eps, rms, (TH_*)h, ldh, T_, W, slabs, st)
 #define LAUNCH_SAN(TH_)                                                                                              \
   if (rows4 && S == 1) LAUNCH_SR(TH_, 1);                                                                            \
   else if (rows4 && S == 2) LAUNCH_SR(TH_, 2);                                                                       \

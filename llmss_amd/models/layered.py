@@ -128,7 +128,7 @@ class LatentAttention:
         y = ops.head_expand(o, W.uv, dt)
         if W.gate_col is not None:
             y = ops.gate_mul(y, qc, W.gate_col)
-        return ops.linear_f(y, W.o, dt)
+        return ops.linear_f(y, W.o, dt, closing=model.closing)
 
 
 class DiffAttention:
@@ -159,7 +159,7 @@ class DiffAttention:
                           num_decode=0 if single else inp.num_decode, sink=False, chunk=spec.chunk, vshare=2,
                           precise=True)
         y = ops.diff_combine(O, W.lam, eps, 1.0 - spec.diff, H, G, spec.vdim, dt)
-        return ops.linear_f(y, W.o, dt)
+        return ops.linear_f(y, W.o, dt, closing=model.closing)
 
 
 class MoEFeedForward:
@@ -234,7 +234,7 @@ class DeltaMixer:
         dt = model.dtype
         y = torch.empty(h.shape[0], spec.heads * spec.vdim, dtype=dt, device=h.device)
         DeltaMixer.mix(model, W, spec, ops.linear_f(h, W.proj, dt), W.cols, inp, cu, caches[i][2], 1.0, y, dt)
-        return ops.linear_f(y, W.o, dt)
+        return ops.linear_f(y, W.o, dt, closing=model.closing)
 
 
 class ParallelMixer:
@@ -278,7 +278,7 @@ class ParallelMixer:
         # right: the gated delta rule
         DeltaMixer.mix(model, W, r, proj, {n: c["r" + n] for n in "qgab"}, inp, cu, st, spec.right_scale, both[:, nl:],
                        torch.float32)
-        return ops.linear_f(both, W.o, dt)
+        return ops.linear_f(both, W.o, dt, closing=model.closing)
 
 
 class DecayMixer:
@@ -309,7 +309,7 @@ class DecayMixer:
                                  num_decode=0 if inp.kind == "decode" else inp.num_decode)
         y = ops.gated_group_norm(o, proj[:, c["g"]:c["g"] + nv], W.norm, model.cfg.norm_eps, "sigmoid", 1.0,
                                  out_dtype=dt)
-        return ops.linear_f(y, W.o, dt)
+        return ops.linear_f(y, W.o, dt, closing=model.closing)
 
 
 class DenseFeedForward:
@@ -319,11 +319,11 @@ class DenseFeedForward:
     def forward(model: "LayeredLM", W, spec, h):
         dt = model.dtype
         if not spec.gated and spec.act in ("gelu", "relu2"):  # the activation rides in the GEMM's epilogue
-            return ops.linear_f(ops.linear_f(h, W.gu, dt, act=spec.act), W.down, dt)
+            return ops.linear_f(ops.linear_f(h, W.gu, dt, act=spec.act), W.down, dt, closing=model.closing)
         if not spec.gated:
-            return ops.linear_f(ops.act_fn(ops.linear_f(h, W.gu, dt), spec.act, W.act_params), W.down, dt)
+            return ops.linear_f(ops.act_fn(ops.linear_f(h, W.gu, dt), spec.act, W.act_params), W.down, dt, closing=model.closing)
         gu = model.proj = ops.linear_f(h, W.gu, dt)  # (columns past 2 ff: a sandwich block's gate logits)
-        return ops.linear_f(ops.glu_act(gu, spec.ff, spec.act), W.down, dt)
+        return ops.linear_f(ops.glu_act(gu, spec.ff, spec.act), W.down, dt, closing=model.closing)
 
 
 class PoolAttention:
@@ -370,7 +370,7 @@ class PoolAttention:
                                  spec.kv_heads, spec.dim, spec.vdim, spec.scale, spec.window, spec.pool, dt,
                                  max_qlen=1 if single else max(1, inp.max_seqlen),
                                  num_decode=0 if single else inp.num_decode, max_ctx=inp.max_ctx)
-        return ops.linear_f(y, W.o, dt)
+        return ops.linear_f(y, W.o, dt, closing=model.closing)
 
 
 class SSDMixer:
@@ -408,7 +408,7 @@ class SSDMixer:
                                num_decode=0 if inp.kind == "decode" else inp.num_decode)
         y = ops.gated_group_norm(y, proj[:, c["z"]:c["z"] + inner], W.norm, model.cfg.norm_eps, "silu", 1.0,
                                  out_dtype=dt, groups=spec.norm_groups, gate_first=True)
-        return ops.linear_f(y, W.o, dt)
+        return ops.linear_f(y, W.o, dt, closing=model.closing)
 
 
 class WindowAttention:
@@ -580,6 +580,10 @@ class LayeredLM:
         self._cu_decode = {}
         self._angles = {}
         self.tap = None  # tap(i, x): called with the fp32 residual after layer (run) i (debugging, tests)
+        # sublayers' outputs go straight into the residual streams' or the sandwich block's closing op, whose kernel of whole rows in
+        # registers takes the slabs of a split product too (a norm in one part, up to four streams, widths in fours)
+        self.closing = cfg.hidden_size % 4 == 0 and (
+            cfg.norm_groups == 1 if cfg.sandwich else not cfg.post_norm and not cfg.parallel_block and cfg.streams <= 4)
         self.proj = None  # the last sublayer's first GEMM output (a sandwich block reads its gate logits there)
 
     @property

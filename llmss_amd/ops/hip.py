@@ -893,10 +893,13 @@ def _mfma_ok(x, w, out_dtype) -> bool:
             and x.data_ptr() % 16 == 0 and (x.stride(0) * 2) % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-def linear_f(x, w, out_dtype, bias=None, act="none"):
+def linear_f(x, w, out_dtype, bias=None, act="none", closing=False):
     """act(x [M, K] . w [N, K]^T + bias) -> [M, N] in ``out_dtype`` with fp32 accumulation: the MFMA GEMM where it applies
     (bias and activation in its epilogue), else the tile GEMM or the strided VALU GEMM (fp32 storage, fp32 output, odd
-    shapes) and the activation in a launch of its own."""
+    shapes) and the activation in a launch of its own. ``closing``: the result goes straight into stream_add_norm or
+    sandwich_add_norm, which may be given the slabs of a product whose K was split (:class:`PartialSum`) instead: where rows are few
+    and fit a workgroup's registers, a launch to sum them costs more than reading them there (64 x 2048 x 5632 in eight slabs: 12.4 us with
+    its sum, 8.8 without)."""
     M, K = x.shape
     N = w.shape[0]
     _rows(x, "x")
@@ -907,6 +910,10 @@ def linear_f(x, w, out_dtype, bias=None, act="none"):
     if M == 0:
         return torch.empty(0, N, dtype=out_dtype, device=x.device)
     if _mfma_ok(x, w, out_dtype):
+        if closing and bias is None and M <= 64 and N <= 2048:
+            nt, split = lib().gemm_plan(M, N, K, False, False, False)
+            if split > 1:  # (the plan of the finished product, but for its sum)
+                return linear(x, w, nt_hint=nt, split_hint=split, partial_ok=True)
         return linear(x, w, bias, act)
     y = torch.empty(M, N, dtype=out_dtype, device=x.device)
     gemm_any(x, w, y, M, N, K, 1, 0, x.stride(0), 0, K, 1, 0, N, bias)
@@ -1238,14 +1245,18 @@ def embed_streams(ids, positions, table, pos_table, streams):
 def stream_add_norm(x, y, mix, outw, c, inw, w, eps, rms, out_dtype):
     S, T, W = x.shape
     _check(x.dtype == torch.float32 and x.is_contiguous() and x.is_cuda, "x fp32 [S, T, W] contiguous")
-    dt = None
+    dt, slabs = None, 0
     if y is not None:
-        _rows(y, "y", W)
-        _check(y.shape[0] == T, "y rows")
+        if isinstance(y, PartialSum):
+            _check(y.shape == (T, W) and y.bias is None, "partial y [T, W] without bias")
+            slabs = y.S
+        else:
+            _rows(y, "y", W)
+            _check(y.shape[0] == T, "y rows")
         _f32c(mix, "mix")
         _f32c(outw, "outw")
         _check(mix.numel() == S * S and outw.numel() == S, "mix [S, S], outw [S]")
-        dt = y.dtype
+        dt = torch.bfloat16 if slabs else y.dtype
     h = None
     if w is not None:
         _check(w.is_contiguous() and w.numel() == W and w.is_cuda, "norm weight [W]")
@@ -1259,9 +1270,10 @@ def stream_add_norm(x, y, mix, outw, c, inw, w, eps, rms, out_dtype):
     if dt is None or T == 0:
         return h
     _check(dt in _DT, "storage type bf16 / fp32")
-    lib().stream_add_norm(x.data_ptr(), _ptr(y), y.stride(0) if y is not None else 0, _ptr(mix), _ptr(outw), float(c),
+    lib().stream_add_norm(x.data_ptr(), y.buf.data_ptr() if slabs else _ptr(y),
+                          W if slabs else (y.stride(0) if y is not None else 0), _ptr(mix), _ptr(outw), float(c),
                           _ptr(inw) if w is not None else 0, _ptr(w), float(eps), int(bool(rms)), _ptr(h), W, S, T, W,
-                          _DT[dt], int(h is not None and h.dtype == torch.float32), _stream())
+                          _DT[dt], int(h is not None and h.dtype == torch.float32), slabs, _stream())
     return h
 
 
@@ -1749,15 +1761,18 @@ def diff_combine(O, lam, eps, mult, heads, kv_heads, vdim, out_dtype):
 
 # ------------------- blocks normed on both sides / token input / windowed sigmoid attention with pooled blocks / SSD
 def sandwich_add_norm(x, y, r, rb, wpost, eps, add, wnext, out_dtype, groups=1):
-    """``y``: rows in the storage type, a :class:`MoEPending` (combined while it is read) or a ``PairPending`` (the results
-    of two mixers, normed and joined while they are read)."""
+    """``y``: rows in the storage type, a :class:`MoEPending` (combined while it is read), a ``PairPending`` (the results
+    of two mixers, normed and joined while they are read) or a :class:`PartialSum` (summed while it is read)."""
     T, W = x.shape
     _rows(x, "x", dtype=torch.float32)
     _check(x.is_contiguous(), "x contiguous")
     _check(out_dtype in _DT, "storage type bf16 / fp32")
     pend = y if isinstance(y, MoEPending) else None
     pair = y if isinstance(y, PairPending) else None
+    part = y if isinstance(y, PartialSum) else None
     sh = None
+    if part is not None:
+        _check(part.shape == (T, W) and part.bias is None and out_dtype == torch.bfloat16, "partial y [T, W] without bias, bf16")
     if pair is not None:
         for t_, nm in ((pair.yl, "left"), (pair.yr, "right")):
             _rows(t_, nm, W, out_dtype)
@@ -1778,7 +1793,7 @@ def sandwich_add_norm(x, y, r, rb, wpost, eps, add, wnext, out_dtype, groups=1):
         sh = pend.shared
         if sh is not None:
             _rows(sh, "shared", W, out_dtype)
-    elif y is not None:
+    elif y is not None and part is None:
         _rows(y, "y", W, out_dtype)
         _check(y.shape[0] == T, "y rows")
     if y is not None:
@@ -1796,8 +1811,9 @@ def sandwich_add_norm(x, y, r, rb, wpost, eps, add, wnext, out_dtype, groups=1):
         _f32c(wnext, "wnext")
         _check(wnext.numel() == W, "wnext [W]")
         h = torch.empty(T, W, dtype=out_dtype, device=x.device)
-    dense = y if pend is None else None
-    lib().sandwich_add_norm(x.data_ptr(), _ptr(dense), dense.stride(0) if dense is not None else 0,
+    dense = y if pend is None and part is None else None
+    lib().sandwich_add_norm(x.data_ptr(), part.buf.data_ptr() if part else _ptr(dense),
+                            W if part else (dense.stride(0) if dense is not None else 0),
                             _ptr(pend.y) if pend else 0, _ptr(pend.place) if pend else 0,
                             _ptr(pend.wts) if pend else 0, pend.top if pend else 0, _ptr(sh),
                             sh.stride(0) if sh is not None else 0, _ptr(r) if y is not None else 0,
@@ -1807,7 +1823,7 @@ def sandwich_add_norm(x, y, r, rb, wpost, eps, add, wnext, out_dtype, groups=1):
                             _ptr(pair.yr) if pair else 0, pair.yr.stride(0) if pair else 0, _ptr(pair.wl) if pair else 0,
                             _ptr(pair.wr) if pair else 0, *(pair.scales if pair and pair.scales else (0.0, 0.0)),
                             W if add is not None and add.dim() == 2 else 0,
-                            _ptr(pend.shared_w) if pend else 0, T, W, _DT[out_dtype], _stream())
+                            _ptr(pend.shared_w) if pend else 0, part.S if part else 0, T, W, _DT[out_dtype], _stream())
     return h
 
 

@@ -474,8 +474,9 @@ def resid_add_norm(x: torch.Tensor, a, b, w, woff: float, eps: float, out_dtype,
 
 
 def linear_f(x: torch.Tensor, w: torch.Tensor, out_dtype, bias: Optional[torch.Tensor] = None,
-             act: str = "none") -> torch.Tensor:
-    """act(x [M, K] . w [N, K]^T + bias [N]) with fp32 accumulation -> [M, N] in ``out_dtype``."""
+             act: str = "none", closing: bool = False) -> torch.Tensor:
+    """act(x [M, K] . w [N, K]^T + bias [N]) with fp32 accumulation -> [M, N] in ``out_dtype``. ``closing``: a block's closing op takes
+    the result next (it only steers how the GPU kernels hand it over)."""
     y = x.float() @ w.float().t()
     return _act(y if bias is None else y + bias.float(), act).to(out_dtype)
 

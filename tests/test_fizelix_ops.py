@@ -144,6 +144,33 @@ def test_sandwich_add_norm_at_the_widths_of_its_kernels(dtype, T, W, what):
             close(got, rms(want) * wn, dtype, "next input")
 
 
+@gpu
+@pytest.mark.parametrize("M,N,K", [(33, 2048, 4096), (64, 1024, 5632), (65, 2048, 2048), (33, 1000, 2048), (8, 1024, 1024)])
+def test_closing_ops_sum_split_products(M, N, K):
+    """The product before a closing op as its kernel leaves it - slabs of a split K where rows are few - against the product finished
+    first: a sandwich block's close with gate and addend, and two residual streams. What is off is y's rounding to bf16 (2^-9)."""
+    from llmss_amd.ops import hip as H
+
+    torch.manual_seed(0)
+    r = lambda *s, dt=torch.float32: torch.randn(*s, device="cuda").to(dt)
+    a, w = r(M, K, dt=torch.bfloat16), (r(N, K) * K ** -0.5).to(torch.bfloat16)
+    y = lambda: H.linear_f(a, w, torch.bfloat16, closing=True)
+    assert isinstance(y(), H.PartialSum) == (M in (33, 64)), "which products leave slabs"
+    full = (a.float() @ w.float().T).to(torch.bfloat16)
+    x, gate, rb, wp, add, wn = r(M, N), r(M, N, dt=torch.bfloat16), r(N), r(N), r(M, N), r(N)
+    x2 = x.clone()
+    got = H.sandwich_add_norm(x, y(), gate, rb, wp, 1e-5, add, wn, torch.bfloat16)
+    want = H.sandwich_add_norm(x2, full, gate, rb, wp, 1e-5, add, wn, torch.bfloat16)
+    close(x, x2.cpu(), torch.bfloat16, "residual")
+    close(got, want.cpu(), torch.bfloat16, "next input")
+    xs, mix, outw, inw = r(2, M, N), r(2, 2), r(2), r(2)
+    xs2, nw = xs.clone(), wn.to(torch.bfloat16)
+    got = H.stream_add_norm(xs, y(), mix, outw, 0.7, inw, nw, 1e-5, False, torch.bfloat16)
+    want = H.stream_add_norm(xs2, full, mix, outw, 0.7, inw, nw, 1e-5, False, torch.bfloat16)
+    close(xs, xs2.cpu(), torch.bfloat16, "streams")
+    close(got, want.cpu(), torch.bfloat16, "next input of the streams")
+
+
 @pytest.mark.parametrize("device,dtype", RUNS)
 @pytest.mark.parametrize("W,d,part", [(48, 6, 2), (50, 1, 0), (264, 19, 1)])
 def test_token_side_add(device, dtype, W, d, part):
