@@ -36,56 +36,90 @@ __device__ __forceinline__ float glu_value(float g, float u, float limit, float 
 }
 
 // ------------------------------------------------------------------------------------------------ routing
-// A wave routes one token of up to 128 outputs: lane e holds the logits of e and e + 64 (bias added; -inf past the last); an
-// output's rank among all choice values (ties: the lower index first) says whether and where it is chosen. row: LDS, 16-byte
-// aligned, room for the outputs in whole fours.
-__device__ __forceinline__ void route_ranked(float (&sc)[2], float* row, const float* __restrict__ corr, int* __restrict__ idx,
+// L lanes route one token of up to L * J outputs: lane e holds the logits of e (and e + 64; bias added; -inf past the last) and what
+// corr adds to their scores; an output's rank among all choice values (ties: the lower index first) says whether and where it is
+// chosen. row: LDS, 16-byte aligned, room for the outputs in whole fours. (The reads of the row unrolled, groups of lanes no wider than the
+// outputs: with two outputs a lane and a wave a token whatever their number, this was a third of a prompt's routing.)
+template <int L, int J>
+__device__ __forceinline__ void route_ranked(float (&sc)[J], const float (&cr)[J], float* row, int* __restrict__ idx,
                                              float* __restrict__ wts, int E, int top, int norm, int smax) {
-  const int lane = threadIdx.x & 63;
-  float ch[2];
+  static_assert(L == 64 || J == 1, "several outputs a lane: whole waves");
+  const int lane = threadIdx.x & (L - 1);
+  auto all_max = [](float x) {
+#pragma unroll
+    for (int o = L / 2; o > 0; o >>= 1) x = fmaxf(x, __shfl_xor(x, o, 64));
+    return x;
+  };
+  auto all_sum = [](float x) {
+#pragma unroll
+    for (int o = L / 2; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    return x;
+  };
+  float ch[J];
   float mx = -INFINITY, den = 0.f;
-  if (smax) mx = warp_max(fmaxf(sc[0], sc[1]));
+  if (smax) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) mx = fmaxf(mx, sc[j]);
+    mx = all_max(mx);
+  }
   if (smax == 1) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) den += lane + 64 * j < E ? expf(sc[j] - mx) : 0.f;
-    den = warp_sum(den);
+    for (int j = 0; j < J; ++j) den += lane + 64 * j < E ? expf(sc[j] - mx) : 0.f;
+    den = all_sum(den);
   }
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < J; ++j) {
     const int e = lane + 64 * j;
     if (smax != 2 && e < E) sc[j] = smax ? expf(sc[j] - mx) / den : 1.f / (1.f + expf(-sc[j]));
-    ch[j] = e < E ? sc[j] + (corr ? corr[e] : 0.f) : -INFINITY;
+    ch[j] = e < E ? sc[j] + cr[j] : -INFINITY;
     if (!(ch[j] == ch[j])) ch[j] = -INFINITY;  // (a NaN ranks last: the ranks stay a permutation)
     if (e < ((E + 3) & ~3)) row[e] = ch[j];
   }
   __builtin_amdgcn_wave_barrier();
   __threadfence_block();
-  int rank[2] = {0, 0};
-  for (int e0 = 0; e0 < E; e0 += 4) {
+  int rank[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) rank[j] = 0;
+#pragma unroll 4
+  for (int e0 = 0; e0 < E; e0 += 4) {  // (the last four are filled up with -inf behind every output: they count for none)
     const f32x4 o = *reinterpret_cast<const f32x4*>(row + e0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (e0 + i >= E) continue;
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) rank[j] += o[i] > ch[j] || (o[i] == ch[j] && e0 + i < lane + 64 * j) ? 1 : 0;
-    }
+      for (int j = 0; j < J; ++j) rank[j] += o[i] > ch[j] || (o[i] == ch[j] && e0 + i < lane + 64 * j) ? 1 : 0;
   }
   float sum = 0.f;
-  bool in[2];
+  bool in[J];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < J; ++j) {
     in[j] = lane + 64 * j < E && rank[j] < top;
     if (smax == 2) sc[j] = expf(sc[j] - mx);  // (the largest is always chosen)
     sum += in[j] ? sc[j] : 0.f;
   }
-  sum = warp_sum(sum);
+  sum = all_sum(sum);
   const float inv = smax == 2 ? 1.f / sum : norm ? 1.f / (sum + 1e-20f) : 1.f;
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < J; ++j)
     if (in[j]) {
       idx[rank[j]] = lane + 64 * j;
       wts[rank[j]] = sc[j] * inv;
     }
+}
+
+// the same by a whole wave, corr in memory
+__device__ __forceinline__ void route_ranked(float (&sc)[2], float* row, const float* __restrict__ corr, int* __restrict__ idx,
+                                             float* __restrict__ wts, int E, int top, int norm, int smax) {
+  const int lane = threadIdx.x & 63;
+  float cr[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) cr[j] = corr && lane + 64 * j < E ? corr[lane + 64 * j] : 0.f;
+  if (E > 64) {
+    route_ranked<64, 2>(sc, cr, row, idx, wts, E, top, norm, smax);
+  } else {
+    float s1[1] = {sc[0]};
+    const float c1[1] = {cr[0]};
+    route_ranked<64, 1>(s1, c1, row, idx, wts, E, top, norm, smax);
+  }
 }
 
 // one wave per token; lanes over experts
@@ -171,6 +205,9 @@ void launch_moe_route(const void* z, const void* corr, void* idx, void* wts, int
 // Router logits and routing in one launch, for steps of few tokens (a decode step): one workgroup per token, its waves
 // share the experts' dot products z_e = h . W_r[e] (fp32 accumulation over lanes), then the token is routed
 // as moe_route_kernel does. A prompt's thousands of tokens take the matrix-core GEMM and moe_route instead.
+// Bound by the chain of a wave's reads (the weights are cold: the layer's experts went through the caches since), so the row and up to
+// three outputs' weights are asked for at once. 33 rows of
+// 2048, 33 outputs: 10.2 -> 6.6 us, 8 rows of 1024, 17 outputs: 5.1 -> 3.9 (each with the faster routing above)
 template <typename T>
 __global__ __launch_bounds__(1024) void moe_router_kernel(const T* __restrict__ h, int64_t ldh, const T* __restrict__ wr,
                                                          const float* __restrict__ corr, int* __restrict__ idx,
@@ -182,37 +219,69 @@ __global__ __launch_bounds__(1024) void moe_router_kernel(const T* __restrict__ 
   const bool ranked = E <= 128;
   const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;
   const T* x = h + (int64_t)t * ldh;
-  for (int e = wv; e < E + (sg ? 1 : 0); e += nw) {
-    const T* w = wr + (int64_t)e * K;
-    float acc = 0.f;
-    if (vec) {  // K % 8 == 0, rows 16-byte aligned - eight elements per lane, two or four 16-byte accesses
-      typedef T vec8 __attribute__((ext_vector_type(8)));
-#pragma unroll 4
-      for (int k = lane * 8; k < K; k += 512) {
-        const vec8 xv = *reinterpret_cast<const vec8*>(x + k), wv = *reinterpret_cast<const vec8*>(w + k);
+  const int EG = E + (sg ? 1 : 0);
+  auto put = [&](int e, float acc) {  // (one lane) an output's sum over K
+    if (e == E) {
+      sg[t] = 1.f / (1.f + expf(-acc));
+      return;
+    }
+    if (zb) acc += zb[e];
+    if (ranked) {
+      sc[e] = acc;
+      return;
+    }
+    const float s = smax ? acc : 1.f / (1.f + expf(-acc));
+    sc[e] = s;
+    ch[e] = s + (corr ? corr[e] : 0.f);
+  };
+  if (vec) {  // K % 8 == 0, rows 16-byte aligned - eight elements per lane, two or four 16-byte accesses
+    typedef T vec8 __attribute__((ext_vector_type(8)));
+    constexpr int U = sizeof(T) == 2 ? 4 : 2;  // chunks of 512 numbers in flight
+    auto dots = [&](int e0, auto n_c) {        // outputs e0, e0 + nw, ..
+      constexpr int NE = decltype(n_c)::value;
+      float acc[NE];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const T xi = xv[i], wi = wv[i];
-          acc = fmaf(El<T>::ld(&xi), El<T>::ld(&wi), acc);
+      for (int n = 0; n < NE; ++n) acc[n] = 0.f;
+      for (int k0 = lane * 8; k0 < K; k0 += 512 * U) {
+        vec8 xv[U], wt[NE][U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int k = min(k0 + 512 * u, K - 8);
+          xv[u] = *reinterpret_cast<const vec8*>(x + k);
+#pragma unroll
+          for (int n = 0; n < NE; ++n) wt[n][u] = *reinterpret_cast<const vec8*>(wr + (int64_t)(e0 + n * nw) * K + k);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // all loads are issued before the first sum waits for one
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (k0 + 512 * u >= K) break;
+#pragma unroll
+          for (int n = 0; n < NE; ++n)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const T xi = xv[u][i], wi = wt[n][u][i];
+              acc[n] = fmaf(El<T>::ld(&xi), El<T>::ld(&wi), acc[n]);
+            }
         }
       }
-    } else {
-      for (int k = lane; k < K; k += 64) acc = fmaf(El<T>::ld(x + k), El<T>::ld(w + k), acc);
+#pragma unroll
+      for (int n = 0; n < NE; ++n) {
+        acc[n] = warp_sum(acc[n]);
+        if (lane == 0) put(e0 + n * nw, acc[n]);
+      }
+    };
+    for (int e0 = wv; e0 < EG; e0 += 3 * nw) {
+      if (e0 + 2 * nw < EG) dots(e0, std::integral_constant<int, 3>{});
+      else if (e0 + nw < EG) dots(e0, std::integral_constant<int, 2>{});
+      else dots(e0, std::integral_constant<int, 1>{});
     }
-    acc = warp_sum(acc);
-    if (lane == 0) {
-      if (e == E) {
-        sg[t] = 1.f / (1.f + expf(-acc));
-        continue;
-      }
-      if (zb) acc += zb[e];
-      if (ranked) {
-        sc[e] = acc;
-        continue;
-      }
-      const float s = smax ? acc : 1.f / (1.f + expf(-acc));
-      sc[e] = s;
-      ch[e] = s + (corr ? corr[e] : 0.f);
+  } else {
+    for (int e = wv; e < EG; e += nw) {
+      const T* w = wr + (int64_t)e * K;
+      float acc = 0.f;
+      for (int k = lane; k < K; k += 64) acc = fmaf(El<T>::ld(x + k), El<T>::ld(w + k), acc);
+      acc = warp_sum(acc);
+      if (lane == 0) put(e, acc);
     }
   }
   __syncthreads();
@@ -363,6 +432,100 @@ __global__ __launch_bounds__(512) void moe_router_mfma_kernel(const bf16_t* __re
   }
 }
 
+// Up to 48 outputs: both operands through LDS. The form above reads 16 bytes of 16 rows side by side, neighbouring lanes in different
+// rows, and gets 12 KB a microsecond into a CU; here a wave reads whole kilobytes of a row, 512 numbers of 16 * TG tokens and all outputs
+// a stage (rows dealt to the waves), the next stage in registers behind the products of this one. A wave's products are two of a stage's
+// sixteen steps of 32; parts and routing as above. Rows of 520 numbers in LDS: 16 rows' pieces lie in 64 different banks. 8261 rows of
+// 2048, 33 outputs: 41.6 -> 15.5 us, 8192 rows, 32 outputs: 20.6 -> 11.4, 300 rows: 15.0 -> 7.5.
+template <int OR, int TG>
+__global__ __launch_bounds__(512, 4) void moe_router_tile_kernel(const bf16_t* __restrict__ h, int64_t ldh,
+                                                                 const bf16_t* __restrict__ wr, const float* __restrict__ corr,
+                                                                 int* __restrict__ idx, float* __restrict__ wts, int T_, int E,
+                                                                 int K, int top, int norm, int smax,
+                                                                 const float* __restrict__ zb, float* __restrict__ sg) {
+  constexpr int NT = (OR + 15) / 16, LD = 16 * NT + 4, KS = 512, LDK = KS + 8, ROWS = 16 * TG + OR, NL = ROWS / 8;
+  constexpr int BYTES = ROWS * LDK * 2 > 4 * 16 * TG * LD * 4 ? ROWS * LDK * 2 : 4 * 16 * TG * LD * 4;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[BYTES];
+  bf16_t* st = reinterpret_cast<bf16_t*>(smem);                    // [ROWS][LDK]: tokens, then outputs
+  float(*part)[16 * TG][LD] = reinterpret_cast<float(*)[16 * TG][LD]>(smem);  // (after the last product)
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, g = lane >> 4;
+  const int t0 = blockIdx.x * 16 * TG, EG = E + (sg ? 1 : 0);
+  f32x4 acc[TG][NT];
+#pragma unroll
+  for (int n = 0; n < TG; ++n)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[n][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u16x8 v[NL];
+  auto load = [&](int k0) {
+    const int k = min(k0 + lane * 8, K - 8);
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int r = w + 8 * i;  // (16 * TG is a multiple of 8: a load is of tokens or of outputs in every wave)
+      const bf16_t* row = i < 2 * TG ? h + (int64_t)min(t0 + r, T_ - 1) * ldh : wr + (int64_t)min(r - 16 * TG, EG - 1) * K;
+      v[i] = *reinterpret_cast<const u16x8*>(row + k);
+    }
+  };
+  load(0);
+  for (int k0 = 0; k0 < K; k0 += KS) {
+    if (k0) __syncthreads();  // every wave has read the stage before
+#pragma unroll
+    for (int i = 0; i < NL; ++i) *reinterpret_cast<u16x8*>(st + (w + 8 * i) * LDK + lane * 8) = v[i];
+    __syncthreads();
+    if (k0 + KS < K) load(k0 + KS);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int ks = w + 8 * u;
+      if (k0 + 32 * ks >= K) break;  // (K a multiple of 32)
+      s16x8 av[TG], bv[NT];
+#pragma unroll
+      for (int n = 0; n < TG; ++n) av[n] = *reinterpret_cast<const s16x8*>(st + (16 * n + li) * LDK + 32 * ks + 8 * g);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) bv[j] = *reinterpret_cast<const s16x8*>(st + min(16 * (TG + j) + li, ROWS - 1) * LDK + 32 * ks + 8 * g);
+#pragma unroll
+      for (int n = 0; n < TG; ++n)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[n][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[n], bv[j], acc[n][j], 0, 0, 0);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {  // waves 4 - 7 leave theirs, then 0 - 3 add their own
+    if (half ? w < 4 : w >= 4) {
+#pragma unroll
+      for (int n = 0; n < TG; ++n)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float& z = part[w & 3][16 * n + 4 * g + i][16 * j + li];
+            z = half ? z + acc[n][j][i] : acc[n][j][i];
+          }
+    }
+    __syncthreads();
+  }
+  // a wave routes 2 * TG tokens, as many at once as groups of lanes fit (the gate's output is one of the columns, none of the experts)
+  auto route = [&](auto lanes_c) {
+    constexpr int LN = decltype(lanes_c)::value;
+    const int e = lane & (LN - 1);
+    float cr[1] = {corr && e < E ? corr[e] : 0.f};
+    const float b = zb && e < E ? zb[e] : 0.f;
+#pragma unroll
+    for (int r0 = 0; r0 < 2 * TG; r0 += 64 / LN) {
+      const int r = 2 * TG * w + r0 + lane / LN;
+      const int64_t t = t0 + r;
+      if (r0 + lane / LN >= 2 * TG || t >= T_) continue;
+      auto z_of = [&](int c) { return (part[0][r][c] + part[1][r][c]) + (part[2][r][c] + part[3][r][c]); };
+      float sc[1] = {e < E ? z_of(e) + b : -INFINITY};
+      if (sg && e == 0) sg[t] = 1.f / (1.f + expf(-z_of(E)));
+      __builtin_amdgcn_wave_barrier();
+      route_ranked<LN, 1>(sc, cr, &part[0][r][0], idx + t * top, wts + t * top, E, top, norm, smax);  // (the row is this group's alone)
+    }
+  };
+  if (E <= 16) route(std::integral_constant<int, 16>{});
+  else if (E <= 32) route(std::integral_constant<int, 32>{});
+  else route(std::integral_constant<int, 64>{});
+}
+
 // may a router of E outputs (+ gate) over bf16 rows of K numbers take the matrix-core form?
 bool moe_router_mfma_ok(int E, int gate, int K) { return E + (gate ? 1 : 0) <= 16 * MR_NT && E <= 128 && K % 32 == 0; }
 
@@ -376,32 +539,81 @@ void launch_moe_router_mfma(const void* h, int64_t ldh, const void* wr, const vo
   moe_router_mfma_kernel<NT_><<<(T_ + 15) / 16, 512, 0, st>>>((const bf16_t*)h, ldh, (const bf16_t*)wr, (const float*)corr, \
                                                               (int*)idx, (float*)wts, T_, E, K, top, norm, smax,            \
                                                               (const float*)zb, (float*)sg)
-  const int nt = (E + (sg ? 1 : 0) + 15) / 16;
-  if (nt <= 1) LAUNCH_MR(1);
-  else if (nt <= 2) LAUNCH_MR(2);
-  else if (nt <= 3) LAUNCH_MR(3);
-  else if (nt <= 5) LAUNCH_MR(5);
+#define LAUNCH_MRT(OR_, TG_)                                                                                              \
+  moe_router_tile_kernel<OR_, TG_><<<(T_ + 16 * TG_ - 1) / (16 * TG_), 512, 0, st>>>(                                     \
+      (const bf16_t*)h, ldh, (const bf16_t*)wr, (const float*)corr, (int*)idx, (float*)wts, T_, E, K, top, norm, smax,    \
+      (const float*)zb, (float*)sg)
+#define LAUNCH_MRT_T(OR_)              \
+  do {                                 \
+    if (two) LAUNCH_MRT(OR_, 2);       \
+    else LAUNCH_MRT(OR_, 1);           \
+  } while (0)
+  const int eg = E + (sg ? 1 : 0);
+  const bool two = T_ > 4096;  // (until then 16 tokens a workgroup are a CU's share: 4096 rows of 2048 8.8 us, 4097 rows 11.1)
+  if (eg <= 16) LAUNCH_MRT_T(16);
+  else if (eg <= 32) LAUNCH_MRT_T(32);
+  else if (eg <= 40) LAUNCH_MRT_T(40);  // (two workgroups of 32 tokens to a CU's LDS)
+  else if (eg <= 48) LAUNCH_MRT_T(48);
+  else if (eg <= 80) LAUNCH_MR(5);
   else LAUNCH_MR(MR_NT);
+#undef LAUNCH_MRT_T
+#undef LAUNCH_MRT
 #undef LAUNCH_MR
   HIP_CHECK_LAUNCH();
 }
 
 // ------------------------------------------------------------------------------------------------ grouping
-// One workgroup. meta = [ntiles | off[E + 1] | tile_expert[maxt] | tile_row0[maxt]], order [P], place [P].
+// meta = [ntiles | off[E + 1] | tile_expert[maxt] | tile_row0[maxt]], order [P], place [P].
+// One wave turns the experts' counts into their first rows (off, and `cur` in LDS for the caller's own use) and the list of tiles: a lane an
+// expert, sums over the lanes. meta null: only `cur`.
+__device__ __forceinline__ void group_scan(const int* cnt, int* cur, int E, int maxt, int tile_rows, int* meta) {
+  const int lane = threadIdx.x & 63;
+  int* off = meta + 1;
+  int* tile_e = meta + 1 + (E + 1);
+  int* tile_r = tile_e + maxt;
+  int o = 0, nt = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int e = e0 + lane, c = e < E ? cnt[e] : 0, t = (c + tile_rows - 1) / tile_rows;
+    int so = c, st = t;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int uo = __shfl_up(so, d, 64), ut = __shfl_up(st, d, 64);
+      so += lane >= d ? uo : 0;
+      st += lane >= d ? ut : 0;
+    }
+    const int eo = o + so - c, et = nt + st - t;
+    if (e < E) {
+      cur[e] = eo;
+      if (meta) {
+        off[e] = eo;
+        for (int i = 0; i < t && et + i < maxt; ++i) {
+          tile_e[et + i] = e;
+          tile_r[et + i] = eo + i * tile_rows;
+        }
+      }
+    }
+    o += __shfl(so, 63, 64);
+    nt += __shfl(st, 63, 64);
+  }
+  if (meta && lane == 0) {
+    off[E] = o;
+    meta[0] = nt < maxt ? nt : maxt;
+  }
+}
+
+// One workgroup, for steps of few pairs. Bound by its chain: the counts, their sums, the rows. (With the sums formed by one thread, an
+// expert after the other, and the pairs read twice: 132 pairs of 32 experts 6.3 us, 2.7 here.)
 __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__ idx, int P, int E, int maxt,
                                                          int* __restrict__ meta, int* __restrict__ order,
                                                          int* __restrict__ place, int tile_rows) {
   extern __shared__ int sm[];  // cnt[E], cur[E]
   int* cnt = sm;
   int* cur = sm + E;
-  int* off = meta + 1;
-  int* tile_e = meta + 1 + (E + 1);
-  int* tile_r = tile_e + maxt;
   for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
   constexpr int U = 8;  // pairs per thread whose loads and atomics are in flight together
+  int e[U];
   for (int p0 = threadIdx.x; p0 < P; p0 += blockDim.x * U) {
-    int e[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int p = p0 + u * blockDim.x;
@@ -412,32 +624,19 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
       if (e[u] < E) atomicAdd(&cnt[e[u]], 1);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int o = 0, nt = 0;
-    for (int e = 0; e < E; ++e) {
-      off[e] = o;
-      cur[e] = o;
-      for (int r = 0; r < cnt[e]; r += tile_rows) {
-        if (nt < maxt) {
-          tile_e[nt] = e;
-          tile_r[nt] = o + r;
-        }
-        ++nt;
-      }
-      o += cnt[e];
-    }
-    off[E] = o;
-    meta[0] = nt < maxt ? nt : maxt;
-  }
+  if (threadIdx.x < 64) group_scan(cnt, cur, E, maxt, tile_rows, meta);
   __syncthreads();
   // rows within an expert take whatever order the atomics give: every pair's row is computed on its own, so the
   // values do not depend on where the row lands
+  const bool again = P > (int)blockDim.x * U;  // (else the experts are still at hand)
   for (int p0 = threadIdx.x; p0 < P; p0 += blockDim.x * U) {
-    int e[U], o[U];
+    int o[U];
+    if (again) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int p = p0 + u * blockDim.x;
-      e[u] = p < P ? idx[p] : E;
+      for (int u = 0; u < U; ++u) {
+        const int p = p0 + u * blockDim.x;
+        e[u] = p < P ? idx[p] : E;
+      }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) o[u] = e[u] < E ? atomicAdd(&cur[e[u]], 1) : -1;  // (-1: an identity expert, no row of its own)
@@ -451,11 +650,65 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
   }
 }
 
-void launch_moe_group(const void* idx, int P, int E, int maxt, void* meta, void* order, void* place, int tile_rows,
+// Many pairs: 1024 of them a workgroup. One launch leaves every workgroup's counts behind `meta`, the next sums those of all workgroups and
+// of the ones before its own, and hands out the rows from there. One workgroup alone is bound by its LDS atomics, two a pair:
+// 33044 pairs of 32 experts 46 us with the sums above by one thread, 19.6, in two launches 6.0; 2048 pairs 3.4 and 4.4, 4096 pairs 4.4
+// and 4.8, 8192 pairs 6.5 and 5.1.
+__global__ __launch_bounds__(1024) void moe_count_kernel(const int* __restrict__ idx, int P, int E, int* __restrict__ hist) {
+  extern __shared__ int sm[];  // cnt[E]
+  for (int e = threadIdx.x; e < E; e += 1024) sm[e] = 0;
+  __syncthreads();
+  const int p = blockIdx.x * 1024 + threadIdx.x, e = p < P ? idx[p] : E;
+  if (e < E) atomicAdd(&sm[e], 1);
+  __syncthreads();
+  for (int i = threadIdx.x; i < E; i += 1024) hist[(int64_t)blockIdx.x * E + i] = sm[i];
+}
+
+__global__ __launch_bounds__(1024) void moe_place_kernel(const int* __restrict__ idx, int P, int E, int maxt,
+                                                         const int* __restrict__ hist, int* __restrict__ meta,
+                                                         int* __restrict__ order, int* __restrict__ place, int tile_rows) {
+  extern __shared__ int sm[];  // cnt[E], cur[E], before[E]
+  int* cnt = sm;
+  int* cur = sm + E;
+  int* before = sm + 2 * E;
+  const int p = blockIdx.x * 1024 + threadIdx.x, e = p < P ? idx[p] : E;
+  for (int i = threadIdx.x; i < E; i += 1024) cnt[i] = before[i] = 0;
+  __syncthreads();
+  const int n = gridDim.x * E, own = blockIdx.x * E;
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    const int c = hist[i];
+    if (c == 0) continue;
+    atomicAdd(&cnt[i % E], c);
+    if (i < own) atomicAdd(&before[i % E], c);
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) group_scan(cnt, cur, E, maxt, tile_rows, blockIdx.x == 0 ? meta : nullptr);
+  __syncthreads();
+  if (p >= P) return;
+  int o = -1;
+  if (e < E) {
+    o = cur[e] + atomicAdd(&before[e], 1);
+    order[o] = p;
+  }
+  place[p] = o;
+}
+
+// blocks > 1: workgroups of 1024 pairs, and `meta` has room for blocks * E counts behind its 2 + E + 2 * maxt numbers
+void launch_moe_group(const void* idx, int P, int E, int maxt, void* meta, void* order, void* place, int tile_rows, int blocks,
                       hipStream_t st) {
   if (P == 0) return;
   if (tile_rows <= 0) throw std::runtime_error("moe_group: tile rows");
   if (E > 4096) throw std::runtime_error("moe_group: more than 4096 experts");
+  if (blocks > 1) {
+    if (blocks != (P + 1023) / 1024 || (int64_t)blocks * E > 0x7fffffff) throw std::runtime_error("moe_group: workgroups of 1024 pairs");
+    int* hist = (int*)meta + 2 + E + 2 * (int64_t)maxt;
+    moe_count_kernel<<<blocks, 1024, E * sizeof(int), st>>>((const int*)idx, P, E, hist);
+    HIP_CHECK_LAUNCH();
+    moe_place_kernel<<<blocks, 1024, 3 * E * sizeof(int), st>>>((const int*)idx, P, E, maxt, hist, (int*)meta, (int*)order,
+                                                                (int*)place, tile_rows);
+    HIP_CHECK_LAUNCH();
+    return;
+  }
   moe_group_kernel<<<1, 1024, 2 * E * sizeof(int), st>>>((const int*)idx, P, E, maxt, (int*)meta, (int*)order,
                                                           (int*)place, tile_rows);
   HIP_CHECK_LAUNCH();

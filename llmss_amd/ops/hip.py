@@ -1081,7 +1081,7 @@ def moe_route(z, corr, top, normalize=True, score="sigmoid", bias=None, gate=Fal
     return (idx, wts, sg) if gate else (idx, wts)
 
 
-ROUTER_MFMA_MIN_ROWS = 256  # from here on a workgroup per token reads the router's weights too often
+ROUTER_MFMA_MIN_ROWS = 256  # until then a workgroup per token is as fast: 33 outputs of 2048 numbers 7.1 us at 256 rows, 7.5 on the matrix cores
 ROUTER_FUSED_MAX_ROWS = 1024  # steps of at most this many tokens compute logits and routing in one launch
 
 
@@ -1119,6 +1119,7 @@ _MOE_PP = os.environ.get("LLMSS_MOE_PP", "1") != "0"  # 0: grouped products on t
 MOE_PP_ROWS_TWO, MOE_PP_ROWS = 256, 128
 # And up to which those of 16 rows are: the same three layers gain 1.05 - 1.4 at 4 pairs, 1.0 - 1.5 at 8, 0.8 - 1.3 at 16, 0.65 - 1.1 at 24.
 MOE_DEC_ROWS = 8
+MOE_GROUP_PAIRS = 4096  # pairs up to which one workgroup groups them: 4096 in 4.4 us (4.8 in two launches), 8192 in 6.5 (5.1)
 
 
 def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=True, act="glu_clamp",
@@ -1172,7 +1173,8 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     maxt = -(-P // rows) + min(E, P)
     _check(maxt <= 65535, "too many (token, expert) pairs in one step")
     dev = h.device
-    meta = torch.empty(1 + (E + 1) + 2 * maxt, dtype=torch.int32, device=dev)
+    blocks = -(-P // 1024) if P > MOE_GROUP_PAIRS else 1  # (each leaves its counts behind meta)
+    meta = torch.empty(1 + (E + 1) + 2 * maxt + (blocks * E if blocks > 1 else 0), dtype=torch.int32, device=dev)
     order = torch.empty(P, dtype=torch.int32, device=dev)
     place = torch.empty(P, dtype=torch.int32, device=dev)
     act_ = torch.empty(P, F, dtype=h.dtype, device=dev)
@@ -1182,7 +1184,7 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     pw, silu = (wts.data_ptr() if weight_input else 0), int(act == "silu")
     L = lib()
     st = _stream()
-    L.moe_group(idx.data_ptr(), P, E, maxt, meta.data_ptr(), order.data_ptr(), place.data_ptr(), rows, st)
+    L.moe_group(idx.data_ptr(), P, E, maxt, meta.data_ptr(), order.data_ptr(), place.data_ptr(), rows, blocks, st)
     if pp:
         if gate is not None:
             L.moe_pp_glu(h.data_ptr(), h.stride(0), gate.data_ptr(), up.data_ptr(), meta.data_ptr(), order.data_ptr(),
