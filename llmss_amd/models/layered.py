@@ -400,7 +400,7 @@ class SSDMixer:
         inner, gn = spec.inner, spec.groups * spec.state
         proj = model.proj = ops.linear_f(h, W.proj, dt)
         xbc = ops.causal_conv(proj[:, c["xbc"]:c["xbc"] + spec.conv_channels], W.conv, st["tail"], cu, inp.ctx_lens,
-                              inp.state_slots, False, True, dt, bias=W.conv_b)
+                              inp.state_slots, False, True, dt, bias=W.conv_b, single=inp.kind == "decode")
         y = ops.ssd_recurrence(xbc[:, :inner], xbc[:, inner:inner + gn], xbc[:, inner + gn:],
                                proj[:, c["dt"]:c["dt"] + spec.heads], W.A_log, W.dt_bias, W.D, st["S"], cu,
                                inp.ctx_lens, inp.state_slots, spec.heads, spec.groups, spec.state, spec.vdim,
