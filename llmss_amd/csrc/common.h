@@ -117,6 +117,13 @@ __device__ __forceinline__ float silu(float x) { return x / (1.f + __expf(-x)); 
 
 enum Act : int { ACT_NONE = 0, ACT_GELU_TANH = 1, ACT_GELU = 2, ACT_RELU = 3, ACT_SILU_GLU = 4, ACT_RELU2 = 5 };
 
+// the gate of a gated product (glu): SiLU, or the tanh form of GELU where the product's activation says so, as g / (1 + exp(-2 z)), which
+// is 0.5 g (1 + tanh(z)) without the cancellation where tanh nears -1
+__device__ __forceinline__ float gelu_gate(float g) {
+  return g / (1.f + __expf(-1.5957691216057308f * (g + 0.044715f * g * g * g)));
+}
+__device__ __forceinline__ float glu_gate(float g, int act) { return act == ACT_GELU_TANH ? gelu_gate(g) : silu(g); }
+
 __device__ __forceinline__ float apply_act(float x, int act) {
   switch (act) {
     case ACT_GELU_TANH: return gelu_tanh(x);
@@ -396,7 +403,7 @@ __device__ __forceinline__ void img_store_rows(const float* ct, int rows, int r0
         }
       }
     }
-  } else if (glu) {  // out col 16p + j = silu(gate col 32p + j) * up col 32p + 16 + j, 8 per thread-step
+  } else if (glu) {  // out col 16p + j = gate(gate col 32p + j) * up col 32p + 16 + j, 8 per thread-step
     constexpr int VPR = BN / 16;
     for (int v = threadIdx.x; v < rows * VPR; v += NTHR) {
       const int r = v / VPR, oc = (v - r * VPR) * 8;
@@ -411,7 +418,7 @@ __device__ __forceinline__ void img_store_rows(const float* ct, int rows, int r0
       for (int e = 0; e < 8; ++e) {
         float gv = gx[e], uv = ux[e];
         if (bias) { gv += bf2f(bias[ng + e]); uv += bf2f(bias[ng + 16 + e]); }
-        o[e] = f2bf(silu(gv) * uv);
+        o[e] = f2bf(glu_gate(gv, act) * uv);
       }
       bf16_t* dst = Y + (int64_t)m * ldy + n0 / 2 + oc;
       if (ng + 16 + 7 < N && (ldy & 7) == 0) *reinterpret_cast<u16x8*>(dst) = o;

@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256, 2) void gemm_stream_kernel(const bf16_t* __res
           if (nu < N) {
             const float gv = epi_value(acc[mt][2 * p][i], ng, wscale, bias, ACT_NONE);
             const float uv = epi_value(acc[mt][2 * p + 1][i], nu, wscale, bias, ACT_NONE);
-            Y[(int64_t)m * ldy + n0 / 2 + p * 16 + li] = f2bf(silu(gv) * uv);
+            Y[(int64_t)m * ldy + n0 / 2 + p * 16 + li] = f2bf(glu_gate(gv, act) * uv);
           }
         }
       } else {
@@ -381,7 +381,7 @@ __global__ __launch_bounds__(256, 2) void gemm_stream2_kernel(const bf16_t* __re
           if (nu < N) {
             const float gv = epi_value(acc[mt][2 * p][i], ng, wscale, bias, ACT_NONE);
             const float uv = epi_value(acc[mt][2 * p + 1][i], nu, wscale, bias, ACT_NONE);
-            Y[(int64_t)m * ldy + n0 / 2 + p * 16 + li] = f2bf(silu(gv) * uv);
+            Y[(int64_t)m * ldy + n0 / 2 + p * 16 + li] = f2bf(glu_gate(gv, act) * uv);
           }
         }
       } else {
@@ -422,7 +422,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
       const int ng = 32 * p + i, nu = ng + 16;
       float gv = slab_sum(part, S, stride, (int64_t)m * N + ng), uv = slab_sum(part, S, stride, (int64_t)m * N + nu);
       if (bias) { gv += bf2f(bias[ng]); uv += bf2f(bias[nu]); }
-      Y[(int64_t)m * ldy + c] = f2bf(silu(gv) * uv);
+      Y[(int64_t)m * ldy + c] = f2bf(glu_gate(gv, act) * uv);
     } else {
       float v = slab_sum(part, S, stride, (int64_t)m * N + c);
       if (bias) v += bf2f(bias[c]);
@@ -669,7 +669,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_tiled_kernel(const bf16_t* __res
             float gv = acc[mt][2 * p][i], uv = acc[mt][2 * p + 1][i];
             if constexpr (F8) { gv *= wscale[ng]; uv *= wscale[nu]; }
             if (bias) { gv += bf2f(bias[ng]); uv += bf2f(bias[nu]); }
-            Y[(int64_t)m * ldy + wn0 / 2 + p * 16 + li] = f2bf(silu(gv) * uv);
+            Y[(int64_t)m * ldy + wn0 / 2 + p * 16 + li] = f2bf(glu_gate(gv, act) * uv);
           }
         }
       } else {
@@ -863,7 +863,7 @@ __global__ __launch_bounds__(512, 1) void gemm_big_kernel(const void* __restrict
             float gv = acc[m][2 * p][i], uv = acc[m][2 * p + 1][i];
             if constexpr (F8) { gv *= sx * ws[ng]; uv *= sx * ws[nu]; }
             if (bias) { gv += bf2f(bias[ng]); uv += bf2f(bias[nu]); }
-            Y[(int64_t)row * ldy + wn0 / 2 + p * 16 + li] = f2bf(silu(gv) * uv);
+            Y[(int64_t)row * ldy + wn0 / 2 + p * 16 + li] = f2bf(glu_gate(gv, act) * uv);
           }
         }
       } else {
@@ -1112,7 +1112,7 @@ __device__ __forceinline__ void tile_epilogue(const f32x4 (&acc)[MTW][NTW], bf16
           if (nu < N) {
             float gv = acc[mt][2 * p][i], uv = acc[mt][2 * p + 1][i];
             if (bias) { gv += bf2f(bias[ng]); uv += bf2f(bias[nu]); }
-            Y[(int64_t)m * ldy + wn0 / 2 + p * 16 + li] = f2bf(silu(gv) * uv);
+            Y[(int64_t)m * ldy + wn0 / 2 + p * 16 + li] = f2bf(glu_gate(gv, act) * uv);
           }
         }
       } else {
@@ -1381,7 +1381,7 @@ __global__ __launch_bounds__(256) void gemm_f8f8_kernel(const unsigned char* __r
           if (nu < N) {
             float gv = acc[mt][2 * p][i] * sx * ws[ng], uv = acc[mt][2 * p + 1][i] * sx * ws[nu];
             if (bias) { gv += bf2f(bias[ng]); uv += bf2f(bias[nu]); }
-            Y[(int64_t)m * ldy + wn0 / 2 + p * 16 + li] = f2bf(silu(gv) * uv);
+            Y[(int64_t)m * ldy + wn0 / 2 + p * 16 + li] = f2bf(glu_gate(gv, act) * uv);
           }
         }
       } else {
@@ -1449,7 +1449,7 @@ int launch_gemm_f8f8(const void* xq, int64_t ldx, const void* xs, const void* wq
   }
   if ((asc || mxq) && !mid) throw std::runtime_error("gemm_f8f8: MX-fp8 activations need a gemm_mid tile (7-15)");
   if (asc && (xs || K % 128)) throw std::runtime_error("gemm_f8f8: MX scales replace xs; K % 128 == 0");
-  if (mxq && (!mxs || !glu || bn % 64 || N % 128 || ldy != N / 2 || partial_out))
+  if (mxq && (!mxs || !glu || act == ACT_GELU_TANH || bn % 64 || N % 128 || ldy != N / 2 || partial_out))
     throw std::runtime_error("gemm_f8f8: MX output needs SwiGLU, BN % 64 == 0, N % 128 == 0, dense rows, no slabs");
   const int tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
   const int nk = (K + TBK8 - 1) / TBK8;

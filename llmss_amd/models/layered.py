@@ -322,6 +322,9 @@ class DenseFeedForward:
             return ops.linear_f(ops.linear_f(h, W.gu, dt, act=spec.act), W.down, dt, closing=model.closing)
         if not spec.gated:
             return ops.linear_f(ops.act_fn(ops.linear_f(h, W.gu, dt), spec.act, W.act_params), W.down, dt, closing=model.closing)
+        if W.interleaved:  # gated in the product's epilogue
+            return ops.linear_f(ops.linear(h, W.gu, None, "gelu_tanh" if spec.act == "gelu_tanh" else "none", True), W.down, dt,
+                                closing=model.closing)
         gu = model.proj = ops.linear_f(h, W.gu, dt)  # (columns past 2 ff: a sandwich block's gate logits)
         return ops.linear_f(ops.glu_act(gu, spec.ff, spec.act), W.down, dt, closing=model.closing)
 
@@ -619,7 +622,7 @@ class LayeredLM:
             for nm in ("shared_gu", "shared_down", "gu", "down"):
                 if getattr(L, "mlp", None) is not None and getattr(L.mlp, nm, None) is not None and \
                         getattr(L.mlp, nm).dim() == 2:
-                    put(nm, getattr(L.mlp, nm), nm == "shared_gu" and L.mlp.shared_interleaved)
+                    put(nm, getattr(L.mlp, nm), nm == "shared_gu" and L.mlp.shared_interleaved or nm == "gu" and L.mlp.interleaved)
         put("head", self.w.head.w)
         return out
 

@@ -789,10 +789,12 @@ class DecayMixWeights:
 class DenseMLPWeights:
     """``gu`` [2 ff, W]: gate rows, then up rows (an ungated feed-forward: [ff, W], the up rows alone); ``down``
     [W, ff]; ``act_params``: the activation's learned numbers in the form the kernel takes (xIELU: softplus(p),
-    1/2 + softplus(q))."""
+    1/2 + softplus(q)). ``interleaved``: the rows of gate and up alternate in groups of 16, for the products whose epilogue
+    applies the gate."""
     gu: torch.Tensor
     down: torch.Tensor
     act_params: tuple = ()
+    interleaved: bool = False
 
     def tensors(self):
         return [self.gu, self.down]
@@ -876,7 +878,7 @@ def _cat_rows(parts, pad_to: int = 8):
 def _babotar_finish(cfg: ModelConfig, get, has, device, dtype) -> ModelWeights:
     """``get(name)`` returns the checkpoint tensor of that name (CPU), ``has(name)`` whether it exists. Shapes are
     checked against the config; the head-mixing matrix and the q / k / v biases are optional tensors."""
-    from ..ops.reference import rope_angle_table
+    from ..ops.reference import glu_interleave, rope_angle_table
 
     shapes = babotar_shapes(cfg)
     optional = (".talk", ".q.b", ".k.b", ".v.b")
@@ -930,7 +932,11 @@ def _babotar_finish(cfg: ModelConfig, get, has, device, dtype) -> ModelWeights:
                 dev(g(pr + "norm")), dev(torch.cat([g(pl + "o"), g(pr + "o")], 1)))
         mlp = None
         if spec.mlp is not None:
-            mlp = DenseMLPWeights(dev(torch.cat([g(p + "mlp.gate"), g(p + "mlp.up")], 0)), dev(g(p + "mlp.down")))
+            parts = (g(p + "mlp.gate"), g(p + "mlp.up"))
+            # (the epilogue form needs bf16 rows of whole 16-byte pieces and whole groups of 16)
+            fused = dtype == torch.bfloat16 and W % 16 == 0 and spec.mlp.ff % 16 == 0 and spec.mlp.act in ("gelu_tanh", "silu")
+            mlp = DenseMLPWeights(dev(glu_interleave(*parts) if fused else torch.cat(parts, 0)), dev(g(p + "mlp.down")),
+                                  interleaved=fused)
         layers.append(SeqBlockWeights(
             dev(g(p + "norm1")), dev(g(p + "norm2")) if mlp is not None else None, hc(1),
             hc(2) if mlp is not None else None, dev(g(p + "canon1")) if cfg.canon_taps else None, mix, mlp))

@@ -312,7 +312,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None, act: str = "none", glu: 
         y = y + bias.float()
     if glu:
         g, u = glu_split(y, -1)
-        y = F.silu(g) * u
+        y = (F.gelu(g, approximate="tanh") if act == "gelu_tanh" else F.silu(g)) * u
     else:
         y = _act(y, act)
     return y.to(x.dtype)
