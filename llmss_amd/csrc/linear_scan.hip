@@ -227,7 +227,7 @@ __device__ __forceinline__ void linear_mend(const LinearArgs& A, int h, int b, i
 // Bound by the chain of chunks: a prompt step of 8 sequences has one (decay) or two (ssd) workgroups per CU, each 16 dependent
 // chunks. 8 x 1024 tokens: ssd, 64 heads 128 x 64, 2160 us token by token, 310 us with fp32 instructions throughout, 182 us here
 // (no workgroup exchanges anything inside a chunk but the scores); decay, 16 heads 128 x 128, 1230 us with its activation pass,
-// 293 us here.
+// 256 us here.
 //
 // Workgroup (head, block of 64 value columns, sequence), 4 waves, the portion's chunks in order. A wave owns 16 value columns:
 // its part of the state lives in registers in the accumulator layout (lane (li, g): column li, rows 16 tile + 4 g + i), and so do
@@ -266,48 +266,70 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
   f32x4 S[KT];
   float* sp = A.S + (((int64_t)slot * H + h) * dim) * (int64_t)vdim;
 #pragma unroll
-  for (int kt = 0; kt < KT; ++kt)
+  for (int kt = 0; kt < KT; ++kt) S[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // (numbers that are not there are read from the nearest place that is and replaced afterwards, here and in the rows below: behind a
+  // condition of its own, or with its zero beside it, every load was waited for before the next)
+  if (cont) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 16 * kt + 4 * g + i;
-      S[kt][i] = (cont && r < dim && col < vdim) ? sp[(int64_t)r * vdim + col] : 0.f;
-    }
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[kt][i] = sp[(int64_t)min(16 * kt + 4 * g + i, dim - 1) * vdim + colc];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[kt][i] = 16 * kt + 4 * g + i < dim && col < vdim ? S[kt][i] : 0.f;
+  }
   constexpr int CHK = DKP / 8, NK = C * CHK / 256;
   static_assert((C * CHK) % 256 == 0, "whole 16-byte pieces per thread");
   u16x8 rq[NK], rk[NK];
-  bf16_t rv[16];
-  float rd = 0.f;
+  bf16_t rv[16], rd = 0;
   const u16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-  auto fetch = [&](int j0) {
+  auto fetch = [&](int j0) {  // the portion's last row again and again past its end, a row's first piece past its last
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
       const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 8;
-      const bool in = j0 + r < qlen && d < dim;
-      const int64_t tt = t0 + j0 + r;
-      rq[j] = in ? *reinterpret_cast<const u16x8*>((const bf16_t*)A.q + tt * A.ldq + (int64_t)gq * dim + d) : zero8;
-      rk[j] = in ? *reinterpret_cast<const u16x8*>((const bf16_t*)A.k + tt * A.ldk + (int64_t)gq * dim + d) : zero8;
+      const int64_t tt = t0 + min(j0 + r, qlen - 1), at = (int64_t)gq * dim + (d < dim ? d : 0);
+      rq[j] = *reinterpret_cast<const u16x8*>((const bf16_t*)A.q + tt * A.ldq + at);
+      rk[j] = *reinterpret_cast<const u16x8*>((const bf16_t*)A.k + tt * A.ldk + at);
     }
 #pragma unroll
     for (int j = 0; j < 16; ++j) {  // token 16 (j / 4) + 4 g + j % 4 at this lane's column
       const int r = j0 + 16 * (j >> 2) + 4 * g + (j & 3);
       rv[j] = ((const bf16_t*)A.v)[(int64_t)(t0 + min(r, qlen - 1)) * A.ldv + (int64_t)h * vdim + colc];
-      if (r >= qlen) rv[j] = 0;
     }
-    if (MODE == 2 && w == 0) rd = bf2f(((const bf16_t*)A.dt)[(int64_t)(t0 + min(j0 + lane, qlen - 1)) * A.lddt + h]);
+    if (MODE == 2) rd = ((const bf16_t*)A.dt)[(int64_t)(t0 + min(j0 + lane, qlen - 1)) * A.lddt + h];
   };
-  auto stage = [&](LT* dst, const u16x8& x) {
-    if constexpr (MODE == 2) {
-      *reinterpret_cast<u16x8*>(dst) = x;
-    } else {
-      f32x4 lo, hi;
+  // rows into LDS and V into registers; the choice of the activation is made once for all of them (at each number it cost more than the
+  // number, one after the other: decay, 16 heads 128 x 128 of 8 x 1024 tokens, with the places and factors read ahead 369 -> 256 us)
+  auto stage_as = [&](int j0, f32x4 (&v)[4], auto silu_c) {
+    constexpr bool SILU = decltype(silu_c)::value;
+    auto stage = [&](LT* dst, const u16x8& x) {
+      if constexpr (MODE == 2) {
+        *reinterpret_cast<u16x8*>(dst) = x;
+      } else {
+        f32x4 lo, hi;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float u = bf2f(x[i]), v = bf2f(x[4 + i]);
-        lo[i] = A.silu ? lin_silu<bf16_t>(u) : u;
-        hi[i] = A.silu ? lin_silu<bf16_t>(v) : v;
+        for (int i = 0; i < 4; ++i) {
+          const float u = bf2f(x[i]), z = bf2f(x[4 + i]);
+          lo[i] = SILU ? lin_silu<bf16_t>(u) : u;
+          hi[i] = SILU ? lin_silu<bf16_t>(z) : z;
+        }
+        *reinterpret_cast<f32x4*>(dst) = lo;
+        *reinterpret_cast<f32x4*>(dst + 4) = hi;
       }
-      *reinterpret_cast<f32x4*>(dst) = lo;
-      *reinterpret_cast<f32x4*>(dst + 4) = hi;
+    };
+#pragma unroll
+    for (int j = 0; j < NK; ++j) {
+      const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 8;
+      const bool in = j0 + r < qlen && d < dim;
+      stage(&Qs[r * LDK + d], in ? rq[j] : zero8);
+      stage(&Ks[r * LDK + d], in ? rk[j] : zero8);
+    }
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const float x = j0 + 16 * (j >> 2) + 4 * g + (j & 3) < qlen ? bf2f(rv[j]) : 0.f;
+      v[j >> 2][j & 3] = MODE == 0 && SILU ? lin_silu<bf16_t>(x) : x;
     }
   };
   const float dskip = MODE == 2 && A.skip ? A.skip[h] : 0.f;
@@ -320,24 +342,15 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
   for (int j0 = 0; j0 < qlen; j0 += C) {
     const int nt = min(C, qlen - j0);
     __syncthreads();  // the previous chunk's readers are done
-#pragma unroll
-    for (int j = 0; j < NK; ++j) {
-      const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 8;
-      stage(&Qs[r * LDK + d], rq[j]);
-      stage(&Ks[r * LDK + d], rk[j]);
-    }
     f32x4 v[4];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const float x = bf2f(rv[j]);
-      v[j >> 2][j & 3] = MODE == 0 && A.silu ? lin_silu<bf16_t>(x) : x;
-    }
+    if (MODE != 2 && A.silu) stage_as(j0, v, std::true_type{});
+    else stage_as(j0, v, std::false_type{});
     if (w == 0) {
       const bool in = lane < nt;
       double F;
       float e = in ? 1.0f : 0.f;
       if (MODE == 2) {
-        e = in ? lin_softplus(rd + dtb) : 0.f;
+        e = in ? lin_softplus(bf2f(rd) + dtb) : 0.f;
         F = in ? at_least((double)(-ea * e), -1e8) : 0.0;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -400,6 +413,9 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
           p[ct] = NCH == 4 ? (c[0] + c[1]) + (c[NCH - 2] + c[NCH - 1]) : c[0] + c[1];
         }
       }
+      double Ft[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) Ft[i] = Fs[16 * w + 4 * g + i];
 #pragma unroll
       for (int ct = 0; ct < 4; ++ct) {
         if (ct > w) continue;
@@ -409,9 +425,8 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int t = 16 * w + 4 * g + i;
-          float f = expf((float)(Fs[t] - Fv)) * ev;
-          if (alt && ((t - s) & 1)) f = -f;
-          Ps[t * LDP + s] = s <= t ? p[ct][i] * f : 0.f;
+          const float f = expf((float)(Ft[i] - Fv)) * ev, z = p[ct][i] * (alt && ((t - s) & 1) ? -f : f);
+          Ps[t * LDP + s] = s <= t ? z : 0.f;
         }
       }
     }
