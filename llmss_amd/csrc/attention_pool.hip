@@ -45,24 +45,79 @@ __global__ __launch_bounds__(256) void rope_pairs_cache_kernel(const T* __restri
     for (int i = threadIdx.x; i < nv; i += blockDim.x) vc[slot * nv + i] = row[off_v + i];
 }
 
+__device__ __forceinline__ int64_t pool_row(const int* btr, int blk, int pool, int bs, int per) {
+  const int p = blk * pool;
+  return (int64_t)btr[p / bs] * per + (p % bs) / pool;
+}
+
+// pooled caches beside the pages (pool 0: none), the block tables and the sequences' lengths: of steps of single rows
+template <typename T>
+struct PoolArgs {
+  T *kp, *vp;
+  const int* __restrict__ bt;
+  int maxb;
+  const int* __restrict__ ctx;
+  int bs, pool, per;
+};
+
 // The same four numbers (two pairs) an access; in steps of few rows a row is spread over gridDim.y workgroups, so that a thread has one
 // access to wait for. 8192 rows of 2048 + 2 x 1024, bf16: 55 -> 28 us, 33 rows 10 -> 5 us.
-template <typename T>
+// POOL: row t is the last position of sequence t, and a row that completes a block of `pool` positions forms the block's means too (as
+// pool_update does: the cached rows in order, in fp32, the row itself as it is cached): columns are apart, so a thread needs nothing but its
+// own. A launch of its own for them takes 10.7 us a layer and step, few of whose rows complete a block; here, 33 rows of 4096 + 2 x 1024, 6.1 us with and
+// 4.7 without them (11.0 with the pages read behind each other).
+template <typename T, bool POOL>
 __global__ __launch_bounds__(256) void rope_pairs_vec_kernel(const T* __restrict__ proj, int64_t ldp, int off_q,
                                                              int off_k, int off_v, const float* __restrict__ cs,
-                                                             int rdims, float* __restrict__ qout,
-                                                             T* __restrict__ kc, T* __restrict__ vc,
-                                                             const int64_t* __restrict__ slots, int H, int G,
-                                                             int dim, int vdim) {
+                                                             int rdims, float* __restrict__ qout, T* kc, T* vc,
+                                                             const int64_t* __restrict__ slots, int H, int G, int dim,
+                                                             int vdim, PoolArgs<T> pl) {
   const int t = blockIdx.x;
   const T* row = proj + (int64_t)t * ldp;
   const float* ang = cs ? cs + (int64_t)t * rdims : nullptr;
   const int64_t slot = slots[t];
   const int nq = H * dim, nk = G * dim, nv = G * vdim;
+  int64_t at = -1;  // the pooled row that this row completes
+  int first = 0;    // its first position
+  if constexpr (POOL) {
+    const int L = pl.ctx[t];
+    if (slot >= 0 && L > 0 && L % pl.pool == 0) {
+      first = L - pl.pool;
+      at = pool_row(pl.bt + (int64_t)t * pl.maxb, first / pl.pool, pl.pool, pl.bs, pl.per);
+    }
+  }
+  // columns i .. i + 3 of the block's mean: the rows before this one from `base` [n a row], v this one's
+  auto mean = [&](T* to, const T* base, int n, int i, f32x4 v) {
+    constexpr int U = 16;
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+    for (int j0 = 0; j0 < pl.pool - 1; j0 += U) {
+      int pg[U], off[U];  // all pages asked for, then all rows, then the sums
+      f32x4 x[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = first + min(j0 + u, pl.pool - 2);
+        off[u] = j % pl.bs;
+        pg[u] = pl.bt[(int64_t)t * pl.maxb + j / pl.bs];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = ld4(base + ((int64_t)pg[u] * pl.bs + off[u]) * n + i);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (j0 + u < pl.pool - 1) a += x[u];
+    }
+    T own[4] __attribute__((aligned(16)));
+    st4(own, v);
+    a += ld4(own);
+    st4(to + at * n + i, a * (1.0f / (float)pl.pool));
+  };
   for (int e = (blockIdx.y * 256 + threadIdx.x) * 4; e < nq + nk + nv; e += gridDim.y * 1024) {
     if (e >= nq + nk) {
       const int i = e - nq - nk;
-      if (slot >= 0) st4(vc + slot * nv + i, ld4(row + off_v + i));
+      const f32x4 v = ld4(row + off_v + i);
+      if (slot >= 0) st4(vc + slot * nv + i, v);
+      if (POOL && at >= 0) mean(pl.vp, vc, nv, i, v);
       continue;
     }
     const bool isq = e < nq;
@@ -74,35 +129,45 @@ __global__ __launch_bounds__(256) void rope_pairs_vec_kernel(const T* __restrict
       v = f32x4{fmaf(v[0], a[0], -v[1] * a[1]), fmaf(v[1], a[0], v[0] * a[1]), fmaf(v[2], a[2], -v[3] * a[3]),
                 fmaf(v[3], a[2], v[2] * a[3])};
     }
-    if (isq) *reinterpret_cast<f32x4*>(qout + (int64_t)t * nq + i) = v;
-    else if (slot >= 0) st4(kc + slot * nk + i, v);
+    if (isq) {
+      *reinterpret_cast<f32x4*>(qout + (int64_t)t * nq + i) = v;
+    } else {
+      if (slot >= 0) st4(kc + slot * nk + i, v);
+      if (POOL && at >= 0) mean(pl.kp, kc, nk, i, v);
+    }
   }
 }
 
-void launch_rope_pairs_cache(const void* proj, int64_t ldp, int off_q, int off_k, int off_v, const void* cs, int rdims,
+// pool > 0: rows are single ones (row t belongs to sequence t) that complete the pooled caches' blocks too. -> whether they did (else
+// pool_update is the caller's)
+bool launch_rope_pairs_cache(const void* proj, int64_t ldp, int off_q, int off_k, int off_v, const void* cs, int rdims,
                              void* qout, void* kc, void* vc, const void* slots, int T_, int H, int G, int dim, int vdim,
-                             int dt, hipStream_t st) {
-  if (T_ == 0) return;
+                             int dt, void* kp, void* vp, const void* bt, int maxb, const void* ctx, int bs, int pool, int per,
+                             hipStream_t st) {
+  if (T_ == 0) return true;
   if (rdims < 0 || rdims % 2 || rdims > dim) throw std::runtime_error("rope_pairs_cache: bad rotated dimensions");
+  if (pool > 0 && (bs < 1 || per < (bs + pool - 1) / pool)) throw std::runtime_error("rope_pairs_cache: bad pool");
   const int a4 = dt == 0 ? 7 : 15;  // four numbers of the storage type
   if (dim % 4 == 0 && vdim % 4 == 0 && rdims % 4 == 0 && ldp % 4 == 0 && !((off_q | off_k | off_v) & 3) &&
       !(((uintptr_t)proj | (uintptr_t)kc | (uintptr_t)vc) & a4) && !(((uintptr_t)qout | (uintptr_t)cs) & 15)) {
+    const bool pooled = pool > 0 && !(((uintptr_t)kp | (uintptr_t)vp) & a4);
     const dim3 g(T_, T_ <= 256 ? (H * dim + G * (dim + vdim) + 1023) / 1024 : 1);
-    DISPATCH_T(dt, T, (rope_pairs_vec_kernel<T><<<g, 256, 0, st>>>(
-        (const T*)proj, ldp, off_q, off_k, off_v, rdims ? (const float*)cs : nullptr, rdims, (float*)qout, (T*)kc, (T*)vc,
-        (const int64_t*)slots, H, G, dim, vdim)));
+#define LAUNCH_RP(POOL_)                                                                                                  \
+  DISPATCH_T(dt, T, (rope_pairs_vec_kernel<T, POOL_><<<g, 256, 0, st>>>(                                                  \
+      (const T*)proj, ldp, off_q, off_k, off_v, rdims ? (const float*)cs : nullptr, rdims, (float*)qout, (T*)kc, (T*)vc,  \
+      (const int64_t*)slots, H, G, dim, vdim,                                                                             \
+      PoolArgs<T>{(T*)kp, (T*)vp, (const int*)bt, maxb, (const int*)ctx, bs, pool, per})))
+    if (pooled) LAUNCH_RP(true);
+    else LAUNCH_RP(false);
+#undef LAUNCH_RP
     HIP_CHECK_LAUNCH();
-    return;
+    return pooled;
   }
   DISPATCH_T(dt, T, (rope_pairs_cache_kernel<T><<<T_, 256, 0, st>>>(
       (const T*)proj, ldp, off_q, off_k, off_v, rdims ? (const float*)cs : nullptr, rdims, (float*)qout, (T*)kc, (T*)vc,
       (const int64_t*)slots, H, G, dim, vdim)));
   HIP_CHECK_LAUNCH();
-}
-
-__device__ __forceinline__ int64_t pool_row(const int* btr, int blk, int pool, int bs, int per) {
-  const int p = blk * pool;
-  return (int64_t)btr[p / bs] * per + (p % bs) / pool;
+  return false;
 }
 
 // grid (B, blocks a portion can complete): workgroup (b, n) takes block p0 / pool + n of sequence b

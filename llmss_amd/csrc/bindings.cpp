@@ -204,9 +204,10 @@ void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const void* e
 void launch_token_side_add(void* x, const void* ids, const void* table, int64_t ldt, int vocab, int col0, int d,
                            const void* wg, const void* wp, const void* wn, const void* add, const void* wnext, void* h,
                            int64_t ldh, float eps, int T_, int W, int dt, hipStream_t st);
-void launch_rope_pairs_cache(const void* proj, int64_t ldp, int off_q, int off_k, int off_v, const void* cs, int rdims,
+bool launch_rope_pairs_cache(const void* proj, int64_t ldp, int off_q, int off_k, int off_v, const void* cs, int rdims,
                              void* qout, void* kc, void* vc, const void* slots, int T_, int H, int G, int dim, int vdim,
-                             int dt, hipStream_t st);
+                             int dt, void* kp, void* vp, const void* bt, int maxb, const void* ctx, int bs, int pool, int per,
+                             hipStream_t st);
 void launch_pool_update(const void* kc, const void* vc, void* kp, void* vp, const void* bt, int maxb, const void* cu,
                         const void* ctx, int B, int max_qlen, int nk, int nv, int bs, int pool, int per, int dt,
                         hipStream_t st);
@@ -697,9 +698,10 @@ PYBIND11_MODULE(_C, m) {
   });
   m.def("rope_pairs_cache", [](uintptr_t proj, int64_t ldp, int off_q, int off_k, int off_v, uintptr_t cs, int rdims,
                                uintptr_t qout, uintptr_t kc, uintptr_t vc, uintptr_t slots, int T, int H, int G,
-                               int dim, int vdim, int dt, uintptr_t st) {
-    launch_rope_pairs_cache(CP(proj), ldp, off_q, off_k, off_v, CP(cs), rdims, P(qout), P(kc), P(vc), CP(slots), T, H,
-                            G, dim, vdim, dt, S(st));
+                               int dim, int vdim, int dt, uintptr_t kp, uintptr_t vp, uintptr_t bt, int maxb,
+                               uintptr_t ctx, int bs, int pool, int per, uintptr_t st) {
+    return launch_rope_pairs_cache(CP(proj), ldp, off_q, off_k, off_v, CP(cs), rdims, P(qout), P(kc), P(vc), CP(slots), T, H,
+                                   G, dim, vdim, dt, P(kp), P(vp), CP(bt), maxb, CP(ctx), bs, pool, per, S(st));
   });
   m.def("pool_update", [](uintptr_t kc, uintptr_t vc, uintptr_t kp, uintptr_t vp, uintptr_t bt, int maxb, uintptr_t cu,
                           uintptr_t ctx, int B, int max_qlen, int nk, int nv, int bs, int pool, int per, int dt,

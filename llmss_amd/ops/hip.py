@@ -1857,7 +1857,7 @@ def token_side_add(x, ids, table, col0, gate_w, proj_w, norm_w, eps, add, wnext,
     return h
 
 
-def rope_pairs_cache(proj, off_q, off_k, off_v, cs, k_cache, v_cache, slots, heads, kv_heads, dim, vdim):
+def rope_pairs_cache(proj, off_q, off_k, off_v, cs, k_cache, v_cache, slots, heads, kv_heads, dim, vdim, pooled=None):
     T = proj.shape[0]
     _rows(proj, "proj")
     nq, nk, nv = heads * dim, kv_heads * dim, kv_heads * vdim
@@ -1874,9 +1874,19 @@ def rope_pairs_cache(proj, off_q, off_k, off_v, cs, k_cache, v_cache, slots, hea
                "angles [T, rotated dims / 2, 2], rotated dims <= dim")
         rdims = 2 * cs.shape[1]
     q = torch.empty(T, nq, dtype=torch.float32, device=proj.device)
-    lib().rope_pairs_cache(proj.data_ptr(), proj.stride(0), int(off_q), int(off_k), int(off_v), _ptr(cs), rdims,
-                           q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), slots.data_ptr(), T, heads, kv_heads,
-                           dim, vdim, _dt(proj, "proj"), _stream())
+    args = (0, 0, 0, 0, 0, 0, 0, 0)
+    if pooled is not None:
+        kp, vp, tables, cu, ctx, pool = pooled
+        per = _pool_caches(k_cache, v_cache, kp, vp, pool)
+        _i32(ctx, "ctx_lens", T)
+        _i32(tables, "block_tables")
+        _check(tables.dim() == 2 and tables.shape[0] >= T and pool >= 1 and cu.numel() == T + 1, "one row per sequence, block tables, pool")
+        args = (kp.data_ptr(), vp.data_ptr(), tables.data_ptr(), tables.shape[1], ctx.data_ptr(), k_cache.shape[1], int(pool), per)
+    done = lib().rope_pairs_cache(proj.data_ptr(), proj.stride(0), int(off_q), int(off_k), int(off_v), _ptr(cs), rdims,
+                                  q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), slots.data_ptr(), T, heads, kv_heads,
+                                  dim, vdim, _dt(proj, "proj"), *args, _stream())
+    if pooled is not None and not done:
+        pool_update(k_cache, v_cache, kp, vp, tables, cu, ctx, pool, max_qlen=1)
     return q
 
 

@@ -1062,11 +1062,12 @@ def token_side_add(x, ids, table, col0: int, gate_w, proj_w, norm_w, eps: float,
 
 
 def rope_pairs_cache(proj, off_q: int, off_k: int, off_v: int, cs, k_cache, v_cache, slots, heads: int,
-                     kv_heads: int, dim: int, vdim: int):
+                     kv_heads: int, dim: int, vdim: int, pooled=None):
     """From the projection rows: q and k with the neighbouring pairs (2i, 2i + 1), i < cs.shape[1], of every head
     turned by ``cs`` [T, dims / 2, 2] = (cos, sin) (None: no rotation), v as it is. Returns q fp32 [T, heads * dim];
     k / v go into the paged caches [blocks, block_size, kv_heads * dim | kv_heads * vdim] at ``slots`` (< 0: not
-    cached)."""
+    cached). ``pooled`` (kp_cache, vp_cache, block_tables, cu, ctx_lens, pool), for steps of single rows (row t is sequence t's last
+    position): :func:`pool_update` as well."""
     T = proj.shape[0]
     nq, nk, nv = heads * dim, kv_heads * dim, kv_heads * vdim
     q = proj[:, off_q:off_q + nq].float().reshape(T, heads, dim)
@@ -1076,6 +1077,8 @@ def rope_pairs_cache(proj, off_q: int, off_k: int, off_v: int, cs, k_cache, v_ca
     keep = slots >= 0
     k_cache.view(-1, nk)[slots[keep]] = k.reshape(T, nk)[keep].to(k_cache.dtype)
     v_cache.view(-1, nv)[slots[keep]] = proj[:, off_v:off_v + nv][keep].to(v_cache.dtype)
+    if pooled is not None:
+        pool_update(k_cache, v_cache, *pooled)
     return q.reshape(T, nq).contiguous()
 
 
