@@ -75,7 +75,8 @@ __global__ __launch_bounds__(256) void rope_bias_cache_kernel(const T* __restric
 }
 
 // The same four numbers an access, a dimension's partner by a load of its own; in steps of few rows a row is spread over gridDim.y
-// workgroups, so that a thread has one access to wait for. 8192 rows of 2048 + 2 x 512, bf16: 75 -> 49 us, 64 rows 11.6 -> 5.4 us.
+// workgroups, so that a thread has one access to wait for. 8192 rows of 2048 + 2 x 512, bf16: 75 -> 49 us, 64 rows 11.6 -> 5.4 us; with a
+// number, its partner, their biases and angles asked for together 49 -> 43 and 5.4 -> 4.8 (prompt rows spread likewise: 44).
 template <typename T>
 __global__ __launch_bounds__(256) void rope_bias_vec_kernel(const T* __restrict__ proj, int64_t ldp, int off_q,
                                                             int off_k, int off_v, const T* __restrict__ bias,
@@ -92,32 +93,39 @@ __global__ __launch_bounds__(256) void rope_bias_vec_kernel(const T* __restrict_
   const T* row = proj + (int64_t)t * ldp;
   const int64_t slot = slots[t];
   const int nq = H * dim, nk = G * dim, nv = G * vdim;
+  typedef T raw4 __attribute__((ext_vector_type(4)));
+  const auto num = [](const raw4& r) {
+    const T x[4] __attribute__((aligned(16))) = {r[0], r[1], r[2], r[3]};
+    return ld4(x);
+  };
   for (int e = (blockIdx.y * 256 + threadIdx.x) * 4; e < nq + nk + nv; e += gridDim.y * 1024) {
-    if (e >= nq + nk) {
-      const int i = e - nq - nk;
-      f32x4 v = ld4(row + off_v + i);
-      if (bias) v += ld4(bias + e);
-      if (slot >= 0) st4(vc + slot * (int64_t)nv + i, v);
-      continue;
-    }
-    const bool isk = e >= nq;
-    const int idx = isk ? e - nq : e;
+    const bool isv = e >= nq + nk, isk = !isv && e >= nq;
+    const int idx = isv ? e - nq - nk : isk ? e - nq : e;
     const int d = idx % dim;
-    const T* src = row + (isk ? off_k : off_q) + idx;
-    f32x4 v = ld4(src);
-    if (bias) v += ld4(bias + e);
-    if (d < rot) {
-      const bool low = d < half;
-      const int i = low ? d : d - half, o = low ? half : -half;
-      f32x4 u = ld4(src + o);
-      if (bias) u += ld4(bias + e + o);
-      const f32x4 a = *reinterpret_cast<const f32x4*>(tab + 2 * i), b = *reinterpret_cast<const f32x4*>(tab + 2 * i + 4);
+    const bool turn = !isv && d < rot, low = d < half;
+    const int o = turn ? (low ? half : -half) : 0, i = turn ? (low ? d : d - half) : 0;
+    // everything is asked for before the first number is touched (what is not turned reads itself and the first angles)
+    const T* src = row + (isv ? off_v : isk ? off_k : off_q) + idx;
+    const raw4 rv = *reinterpret_cast<const raw4*>(src), ru = *reinterpret_cast<const raw4*>(src + o);
+    raw4 bv, bu;
+    f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
+    if (bias) bv = *reinterpret_cast<const raw4*>(bias + e), bu = *reinterpret_cast<const raw4*>(bias + e + o);
+    if (rot) a = *reinterpret_cast<const f32x4*>(tab + 2 * i), b = *reinterpret_cast<const f32x4*>(tab + 2 * i + 4);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 v = num(rv), u = num(ru);
+    if (bias) v += num(bv), u += num(bu);
+    if (turn) {
       const f32x4 c = {a[0], a[2], b[0], b[2]}, s = {a[1], a[3], b[1], b[3]};
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[q] = low ? v[q] * c[q] - u[q] * s[q] : v[q] * c[q] + u[q] * s[q];
     }
-    if (!isk) *reinterpret_cast<f32x4*>(qout + (int64_t)t * nq + idx) = v;
-    else if (slot >= 0) st4(kc + slot * (int64_t)nk + idx, v);
+    if (isv) {
+      if (slot >= 0) st4(vc + slot * (int64_t)nv + idx, v);
+    } else if (isk) {
+      if (slot >= 0) st4(kc + slot * (int64_t)nk + idx, v);
+    } else {
+      *reinterpret_cast<f32x4*>(qout + (int64_t)t * nq + idx) = v;
+    }
   }
 }
 
