@@ -208,18 +208,34 @@ class DecoderLM:
                  torch.zeros(shp, dtype=dt, device=self.device)) for _ in range(self.cfg.num_layers)]
 
     # ---------------------------------------------------------------------------- forward
+    def _qkv_plan(self, M: int, N: int, K: int):
+        """(nt_hint, split_hint) of the QKV product with RoPE and the cache write in its epilogue, None: two launches. Without a tuned
+        plan of either form: where the static plan of a finished product is the decode kernel's, unsplit. The two launches may
+        split K, whose slabs rope_cache sums on the way, but are the slower ones at every size measured (us, two and one):
+        4800 x 1600, one row 8.9 and 6.3, 64 rows 13.4 and 9.7; 12288 x 4096 23.6 and 19.9, 28.7 and 24.1; 6144 x 4096 14.6 and
+        11.7, 18.3 and 17.7; 3072 x 1024 6.8 and 4.8, 10.4 and 6.7."""
+        lib = _hip_ops().lib()
+        if lib.gemm_tuned_get(M, N, K, False, 3) is not None:
+            return 0, 0
+        if M > 64 or self.cfg.head_dim % 8 or lib.gemm_tuned_get(M, N, K, False, 0) is not None:
+            return None
+        nt, split = lib.gemm_plan(M, N, K, False, False, False)
+        return (nt, split) if nt >> 8 & 1024 and split == 1 else None  # (the hint bit of csrc/gemm_dec.hip)
+
     def _qkv_rope_cache(self, L, y, inp: StepInput, kc, vc):
         """QKV projection, RoPE and the paged KV write of the step's tokens -> the bf16 qkv rows.
 
-        Where the autotuner found it faster (a kind-3 plan for this M, ops/autotune.py tune_qkv_epilogue)
-        this is ONE GEMM launch whose epilogue rotates q / k and stores k / v to the cache; otherwise the
-        GEMM (split-K slabs allowed) followed by the rope_cache kernel, which sums the slabs itself."""
+        Where the autotuner found it faster (a kind-3 plan for this M, ops/autotune.py tune_qkv_epilogue), or nothing is tuned and the
+        decode kernel's unsplit plan serves (:meth:`_qkv_plan`), this is ONE GEMM launch whose epilogue rotates q / k
+        and stores k / v to the cache; otherwise the GEMM (split-K slabs allowed) followed by the rope_cache kernel, which sums
+        the slabs itself."""
         cfg, p = self.cfg, self.plan
         do_rope = cfg.position == "rope"
-        if y.is_cuda and self.qkv_epi and not self.kv_fp8 and L.qkv.w.dim() == 2 and L.qkv.w_scale is None \
-                and _hip_ops().lib().gemm_tuned_get(y.shape[0], L.qkv.N, L.qkv.K, False, 3) is not None:
-            out = _hip_ops().linear_qkv(y, L.qkv.w, L.qkv.b, inp.positions, self.w.cos, self.w.sin, kc, vc, inp.slots,
-                                        p.nh_l, p.nkv_l, cfg.head_dim, cfg.rotary_dim, cfg.rope_style, do_rope)
+        if y.is_cuda and self.qkv_epi and not self.kv_fp8 and L.qkv.w.dim() == 2 and L.qkv.w_scale is None:
+            plan = self._qkv_plan(y.shape[0], L.qkv.N, L.qkv.K)
+            out = None if plan is None else _hip_ops().linear_qkv(
+                y, L.qkv.w, L.qkv.b, inp.positions, self.w.cos, self.w.sin, kc, vc, inp.slots, p.nh_l, p.nkv_l, cfg.head_dim,
+                cfg.rotary_dim, cfg.rope_style, do_rope, *plan)
             if out is not None:
                 return out
         qkv = L.qkv(y, partial_ok=True)
