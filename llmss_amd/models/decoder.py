@@ -211,9 +211,10 @@ class DecoderLM:
     def _qkv_plan(self, M: int, N: int, K: int):
         """(nt_hint, split_hint) of the QKV product with RoPE and the cache write in its epilogue, None: two launches. Without a tuned
         plan of either form: where the static plan of a finished product is the decode kernel's, unsplit. The two launches may
-        split K, whose slabs rope_cache sums on the way, but are the slower ones at every size measured (us, two and one):
-        4800 x 1600, one row 8.9 and 6.3, 64 rows 13.4 and 9.7; 12288 x 4096 23.6 and 19.9, 28.7 and 24.1; 6144 x 4096 14.6 and
-        11.7, 18.3 and 17.7; 3072 x 1024 6.8 and 4.8, 10.4 and 6.7."""
+        split K, whose slabs rope_cache sums on the way, but are not the faster ones (us, two and one): 4800 x 1600, one row 8.9
+        and 6.3, 64 rows 13.4 and 9.7; 12288 x 4096 23.6 and 19.9, 28.7 and 24.1; 6144 x 4096 14.6 and 11.7, 18.3 and 17.7; 3072 x
+        1024 6.8 and 4.8, 10.4 and 6.7; 15360 x 5120 31.2 and 27.5, 42.0 and 35.2; 10240 x 8192 32.2 and 32.6, 16 rows 34.3 and
+        32.6."""
         lib = _hip_ops().lib()
         if lib.gemm_tuned_get(M, N, K, False, 3) is not None:
             return 0, 0
