@@ -234,8 +234,6 @@ class DecoderLM:
         do_rope = cfg.position == "rope"
         if y.is_cuda and self.qkv_epi and not self.kv_fp8 and L.qkv.w.dim() == 2 and L.qkv.w_scale is None:
             plan = self._qkv_plan(y.shape[0], L.qkv.N, L.qkv.K)
-            if plan is not None and plan[0] and ((y.data_ptr() | L.qkv.w.data_ptr()) & 15 or y.stride(0) % 8):
-                plan = None  # (as for every static plan: rows in pieces of 16 bytes)
             out = None if plan is None else _hip_ops().linear_qkv(
                 y, L.qkv.w, L.qkv.b, inp.positions, self.w.cos, self.w.sin, kc, vc, inp.slots, p.nh_l, p.nkv_l, cfg.head_dim,
                 cfg.rotary_dim, cfg.rope_style, do_rope, *plan)
