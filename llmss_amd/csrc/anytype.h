@@ -34,17 +34,18 @@ __device__ __forceinline__ void st4(T* p, f32x4 v) {
   else *reinterpret_cast<u16x4*>(p) = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
 }
 
-// Four columns of a product whose K was split: the sum of `slabs` fp32 slabs `stride` apart, eight loads in flight, added in their order
-__device__ __forceinline__ f32x4 slab_sum(const float* p, int slabs, int64_t stride) {
-  f32x4 a = {0.f, 0.f, 0.f, 0.f};
+// Four columns (V f32x4) or one (float) of a product whose K was split: the sum of `slabs` fp32 slabs `stride` apart, eight loads in flight,
+// added in their order
+template <typename V>
+__device__ __forceinline__ V slab_sum(const float* p, int slabs, int64_t stride) {
+  const V zero = {};
+  V a = zero;
   for (int s0 = 0; s0 < slabs; s0 += 8) {
-    f32x4 v[8];
+    V v[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const f32x4*>(p + min(s0 + j, slabs - 1) * stride);
+    for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const V*>(p + min(s0 + j, slabs - 1) * stride);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] += s0 + j < slabs ? v[j][i] : 0.f;
+    for (int j = 0; j < 8; ++j) a += s0 + j < slabs ? v[j] : zero;
   }
   return a;
 }

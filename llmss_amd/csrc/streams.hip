@@ -51,13 +51,14 @@ void launch_embed_streams(const void* ids, const void* positions, const void* ta
 // If w: u = sum_s inw[s] x_s (inw null: the plain sum), h[t] = norm(u) * w, with
 // rms = 0: (u - mean) / sqrt(var + eps), var the mean squared deviation; rms = 1: u / sqrt(mean(u^2) + eps).
 // TH: storage type of h (the model's, or float when a convolution follows).
+// slabs > 0: y is the fp32 slabs [slabs][T][W] of a product whose K was split, summed here instead of in a launch of their own.
 template <typename T, typename TH>
 __global__ __launch_bounds__(256) void stream_add_norm_kernel(float* __restrict__ x, const T* __restrict__ y,
                                                               int64_t ldy, const float* __restrict__ mix,
                                                               const float* __restrict__ outw, float c,
                                                               const float* __restrict__ inw, const T* __restrict__ w,
                                                               float eps, int rms, TH* __restrict__ h, int64_t ldh,
-                                                              int S, int T_, int W) {
+                                                              int S, int T_, int W, int slabs) {
   extern __shared__ float u_s[];  // W floats, then 32 for the reductions
   float* red = u_s + W;
   const int t = blockIdx.x;
@@ -68,7 +69,8 @@ __global__ __launch_bounds__(256) void stream_add_norm_kernel(float* __restrict_
     for (int s = 0; s < MAX_STREAMS; ++s)
       if (s < S) xs[s] = x[((int64_t)s * T_ + t) * W + col];
     if (y) {
-      const float yv = El<T>::ld(y + (int64_t)t * ldy + col) * c;
+      const float yv = c * (slabs ? slab_sum<float>((const float*)y + (int64_t)t * W + col, slabs, (int64_t)T_ * W)
+                                  : El<T>::ld(y + (int64_t)t * ldy + col));
       float nx[MAX_STREAMS];
 #pragma unroll
       for (int s = 0; s < MAX_STREAMS; ++s) {
@@ -111,7 +113,6 @@ __global__ __launch_bounds__(256) void stream_add_norm_kernel(float* __restrict_
 // The same for up to four streams of rows of up to 4096: a thread keeps NC times four columns of every stream in registers, all
 // loads are issued before the first is used, and nothing passes through LDS but the two sums. The kernel above, with a load of four
 // bytes waited for at a time, is bound by latency: 8192 rows of 2048, two streams, bf16: 136 -> 59 us (5.7 TB/s).
-// slabs > 0: y is the fp32 slabs [slabs][T][W] of a product whose K was split, summed here instead of in a launch of their own.
 template <typename T, typename TH, int S, int NC>
 __global__ __launch_bounds__(256) void stream_rows_kernel(float* __restrict__ x, const T* __restrict__ y, int64_t ldy,
                                                           const float* __restrict__ mix, const float* __restrict__ outw, float c,
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(256) void stream_rows_kernel(float* __restrict__ x,
     if (col < W) {
 #pragma unroll
       for (int s = 0; s < S; ++s) xs[s][i] = ld4(x + ((int64_t)s * T_ + t) * W + col);
-      if (slabs) yv[i] = slab_sum((const float*)y + (int64_t)t * W + col, slabs, (int64_t)T_ * W);
+      if (slabs) yv[i] = slab_sum<f32x4>((const float*)y + (int64_t)t * W + col, slabs, (int64_t)T_ * W);
       else if (y) yv[i] = ld4(y + (int64_t)t * ldy + col);
       if (w) wv[i] = ld4(w + col);
     }
@@ -208,8 +209,9 @@ void launch_stream_add_norm(void* x, const void* y, int64_t ldy, const void* mix
   // (rows in steps of four numbers; x lies in rows of W, so W decides for it)
   const int es = dt == 0 ? 2 : 4, eh = h_f32 ? 4 : es;
   const bool rows4 = S <= 4 && W % 4 == 0 && W <= 4096 && ldy % 4 == 0 && ldh % 4 == 0 && !((uintptr_t)x & 15) &&
-                     !(((uintptr_t)y | (uintptr_t)w) & (4 * es - 1)) && !((uintptr_t)h & (4 * eh - 1));
-  if (slabs < 0 || (slabs && (!y || !rows4 || ((uintptr_t)y & 15)))) throw std::runtime_error("stream_add_norm: slabs of rows of four only");
+                     !(((uintptr_t)y | (uintptr_t)w) & (4 * es - 1)) && !((uintptr_t)h & (4 * eh - 1)) &&
+                     !(slabs && ((uintptr_t)y & 15));
+  if (slabs < 0 || (slabs && !y)) throw std::runtime_error("stream_add_norm: slabs of a product only");
 #define LAUNCH_SR(TH_, S_)                                                                                           \
   launch_stream_rows<T, TH_, S_>((float*)x, (const T*)y, ldy, (const float*)mix, (const float*)outw, c, (const float*)inw, \
                                  (const T*)w, eps, rms, (TH_*)h, ldh, T_, W, slabs, st)
@@ -220,7 +222,7 @@ void launch_stream_add_norm(void* x, const void* y, int64_t ldy, const void* mix
   else if (rows4) LAUNCH_SR(TH_, 4);                                                                                 \
   else stream_add_norm_kernel<T, TH_><<<T_, 256, lds, st>>>((float*)x, (const T*)y, ldy, (const float*)mix,                \
                                                        (const float*)outw, c, (const float*)inw, (const T*)w, eps, rms, \
-                                                       (TH_*)h, ldh, S, T_, W)
+                                                       (TH_*)h, ldh, S, T_, W, slabs)
   DISPATCH_T(dt, T, {
     if (h_f32) {
       LAUNCH_SAN(float);

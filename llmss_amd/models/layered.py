@@ -583,8 +583,9 @@ class LayeredLM:
         self._cu_decode = {}
         self._angles = {}
         self.tap = None  # tap(i, x): called with the fp32 residual after layer (run) i (debugging, tests)
-        # sublayers' outputs go straight into the residual streams' or the sandwich block's closing op, whose kernel of whole rows in
-        # registers takes the slabs of a split product too (a norm in one part, up to four streams, widths in fours)
+        # sublayers' outputs go straight into the residual streams' or the sandwich block's closing op, which takes the slabs of a split
+        # product too: asked for where its kernel of whole rows in registers can serve (a norm in one part, up to four streams, widths in
+        # fours), though operands at odd places - a gate behind an odd number of columns - leave it to the general kernel
         self.closing = cfg.hidden_size % 4 == 0 and (
             cfg.norm_groups == 1 if cfg.sandwich else not cfg.post_norm and not cfg.parallel_block and cfg.streams <= 4)
         self.proj = None  # the last sublayer's first GEMM output (a sandwich block reads its gate logits there)

@@ -539,3 +539,16 @@ def test_fp32_decode_graphs_reproduce_the_oracle_exactly(cases):
     outs = eng.generate(prompts, SamplingParams(max_new_tokens=20, is_greedy=True, ignore_eos=True))
     for p, out in zip(prompts, outs):
         assert out == oracle.greedy(c.cfg, c.sd, p, 20)
+
+
+@pytest.mark.parametrize("device,dtype", RUNS)
+def test_gate_logits_behind_an_odd_number_of_columns(tmp_path, monkeypatch, device, dtype):
+    """30 state-space heads: the residual gate's columns of the mixer's projection start at 2 inner + 2 groups state + heads = 3902, which is
+    no multiple of four numbers, and the output products of 33 and 64 rows leave slabs of a split K to the closing op."""
+    monkeypatch.setitem(CONFIGS, "heads30", model(97, 512, 1e-5, 1.0, 1.0, 0, None, [ssd(30, 64, 16, 1, 4, 1, mlp=dense(48)),
+                                                                                  ssd(30, 64, 16, 1, 4, 1)]))
+    c = Case("heads30", tmp_path, device, dtype)
+    assert c.model.w.layers[0].mix.cols["rg"] == 3902
+    for n in (33, 64):
+        t = toks(n, c.V, n)
+        c.close(c.engine().replay_step([(0, t, list(range(n)))], end=[0]), c.ref(t), f"{n} rows")

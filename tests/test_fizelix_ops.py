@@ -171,6 +171,37 @@ def test_closing_ops_sum_split_products(M, N, K):
     close(got, want.cpu(), torch.bfloat16, "next input of the streams")
 
 
+@gpu
+@pytest.mark.parametrize("M,N,K", [(33, 1600, 3200), (64, 512, 1920)])
+@pytest.mark.parametrize("col,extra", [(0, 0), (0, 2), (2, 6), (2, 0), (3, 1)])
+def test_closing_ops_sum_split_products_beside_operands_at_odd_places(M, N, K, col, extra):
+    """The same where the gate is what a model has: columns of the projection from ``col`` on, rows N + col + extra apart, and where the
+    norm's weight, the addend and the next weight start ``col`` numbers into their memory. None of it turns slabs away. Tolerances
+    as above."""
+    from llmss_amd.ops import hip as H
+
+    torch.manual_seed(0)
+    r = lambda *s, dt=torch.float32: torch.randn(*s, device="cuda").to(dt)
+    at = lambda t: torch.cat([t.new_zeros(col), t.flatten()])[col:].view(t.shape)
+    a, w = r(M, K, dt=torch.bfloat16), (r(N, K) * K ** -0.5).to(torch.bfloat16)
+    y = lambda: H.linear_f(a, w, torch.bfloat16, closing=True)
+    assert isinstance(y(), H.PartialSum)
+    full = (a.float() @ w.float().T).to(torch.bfloat16)
+    proj = r(M, N + col + extra, dt=torch.bfloat16)
+    x, gate, rb, wp, add, wn = r(M, N), proj[:, col:col + N], at(r(N)), at(r(N)), at(r(M, N)), at(r(N))
+    x2 = x.clone()
+    got = H.sandwich_add_norm(x, y(), gate, rb, wp, 1e-5, add, wn, torch.bfloat16)
+    want = H.sandwich_add_norm(x2, full, gate, rb, wp, 1e-5, add, wn, torch.bfloat16)
+    close(x, x2.cpu(), torch.bfloat16, "residual")
+    close(got, want.cpu(), torch.bfloat16, "next input")
+    xs, mix, outw, inw = r(2, M, N), r(2, 2), r(2), r(2)
+    xs2, nw = xs.clone(), at(wn.to(torch.bfloat16))
+    got = H.stream_add_norm(xs, y(), mix, outw, 0.7, inw, nw, 1e-5, False, torch.bfloat16)
+    want = H.stream_add_norm(xs2, full, mix, outw, 0.7, inw, nw, 1e-5, False, torch.bfloat16)
+    close(xs, xs2.cpu(), torch.bfloat16, "streams")
+    close(got, want.cpu(), torch.bfloat16, "next input of the streams")
+
+
 @pytest.mark.parametrize("device,dtype", RUNS)
 @pytest.mark.parametrize("W,d,part", [(48, 6, 2), (50, 1, 0), (264, 19, 1)])
 def test_token_side_add(device, dtype, W, d, part):
