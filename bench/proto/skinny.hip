@@ -447,7 +447,7 @@ int main(int argc, char** argv) {
     vs.push_back({nm, [=](const bf16_t* W, int) {                                                               \
       dim3 grid((N + BN - 1) / BN, S);                                                                          \
       gemm_tiled_kernel<64, BN, NS, true><<<grid, 256>>>(X, K, W, K, nullptr, Y, N, S > 1 ? (float*)ws : nullptr, \
-                                                         M, N, K, 0, 0, nullptr);                               \
+                                                         M, N, K, 0, 0, nullptr, nullptr, QkvEpi{});            \
     }});                                                                                                        \
   }
     T(256, 2)

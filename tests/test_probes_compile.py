@@ -10,7 +10,6 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 PROBES = sorted(os.path.relpath(p, ROOT) for p in glob.glob(os.path.join(ROOT, "bench", "**", "*.hip"), recursive=True))
-PROBES.remove("bench/proto/skinny.hip")
 
 
 @pytest.mark.skipif(shutil.which(HIPCC) is None, reason="needs hipcc")
