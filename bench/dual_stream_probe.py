@@ -45,7 +45,8 @@ def main():
         n = r1 - r0
         return StepInput("decode", ids[r0:r1], pos[r0:r1], slots[r0:r1], block_tables=bt[r0:r1],
                          ctx_lens=cl[r0:r1], max_ctx=ctx + 1,
-                         decode_splits=H.decode_splits(n, m.plan.nkv_l, ctx + 1, bs))
+                         decode_splits=H.decode_splits(n, m.plan.nkv_l, ctx + 1, bs, m.plan.nh_l // m.plan.nkv_l,
+                                                       m.cfg.head_dim, m.kv_fp8))
 
     def fwd(inp):
         h = m.hidden_states(inp, kv)

@@ -405,7 +405,9 @@ class LLMEngine:
             m.tbo_min = old
 
     def _splits(self, b):
-        return _hip_ops.decode_splits(b, self.model.plan.nkv_l, self.max_model_len, self.block_size)
+        p = self.model.plan
+        return _hip_ops.decode_splits(b, p.nkv_l, self.max_model_len, self.block_size, p.nh_l // max(1, p.nkv_l), self.cfg.head_dim,
+                                      bool(self.model.kv_fp8))
 
     # -------------------------------------------------------------------------- requests
     def add_request(self, prompt_ids: Sequence[int], params: Optional[SamplingParams] = None,

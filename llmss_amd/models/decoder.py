@@ -421,7 +421,8 @@ class DecoderLM:
     def _sub_step(self, inp: StepInput, r0: int, r1: int, block_size: int) -> StepInput:
         splits = inp.decode_splits
         if splits is not None and inp.input_ids.is_cuda:
-            splits = _hip_ops().decode_splits(r1 - r0, self.plan.nkv_l, inp.max_ctx, block_size)
+            splits = _hip_ops().decode_splits(r1 - r0, self.plan.nkv_l, inp.max_ctx, block_size,
+                                              self.plan.nh_l // self.plan.nkv_l, self.cfg.head_dim, self.kv_fp8)
         return StepInput("decode", inp.input_ids[r0:r1], inp.positions[r0:r1], inp.slots[r0:r1],
                          block_tables=inp.block_tables[r0:r1], ctx_lens=inp.ctx_lens[r0:r1], max_ctx=inp.max_ctx,
                          decode_splits=splits)

@@ -329,18 +329,23 @@ class workspace_slot:
 _DECODE_WS = _Slotted(DecodeWorkspace)
 
 
-def decode_splits(B: int, nkv: int, max_ctx: int, block_size: int) -> tuple:
-    """(num_splits, partition_size): ~8 workgroups per CU (2048), partitions >= 256 tokens.
+def decode_splits(B: int, nkv: int, max_ctx: int, block_size: int, group: int = 1, head_dim: int = 128, fp8: bool = False) -> tuple:
+    """(num_splits, partition_size): ~8 workgroups per CU (2048), partitions >= 256 tokens. ``group``: query heads of a kv head;
+    ``fp8``: rows of the fp8 cache.
 
     Measured (bench/attn_bench.py): with few (sequence, kv-head) pairs - GQA / TP-sharded kv heads -
     each workgroup otherwise walks the whole context serially and the KV stream drops to 2-3 TB/s.
 
-    From 640 (sequence, kv-head) pairs on and up to 2048 positions: one partition, no sum behind it. 2.5 workgroups per CU are
-    in flight at once, and the start and end of each cost more than a fuller chip gives (us, three or four partitions and
-    one: 23 sequences of 32 heads to 1777 positions in fp8 67 and 61, 31 to 513 in bf16 41 and 38; at 4000 positions 48 of 8 heads
-    in bf16 would lose 13 %). A partition's pages stay within what the kernel stages (256)."""
+    From 640 (sequence, kv-head) pairs on, contexts that one workgroup walks as fast as the chip is done with the others take one
+    partition, with no sum behind it: fp8 rows of up to 128 numbers, one or two heads a row, to 800 positions, and bf16 rows of 64, one
+    head, to 512. The lengths behind ``max_ctx`` are not known here, so the line lies where no mix of them was slower (old time over
+    new, 640 - 2000 pairs, all of one length, evenly spread, or one long one among others an eighth as long): there 0.97 - 1.8, 1.2 on average;
+    fp8 rows of 128 at 1024 positions 0.94 - 1.5, at 2048 0.75 - 1.2; bf16 rows of 128 at 400 0.83 - 1.2, at 2048 0.53 - 1.1; groups of
+    four and eight 0.7 - 1.3 at 520, 0.54 - 1.1 at 2048. us, two or three partitions and one: 22 sequences of 32 heads at 800 positions in fp8 37.7
+    and 33.6, 31 of 25 heads of 64 at 520 in bf16 25.1 and 20.9. A partition's pages stay within what the kernel stages (256)."""
     wgs = max(1, B * nkv)
-    if wgs >= 640 and max_ctx <= min(2048, 256 * block_size):
+    alone = 800 if fp8 and group <= 2 and head_dim <= 128 else 512 if not fp8 and group == 1 and head_dim <= 64 else 0
+    if wgs >= 640 and max_ctx <= min(alone, 256 * block_size):
         return 1, math.ceil(max_ctx / block_size) * block_size
     want = max(1, math.ceil(2048 / wgs))
     nsplit = max(1, min(want, math.ceil(max_ctx / 256)))
@@ -361,7 +366,7 @@ def attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, nh, nkv, D, scale, 
     _check(ctx_lens.dtype == torch.int32 and ctx_lens.numel() >= B and ctx_lens.is_contiguous(), "ctx_lens int32")
     bs = k_cache.shape[2]
     _check(block_tables.shape[1] * bs >= max_ctx, "block table too short for max_ctx")
-    nsplit, psize = splits if splits is not None else decode_splits(B, nkv, max_ctx, bs)
+    nsplit, psize = splits if splits is not None else decode_splits(B, nkv, max_ctx, bs, nh // nkv, D, kv8)
     _check(nsplit * psize >= max_ctx, "splits do not cover max_ctx")
     y = out if out is not None else torch.empty(B, nh * D, dtype=q.dtype, device=q.device)
     po, pml = _DECODE_WS.get(B, nh, nsplit, D, q.device) if nsplit > 1 else (None, None)

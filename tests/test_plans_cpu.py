@@ -134,3 +134,20 @@ def test_products_are_cut_where_the_last_wave_of_tiles_is_nearly_empty(M, N, K, 
     rows, cols = H.lib().gemm_cut(M, N, K, glu)
     assert not (rows and cols) and rows % 256 == 0 and cols % 256 == 0 and rows < M and cols < N
     assert bool(rows or cols) == (cut is not None) and (cut != "rows" or rows == 8192)
+
+
+@pytest.mark.parametrize("block", [2, 16, 48])
+@pytest.mark.parametrize("group,head_dim,fp8,alone", [(1, 128, True, 800), (2, 128, True, 800), (1, 64, True, 800), (1, 64, False, 512),
+                                                      (4, 128, True, 0), (1, 256, True, 0), (1, 128, False, 0), (2, 64, False, 0),
+                                                      (8, 128, False, 0)])
+def test_one_partition_only_where_no_mix_of_lengths_is_slower(group, head_dim, fp8, alone, block):
+    """Decode attention's partitions: one from 640 (sequence, kv-head) pairs up to the positions that a workgroup walks in time, or where a
+    partition of 256 holds them or the pairs fill the chip; elsewhere as many as fill it, of at least 256. They cover the contexts."""
+    from llmss_amd.ops import hip as H
+
+    for pairs in (1, 639, 640, 1000, 2047, 2048, 5000):
+        for ctx in (1, 256, 257, 400, 512, 513, 800, 801, 2048, 4000):
+            n, size = H.decode_splits(pairs, 1, ctx, block, group, head_dim, fp8)
+            assert n * size >= ctx and size % block == 0 and (n - 1) * size < ctx
+            one = pairs >= 640 and ctx <= min(alone, 256 * block) or ctx <= 256 or pairs >= 2048
+            assert (n == 1) == one and n <= -(-2048 // pairs)
