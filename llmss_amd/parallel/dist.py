@@ -12,8 +12,10 @@ and ``FakeGroup`` (``dist.py:14-37``). Differences, by design:
   bootstrapped over a CPU (gloo) process group: collectives are raw ``ncclAllReduce`` /
   ``ncclAllGather`` calls on the caller's current HIP stream, so they are captured into the decode
   HIP graphs with the rest of the step, with no torch Work / event / watchdog in the loop.
-  ``LLMSS_COMM=torch`` selects torch's ``nccl`` process group instead (RCCL as well), created with
-  the reference's high-priority-stream option (``dist.py:52-53``).
+  ``LLMSS_COMM=torch`` selects torch's ``nccl`` process group instead (RCCL as well), on a stream of normal
+  priority where the reference asks for a high one (``dist.py:52-53``): beside a queue of higher priority the compute
+  queue's waves are preempted for every communication kernel, which made those overlapped with it about 3 times slower,
+  and work on streams of different priorities can stop for good.
 * ``DEBUG=1`` keeps the reference's "fake" semantics: every rank computes with its own shard and
   no communication happens (shape/loader debugging only, numerically wrong by construction).
 """
@@ -360,13 +362,6 @@ def _env_int(name: str, default: int) -> int:
     return int(v) if v not in (None, "") else default
 
 
-def _pg_options(backend: str):
-    """torch ``nccl`` process groups get the reference's high-priority internal stream (``dist.py:52-53``)."""
-    if backend != "nccl" or not hasattr(dist, "ProcessGroupNCCL"):
-        return None
-    return dist.ProcessGroupNCCL.Options(is_high_priority_stream=True)
-
-
 def comm_mode() -> str:
     """Data plane on GPUs: 'native' (csrc/comm.cpp RcclComm, default) or 'torch' (torch's nccl process group)."""
     m = os.environ.get("LLMSS_COMM", "native")
@@ -633,7 +628,6 @@ def initialize_distributed(timeout_s: Optional[int] = None, backend: Optional[st
         kwargs = dict(backend=backend, world_size=world_size, rank=rank, timeout=timedelta(seconds=timeout_s))
         if backend == "nccl":
             kwargs["device_id"] = torch.device("cuda", torch.cuda.current_device())
-            kwargs["pg_options"] = _pg_options(backend)
         dist.init_process_group(**kwargs)
     tp = world_size // dp
     comm, err = None, ""
@@ -659,7 +653,7 @@ def initialize_distributed(timeout_s: Optional[int] = None, backend: Optional[st
             # bootstrap and stream handling) instead of failing the run
             log.warning("rank %d: native RCCL communicator failed (%s); data plane on torch's nccl group",
                         rank, err or "on a peer")
-            data = dist.new_group(list(range(world_size)), backend="nccl", pg_options=_pg_options("nccl"))
+            data = dist.new_group(list(range(world_size)), backend="nccl")
             return TPGroup(rank, world_size, group=data), rank, world_size
     log.info("rank %d/%d initialised: process group %s, data plane %s", rank, world_size, backend,
              "native RCCL" if comm is not None else backend)
@@ -671,7 +665,7 @@ def initialize_distributed(timeout_s: Optional[int] = None, backend: Optional[st
     mine = None
     for r in range(dp):  # new_group is collective over the world: every rank creates every group
         ranks = list(range(r * tp, (r + 1) * tp))
-        data = dist.new_group(ranks, backend=backend, pg_options=_pg_options(backend)) if tp > 1 else None
+        data = dist.new_group(ranks, backend=backend) if tp > 1 else None
         ctrl = dist.new_group(ranks, backend="gloo", timeout=timedelta(seconds=ctrl_timeout)) if tp > 1 else None
         if rank in ranks:
             mine = (r, data, ctrl)

@@ -95,3 +95,30 @@ def test_dp2_tp2_world_split(tmp_path):
                 p.terminate()
     assert [p.exitcode for p in procs] == [0] * 4
     assert res[0] == want[0::2] and res[1] == want[1::2]
+
+
+def test_torch_data_plane_asks_for_no_stream_priority(monkeypatch):
+    """The nccl process group is created with torch's own options: streams of different priorities beside each other slow the compute
+    queue down and can stop for good."""
+    import torch
+    import torch.distributed as dist
+
+    from llmss_amd.parallel.dist import initialize_distributed
+
+    class Made(Exception):
+        pass
+
+    def init(**kwargs):
+        seen.update(kwargs)
+        raise Made
+    seen = {}
+    for k, v in dict(RANK="0", WORLD_SIZE="2", LOCAL_RANK="0").items():
+        monkeypatch.setenv(k, v)
+    monkeypatch.delenv("DEBUG", raising=False)
+    monkeypatch.setattr(dist, "is_initialized", lambda: False)
+    monkeypatch.setattr(dist, "init_process_group", init)
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    with pytest.raises(Made):
+        initialize_distributed(backend="nccl")
+    assert seen["backend"] == "nccl" and not getattr(seen.get("pg_options"), "is_high_priority_stream", False)
