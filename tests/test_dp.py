@@ -6,6 +6,7 @@ import os
 import socket
 import threading
 
+import pytest
 import torch
 import torch.multiprocessing as mp
 
@@ -100,7 +101,6 @@ def test_dp2_tp2_world_split(tmp_path):
 def test_torch_data_plane_asks_for_no_stream_priority(monkeypatch):
     """The nccl process group is created with torch's own options: streams of different priorities beside each other slow the compute
     queue down and can stop for good."""
-    import torch
     import torch.distributed as dist
 
     from llmss_amd.parallel.dist import initialize_distributed
