@@ -19,10 +19,11 @@
 // whole rows (all groups' keys side by side) an instruction, into registers a tile ahead and then to LDS. Operands straight from
 // the cache, each wave its own 64-byte pieces, took 5.3 us per 32 keys of both walks at 16 heads, this 3.5: about half of it the vector
 // ALUs (3 transcendental instructions a pair of row and key and head in either walk), the rest barriers and waits for LDS.
-// us, the two kernels of attention_sink.hip and this: 16 heads of 128, 8 prompts of 1024 604 -> 152, one of 4000 716 -> 442, 64 of 24
-// 53 -> 17; 8 heads 140 -> 95, 328 -> 302, 24 -> 11. One workgroup walks all keys of its rows, where the other form spreads groups and
-// column chunks over workgroups: while those still fit the chip it is the faster one (2 portions of 512 behind 1500 keys: 154 and 174,
-// one row behind 4000: 235 and 438), which is what the caller's rule goes by.
+// us, the two kernels of attention_sink.hip and this: 16 heads of 128, 8 prompts of 1024 418 and 153, 64 of 24 47 and 17, one of 4000 442 and
+// 429; 8 heads 112 and 95, 23 and 10, 168 and 302. One workgroup walks all keys of its rows, where the other form spreads groups and
+// column chunks over workgroups: while those still fit the chip it is the faster one (2 portions of 512 behind 1500 keys: 104 and 174,
+// one row behind 4000: 149 and 438), which is what the caller's rule weighs. Two and four groups only: 32 keys and values of eight, with their 32
+// heads' weights in fp32 and mixed, would take 224 KB of LDS.
 #include "anytype.h"
 
 namespace {

@@ -1609,14 +1609,42 @@ def sink_attn(q, k_cache, v_cache, block_tables, cu, ctx_lens, heads, kv_heads, 
     return out
 
 
-def _mix_in_one(n: int, rows: int, kv_heads: int, vdim: int, longest: int) -> bool:
-    """Whether ``n`` sequences of at most ``rows`` rows and ``longest`` keys take csrc/attention_mix.hip, one workgroup per 16 rows. The
-    general kernel has kv_heads * column chunks (256 wide) times as many, each as long: while they fit the chip (two per CU) it is as fast
-    or faster, and far slower beyond that. Short contexts are a matter of launches: one instead of two (us, 16 heads: one row
-    behind 32 keys 20 and 11, behind 512 43 and 62; 64 rows behind 256 46 and 36, behind 1024 118 and 119)."""
+# What soft-capped sink attention with head mixing costs in its two forms, us, by (steps of single rows, value groups): a start, a key of the
+# longest context, a key of a 16-row block where all blocks share the chip (of each group and column chunk in the general form, at 512
+# workgroups), a row. Fitted over 20980 random steps (1 - 64 single rows, 1 - 32 portions to 4000 rows, fresh, behind prefixes, one long
+# one among short ones; 8 and 16 heads of 128 and 64): 2.5 - 5 % off on average.
+_MIX_COST = {  # sink_attn and talk_mix, sink_attn_mix's own kernel
+    (False, 4): ((21.0, 0.0345, 0.0522, 0.0214), (13.6, 0.106, 0.239, 0.00185)),
+    (False, 2): ((15.8, 0.0342, 0.0542, 0.00539), (9.16, 0.0734, 0.115, 0.00103)),
+    (True, 4): ((19.7, 0.0335, 0.0756, 0.0451), (11.1, 0.103, 0.737, 0.00686)),
+    (True, 2): ((14.3, 0.0325, 0.166, 0.0174), (8.27, 0.0712, 0.469, 0.00312)),
+}
+
+
+def _mix_in_one(n: int, rows: int, kv_heads: int, vdim: int, longest: int, total: int = 0) -> bool:
+    """Whether ``n`` sequences of at most ``rows`` rows, ``total`` in all (0: all as long), and at most ``longest`` keys take csrc/attention_mix.hip. It has one
+    workgroup per 16 rows, whose walk over the keys is about three times as long as the general kernel's, which has kv_heads * column
+    chunks (256 wide) times as many: so it pays where those do not fit the chip at once, or where contexts are short and a launch counts.
+    The lengths behind the bounds are not known here. The general form is taken at the least work that they allow (rows spread
+    evenly beside the longest portion, no prefixes), the one kernel with the longest portion behind the longest prefix, on the part of
+    the chip that its workgroups meet: every n-th one is its own, and they go round 8 dies of 4 engines. Against the general form:
+    0.83 of the time on average over the portions of those steps, 0.79 over the single rows, 1.10 at worst. us, general form and one
+    kernel, 16 heads of 128 in four groups: 8 prompts of 1024 418 and 153, one of 1212 80 and 142, 26 portions of 41 rows behind up to 3900
+    keys 168 and 433, one prompt of 2176 beside 31 short ones 601 and 2161, 33 single rows behind up to 486 keys 40 and 63."""
+    g, m = _MIX_COST[rows == 1, kv_heads]
+    total = total or n * rows
+    per = kv_heads * -(-kv_heads * vdim // 256)  # the general form's workgroups per 16 rows
     if rows == 1:
-        return longest <= (192 if n < 32 else 512)
-    return longest <= 256 or n * -(-rows // 16) * kv_heads * -(-kv_heads * vdim // 256) > 512
+        keys, least, most = n, 1, longest
+    else:
+        rest = (total - rows) / max(1, n - 1)
+        least, most = rows * (rows + 16) / 32, rows * (longest - rows / 2 + 8) / 16
+        keys = least + (n - 1) * rest * (rest + 16) / 32
+
+    def us(c, keys, alone, wgs, share):
+        return c[0] + math.hypot((c[1] * longest) ** 2, (c[2] * wgs * max(keys, alone * share) / 512) ** 2) ** 0.5 + c[3] * total
+
+    return us(m, keys, most, 1, math.gcd(n, 32)) < us(g, keys, least, per, max(1, math.gcd(n * per, 32) / per))
 
 
 def sink_attn_mix(q, k_cache, v_cache, block_tables, cu, ctx_lens, talk, c, heads, kv_heads, dim, vdim, scale, softcap,
@@ -1633,7 +1661,7 @@ def sink_attn_mix(q, k_cache, v_cache, block_tables, cu, ctx_lens, talk, c, head
              and lib().mix_attn_ok(heads, kv_heads, dim, vdim, bs, maxb, cap) and out.stride(0) % 4 == 0
              and not (k_cache.data_ptr() % 16 or v_cache.data_ptr() % 16 or q.data_ptr() % 16 or out.data_ptr() % 8) and 0 <= nd <= B)
     longest = min(int(max_ctx) or maxb * bs, maxb * bs)
-    one = [built and _mix_in_one(n, ql, kv_heads, vdim, longest) for _, n, ql in parts]
+    one = [built and _mix_in_one(n, ql, kv_heads, vdim, longest, n if ql == 1 and first == 0 else T - nd) for first, n, ql in parts]
     if not any(one):
         O = sink_attn(q, k_cache, v_cache, block_tables, cu, ctx_lens, heads, kv_heads, dim, vdim, scale, softcap,
                       talk is not None, max_qlen=max_qlen, num_decode=num_decode)

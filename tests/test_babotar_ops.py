@@ -336,9 +336,28 @@ def test_heads_mixed_before_the_values_at_the_edges_of_the_tiles(device, dtype, 
         attention_case(device, dtype, H, G, d, dv, [560, 530], [[560], [530]], d ** -0.5, cap, True, bs=bs, seed=8, mix=True)
 
 
+# us of 16 heads in four groups, 8 in two: sink_attn and talk_mix, one kernel
+@pytest.mark.parametrize("n,rows,total,longest,G,one", [
+    (8, 1024, 8192, 1024, 4, True),
+    (64, 24, 1536, 24, 4, True),
+    (1, 1212, 1212, 1212, 4, False),  # 80, 142
+    (26, 41, 646, 3949, 4, False),  # 168, 433
+    (32, 2176, 4408, 2176, 4, False),  # 601, 2161
+    (3, 349, 877, 3371, 4, False),  # 157, 368
+    (33, 1, 33, 486, 4, False),  # 40, 63
+    (42, 1, 42, 493, 2, False),  # 30, 44
+    (64, 1, 64, 32, 4, True),
+    (1, 1, 1, 32, 2, True),
+    (10, 840, 5871, 840, 2, True)])
+def test_heads_are_mixed_before_the_values_only_where_that_was_faster(n, rows, total, longest, G, one):
+    from llmss_amd.ops import hip as H
+
+    assert H._mix_in_one(n, rows, G, 128, longest, total) == one
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("nd,n,prefix,one", [(3, 520, 0, (False, True)), (3, 40, 400, (False, False)), (40, 40, 100, (True, True)),
-                                             (40, 400, 0, (True, False)), (0, 520, 96, (True,))])
+@pytest.mark.parametrize("nd,n,prefix,one", [(40, 150, 0, (False, True)), (3, 40, 400, (False, False)), (40, 90, 0, (True, True)),
+                                             (40, 40, 100, (True, False)), (0, 1300, 40, (True,))])
 def test_single_rows_and_portions_choose_their_form_of_mixing_alone(nd, n, prefix, one):
     """A step of single rows and two portions, each part in one kernel or in two by its own sizes; a padded row without keys."""
     from llmss_amd.ops import hip as H
@@ -357,7 +376,7 @@ def test_single_rows_and_portions_choose_their_form_of_mixing_alone(nd, n, prefi
     cu = torch.tensor([0] + rows, device=device).cumsum(0).to(torch.int32)
     ctx = i32(lens, device)
     parts = [(k, r) for k, r in ((nd, 1), (2, n)) if k]
-    assert tuple(H._mix_in_one(k, r, G, dv, maxb * bs) for k, r in parts) == one
+    assert tuple(H._mix_in_one(k, r, G, dv, maxb * bs, k if r == 1 else 2 * n - 3) for k, r in parts) == one
     out = torch.full((len(q), H_ * dv), float("nan"), dtype=torch.bfloat16, device=device)
     H.sink_attn_mix(q, kc, vc, bt, cu, ctx, talk, 0.8, H_, G, d, dv, d ** -0.5, 30.0, out, max_qlen=n, num_decode=nd)
     O = H.sink_attn(q, kc, vc, bt, cu, ctx, H_, G, d, dv, d ** -0.5, 30.0, True)  # vector kernel, fp32 weights
