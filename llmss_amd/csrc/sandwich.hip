@@ -111,9 +111,10 @@ __device__ __forceinline__ void norm_out(float* buf, float ss, const SandwichArg
   }
 }
 
-// Takes slabs like the kernel of whole rows below, at any alignment: 33 rows of 1600, two launches with the product (K = 3200) that leaves four
-// slabs and a gate of odd columns, 16.0 us, 17.3 with the product finished first.
-template <typename T, int V>
+// SLABS: y is slabs, as the kernel of whole rows below takes them, at any alignment: 33 rows of 1600, two launches with the product (K =
+// 3200) that leaves four slabs and a gate of odd columns, 16.0 us, 17.3 with the product finished first. (A choice at run time beside the others
+// costs rows without slabs a quarter: 1557 x 4096 15.3 -> 19.8 us.)
+template <typename T, int V, bool SLABS = false>
 __global__ __launch_bounds__(512) void sandwich_add_norm_kernel(SandwichArgs p) {
   extern __shared__ __attribute__((aligned(16))) float buf[];
   __shared__ float red[32];
@@ -161,7 +162,7 @@ __global__ __launch_bounds__(512) void sandwich_add_norm_kernel(SandwichArgs p) 
 #pragma unroll
           for (int i = 0; i < V; ++i) v[i] = fmaf(p.cl, a[i], p.cr * b[i]);
         }
-      } else if (p.slabs) {
+      } else if (SLABS) {
         const float* sp = (const float*)p.y + (int64_t)t * W + c;
         if constexpr (V == 4) {
           const f32x4 q = slab_sum<f32x4>(sp, p.slabs, (int64_t)gridDim.x * W);
@@ -354,6 +355,8 @@ void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const void* e
   DISPATCH_T(dt, T, {
     if (rows && W <= 2048) sandwich_rows_kernel<T, 1><<<T_, W > 1024 ? 512 : 256, 0, st>>>(p);
     else if (rows) sandwich_rows_kernel<T, 2><<<T_, 512, 0, st>>>(p);
+    else if (slabs && vec) sandwich_add_norm_kernel<T, 4, true><<<T_, th, lds, st>>>(p);
+    else if (slabs) sandwich_add_norm_kernel<T, 1, true><<<T_, th, lds, st>>>(p);
     else if (vec) sandwich_add_norm_kernel<T, 4><<<T_, th, lds, st>>>(p);
     else sandwich_add_norm_kernel<T, 1><<<T_, th, lds, st>>>(p);
   });

@@ -51,8 +51,9 @@ void launch_embed_streams(const void* ids, const void* positions, const void* ta
 // If w: u = sum_s inw[s] x_s (inw null: the plain sum), h[t] = norm(u) * w, with
 // rms = 0: (u - mean) / sqrt(var + eps), var the mean squared deviation; rms = 1: u / sqrt(mean(u^2) + eps).
 // TH: storage type of h (the model's, or float when a convolution follows).
-// slabs > 0: y is the fp32 slabs [slabs][T][W] of a product whose K was split, summed here instead of in a launch of their own.
-template <typename T, typename TH>
+// SLABS: y is the fp32 slabs [slabs][T][W] of a product whose K was split, summed here instead of in a launch of their own (in
+// the kernel of whole rows below: slabs > 0).
+template <typename T, typename TH, bool SLABS>
 __global__ __launch_bounds__(256) void stream_add_norm_kernel(float* __restrict__ x, const T* __restrict__ y,
                                                               int64_t ldy, const float* __restrict__ mix,
                                                               const float* __restrict__ outw, float c,
@@ -69,7 +70,7 @@ __global__ __launch_bounds__(256) void stream_add_norm_kernel(float* __restrict_
     for (int s = 0; s < MAX_STREAMS; ++s)
       if (s < S) xs[s] = x[((int64_t)s * T_ + t) * W + col];
     if (y) {
-      const float yv = c * (slabs ? slab_sum<float>((const float*)y + (int64_t)t * W + col, slabs, (int64_t)T_ * W)
+      const float yv = c * (SLABS ? slab_sum<float>((const float*)y + (int64_t)t * W + col, slabs, (int64_t)T_ * W)
                                   : El<T>::ld(y + (int64_t)t * ldy + col));
       float nx[MAX_STREAMS];
 #pragma unroll
@@ -215,14 +216,17 @@ void launch_stream_add_norm(void* x, const void* y, int64_t ldy, const void* mix
 #define LAUNCH_SR(TH_, S_)                                                                                           \
   launch_stream_rows<T, TH_, S_>((float*)x, (const T*)y, ldy, (const float*)mix, (const float*)outw, c, (const float*)inw, \
                                  (const T*)w, eps, rms, (TH_*)h, ldh, T_, W, slabs, st)
+#define LAUNCH_SG(TH_, SLABS_)                                                                                       \
+  stream_add_norm_kernel<T, TH_, SLABS_><<<T_, 256, lds, st>>>((float*)x, (const T*)y, ldy, (const float*)mix,             \
+                                                               (const float*)outw, c, (const float*)inw, (const T*)w, eps, \
+                                                               rms, (TH_*)h, ldh, S, T_, W, slabs)
 #define LAUNCH_SAN(TH_)                                                                                              \
   if (rows4 && S == 1) LAUNCH_SR(TH_, 1);                                                                            \
   else if (rows4 && S == 2) LAUNCH_SR(TH_, 2);                                                                       \
   else if (rows4 && S == 3) LAUNCH_SR(TH_, 3);                                                                       \
   else if (rows4) LAUNCH_SR(TH_, 4);                                                                                 \
-  else stream_add_norm_kernel<T, TH_><<<T_, 256, lds, st>>>((float*)x, (const T*)y, ldy, (const float*)mix,                \
-                                                       (const float*)outw, c, (const float*)inw, (const T*)w, eps, rms, \
-                                                       (TH_*)h, ldh, S, T_, W, slabs)
+  else if (slabs) LAUNCH_SG(TH_, true);                                                                              \
+  else LAUNCH_SG(TH_, false)
   DISPATCH_T(dt, T, {
     if (h_f32) {
       LAUNCH_SAN(float);
@@ -231,6 +235,7 @@ void launch_stream_add_norm(void* x, const void* y, int64_t ldy, const void* mix
     }
   });
 #undef LAUNCH_SAN
+#undef LAUNCH_SG
 #undef LAUNCH_SR
   HIP_CHECK_LAUNCH();
 }
