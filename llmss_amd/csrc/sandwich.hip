@@ -241,8 +241,8 @@ __global__ __launch_bounds__(512) void sandwich_add_norm_kernel(SandwichArgs p) 
 
 // The same for rows of up to 4096 and a norm of one part: a thread keeps NC times four columns of everything in registers, all loads are
 // issued before the first sum, and only two sums pass through LDS. The kernel above asks for the stream and the weights behind the
-// first sum, a round trip more. us, plain rows / gated / four experts' rows: 33 x 2048 4.4 / 4.8 / 5.1 -> 3.7 / 4.1 / 4.3, 8192 x 2048
-// 35.7 / 53.4 / 101 -> 34.2 / 50.5 / 92 (5.5 TB/s of the last), 8192 x 1024 24.7 / 28.3 / 51 -> 20.6 / 24.1 / 41. With eight columns a thread the
+// first sum, a round trip more. us, plain rows / gated / four experts' rows: 33 x 2048 5.0 / 5.3 / 5.5 -> 4.3 / 4.7 / 4.8, 8192 x 2048
+// 36.3 / 42.4 / 84.7 -> 36.4 / 43.9 / 72.6, 8192 x 1024 24.8 / 28.3 / 37.8 -> 20.6 / 24.5 / 34.1. With eight columns a thread the
 // registers leave half the waves: 8192 x 4096 84.6 -> 106, so more than 512 such rows keep the kernel above.
 template <typename T, int NC>
 __global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p) {
@@ -349,11 +349,16 @@ void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const void* e
                    al16(wl) && al16(wr);
   const size_t lds = ((size_t)W + (groups > 1 ? groups : 0)) * 4;
   const int th = T_ <= 512 && W > 1024 ? 512 : 256;  // few rows: more waves to a row
-  // (identity experts and norms in parts keep the general kernel)
-  const bool rows = vec && groups == 1 && !ident && (W <= 2048 || (W <= 4096 && T_ <= 512));
+  // (identity experts and norms in parts keep the general kernel, and so do many rows wider than 1280 unless experts' rows are summed: 1600 -
+  // 8192 rows of 1536 - 2048 in registers took 1.00 - 1.04 of the general kernel's time, gated 1.01 - 1.05, none 1.05 - 1.10, experts' 0.92 - 0.94,
+  // but 1551 with one expert each 1.20: two waves of eight-wave workgroups where the general kernel's four fit at once)
+  const bool rows = vec && groups == 1 && !ident && (W <= 1280 || (W <= 2048 && (T_ <= 1024 || (ey && T_ > 2048))) || (W <= 4096 && T_ <= 512));
   if (slabs < 0 || (slabs && (!y || y2))) throw std::runtime_error("sandwich_add_norm: slabs of one product only");
+  // whole waves, no more than the row has columns for (256 and 512 threads: 1600 rows and more of 256 1.44, of 1280 1.11 times as long), but for
+  // 448, which spread unevenly over the SIMDs (1792 wide: 1.07)
+  const int rth = W <= 1536 ? (W / 4 + 63) / 64 * 64 : 512;
   DISPATCH_T(dt, T, {
-    if (rows && W <= 2048) sandwich_rows_kernel<T, 1><<<T_, W > 1024 ? 512 : 256, 0, st>>>(p);
+    if (rows && W <= 2048) sandwich_rows_kernel<T, 1><<<T_, rth, 0, st>>>(p);
     else if (rows) sandwich_rows_kernel<T, 2><<<T_, 512, 0, st>>>(p);
     else if (slabs && vec) sandwich_add_norm_kernel<T, 4, true><<<T_, th, lds, st>>>(p);
     else if (slabs) sandwich_add_norm_kernel<T, 1, true><<<T_, th, lds, st>>>(p);

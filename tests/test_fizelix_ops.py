@@ -109,7 +109,8 @@ def test_sandwich_add_norm(device, dtype, W):
 
 @gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("T,W", [(3, 4), (5, 1020), (2, 1024), (4, 1028), (3, 2048), (6, 2052), (2, 4096), (513, 2052), (3, 4100)])
+@pytest.mark.parametrize("T,W", [(3, 4), (5, 1020), (2, 1024), (4, 1028), (3, 2048), (6, 2052), (2, 4096), (513, 2052), (3, 4100),
+                                 (3, 60), (1025, 1280), (1024, 1284), (1025, 1284), (2, 1536), (2, 1540)])
 @pytest.mark.parametrize("what", ["plain", "gated", "experts", "pair", "normed pair", "none"])
 def test_sandwich_add_norm_at_the_widths_of_its_kernels(dtype, T, W, what):
     """Rows around what a workgroup's registers hold and around the number of rows that keeps the general kernel; every kind of y:
