@@ -367,11 +367,24 @@ static int extend_group(int G) {
   return 1;
 }
 
+// Whether a step of `total` rows (0: not known, the longest portion B times) takes two groups of slots a wave, half as many workgroups that are
+// each 1.4 - 1.6 times as long: from as many of them on as the rows fill, whatever the portions' lengths. 28 thousand random steps (1 - 24
+// portions to 4000 rows, even, uneven and one long one, to 3000 keys of prefix), time of two groups over one by that number: heads of 128, 320 -
+// 420 1.02, 420 - 520 0.95, 520 - 640 0.90, from 800 on 0.80; heads of 64, 420 - 520 1.15, 640 - 800 1.05, 800 - 1100 1.02, beyond 0.93.
+// (By the longest portion alone, from 320 on, steps of uneven portions took up to 1.6 times as long.) us, 32 heads of 128, one group and
+// two: 2 portions of 950 behind as many 111 and 94, 1 of 1500 162 and 135. Heads of 256 would leave a wave per SIMD: 7 x 1433 rows of 16
+// heads 289 and 410. The twin's rows need a wave.
+bool attn_extend_two(int total, int B, int max_qlen, int nh, int nkv, int D) {
+  const int G = nh / nkv, GE = extend_group(G), rows = 128 / GE;
+  const int64_t t = total > 0 ? total : (int64_t)max_qlen * B;
+  return D <= 128 && max_qlen > 64 / GE && (t + rows - 1) / rows * nkv * (G / GE) >= (D <= 64 ? 1024 : 420);
+}
+
 void launch_attn_extend(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
                         const void* block_tables, int max_blocks, const void* cu_q, const void* ctx_lens, void* out,
                         int64_t out_stride, int B, int max_qlen, int nh, int nkv, int D, int bs, float scale,
                         hipStream_t st, bool kv8, void* q8v, void* s8v, int window, int nsplit, int split_keys,
-                        void* part_o, void* part_ml) {
+                        void* part_o, void* part_ml, int total) {
   if (nh % nkv) throw std::runtime_error("attn_extend: nh must be a multiple of nkv");
   if (B == 0 || max_qlen == 0) return;
   const int G = nh / nkv, GE = extend_group(G);
@@ -380,11 +393,7 @@ void launch_attn_extend(const void* q, int64_t q_stride, const void* k_cache, co
   if ((Q8 != nullptr) != (S8 != nullptr)) throw std::runtime_error("attn_extend: fp8 twin needs both q8 and s8");
   if (Q8 && !(nkv == 1 && GE == G && G <= 16 && (G & (G - 1)) == 0))
     throw std::runtime_error("attn_extend: the fp8 twin needs one kv head and a power-of-two query group <= 16");
-  // Two groups of slots a wave from 320 workgroups of them on (us, 32 heads of 128, one group and two: 2 portions of 950 behind as many,
-  // 512 workgroups, 111 and 94; 1 of 1500, 384, 162 and 135; 2 of 600, 320, 70 and 60; 1 of 1000, 256, 68 and 86; 25 heads of 64, 2 of 700,
-  // 300, 36 and 47). Heads of 256 would leave a wave per SIMD: 7 x 1433 rows of 16 heads 289 and 410. The twin's rows need a wave.
-  const int64_t wgs = (int64_t)((max_qlen + 128 / GE - 1) / (128 / GE)) * nkv * (G / GE) * B;
-  const bool two = D <= 128 && nsplit <= 1 && !Q8 && max_qlen > 64 / GE && wgs >= 320;
+  const bool two = nsplit <= 1 && !Q8 && attn_extend_two(total, B, max_qlen, nh, nkv, D);
   const int rows = (two ? 128 : 64) / GE;
   dim3 grid((max_qlen + rows - 1) / rows, nkv * (G / GE), B);
   if (nsplit > 1) {

@@ -151,3 +151,14 @@ def test_one_partition_only_where_no_mix_of_lengths_is_slower(group, head_dim, f
             assert n * size >= ctx and size % block == 0 and (n - 1) * size < ctx
             one = pairs >= 640 and ctx <= min(alone, 256 * block) or ctx <= 256 or pairs >= 2048
             assert (n == 1) == one and n <= -(-2048 // pairs)
+
+
+@pytest.mark.parametrize("total,B,longest,nh,nkv,D,two", [
+    (1900, 2, 950, 32, 32, 128, True), (3406, 19, 315, 8, 2, 128, False), (775, 12, 500, 8, 8, 128, False), (672, 2, 640, 32, 32, 128, False),
+    (1202, 6, 296, 64, 64, 64, False), (0, 2, 950, 32, 32, 128, True), (4096, 4, 1024, 64, 64, 64, True), (9000, 9, 1000, 16, 16, 256, False),
+    (64, 64, 1, 32, 8, 128, False)])
+def test_two_row_groups_a_wave_only_where_the_rows_fill_the_chip(total, B, longest, nh, nkv, D, two):
+    """Attention behind prefixes: by the rows of the step, not by the longest portion as if all were as long."""
+    from llmss_amd.ops import hip as H
+
+    assert H.lib().attn_extend_two(total, B, longest, nh, nkv, D) == two
