@@ -1731,6 +1731,9 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
       if (s > 1) older += s * 8.0 * M * N / c.slab + (slabs ? 0.0 : c.sum);
       if (s > 1 && !slabs && K <= 5120) faster = 1.0;  // (else two launches, the second waiting for the first)
     }
+    // gated products take the older kernels longer than their plain ones of the same size: 12 x 17472 x 3488 63 us, on the decode kernel 38, 61 x
+    // 18688 x 4656 78, on tiles of 96 columns 58
+    if (glu) older *= M <= 16 ? 1.4 : 1.15;
     const DecCost& c = kDecCost[M <= 16 ? 0 : M <= 32 ? 1 : 2];
     double best = 0;
     int code = 0, sp = 1;

@@ -162,3 +162,14 @@ def test_two_row_groups_a_wave_only_where_the_rows_fill_the_chip(total, B, longe
     from llmss_amd.ops import hip as H
 
     assert H.lib().attn_extend_two(total, B, longest, nh, nkv, D) == two
+
+
+@pytest.mark.parametrize("M,N,K,code", [(12, 17472, 3488, 1024), (7, 2592, 4096, 1024), (2, 2272, 3696, 1024), (61, 18688, 4656, 15),
+                                        (64, 22016, 4096, None), (40, 8192, 2048, None)])
+def test_gated_products_of_few_rows_leave_the_older_kernels(M, N, K, code):
+    """Pairs of columns and their split sums cost the older kernels more than plain products: the decode kernel (hint bit 1024) or tiles of
+    96 columns (15) where those were the faster ones; None: whatever the model says, unsplit."""
+    from llmss_amd.ops import hip as H
+
+    nt, split = H.lib().gemm_plan(M, N, K, False, True, False)
+    assert split == 1 and (code is None or (nt >> 8) & (1024 if code == 1024 else 15) == code), (hex(nt), split)
