@@ -933,8 +933,10 @@ def _babotar_finish(cfg: ModelConfig, get, has, device, dtype) -> ModelWeights:
         mlp = None
         if spec.mlp is not None:
             parts = (g(p + "mlp.gate"), g(p + "mlp.up"))
-            # (the epilogue form needs bf16 rows of whole 16-byte pieces and whole groups of 16)
-            fused = dtype == torch.bfloat16 and W % 16 == 0 and spec.mlp.ff % 16 == 0 and spec.mlp.act in ("gelu_tanh", "silu")
+            # (the epilogue form needs bf16 rows of whole 16-byte pieces and whole groups of 16; products narrower than their K, which the
+            # plain ones split, take up to 1.6 times as long with the gate inside: one row, 2 ff = 768, W = 7632 14 and 20 us)
+            fused = dtype == torch.bfloat16 and W % 16 == 0 and spec.mlp.ff % 16 == 0 and 2 * spec.mlp.ff >= W \
+                and spec.mlp.act in ("gelu_tanh", "silu")
             mlp = DenseMLPWeights(dev(glu_interleave(*parts) if fused else torch.cat(parts, 0)), dev(g(p + "mlp.down")),
                                   interleaved=fused)
         layers.append(SeqBlockWeights(

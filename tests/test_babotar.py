@@ -400,3 +400,26 @@ def test_fp32_decode_graphs_reproduce_the_oracle_exactly(cases):
     outs = eng.generate(prompts, SamplingParams(max_new_tokens=20, is_greedy=True, ignore_eos=True))
     for p, out in zip(prompts, outs):
         assert out == oracle.greedy(c.cfg, c.sd, p, 20)
+
+
+@pytest.mark.parametrize("width,ff,dtype,fused", [(64, 48, "bfloat16", True), (64, 32, "bfloat16", True), (96, 32, "bfloat16", False),
+                                                  (64, 40, "bfloat16", False), (40, 48, "bfloat16", False), (64, 48, "float32", False)])
+def test_rows_of_gate_and_up_alternate_where_the_epilogue_gates(width, ff, dtype, fused):
+    """bf16, whole pieces and groups of 16, at least as many columns as K; the feed-forward gives the same either way."""
+    from llmss_amd.models.layered import create_model
+    from llmss_amd.models.weights import random_babotar_weights
+
+    d = dict(architecture="Babotar", vocab=61, width=width, max_positions=64, norm=dict(eps=1e-6), layers=[lig(1, 8, 8, [0.9], ff=ff)])
+    mc = ModelConfig.from_hf_dict(d)
+    m = create_model(mc, random_babotar_weights(mc, dtype=getattr(torch, dtype), seed=3))
+    W = m.w.layers[0].mlp
+    assert W.interleaved == fused
+    h = torch.randn(5, width, generator=torch.Generator().manual_seed(1)).to(getattr(torch, dtype))
+    from llmss_amd.models.layered import DenseFeedForward
+
+    got = DenseFeedForward.forward(m, W, mc.layer_specs[0].mlp, h).float()
+    gu = W.gu.view(-1, 2, 16, width).transpose(0, 1).reshape(2 * ff, width) if fused else W.gu[:2 * ff]
+    g, u = (h.float() @ gu.float().T).chunk(2, -1)
+    want = (torch.nn.functional.gelu(g, approximate="tanh") * u) @ W.down.float().T
+    # the gated row's rounding to bf16 and the result's (2^-9 each), the products' before the gate without the epilogue
+    assert float((got - want).norm() / want.norm()) < (1e-5 if dtype == "float32" else 1.5e-2)
