@@ -12,7 +12,7 @@ DEVICES = ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)]
 @pytest.mark.parametrize("dtype,out_dtype", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16),
                                              (torch.float32, torch.bfloat16)])
 @pytest.mark.parametrize("residual,bias,silu", [(True, False, False), (True, True, False), (True, False, True), (False, True, True)])
-@pytest.mark.parametrize("C,taps", [(40, 4), (70, 3), (1032, 9), (8, 1), (12, 2), (16, 12)])
+@pytest.mark.parametrize("C,taps", [(40, 4), (70, 3), (1032, 9), (8, 1), (12, 2), (16, 12), (72, 5), (40, 6), (16, 8)])
 def test_single_rows(device, dtype, out_dtype, residual, bias, silu, C, taps):
     gen = torch.Generator().manual_seed(C + taps)
     B, steps, R = 5, 14, taps - 1
