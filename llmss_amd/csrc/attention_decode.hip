@@ -52,7 +52,7 @@ __device__ __forceinline__ float token_sum(float s) {
 // UNROLL tokens. 8 bytes a lane, a rescaled accumulator per token and a division per row's address made about 120
 // vector instructions a wave for 4 tokens' K and V (1.1 KB), this about 55. Rows of D + 16 bytes share their 128-byte lines with
 // their neighbours, which other waves read: no non-temporal hint, that fetches a shared line again. 23 sequences of 32 heads to
-// 1777 positions (298 MB): 76 us and 5 for the sum of three partitions -> 61 in one (4.9 TB/s), 64 of 192 positions 28.9 -> 26.5,
+// 1777 positions (298 MB): 76 us and 5 for the sum of three partitions -> 67 with it, 61 in one (4.9 TB/s), 64 of 192 positions 28.9 -> 26.5,
 // one of 1777 16.3 -> 11.0. Larger groups keep 8 bytes: their accumulators would not fit beside the rows in flight.
 constexpr int decode_elems(int GB, bool KV8) { return KV8 && GB <= 2 ? 16 : 8; }  // dims a lane holds of a token's row
 
@@ -267,32 +267,62 @@ __global__ __launch_bounds__(256, (decode_elems(GB, KV8) == 16 ? (GB == 1 ? 4 : 
   if (lds_pages) walk(std::true_type{});
   else walk(std::false_type{});
 
-  // merge token slots inside the wave
-#pragma unroll
-  for (int o = LPT; o < 64; o <<= 1) {
+  // merge token slots inside the wave. 16 dims a lane: the maximum first, then half of the dims given away a step, so that a lane ends with
+  // the sums of its own few (15 exchanges a head of 64 for 72 where every lane forms all of them, which short contexts are mostly made of: 67
+  // sequences of 64 heads of 64 in pairs to 30 positions 21 -> 12.8 us, 12.1 with 8 dims a lane)
+  constexpr int HELD = E == 16 ? E / TPW : E;  // dims a lane holds after it, from `held` of its own on
+  int held = 0;
+  if constexpr (E == 16) {
 #pragma unroll
     for (int h = 0; h < GB; ++h) {
-      const float mo = __shfl_xor(m[h], o, 64), lo = __shfl_xor(l[h], o, 64);
-      const float mn = fmaxf(m[h], mo);
-      const float a = exp2f(m[h] - mn), c = exp2f(mo - mn);
-      l[h] = l[h] * a + lo * c;
+      float mx = m[h];
 #pragma unroll
-      for (int j = 0; j < E; ++j) {
-        const float ao = __shfl_xor(acc[h][j], o, 64);
-        acc[h][j] = acc[h][j] * a + ao * c;
+      for (int o = LPT; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+      const float f = exp2f(m[h] - mx);
+      m[h] = mx;
+      l[h] *= f;
+#pragma unroll
+      for (int j = 0; j < E; ++j) acc[h][j] *= f;
+#pragma unroll
+      for (int o = LPT, half = E / 2; o < 64; o <<= 1, half >>= 1) {
+        const bool upper = lane & o;
+        l[h] += __shfl_xor(l[h], o, 64);
+#pragma unroll
+        for (int j = 0; j < half; ++j) {
+          const float keep = upper ? acc[h][half + j] : acc[h][j], give = upper ? acc[h][j] : acc[h][half + j];
+          acc[h][j] = keep + __shfl_xor(give, o, 64);
+        }
       }
-      m[h] = mn;
+    }
+#pragma unroll
+    for (int o = LPT, half = E / 2; o < 64; o <<= 1, half >>= 1) held += lane & o ? half : 0;
+  } else {
+#pragma unroll
+    for (int o = LPT; o < 64; o <<= 1) {
+#pragma unroll
+      for (int h = 0; h < GB; ++h) {
+        const float mo = __shfl_xor(m[h], o, 64), lo = __shfl_xor(l[h], o, 64);
+        const float mn = fmaxf(m[h], mo);
+        const float a = exp2f(m[h] - mn), c = exp2f(mo - mn);
+        l[h] = l[h] * a + lo * c;
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+          const float ao = __shfl_xor(acc[h][j], o, 64);
+          acc[h][j] = acc[h][j] * a + ao * c;
+        }
+        m[h] = mn;
+      }
     }
   }
   // merge the 4 waves through LDS: [wave][GB][D] acc + [wave][GB] (m, l)
   __shared__ float s_acc[4][GB][D];
   __shared__ float s_ml[4][GB][2];
-  if (slot == 0) {
+  if (E == 16 || slot == 0) {
 #pragma unroll
     for (int h = 0; h < GB; ++h) {
 #pragma unroll
-      for (int j = 0; j < E; ++j) s_acc[w][h][sub * E + j] = acc[h][j];
-      if (sub == 0) { s_ml[w][h][0] = m[h]; s_ml[w][h][1] = l[h]; }
+      for (int j = 0; j < HELD; ++j) s_acc[w][h][sub * E + held + j] = acc[h][j];
+      if (slot == 0 && sub == 0) { s_ml[w][h][0] = m[h]; s_ml[w][h][1] = l[h]; }
     }
   }
   __syncthreads();

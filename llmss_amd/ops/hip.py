@@ -339,8 +339,8 @@ def decode_splits(B: int, nkv: int, max_ctx: int, block_size: int, group: int = 
     From 640 (sequence, kv-head) pairs on, contexts that one workgroup walks as fast as the chip is done with the others take one
     partition, with no sum behind it: fp8 rows of up to 128 numbers, one or two heads a row, to 800 positions, and bf16 rows of 64, one
     head, to 512. The lengths behind ``max_ctx`` are not known here, so the line lies where no mix of them was slower (old time over
-    new, 640 - 2000 pairs, all of one length, evenly spread, or one long one among others an eighth as long): there 0.97 - 1.8, 1.2 on average;
-    fp8 rows of 128 at 1024 positions 0.94 - 1.5, at 2048 0.75 - 1.2; bf16 rows of 128 at 400 0.83 - 1.2, at 2048 0.53 - 1.1; groups of
+    new, 640 - 2000 pairs, all of one length, evenly spread, or one long one among others an eighth as long): there 0.97 - 1.6, 1.15 on average;
+    fp8 rows of 128 at 1024 positions 0.91 - 1.3, at 2048 0.75 - 1.2; bf16 rows of 128 at 400 0.83 - 1.2, at 2048 0.53 - 1.1; groups of
     four and eight 0.7 - 1.3 at 520, 0.54 - 1.1 at 2048. us, two or three partitions and one: 22 sequences of 32 heads at 800 positions in fp8 37.7
     and 33.6, 31 of 25 heads of 64 at 520 in bf16 25.1 and 20.9. A partition's pages stay within what the kernel stages (256)."""
     wgs = max(1, B * nkv)
