@@ -1353,14 +1353,16 @@ def _rec_common(q, k, v, state, cu, ctx_lens, state_slots, heads, kv_heads, dim,
 
 
 # What the sequences of a step cost in the three forms of a matrix-state recurrence, in us, fitted over 670 random steps of each kind
-# (1 - 170 sequences, up to 400 rows, 2 - 64 heads of 16 - 256 x 16 - 128, a third of them behind 1 - 70 single rows; 6 - 15 % off on
-# average, the choice 1 % above the best form). Chunk by chunk: a start, a part that grows with the state's 16-row tiles and one for
+# (1 - 170 sequences, up to 400 rows, 2 - 64 heads of 16 - 256 x 16 - 128, a third of them behind 1 - 70 single rows). The chunks of decay and
+# the delta rule's preparation have become faster since; over 29 thousand other steps, with portions of up to 1433 rows, the costs are 8 - 14 %
+# off on average and the choice 1.5 (decay), 1.1 (ssd) and 0.7 % (delta) above the best form, 1.0, 0.7 and 0.8 % with costs fitted again,
+# which is why these stand. Chunk by chunk: a start, a part that grows with the state's 16-row tiles and one for
 # each 16 rows, for the longest portion and again for all workgroups at 256 at a time. Token by token: a start, the rows of the longest
 # portion, and the numbers of all rows and states; key dimensions above 128 cost more. Single rows apart: a launch and their states.
 # Chunks at every size from a few rows on took up to 4 times the walk where many sequences fill the chip with short portions or narrow
 # values (53 of up to 14 rows, decay, 32 heads 128 x 64: 82 -> 152 us; 59 of up to 7, delta, 32 heads 128 x 32: 71 -> 217), single rows
 # always apart 1.14 times on average over fp32 rows (one beside a portion of two, decay, 16 heads 128 x 128: 13.4 -> 19.3 us). With this
-# choice: 0.52 (decay), 0.26 (ssd) and 0.52 (delta) of the walk's time.
+# choice: 0.52 (decay), 0.33 (ssd) and 0.59 (delta) of the walk's time over those.
 _REC_COST = {  # (start, part, by tiles, 16 rows, by tiles, workgroups), (start, row, above 128, rows' numbers, columns beside, states', above 128), (launch, numbers)
     "decay": ((3.52, 0.688, 0.82, 0.599, 0.265, 1.05), (10.3, 0.714, 2.06, 0.2, 14.7, 1.21, 2.67), (3.76, 1.09)),
     "ssd": ((1.65, 1.83, 0.816, 0.809, 0.11, 0.57), (7.9, 1.52, 1.33, 0.333, 0.449, 2.19, 2.64), (5.27, 0.976)),
