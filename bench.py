@@ -1,6 +1,6 @@
 """Headline benchmark: output tokens/s (node) + p50 latency for batched generation.
 
-Config (BASELINE.json): Llama-2-7B with tensor parallelism TP = N (one process per GPU, RCCL over
+Config: Llama-2-7B with tensor parallelism TP = N (one process per GPU, RCCL over
 xGMI; TP=8 at N=8) - or ``--model gpt2-xl`` for the GPT-2-XL TP=1 configuration. Random-init
 weights of the exact architecture and synthetic prompt token ids (no network, no checkpoints).
 
@@ -69,7 +69,7 @@ def main():
                          "step's concurrent requests)")
     ap.add_argument("--secondary-serve", default="grpc", choices=["grpc", "engine"],
                     help="secondary config timed through the in-process gRPC Generate service with a separate "
-                         "client process (BASELINE config #2 'served over gRPC'; the engine-direct number is "
+                         "client process (served over gRPC; the engine-direct number is "
                          "reported too), or engine-direct only")
     ap.add_argument("--timeout", type=float, default=float(os.environ.get("LLMSS_BENCH_TIMEOUT_S", "2400")),
                     help="launcher mode: kill every rank and exit 124 after this many seconds")
@@ -214,7 +214,7 @@ def main():
     if RCCL_TUNE_INFO:
         res["rccl_setting_probe"] = dict(RCCL_TUNE_INFO)
     if args.secondary not in ("", "none") and args.simulate_tp <= 1 and args.secondary != args.model:
-        # second BASELINE headline config (GPT-2-XL TP=1, 25 heads: no TP split), driver-timed in the same run;
+        # second headline config (GPT-2-XL TP=1, 25 heads: no TP split), timed in the same run;
         # with N GPUs every rank serves its own TP=1 replica (data parallel) and the node total is reported
         if torch.cuda.is_available():
             torch.cuda.empty_cache()

@@ -1,4 +1,4 @@
-"""Serving benchmark: concurrent gRPC clients against the engine (BASELINE: "GPT-2-XL TP=1 bf16 on
+"""Serving benchmark: concurrent gRPC clients against the engine ("GPT-2-XL TP=1 bf16 on
 one MI355X served over gRPC"; "pubsub producer/consumer under concurrent gRPC clients").
 
   --mode grpc    clients -> gRPC Generate service on the engine driver (direct)

@@ -4,9 +4,9 @@ Same flags, defaults, validation and the same three stdout lines as the referenc
 (``generate.py:21-40,192-196``); launched with ``torchrun --nproc_per_node N generate.py ...``
 (one rank per GPU, RCCL) or plain ``python generate.py ...`` (TP=1, GPU or CPU).
 
-Deliberate fixes: TP=1 works (Q2); temperature/top-k/top-p are actually applied
-(Q1); prompts are not padded, each sequence has its own length and positions (Q3); load time and
-generation throughput are reported on extra lines after the original three (Q12).
+Deliberate fixes: TP=1 works; temperature/top-k/top-p are actually applied;
+prompts are not padded, each sequence has its own length and positions; load time and
+generation throughput are reported on extra lines after the original three.
 ``--use_cache`` absent keeps the reference's recompute mode (the whole prefix is re-run every
 token, generate.py:146-190) over the same kernels.
 """

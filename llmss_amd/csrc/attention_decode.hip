@@ -1,4 +1,4 @@
-// Paged split-K decode attention for one new token per sequence (SURVEY K11-K14 for S=1;
+// Paged split-K decode attention for one new token per sequence (S=1;
 // reference: eager fp32 QK^T, CPU causal-mask copy, softmax, @V over a torch.cat'd cache,
 // gptj_modeling.py:128-169; MQA baddbmm + TorchScript softmax + bmm,
 // gpt_bigcode_modeling.py:170-246).

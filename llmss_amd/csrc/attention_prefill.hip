@@ -1,4 +1,4 @@
-// Causal variable-length flash-attention forward for prefill on MFMA (SURVEY K11-K14 for
+// Causal variable-length flash-attention forward for prefill on MFMA (for
 // S>1; reference materialises the [S,T] score matrix in fp32 with a CPU-built causal mask,
 // gptj_modeling.py:128-169, gpt_bigcode_modeling.py:170-246).
 //
@@ -412,7 +412,7 @@ void launch_attn_prefill(const void* qkv, int64_t row_stride, int T, const void*
   auto O = (bf16_t*)out;
   const float sl = scale * kLog2eP;
   // v3 by default (profiles/r3_prefill_attn, bench/attn_prefill_bench.py: faster than v1 and v2 on every
-  // measured config); v2 keeps round 2's dispatch (v1 for D = 256 and D = 64 beyond 2K tokens)
+  // measured config); v2 keeps its dispatch (v1 for D = 256 and D = 64 beyond 2K tokens)
   const bool fast = g_prefill_version == 3;
   if (fast || (g_prefill_version == 2 && D != 256 && !(D == 64 && max_seqlen > 2048))) {
     if (row_stride % 8 || k_off % 8 || v_off % 8)

@@ -1,7 +1,7 @@
 // A modelled collective for the simulated TP=N shard (bench.py --simulate-tp N --sim-comm LAT,GBPS,CHANNELS): the
 // stand-in for an RCCL all-reduce that, like RCCL's kernels, occupies CHANNELS workgroups on as many CUs and streams
 // memory - instead of one sleeping workgroup (torch.cuda._sleep), which leaves every other CU and the whole memory
-// system to the compute that the schedules overlap with it ("a model that is too kind"). Each
+// system to the compute that the schedules overlap with it. Each
 // workgroup copies its share of the collective's local memory traffic through a scratch buffer, then holds its CU
 // until the modelled time has passed on the device's constant wall clock; every workgroup reaches the same
 // deadline, so the grid drains by construction.

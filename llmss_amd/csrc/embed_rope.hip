@@ -1,4 +1,4 @@
-// Token/position embedding gather (SURVEY K1/K2) and the fused RoPE + paged-KV-cache write
+// Token/position embedding gather and the fused RoPE + paged-KV-cache write
 // (K8/K10; reference: gptj_modeling.py:26-47,199-236 builds fp32 sin/cos on the CPU, applies a
 // repeat_interleave'd rotate_every_two and torch.cat's the KV cache every step, O(T) per token;
 // gpt_bigcode_modeling.py:288-292 concatenates a [B,T,2D] cache).

@@ -1,4 +1,4 @@
-// Tensor-parallel linear layers on MFMA (SURVEY K4-K7/K15/K16; reference: F.linear -> cuBLAS
+// Tensor-parallel linear layers on MFMA (reference: F.linear -> cuBLAS
 // in FastLinear/TensorParallel{Column,Row}Linear, utils/layers.py:39-179, with bias and
 // activation as separate ATen kernels).
 //
@@ -6,7 +6,7 @@
 //   epilogue: (* w_scale[n]) (+ bias[n]) then act (gelu_tanh | gelu | relu) or SwiGLU
 //   SwiGLU ("silu_glu"): W rows are interleaved in 16-row groups at load time, group 2p = gate
 //   rows [16p, 16p+16), group 2p+1 = up rows [16p, 16p+16); the kernel writes
-//   Y[:, 16p + i] = silu(gate) * up, so the [M, 2F] intermediate never reaches HBM.
+//   Y[:, 16p + i] = silu(gate) * up (or the tanh form of GELU), so the [M, 2F] intermediate never reaches HBM.
 //
 // Kernel family (launch_gemm picks one per call; explicit hints and the autotuned plan table,
 // ops/autotune.py, override the static planner):
@@ -1248,7 +1248,7 @@ __global__ __launch_bounds__(256) void gemm_streamk_kernel(const bf16_t* __restr
 }
 
 // -------------------------------------------------------------------------------------------
-// W8A8 GEMM on the MX-fp8 matrix cores (BASELINE: Llama-2-70B TP=8 fp8, "CDNA4 fp8 MFMA").
+// W8A8 GEMM on the MX-fp8 matrix cores (Llama-2-70B in fp8, TP=8).
 // Y = (Xq . Wq^T) * xs[m] * ws[n] (+ bias, act / SwiGLU): Xq = per-token fp8-e4m3 activations
 // (quant_fp8_rows on X), Wq = per-channel fp8-e4m3 weights. The 16x16x128 f8f6f4 MFMA with unit
 // block scales (E8M0 127) runs at the fp8 peak (2x bf16; the unscaled 16x16x32 fp8 form runs at

@@ -1,4 +1,4 @@
-// Token-level cross-entropy of LM logits (SURVEY K20; reference: CrossEntropyLoss on shifted
+// Token-level cross-entropy of LM logits (reference: CrossEntropyLoss on shifted
 // labels, gptj_modeling.py:612-622 / gpt_bigcode_modeling.py:896-902, an fp32 [B*(S-1), V]
 // log-softmax materialised by ATen).
 //

@@ -1,4 +1,4 @@
-// Fused residual-add + LayerNorm / RMSNorm (SURVEY K3/K17/K22; reference applies
+// Fused residual-add + LayerNorm / RMSNorm (reference applies
 // nn.LayerNorm after a separate residual add, gptj_modeling.py:295-310,
 // gpt_bigcode_modeling.py:366-407; the optional external dropout_add_ln_fwd kernel at
 // utils/layers.py:217-253 is the same fusion, which the reference never calls).

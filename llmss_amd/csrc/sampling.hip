@@ -1,4 +1,4 @@
-// Fused token sampler (SURVEY K18/K19; reference: rank-0-only argmax / softmax+multinomial with
+// Fused token sampler (reference: rank-0-only argmax / softmax+multinomial with
 // HF TopP/TopK/Temperature warpers that are never applied because of an inverted condition,
 // generate.py:109-126, consumer_server.py:130-147 - quirk Q1; here the documented intent is
 // implemented: temperature -> top-k -> top-p -> sample).
@@ -588,7 +588,7 @@ __global__ __launch_bounds__(CAND_THREADS) void cand_topk_kernel(const bf16_t* _
   }
   __syncthreads();
   if (nout > KC) {
-    // more than KC keys tie at the boundary (ADVICE r2): the atomic slot order above kept an arbitrary subset
+    // more than KC keys tie at the boundary: the atomic slot order above kept an arbitrary subset
     // of the ties, which could drop the lowest-index one that greedy / top-k tie-breaking needs. Rewrite the
     // row deterministically: every key above the boundary (fewer than K <= KC of them), then the ties in
     // ascending vocabulary index (a ballot rank per wave + wave offsets, in (e, t) = index order).

@@ -197,7 +197,7 @@ class LLMEngine:
         if self.tp.is_real and self.tp.host_staged:  # gloo-staged device collectives cannot be captured
             self.use_graphs = False
         self.graphs: Dict[tuple, torch.cuda.CUDAGraph] = {}  # (batch bucket, candidate sampler) -> graph
-        # vocab-parallel sampling from per-rank candidates (SURVEY R11 "better"): greedy / top-k <= 64 rows
+        # vocab-parallel sampling from per-rank candidates: greedy / top-k <= 64 rows
         # gather [B, tp, 128] (value, id) pairs instead of [B, V] logits
         from ..ops.hip import CAND_KC, CAND_MAX_SHARD
 
@@ -372,7 +372,7 @@ class LLMEngine:
         communicator, LLMSS_TP_RSAG=auto (default), buckets divisible by the TP degree of at least
         8 rows per rank. Not for fp8-weight models: their default schedule feeds the
         GEMMs the fp8 twin that add_norm writes, which the row-sharded add + norm does not produce, so the A/B would
-        not compare like with like (ADVICE round 4)."""
+        not compare like with like."""
         m = self.model
         if not (self.is_gpu and self.tp.is_real and not self.tp.host_staged and m.rsag_mode == "auto"):
             return []
@@ -889,7 +889,7 @@ class LLMEngine:
     def _ab_buckets(cands: List[int]) -> List[int]:
         """The buckets the schedule A/B times: the largest candidate, the largest one at most half of it and the
         smallest one; every other candidate bucket adopts the winner of the nearest timed bucket (engine start-up at
-        TP=8: 3 timed buckets instead of up to 15, VERDICT r5 item 6)."""
+        TP=8: 3 timed buckets instead of up to 15)."""
         cands = sorted(cands)
         if not cands:
             return []

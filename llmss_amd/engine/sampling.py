@@ -1,7 +1,7 @@
 """Per-request sampling parameters (mirrors the reference CLI/HTTP fields, generate.py:21-40,
 producer_server.py:9-15) plus the deterministic per-step seed used identically on every rank.
 
-Filter order (SURVEY Q1). The reference builds HF warpers in the order TopP -> TopK -> Temperature
+Filter order. The reference builds HF warpers in the order TopP -> TopK -> Temperature
 (generate.py:111-119) but then inverts its own test (``if not list_of_warpers``), so the warpers
 are never applied: its effective sampler is plain multinomial sampling from softmax(logits) at
 temperature 1 whatever the flags say. Here the flags are honoured in the order HF ``generate()``

@@ -950,7 +950,7 @@ def _rope_theta(d: Dict[str, Any]) -> float:
 
 
 # -------------------------------------------------------------------- presets
-# Public HF architectures (SURVEY.md §7.5) used for random-init benches and smoke tests.
+# Public HF architectures used for random-init benches and smoke tests.
 _PRESETS: Dict[str, Dict[str, Any]] = {
     "gpt2": dict(model_type="gpt2", n_embd=768, n_layer=12, n_head=12, n_positions=1024, vocab_size=50257),
     "gpt2-medium": dict(model_type="gpt2", n_embd=1024, n_layer=24, n_head=16, n_positions=1024, vocab_size=50257),

@@ -164,7 +164,7 @@ class TensorParallelEmbedding(nn.Module):
         self.reduce = reduce
         full = weights.get_tensor(f"{prefix}.weight")
         V = full.shape[0]
-        block = -(-V // pg.size())  # every id has an owner, also when V % tp != 0 (reference quirk Q6)
+        block = -(-V // pg.size())  # every id has an owner, also when V % tp != 0 (a quirk of the reference)
         self.min_id = pg.rank() * block
         self.max_id = min(V, self.min_id + block)
         self.weight = nn.Parameter(full, requires_grad=False)  # replicated: lookups need no all-reduce

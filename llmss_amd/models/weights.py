@@ -4,16 +4,16 @@ One layout serves every family (the decoder in ``decoder.py`` is family-agnostic
 
 * ``qkv_w``  [nh_l*D + 2*nkv_l*D, H]  column-parallel, q|k|v fused at load time
   (reference loads separate q/k/v for GPT-J, ``gptj_modeling.py:84-92``, and for BigCode loads
-  the FULL c_attn on every rank then slices, ``gpt_bigcode_modeling.py:122-155`` - quirk Q8).
+  the FULL c_attn on every rank then slices, ``gpt_bigcode_modeling.py:122-155``).
 * ``o_w``    [H, nh_l*D]  row-parallel; its bias lives on rank 0 only (``layers.py:161-173``).
 * ``up_w``   [F_l, H] or, for SwiGLU, [2*F_l, H] with gate/up interleaved in 16-row groups so
   the GEMM epilogue emits silu(gate)*up directly.
 * ``down_w`` [H, F_l] row-parallel (bias on rank 0).
 * ``wte``    full table replicated on every rank (no embedding all-reduce; reference C1).
 * ``head_w`` [Vp/tp, H] vocab-parallel with the vocab padded to a multiple of 16*tp (fixes the
-  reference's silent loss of ids >= tp*floor(V/tp), quirk Q6); GPT-J's lm_head bias is loaded
-  (the reference drops it, quirk Q5). Tied heads (GPT-2, BigCode) share the checkpoint tensor
-  (read once per rank; the reference loads wte twice, Q9).
+  reference's silent loss of ids >= tp*floor(V/tp)); GPT-J's lm_head bias is loaded
+  (the reference drops it). Tied heads (GPT-2, BigCode) share the checkpoint tensor
+  (read once per rank; the reference loads wte twice).
 
 KV heads: sharded when nkv >= tp, otherwise each rank keeps exactly the kv head(s) its query
 heads use (MQA: every rank holds the single kv head), generalising the reference's MQA
@@ -437,7 +437,7 @@ def load_hf_weights(cfg: ModelConfig, reader, tp: int = 1, rank: int = 0, device
 
 
 # ------------------------------------------------------------------------------ per-rank shard cache
-# a restart of a large TP deployment should not re-read, re-shard, re-interleave and
+# A restart of a large TP deployment should not re-read, re-shard, re-interleave and
 # re-quantize the HF checkpoint on every rank. The finished per-rank weights (this rank's shards,
 # padded head, SwiGLU interleave, fp8 + scales) are written once as one safetensors file per rank
 # and mmap-loaded by the native reader afterwards.

@@ -83,7 +83,8 @@ def attn_extend(q, k_cache, v_cache, block_tables, cu_q, ctx_lens, max_qlen, nh,
 
 
 def linear(x, w, bias=None, act="none", glu=False, w_scale: Optional[torch.Tensor] = None, partial_ok=False):
-    """partial_ok: on GPU the result may be a split-K PartialSum that only add_norm consumes."""
+    """partial_ok: on GPU the result may be a split-K PartialSum that only add_norm consumes. ``glu``: gate times up, the gate SiLU or,
+    with ``act`` "gelu_tanh", the tanh form of GELU."""
     if x.is_cuda:
         return _hip().linear(x, w, bias, act, glu, w_scale, partial_ok=partial_ok)
     return ref.linear(x, w, bias, act, glu, w_scale)

@@ -506,7 +506,7 @@ def _w8a8_mid_plan(M, N, K, glu):
 
 
 def mx_mlp_ok(M: int, up, down) -> bool:
-    """The gate/up SwiGLU GEMM can write its output as MX-fp8 for the down projection (VERDICT r5 missing #4: no bf16
+    """The gate/up SwiGLU GEMM can write its output as MX-fp8 for the down projection (no bf16
     intermediate, no per-token quantisation launch): both run tuned W8A8 gemm_mid plans at M rows, the gate/up plan is
     unsplit with whole 32-output blocks per tile (BN % 64 == 0)."""
     if up.w_scale is None or down.w_scale is None or not up.glu or up.N % 128 or down.K % 128 or up.N // 2 != down.K:

@@ -7,7 +7,7 @@ and ``FakeGroup`` (``dist.py:14-37``). Differences, by design:
   same code runs on one node or several.
 * ``world_size == 1`` is a first-class case: :class:`TPGroup` with ``size == 1`` turns every
   collective into the identity and *never* needs a default process group (the reference's
-  single-GPU ``generate.py`` crashes on an un-grouped ``dist.broadcast`` — SURVEY Q2).
+  single-GPU ``generate.py`` crashes on an un-grouped ``dist.broadcast``).
 * On GPUs the data plane is a native RCCL communicator (``llmss_amd._C.RcclComm``, csrc/comm.cpp)
   bootstrapped over a CPU (gloo) process group: collectives are raw ``ncclAllReduce`` /
   ``ncclAllGather`` calls on the caller's current HIP stream, so they are captured into the decode
@@ -517,7 +517,7 @@ def _check_all_reduce(comm, tp: int, rank: int):
 def _tune_native_comm(comm, rank: int, tp: int, nbytes: int, group=None, make_comm=None):
     """Start-up probe of the RCCL protocol / algorithm for the decode all-reduce (``nbytes``, the bench's 64
     sequences per GPU x hidden 4096 x bf16 at TP=8 = 4 MiB by default, LLMSS_RCCL_TUNE_BYTES). Opt-in
-    (``LLMSS_RCCL_TUNE=1``) until it has run on a multi-GPU node (ADVICE round 4). Every candidate of
+    (``LLMSS_RCCL_TUNE=1``) until it has run on a multi-GPU node. Every candidate of
     RCCL_CANDIDATES gets a communicator built under its environment (bounded init), must sum correctly on a
     fresh buffer, and has its graph-replayed all-reduce timed on every rank; each of these steps is agreed over
     gloo, so a step that fails on one rank drops the candidate on all of them (no rank leaves the probe's
@@ -746,14 +746,14 @@ def initialize_torch_distributed():
     ``generate.py:62`` - after :func:`initialize_distributed` has set up the native data plane, which
     ``as_tp_group(process_group)`` (and so ``Weights`` / ``MODEL_REGISTRY``) picks up again. Unlike the reference
     the default process group exists at ``world_size == 1`` too when torch.distributed is used at all later
-    (un-grouped ``dist.broadcast`` in the reference's single-GPU generate.py raises, SURVEY Q2): here callers get
+    (un-grouped ``dist.broadcast`` in the reference's single-GPU generate.py raises): here callers get
     a FakeGroup and no default group, exactly like the reference, so use the returned group."""
     tp, rank, world_size = initialize_distributed()
     if world_size == 1 or tp.fake:
         return FakeGroup(rank, world_size), rank, world_size
     if tp.dp > 1:
         # data-parallel replicas (LLMSS_DP): this rank's replica, not the world, is the tensor-parallel group -
-        # its CPU control group stands in for the process group (ADVICE round 4: WORLD would shard the model
+        # its CPU control group stands in for the process group (WORLD would shard the model
         # over every replica's ranks)
         if tp.size == 1:
             return FakeGroup(0, 1), rank, world_size

@@ -10,7 +10,7 @@ requests / aborts over a dedicated gloo (CPU/TCP) group, and all ranks then run 
 tokens, no token broadcast). When there is no work the leader blocks on its inbox and followers
 block in a CPU receive - nothing spins on the GPU.
 
-Failure handling (SURVEY 5.3; the reference has none beyond the 60 s NCCL timeout):
+Failure handling (the reference has none beyond the 60 s NCCL timeout):
 * leader heartbeat: an idle leader still broadcasts a heartbeat every ``heartbeat_s``; followers
   wait on the control group with ``leader_timeout_s``, so a lost leader ends them cleanly instead
   of hanging in a collective forever.

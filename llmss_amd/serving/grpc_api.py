@@ -1,5 +1,5 @@
 """gRPC ``llmss.Generate`` service (``proto/generate.proto``). The reference advertises gRPC in its
-README tagline (README.md:2) but ships none; this is new API surface (BASELINE north star).
+README tagline (README.md:2) but ships none; this is new API surface.
 
 ``grpc_tools``/``protoc`` are not available, so the message classes are built at import time from
 a ``FileDescriptorProto`` that mirrors ``proto/generate.proto`` field for field, and the service
@@ -120,7 +120,7 @@ class AioServer:
     The loop's one task, ``main``, owns the server's whole life: it starts the server, waits for either a stop
     request or the server terminating on its own, runs ``server.stop(grace)`` ITSELF, and only then returns -
     after which every task still pending on the loop (servicer coroutines of cancelled calls) is cancelled and
-    drained and the loop is closed. Root cause of round 4's "loop ended early" (profiles/r4_serving): ``stop()``
+    drained and the loop is closed. What "loop ended early" came from once (profiles/r4_serving): ``stop()``
     used to schedule ``server.stop()`` onto the loop from another thread while ``main`` awaited
     ``wait_for_termination()``. The server signals termination part-way through its own ``stop()``, so ``main``
     returned, ``run_until_complete`` stopped the loop, and the scheduled stop coroutine was left unfinished

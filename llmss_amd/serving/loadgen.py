@@ -1,6 +1,6 @@
 """Closed-batch gRPC load generator (client process of ``bench.py``'s served configuration).
 
-BASELINE config #2 is "GPT-2-XL TP=1 bf16 on one MI355X served over gRPC" - the reference serves its
+The workload is GPT-2-XL, TP=1, bf16 on one MI355X, served over gRPC - the reference serves its
 model over HTTP -> Redis -> consumer (``poc-server/producer-consumer/producer_server.py:45-55``) and has
 no gRPC. ``bench.py`` runs the engine behind the in-process gRPC ``Generate`` service and this process
 acts as the clients: it is started before the bench touches the GPU, learns the server port on stdin,

@@ -1,4 +1,4 @@
-"""Data-parallel replicas behind one front-end (SURVEY 2.4 "DP replicas", optional).
+"""Data-parallel replicas behind one front-end (optional).
 
 Reference: none - its consumer notes that several subscribers *could* pop the same ``pqueue``
 (consumer_server.py:68-72), but replies go to one shared, uncorrelated ``squeue``

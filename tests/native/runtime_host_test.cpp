@@ -1,5 +1,5 @@
 // Host-only test of the native runtime (csrc/runtime.cpp without its Python bindings), built and run
-// under AddressSanitizer + UndefinedBehaviorSanitizer by tests/test_native_asan.py (SURVEY 5.2).
+// under AddressSanitizer + UndefinedBehaviorSanitizer by tests/test_native_asan.py.
 // Exercises the KV block allocator, the continuous-batching scheduler (admission, decode, block
 // growth, preemption by recompute, finish/abort) and the safetensors reader (row / column shard
 // copies, multi-threaded, malformed headers rejected).

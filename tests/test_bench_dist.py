@@ -69,7 +69,7 @@ _TINY = ["--model", "tiny-llama", "--secondary", "none", "--batch-per-gpu", "2",
 
 def test_bench_self_launches_ranks():
     """`python bench.py --gpus 2` without torchrun: the process becomes a launcher for 2 ranks and forwards
-    rank 0's single JSON line (VERDICT r2 item 1)."""
+    rank 0's single JSON line."""
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2", "--steps", "2", "--warmup", "1"]
                        + _TINY, env=_cpu_env(), capture_output=True, text=True, timeout=300, cwd=ROOT)
     assert r.returncode == 0, r.stderr[-3000:]

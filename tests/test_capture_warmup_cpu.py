@@ -1,4 +1,4 @@
-"""Every collective a captured decode graph issues was issued eagerly before the capture (VERDICT r5 item 6): a
+"""Every collective a captured decode graph issues was issued eagerly before the capture: a
 native RCCL communicator sets up each algorithm's peer connections lazily on first use, which must never happen
 inside a HIP graph capture. The engine warms every (bucket, sampler mode) eagerly before capture_graphs captures it,
 and every A/B schedule (tbo / rsag / col) once per bucket with the first sampler mode before its captures. This CPU

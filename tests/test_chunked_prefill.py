@@ -1,4 +1,4 @@
-"""Chunked prefill and mixed prefill+decode steps (SURVEY 5.7): a prompt cut into chunks that attend
+"""Chunked prefill and mixed prefill+decode steps: a prompt cut into chunks that attend
 their cached prefix through the paged cache, decodes riding along with prompt chunks, and requests
 arriving while others decode must give exactly the tokens of whole-prompt prefill (fp32 on CPU).
 

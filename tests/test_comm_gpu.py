@@ -169,7 +169,7 @@ def _graph_node_types(g):
 
 
 def test_captured_collectives_are_graph_nodes(comm):
-    """'capture succeeded' is not the check. Out-of-place all-gather / all-reduce /
+    """'Capture succeeded' is not the check. Out-of-place all-gather / all-reduce /
     reduce-scatter on the native communicator captured into one graph leave one node each (a one-rank
     collective is a device copy: memcpy or kernel nodes, never an empty graph), and the replay moves the
     CURRENT inputs."""
@@ -244,7 +244,7 @@ def test_rccl_setting_probe_one_rank(monkeypatch):
 
 
 def test_rccl_init_deadline_without_peer():
-    """Bounded communicator init (csrc/comm.cpp, VERDICT round 4 item 5): a 2-rank communicator whose second rank
+    """Bounded communicator init (csrc/comm.cpp): a 2-rank communicator whose second rank
     never arrives raises at the deadline (non-blocking ncclCommInitRankConfig polled, then ncclCommAbort) instead
     of blocking forever; a 1-rank communicator still initialises and reports its set-up time."""
     import time
@@ -266,7 +266,7 @@ def test_rccl_init_deadline_without_peer():
 
 
 def test_col_schedule_ab_at_capture(comm, monkeypatch):
-    """the column-chunked decode schedule (DecoderLM._reduce_cols: each row-parallel output
+    """The column-chunked decode schedule (DecoderLM._reduce_cols: each row-parallel output
     as weight-row slices whose all-reduces run on the comm stream beside the next slice's GEMM) is a fourth
     capture-time A/B candidate on a native-comm TP group: both timings recorded, one graph kept per bucket, and
     what it keeps decodes exactly like eager (one-rank stand-in for TP=2, as the micro-batch A/B test)."""

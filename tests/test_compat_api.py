@@ -1,5 +1,5 @@
 """Reference API compatibility: MODEL_REGISTRY façade (HF-style forward with past_key_values) and the
-generate.py CLI (same flags, same three stdout lines), on CPU at TP=1 (BASELINE config #1 plumbing)."""
+generate.py CLI (same flags, same three stdout lines), on CPU at TP=1."""
 import subprocess
 import sys
 

@@ -98,7 +98,7 @@ def test_gpu_sharded_candidates_one_gpu(shards, V, Vp):
 @pytest.mark.gpu
 @pytest.mark.parametrize("tp", [2, 8])
 def test_gpu_candidates_tie_mass_above_kc(tp):
-    """more than KC = 128 logits of a shard tie at the top-k boundary. The candidate kernel keeps the
+    """More than KC = 128 logits of a shard tie at the top-k boundary. The candidate kernel keeps the
     lowest-index ties (the same set every run), so greedy rows - lowest index among the maxima - equal the
     full-row v3 sampler. Sampled rows keep every boundary tie in v3 (x >= k-th value) but at most KC per shard
     here: they draw a token from the kept top set, not necessarily v3's (a documented limit of carrying KC

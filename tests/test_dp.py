@@ -1,4 +1,4 @@
-"""Data-parallel replicas (SURVEY 2.4, optional): an in-process Router over independent engines
+"""Data-parallel replicas (optional): an in-process Router over independent engines
 (least-loaded dispatch, request ids unique across replicas, results identical to one engine) and a
 torchrun-style world split into dp x tp groups (dp=2 x tp=2 over gloo: each replica's sharded engine
 reproduces TP=1)."""

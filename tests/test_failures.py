@@ -1,4 +1,4 @@
-"""Failure detection in the serving driver (SURVEY 5.3): server-side deadlines, a follower that
+"""Failure detection in the serving driver: server-side deadlines, a follower that
 dies mid-generation (every in-flight request must fail, not hang), a leader that disappears
 (followers must notice through the heartbeat timeout), and the fault-injection hook."""
 import os
@@ -184,7 +184,7 @@ def _init_worker(rank, port, root, q):
 
 
 def test_rccl_init_bounded_when_a_peer_never_joins(tmp_path):
-    """rank 1 passes the pre-init agreement and then never joins the communicator init
+    """Rank 1 passes the pre-init agreement and then never joins the communicator init
     (fault-injected, as a peer that died). Rank 0's bounded init raises at its deadline instead of blocking, and
     both ranks then agree on the failure over gloo (the native deadline itself: tests/test_comm_gpu.py)."""
     s = socket.socket()

@@ -139,7 +139,7 @@ def _to(obj, dev):
 
 
 def test_fp8_w8a8_prefill_and_decode_vs_fake_quant_oracle(tmp_path, monkeypatch):
-    """the W8A8 path end to end (per-token e4m3 activations on the MX-fp8 matrix cores), not W8A16.
+    """The W8A8 path end to end (per-token e4m3 activations on the MX-fp8 matrix cores), not W8A16.
     Prefill: 153 prompt tokens, so every fp8 GEMM runs W8A8 (untuned calls above 128 rows), its activations quantised
     by add_norm's fp8 twin (qkv, up) or the quantisation kernel (o, down). Decode: 4 rows with W8A8 plans forced into
     the tuned table for every fp8 shape. Oracle: the same quantised weights in the CPU reference model with every fp8
@@ -249,7 +249,7 @@ def test_fp8_w8a8_prefill_and_decode_vs_fake_quant_oracle(tmp_path, monkeypatch)
 
 
 def test_fp8_mlp_mx_handoff_vs_fake_quant_oracle(tmp_path, monkeypatch):
-    """VERDICT r5 missing #4 at model level: with W8A8 gemm_mid plans for every fp8 GEMM (forced into the tuned table,
+    """At model level: with W8A8 gemm_mid plans for every fp8 GEMM (forced into the tuned table,
     prefill 153 rows and decode 4 rows), DecoderLM._mlp has the gate/up epilogue write its SwiGLU output as MX-fp8 and
     the down projection consume it - no bf16 intermediate, no quantisation launch. Oracle: the CPU reference with
     per-token fake-quant activations for qkv / o / gate-up and MX fake-quant (ops/reference.py fake_quant_mx_act) for

@@ -833,7 +833,7 @@ def test_quant_fp8_activation_rows(K):
 
 @pytest.mark.parametrize("M", [64, 256, 512])
 def test_w8a8_decode_plan_in_graph(M):
-    """a tuned W8A8 plan (fp8 activations quantised into the reusable scratch, MX-fp8
+    """A tuned W8A8 plan (fp8 activations quantised into the reusable scratch, MX-fp8
     MFMA) runs inside a captured HIP graph and replays exactly the eager values; both match fp32 math on
     the same fp8 operands. The plan goes through the tuned table exactly as a decode step consults it."""
     from llmss_amd import _native
@@ -921,7 +921,7 @@ def test_gemm_w8a8_mid_tiles(tile, depth, split, M, N, K):
 @pytest.mark.parametrize("up_tile", [8, 11, 10, 13, 9, 12])
 @pytest.mark.parametrize("M,F,K", [(512, 1024, 2048), (129, 512, 1024), (64, 256, 1024)])
 def test_w8a8_swiglu_mx_output_feeds_the_down_projection(up_tile, M, F, K):
-    """a W8A8 SwiGLU GEMM writes its output as MX-fp8 (e4m3 + one e8m0 scale per 32 outputs)
+    """A W8A8 SwiGLU GEMM writes its output as MX-fp8 (e4m3 + one e8m0 scale per 32 outputs)
     and the down projection consumes it on the MX-fp8 MFMA with per-lane block scales, so no bf16 intermediate and no
     quantisation launch sit between them.
     * producer: bit-identical to the CPU MX quantisation (ops/reference.py quant_mx_fp8) of the same kernel's bf16

@@ -1,4 +1,4 @@
-"""LM cross-entropy kernel (SURVEY K20, csrc/loss.hip) against torch's fp32 CrossEntropyLoss, and the
+"""LM cross-entropy kernel (csrc/loss.hip) against torch's fp32 CrossEntropyLoss, and the
 façade's ``labels=`` loss on the GPU."""
 import pytest
 import torch

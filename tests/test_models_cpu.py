@@ -105,7 +105,7 @@ def test_random_weights_shapes():
 
 @pytest.mark.parametrize("name", ["llama", "gpt2", "gptj"])
 def test_shard_cache_roundtrip(tmp_path, name):
-    """Per-rank shard cache (SURVEY 5.4): the second build mmaps the cached shard, same logits."""
+    """Per-rank shard cache: the second build mmaps the cached shard, same logits."""
     from llmss_amd.engine import build_model
     from llmss_amd.models.decoder import StepInput
 

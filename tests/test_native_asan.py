@@ -1,6 +1,6 @@
 """The native host runtime (csrc/runtime.cpp: block allocator, scheduler, safetensors reader)
 compiled alone under AddressSanitizer + UndefinedBehaviorSanitizer and driven by a C++ test
-(tests/native/runtime_host_test.cpp) - SURVEY 5.2's host-code sanitizer run. CPU only."""
+(tests/native/runtime_host_test.cpp) - the sanitizer run of the host code. CPU only."""
 import os
 import shutil
 import subprocess

@@ -108,7 +108,7 @@ def test_reference_generate_sequence_world1_and_world2(tmp_path, monkeypatch):
 def test_reference_generate_sequence_dp2(tmp_path):
     """World 4 with two data-parallel replicas (LLMSS_DP=2): initialize_torch_distributed hands each rank its
     replica's group (TP=2), not the world, so Weights / MODEL_REGISTRY shard over 2 ranks and every replica
-    computes the world-1 logits (ADVICE round 4)."""
+    computes the world-1 logits."""
     d = str(tmp_path / "llama")
     save_hf_model("llama", d, vocab=101)
     prompt = torch.randint(0, 100, (2, 7))

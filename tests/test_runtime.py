@@ -182,7 +182,7 @@ def _drive(s, max_steps=500):
 
 @pytest.mark.parametrize("chunk", [8, 0])
 def test_scheduler_chunked_prefill_pool_exhaustion(native, chunk):
-    """concurrent chunked prompts that together hold the whole KV pool while nothing
+    """Concurrent chunked prompts that together hold the whole KV pool while nothing
     decodes used to make every later schedule() idle forever. Now the newest is preempted."""
     s = native.Scheduler(num_blocks=8, block_size=4, max_num_seqs=4, max_batched_tokens=16, max_model_len=64,
                          prefill_chunk=chunk)

@@ -224,7 +224,7 @@ def test_grpc_direct_and_broker(driver):
 
 
 def test_broker_grpc_stream_streams_tokens(driver):
-    """VERDICT r2 missing 5: GenerateStream on the pub/sub path yields the tokens as the engine samples them
+    """GenerateStream on the pub/sub path yields the tokens as the engine samples them
     (one broker message per engine step), not one message after the whole reply."""
     drv, tok, m = driver
     b = MemoryBroker()
@@ -243,7 +243,7 @@ def test_broker_grpc_stream_streams_tokens(driver):
 
 
 def test_durable_queue_requeues_after_consumer_crash(driver):
-    """a request popped by a consumer that then died stays in its processing list; a
+    """A request popped by a consumer that then died stays in its processing list; a
     consumer restarted with the same id re-queues and serves it, and acknowledges every reply."""
     from llmss_amd.serving.consumer import processing_key
 
@@ -267,7 +267,7 @@ def test_durable_queue_requeues_after_consumer_crash(driver):
 
 
 def test_durable_intake_recovers_requests_of_a_failed_batch_pop(driver):
-    """the connection drops after the server ran part of the intake's batch pop. The requests those pops
+    """The connection drops after the server ran part of the intake's batch pop. The requests those pops
     moved into the processing list are resubmitted at once (no restart needed), none is served twice, every one is
     answered and acknowledged."""
     from llmss_amd.serving.consumer import processing_key
@@ -580,7 +580,7 @@ def test_aio_server_stop_after_its_loop_ended(driver):
 
 
 def test_aio_server_stop_completes_on_its_own_loop(driver):
-    """Root cause of round 4's stuck stop (profiles/r4_serving): the server signals termination part-way through
+    """What a stuck stop came from once (profiles/r4_serving): the server signals termination part-way through
     its own stop(), so a stop coroutine scheduled from outside raced the loop's exit and never finished. Now the
     loop's main task runs server.stop(grace) itself: with streams in flight, stop().wait() returns, the stop ran
     to the end (stop_completed), the streams end, pending servicer tasks are drained, the loop is closed and the
