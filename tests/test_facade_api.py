@@ -127,7 +127,8 @@ def _layers_worker(rank, port, d, q):
     ids = torch.tensor([[1, 50, 100]])
     out = _layers_forward(w, d, x, ids)
     if rank == 0:
-        q.put(out)
+        # by value: a tensor's storage would be fetched from this process, which may be gone
+        q.put([t.detach().numpy() if torch.is_tensor(t) else t for t in out])
     torch.distributed.barrier()
     torch.distributed.destroy_process_group()
 
@@ -159,7 +160,7 @@ def test_tp_layer_library_tp2_matches_tp1(tmp_path):
     for p in procs:
         p.start()
     try:
-        got = q.get(timeout=240)
+        got = [a if isinstance(a, torch.Size) else torch.from_numpy(a) for a in q.get(timeout=240)]
         for p in procs:
             p.join(60)
     finally:
@@ -174,7 +175,7 @@ def test_tp_layer_library_tp2_matches_tp1(tmp_path):
 
 
 def test_pool_exhaustion_leaves_pool_intact(tmp_path):
-    """a call that cannot get its KV blocks raises without leaking the blocks of earlier rows."""
+    """A call that cannot get its KV blocks raises without leaking the blocks of earlier rows."""
     d = str(tmp_path / "llama")
     save_hf_model("llama", d)
     model, _ = _load(d)
