@@ -1849,9 +1849,10 @@ static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int
 // 0.8 full only 0.78 of it (0.6 - 0.94 over eleven shapes: the clock rises as tiles end); up to 64 rows left over read all weights at
 // 4.5 TB/s behind 8 us. us, one launch and two: 1773 x 12288 x 4096 172 -> 151 (predicted 174 and 155), SwiGLU x 22016 280 -> 266,
 // 8261 x 2048 x 2048 91 -> 61, 8261 x 6400 x 2048 190 -> 174, 3999 x 22016 x 4096 570 -> 551. Left whole, as predicted: 8192 x 5120 x 2048
-// (2.5 waves) 141 and 143, 8192 x 9472 x 2048 (4.6) 255 and 255, 5000 x 12288 x 4096 (3.75) 359 and 357. Over 4840 random products that it
-// cuts, 257 - 10000 rows: 0.91 of the time from K = 1024 on, 1.11 at worst, and 1.00 - 1.005 at the 95th percentile; below, where a tile's
-// start and end are half of it, 0.98 and 1.2 at worst, so those stay whole.
+// (2.5 waves) 141 and 143, 8192 x 9472 x 2048 (4.6) 255 and 255, 5000 x 12288 x 4096 (3.75) 359 and 357. Over 3286 random products that it
+// cuts, 257 - 10000 rows and whole steps of k, two launches take 0.886 of the time from K = 1024 on, 1.11 at worst. Below, a tile's start and end
+// are half of it, and what is promised up to there does not come: gated products 0.87 (0.98 at worst), others 0.954 where more than 6.5 % are
+// promised (95 products; 1.15 at worst, all of those at 6.5 - 10 %: 3764 x 5664 x 256 27 -> 31), 1.02 where less, so those stay whole.
 struct GemmCut {
   int rows, cols;  // of the first launch; 0: not cut
   int hint;        // plan of the second (0: the plan of its size)
@@ -1865,8 +1866,7 @@ static GemmCut gemm_cut(int M, int N, int K, bool glu) {
     return std::max(t, (2.0 * n * K + 2.0 * m * K + 2.0 * m * (glu ? n / 2 : n)) / 4.0e6);
   };
   GemmCut cut{0, 0, 0};
-  if (K < 1024) return cut;
-  double best = 0.97 * tiles_us(kTileCost[0], M, N);
+  double best = (K < 1024 && !glu ? 0.935 : 0.97) * tiles_us(kTileCost[0], M, N);
   auto consider = [&](int rows, int cols) {
     if (rows <= 0 || cols <= 0 || (rows >= M && cols >= N)) return;
     const int last = (rows < M ? rows / 256 * ntn : ntm * (cols / 256)) % 256;

@@ -125,7 +125,8 @@ def test_fp8_products_of_few_rows_take_the_decode_kernel(M, N, K, glu, slabs, de
 
 @pytest.mark.parametrize("M,N,K,glu,cut", [(8192, 12288, 4096, False, None), (8192, 5120, 2048, False, None), (5000, 12288, 4096, False, None),
                                            (8261, 2048, 2048, False, "rows"), (1773, 12288, 4096, False, "any"), (3999, 22016, 4096, True, "any"),
-                                           (2500, 6144, 2048, False, None), (3764, 5664, 256, False, None), (1017, 21472, 512, False, None)])
+                                           (2500, 6144, 2048, False, None), (9999, 10160, 256, False, None), (6783, 10256, 384, False, None),
+                                           (1649, 11200, 512, True, "any"), (8261, 2048, 512, False, "rows")])
 def test_products_are_cut_where_the_last_wave_of_tiles_is_nearly_empty(M, N, K, glu, cut):
     """Whole waves of 256 x 256 tiles in one launch and the rest in another: never for products that fill their waves, at multiples
     of a tile, by rows or by columns but not both."""
