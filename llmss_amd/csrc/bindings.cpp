@@ -96,7 +96,9 @@ bool moe_pp_glu_ok(int64_t ldh, int maxt, int top, int F, int K);
 void launch_moe_pp_glu(const void* h, int64_t ldh, const void* Wg, const void* Wu, const void* meta, const void* order, void* act,
                        int E, int maxt, int top, int F, int K, float limit, float alpha, const void* pw, int silu, hipStream_t st);
 void launch_moe_dec(int mode, const void* X, int64_t ldx, const void* W, const void* W2, const void* meta, const void* order, void* C,
-                    int E, int maxt, int top, int N, int K, float limit, float alpha, const void* pw, int silu, hipStream_t st);
+                    int E, int maxt, int top, int N, int K, float limit, float alpha, const void* pw, int silu, const void* idx,
+                    void* place, int T, const void* sX, const void* sW, void* sC, void* sD, int64_t sldd, int sN, int sK, int sE,
+                    int sinter, float slimit, hipStream_t st);
 void launch_moe_down_tile(const void* act, const void* wd, const void* meta, void* y, int E, int maxt, int N, int F,
                           int tile_rows, hipStream_t st);
 void launch_latent_norm_cache(const void* src, int64_t ld, int off, const void* w, float eps, void* cache,
@@ -445,8 +447,11 @@ PYBIND11_MODULE(_C, m) {
     launch_moe_pp_glu(CP(h), ldh, CP(Wg), CP(Wu), CP(meta), CP(order), P(act), E, maxt, top, F, K, limit, alpha, CP(pw), silu, S(st));
   });
   m.def("moe_dec", [](int mode, uintptr_t X, int64_t ldx, uintptr_t W, uintptr_t W2, uintptr_t meta, uintptr_t order, uintptr_t C,
-                      int E, int maxt, int top, int N, int K, float limit, float alpha, uintptr_t pw, int silu, uintptr_t st) {
-    launch_moe_dec(mode, CP(X), ldx, CP(W), CP(W2), CP(meta), CP(order), P(C), E, maxt, top, N, K, limit, alpha, CP(pw), silu, S(st));
+                      int E, int maxt, int top, int N, int K, float limit, float alpha, uintptr_t pw, int silu, uintptr_t idx,
+                      uintptr_t place, int T, uintptr_t sX, uintptr_t sW, uintptr_t sC, uintptr_t sD, int64_t sldd, int sN, int sK,
+                      int sE, int sinter, float slimit, uintptr_t st) {
+    launch_moe_dec(mode, CP(X), ldx, CP(W), CP(W2), CP(meta), CP(order), P(C), E, maxt, top, N, K, limit, alpha, CP(pw), silu, CP(idx),
+                   P(place), T, CP(sX), CP(sW), P(sC), P(sD), sldd, sN, sK, sE, sinter, slimit, S(st));
   });
   m.def("moe_down_tile", [](uintptr_t act, uintptr_t wd, uintptr_t meta, uintptr_t y, int E, int maxt, int N, int F,
                             int tile_rows, uintptr_t st) {

@@ -177,19 +177,18 @@ class MoEFeedForward:
                 sh = ops.linear_f(ops.linear_f(h, W.shared_gu, dt, act="gelu"), W.shared_down, dt)
             return ops.moe_experts(h, idx, wts, None, W.up, W.down, 0.0, 0.0, shared=sh, combine=False, act="gelu",
                                    identity=spec.identity > 0)
-        if W.shared_interleaved:
-            sh = ops.linear_f(ops.linear(h, W.shared_gu, None, "none", True), W.shared_down, dt)
-        elif W.shared_gu is not None:
-            # (a sandwich block's gate logits ride in this GEMM as extra columns: model.proj)
-            gu = model.proj = ops.linear_f(h, W.shared_gu, dt)
-            if spec.shared is not None:
-                a = ops.glu_act(gu, spec.shared.ff, "silu") if spec.act == "silu" else \
-                    ops.glu_clamp(gu, spec.shared.ff, spec.shared.limit, GLU_ALPHA)
-                sh = ops.linear_f(a, W.shared_down, dt)
         # combine=False: on the GPU the weighted sum over the chosen experts happens inside the next residual add
-        return ops.moe_experts(h, idx, wts, W.gate, W.up, W.down, spec.expert.limit, GLU_ALPHA, shared=sh,
-                               combine=False, act=spec.act, weight_input=spec.weight_input,
-                               shared_w=route[2] if spec.shared_gate else None, interleaved=W.interleaved)
+        kw = dict(combine=False, act=spec.act, weight_input=spec.weight_input, shared_w=route[2] if spec.shared_gate else None,
+                  interleaved=W.interleaved)
+        # (a sandwich block's gate logits ride in the shared expert's first GEMM as extra columns: model.proj)
+        if spec.shared is not None and W.shared_gu is not None:
+            kw["shared_mlp"] = (W.shared_gu, W.shared_down, spec.shared.ff, W.shared_interleaved, spec.shared.limit)
+            y, proj = ops.moe_experts(h, idx, wts, W.gate, W.up, W.down, spec.expert.limit, GLU_ALPHA, **kw)
+            model.proj = proj if proj is not None else model.proj
+            return y
+        if W.shared_gu is not None:
+            model.proj = ops.linear_f(h, W.shared_gu, dt)
+        return ops.moe_experts(h, idx, wts, W.gate, W.up, W.down, spec.expert.limit, GLU_ALPHA, **kw)
 
 
 class DeltaMixer:

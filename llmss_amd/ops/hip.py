@@ -1124,12 +1124,17 @@ _MOE_PP = os.environ.get("LLMSS_MOE_PP", "1") != "0"  # 0: grouped products on t
 MOE_PP_ROWS_TWO, MOE_PP_ROWS = 256, 128
 # And up to which those of 16 rows are: the same three layers gain 1.05 - 1.4 at 4 pairs, 1.0 - 1.5 at 8, 0.8 - 1.3 at 16, 0.65 - 1.1 at 24.
 MOE_DEC_ROWS = 8
+MOE_DEC_PAIRS = 1024  # pairs (and experts) up to which that kernel finds every expert's rows itself, without a grouping launch
+MOE_SHARED_ROWS = 64  # rows up to which it takes the shared expert along: two tiles, each reading that expert's weights
 MOE_GROUP_PAIRS = 4096  # pairs up to which one workgroup groups them: 4096 in 4.4 us (4.8 in two launches), 8192 in 6.5 (5.1)
 
 
 def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=True, act="glu_clamp",
-                weight_input=False, identity=False, shared_w=None, interleaved=False):
-    """``identity``: indices from E on are identity experts. ``combine=False``: leave the weighting and summing to the next residual add (returns a :class:`MoEPending`).
+                weight_input=False, identity=False, shared_w=None, interleaved=False, shared_mlp=None):
+    """``shared_mlp`` = (gate | up [| further] rows [2 Fs + D, K], down [N, Fs], Fs, gate and up rows in alternating groups of 16?, limit):
+    the shared expert's weights in the place of its rows; returns (result, [T, 2 Fs + D] whose last D columns are the products with the
+    further rows, or None without any). A step of few rows takes its products into the experts' own launches.
+    ``identity``: indices from E on are identity experts. ``combine=False``: leave the weighting and summing to the next residual add (returns a :class:`MoEPending`).
     ``weight_input``: the weights scale the two input products in the gate / up epilogue (the experts have no
     biases), and the outputs are summed plainly (``MoEPending.wts`` is None)."""
     T, K = h.shape
@@ -1153,10 +1158,16 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
         _check(shared.shape[0] == T, "shared rows")
     if shared_w is not None:
         _check(shared_w.dtype == torch.float32 and shared_w.is_contiguous() and shared_w.numel() == T and shared_w.is_cuda
-               and shared is not None, "shared_w fp32 [T]")
+               and (shared is not None or shared_mlp is not None), "shared_w fp32 [T]")
+    if shared_mlp is not None:
+        sgu, sdown, Fs, sinter, slimit = shared_mlp
+        D = sgu.shape[0] - 2 * Fs
+        _check(shared is None and D >= 0 and sgu.dtype == h.dtype and sgu.is_contiguous() and sgu.shape[1] == K and sgu.is_cuda
+               and sdown.dtype == h.dtype and sdown.is_contiguous() and tuple(sdown.shape) == (N, Fs) and sdown.is_cuda
+               and (not sinter or D == 0) and act in ("glu_clamp", "silu"), "shared expert's weights")
     out = torch.empty(T, N, dtype=torch.float32, device=h.device) if combine or T == 0 else None
     if T == 0:
-        return out
+        return out if shared_mlp is None else (out, torch.empty(0, sgu.shape[0], dtype=h.dtype, device=h.device) if D else None)
     P = T * top
     # rows per tile of the grouped GEMMs: 128 where the experts get enough rows to fill big tiles (bf16 only)
     rows = 128 if h.dtype == torch.bfloat16 and P >= 128 * E else 64
@@ -1171,6 +1182,16 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
         pp = False
     # and those with a few rows each: weights straight into the matrix instructions' operands
     dec = h.dtype == torch.bfloat16 and P <= MOE_DEC_ROWS * E and K % 32 == 0 and F % 32 == 0 and aligned and not pp
+    own = dec and P <= MOE_DEC_PAIRS and E <= MOE_DEC_PAIRS  # (no grouping: results in the pairs' order)
+    within = own and shared_mlp is not None and T <= MOE_SHARED_ROWS and Fs % 32 == 0 and not (sgu.data_ptr() | sdown.data_ptr()) & 15
+    gu = None
+    if shared_mlp is not None and not within:  # the shared expert on its own
+        if sinter:
+            shared = linear_f(linear(h, sgu, None, "none", True), sdown, h.dtype)
+        else:
+            gu = linear_f(h, sgu, h.dtype)
+            shared = linear_f(glu_act(gu, Fs, "silu") if act == "silu" else glu_clamp(gu, Fs, slimit, alpha), sdown, h.dtype)
+            gu = gu if D else None
     if pp:
         rows = 256
     if dec:
@@ -1179,8 +1200,9 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     _check(maxt <= 65535, "too many (token, expert) pairs in one step")
     dev = h.device
     blocks = -(-P // 1024) if P > MOE_GROUP_PAIRS else 1  # (each leaves its counts behind meta)
-    meta = torch.empty(1 + (E + 1) + 2 * maxt + (blocks * E if blocks > 1 else 0), dtype=torch.int32, device=dev)
-    order = torch.empty(P, dtype=torch.int32, device=dev)
+    if not own:
+        meta = torch.empty(1 + (E + 1) + 2 * maxt + (blocks * E if blocks > 1 else 0), dtype=torch.int32, device=dev)
+        order = torch.empty(P, dtype=torch.int32, device=dev)
     place = torch.empty(P, dtype=torch.int32, device=dev)
     act_ = torch.empty(P, F, dtype=h.dtype, device=dev)
     y = torch.empty(P, N, dtype=torch.float32, device=dev)
@@ -1189,8 +1211,22 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     pw, silu = (wts.data_ptr() if weight_input else 0), int(act == "silu")
     L = lib()
     st = _stream()
-    L.moe_group(idx.data_ptr(), P, E, maxt, meta.data_ptr(), order.data_ptr(), place.data_ptr(), rows, blocks, st)
-    if pp:
+    if not own:
+        L.moe_group(idx.data_ptr(), P, E, maxt, meta.data_ptr(), order.data_ptr(), place.data_ptr(), rows, blocks, st)
+    if own:
+        sact = None
+        if within:
+            sact, shared = (torch.empty(T, n, dtype=h.dtype, device=dev) for n in (Fs, N))
+            gu = torch.empty(T, 2 * Fs + D, dtype=h.dtype, device=dev) if D else None
+        L.moe_dec(1 if act == "gelu" else 0, h.data_ptr(), h.stride(0), up.data_ptr() if gate is None else gate.data_ptr(),
+                  0 if gate is None else up.data_ptr(), 0, 0, act_.data_ptr(), E, 0, top, F, K, float(limit), float(alpha), pw, silu,
+                  idx.data_ptr(), place.data_ptr(), T, 0, sgu.data_ptr() if within else 0, _ptr(sact),
+                  gu.data_ptr() + 2 * Fs * gu.element_size() if gu is not None else 0, 2 * Fs + D if gu is not None else 0,
+                  Fs if within else 0, K, D if within else 0, int(within and sinter), float(slimit) if within else 0.0, st)
+        L.moe_dec(2, act_.data_ptr(), F, down.data_ptr(), 0, 0, 0, y.data_ptr(), E, 0, top, N, F, 0.0, 0.0, 0, 0, idx.data_ptr(), 0, T,
+                  _ptr(sact), sdown.data_ptr() if within else 0, _ptr(shared) if within else 0, 0, 0, 0, Fs if within else 0, 0, 0, 0.0,
+                  st)
+    elif pp:
         if gate is not None:
             L.moe_pp_glu(h.data_ptr(), h.stride(0), gate.data_ptr(), up.data_ptr(), meta.data_ptr(), order.data_ptr(),
                          act_.data_ptr(), E, maxt, top, F, K, float(limit), float(alpha), pw, silu, st)
@@ -1202,9 +1238,9 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     elif dec:
         L.moe_dec(1 if act == "gelu" else 0, h.data_ptr(), h.stride(0), up.data_ptr() if gate is None else gate.data_ptr(),
                   0 if gate is None else up.data_ptr(), meta.data_ptr(), order.data_ptr(), act_.data_ptr(), E, maxt, top, F, K,
-                  float(limit), float(alpha), pw, silu, st)
+                  float(limit), float(alpha), pw, silu, 0, 0, T, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0.0, st)
         L.moe_dec(2, act_.data_ptr(), F, down.data_ptr(), 0, meta.data_ptr(), order.data_ptr(), y.data_ptr(), E, maxt, 1, N, F,
-                  0.0, 0.0, 0, 0, st)
+                  0.0, 0.0, 0, 0, 0, 0, T, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0.0, st)
     elif h.dtype == torch.bfloat16:  # matrix cores (csrc/gemm_tile.hip)
         L.moe_gate_up_tile(h.data_ptr(), h.stride(0), up.data_ptr() if interleaved else _ptr(gate), up.data_ptr(),
                            meta.data_ptr(), order.data_ptr(), act_.data_ptr(), E, maxt, top, F, K, float(limit), float(alpha),
@@ -1215,11 +1251,12 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
                       act_.data_ptr(), E, maxt, top, F, K, float(limit), float(alpha), dt, pw, silu, st)
         L.moe_down(act_.data_ptr(), down.data_ptr(), meta.data_ptr(), y.data_ptr(), E, maxt, N, F, dt, st)
     if not combine:
-        return MoEPending(y, place, None if weight_input else wts, shared, top, h if identity else None, shared_w)
+        pend = MoEPending(y, place, None if weight_input else wts, shared, top, h if identity else None, shared_w)
+        return pend if shared_mlp is None else (pend, gu)
     L.moe_combine(y.data_ptr(), place.data_ptr(), 0 if weight_input else wts.data_ptr(), _ptr(shared),
                   shared.stride(0) if shared is not None else 0, out.data_ptr(), T, N, top, dt,
                   h.data_ptr() if identity else 0, h.stride(0), _ptr(shared_w), st)
-    return out
+    return out if shared_mlp is None else (out, gu)
 
 
 # ----------------------------------- residual streams / convolution tails / matrix-state recurrences / sink attention

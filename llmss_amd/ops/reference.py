@@ -620,7 +620,7 @@ def moe_experts(h: torch.Tensor, idx: torch.Tensor, wts: torch.Tensor, gate: tor
                 down: torch.Tensor, limit: float, alpha: float, shared: Optional[torch.Tensor] = None,
                 combine: bool = True, act: str = "glu_clamp", weight_input: bool = False,
                 identity: bool = False, shared_w: Optional[torch.Tensor] = None,
-                interleaved: bool = False) -> torch.Tensor:
+                interleaved: bool = False, shared_mlp=None) -> torch.Tensor:
     """sum_j wts[t, j] * down_e(glu(gate_e h, up_e h)) (+ shared) with e = idx[t, j] -> fp32 [T, N]. Stacked expert
     weights gate / up [E, F, K], down [E, N, F]; the activation is rounded to the storage type between the
     products, as the grouped GEMMs do. ``act`` "silu": silu(g) * u without clamps. ``weight_input``: the weight
@@ -628,7 +628,17 @@ def moe_experts(h: torch.Tensor, idx: torch.Tensor, wts: torch.Tensor, gate: tor
     weight is applied to the two products). ``act`` "gelu": experts without a gate (``gate`` None), down_e(gelu(up_e
     h)), the error-function form. ``identity``: an index from E on is an
     identity expert, its output is h[t] itself. ``shared_w`` fp32 [T] multiplies the shared rows.
-    ``interleaved`` (``gate`` None): up [E, 2F, K] holds gate and up rows in alternating groups of 16."""
+    ``interleaved`` (``gate`` None): up [E, 2F, K] holds gate and up rows in alternating groups of 16.
+    ``shared_mlp`` = (gate | up [| further] rows [2 Fs + D, K], down [N, Fs], Fs, gate and up in alternating groups of 16?, limit): the
+    shared expert's weights in the place of its rows; returns (result, [T, 2 Fs + D] whose last D columns are the products with the further
+    rows, or None without any)."""
+    if shared_mlp is not None:
+        sgu, sdown, Fs, sinter, slimit = shared_mlp
+        gu = linear(h, sgu, None, "none", True) if sinter else linear_f(h, sgu, h.dtype)
+        a = gu if sinter else glu_act(gu, Fs, "silu") if act == "silu" else glu_clamp(gu, Fs, slimit, alpha)
+        out = moe_experts(h, idx, wts, gate, up, down, limit, alpha, linear_f(a, sdown, h.dtype), combine, act, weight_input, identity,
+                          shared_w, interleaved)
+        return out, gu if sgu.shape[0] > 2 * Fs else None
     if interleaved:
         gate, up = glu_split(up, 1)
     T = h.shape[0]
