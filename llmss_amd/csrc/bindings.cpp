@@ -204,6 +204,13 @@ void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const void* e
                               int groups, const void* ident, int64_t ldi, const void* y2, int64_t ldy2, const void* wl,
                               const void* wr, float cl, float cr, int64_t lda, const void* sw, int slabs, int T_, int W, int dt,
                               hipStream_t st);
+void launch_sandwich_tail(void* x, const void* y, int64_t ldy, const void* ey, const void* place, const void* wts, int top,
+                          const void* shared_, int64_t lds_, const void* r, int64_t ldr, const void* rb, const void* wpost,
+                          const void* add, const void* wnext, void* h, int64_t ldh, float eps, const void* y2, int64_t ldy2,
+                          const void* wl, const void* wr, float cl, float cr, int64_t lda, const void* sw, int slabs, int T_, int W,
+                          int kind, const void* router, const void* corr, void* idx, void* rwts, int E, int rtop, int norm, int smax,
+                          const void* zb, void* sg, const void* ids, const void* table, int64_t ldt, int vocab, int col0, int d,
+                          const void* wg, const void* wp, const void* wn, hipStream_t st);
 void launch_token_side_add(void* x, const void* ids, const void* table, int64_t ldt, int vocab, int col0, int d,
                            const void* wg, const void* wp, const void* wn, const void* add, const void* wnext, void* h,
                            int64_t ldh, float eps, int T_, int W, int dt, hipStream_t st);
@@ -696,6 +703,18 @@ PYBIND11_MODULE(_C, m) {
     launch_sandwich_add_norm(P(x), CP(y), ldy, CP(ey), CP(place), CP(wts), top, CP(sh), lds_, CP(r), ldr, CP(rb),
                              CP(wpost), CP(add), CP(wnext), P(h), ldh, eps, groups, CP(ident), ldi, CP(y2), ldy2,
                              CP(wl), CP(wr), cl, cr, lda, CP(sw), slabs, T, W, dt, S(st));
+  });
+  m.def("sandwich_tail", [](uintptr_t x, uintptr_t y, int64_t ldy, uintptr_t ey, uintptr_t place, uintptr_t wts, int top, uintptr_t sh,
+                            int64_t lds_, uintptr_t r, int64_t ldr, uintptr_t rb, uintptr_t wpost, uintptr_t add, uintptr_t wnext,
+                            uintptr_t h, int64_t ldh, float eps, uintptr_t y2, int64_t ldy2, uintptr_t wl, uintptr_t wr, float cl,
+                            float cr, int64_t lda, uintptr_t sw, int slabs, int T, int W, int kind, uintptr_t router, uintptr_t corr,
+                            uintptr_t idx, uintptr_t rwts, int E, int rtop, int norm, int smax, uintptr_t zb, uintptr_t sg,
+                            uintptr_t ids, uintptr_t table, int64_t ldt, int vocab, int col0, int d, uintptr_t wg, uintptr_t wp,
+                            uintptr_t wn, uintptr_t st) {
+    launch_sandwich_tail(P(x), CP(y), ldy, CP(ey), CP(place), CP(wts), top, CP(sh), lds_, CP(r), ldr, CP(rb), CP(wpost), CP(add),
+                         CP(wnext), P(h), ldh, eps, CP(y2), ldy2, CP(wl), CP(wr), cl, cr, lda, CP(sw), slabs, T, W, kind, CP(router),
+                         CP(corr), P(idx), P(rwts), E, rtop, norm, smax, CP(zb), P(sg), CP(ids), CP(table), ldt, vocab, col0, d, CP(wg),
+                         CP(wp), CP(wn), S(st));
   });
   m.def("token_side_add", [](uintptr_t x, uintptr_t ids, uintptr_t table, int64_t ldt, int vocab, int col0, int d,
                              uintptr_t wg, uintptr_t wp, uintptr_t wn, uintptr_t add, uintptr_t wnext, uintptr_t h,

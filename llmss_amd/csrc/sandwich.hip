@@ -18,6 +18,7 @@
 // Norm weights, biases and layer scales are fp32. One workgroup per row; the gated row lives in LDS between the
 // pass that sums its squares and the pass that adds it, and the updated x between that pass and the norm.
 #include "anytype.h"
+#include "route.h"
 
 struct SandwichArgs {
   float* x;
@@ -239,23 +240,70 @@ __global__ __launch_bounds__(512) void sandwich_add_norm_kernel(SandwichArgs p) 
   norm_out<T, V>(buf, ss2, p, t, red);
 }
 
+struct SideArgs {
+  const int64_t* ids;
+  const void* table;  // [vocab, ldt] in the storage type
+  int64_t ldt;
+  int vocab, col0, d;
+  const void* wg;  // [d, W]
+  const void* wp;  // [W, d]
+  const float* wn;
+};
+
+__device__ __forceinline__ float gelu_tanh_f(float z) {
+  return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+}
+
+// What a row goes through after its closing op, in the same launch (steps of few bf16 rows up to 2048 wide, workgroups of eight waves). A
+// decode step is the chain of its launches and of their loads, so a tail's weights are asked for behind the closing op's operands and before
+// its first sum.
+struct NoTail {
+  static constexpr int kind = 0;
+};
+// the router of the next sublayer's experts, over h as moe_router (moe.hip) has it: the same sums in the same order
+struct RouteTail {
+  static constexpr int kind = 1;
+  const bf16_t* wr;  // [E (+ 1), W]
+  const float* corr;
+  int* idx;
+  float* wts;
+  int E, top, norm, smax;
+  const float* zb;
+  float* sg;
+};
+// the token input (D its numbers, NW at least W / 256), before `add` and the norm
+template <int D_, int NW_>
+struct SideTail : SideArgs {
+  static constexpr int kind = 2, D = D_, NW = NW_;
+};
+
 // The same for rows of up to 4096 and a norm of one part: a thread keeps NC times four columns of everything in registers, all loads are
 // issued before the first sum, and only two sums pass through LDS. The kernel above asks for the stream and the weights behind the
 // first sum, a round trip more. us, plain rows / gated / four experts' rows: 33 x 2048 5.0 / 5.3 / 5.5 -> 4.3 / 4.7 / 4.8, 8192 x 2048
 // 36.3 / 42.4 / 84.7 -> 36.4 / 43.9 / 72.6, 8192 x 1024 24.8 / 28.3 / 37.8 -> 20.6 / 24.5 / 34.1. With eight columns a thread the
 // registers leave half the waves: 8192 x 4096 84.6 -> 106, so more than 512 such rows keep the kernel above.
-template <typename T, int NC>
-__global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p) {
+// With a tail, one launch against two, in a decode step (kernel times, us): the router of 17 outputs over 8 rows of 1024 11.0 -> 7.9, of 32
+// over 33 rows of 2048 13.8 -> 11.1, the token input of 32 numbers 17.1 -> 14.7 (each of 33 workgroups draws its 256 KB of weights through one
+// CU). A tail's kernel for every form of y at once, its loads behind a branch a column: 8.7, 11.3 and 16.2.
+// FORM: what y is, where a launch is a chain that fetches its code as it goes (tails); else found at run time
+enum { Y_ANY = -1, Y_NONE, Y_ROWS, Y_SLABS, Y_PAIR, Y_EXPERTS };
+template <typename T, int NC, typename TAIL, int FORM>
+__global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p, TAIL a) {
+  constexpr bool ROUTE = TAIL::kind == 1, SIDE = TAIL::kind == 2;
+  static_assert(TAIL::kind == 0 || (NC == 1 && sizeof(T) == 2), "tails: bf16 rows, four columns a thread");
   __shared__ float red[32];
-  const int t = blockIdx.x, W = p.W;
+  __shared__ __attribute__((aligned(16))) float row[TAIL::kind == 0 ? 1 : ROUTE ? 1024 + 132 : 2048 + 64];
+  const int t = blockIdx.x, W = p.W, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   float* xr = p.x + (int64_t)t * W;
-  const bool has_y = p.y != nullptr || p.ey != nullptr;
+  const int form = FORM != Y_ANY ? FORM : p.y2 ? Y_PAIR : p.slabs ? Y_SLABS : p.y ? Y_ROWS : p.ey ? Y_EXPERTS : Y_NONE;
+  const bool has_y = form != Y_NONE;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   f32x4 x[NC], v[NC], wp[NC], wn[NC], ad[NC];
-  int col[NC];
+  int col[NC], at[NC];
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
     col[i] = 4 * (threadIdx.x + blockDim.x * i);
+    at[i] = min(col[i], W - 4);
     x[i] = v[i] = wp[i] = wn[i] = ad[i] = zero;
   }
 #define EACH(...)                     \
@@ -263,19 +311,87 @@ __global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p) {
     if (col[i] < W) {                 \
       __VA_ARGS__;                    \
     }
-  EACH(x[i] = ld4(xr + col[i]))
-  if (p.wnext) EACH(wn[i] = ld4(p.wnext + col[i]))
-  if (p.add) EACH(ad[i] = ld4(p.add + (int64_t)t * p.lda + col[i]))
+// loads: threads past the row take its last columns and drop them; as they lie in memory, for a conversion right behind a load waits for it
+// before the next one is issued
+#define LOAD(...) _Pragma("unroll") for (int i = 0; i < NC; ++i) { __VA_ARGS__; }
+  typedef typename std::conditional<sizeof(T) == 2, u16x4, f32x4>::type Raw;
+  auto raw = [](const void* q, int64_t o) { return *reinterpret_cast<const Raw*>((const T*)q + o); };
+  auto num = [](const Raw& q) {
+    if constexpr (sizeof(T) == 2) return f32x4{bf2f(q[0]), bf2f(q[1]), bf2f(q[2]), bf2f(q[3])};
+    else return q;
+  };
+  // ---- a tail's weights
+  constexpr int RO = ROUTE ? 5 : 1, RC = ROUTE ? 4 : 1;  // a wave's outputs wv, wv + 8, .. of the first look; pieces of 512 of the width
+  u16x8 rw[RO][RC];
+  float rcorr[2] = {0.f, 0.f}, rbias[2] = {0.f, 0.f};
+  constexpr int SR = [] { if constexpr (SIDE) return TAIL::D / 8; else return 1; }();  // gate rows of a wave
+  constexpr int SW = [] { if constexpr (SIDE) return TAIL::NW; else return 1; }();
+  u16x4 sgw[SR][SW];
+  u16x8 spw[SIDE ? 4 : 1][SR];
+  f32x4 swn = zero;
+  bf16_t ser = 0;
+  int64_t id = 0;
+  int eg = 0;
+  auto load_route = [&](int e0) {
+    if constexpr (ROUTE) {
+#pragma unroll
+      for (int n = 0; n < RO; ++n)
+#pragma unroll
+        for (int u = 0; u < RC; ++u)
+          rw[n][u] = *reinterpret_cast<const u16x8*>(a.wr + (int64_t)min(e0 + 8 * n, eg - 1) * W + min(lane * 8 + 512 * u, W - 8));
+    }
+  };
+  auto load_proj = [&]() {
+    if constexpr (SIDE) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < SR; ++j)
+          spw[i][j] = *reinterpret_cast<const u16x8*>((const bf16_t*)a.wp + (int64_t)(at[0] + i) * TAIL::D + 8 * j);
+    }
+  };
+  auto load_tail = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (ROUTE) {
+      load_route(wv);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if (a.corr) rcorr[j] = a.corr[min(lane + 64 * j, a.E - 1)];
+        if (a.zb) rbias[j] = a.zb[min(lane + 64 * j, a.E - 1)];
+      }
+    }
+    if constexpr (SIDE) {
+#pragma unroll
+      for (int r = 0; r < SR; ++r)
+#pragma unroll
+        for (int k = 0; k < SW; ++k)
+          sgw[r][k] = *reinterpret_cast<const u16x4*>((const bf16_t*)a.wg + (int64_t)(wv * SR + r) * W + min(k * 256, W - 256) + lane * 4);
+      if constexpr (TAIL::D == 32) load_proj();  // (the deeper form's registers hold one of the two at a time)
+      swn = ld4(a.wn + at[0]);
+      id = id < 0 ? 0 : (id >= a.vocab ? a.vocab - 1 : id);
+      ser = ((const bf16_t*)a.table)[id * a.ldt + a.col0 + wv * SR + min(lane, SR - 1)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if constexpr (ROUTE) eg = a.E + (a.sg ? 1 : 0);
+  if constexpr (SIDE) id = a.ids[t];
+  LOAD(x[i] = ld4(xr + at[i]))
+  if (p.wnext) LOAD(wn[i] = ld4(p.wnext + at[i]))
+  if (p.add) LOAD(ad[i] = ld4(p.add + (int64_t)t * p.lda + at[i]))
+  if (!has_y) load_tail();
   if (has_y) {
-    f32x4 z[NC], b[NC];
-    EACH(wp[i] = ld4(p.wpost + col[i]))
-    if (p.r) EACH(z[i] = ld4((const T*)p.r + (int64_t)t * p.ldr + col[i]); b[i] = ld4(p.rb + col[i]))
-    if (p.y2) {
-      f32x4 y2[NC];
-      EACH(v[i] = ld4((const T*)p.y + (int64_t)t * p.ldy + col[i]); y2[i] = ld4((const T*)p.y2 + (int64_t)t * p.ldy2 + col[i]))
+    Raw z[NC];
+    f32x4 b[NC];
+    LOAD(wp[i] = ld4(p.wpost + at[i]))
+    if (p.r) LOAD(z[i] = raw(p.r, (int64_t)t * p.ldr + at[i]); b[i] = ld4(p.rb + at[i]))
+    if (form == Y_PAIR) {
+      Raw q1[NC], q2[NC];
+      f32x4 y2[NC], wa[NC], wb[NC];
+      LOAD(q1[i] = raw(p.y, (int64_t)t * p.ldy + at[i]); q2[i] = raw(p.y2, (int64_t)t * p.ldy2 + at[i]))
+      if (p.wl) LOAD(wa[i] = ld4(p.wl + at[i]); wb[i] = ld4(p.wr + at[i]))
+      load_tail();
+      LOAD(v[i] = num(q1[i]); y2[i] = num(q2[i]))
       if (p.wl) {  // two mixers: the root mean square of each row first
-        f32x4 wa[NC], wb[NC];
-        EACH(wa[i] = ld4(p.wl + col[i]); wb[i] = ld4(p.wr + col[i]))
         float sl = 0.f, sr = 0.f;
         EACH(for (int e = 0; e < 4; ++e) sl = fmaf(v[i][e], v[i][e], sl), sr = fmaf(y2[i][e], y2[i][e], sr))
         const f32x2 s2 = block_sum2(sl, sr, red);
@@ -284,13 +400,26 @@ __global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p) {
       } else {
         EACH(for (int e = 0; e < 4; ++e) v[i][e] = fmaf(p.cl, v[i][e], p.cr * y2[i][e]))
       }
-    } else if (p.slabs) {
-      EACH(v[i] = slab_sum<f32x4>((const float*)p.y + (int64_t)t * W + col[i], p.slabs, (int64_t)gridDim.x * W))
-    } else if (p.y) {
-      EACH(v[i] = ld4((const T*)p.y + (int64_t)t * p.ldy + col[i]))
+    } else if (form == Y_SLABS) {
+      f32x4 q[8][NC];
+      const int64_t ls = (int64_t)gridDim.x * W;
+      const float* sp = (const float*)p.y + (int64_t)t * W;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        LOAD(q[j][i] = ld4(sp + min(j, p.slabs - 1) * ls + at[i]))
+      load_tail();
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j < p.slabs) LOAD(v[i] += q[j][i])
+      for (int j = 8; j < p.slabs; ++j) LOAD(v[i] += ld4(sp + j * ls + at[i]))
+    } else if (form == Y_ROWS) {
+      Raw q[NC];
+      LOAD(q[i] = raw(p.y, (int64_t)t * p.ldy + at[i]))
+      load_tail();
+      LOAD(v[i] = num(q[i]))
     } else {
-      f32x4 sh[NC];
-      if (p.shared_) EACH(sh[i] = ld4((const T*)p.shared_ + (int64_t)t * p.lds_ + col[i]))
+      Raw sh[NC];
+      if (p.shared_) LOAD(sh[i] = raw(p.shared_, (int64_t)t * p.lds_ + at[i]))
       for (int j0 = 0; j0 < p.top; j0 += 4) {  // four pairs in flight
         f32x4 e[4][NC];
         float wj[4];
@@ -299,43 +428,152 @@ __global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p) {
           const int jj = min(j0 + j, p.top - 1);
           const float* er = p.ey + (int64_t)p.place[(int64_t)t * p.top + jj] * W;
           wj[j] = p.wts ? p.wts[(int64_t)t * p.top + jj] : 1.0f;
-          EACH(e[j][i] = ld4(er + col[i]))
+          LOAD(e[j][i] = ld4(er + at[i]))
         }
+        if (j0 == 0) load_tail();
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           if (j0 + j >= p.top) continue;
-          EACH(for (int k = 0; k < 4; ++k) v[i][k] = fmaf(wj[j], e[j][i][k], v[i][k]))
+          LOAD(for (int k = 0; k < 4; ++k) v[i][k] = fmaf(wj[j], e[j][i][k], v[i][k]))
         }
       }
       const float swt = p.sw ? p.sw[t] : 1.0f;
-      if (p.shared_) EACH(for (int e = 0; e < 4; ++e) v[i][e] = fmaf(swt, sh[i][e], v[i][e]))
+      if (p.shared_) LOAD(const f32x4 q = num(sh[i]); for (int e = 0; e < 4; ++e) v[i][e] = fmaf(swt, q[e], v[i][e]))
     }
-    if (p.r) EACH(for (int e = 0; e < 4; ++e) v[i][e] = v[i][e] / (1.0f + expf(-(z[i][e] + b[i][e]))))
+    if (p.r) LOAD(const f32x4 q = num(z[i]); for (int e = 0; e < 4; ++e) v[i][e] = v[i][e] / (1.0f + expf(-(q[e] + b[i][e]))))
     float ss = 0.f;
     EACH(for (int e = 0; e < 4; ++e) ss = fmaf(v[i][e], v[i][e], ss))
     ss = block_sum(ss, red);
     const float inv = 1.0f / sqrtf(ss / (float)W + p.eps);
     EACH(for (int e = 0; e < 4; ++e) x[i][e] = fmaf(v[i][e] * inv, wp[i][e], x[i][e]))
   }
+  if constexpr (SIDE) {
+    constexpr int D = TAIL::D;
+    float* gs = row + 2048;
+    EACH(*reinterpret_cast<f32x4*>(row + col[i]) = x[i])
+    __syncthreads();
+    float acc[SR];
+#pragma unroll
+    for (int r = 0; r < SR; ++r) acc[r] = 0.f;
+#pragma unroll
+    for (int k = 0; k < SW; ++k)
+      if (k * 256 < W) {
+        const f32x4 xv = *reinterpret_cast<const f32x4*>(row + k * 256 + lane * 4);
+#pragma unroll
+        for (int r = 0; r < SR; ++r)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[r] = fmaf(bf2f(sgw[r][k][i]), xv[i], acc[r]);
+      }
+    if constexpr (D != 32) load_proj();
+#pragma unroll
+    for (int r = 0; r < SR; ++r) {
+      acc[r] = warp_sum(acc[r]);
+      if (lane == r) gs[wv * SR + r] = gelu_tanh_f(acc[r]) * bf2f(ser);
+    }
+    __syncthreads();
+    f32x4 y = zero;
+    if (col[0] < W) {
+#pragma unroll
+      for (int j = 0; j < SR; ++j) {
+        const f32x4 g0 = *reinterpret_cast<const f32x4*>(gs + 8 * j), g1 = *reinterpret_cast<const f32x4*>(gs + 8 * j + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            y[i] = fmaf(bf2f(spw[i][j][e]), g0[e], y[i]);
+            y[i] = fmaf(bf2f(spw[i][j][4 + e]), g1[e], y[i]);
+          }
+      }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ss = fmaf(y[i], y[i], ss);
+    const float inv = 1.0f / sqrtf(block_sum(ss, red) / (float)W + p.eps);
+    EACH(for (int e = 0; e < 4; ++e) x[i][e] = fmaf(y[e] * inv, swn[e], x[i][e]))
+  }
   if (p.add) EACH(for (int e = 0; e < 4; ++e) x[i][e] += ad[i][e])
-  if (has_y || p.add) EACH(st4(xr + col[i], x[i]))
+  if (has_y || p.add || SIDE) EACH(st4(xr + col[i], x[i]))
   if (!p.wnext) return;
   float ss = 0.f;
   EACH(for (int e = 0; e < 4; ++e) ss = fmaf(x[i][e], x[i][e], ss))
   ss = block_sum(ss, red);
   const float inv = 1.0f / sqrtf(ss / (float)W + p.eps);
-  EACH(f32x4 o; for (int e = 0; e < 4; ++e) o[e] = x[i][e] * inv * wn[i][e]; st4((T*)p.h + (int64_t)t * p.ldh + col[i], o))
+  EACH(f32x4 o; for (int e = 0; e < 4; ++e) o[e] = x[i][e] * inv * wn[i][e]; st4((T*)p.h + (int64_t)t * p.ldh + col[i], o);
+       if constexpr (ROUTE) st4((bf16_t*)row + col[i], o))
 #undef EACH
+#undef LOAD
+  if constexpr (ROUTE) {
+    float* sc = row + 1024;
+    __syncthreads();
+    u16x8 hv[RC];
+#pragma unroll
+    for (int u = 0; u < RC; ++u) hv[u] = *reinterpret_cast<const u16x8*>((const bf16_t*)row + min(lane * 8 + 512 * u, W - 8));
+    for (int e0 = wv; e0 < eg; e0 += 8 * RO) {
+      if (e0 != wv) load_route(e0);
+#pragma unroll
+      for (int n = 0; n < RO; ++n) {
+        const int e = e0 + 8 * n;
+        if (e >= eg) break;
+        float z = 0.f;
+#pragma unroll
+        for (int u = 0; u < RC; ++u) {
+          if (lane * 8 + 512 * u >= W) break;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) z = fmaf(bf2f(hv[u][i]), bf2f(rw[n][u][i]), z);
+        }
+        z = warp_sum(z);
+        if (lane != 0) continue;
+        if (e == a.E) a.sg[t] = 1.f / (1.f + expf(-z));
+        else sc[e] = z;
+      }
+    }
+    __syncthreads();
+    if (wv) return;
+    float z[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) z[j] = lane + 64 * j < a.E ? sc[lane + 64 * j] + rbias[j] : -INFINITY;
+    __builtin_amdgcn_wave_barrier();
+    route_ranked(z, sc, rcorr, a.idx + (int64_t)t * a.top, a.wts + (int64_t)t * a.top, a.E, a.top, a.norm, a.smax);
+  }
 }
 
 static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const void* ey, const void* place, const void* wts,
+struct SandwichTail {
+  int kind;  // 0: none, 1: route, 2: side
+  RouteTail route;
+  SideArgs side;
+};
+
+template <typename TAIL>
+static void launch_tail(const SandwichArgs& p, const TAIL& a, int T_, hipStream_t st) {
+  if (p.y2) sandwich_rows_kernel<bf16_t, 1, TAIL, Y_PAIR><<<T_, 512, 0, st>>>(p, a);
+  else if (p.slabs) sandwich_rows_kernel<bf16_t, 1, TAIL, Y_SLABS><<<T_, 512, 0, st>>>(p, a);
+  else if (p.y) sandwich_rows_kernel<bf16_t, 1, TAIL, Y_ROWS><<<T_, 512, 0, st>>>(p, a);
+  else if (p.ey) sandwich_rows_kernel<bf16_t, 1, TAIL, Y_EXPERTS><<<T_, 512, 0, st>>>(p, a);
+  else sandwich_rows_kernel<bf16_t, 1, TAIL, Y_NONE><<<T_, 512, 0, st>>>(p, a);
+}
+
+// rows a token input can follow in the closing op's launch
+static bool side_tail_ok(const SideArgs& s, int W) {
+  return (s.d == 32 || s.d == 64) && W % 256 == 0 && W <= 2048 && al16(s.wp) && al16(s.wn) && ((uintptr_t)s.wg & 7) == 0;
+}
+static void launch_side_tail(const SandwichArgs& p, const SideArgs& s, int T_, hipStream_t st) {
+  if (!side_tail_ok(s, p.W)) throw std::runtime_error("sandwich_add_norm: token input of 32 or 64 numbers over aligned rows of whole 256s");
+#define LAUNCH_ROW(D_, NW_) launch_tail(p, SideTail<D_, NW_>{s}, T_, st)
+  if (s.d == 32 && p.W <= 1024) LAUNCH_ROW(32, 4);
+  else if (s.d == 32) LAUNCH_ROW(32, 8);
+  else if (p.W <= 1024) LAUNCH_ROW(64, 4);
+  else LAUNCH_ROW(64, 8);
+#undef LAUNCH_ROW
+}
+
+static void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const void* ey, const void* place, const void* wts,
                               int top, const void* shared_, int64_t lds_, const void* r, int64_t ldr, const void* rb,
                               const void* wpost, const void* add, const void* wnext, void* h, int64_t ldh, float eps,
                               int groups, const void* ident, int64_t ldi, const void* y2, int64_t ldy2, const void* wl,
                               const void* wr, float cl, float cr, int64_t lda, const void* sw, int slabs, int T_, int W, int dt,
-                              hipStream_t st) {
+                              const SandwichTail& tail, hipStream_t st) {
   if (T_ == 0) return;
   if (groups < 1 || W % groups) throw std::runtime_error("sandwich_add_norm: the norm's parts must divide the row");
   if (((size_t)W + groups) * 4 > 64 * 1024) throw std::runtime_error("sandwich_add_norm: rows wider than 16384");
@@ -354,32 +592,31 @@ void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const void* e
   // but 1551 with one expert each 1.20: two waves of eight-wave workgroups where the general kernel's four fit at once)
   const bool rows = vec && groups == 1 && !ident && (W <= 1280 || (W <= 2048 && (T_ <= 1024 || (ey && T_ > 2048))) || (W <= 4096 && T_ <= 512));
   if (slabs < 0 || (slabs && (!y || y2))) throw std::runtime_error("sandwich_add_norm: slabs of one product only");
+  if (tail.kind) {
+    if (!vec || groups != 1 || ident || dt != 0 || W > 2048) throw std::runtime_error("sandwich_add_norm: a tail needs whole bf16 rows of up to 2048 at aligned places");
+    if (tail.kind == 1) {
+      const RouteTail& r_ = tail.route;
+      if (!wnext || W % 8 || !al16(r_.wr) || r_.E < 1 || r_.E > 128 || r_.top < 1 || r_.top > r_.E)
+        throw std::runtime_error("sandwich_add_norm: router of 1 - 128 outputs over aligned rows");
+      launch_tail(p, r_, T_, st);
+    } else {
+      launch_side_tail(p, tail.side, T_, st);
+    }
+    HIP_CHECK_LAUNCH();
+    return;
+  }
   // whole waves, no more than the row has columns for (256 and 512 threads: 1600 rows and more of 256 1.44, of 1280 1.11 times as long), but for
   // 448, which spread unevenly over the SIMDs (1792 wide: 1.07)
   const int rth = W <= 1536 ? (W / 4 + 63) / 64 * 64 : 512;
   DISPATCH_T(dt, T, {
-    if (rows && W <= 2048) sandwich_rows_kernel<T, 1><<<T_, rth, 0, st>>>(p);
-    else if (rows) sandwich_rows_kernel<T, 2><<<T_, 512, 0, st>>>(p);
+    if (rows && W <= 2048) sandwich_rows_kernel<T, 1, NoTail, Y_ANY><<<T_, rth, 0, st>>>(p, NoTail{});
+    else if (rows) sandwich_rows_kernel<T, 2, NoTail, Y_ANY><<<T_, 512, 0, st>>>(p, NoTail{});
     else if (slabs && vec) sandwich_add_norm_kernel<T, 4, true><<<T_, th, lds, st>>>(p);
     else if (slabs) sandwich_add_norm_kernel<T, 1, true><<<T_, th, lds, st>>>(p);
     else if (vec) sandwich_add_norm_kernel<T, 4><<<T_, th, lds, st>>>(p);
     else sandwich_add_norm_kernel<T, 1><<<T_, th, lds, st>>>(p);
   });
   HIP_CHECK_LAUNCH();
-}
-
-struct SideArgs {
-  const int64_t* ids;
-  const void* table;  // [vocab, ldt] in the storage type
-  int64_t ldt;
-  int vocab, col0, d;
-  const void* wg;  // [d, W]
-  const void* wp;  // [W, d]
-  const float* wn;
-};
-
-__device__ __forceinline__ float gelu_tanh_f(float z) {
-  return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
 }
 
 // buf: [W] the x row, then [W] the projected row, then [d] the gated numbers
@@ -460,97 +697,6 @@ __global__ __launch_bounds__(512) void token_side_add_kernel(SandwichArgs p, Sid
     }
   }
   norm_out<T, V>(xs, ss2, p, t, red);
-}
-
-// The token input of a few bf16 rows, up to 2048 wide (NW: at least W / 256): the kernel above with everything that a row needs asked for
-// at the start - a wave its gate rows, a thread the projection's rows of its four columns - since a decode step is nothing but the
-// chain of its loads: 24 -> 15 us for 33 rows
-// of 2048 in a decode step. A CU holds one workgroup: up to 256 rows (12.6 us), at 1006 it takes 43 us and the kernel above 26.
-template <int D, int NW>
-__global__ __launch_bounds__(512) void token_side_row_kernel(SandwichArgs p, SideArgs s) {
-  constexpr int R = D / 8;  // gate rows of a wave
-  __shared__ __attribute__((aligned(16))) float xs[NW * 256];
-  __shared__ __attribute__((aligned(16))) float gs[D];
-  __shared__ float red[32];
-  const int t = blockIdx.x, W = p.W, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, c = threadIdx.x * 4;
-  const bool live = c < W;
-  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  float* xr = p.x + (int64_t)t * W;
-  f32x4 xv = live ? *reinterpret_cast<const f32x4*>(xr + c) : zero;
-  int64_t id = s.ids[t];
-  u16x4 wg[R][NW];
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int k = 0; k < NW; ++k)
-      if (k * 256 < W) wg[r][k] = *reinterpret_cast<const u16x4*>((const bf16_t*)s.wg + (int64_t)(wv * R + r) * W + k * 256 + lane * 4);
-  u16x8 wp[4][D / 8];
-  auto load_wp = [&]() {
-    if (live) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < D / 8; ++j) wp[i][j] = *reinterpret_cast<const u16x8*>((const bf16_t*)s.wp + (int64_t)(c + i) * D + 8 * j);
-    }
-  };
-  if constexpr (D == 32) load_wp();  // (the deeper form's registers hold one of the two at a time)
-  const f32x4 wn = live ? *reinterpret_cast<const f32x4*>(s.wn + c) : zero;
-  const f32x4 wx = live && p.wnext ? *reinterpret_cast<const f32x4*>(p.wnext + c) : zero;
-  const f32x4 ad = live && p.add ? *reinterpret_cast<const f32x4*>(p.add + (int64_t)t * W + c) : zero;
-  id = id < 0 ? 0 : (id >= s.vocab ? s.vocab - 1 : id);
-  const float er = lane < R ? bf2f(((const bf16_t*)s.table)[id * s.ldt + s.col0 + wv * R + lane]) : 0.f;
-  if (live) *reinterpret_cast<f32x4*>(xs + c) = xv;
-  __syncthreads();
-  float a[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) a[r] = 0.f;
-#pragma unroll
-  for (int k = 0; k < NW; ++k)
-    if (k * 256 < W) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(xs + k * 256 + lane * 4);
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) a[r] = fmaf(bf2f(wg[r][k][i]), v[i], a[r]);
-    }
-  if constexpr (D != 32) load_wp();
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    a[r] = warp_sum(a[r]);
-    if (lane == r) gs[wv * R + r] = gelu_tanh_f(a[r]) * er;
-  }
-  __syncthreads();
-  f32x4 y = zero;
-  if (live) {
-#pragma unroll
-    for (int j = 0; j < D / 8; ++j) {
-      const f32x4 g0 = *reinterpret_cast<const f32x4*>(gs + 8 * j), g1 = *reinterpret_cast<const f32x4*>(gs + 8 * j + 4);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          y[i] = fmaf(bf2f(wp[i][j][e]), g0[e], y[i]);
-          y[i] = fmaf(bf2f(wp[i][j][4 + e]), g1[e], y[i]);
-        }
-    }
-  }
-  float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) ss = fmaf(y[i], y[i], ss);
-  const float inv = 1.0f / sqrtf(block_sum(ss, red) / (float)W + p.eps);
-  float ss2 = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    xv[i] = fmaf(y[i] * inv, wn[i], xv[i]);
-    if (p.add) xv[i] += ad[i];
-    ss2 = fmaf(xv[i], xv[i], ss2);
-  }
-  if (live) *reinterpret_cast<f32x4*>(xr + c) = xv;
-  if (!p.wnext) return;
-  const float invx = 1.0f / sqrtf(block_sum(ss2, red) / (float)W + p.eps);
-  if (live)
-    *reinterpret_cast<u16x4*>((bf16_t*)p.h + (int64_t)t * p.ldh + c) =
-        u16x4{f2bf(xv[0] * invx * wx[0]), f2bf(xv[1] * invx * wx[1]), f2bf(xv[2] * invx * wx[2]), f2bf(xv[3] * invx * wx[3])};
 }
 
 // The token input for bf16 weights, 16 rows per workgroup on the matrix cores (the kernel above reads both small matrices from L2
@@ -713,11 +859,11 @@ void launch_token_side_add(void* x, const void* ids, const void* table, int64_t 
     HIP_CHECK_LAUNCH();
     return;
   }
-  if (dt == 0 && vec && T_ <= 256 && (d == 32 || d == 64) && W % 256 == 0 && W <= 2048 && al16(wp)) {
-    if (d == 32 && W <= 1024) token_side_row_kernel<32, 4><<<T_, 512, 0, st>>>(p, s);
-    else if (d == 32) token_side_row_kernel<32, 8><<<T_, 512, 0, st>>>(p, s);
-    else if (W <= 1024) token_side_row_kernel<64, 4><<<T_, 512, 0, st>>>(p, s);
-    else token_side_row_kernel<64, 8><<<T_, 512, 0, st>>>(p, s);
+  // (a row per workgroup, everything it needs asked for at the start: 33 rows of 2048 in a decode step 24 -> 15 us. A CU holds one
+  // workgroup: up to 256 rows (12.6 us), at 1006 it takes 43 us and the kernel above 26.)
+  if (dt == 0 && vec && T_ <= 256 && side_tail_ok(s, W)) {
+    p.lda = W;
+    launch_side_tail(p, s, T_, st);
     HIP_CHECK_LAUNCH();
     return;
   }
@@ -726,4 +872,35 @@ void launch_token_side_add(void* x, const void* ids, const void* table, int64_t 
     else token_side_add_kernel<T, 1><<<T_, 512, lds, st>>>(p, s);
   });
   HIP_CHECK_LAUNCH();
+}
+
+void launch_sandwich_tail(void* x, const void* y, int64_t ldy, const void* ey, const void* place, const void* wts, int top,
+                          const void* shared_, int64_t lds_, const void* r, int64_t ldr, const void* rb, const void* wpost,
+                          const void* add, const void* wnext, void* h, int64_t ldh, float eps, const void* y2, int64_t ldy2,
+                          const void* wl, const void* wr, float cl, float cr, int64_t lda, const void* sw, int slabs, int T_, int W,
+                          int kind, const void* router, const void* corr, void* idx, void* rwts, int E, int rtop, int norm, int smax,
+                          const void* zb, void* sg, const void* ids, const void* table, int64_t ldt, int vocab, int col0, int d,
+                          const void* wg, const void* wp, const void* wn, hipStream_t st) {
+  SandwichTail t{kind};
+  if (kind == 1) {
+    t.route.wr = (const bf16_t*)router, t.route.corr = (const float*)corr, t.route.idx = (int*)idx, t.route.wts = (float*)rwts;
+    t.route.E = E, t.route.top = rtop, t.route.norm = norm, t.route.smax = smax;
+    t.route.zb = (const float*)zb, t.route.sg = (float*)sg;
+  } else if (kind == 2) {
+    t.side = SideArgs{(const int64_t*)ids, table, ldt, vocab, col0, d, wg, wp, (const float*)wn};
+  } else {
+    throw std::runtime_error("sandwich_tail: kind");
+  }
+  launch_sandwich_add_norm(x, y, ldy, ey, place, wts, top, shared_, lds_, r, ldr, rb, wpost, add, wnext, h, ldh, eps, 1, nullptr, 0, y2,
+                           ldy2, wl, wr, cl, cr, lda, sw, slabs, T_, W, 0, t, st);
+}
+
+void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const void* ey, const void* place, const void* wts,
+                              int top, const void* shared_, int64_t lds_, const void* r, int64_t ldr, const void* rb,
+                              const void* wpost, const void* add, const void* wnext, void* h, int64_t ldh, float eps,
+                              int groups, const void* ident, int64_t ldi, const void* y2, int64_t ldy2, const void* wl,
+                              const void* wr, float cl, float cr, int64_t lda, const void* sw, int slabs, int T_, int W, int dt,
+                              hipStream_t st) {
+  launch_sandwich_add_norm(x, y, ldy, ey, place, wts, top, shared_, lds_, r, ldr, rb, wpost, add, wnext, h, ldh, eps, groups, ident, ldi,
+                           y2, ldy2, wl, wr, cl, cr, lda, sw, slabs, T_, W, dt, SandwichTail{}, st);
 }

@@ -166,10 +166,16 @@ class MoEFeedForward:
     """Feed-forward ``moe``."""
 
     @staticmethod
-    def forward(model: "LayeredLM", W, spec, h):
+    def route_args(W, spec) -> tuple:
+        """What ops.moe_router takes behind its rows."""
+        return W.router, W.correction, spec.top, spec.normalize, spec.score, W.bias, spec.shared_gate
+
+    @staticmethod
+    def forward(model: "LayeredLM", W, spec, h, route=None):
+        """``route``: the router's result over h, where a closing op has formed it."""
         dt = model.dtype
-        route = ops.moe_router(h, W.router, W.correction, spec.top, spec.normalize, spec.score, bias=W.bias,
-                               gate=spec.shared_gate)
+        if route is None:
+            route = ops.moe_router(h, *MoEFeedForward.route_args(W, spec))
         idx, wts = route[:2]
         sh = None
         if spec.act == "gelu":  # experts without a gate
@@ -841,19 +847,21 @@ class LayeredLM:
                 tail = (None, None)  # close the layer first, tap, then add / norm on their own
             else:
                 tail = (add, nxt)
-            side = L.side_gate is not None
             y = MIXERS[spec.mixer.kind].forward(self, r, L.mix, spec.mixer, h, inp, cu, kv_caches)
             gate = None if L.rg1_b is None else self.proj[:, L.mix.cols["rg"]:L.mix.cols["rg"] + W_]
-            after = (None, L.norm2) if spec.mlp is not None else ((None, None) if side else tail)
-            h = ops.sandwich_add_norm(x, y, gate, L.rg1_b, L.post1, eps, *after, dt, ng)
-            if spec.mlp is not None:
-                y = FFNS[spec.mlp.kind].forward(self, L.mlp, spec.mlp, h)
-                after = (None, None) if side else tail
+            side = (inp.input_ids, w.extra["side"], L.side_col, L.side_gate, L.side_proj, L.side_norm) if L.side_gate is not None else None
+            if spec.mlp is None:
+                h = ops.sandwich_add_norm(x, y, gate, L.rg1_b, L.post1, eps, *tail, dt, ng, side=side)
+            else:
+                moe = spec.mlp.kind == "moe"  # (its router reads h: part of the closing op where rows are few)
+                h = ops.sandwich_add_norm(x, y, gate, L.rg1_b, L.post1, eps, None, L.norm2, dt, ng,
+                                          route=MoEFeedForward.route_args(L.mlp, spec.mlp) if moe else None)
+                if moe:
+                    y = MoEFeedForward.forward(self, L.mlp, spec.mlp, *h)
+                else:
+                    y = FFNS[spec.mlp.kind].forward(self, L.mlp, spec.mlp, h)
                 gate = None if L.rg2_b is None else self.proj[:, L.rg2_col:L.rg2_col + W_]
-                h = ops.sandwich_add_norm(x, y, gate, L.rg2_b, L.post2, eps, *after, dt, ng)
-            if side:
-                h = ops.token_side_add(x, inp.input_ids, w.extra["side"], L.side_col, L.side_gate, L.side_proj,
-                                       L.side_norm, eps, *tail, dt)
+                h = ops.sandwich_add_norm(x, y, gate, L.rg2_b, L.post2, eps, *tail, dt, ng, side=side)
             if self.tap is not None:
                 self.tap(r, x)
                 h = ops.sandwich_add_norm(x, None, None, None, None, eps, add, nxt, dt, ng)

@@ -1834,10 +1834,37 @@ def diff_combine(O, lam, eps, mult, heads, kv_heads, vdim, out_dtype):
 
 
 # ------------------- blocks normed on both sides / token input / windowed sigmoid attention with pooled blocks / SSD
-def sandwich_add_norm(x, y, r, rb, wpost, eps, add, wnext, out_dtype, groups=1):
+TAIL_ROWS = 256  # rows up to which the next router or the token input rides in the closing op's launch, a workgroup per row
+
+
+def sandwich_add_norm(x, y, r, rb, wpost, eps, add, wnext, out_dtype, groups=1, route=None, side=None):
     """``y``: rows in the storage type, a :class:`MoEPending` (combined while it is read), a ``PairPending`` (the results
-    of two mixers, normed and joined while they are read) or a :class:`PartialSum` (summed while it is read)."""
+    of two mixers, normed and joined while they are read) or a :class:`PartialSum` (summed while it is read). ``route``, ``side``: in the
+    same launch where rows are few (csrc/sandwich.hip), else in one of their own."""
     T, W = x.shape
+    tail = None
+    if route is not None or side is not None:
+        _check(route is None or (side is None and wnext is not None), "route: over h, without a token input")
+        ok = (0 < T <= TAIL_ROWS and out_dtype == torch.bfloat16 and groups == 1 and W <= 2048 and not x.data_ptr() & 15
+              and not (isinstance(y, MoEPending) and y.ident is not None))
+        for t_ in (y.shared if isinstance(y, MoEPending) else y, r, getattr(y, "yl", None), getattr(y, "yr", None)):
+            ok = ok and (not isinstance(t_, torch.Tensor) or (not t_.data_ptr() & 7 and t_.stride(0) % 4 == 0))
+        for t_ in (rb, wpost, add, wnext, getattr(y, "wl", None), getattr(y, "wr", None)):
+            ok = ok and not _ptr(t_) & 15
+        if route is not None:
+            w_, corr, top_, normalize, score, bias, gate = route
+            E_ = w_.shape[0] - int(bool(gate))
+            tail = "route" if ok and W % 8 == 0 and E_ <= 128 and not w_.data_ptr() & 15 else None
+        else:
+            d_ = side[3].shape[0]
+            tail = "side" if (ok and d_ in (32, 64) and W % 256 == 0 and not (side[4].data_ptr() | side[5].data_ptr()) & 15
+                              and not side[3].data_ptr() & 7) else None
+        if tail is None and route is not None:
+            h = sandwich_add_norm(x, y, r, rb, wpost, eps, add, wnext, out_dtype, groups)
+            return h, moe_router(h, *route)
+        if tail is None:
+            sandwich_add_norm(x, y, r, rb, wpost, eps, None, None, out_dtype, groups)
+            return token_side_add(x, *side, eps, add, wnext, out_dtype)
     _rows(x, "x", dtype=torch.float32)
     _check(x.is_contiguous(), "x contiguous")
     _check(out_dtype in _DT, "storage type bf16 / fp32")
@@ -1886,6 +1913,31 @@ def sandwich_add_norm(x, y, r, rb, wpost, eps, add, wnext, out_dtype, groups=1):
         _check(wnext.numel() == W, "wnext [W]")
         h = torch.empty(T, W, dtype=out_dtype, device=x.device)
     dense = y if pend is None and part is None else None
+    if tail is not None:
+        rt, sd, res = (0,) * 10, (0,) * 9, h
+        if route is not None:
+            _check(w_.dtype == out_dtype and w_.is_contiguous() and w_.shape[1] == W and w_.is_cuda, "router [E (+ 1), W] in the storage type")
+            _route_args(E_, top_, corr, bias, score)
+            idx, wts = torch.empty(T, top_, dtype=torch.int32, device=x.device), torch.empty(T, top_, dtype=torch.float32, device=x.device)
+            sg = torch.empty(T, dtype=torch.float32, device=x.device) if gate else None
+            rt = (w_.data_ptr(), _ptr(corr), idx.data_ptr(), wts.data_ptr(), E_, top_, int(bool(normalize)), _SCORE[score], _ptr(bias), _ptr(sg))
+            res = h, ((idx, wts, sg) if gate else (idx, wts))
+        else:
+            ids, table, col0, gate_w, proj_w, norm_w = side
+            _side_check(ids, table, col0, gate_w, proj_w, norm_w, T, W, out_dtype)
+            sd = (ids.data_ptr(), table.data_ptr(), table.stride(0), table.shape[0], int(col0), gate_w.shape[0], gate_w.data_ptr(),
+                  proj_w.data_ptr(), norm_w.data_ptr())
+        lib().sandwich_tail(x.data_ptr(), part.buf.data_ptr() if part else _ptr(dense),
+                            W if part else (dense.stride(0) if dense is not None else 0), _ptr(pend.y) if pend else 0,
+                            _ptr(pend.place) if pend else 0, _ptr(pend.wts) if pend else 0, pend.top if pend else 0, _ptr(sh),
+                            sh.stride(0) if sh is not None else 0, _ptr(r) if y is not None else 0,
+                            r.stride(0) if (r is not None and y is not None) else 0, _ptr(rb), _ptr(wpost), _ptr(add), _ptr(wnext),
+                            _ptr(h), W, float(eps), _ptr(pair.yr) if pair else 0, pair.yr.stride(0) if pair else 0,
+                            _ptr(pair.wl) if pair else 0, _ptr(pair.wr) if pair else 0,
+                            *(pair.scales if pair and pair.scales else (0.0, 0.0)), W if add is not None and add.dim() == 2 else 0,
+                            _ptr(pend.shared_w) if pend else 0, part.S if part else 0, T, W, 1 if route is not None else 2, *rt, *sd,
+                            _stream())
+        return res
     lib().sandwich_add_norm(x.data_ptr(), part.buf.data_ptr() if part else _ptr(dense),
                             W if part else (dense.stride(0) if dense is not None else 0),
                             _ptr(pend.y) if pend else 0, _ptr(pend.place) if pend else 0,
@@ -1901,10 +1953,7 @@ def sandwich_add_norm(x, y, r, rb, wpost, eps, add, wnext, out_dtype, groups=1):
     return h
 
 
-def token_side_add(x, ids, table, col0, gate_w, proj_w, norm_w, eps, add, wnext, out_dtype):
-    T, W = x.shape
-    _rows(x, "x", dtype=torch.float32)
-    _check(x.is_contiguous(), "x contiguous")
+def _side_check(ids, table, col0, gate_w, proj_w, norm_w, T, W, out_dtype):
     d = gate_w.shape[0]
     _check(ids.dtype == torch.int64 and ids.is_contiguous() and ids.is_cuda and ids.numel() == T, "ids: int64 [T] cuda")
     _rows(table, "token table", dtype=out_dtype)
@@ -1915,6 +1964,14 @@ def token_side_add(x, ids, table, col0, gate_w, proj_w, norm_w, eps, add, wnext,
            "proj [W, d] in the storage type")
     _f32c(norm_w, "norm_w")
     _check(norm_w.numel() == W, "norm_w [W]")
+
+
+def token_side_add(x, ids, table, col0, gate_w, proj_w, norm_w, eps, add, wnext, out_dtype):
+    T, W = x.shape
+    _rows(x, "x", dtype=torch.float32)
+    _check(x.is_contiguous(), "x contiguous")
+    _side_check(ids, table, col0, gate_w, proj_w, norm_w, T, W, out_dtype)
+    d = gate_w.shape[0]
     if add is not None:
         _f32c(add, "add")
         _check(tuple(add.shape) == (T, W), "add fp32 [T, W]")

@@ -1040,11 +1040,19 @@ def _rms_parts(x, eps: float, groups: int):
     return (xg * torch.rsqrt(xg.pow(2).mean(-1, keepdim=True) + eps)).view(x.shape)
 
 
-def sandwich_add_norm(x, y, r, rb, wpost, eps: float, add, wnext, out_dtype, groups: int = 1):
+def sandwich_add_norm(x, y, r, rb, wpost, eps: float, add, wnext, out_dtype, groups: int = 1, route=None, side=None):
     """x fp32 [T, W], in place: with ``y`` [T, W], x += rms_norm(y * sigmoid(r + rb)) * wpost (``r`` [T, W] gate
     logits and ``rb`` [W] their bias, or None for no gate; ``wpost`` fp32 [W]); with ``add`` (fp32 [T, W] or [W]) x += add;
     with ``wnext`` (fp32 [W]) returns rms_norm(x) * wnext in ``out_dtype``, else None. ``groups``: both norms are taken in
-    that many equal consecutive parts of the row. ``y`` may be a :class:`PairPending`."""
+    that many equal consecutive parts of the row. ``y`` may be a :class:`PairPending`. ``route``: the arguments of :func:`moe_router`
+    behind its rows; returns (h, its result over h). ``side``: those of :func:`token_side_add` from ids to norm_w, taken between the
+    closing and ``add``."""
+    if route is not None:
+        h = sandwich_add_norm(x, y, r, rb, wpost, eps, add, wnext, out_dtype, groups)
+        return h, moe_router(h, *route)
+    if side is not None:
+        sandwich_add_norm(x, y, r, rb, wpost, eps, None, None, out_dtype, groups)
+        return token_side_add(x, *side, eps, add, wnext, out_dtype)
     if isinstance(y, PairPending):
         l, rr = y.yl.float(), y.yr.float()
         y = y.scales[0] * l + y.scales[1] * rr if y.scales is not None else 0.5 * (_rms_parts(l, eps, 1) * y.wl.float() + _rms_parts(rr, eps, 1) * y.wr.float())
