@@ -2333,6 +2333,30 @@ int launch_gemm_qkv(const void* x, int64_t ldx, const void* w, int64_t ldw, cons
   }
   int tsel = nt_hint >> 8, s = split_hint;
   gemm_tiled_plan(M, N, K, &tsel, &s, false);
+  if (tsel == 4) {  // 256 x 256 tiles, and what they leave over as launch_gemm has it
+    if ((qe.do_rope && qe.style != 1) || 256 % qe.D || !gemm_quad_ok(N, K, ldx, ldw, 256, y, ldy, 2, false)) return -1;
+    const GemmCut cut = gemm_cut(M, N, K, false);
+    const int rows = cut.rows ? cut.rows : M, cols = cut.cols ? cut.cols : N;
+    launch_gemm_quad(0, (const bf16_t*)x, ldx, (const bf16_t*)w, ldw, (const bf16_t*)bias, (bf16_t*)y, ldy, rows, cols, K, 0, 0,
+                     g_big_group_m, tiles_of(rows, cols, 256, 256), PpGroup{}, st, &qe);
+    if (rows == M && cols == N) return 0;
+    QkvEpi re = qe;  // the rest: its own rows, or the heads from column `cols` on
+    if (re.pos) re.pos += rows < M ? rows : 0;
+    if (re.slot) re.slot += rows < M ? rows : 0;
+    if (cols < N) re.nh -= cols / qe.D;
+    const bf16_t* rx = (const bf16_t*)x + (rows < M ? rows * ldx : 0);
+    bf16_t* ry = (bf16_t*)y + (rows < M ? rows * ldy : cols);
+    const bf16_t* rw = (const bf16_t*)w + (cols < N ? (int64_t)cols * ldw : 0);
+    const bf16_t* rb = bias ? (const bf16_t*)bias + (cols < N ? cols : 0) : nullptr;
+    const int m = rows < M ? M - rows : M, n = cols < N ? N - cols : N;
+    int nt = cut.hint, sp = 1;
+    if (!nt) {  // up to 64 rows: the decode kernel where its plan is unsplit, else 64 x 64 tiles
+      gemm_static_plan(m, n, K, false, false, ws_bytes, &nt, &sp);
+      if (!((nt >> 8) & kDecHint) || sp > 1) nt = 3 << 8;
+    }
+    launch_tiled(rx, ldx, rw, ldw, rb, ry, ldy, m, n, K, 0, 0, nt >> 8, 1, workspace, ws_bytes, false, st, nullptr, &re);
+    return 0;
+  }
   if ((tsel & 15) == 4 || (tsel & 128)) return -1;
   int bm, bn;
   tile_dims(tsel & 15, &bm, &bn);

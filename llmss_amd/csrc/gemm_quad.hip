@@ -22,11 +22,18 @@
 
 // GLU 1: SiLU gates, 2: the tanh form of GELU, 8192 x 11264 x 2048 with its gate 323 us (the product alone 306, with a launch of its own for the
 // gate 356; 64 rows 15.5 and 17.3, one row 11.2 and 13.0)
-template <int GRP, int GLU>
+// QKV: the query / key / value product, its rows turned (neighbouring pairs, or not at all) and its keys and values written to the paged cache on
+// the way out (common.h QkvEpi). The wave's 128 columns go out as one image of bf16 - the numbers are rounded before they are turned, as where
+// the rotation is a launch of its own - whose 16 pieces of a row are one lane's columns throughout; where a row lies in the cache is
+// looked up once a row and kept in the ring's fifth buffer.
+// Against the product and a rotation of its own, which reads and writes all of it again (us): 8192 x 12288 x 4096 676 -> 621, 3999 rows 343 ->
+// 315; 8192 x 4800 x 1600 without a rotation 159 -> 140.
+template <int GRP, int GLU, bool QKV = false>
 __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restrict__ X, int64_t ldx,
                                                            const bf16_t* __restrict__ W, int64_t ldw,
                                                            const bf16_t* __restrict__ bias, bf16_t* __restrict__ Y,
-                                                           int64_t ldy, int M, int N, int K, int act, int group_m, PpGroup gr) {
+                                                           int64_t ldy, int M, int N, int K, int act, int group_m, PpGroup gr, QkvEpi qe) {
+  static_assert(!QKV || (GRP == 0 && GLU == 0), "QKV: plain products");
   // a ring of five buffers, each 64 of k (128 bytes, a line) of 256 rows: X of step 0, W of step 0, X of step 1, ...
   constexpr int BUF = 32768, NB = 5, QA = 6;
   constexpr bool GATHER = GRP == 1 || GRP == 3;
@@ -170,6 +177,81 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
   // 2 p and 2 p + 1 (GLU: four gates and their four ups). The bf16 stores bypass the caches' replacement, which keeps X and W of the tiles
   // to come: 632 -> 606 us at 8192 x 12288 x 4096, 1.5 % of a prompt step.
   char* img = smem + w * BUF;
+  if constexpr (QKV) {
+    const int D = qe.D, nq = qe.nh * D, nqk = nq + qe.nkv * D, rh = qe.rot >> 1, nw0 = n0 + wc * 128, mw0 = m0 + wr * 128;
+    const bool rope = qe.do_rope != 0 && nw0 < nqk, cached = qe.kc != nullptr && nw0 + 127 >= nq;
+    int* rpos = reinterpret_cast<int*>(smem + 4 * BUF + w * 2048);                  // [128] the rows' positions
+    int64_t* rbase = reinterpret_cast<int64_t*>(smem + 4 * BUF + w * 2048 + 512);  // [128] and first numbers in the cache, -1: not cached
+    int64_t ps[2] = {0, 0}, sl[2] = {-1, -1};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int m = min(mw0 + lane + 64 * i, M - 1);
+      if (rope) ps[i] = qe.pos[m];
+      if (cached) sl[i] = qe.slot[m];
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int n = nw0 + 32 * p + 8 * g;
+      float b[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (bias && n < N) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) b[i] = bf2f(bias[n + i]);
+      }
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt) {
+        u16x8 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          o[i] = f2bf(acc[2 * p][mt][i] + b[i]);
+          o[4 + i] = f2bf(acc[2 * p + 1][mt][i] + b[4 + i]);
+        }
+        *reinterpret_cast<u16x8*>(img + (16 * mt + li) * 256 + (((4 * p + g) ^ li) << 4)) = o;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      rpos[lane + 64 * i] = (int)ps[i];
+      const unsigned u = (unsigned)sl[i], bs = (unsigned)qe.block_size, blk = u / bs;
+      rbase[lane + 64 * i] = sl[i] < 0 ? -1 : ((int64_t)blk * qe.nkv * bs + (u - blk * bs)) * D;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int c = lane & 15, n = nw0 + 8 * c, d = n % D;
+    const bool is_v = n >= nqk, turn = rope && !is_v && d < qe.rot, keep = cached && n >= nq && n < N;
+    bf16_t* const cache = (is_v ? qe.vc : qe.kc) + (int64_t)((n - (is_v ? nqk : nq)) / D) * qe.block_size * D + d;
+    const int a = turn ? d >> 1 : 0;  // (columns that do not turn read an angle that nobody uses)
+    constexpr int U = 4;
+#pragma unroll 1
+    for (int i0 = 0; i0 < 32; i0 += U) {
+      f32x4 cs[U], sn[U];
+      if (rope) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int64_t at = (int64_t)rpos[4 * (i0 + u) + g] * rh + a;
+          cs[u] = *reinterpret_cast<const f32x4*>(qe.cos_t + at);
+          sn[u] = *reinterpret_cast<const f32x4*>(qe.sin_t + at);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int r = 4 * (i0 + u) + g, m = mw0 + r;
+        u16x8 o = *reinterpret_cast<const u16x8*>(img + r * 256 + ((c ^ (r & 15)) << 4));
+        if (turn) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float x = bf2f(o[2 * i]), y = bf2f(o[2 * i + 1]);
+            o[2 * i] = f2bf(x * cs[u][i] - y * sn[u][i]);
+            o[2 * i + 1] = f2bf(y * cs[u][i] + x * sn[u][i]);
+          }
+        }
+        if (m >= M || n >= N) continue;
+        __builtin_nontemporal_store(o, reinterpret_cast<u16x8*>(Y + (int64_t)m * ldy + n));
+        const int64_t base = rbase[r];
+        if (keep && base >= 0) __builtin_nontemporal_store(o, reinterpret_cast<u16x8*>(cache + base));
+      }
+    }
+    return;
+  }
   auto flush = [&](int c0) {  // the image is columns c0 .. c0 + 63 of the output
     if constexpr (GRP == 2) {
       const int n = c0 + 4 * li;
@@ -292,9 +374,10 @@ bool gemm_quad_ok(int N, int K, int64_t ldx, int64_t ldw, int64_t rows, const vo
 
 void launch_gemm_quad(int grp, const bf16_t* X, int64_t ldx, const bf16_t* W, int64_t ldw, const bf16_t* bias, bf16_t* Y,
                       int64_t ldy, int M, int N, int K, int act, int glu, int group_m, unsigned nwg, const PpGroup& gr,
-                      hipStream_t st) {
-#define LAUNCH_Q(G_, U_) gemm_quad_kernel<G_, U_><<<nwg, 256, 0, st>>>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, act, group_m, gr)
-  if (grp == 2) LAUNCH_Q(2, 0);
+                      hipStream_t st, const QkvEpi* qe) {
+#define LAUNCH_Q(G_, U_) gemm_quad_kernel<G_, U_><<<nwg, 256, 0, st>>>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, act, group_m, gr, QkvEpi{})
+  if (qe) gemm_quad_kernel<0, 0, true><<<nwg, 256, 0, st>>>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, act, group_m, gr, *qe);
+  else if (grp == 2) LAUNCH_Q(2, 0);
   else if (grp == 3) LAUNCH_Q(3, 1);
   else if (grp == 1 && glu) LAUNCH_Q(1, 1);
   else if (grp == 1) LAUNCH_Q(1, 0);

@@ -214,13 +214,17 @@ class DecoderLM:
         split K, whose slabs rope_cache sums on the way; over 175 random layers of 1 - 64 rows one launch takes 0.87 of their time, and 1.07
         at worst (us, two and one: 4800 x 1600, one row 8.9 and 6.3, 64 rows 13.4 and 9.7; 12288 x 4096 23.6 and 19.9, 28.7 and 24.1;
         6144 x 4096 14.6 and 11.7, 18.3 and 17.7; 3072 x 1024 6.8 and 4.8, 10.4 and 6.7; 15360 x 5120 31.2 and 27.5, 42.0 and 35.2; 10240 x
-        8192 32.2 and 32.6, 16 rows 34.3 and 32.6; 1536 x 5040, 15 rows 11.9 and 12.7)."""
+        8192 32.2 and 32.6, 16 rows 34.3 and 32.6; 1536 x 5040, 15 rows 11.9 and 12.7). Prompts: where the two launches would not split K
+        either and from 128 rows on (66 rows of 12288 x 4096 39.2 and 39.5; 256 rows of 12288 x 4096: 47.5 in two with K split, 62.9 in one without). 12288 x 4096, 1024 rows 109 and 100,
+        1773 rows 192 and 177, 8192 rows 676 and 621; 4800 x 1600, 512 rows 32.6 and 25.5, 2048 rows 49 and 42, 8192 rows 159 and 140."""
         lib = _hip_ops().lib()
         if lib.gemm_tuned_get(M, N, K, False, 3) is not None:
             return 0, 0
-        if M > 64 or self.cfg.head_dim % 8 or lib.gemm_tuned_get(M, N, K, False, 0) is not None:
+        if self.cfg.head_dim % 8 or lib.gemm_tuned_get(M, N, K, False, 0) is not None:
             return None
-        nt, split = lib.gemm_plan(M, N, K, False, False, False)
+        nt, split = lib.gemm_plan(M, N, K, False, False, M > 64)
+        if M > 64:
+            return (nt, 1) if split <= 1 and nt >> 8 and M >= 128 else None
         return (nt, split) if nt >> 8 & 1024 and split == 1 else None  # (the hint bit of csrc/gemm_dec.hip)
 
     def _qkv_rope_cache(self, L, y, inp: StepInput, kc, vc):

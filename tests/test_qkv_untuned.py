@@ -42,3 +42,36 @@ def test_one_launch_and_two(preset, over, M, monkeypatch):
             assert ((a.double() - b.double()).abs() <= lim).all()
         else:
             assert torch.equal(a, b)
+
+
+# 256 x 256 tiles: whole and partial ones, rows or columns left over to other tiles (up to 64 rows: the decode kernel), heads of half a wave's
+# columns to all of a tile's, one key head, pairs turned in part or not at all, rows that are not cached
+@pytest.mark.parametrize("M,K,nh,nkv,D,rot", [(1, 64, 2, 1, 128, 128), (300, 128, 3, 3, 64, 64), (257, 192, 2, 2, 256, 64), (520, 64, 5, 1, 64, 0),
+                                              (8261, 256, 8, 4, 128, 128), (8230, 1024, 8, 4, 128, 128), (8230, 256, 16, 8, 64, 64),
+                                              (4352, 1024, 32, 2, 128, 32)])
+def test_tiles_of_prompts(M, K, nh, nkv, D, rot):
+    from llmss_amd.ops import hip
+    g = torch.Generator().manual_seed(M)
+    N = (nh + 2 * nkv) * D
+    x, w = torch.randn(M, K, generator=g).bfloat16().cuda(), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16().cuda()
+    b = torch.randn(N, generator=g).bfloat16().cuda() if M % 2 else None
+    pos = torch.randint(0, 90, (M,), generator=g).cuda()
+    ang = torch.rand(90, max(rot // 2, 4), generator=g).cuda() * 6
+    cos, sin = ang.cos(), ang.sin()
+    nb = -(-M // 16) + 1
+    slots = torch.randperm(nb * 16, generator=g)[:M].cuda()
+    slots[M // 3] = -1
+    res = []
+    for one in (True, False):
+        kc, vc = (torch.zeros(nb, nkv, 16, D, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        if one:
+            y = hip.linear_qkv(x, w, b, pos, cos, sin, kc, vc, slots, nh, nkv, D, rot, "gptj", rot > 0, 4 << 8, 1)
+            assert y is not None
+        else:
+            y = hip.rope_cache(hip.linear(x, w, b, nt_hint=4 << 8, split_hint=1), pos, cos, sin, kc, vc, slots, nh, nkv, D, rot, "gptj", rot > 0)
+        res.append((y, kc, vc))
+    for a, c in zip(*res):  # bf16 rows turned in fp32, from sums that may be in another order: a rounding each, of a number and its partner
+        assert ((a.double() - c.double()).abs() <= 2.0 ** -7 * (c.double().abs() + (c.double().abs().amax() if rot else 0.0)) + 1e-5).all()
+    assert (res[0][1][nb - 1].abs().sum() > 0) == (res[1][1][nb - 1].abs().sum() > 0)
+    # halves that turn against each other are not this form's
+    assert rot == 0 or hip.linear_qkv(x, w, b, pos, cos, sin, None, None, None, nh, nkv, D, rot, "neox", True, 4 << 8, 1) is None
