@@ -2,11 +2,13 @@
 //
 // Bound by the experts' weights, each read once: a step of 33 tokens over 32 experts of 2048 x 768 reads 300 MB. A workgroup takes two
 // groups of 16 weight rows - 16 gate and their 16 up rows, or 32 rows of one matrix - against a tile's rows; its four waves
-// split K and meet in LDS, and a wave asks for eight steps of 32 at once (24 KB in flight a wave) straight into the matrix
-// instructions' operands: no staging, no barrier before the end, two steps to a 128-byte line. The 64-row tiles that larger steps
+// split K and meet in LDS, and a wave asks for four steps of 64 at once (24 KB in flight a wave) straight into the matrix
+// instructions' operands: no staging, no barrier before the end. The 64-row tiles that larger steps
 // take keep one step of 64 in flight and four waves behind barriers.
 // All products of a layer, weights from memory, against those (us): 32 experts of 2048 x 768, 4 rows each, 81 -> 75; 16 of 1024 x 512
 // 37 -> 25; 8 of 4096 x 2048 120 -> 86, one row each 110 -> 63. A tile more for an expert reads its weights again.
+// Whole lines past the caches' replacement (md_products64) against half lines of 16 rows: 217 MB of gate and up rows (33 tokens, 32 experts and a
+// shared one) 53 -> 40 us, 5.4 TB/s, 105 MB of down rows 31.5 -> 25.8; reads alone, 210 MB, 36.9 and 32.5 us, half lines past the caches 38.3.
 //
 // Who chose whom: up to MD_PAIRS (token, expert) pairs a workgroup finds its expert's pairs itself, with one look at all choices, and the
 // rows of the results are the pairs' own numbers: no grouping launch before the products. Beyond that it reads moe.hip's tile list, 16 rows a tile. The shared expert's products, and
@@ -46,7 +48,58 @@ struct MoeDecArgs {
   float slimit;
 };
 
-// G groups of 16 rows against the two groups of weight rows, steps [s, s1) of 32
+// G groups of 16 rows against the two groups of weight rows, steps [s, s1) of 64: a load takes whole lines, 128 bytes of eight rows (lane l: piece
+// l / 8 of row l % 8), past the caches' replacement - every weight is read once. The matrix instructions want 16 rows side by side: of two
+// such loads, lanes 0 - 7 and 8 - 15 of every 16 change places, and lane (li, g) holds pieces 2 g and 2 g + 1 of row li. wa: this lane's place
+// in rows 0 - 7 and in rows 8 - 15
+template <int G, int U>
+__device__ __forceinline__ void md_products64(const bf16_t* const (&wa)[2], const bf16_t* const (&wb)[2], const bf16_t* const (&x)[G], int s,
+                                              int s1, f32x4 (&aa)[G], f32x4 (&ab)[G]) {
+#pragma unroll
+  for (int q = 0; q < G; ++q) aa[q] = ab[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto turn = [](const s16x8& lo, const s16x8& hi, s16x8& even, s16x8& odd) {
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    const i32x4 l = __builtin_bit_cast(i32x4, lo), h = __builtin_bit_cast(i32x4, hi);
+    i32x4 e, o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      e[i] = __builtin_amdgcn_update_dpp(l[i], h[i], 0x128, 0xf, 0xc, false);  // (the row of 16 turned by 8, into its lanes 8 - 15)
+      o[i] = __builtin_amdgcn_update_dpp(h[i], l[i], 0x128, 0xf, 0x3, false);
+    }
+    even = __builtin_bit_cast(s16x8, e), odd = __builtin_bit_cast(s16x8, o);
+  };
+  for (; s < s1; s += U) {
+    s16x8 fx[G][U][2], fa[U][2], fb[U][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = min(s + u, s1 - 1) * 64;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        fa[u][i] = __builtin_nontemporal_load(reinterpret_cast<const s16x8*>(wa[i] + k));
+        fb[u][i] = __builtin_nontemporal_load(reinterpret_cast<const s16x8*>(wb[i] + k));
+#pragma unroll
+        for (int q = 0; q < G; ++q) fx[q][u][i] = *reinterpret_cast<const s16x8*>(x[q] + k + 8 * i);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (s + u < s1) {
+        s16x8 a0, a1, b0, b1;
+        turn(fa[u][0], fa[u][1], a0, a1);
+        turn(fb[u][0], fb[u][1], b0, b1);
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+          aa[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, fx[q][u][0], aa[q], 0, 0, 0);
+          ab[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0, fx[q][u][0], ab[q], 0, 0, 0);
+          aa[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, fx[q][u][1], aa[q], 0, 0, 0);
+          ab[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1, fx[q][u][1], ab[q], 0, 0, 0);
+        }
+      }
+  }
+}
+
+// The same in steps of 32, straight in the operands' places (K no multiple of 64)
 template <int G, int U>
 __device__ __forceinline__ void md_products(const bf16_t* wa, const bf16_t* wb, const bf16_t* const (&x)[G], int s, int s1, f32x4 (&aa)[G],
                                             f32x4 (&ab)[G]) {
@@ -104,7 +157,7 @@ __device__ __forceinline__ int2 md_extra(const MoeDecArgs& p, int j, int* cnt) {
   return found;
 }
 
-template <int MODE, bool LIST>
+template <int MODE, bool LIST, bool LINES>
 __global__ __launch_bounds__(256, 4) void moe_dec_kernel(MoeDecArgs p) {
   constexpr int BN = MODE == MD_GLU ? 16 : 32, G = LIST ? 1 : 2;
   __shared__ __attribute__((aligned(16))) float part[4][2][16 * G][20];  // (rows of 20: 16-byte places, spread over the banks)
@@ -182,39 +235,50 @@ __global__ __launch_bounds__(256, 4) void moe_dec_kernel(MoeDecArgs p) {
   auto pair_of = [&](int r) { return LIST || shared_ ? row0 + r : list[r]; };  // the row's place in the results
   auto x_of = [&](int r) {
     const int q = pair_of(min(r, rows - 1));
-    return x + (int64_t)(MODE == MD_DOWN || shared_ ? q : LIST ? p.order[q] / p.top : q / p.top) * ldx + 8 * g;
+    return x + (int64_t)(MODE == MD_DOWN || shared_ ? q : LIST ? p.order[q] / p.top : q / p.top) * ldx + (LINES ? 16 : 8) * g;
   };
-  const bf16_t *wa, *wb;
-  if (MODE == MD_GLU && !plain) {
-    const int n = min(n0 + li, N - 1);
-    if (inter) {
-      wa = W + (int64_t)((n >> 4) * 32 + (n & 15)) * K;
-      wb = wa + (int64_t)16 * K;
-    } else {
-      wa = W + (int64_t)n * K;
-      wb = W2 + (int64_t)n * K;
-    }
-  } else {
-    wa = W + (int64_t)min(n0 + li, N - 1) * K;
-    wb = W + (int64_t)min(n0 + 16 + li, N - 1) * K;
-  }
-  wa += 8 * g, wb += 8 * g;
-  const int nk = K >> 5, per = ((nk + 7) >> 3) * 2, s0 = w * per, s1 = min(nk, s0 + per);  // (a wave starts at a line)
+  auto wa_of = [&](int r) {  // row r of the first group of weight rows, and of the second
+    const int n = min(n0 + r, N - 1);
+    return W + (int64_t)(MODE == MD_GLU && !plain && inter ? (n >> 4) * 32 + (n & 15) : n) * K;
+  };
+  auto wb_of = [&](int r) {
+    if (MODE == MD_GLU && !plain) return inter ? wa_of(r) + (int64_t)16 * K : W2 + (int64_t)min(n0 + r, N - 1) * K;
+    return W + (int64_t)min(n0 + 16 + r, N - 1) * K;
+  };
   auto keep = [&](int q, const f32x4& a, const f32x4& b) {
     *reinterpret_cast<f32x4*>(&part[w][0][16 * q + li][4 * g]) = a;
     *reinterpret_cast<f32x4*>(&part[w][1][16 * q + li][4 * g]) = b;
   };
-  if (LIST || rows <= 16) {
-    f32x4 aa[1], ab[1];
-    const bf16_t* const xs[1] = {x_of(li)};
-    md_products<1, 8>(wa, wb, xs, s0, s1, aa, ab);
-    keep(0, aa[0], ab[0]);
-  } else if constexpr (G == 2) {
-    f32x4 aa[2], ab[2];
-    const bf16_t* const xs[2] = {x_of(li), x_of(16 + li)};
-    md_products<2, 5>(wa, wb, xs, s0, s1, aa, ab);
-    keep(0, aa[0], ab[0]);
-    keep(G - 1, aa[1], ab[1]);
+  f32x4 aa[G], ab[G];
+  if constexpr (LINES) {
+    const int nk = K >> 6, per = (nk + 3) >> 2, s0 = w * per, s1 = min(nk, s0 + per), r8 = lane & 7, c8 = (lane >> 3) * 8;
+    const bf16_t* const wa[2] = {wa_of(r8) + c8, wa_of(8 + r8) + c8};
+    const bf16_t* const wb[2] = {wb_of(r8) + c8, wb_of(8 + r8) + c8};
+    if (LIST || rows <= 16) {
+      f32x4 a1[1], b1[1];
+      const bf16_t* const xs[1] = {x_of(li)};
+      md_products64<1, 4>(wa, wb, xs, s0, s1, a1, b1);
+      keep(0, a1[0], b1[0]);
+    } else if constexpr (G == 2) {
+      const bf16_t* const xs[2] = {x_of(li), x_of(16 + li)};
+      md_products64<2, 2>(wa, wb, xs, s0, s1, aa, ab);
+      keep(0, aa[0], ab[0]);
+      keep(G - 1, aa[G - 1], ab[G - 1]);
+    }
+  } else {
+    const int nk = K >> 5, per = ((nk + 7) >> 3) * 2, s0 = w * per, s1 = min(nk, s0 + per);  // (a wave starts at a line)
+    const bf16_t *wa = wa_of(li) + 8 * g, *wb = wb_of(li) + 8 * g;
+    if (LIST || rows <= 16) {
+      f32x4 a1[1], b1[1];
+      const bf16_t* const xs[1] = {x_of(li)};
+      md_products<1, 8>(wa, wb, xs, s0, s1, a1, b1);
+      keep(0, a1[0], b1[0]);
+    } else if constexpr (G == 2) {
+      const bf16_t* const xs[2] = {x_of(li), x_of(16 + li)};
+      md_products<2, 5>(wa, wb, xs, s0, s1, aa, ab);
+      keep(0, aa[0], ab[0]);
+      keep(G - 1, aa[G - 1], ab[G - 1]);
+    }
   }
   __syncthreads();
   const int c = threadIdx.x & 15;
@@ -248,6 +312,20 @@ __global__ __launch_bounds__(256, 4) void moe_dec_kernel(MoeDecArgs p) {
   }
 }
 
+template <bool LIST>
+static void launch_moe_dec_t(int mode, bool lines, dim3 g, const MoeDecArgs& a, hipStream_t st) {
+#define MD_LAUNCH(M_)                                                       \
+  do {                                                                      \
+    if (lines) moe_dec_kernel<M_, LIST, true><<<g, 256, 0, st>>>(a);        \
+    else moe_dec_kernel<M_, LIST, false><<<g, 256, 0, st>>>(a);             \
+  } while (0)
+  if (mode == MD_GLU) MD_LAUNCH(MD_GLU);
+  else if (mode == MD_GELU) MD_LAUNCH(MD_GELU);
+  else MD_LAUNCH(MD_DOWN);
+#undef MD_LAUNCH
+  HIP_CHECK_LAUNCH();
+}
+
 // mode 0: act [pairs, N] = glu(X W^T, X W2^T) (W2 null: gate and up rows of W [E, 2 N, K] in alternating groups of 16), 1: gelu(X W^T),
 // rows of X gathered by token; 2: C = X W^T in fp32, rows of X in the results' order. With a tile list (meta, order, at most maxt tiles):
 // results in expert order; without: idx [T, top], results in the pairs' order, `place` [T * top] for modes 0 and 1.
@@ -269,11 +347,7 @@ void launch_moe_dec(int mode, const void* X, int64_t ldx, const void* W, const v
   if (list) {
     if (maxt > 65535) throw std::runtime_error("moe_dec: too many row tiles");
     if (sW) throw std::runtime_error("moe_dec: no shared expert beside a tile list");
-    dim3 g((N + bn - 1) / bn, maxt);
-    if (mode == MD_GLU) moe_dec_kernel<MD_GLU, true><<<g, 256, 0, st>>>(a);
-    else if (mode == MD_GELU) moe_dec_kernel<MD_GELU, true><<<g, 256, 0, st>>>(a);
-    else moe_dec_kernel<MD_DOWN, true><<<g, 256, 0, st>>>(a);
-    HIP_CHECK_LAUNCH();
+    launch_moe_dec_t<true>(mode, K % 64 == 0, dim3((N + bn - 1) / bn, maxt), a, st);
     return;
   }
   const int64_t P = (int64_t)T_ * top;
@@ -289,9 +363,5 @@ void launch_moe_dec(int mode, const void* X, int64_t ldx, const void* W, const v
     wgs += (int64_t)((T_ + MD_ROWS - 1) / MD_ROWS) * (((mode == MD_GLU ? sN : N) + bn - 1) / bn + (sE + 31) / 32);
   }
   if (wgs > 0x7fffffff) throw std::runtime_error("moe_dec: too many workgroups");
-  dim3 g((unsigned)wgs);
-  if (mode == MD_GLU) moe_dec_kernel<MD_GLU, false><<<g, 256, 0, st>>>(a);
-  else if (mode == MD_GELU) moe_dec_kernel<MD_GELU, false><<<g, 256, 0, st>>>(a);
-  else moe_dec_kernel<MD_DOWN, false><<<g, 256, 0, st>>>(a);
-  HIP_CHECK_LAUNCH();
+  launch_moe_dec_t<false>(mode, K % 64 == 0 && (!sW || sK % 64 == 0), dim3((unsigned)wgs), a, st);
 }
