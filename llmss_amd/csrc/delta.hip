@@ -69,7 +69,7 @@ __global__ __launch_bounds__(512) void delta_step_kernel(DeltaStepArgs A) {
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int r = rg + u * RG;
-    s[u] = (pos > 0 && rg < RG && r < dim) ? *reinterpret_cast<const f32x4*>(sp + (int64_t)r * vdim) : f32x4{0.f, 0.f, 0.f, 0.f};
+    s[u] = (pos > 0 && rg < RG && r < dim) ? __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(sp + (int64_t)r * vdim)) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const float zb = El<T>::ld((const T*)A.b + (int64_t)t * A.ldab + h);
   const float za = El<T>::ld((const T*)A.a + (int64_t)t * A.ldab + h) + A.dt_bias[h];
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(512) void delta_step_kernel(DeltaStepArgs A) {
         f32x4 x;
 #pragma unroll
         for (int i = 0; i < 4; ++i) x[i] = fmaf(g, s[u][i], kd * u4[i]);
-        *reinterpret_cast<f32x4*>(sp + (int64_t)r * vdim) = x;
+        __builtin_nontemporal_store(x, reinterpret_cast<f32x4*>(sp + (int64_t)r * vdim));
       }
     }
   }
