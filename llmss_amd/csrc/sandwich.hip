@@ -280,14 +280,13 @@ struct SideTail : SideArgs {
 // The same for rows of up to 4096 and a norm of one part: a thread keeps NC times four columns of everything in registers, all loads are
 // issued before the first sum, and only two sums pass through LDS. The kernel above asks for the stream and the weights behind the
 // first sum, a round trip more. us, plain rows / gated / four experts' rows: 33 x 2048 5.0 / 5.3 / 5.5 -> 4.3 / 4.7 / 4.8, 8192 x 2048
-// 36.3 / 42.4 / 84.7 -> 36.4 / 43.9 / 72.6, 8192 x 1024 24.8 / 28.3 / 37.8 -> 20.6 / 24.5 / 34.1. With eight columns a thread the
-// registers leave half the waves: 8192 x 4096 84.6 -> 106, so more than 512 such rows keep the kernel above.
+// 8192 x 1024 24.8 / 28.3 / 37.8 -> 20.6 / 24.5 / 34.1. NT: the stream, y and what is read with it past the caches' replacement.
 // With a tail, one launch against two, in a decode step (kernel times, us): the router of 17 outputs over 8 rows of 1024 11.0 -> 7.9, of 32
 // over 33 rows of 2048 13.8 -> 11.1, the token input of 32 numbers 17.1 -> 14.7 (each of 33 workgroups draws its 256 KB of weights through one
 // CU). A tail's kernel for every form of y at once, its loads behind a branch a column: 8.7, 11.3 and 16.2.
 // FORM: what y is, where a launch is a chain that fetches its code as it goes (tails); else found at run time
 enum { Y_ANY = -1, Y_NONE, Y_ROWS, Y_SLABS, Y_PAIR, Y_EXPERTS };
-template <typename T, int NC, typename TAIL, int FORM>
+template <typename T, int NC, typename TAIL, int FORM, bool NT = false>
 __global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p, TAIL a) {
   constexpr bool ROUTE = TAIL::kind == 1, SIDE = TAIL::kind == 2;
   static_assert(TAIL::kind == 0 || (NC == 1 && sizeof(T) == 2), "tails: bf16 rows, four columns a thread");
@@ -315,7 +314,14 @@ __global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p, TAIL
 // before the next one is issued
 #define LOAD(...) _Pragma("unroll") for (int i = 0; i < NC; ++i) { __VA_ARGS__; }
   typedef typename std::conditional<sizeof(T) == 2, u16x4, f32x4>::type Raw;
-  auto raw = [](const void* q, int64_t o) { return *reinterpret_cast<const Raw*>((const T*)q + o); };
+  auto raw = [](const void* q, int64_t o) {
+    const Raw* r = reinterpret_cast<const Raw*>((const T*)q + o);
+    return NT ? __builtin_nontemporal_load(r) : *r;
+  };
+  auto wide = [](const float* q) {
+    const f32x4* r = reinterpret_cast<const f32x4*>(q);
+    return NT ? __builtin_nontemporal_load(r) : *r;
+  };
   auto num = [](const Raw& q) {
     if constexpr (sizeof(T) == 2) return f32x4{bf2f(q[0]), bf2f(q[1]), bf2f(q[2]), bf2f(q[3])};
     else return q;
@@ -375,7 +381,7 @@ __global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p, TAIL
   };
   if constexpr (ROUTE) eg = a.E + (a.sg ? 1 : 0);
   if constexpr (SIDE) id = a.ids[t];
-  LOAD(x[i] = ld4(xr + at[i]))
+  LOAD(x[i] = wide(xr + at[i]))
   if (p.wnext) LOAD(wn[i] = ld4(p.wnext + at[i]))
   if (p.add) LOAD(ad[i] = ld4(p.add + (int64_t)t * p.lda + at[i]))
   if (!has_y) load_tail();
@@ -428,7 +434,7 @@ __global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p, TAIL
           const int jj = min(j0 + j, p.top - 1);
           const float* er = p.ey + (int64_t)p.place[(int64_t)t * p.top + jj] * W;
           wj[j] = p.wts ? p.wts[(int64_t)t * p.top + jj] : 1.0f;
-          LOAD(e[j][i] = ld4(er + at[i]))
+          LOAD(e[j][i] = wide(er + at[i]))
         }
         if (j0 == 0) load_tail();
 #pragma unroll
@@ -492,7 +498,7 @@ __global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p, TAIL
     EACH(for (int e = 0; e < 4; ++e) x[i][e] = fmaf(y[e] * inv, swn[e], x[i][e]))
   }
   if (p.add) EACH(for (int e = 0; e < 4; ++e) x[i][e] += ad[i][e])
-  if (has_y || p.add || SIDE) EACH(st4(xr + col[i], x[i]))
+  if (has_y || p.add || SIDE) EACH(if constexpr (NT) __builtin_nontemporal_store(x[i], reinterpret_cast<f32x4*>(xr + col[i])); else st4(xr + col[i], x[i]))
   if (!p.wnext) return;
   float ss = 0.f;
   EACH(for (int e = 0; e < 4; ++e) ss = fmaf(x[i][e], x[i][e], ss))
@@ -587,10 +593,13 @@ static void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const 
                    al16(wl) && al16(wr);
   const size_t lds = ((size_t)W + (groups > 1 ? groups : 0)) * 4;
   const int th = T_ <= 512 && W > 1024 ? 512 : 256;  // few rows: more waves to a row
-  // (identity experts and norms in parts keep the general kernel, and so do many rows wider than 1280 unless experts' rows are summed: 1600 -
-  // 8192 rows of 1536 - 2048 in registers took 1.00 - 1.04 of the general kernel's time, gated 1.01 - 1.05, none 1.05 - 1.10, experts' 0.92 - 0.94,
-  // but 1551 with one expert each 1.20: two waves of eight-wave workgroups where the general kernel's four fit at once)
-  const bool rows = vec && groups == 1 && !ident && (W <= 1280 || (W <= 2048 && (T_ <= 1024 || (ey && T_ > 2048))) || (W <= 4096 && T_ <= 512));
+  // (identity experts and norms in parts keep the general kernel, and so do rows wider than 1280 without y, 2048 x 8192 24.3 and 25.8, from
+  // 1025 to 2048 of them with it, 1500 x 2048 13.6 and 14.7, and many wider than 2048, 8192 x 4096 83.7 and 89.1 us. 4096 x 2048 plain 21.8 ->
+  // 20.1, gated 30.9 -> 27.4, 8192 rows 48.9 -> 44.3 and 58.8 -> 59.6, past the caches 41.4 and 54.4)
+  const bool rows = vec && groups == 1 && !ident && (W <= 1280 || (W <= 2048 && (T_ <= 1024 || ((y || ey) && T_ > 2048))) || (W <= 4096 && T_ <= 512));
+  // a stream that the caches do not keep until the next closing op passes their replacement by, with what is read beside it: also four experts'
+  // rows, 8192 x 2048, 88 -> 72.6; but 8192 x 1024, 34 MB, 20.1 -> 22.7
+  const bool past = (y || ey) && (int64_t)T_ * W * 4 >= (48 << 20);
   if (slabs < 0 || (slabs && (!y || y2))) throw std::runtime_error("sandwich_add_norm: slabs of one product only");
   if (tail.kind) {
     if (!vec || groups != 1 || ident || dt != 0 || W > 2048) throw std::runtime_error("sandwich_add_norm: a tail needs whole bf16 rows of up to 2048 at aligned places");
@@ -609,7 +618,8 @@ static void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const 
   // 448, which spread unevenly over the SIMDs (1792 wide: 1.07)
   const int rth = W <= 1536 ? (W / 4 + 63) / 64 * 64 : 512;
   DISPATCH_T(dt, T, {
-    if (rows && W <= 2048) sandwich_rows_kernel<T, 1, NoTail, Y_ANY><<<T_, rth, 0, st>>>(p, NoTail{});
+    if (rows && W <= 2048 && past) sandwich_rows_kernel<T, 1, NoTail, Y_ANY, true><<<T_, rth, 0, st>>>(p, NoTail{});
+    else if (rows && W <= 2048) sandwich_rows_kernel<T, 1, NoTail, Y_ANY><<<T_, rth, 0, st>>>(p, NoTail{});
     else if (rows) sandwich_rows_kernel<T, 2, NoTail, Y_ANY><<<T_, 512, 0, st>>>(p, NoTail{});
     else if (slabs && vec) sandwich_add_norm_kernel<T, 4, true><<<T_, th, lds, st>>>(p);
     else if (slabs) sandwich_add_norm_kernel<T, 1, true><<<T_, th, lds, st>>>(p);

@@ -73,3 +73,26 @@ def test_token_side(T, W, d, kind, monkeypatch):
     monkeypatch.setattr(hip, "TAIL_ROWS", -1)
     h2 = hip.sandwich_add_norm(x2, y, r, rb, wpost, 1e-5, add, wnext, torch.bfloat16, side=side)
     assert close(x1, x2, 2.0 ** -16) and (wnext is None and h1 is None and h2 is None or close(h1, h2, 2.0 ** -7))
+
+
+# rows in registers on either side of the sizes where that form begins, and streams that pass the caches by
+@pytest.mark.parametrize("T,W", [(2048, 2048), (2049, 1284), (2049, 2048), (6144, 2048), (9600, 1312)])
+@pytest.mark.parametrize("kind", ["plain", "gated", "scaled pair", "experts"])
+def test_many_rows(T, W, kind):
+    from llmss_amd.ops import hip
+    g = torch.Generator().manual_seed(T)
+    y, r, rb = closing(kind, T, W, g)
+    x, wpost, wnext, add = (torch.randn(*s, generator=g).cuda() for s in ((T, W), (W,), (W,), (T, W)))
+    v = y
+    if kind == "scaled pair":
+        v = 0.7 * y.yl.double() + 0.6 * y.yr.double()
+    elif kind == "experts":
+        v = (y.y.double()[y.place.long()].view(T, y.top, W) * y.wts.double()[..., None]).sum(1) + y.shared_w.double()[:, None] * y.shared.double()
+    v = v.double() * (torch.sigmoid(r.double() + rb.double()) if r is not None else 1.0)
+    norm = lambda t: t / torch.sqrt(t.pow(2).mean(-1, keepdim=True) + 1e-5)  # noqa: E731
+    want = x.double() + norm(v) * wpost.double() + add.double()
+    h = hip.sandwich_add_norm(x, y, r, rb, wpost, 1e-5, add, wnext, torch.bfloat16)
+    # fp32: a sum of W squares and some 20 roundings of terms of up to the largest number's size; one to bf16
+    assert ((x.double() - want).abs() <= 2.0 ** -18 * want.abs().amax(-1, keepdim=True)).all()
+    hw = norm(want) * wnext.double()
+    assert ((h.double() - hw).abs() <= 2.0 ** -8 * hw.abs() + 2.0 ** -16 * hw.abs().amax(-1, keepdim=True)).all()
