@@ -16,6 +16,8 @@
 // to the V^T operand through the addresses of the transpose reads.
 // K/V tiles of 64 keys are register-staged into LDS rows padded by 32 B (conflict-free for
 // both the b128 row reads and the tr_b16 column reads at D=128).
+#include <type_traits>
+
 #include "common.h"
 
 constexpr float kLog2eP = 1.4426950408889634f;
@@ -156,8 +158,12 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const bf16_t* __restr
 //   * v_exp_f32 directly (no denormal range fix-ups: p < 2^-126 flushes to 0);
 //   * deferred rescale (guide T13): the running max moves only when a row's max grows by more than 8
 //     (log2 units), so p <= 2^8 and the O *= alpha sweep runs only when some row of the wave moved -
-//     every l-side and o-side factor of a tile uses the same per-row alpha;
+//     every l-side and o-side factor of a tile uses the same per-row alpha; whether one did is asked of the lanes' own scores, so
+//     that a tile whose rows stand exchanges nothing between lanes (the sums meet at the end);
 //   * the row sum accumulates the fp32 probabilities (v2 summed the bf16-rounded ones).
+// us, the mask in a loop of its own, maxima by lane and eight sums of scores side by side, before and now: 3999 tokens, 32 heads of 128 232 ->
+// 176 (158 with rows that are no multiple of 4 KB apart), two of 2048 tokens, 8 key heads 100 -> 82, four of 1000, 25 heads of 64 54 -> 42, two
+// of 2000, 16 heads of 256 130 -> 112. A tile's scores beside the probabilities of the one before: 182; waves' priorities: 184.
 // NW: waves per workgroup (4: two workgroups per CU; 8: one 512-thread workgroup per CU whose K/V tile
 // feeds twice the query rows, halving the LDS-DMA traffic per FLOP).
 template <int D, int QB, bool FAST, int NW = 4>
@@ -260,74 +266,79 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prefill_v2_kernel(const bf16_
   const int w_hi = wrow + 16 * QB - 1;         // this wave's last query row
   const int tq = li >> 2, tp = li & 3;         // transpose-read lane roles (row q, 4 columns 4p..4p+3)
   PF_STAGE(0);
-  for (int j = 0; j < ntiles; ++j) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();              // tile j landed for every wave; slot (j+1)&1 is free
-    asm volatile("" ::: "memory");
-    if (j + 1 < ntiles) PF_STAGE(j + 1);
+  // one tile of 64 keys; MASK: 0 none, 1 by position
+  auto tile = [&](int j, auto mask_c) {
+    constexpr bool MASK = decltype(mask_c)::value;
     const int kv0 = j * BKV;
-    if (kv0 > w_hi) continue;                  // the whole tile is in this wave's causal future
     const char* Ks = smem + (j & 1) * 2 * TILE;
     const char* Vs = Ks + TILE;
-
-    // ---- S^T = K Q^T: 4 key tiles of 16, each K fragment feeds QB MFMAs -------------------------
+    // ---- S^T = K Q^T: 4 key tiles of 16, each K fragment feeds QB MFMAs; 4 QB sums side by side ----
     f32x4 s[QB][4];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
+    for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
       for (int qi = 0; qi < QB; ++qi) s[qi][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const int r = kt * 16 + li;
 #pragma unroll
-      for (int ks = 0; ks < D / 32; ++ks) {
-        const s16x8 kf = *reinterpret_cast<const s16x8*>(Ks + r * D * 2 + (swz(4 * ks + g, r) << 4));
+    for (int ks = 0; ks < D / 32; ++ks) {
+      s16x8 kf[4];
 #pragma unroll
-        for (int qi = 0; qi < QB; ++qi) s[qi][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[qi][ks], s[qi][kt], 0, 0, 0);
+      for (int kt = 0; kt < 4; ++kt) {
+        const int r = kt * 16 + li;
+        kf[kt] = *reinterpret_cast<const s16x8*>(Ks + r * D * 2 + (swz(4 * ks + g, r) << 4));
       }
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int qi = 0; qi < QB; ++qi) s[qi][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kt], qf[qi][ks], s[qi][kt], 0, 0, 0);
     }
-    // ---- mask + online softmax per row block (lane owns query row wrow + 16 qi + li) -------------
+    __builtin_amdgcn_sched_barrier(0);  // (left alone, the last sums become chains of four behind one another)
+    // ---- online softmax per row block (lane owns query row wrow + 16 qi + li) -------------
     s16x8 pf[QB][2];
     if constexpr (FAST) {
-      const bool need_mask = (kv0 + BKV - 1 > wrow) || (kv0 + BKV > len);  // wave-uniform
+      float mx[QB];
+      bool grew = false;
 #pragma unroll
       for (int qi = 0; qi < QB; ++qi) {
         const int qrow = wrow + qi * 16 + li;
-        float mx = -1.0e30f;
-        if (need_mask) {
+        mx[qi] = -1.0e30f;
 #pragma unroll
-          for (int kt = 0; kt < 4; ++kt)
+        for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+          for (int i = 0; i < 4; ++i) {
+            if constexpr (MASK) {
               const int key = kv0 + kt * 16 + 4 * g + i;
-              const float v = (key <= qrow && key < len) ? s[qi][kt][i] : -1.0e30f;
-              s[qi][kt][i] = v;
-              mx = fmaxf(mx, v);
+              s[qi][kt][i] = (key <= qrow && key < len) ? s[qi][kt][i] : -1.0e30f;
             }
-        } else {
+            mx[qi] = fmaxf(mx[qi], s[qi][kt][i]);
+          }
+        mx[qi] *= scale_log2;
+        grew |= mx[qi] > m[qi] + 8.f;
+      }
+      if (__ballot(grew)) {  // some row's maximum moves: lanes of a row agree on it only here
 #pragma unroll
-          for (int kt = 0; kt < 4; ++kt)
+        for (int qi = 0; qi < QB; ++qi) {
+          const float rmx = xor32_max(xor16_max(mx[qi]));
+          const bool resc = rmx > m[qi] + 8.f;
+          const float alpha = resc ? __builtin_amdgcn_exp2f(m[qi] - rmx) : 1.f;
+          if (resc) m[qi] = rmx;
+          lsum[qi] *= alpha;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[qi][kt][i]);
+          for (int i = 0; i < D / 16; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[qi][i][e] *= alpha;
         }
-        mx = xor32_max(xor16_max(mx)) * scale_log2;
-        const bool resc = mx > m[qi] + 8.f;
-        const float alpha = resc ? __builtin_amdgcn_exp2f(m[qi] - mx) : 1.f;
-        if (resc) m[qi] = mx;
+      }
+#pragma unroll
+      for (int qi = 0; qi < QB; ++qi) {
         const float nm = -m[qi];
-        float ps = 0.f;
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const float p = __builtin_amdgcn_exp2f(fmaf(s[qi][kt][i], scale_log2, nm));
-            ps += p;
+            lsum[qi] += p;
             pf[qi][kt >> 1][(kt & 1) * 4 + i] = (short)f2bf(p);
           }
-        ps = xor32_sum(xor16_sum(ps));
-        lsum[qi] = lsum[qi] * alpha + ps;
-        if (__ballot(resc)) {
-#pragma unroll
-          for (int i = 0; i < D / 16; ++i) o[qi][i] *= alpha;
-        }
       }
     } else {
 #pragma unroll
@@ -378,7 +389,32 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prefill_v2_kernel(const bf16_
         for (int qi = 0; qi < QB; ++qi) o[qi][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[qi][ks], o[qi][dt], 0, 0, 0);
       }
     }
+  };
+  // tiles that no mask touches first; the last ones, on the wave's diagonal or the sequence's end, in a loop of their own (the positions'
+  // arithmetic beside the other, though skipped, was a sixth of its vector instructions)
+  const int whole = FAST ? min(min((wrow + 1) / BKV, len / BKV), ntiles) : 0;
+  int j = 0;
+#define PF_NEXT()                                                                            \
+  do {                                                                                       \
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                         \
+    __builtin_amdgcn_s_barrier(); /* tile j landed for every wave; slot (j+1)&1 is free */   \
+    asm volatile("" ::: "memory");                                                           \
+    if (j + 1 < ntiles) PF_STAGE(j + 1);                                                     \
+  } while (0)
+  for (; j < whole; ++j) {
+    PF_NEXT();
+    tile(j, std::false_type{});
   }
+  for (; j < ntiles; ++j) {
+    PF_NEXT();
+    if (j * BKV > w_hi) continue;              // the whole tile is in this wave's causal future
+    tile(j, std::true_type{});
+  }
+  if constexpr (FAST) {  // (the row sums, so far by lane)
+#pragma unroll
+    for (int qi = 0; qi < QB; ++qi) lsum[qi] = xor32_sum(xor16_sum(lsum[qi]));
+  }
+#undef PF_NEXT
 #undef PF_STAGE
 #pragma unroll
   for (int qi = 0; qi < QB; ++qi) {

@@ -671,6 +671,9 @@ def linear(x, w, bias=None, act="none", glu=False, w_scale=None, out=None, nt_hi
     return y
 
 
+QKV_PAD = 128  # numbers
+
+
 def linear_qkv(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, D, rot, style, do_rope=True,
                nt_hint=0, split_hint=0):
     """QKV projection whose GEMM epilogue applies RoPE and writes k / v into the paged cache (one launch
@@ -699,7 +702,10 @@ def linear_qkv(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv
                "slots")
         bs = k_cache.shape[2]
     ws = _GEMM_WS.get(64 << 20, x.device)
-    y = torch.empty(M, N, dtype=x.dtype, device=x.device)
+    # rows a multiple of 4 KB apart lie in few of the caches' channels, head by head, where attention reads them: prompts' rows are kept 256
+    # bytes further apart (3999 rows of 12288, 32 heads of 128: 176 -> 158 us of attention)
+    pad = QKV_PAD if M >= 128 and N * 2 % 4096 == 0 else 0
+    y = torch.empty(M, N + pad, dtype=x.dtype, device=x.device)[:, :N]
     rc = lib().gemm_qkv(x.data_ptr(), x.stride(0), w.data_ptr(), K, _ptr(bias), y.data_ptr(), y.stride(0), M, N, K,
                         ws.data_ptr(), ws.numel() * 4, int(nt_hint), int(split_hint), positions.data_ptr(),
                         _ptr(cos) if do_rope else 0, _ptr(sin) if do_rope else 0, _ptr(k_cache), _ptr(v_cache),
