@@ -27,7 +27,8 @@
 // NS groups of 16 slots a wave: a fragment of keys or values read from LDS feeds the products of all of them. With one group LDS
 // reads take as long as the matrix instructions (32 KB a wave and 64 keys of 128). Tiles that every row of a group sees whole skip
 // the mask. Portions of 950 and 823 rows behind prefixes of as many, 32 heads of 128: 135 -> 94 us (413
-// TFLOP/s), 111 with one group.
+// TFLOP/s), 111 with one group; inside a step 104 -> 88 us with maxima by lane, the masks' positions where there is a mask and four sums a
+// group side by side.
 // SAME: keys and values are one tensor (latent attention, where both are the cached latent row and nkv = 1): the
 // tile is loaded and staged once and serves both products.
 #include "common.h"
@@ -224,64 +225,78 @@ __global__ __launch_bounds__(256, NS) void attn_extend_kernel(
       if (kv0 > wave_qhi) continue;  // whole tile in this wave's causal future (barriers stay uniform)
       if (kv0 + BKV <= wave_klo) continue;  // whole tile older than this wave's windows
 
-      f32x4 s[NS][4];
+      f32x4 s[NS][4];  // (4 NS sums side by side)
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt) {
+      for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
         for (int n = 0; n < NS; ++n) s[n][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ks = 0; ks < D / 32; ++ks) {
-          const s16x8 kf = *reinterpret_cast<const s16x8*>(&Ks[(kt * 16 + li) * LD + 32 * ks + 8 * g]);
+      for (int ks = 0; ks < D / 32; ++ks) {
+        s16x8 kf[4];
 #pragma unroll
-          for (int n = 0; n < NS; ++n) s[n][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[n][ks], s[n][kt], 0, 0, 0);
-        }
+        for (int kt = 0; kt < 4; ++kt) kf[kt] = *reinterpret_cast<const s16x8*>(&Ks[(kt * 16 + li) * LD + 32 * ks + 8 * g]);
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int n = 0; n < NS; ++n) s[n][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kt], qf[n][ks], s[n][kt], 0, 0, 0);
       }
+      __builtin_amdgcn_sched_barrier(0);  // (else the last sums become chains, one behind another)
       // S^T C layout: lane (li, g) holds slot li's scores for keys kv0 + 16kt + 4g + i
       s16x8 pf[NS][2];
+      float mx[NS];
+      bool grew = false;
 #pragma unroll
       for (int n = 0; n < NS; ++n) {
-        float mx = m[n];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[n][kt][i] *= scale_log2;
         const bool whole = kv0 + BKV - 1 <= grp_lo[n] && kv0 + BKV <= kv_end && (window <= 0 || kv0 > grp_hi[n] - window);
-        if (whole) {
+        if (!whole) {
+          int k0 = kv0;
+          asm volatile("" : "+s"(k0));  // (the positions are formed here and not for every tile)
+          // a masked key weighs nothing, also while a slot has seen no visible key yet (its maximum still at its floor)
 #pragma unroll
           for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              s[n][kt][i] *= scale_log2;
-              mx = fmaxf(mx, s[n][kt][i]);
-            }
-        } else {
-#pragma unroll
-          for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int key = kv0 + kt * 16 + 4 * g + i;
-              float v = s[n][kt][i] * scale_log2;
-              v = (key <= qpos[n] && key < kv_end && (window <= 0 || key > qpos[n] - window)) ? v : -1.0e30f;
-              s[n][kt][i] = v;
-              mx = fmaxf(mx, v);
+              const int key = k0 + kt * 16 + 4 * g + i;
+              s[n][kt][i] = (key <= qpos[n] && key < kv_end && (window <= 0 || key > qpos[n] - window)) ? s[n][kt][i] : -INFINITY;
             }
         }
-        mx = xor32_max(xor16_max(mx));
-        const float alpha = __builtin_amdgcn_exp2f(m[n] - mx);
-        m[n] = mx;
-        float ps = 0.f;
+        mx[n] = -1.0e30f;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) mx[n] = fmaxf(mx[n], s[n][kt][i]);
+        grew |= mx[n] > m[n] + 8.f;
+      }
+      // The maximum that the exponents stand against moves only where a row's own has grown by more than 8 (weights stay below 2^8): lanes of a
+      // row exchange theirs, and the outputs are scaled, in such tiles only.
+      if (__ballot(grew)) {
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+          const float rmx = xor32_max(xor16_max(mx[n]));
+          const bool up = rmx > m[n] + 8.f;
+          const float alpha = up ? __builtin_amdgcn_exp2f(m[n] - rmx) : 1.f;
+          if (up) m[n] = rmx;
+          lsum[n] *= alpha;
+#pragma unroll
+          for (int i = 0; i < D / 16; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[n][i][e] *= alpha;
+        }
+      }
+#pragma unroll
+      for (int n = 0; n < NS; ++n)
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            float p = __builtin_amdgcn_exp2f(s[n][kt][i] - mx);
-            // a masked key adds nothing, also while a slot has seen no visible key yet (mx still at its floor)
-            if (!whole) p = s[n][kt][i] > -1.0e29f ? p : 0.f;
-            const bf16_t pb = f2bf(p);
-            ps += bf2f(pb);
+            const bf16_t pb = f2bf(__builtin_amdgcn_exp2f(s[n][kt][i] - m[n]));
+            lsum[n] += bf2f(pb);
             pf[n][kt >> 1][(kt & 1) * 4 + i] = (short)pb;
           }
-        ps = xor32_sum(xor16_sum(ps));
-        lsum[n] = lsum[n] * alpha + ps;
-#pragma unroll
-        for (int i = 0; i < D / 16; ++i) o[n][i] *= alpha;
-      }
 
       const int tq = li >> 2, tp = li & 3;
 #pragma unroll
@@ -301,6 +316,8 @@ __global__ __launch_bounds__(256, NS) void attn_extend_kernel(
   };
   if (lds_pages) walk(std::true_type{});
   else walk(std::false_type{});
+#pragma unroll
+  for (int n = 0; n < NS; ++n) lsum[n] = xor32_sum(xor16_sum(lsum[n]));  // (so far by lane)
   if (nsplit > 1) {  // kernel argument: uniform
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
