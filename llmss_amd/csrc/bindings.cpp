@@ -49,7 +49,7 @@ int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_f
                 const void* bias, void* y, int64_t ldy, int M, int N, int K, int act, bool glu, void* workspace,
                 int64_t ws_bytes, int nt_hint, int split_hint, bool partial_out, hipStream_t st);
 void gemm_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int* nt, int* splitk);
-void gemm_cut_of(int M, int N, int K, bool glu, int* rows, int* cols);
+void gemm_cut_of(int M, int N, int K, bool glu, int* rows, int* cols, int* split);
 void gemm_tuned_set(int M, int N, int K, bool glu, int kind, int nt_hint, int split);
 void gemm_tuned_clear();
 void gemm_reserve_streamk(int n);
@@ -363,9 +363,14 @@ PYBIND11_MODULE(_C, m) {
   }, pybind11::arg(), pybind11::arg(), pybind11::arg(), pybind11::arg(), pybind11::arg("glu") = false,
      pybind11::arg("slabs") = true);
   m.def("gemm_cut", [](int M, int N, int K, bool glu) {  // rows or columns of the first of two launches, 0: one launch
-    int rows, cols;
-    gemm_cut_of(M, N, K, glu, &rows, &cols);
+    int rows, cols, split;
+    gemm_cut_of(M, N, K, glu, &rows, &cols, &split);
     return py::make_tuple(rows, cols);
+  });
+  m.def("gemm_cut_split", [](int M, int N, int K, bool glu) {  // split of the second launch's K
+    int rows, cols, split;
+    gemm_cut_of(M, N, K, glu, &rows, &cols, &split);
+    return split;
   });
   m.def("gemm_tuned_set", &gemm_tuned_set);
   m.def("gemm_tuned_clear", &gemm_tuned_clear);

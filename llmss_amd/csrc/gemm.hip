@@ -1853,19 +1853,26 @@ static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int
 // cuts, 257 - 10000 rows and whole steps of k, two launches take 0.886 of the time from K = 1024 on, 1.11 at worst. Below, a tile's start and end
 // are half of it, and what is promised up to there does not come: gated products 0.87 (0.98 at worst), others 0.954 where more than 6.5 % are
 // promised (95 products; 1.15 at worst, all of those at 6.5 - 10 %: 3764 x 5664 x 256 27 -> 31), 1.02 where less, so those stay whole.
+// The rest's tiles can be too few for the chip (69 x 2048: 32 of 64 x 128, each alone with all of K): K is split where that promises a tenth
+// of the rest's time, priced as in gemm_static_plan. 390 of 5246 random products; over 158 of them 0.982 of the whole product's time
+// (0.96 up to 3.4 MB of slabs, all but six of the 158 at most 1.01; at worst 1.05 with 28 MB, so those end at 24 MB): 8261 x 2048 x 4096
+// 122.8 -> 108.2 us (its rest 27.4 -> 12.7), x 2560 81.9 -> 73.0, 1240 x 13248 x 3392 110.8 -> 100.6, 909 x 20000 x 12160 464 -> 421.
 struct GemmCut {
   int rows, cols;  // of the first launch; 0: not cut
   int hint;        // plan of the second (0: the plan of its size)
+  int split;       // of its K
 };
-static GemmCut gemm_cut(int M, int N, int K, bool glu) {
+static GemmCut gemm_cut(int M, int N, int K, bool glu, int64_t ws_bytes) {
   const int ntm = (M + 255) / 256, ntn = (N + 255) / 256, nk = (K + 63) / 64;
-  auto tiles_us = [&](const TileCost& c, int m, int n) {
-    const int slots = 256 * c.per_cu, wgs = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn), rest = wgs % slots;
-    double t = wgs / slots * (nk * c.step + 5.0);
-    if (rest) t += (nk * (rest <= 256 ? c.alone : c.step) + 5.0) * (rest * 5 <= slots * 4 ? 0.78 : 1.0);
-    return std::max(t, (2.0 * n * K + 2.0 * m * K + 2.0 * m * (glu ? n / 2 : n)) / 4.0e6);
+  auto tiles_us = [&](const TileCost& c, int m, int n, int split = 1) {
+    const int slots = 256 * c.per_cu, wgs = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn) * split, rest = wgs % slots;
+    const int per = (nk + split - 1) / split;
+    double t = wgs / slots * (per * c.step + 5.0);
+    if (rest) t += (per * (rest <= 256 ? c.alone : c.step) + 5.0) * (rest * 5 <= slots * 4 ? 0.78 : 1.0);
+    t = std::max(t, (2.0 * n * K + 2.0 * m * K + 2.0 * m * (glu ? n / 2 : n)) / 4.0e6);
+    return split > 1 ? t + 4.0 + 8.0 * split * m * n / 4.5e6 : t;
   };
-  GemmCut cut{0, 0, 0};
+  GemmCut cut{0, 0, 0, 1};
   double best = (K < 1024 && !glu ? 0.935 : 0.97) * tiles_us(kTileCost[0], M, N);
   auto consider = [&](int rows, int cols) {
     if (rows <= 0 || cols <= 0 || (rows >= M && cols >= N)) return;
@@ -1873,14 +1880,17 @@ static GemmCut gemm_cut(int M, int N, int K, bool glu) {
     if (last && last < 218) return;  // whole waves, the last of them at least 0.85 full
     const int m = rows < M ? M - rows : M, n = cols < N ? N - cols : N;
     double rest = 8.0 + 2.0 * n * K / 4.5e6;
-    int hint = 0;
+    int hint = 0, split = 1;
     for (const TileCost& c : kTileCost) {
       if (m <= 64) break;
-      const double t = tiles_us(c, m, n);
-      if (!hint || t < rest) rest = t, hint = c.tsel << 8;
+      for (int s : {1, 2, 3, 4, 6, 8}) {
+        if (s > 1 && (c.tsel == 4 || K / s < 256 || (int64_t)s * m * n * 4 > std::min<int64_t>(ws_bytes, 24 << 20))) break;
+        const double t = tiles_us(c, m, n, s);
+        if (!hint || t < (s > split ? 0.9 : 1.0) * rest) rest = t, hint = c.tsel << 8, split = s;
+      }
     }
     const double t = tiles_us(kTileCost[0], std::min(rows, M), std::min(cols, N)) + rest;
-    if (t < best) best = t, cut = GemmCut{rows < M ? rows : 0, cols < N ? cols : 0, hint};
+    if (t < best) best = t, cut = GemmCut{rows < M ? rows : 0, cols < N ? cols : 0, hint, split};
   };
   const int waves = (int)std::min<int64_t>((int64_t)ntm * ntn / 256, 64);
   for (int w = 1; w <= waves; ++w) {
@@ -1900,17 +1910,17 @@ int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_f
   gemm_default_plan(M, N, K, w_fp8, glu, partial_out && !glu && act == 0, ws_bytes, gemm_static_takes(w_fp8, x, ldx, w, ldw), &nt_hint,
                     &split_hint);
   if (free_plan && nt_hint == 4 << 8 && y && !(glu && N % 32) && gemm_quad_ok(N, K, ldx, ldw, 256, y, ldy, 2, glu)) {
-    const GemmCut cut = gemm_cut(M, N, K, glu);
+    const GemmCut cut = gemm_cut(M, N, K, glu, ws_bytes);
     if (cut.rows) {
       launch_gemm(x, ldx, w, ldw, false, nullptr, bias, y, ldy, cut.rows, N, K, act, glu, workspace, ws_bytes, 4 << 8, 1, false, st);
       return launch_gemm((const bf16_t*)x + cut.rows * ldx, ldx, w, ldw, false, nullptr, bias, (bf16_t*)y + cut.rows * ldy, ldy,
-                         M - cut.rows, N, K, act, glu, workspace, ws_bytes, cut.hint, cut.hint ? 1 : 0, false, st);
+                         M - cut.rows, N, K, act, glu, workspace, ws_bytes, cut.hint, cut.hint ? cut.split : 0, false, st);
     }
     if (cut.cols) {
       launch_gemm(x, ldx, w, ldw, false, nullptr, bias, y, ldy, M, cut.cols, K, act, glu, workspace, ws_bytes, 4 << 8, 1, false, st);
       return launch_gemm(x, ldx, (const bf16_t*)w + cut.cols * ldw, ldw, false, nullptr, bias ? (const bf16_t*)bias + cut.cols : nullptr,
                          (bf16_t*)y + (glu ? cut.cols / 2 : cut.cols), ldy, M, N - cut.cols, K, act, glu, workspace, ws_bytes, cut.hint,
-                         cut.hint ? 1 : 0, false, st);
+                         cut.hint ? cut.split : 0, false, st);
     }
   }
   if (!y && (!partial_out || slabs_of_plan(M, N, K, w_fp8, glu, act, nt_hint, split_hint, ws_bytes) == 0))
@@ -2335,7 +2345,7 @@ int launch_gemm_qkv(const void* x, int64_t ldx, const void* w, int64_t ldw, cons
   gemm_tiled_plan(M, N, K, &tsel, &s, false);
   if (tsel == 4) {  // 256 x 256 tiles, and what they leave over as launch_gemm has it
     if ((qe.do_rope && qe.style != 1) || 256 % qe.D || !gemm_quad_ok(N, K, ldx, ldw, 256, y, ldy, 2, false)) return -1;
-    const GemmCut cut = gemm_cut(M, N, K, false);
+    const GemmCut cut = gemm_cut(M, N, K, false, 0);  // unsplit: the epilogue needs finished sums
     const int rows = cut.rows ? cut.rows : M, cols = cut.cols ? cut.cols : N;
     launch_gemm_quad(0, (const bf16_t*)x, ldx, (const bf16_t*)w, ldw, (const bf16_t*)bias, (bf16_t*)y, ldy, rows, cols, K, 0, 0,
                      g_big_group_m, tiles_of(rows, cols, 256, 256), PpGroup{}, st, &qe);
@@ -2379,10 +2389,11 @@ int launch_gemm_qkv_args(const void* x, int64_t ldx, const void* w, int64_t ldw,
   return launch_gemm_qkv(x, ldx, w, ldw, bias, y, ldy, M, N, K, workspace, ws_bytes, nt_hint, split_hint, qe, st);
 }
 
-void gemm_cut_of(int M, int N, int K, bool glu, int* rows, int* cols) {
-  const GemmCut c = gemm_cut(M, N, K, glu);
+void gemm_cut_of(int M, int N, int K, bool glu, int* rows, int* cols, int* split) {
+  const GemmCut c = gemm_cut(M, N, K, glu, 64 << 20);
   *rows = c.rows;
   *cols = c.cols;
+  *split = c.split;
 }
 
 // The plan of a product without hints. slabs: of one whose consumer sums split-K slabs itself

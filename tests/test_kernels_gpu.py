@@ -369,6 +369,23 @@ def test_products_cut_in_two_launches(M, N, K, glu, act):
     assert (wide == 7.0).all()
 
 
+@pytest.mark.parametrize("M,N,K,glu,act,bias", [(8261, 2048, 2048, False, "gelu", True), (1240, 13248, 3392, False, "none", True),
+                                                (964, 16576, 2112, True, "none", True), (3558, 9344, 3008, False, "none", False)])
+def test_rest_of_a_cut_product_splits_k(M, N, K, glu, act, bias):
+    """The rest of a product that is cut in two launches, with few tiles: K split in slabs of 32-bit sums, bias, activation and gate after
+    their sum; strided rows, what lies around them stays. Each side's error is a rounding of the result in bf16 and of 32-bit sums."""
+    torch.manual_seed(0)
+    x, w, b = rnd(M, K + 8)[:, :K], rnd(N, K, scale=K ** -0.5), rnd(N, scale=0.1) if bias else None
+    n = N // 2 if glu else N
+    wide = torch.full((M + 2, n + 16), 7.0, dtype=torch.bfloat16, device=dev)
+    y = wide[1:M + 1, 8:n + 8]
+    assert any(H.lib().gemm_cut(M, N, K, glu)) and H.lib().gemm_cut_split(M, N, K, glu) > 1
+    H.linear(x, w, b, act=act, glu=glu, out=y)
+    close(y, R.linear(x.float(), w.float(), b.float() if bias else None, act=act, glu=glu), 2e-2)
+    wide[1:M + 1, 8:n + 8] = 7.0
+    assert (wide == 7.0).all()
+
+
 DEC_BN = {1: 16, 2: 32, 3: 48, 4: 64, 5: 96}  # csrc/gemm_dec.hip tile codes (hint bit 1024 of the tile bits)
 
 
