@@ -1703,6 +1703,45 @@ static double waves_us(int wgs, double read, F us) {
 }
 static int tile_dims(int tsel, int* bm, int* bn);
 static int tiles_of(int M, int N, int bm, int bn);
+
+// 17 - 64 rows whose consumer sums the slabs: the decode kernel on 16 - 64 columns, or, from 33 rows on, 64 x 64 tiles two k-steps deep,
+// whichever is priced lower together with the closing op that reads the slabs. Constants fitted over two thirds of 850 (17 - 32 rows:
+// 800) random products with their add_norm behind them, N to 8192, K of 512 - 12800, weights not in the caches; the choice is 0.9 %
+// (0.5 %) above the best of all on the other third. Against the plans before (tiles one step deep from 33 rows on, below 3072 columns
+// without a look at the decode kernel, and K split by a rule of its length) 0.92 of the time (0.97 to 32 rows), 42 of the 850 more than 1.02,
+// at worst 1.14 (63 x 320 x 1536: 6.6 -> 7.5); above 12800 in K 0.91 over 41 products (1.08 at worst, 64 x 5712 x 25408; to 32 rows not
+// measured, so that those stay with the older price), above 8192 columns 1.01 over 19. us with the closing op: 64 x 2048 x 2048 10.3 -> 9.2,
+// x 4096 11.9 -> 11.2, 33 x 2048 x 4096 10.8 -> 10.0, 64 x 4096 x 4096 15.2 -> 14.8, x 11008 26.1 -> 25.3, 64 x 2640 x 4320 17.9 -> 15.3,
+// 48 x 1488 x 1920 12.0 -> 8.8.
+struct SlabCost {  // as DecCost; us of the closing op in start, slab: bytes of sums written and read per us
+  double start, cu, x, wave, chip, spare, slab;
+};
+static constexpr SlabCost kSlabDec[] = {{4.405, 28.9e3, 0.37, 1.478, 6.19e6, 0.359, 1.57e6}, {4.442, 27.6e3, 0.341, 1.696, 5.2e6, 0.219, 1.98e6}};
+static bool gemm_slab_plan(int M, int N, int K, int64_t ws_bytes, int* nt_hint, int* split) {
+  if (N < 256 || N > 8192 || K < 512 || (M <= 32 && K > 12800)) return false;
+  const SlabCost& c = kSlabDec[M > 32];
+  const double bytes = 2.0 * N * K;
+  double best = 0;
+  auto take = [&](double t, int code, int s) {
+    if (best == 0 || t < best) best = t, *nt_hint = code << 8, *split = s;
+  };
+  for (int s : {2, 4, 8}) {
+    if (K / s < 256 || (int64_t)s * M * N * 4 > ws_bytes) break;
+    for (int bn = 64; bn >= 16; bn -= 16) {
+      const double kk = (double)K / s;
+      take(c.start + s * 8.0 * M * N / c.slab + waves_us((N + bn - 1) / bn * s, kk * bn * 2 / c.chip, [&](int n) {
+             return kk * (bn + c.x * M) * 2 / (c.cu * (1 + c.spare * (256 - n) / 256)) + c.wave;
+           }), bn / 16 | 32 | kDecHint, s);
+    }
+  }
+  for (int s : {2, 3, 4, 6, 8}) {
+    if (M <= 32 || K / s < 128 || (int64_t)s * M * N * 4 > ws_bytes) break;
+    const int per = ((K + 63) / 64 + s - 1) / s, wgs = (N + 63) / 64 * s;
+    take(5.54 + s * 8.0 * M * N / 1.91e6 + std::max(std::max(per * 0.375, (wgs + 255) / 256 * per * 0.353), bytes / 5.95e6), 3 | 32, s);
+  }
+  return best > 0;
+}
+
 // slabs: the consumer sums split-K slabs itself and so gets the product in 32 bits. Where the older rules split K that stays so:
 // only split plans are looked at, their slabs costing a write and a read and no launch.
 static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t ws_bytes, int* nt_hint, int* split) {
@@ -1714,6 +1753,7 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
     slabs = s > 1 && (int64_t)s * M * N * 4 <= ws_bytes;
   }
   if (M <= 64) {
+    if (slabs && M > 16 && gemm_slab_plan(M, N, K, ws_bytes, nt_hint, split)) return;
     if (M > 32 && N < 3072) return;
     const double bytes = 2.0 * N * K, slab = 8.0 * M * N / 2.5e6;
     double older, faster = M <= 16 ? 1.25 : 1.15;

@@ -386,6 +386,24 @@ def test_rest_of_a_cut_product_splits_k(M, N, K, glu, act, bias):
     assert (wide == 7.0).all()
 
 
+@pytest.mark.parametrize("M,N,K,tile", [(33, 256, 1040, False), (64, 2048, 2048, False), (17, 4096, 11008, False), (32, 2816, 12800, False),
+                                        (64, 4096, 11008, True), (64, 4096, 11024, True), (59, 6704, 4320, True), (64, 8192, 1040, True)])
+def test_slabs_of_few_rows(M, N, K, tile):
+    """Products of 17 - 64 rows whose closing op sums the slabs: the planned kernel (column tiles of the decode kernel, or 64 x 64 tiles), odd
+    k-steps, against the sums in 32 bits and the norm of their sum with the residual; a rounding of the result in bf16 each."""
+    torch.manual_seed(0)
+    x, w, r = rnd(M, K + 8)[:, :K], rnd(N, K, scale=K ** -0.5), rnd(M, N)
+    g = (1 + 0.1 * torch.randn(N, device=dev)).to(torch.bfloat16)
+    nt, split = H.lib().gemm_plan(M, N, K, False, False, True)
+    assert split > 1 and bool((nt >> 8) & 1024) != tile
+    p = H.linear(x, w, partial_ok=True)
+    assert isinstance(p, H.PartialSum) and p.S == split
+    total = x.float() @ w.float().t() + r.float()
+    y, res = H.add_norm(p, g, None, 1e-5, True, r.clone())
+    close(res, total, 2e-2)
+    close(y, total * torch.rsqrt(total.pow(2).mean(-1, keepdim=True) + 1e-5) * g.float(), 3e-2)
+
+
 DEC_BN = {1: 16, 2: 32, 3: 48, 4: 64, 5: 96}  # csrc/gemm_dec.hip tile codes (hint bit 1024 of the tile bits)
 
 
