@@ -200,6 +200,133 @@ __global__ __launch_bounds__(256, BM * BN > 128 * 128 ? 2 : 1) void gemm_tile_ke
     }
 }
 
+// The grouped products with whole k-steps and rows of 16-byte alignment: as above, but operands go straight to a ring of NS k-steps in
+// LDS, NS - 1 of them on their way, one barrier a step; 8 rows x 128 bytes a load, chunks XOR-swizzled by row so that fragment reads meet
+// no bank conflict. Bound by the weights of the experts that the tokens reach and, with few rows each, by the latency of a step: the kernel
+// above waits out one step's loads after each, its two barriers between them. Experts start at different k-steps (e * 11): rows of a power of
+// two bytes lie on few memory channels, which all tiles would otherwise walk together (32 experts of 768 x 2048, 80 rows each: 100 -> 94 us of
+// both products; by row tile instead, tiles that share an expert's weights lose each other: 188 rows each 151 -> 158). us of both products
+// against the kernel above: 16 experts of 512 x 1024, 38 rows each 33.2 -> 24.6; 32 of 768 x 2048, 80 rows 120 -> 94, 103 rows 117 -> 99; 64 of
+// 1408 x 2048, 96 rows 360 -> 294, 66 rows 321 -> 277; over 69 random layers (8 - 128 experts, 9 - 260 rows each) 0.82 of the time, 1.06 at worst
+// (before the k-steps were spread). Depth: three steps where the tiles then run at once, else two, so that three workgroups share a CU
+// (above 512 tiles: 640 x 4 rows over 32 experts 118 -> 103 us, below, 400 x 4 rows, 97 -> 91 with three); four or six steps were slower
+// everywhere (822 x 4 rows: 127 and 139 against 120). 128 rows: 128 x 128 tiles for one matrix (64 and 256 columns 111 and 105 against 102 us).
+template <int MODE, typename TC, int BM, int BN, int NS>
+__global__ __launch_bounds__(256) void moe_ring_kernel(GemmTileArgs p) {
+  constexpr int MB = BM / 32, NB = BN / 32;
+  constexpr bool DUAL = MODE == GT_GATE_UP;
+  constexpr int AI = BM / 32, BI = (DUAL ? 2 : 1) * BN / 32;  // 1-KiB loads (8 rows of a k-step) of a wave
+  constexpr int LOADS = AI + BI, SLOT = (BM + (DUAL ? 2 : 1) * BN) * 128;
+  static_assert(NS * SLOT <= 160 * 1024 && (NS - 2) * LOADS <= 63, "LDS and the wait's immediate");
+  __shared__ __attribute__((aligned(16))) char smem[NS * SLOT];
+  const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = (w >> 1) * (BM / 2), wn = (w & 1) * (BN / 2);
+  if ((int)blockIdx.y >= p.meta[0]) return;
+  const int id = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, p.meta[0] * gridDim.x);
+  const int ty = id / gridDim.x, n0 = (id % gridDim.x) * BN;
+  const int e = p.meta[1 + (p.E + 1) + ty], crow0 = p.meta[1 + (p.E + 1) + p.maxt + ty];
+  const int rows = min(BM, p.meta[1 + e + 1] - crow0);
+
+  const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(p.A)), (short)0, 0x7fffffff, 0x00020000);
+  const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(p.B + (int64_t)e * p.sBb)), (short)0,
+                                                    0x7fffffff, 0x00020000);
+  const auto rb2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>((DUAL ? p.B2 : p.B) + (int64_t)e * p.sBb)),
+                                                     (short)0, 0x7fffffff, 0x00020000);
+  // wave w takes rows 8 (w + 4 i) .. + 7 of each operand; past the rows or columns: an offset that reads as zero
+  uint32_t va[AI], vb[BN / 32];
+  const int sr0 = 8 * w + (lane >> 3), ch = ((lane & 7) ^ (sr0 & 7)) << 4;
+#pragma unroll
+  for (int i = 0; i < AI; ++i) {
+    const int sr = sr0 + 32 * i;
+    va[i] = 0x80000000u;
+    if (sr < rows) {
+      const int row = MODE == GT_DOWN ? crow0 + sr : p.order[crow0 + sr] / p.top;
+      va[i] = (uint32_t)(row * p.sAm * 2 + ch);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < BN / 32; ++i) {
+    const int n = n0 + sr0 + 32 * i, row = DUAL && p.ilv ? (n >> 4) * 32 + (n & 15) : n;
+    vb[i] = n < p.N ? (uint32_t)(row * p.sBn * 2 + ch) : 0x80000000u;
+  }
+  const int nk = p.K / 64;
+  const int k0 = (e * 11) % nk;
+#define MR_ISSUE(T_, S_)                                                                                                          \
+  do {                                                                                                                            \
+    const int q_ = (T_) + k0 >= nk ? (T_) + k0 - nk : (T_) + k0;                                                                   \
+    const uint32_t so_ = (T_) < nk ? (uint32_t)q_ * 128u : 0x80000000u;                                                         \
+    char* sl_ = smem + (S_) * SLOT + w * 1024;                                                                                    \
+    _Pragma("unroll") for (int i_ = 0; i_ < AI; ++i_)                                                                             \
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (LDS_AS void*)(sl_ + i_ * 4096), 16, (uint32_t)(va[i_] + so_), 0, 0, 0);       \
+    _Pragma("unroll") for (int i_ = 0; i_ < BN / 32; ++i_)                                                                        \
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (LDS_AS void*)(sl_ + BM * 128 + i_ * 4096), 16, (uint32_t)(vb[i_] + so_), 0, 0, 0); \
+    if (DUAL) _Pragma("unroll") for (int i_ = 0; i_ < BN / 32; ++i_)                                                              \
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb2, (LDS_AS void*)(sl_ + (BM + BN) * 128 + i_ * 4096), 16, (uint32_t)(vb[i_] + so_), 0, 0, 0); \
+  } while (0)
+  f32x4 acc[MB][NB], acc2[DUAL ? MB : 1][DUAL ? NB : 1];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (DUAL) acc2[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s) MR_ISSUE(s, s);
+  const int x0 = (g ^ (li & 7)) << 4, x1 = ((4 + g) ^ (li & 7)) << 4;
+  int slot = 0;
+  for (int t = 0; t < nk; ++t) {
+    // this wave's part of step t is there, and its reads of step t - 1 are done
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * LOADS) : "memory");
+    __builtin_amdgcn_s_barrier();  // every wave's
+    asm volatile("" ::: "memory");
+    MR_ISSUE(t + NS - 1, slot == 0 ? NS - 1 : slot - 1);  // into the slot of step t - 1
+    const char* st = smem + slot * SLOT;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int xo = s ? x1 : x0;
+      s16x8 a[MB];
+#pragma unroll
+      for (int i = 0; i < MB; ++i) a[i] = *reinterpret_cast<const s16x8*>(st + (wm + 16 * i + li) * 128 + xo);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const s16x8 b = *reinterpret_cast<const s16x8*>(st + (BM + wn + 16 * j + li) * 128 + xo);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b, acc[i][j], 0, 0, 0);
+        if constexpr (DUAL) {
+          const s16x8 b2 = *reinterpret_cast<const s16x8*>(st + (BM + BN + wn + 16 * j + li) * 128 + xo);
+#pragma unroll
+          for (int i = 0; i < MB; ++i) acc2[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b2, acc2[i][j], 0, 0, 0);
+        }
+      }
+    }
+    slot = slot == NS - 1 ? 0 : slot + 1;
+  }
+#undef MR_ISSUE
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (loads past the last step write zeros to LDS)
+  TC* C = (TC*)p.C;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = wm + 16 * i + 4 * g + q;
+      if (r >= rows) continue;
+      TC* crow = C + (int64_t)(crow0 + r) * p.sCm;
+      float sw = 1.0f;
+      if constexpr (MODE != GT_DOWN) sw = p.pw ? p.pw[p.order[crow0 + r]] : 1.0f;
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int n = n0 + wn + 16 * j + li;
+        if (n >= p.N) continue;
+        float v = acc[i][j][q];
+        if constexpr (DUAL) v = glu_clamped_t(v * sw, acc2[i][j][q] * sw, p.limit, p.alpha, p.silu);
+        if constexpr (MODE == GT_UP) v = gelu_erf(v * sw);
+        El<TC>::st(crow + n, v);
+      }
+    }
+}
+
 void launch_gemm_tile(const void* A, const void* B, void* C, int M, int N, int K, int batch, int64_t sAb, int64_t sAm,
                       int64_t sBb, int64_t sBn, int64_t sCb, int64_t sCm, int dc, const void* bias, hipStream_t st) {
   if (M <= 0 || N <= 0 || batch <= 0) return;
@@ -220,6 +347,22 @@ void launch_gemm_tile(const void* A, const void* B, void* C, int M, int N, int K
     else gemm_tile_kernel<GT_PLAIN, float, 64, 64><<<g, 256, 0, st>>>(a);
   }
   HIP_CHECK_LAUNCH();
+}
+
+// The ring kernel takes whole k-steps, 16-byte rows, and operands whose places fit 31 bits (`rows`: an upper bound of A's)
+static bool moe_ring_ok(const GemmTileArgs& a, int64_t lda, int64_t rows, int64_t wrows) {
+  return a.K % 64 == 0 && a.K > 0 && lda % 8 == 0 && !(((uintptr_t)a.A | (uintptr_t)a.B | (uintptr_t)a.B2) & 15) &&
+         (rows + 1) * lda * 2 < (1ll << 31) && wrows * a.K * 2 < (1ll << 31);
+}
+
+// 64-row tiles: three steps deep where the list's tiles (about maxt - E / 2) then still run at once, else two
+template <int MODE, typename TC>
+static void moe_ring64(const GemmTileArgs& a, hipStream_t st) {
+  const int cols = (a.N + 63) / 64;
+  constexpr int slot = MODE == GT_GATE_UP ? 24 : 16;  // KB
+  const dim3 g(cols, a.maxt);
+  if ((int64_t)(a.maxt - std::min(a.E / 2, a.maxt / 2)) * cols <= 256 * (160 / (3 * slot))) moe_ring_kernel<MODE, TC, 64, 64, 3><<<g, 256, 0, st>>>(a);
+  else moe_ring_kernel<MODE, TC, 64, 64, 2><<<g, 256, 0, st>>>(a);
 }
 
 // act[r, f] = glu(h[order[r] / top] . gate_e[f], h[..] . up_e[f]) over the tile list (bf16), or gelu(h[..] . up_e[f])
@@ -246,6 +389,12 @@ void launch_moe_gate_up_tile(const void* h, int64_t ldh, const void* wg, const v
   // workgroup per CU; at 128x64 two to three fit and hide each other's staging
   if (!wg) {
     a.B = (const bf16_t*)wu; a.B2 = nullptr;
+    if (moe_ring_ok(a, ldh, (int64_t)maxt * tile_rows / top, F)) {
+      if (tile_rows == 64) moe_ring64<GT_UP, bf16_t>(a, st);
+      else moe_ring_kernel<GT_UP, bf16_t, 128, 128, 2><<<dim3((F + 127) / 128, maxt), 256, 0, st>>>(a);
+      HIP_CHECK_LAUNCH();
+      return;
+    }
     const int bn = tile_rows == 128 && F >= 512 ? 256 : tile_rows;
     dim3 g((F + bn - 1) / bn, maxt);
     if (bn == 256) gemm_tile_kernel<GT_UP, bf16_t, 128, 256><<<g, 256, 0, st>>>(a);
@@ -255,6 +404,12 @@ void launch_moe_gate_up_tile(const void* h, int64_t ldh, const void* wg, const v
     return;
   }
   dim3 g((F + 63) / 64, maxt);
+  if (moe_ring_ok(a, ldh, (int64_t)maxt * tile_rows / top, (int64_t)(ilv ? 2 : 1) * F)) {
+    if (tile_rows == 128) moe_ring_kernel<GT_GATE_UP, bf16_t, 128, 64, 2><<<g, 256, 0, st>>>(a);
+    else moe_ring64<GT_GATE_UP, bf16_t>(a, st);
+    HIP_CHECK_LAUNCH();
+    return;
+  }
   if (tile_rows == 128) gemm_tile_kernel<GT_GATE_UP, bf16_t, 128, 64><<<g, 256, 0, st>>>(a);
   else gemm_tile_kernel<GT_GATE_UP, bf16_t, 64, 64><<<g, 256, 0, st>>>(a);
   HIP_CHECK_LAUNCH();
@@ -272,6 +427,12 @@ void launch_moe_down_tile(const void* act, const void* wd, const void* meta, voi
   a.meta = (const int*)meta; a.E = E; a.maxt = maxt; a.top = 1;
   const int bn = tile_rows == 128 && N >= 512 ? 256 : tile_rows;
   dim3 g((N + bn - 1) / bn, maxt);
+  if (moe_ring_ok(a, F, (int64_t)maxt * tile_rows, N)) {
+    if (tile_rows == 64) moe_ring64<GT_DOWN, float>(a, st);
+    else moe_ring_kernel<GT_DOWN, float, 128, 128, 2><<<dim3((N + 127) / 128, maxt), 256, 0, st>>>(a);
+    HIP_CHECK_LAUNCH();
+    return;
+  }
   if (bn == 256) gemm_tile_kernel<GT_DOWN, float, 128, 256><<<g, 256, 0, st>>>(a);
   else if (tile_rows == 128) gemm_tile_kernel<GT_DOWN, float, 128, 128><<<g, 256, 0, st>>>(a);
   else gemm_tile_kernel<GT_DOWN, float, 64, 64><<<g, 256, 0, st>>>(a);

@@ -1175,10 +1175,18 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     if T == 0:
         return out if shared_mlp is None else (out, torch.empty(0, sgu.shape[0], dtype=h.dtype, device=h.device) if D else None)
     P = T * top
-    # rows per tile of the grouped GEMMs: 128 where the experts get enough rows to fill big tiles (bf16 only)
-    rows = 128 if h.dtype == torch.bfloat16 and P >= 128 * E else 64
     # (both forms below load the weights in pieces of 16 bytes; the tile kernel takes any place)
     aligned = not (h.data_ptr() | up.data_ptr() | down.data_ptr() | _ptr(gate)) & 15 and h.stride(0) % 8 == 0
+    # rows per tile of the grouped GEMMs: 128 where the experts get enough rows to fill big tiles (bf16 only). Whole k-steps go through the
+    # ring of csrc/gemm_tile.hip, whose big tiles pay from half as many rows on, but only where they still fill the chip (us of both products
+    # at 64 and 128 rows: 32 experts of 768 x 2048, 1.5 tiles per CU, 64 rows each 93 and 93, 103 each 120 and 102; 64 of 1408 x 2048, 96 each
+    # 355 and 293; 16 of 512 x 1024, 0.5 - 1 tiles per CU, 38 each 25 and 35, 188 each 36 and 43)
+    rows = 64
+    if h.dtype == torch.bfloat16:
+        if aligned and K % 64 == 0 and F % 64 == 0:
+            rows = 128 if P >= 64 * E and (P // 128 + E // 2) * -(-F // (128 if act == "gelu" else 64)) >= 384 else 64
+        elif P >= 128 * E:
+            rows = 128
     # experts with still more rows each: the dense GEMMs' 256 x 256 tiles; gate and up in one matrix (interleaved) or in two
     pp = (h.dtype == torch.bfloat16 and P >= (MOE_PP_ROWS if gate is None else MOE_PP_ROWS_TWO) * E
           and min(F, N) >= 256 and F % 8 == 0 and K % 8 == 0 and aligned and _MOE_PP)

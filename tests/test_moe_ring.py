@@ -1,0 +1,41 @@
+"""Grouped expert products through the ring of k-steps (csrc/gemm_tile.hip): experts with no rows, one row, and rows about the edges of
+64- and 128-row tiles, columns that end within a tile, fewer k-steps than the ring is deep, against plain products in 32 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+RAGGED = [0, 1, 63, 64, 65, 127, 128, 129, 200, 17]
+
+
+@pytest.mark.parametrize("kind", ["gelu", "interleaved", "silu", "weighted"])
+# rows of each expert, F, K, rows of a tile (576 columns without a gate: 64)
+@pytest.mark.parametrize("counts,F,K,tile", [(RAGGED, 64, 64, 64), (RAGGED, 192, 128, 64), (RAGGED, 320, 1024, 64), ([9, 30], 128, 192, 64),
+                                             ([64] * 60 + [1, 127, 128, 0], 832, 64, 128), ([100] * 40 + RAGGED, 576, 320, 128),
+                                             ([70] * 32, 64, 256, 64)])
+def test_ring_of_steps(kind, counts, F, K, tile):
+    from llmss_amd.ops import glu_interleave, hip
+    E, P = len(counts), sum(counts)
+    cols = -(-F // (128 if kind == "gelu" and F > 576 else 64))
+    assert P > hip.MOE_DEC_ROWS * E and (tile == 128) == (P >= 64 * E and (P // 128 + E // 2) * cols >= 384)
+    g = torch.Generator().manual_seed(P + F)
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(P, generator=g)].int().view(P, 1).cuda()
+    wide = torch.randn(P, K + 8, generator=g).bfloat16().cuda()
+    h, w = wide[:, :K], torch.rand(P, 1, generator=g).cuda() + 0.5
+    gate, up, down = (torch.randn(E, a, b, generator=g).mul(b ** -0.5).bfloat16().cuda() for a, b in ((F, K), (F, K), (K, F)))
+    if kind == "gelu":
+        y = hip.moe_experts(h, idx, w, None, up, down, 0.0, 0.0, act="gelu")
+    elif kind == "interleaved":
+        y = hip.moe_experts(h, idx, w, None, glu_interleave(gate, up, 1).contiguous(), down, 0.0, 0.0, act="silu", interleaved=True)
+    else:
+        y = hip.moe_experts(h, idx, w, gate, up, down, 0.0, 0.0, act="silu", weight_input=kind == "weighted")
+    want = torch.zeros(P, K, device="cuda")
+    for e in range(E):
+        r = (idx[:, 0] == e).nonzero()[:, 0]
+        s = w[r] if kind == "weighted" else 1.0
+        u = h[r].float() @ up[e].float().t() * s
+        a = torch.nn.functional.gelu(u) if kind == "gelu" else torch.nn.functional.silu(h[r].float() @ gate[e].float().t() * s) * u
+        want[r] = a.bfloat16().float() @ down[e].float().t() * (1.0 if kind == "weighted" else w[r])
+    # sums in 32 bits on both sides; an activation that lies near the middle of two bf16 numbers may round to the other (2^-8 of it, few do)
+    assert ((y - want).norm() / want.norm()).item() < 2.0 ** -10
+    assert (y - want).abs().max() <= 2.0 ** -7 * want.abs().max()
