@@ -207,10 +207,9 @@ __global__ __launch_bounds__(256, BM * BN > 128 * 128 ? 2 : 1) void gemm_tile_ke
 // two bytes lie on few memory channels, which all tiles would otherwise walk together (32 experts of 768 x 2048, 80 rows each: 100 -> 94 us of
 // both products; by row tile instead, tiles that share an expert's weights lose each other: 188 rows each 151 -> 158). us of both products
 // against the kernel above: 16 experts of 512 x 1024, 38 rows each 33.2 -> 24.6; 32 of 768 x 2048, 80 rows 120 -> 94, 103 rows 117 -> 99; 64 of
-// 1408 x 2048, 96 rows 360 -> 294, 66 rows 321 -> 277; over 69 random layers (8 - 128 experts, 9 - 260 rows each) 0.82 of the time, 1.06 at worst
-// (before the k-steps were spread). Depth: three steps where the tiles then run at once, else two, so that three workgroups share a CU
-// (above 512 tiles: 640 x 4 rows over 32 experts 118 -> 103 us, below, 400 x 4 rows, 97 -> 91 with three); four or six steps were slower
-// everywhere (822 x 4 rows: 127 and 139 against 120). 128 rows: 128 x 128 tiles for one matrix (64 and 256 columns 111 and 105 against 102 us).
+// 1408 x 2048, 96 rows 360 -> 294, 66 rows 321 -> 277; over 108 random layers (8 - 128 experts, 9 - 130 rows each) 0.81 of the time, 1.08 at
+// worst. Four or six steps were slower everywhere (822 x 4 rows over 32 experts: 127 and 139 against 120). 128 rows: 128 x 128 tiles for one
+// matrix (64 and 256 columns 111 and 105 against 102 us).
 template <int MODE, typename TC, int BM, int BN, int NS>
 __global__ __launch_bounds__(256) void moe_ring_kernel(GemmTileArgs p) {
   constexpr int MB = BM / 32, NB = BN / 32;
@@ -355,14 +354,21 @@ static bool moe_ring_ok(const GemmTileArgs& a, int64_t lda, int64_t rows, int64_
          (rows + 1) * lda * 2 < (1ll << 31) && wrows * a.K * 2 < (1ll << 31);
 }
 
-// 64-row tiles: three steps deep where the list's tiles (about maxt - E / 2) then still run at once, else two
+// 64-row tiles: three steps deep where the list's tiles (a row tile an expert, or half of one beside the full ones) then still run at once,
+// else two. More tiles than that of few rows each are bound by the weights alone, and up to half a wave more would run after the others:
+// those stay on the kernel above, of which more workgroups share a CU (us of both products, there and here: 64 experts of 960 x 1280, 19 rows
+// each 105 and 124, of 896 x 768, 55 rows each 79 and 86; 128 of 512 x 2048, 16 rows each 172 and 191).
 template <int MODE, typename TC>
-static void moe_ring64(const GemmTileArgs& a, hipStream_t st) {
-  const int cols = (a.N + 63) / 64;
+static bool moe_ring64(const GemmTileArgs& a, hipStream_t st) {
   constexpr int slot = MODE == GT_GATE_UP ? 24 : 16;  // KB
+  constexpr int at3 = 256 * (160 / (3 * slot)), at2 = 256 * (160 / (2 * slot));
+  const int cols = (a.N + 63) / 64;
+  const int64_t tiles = (int64_t)std::max(std::min(a.E, a.maxt), a.maxt - a.E / 2) * cols;
+  if (tiles > at2 && (2 * (a.maxt - a.E) < a.E || 2 * tiles <= 3 * at2)) return false;
   const dim3 g(cols, a.maxt);
-  if ((int64_t)(a.maxt - std::min(a.E / 2, a.maxt / 2)) * cols <= 256 * (160 / (3 * slot))) moe_ring_kernel<MODE, TC, 64, 64, 3><<<g, 256, 0, st>>>(a);
+  if (tiles <= at3) moe_ring_kernel<MODE, TC, 64, 64, 3><<<g, 256, 0, st>>>(a);
   else moe_ring_kernel<MODE, TC, 64, 64, 2><<<g, 256, 0, st>>>(a);
+  return true;
 }
 
 // act[r, f] = glu(h[order[r] / top] . gate_e[f], h[..] . up_e[f]) over the tile list (bf16), or gelu(h[..] . up_e[f])
@@ -389,28 +395,22 @@ void launch_moe_gate_up_tile(const void* h, int64_t ldh, const void* wg, const v
   // workgroup per CU; at 128x64 two to three fit and hide each other's staging
   if (!wg) {
     a.B = (const bf16_t*)wu; a.B2 = nullptr;
-    if (moe_ring_ok(a, ldh, (int64_t)maxt * tile_rows / top, F)) {
-      if (tile_rows == 64) moe_ring64<GT_UP, bf16_t>(a, st);
-      else moe_ring_kernel<GT_UP, bf16_t, 128, 128, 2><<<dim3((F + 127) / 128, maxt), 256, 0, st>>>(a);
-      HIP_CHECK_LAUNCH();
-      return;
-    }
+    const bool ring = moe_ring_ok(a, ldh, (int64_t)maxt * tile_rows / top, F);
     const int bn = tile_rows == 128 && F >= 512 ? 256 : tile_rows;
     dim3 g((F + bn - 1) / bn, maxt);
-    if (bn == 256) gemm_tile_kernel<GT_UP, bf16_t, 128, 256><<<g, 256, 0, st>>>(a);
+    if (ring && tile_rows == 128) moe_ring_kernel<GT_UP, bf16_t, 128, 128, 2><<<dim3((F + 127) / 128, maxt), 256, 0, st>>>(a);
+    else if (ring && moe_ring64<GT_UP, bf16_t>(a, st)) {}
+    else if (bn == 256) gemm_tile_kernel<GT_UP, bf16_t, 128, 256><<<g, 256, 0, st>>>(a);
     else if (tile_rows == 128) gemm_tile_kernel<GT_UP, bf16_t, 128, 128><<<g, 256, 0, st>>>(a);
     else gemm_tile_kernel<GT_UP, bf16_t, 64, 64><<<g, 256, 0, st>>>(a);
     HIP_CHECK_LAUNCH();
     return;
   }
   dim3 g((F + 63) / 64, maxt);
-  if (moe_ring_ok(a, ldh, (int64_t)maxt * tile_rows / top, (int64_t)(ilv ? 2 : 1) * F)) {
-    if (tile_rows == 128) moe_ring_kernel<GT_GATE_UP, bf16_t, 128, 64, 2><<<g, 256, 0, st>>>(a);
-    else moe_ring64<GT_GATE_UP, bf16_t>(a, st);
-    HIP_CHECK_LAUNCH();
-    return;
-  }
-  if (tile_rows == 128) gemm_tile_kernel<GT_GATE_UP, bf16_t, 128, 64><<<g, 256, 0, st>>>(a);
+  const bool ring = moe_ring_ok(a, ldh, (int64_t)maxt * tile_rows / top, (int64_t)(ilv ? 2 : 1) * F);
+  if (ring && tile_rows == 128) moe_ring_kernel<GT_GATE_UP, bf16_t, 128, 64, 2><<<g, 256, 0, st>>>(a);
+  else if (ring && moe_ring64<GT_GATE_UP, bf16_t>(a, st)) {}
+  else if (tile_rows == 128) gemm_tile_kernel<GT_GATE_UP, bf16_t, 128, 64><<<g, 256, 0, st>>>(a);
   else gemm_tile_kernel<GT_GATE_UP, bf16_t, 64, 64><<<g, 256, 0, st>>>(a);
   HIP_CHECK_LAUNCH();
 }
@@ -427,13 +427,10 @@ void launch_moe_down_tile(const void* act, const void* wd, const void* meta, voi
   a.meta = (const int*)meta; a.E = E; a.maxt = maxt; a.top = 1;
   const int bn = tile_rows == 128 && N >= 512 ? 256 : tile_rows;
   dim3 g((N + bn - 1) / bn, maxt);
-  if (moe_ring_ok(a, F, (int64_t)maxt * tile_rows, N)) {
-    if (tile_rows == 64) moe_ring64<GT_DOWN, float>(a, st);
-    else moe_ring_kernel<GT_DOWN, float, 128, 128, 2><<<dim3((N + 127) / 128, maxt), 256, 0, st>>>(a);
-    HIP_CHECK_LAUNCH();
-    return;
-  }
-  if (bn == 256) gemm_tile_kernel<GT_DOWN, float, 128, 256><<<g, 256, 0, st>>>(a);
+  const bool ring = moe_ring_ok(a, F, (int64_t)maxt * tile_rows, N);
+  if (ring && tile_rows == 128) moe_ring_kernel<GT_DOWN, float, 128, 128, 2><<<dim3((N + 127) / 128, maxt), 256, 0, st>>>(a);
+  else if (ring && moe_ring64<GT_DOWN, float>(a, st)) {}
+  else if (bn == 256) gemm_tile_kernel<GT_DOWN, float, 128, 256><<<g, 256, 0, st>>>(a);
   else if (tile_rows == 128) gemm_tile_kernel<GT_DOWN, float, 128, 128><<<g, 256, 0, st>>>(a);
   else gemm_tile_kernel<GT_DOWN, float, 64, 64><<<g, 256, 0, st>>>(a);
   HIP_CHECK_LAUNCH();

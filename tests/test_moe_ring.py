@@ -12,11 +12,12 @@ RAGGED = [0, 1, 63, 64, 65, 127, 128, 129, 200, 17]
 # rows of each expert, F, K, rows of a tile (576 columns without a gate: 64)
 @pytest.mark.parametrize("counts,F,K,tile", [(RAGGED, 64, 64, 64), (RAGGED, 192, 128, 64), (RAGGED, 320, 1024, 64), ([9, 30], 128, 192, 64),
                                              ([64] * 60 + [1, 127, 128, 0], 832, 64, 128), ([100] * 40 + RAGGED, 576, 320, 128),
-                                             ([70] * 32, 64, 256, 64)])
+                                             ([70] * 32, 64, 256, 64), ([300, 400, 129, 500, 1, 200, 64, 350], 256, 256, 64), ([20] * 60, 896, 64, 64)])
 def test_ring_of_steps(kind, counts, F, K, tile):
     from llmss_amd.ops import glu_interleave, hip
     E, P = len(counts), sum(counts)
     cols = -(-F // (128 if kind == "gelu" and F > 576 else 64))
+    assert hip._moe_pp_fill(P, E, F if kind == "gelu" else 2 * F, K, K, F) < hip.MOE_PP_FILL or P < hip.MOE_PP_ROWS * E
     assert P > hip.MOE_DEC_ROWS * E and (tile == 128) == (P >= 64 * E and (P // 128 + E // 2) * cols >= 384)
     g = torch.Generator().manual_seed(P + F)
     idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(P, generator=g)].int().view(P, 1).cuda()
