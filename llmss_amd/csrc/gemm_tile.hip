@@ -37,6 +37,7 @@ struct GemmTileArgs {
   int silu;         // GATE_UP: silu(g) * u instead of the clamped form
   int ilv;          // GATE_UP: one weight matrix, gate and up rows in alternating groups of 16 (B the first gate row, B2 the first up row)
   const bf16_t* bias;  // PLAIN: [N] or null
+  int wide;            // PLAIN, bf16 results in the ring kernel: rows and columns in pieces of 16 bytes
 };
 
 // 8 consecutive k of one row (zero beyond the row / k range)
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(256, BM * BN > 128 * 128 ? 2 : 1) void gemm_tile_ke
     }
 }
 
-// The grouped products with whole k-steps and rows of 16-byte alignment: as above, but operands go straight to a ring of NS k-steps in
+// Products with whole k-steps and rows of 16-byte alignment: as above, but operands go straight to a ring of NS k-steps in
 // LDS, NS - 1 of them on their way, one barrier a step; 8 rows x 128 bytes a load, chunks XOR-swizzled by row so that fragment reads meet
 // no bank conflict. Bound by the weights of the experts that the tokens reach and, with few rows each, by the latency of a step: the kernel
 // above waits out one step's loads after each, its two barriers between them. Experts start at different k-steps (e * 11): rows of a power of
@@ -208,10 +209,12 @@ __global__ __launch_bounds__(256, BM * BN > 128 * 128 ? 2 : 1) void gemm_tile_ke
 // both products; by row tile instead, tiles that share an expert's weights lose each other: 188 rows each 151 -> 158). us of both products
 // against the kernel above: 16 experts of 512 x 1024, 38 rows each 33.2 -> 24.6; 32 of 768 x 2048, 80 rows 120 -> 94, 103 rows 117 -> 99; 64 of
 // 1408 x 2048, 96 rows 360 -> 294, 66 rows 321 -> 277; over 108 random layers (8 - 128 experts, 9 - 130 rows each) 0.81 of the time, 1.08 at
-// worst. Four or six steps were slower everywhere (822 x 4 rows over 32 experts: 127 and 139 against 120). 128 rows: 128 x 128 tiles for one
+// worst. Batched and 32-bit-result products (PLAIN), whose K of 128 - 256 is on its way whole and whose bf16 results leave in 16-byte pieces
+// instead of two bytes a lane: 16 heads of 8261 x 256 x 128 45.5 -> 35.6 us, x 128 x 256 37.8 -> 28.4, one of 8261 x 4096 x 1024 in 32 bits 143 -> 112,
+// 64 x 2048 x 2048 23.2 -> 11.6, 8 x 2048 x 1024 12.2 -> 7.3. Four or six steps were slower everywhere (822 x 4 rows over 32 experts: 127 and 139 against 120). 128 rows: 128 x 128 tiles for one
 // matrix (64 and 256 columns 111 and 105 against 102 us).
 template <int MODE, typename TC, int BM, int BN, int NS>
-__global__ __launch_bounds__(256) void moe_ring_kernel(GemmTileArgs p) {
+__global__ __launch_bounds__(256) void tile_ring_kernel(GemmTileArgs p) {
   constexpr int MB = BM / 32, NB = BN / 32;
   constexpr bool DUAL = MODE == GT_GATE_UP;
   constexpr int AI = BM / 32, BI = (DUAL ? 2 : 1) * BN / 32;  // 1-KiB loads (8 rows of a k-step) of a wave
@@ -221,13 +224,21 @@ __global__ __launch_bounds__(256) void moe_ring_kernel(GemmTileArgs p) {
   const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = (w >> 1) * (BM / 2), wn = (w & 1) * (BN / 2);
-  if ((int)blockIdx.y >= p.meta[0]) return;
-  const int id = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, p.meta[0] * gridDim.x);
-  const int ty = id / gridDim.x, n0 = (id % gridDim.x) * BN;
-  const int e = p.meta[1 + (p.E + 1) + ty], crow0 = p.meta[1 + (p.E + 1) + p.maxt + ty];
-  const int rows = min(BM, p.meta[1 + e + 1] - crow0);
+  constexpr bool PLAIN = MODE == GT_PLAIN;
+  int n0 = blockIdx.x * BN, e = blockIdx.z, crow0 = blockIdx.y * BM, rows = min(BM, p.M - crow0);
+  const bf16_t* A = p.A;
+  if constexpr (PLAIN) {
+    A += (int64_t)e * p.sAb + (int64_t)crow0 * p.sAm;
+  } else {
+    if ((int)blockIdx.y >= p.meta[0]) return;
+    const int id = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, p.meta[0] * gridDim.x);
+    const int ty = id / gridDim.x;
+    n0 = (id % gridDim.x) * BN;
+    e = p.meta[1 + (p.E + 1) + ty], crow0 = p.meta[1 + (p.E + 1) + p.maxt + ty];
+    rows = min(BM, p.meta[1 + e + 1] - crow0);
+  }
 
-  const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(p.A)), (short)0, 0x7fffffff, 0x00020000);
+  const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(A)), (short)0, 0x7fffffff, 0x00020000);
   const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(p.B + (int64_t)e * p.sBb)), (short)0,
                                                     0x7fffffff, 0x00020000);
   const auto rb2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>((DUAL ? p.B2 : p.B) + (int64_t)e * p.sBb)),
@@ -240,7 +251,7 @@ __global__ __launch_bounds__(256) void moe_ring_kernel(GemmTileArgs p) {
     const int sr = sr0 + 32 * i;
     va[i] = 0x80000000u;
     if (sr < rows) {
-      const int row = MODE == GT_DOWN ? crow0 + sr : p.order[crow0 + sr] / p.top;
+      const int row = PLAIN ? sr : MODE == GT_DOWN ? crow0 + sr : p.order[crow0 + sr] / p.top;
       va[i] = (uint32_t)(row * p.sAm * 2 + ch);
     }
   }
@@ -250,7 +261,7 @@ __global__ __launch_bounds__(256) void moe_ring_kernel(GemmTileArgs p) {
     vb[i] = n < p.N ? (uint32_t)(row * p.sBn * 2 + ch) : 0x80000000u;
   }
   const int nk = p.K / 64;
-  const int k0 = (e * 11) % nk;
+  const int k0 = PLAIN ? 0 : (e * 11) % nk;
 #define MR_ISSUE(T_, S_)                                                                                                          \
   do {                                                                                                                            \
     const int q_ = (T_) + k0 >= nk ? (T_) + k0 - nk : (T_) + k0;                                                                   \
@@ -305,6 +316,31 @@ __global__ __launch_bounds__(256) void moe_ring_kernel(GemmTileArgs p) {
 #undef MR_ISSUE
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (loads past the last step write zeros to LDS)
   TC* C = (TC*)p.C;
+  if constexpr (PLAIN) C += (int64_t)e * p.sCb;
+  if constexpr (PLAIN && sizeof(TC) == 2) {
+    if (p.wide) {  // bf16 results in whole 16-byte pieces, through LDS
+      constexpr int LD = BN + 8;
+      static_assert(BM * LD * 2 <= NS * SLOT, "the tile's image");
+      bf16_t* im = reinterpret_cast<bf16_t*>(smem);
+      __syncthreads();  // every wave's fragment reads are done
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const int n = n0 + wn + 16 * j + li;
+          const float b = p.bias && n < p.N ? bf2f(p.bias[n]) : 0.f;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) El<TC>::st(im + (wm + 16 * i + 4 * g + q) * LD + wn + 16 * j + li, acc[i][j][q] + b);
+        }
+      __syncthreads();
+      for (int c = threadIdx.x; c < BM * BN / 8; c += 256) {
+        const int row = c / (BN / 8), col = c % (BN / 8) * 8;
+        if (row < rows && n0 + col < p.N)
+          *reinterpret_cast<u16x8*>(C + (int64_t)(crow0 + row) * p.sCm + n0 + col) = *reinterpret_cast<const u16x8*>(im + row * LD + col);
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -313,7 +349,7 @@ __global__ __launch_bounds__(256) void moe_ring_kernel(GemmTileArgs p) {
       if (r >= rows) continue;
       TC* crow = C + (int64_t)(crow0 + r) * p.sCm;
       float sw = 1.0f;
-      if constexpr (MODE != GT_DOWN) sw = p.pw ? p.pw[p.order[crow0 + r]] : 1.0f;
+      if constexpr (MODE != GT_DOWN && !PLAIN) sw = p.pw ? p.pw[p.order[crow0 + r]] : 1.0f;
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
         const int n = n0 + wn + 16 * j + li;
@@ -321,6 +357,7 @@ __global__ __launch_bounds__(256) void moe_ring_kernel(GemmTileArgs p) {
         float v = acc[i][j][q];
         if constexpr (DUAL) v = glu_clamped_t(v * sw, acc2[i][j][q] * sw, p.limit, p.alpha, p.silu);
         if constexpr (MODE == GT_UP) v = gelu_erf(v * sw);
+        if constexpr (PLAIN) v += p.bias ? bf2f(p.bias[n]) : 0.f;
         El<TC>::st(crow + n, v);
       }
     }
@@ -338,6 +375,21 @@ void launch_gemm_tile(const void* A, const void* B, void* C, int M, int N, int K
   a.bias = (const bf16_t*)bias;
   dim3 g((N + T - 1) / T, (M + T - 1) / T, batch);
   if (dc != 0 && dc != 1) throw std::runtime_error("gemm_tile: bad output dtype code");
+  // whole k-steps, rows of 16-byte alignment that fit 31 bits a tile: the ring
+  const bool ring = K > 0 && K % 64 == 0 && !((sAb | sAm | sBb | sBn) & 7) && !(((uintptr_t)A | (uintptr_t)B) & 15) && sAm >= 0 && sBn >= 0 &&
+                    std::max(sAm, sBn) < (1 << 22) && K < (1 << 22);
+  if (ring) {
+    a.wide = N % 8 == 0 && !((sCb | sCm) & 7) && !((uintptr_t)C & 15);
+    if (T == 128) {
+      if (dc == 0) tile_ring_kernel<GT_PLAIN, bf16_t, 128, 128, 2><<<g, 256, 0, st>>>(a);
+      else tile_ring_kernel<GT_PLAIN, float, 128, 128, 2><<<g, 256, 0, st>>>(a);
+    } else {
+      if (dc == 0) tile_ring_kernel<GT_PLAIN, bf16_t, 64, 64, 3><<<g, 256, 0, st>>>(a);
+      else tile_ring_kernel<GT_PLAIN, float, 64, 64, 3><<<g, 256, 0, st>>>(a);
+    }
+    HIP_CHECK_LAUNCH();
+    return;
+  }
   if (T == 128) {
     if (dc == 0) gemm_tile_kernel<GT_PLAIN, bf16_t, 128, 128><<<g, 256, 0, st>>>(a);
     else gemm_tile_kernel<GT_PLAIN, float, 128, 128><<<g, 256, 0, st>>>(a);
@@ -366,8 +418,8 @@ static bool moe_ring64(const GemmTileArgs& a, hipStream_t st) {
   const int64_t tiles = (int64_t)std::max(std::min(a.E, a.maxt), a.maxt - a.E / 2) * cols;
   if (tiles > at2 && (2 * (a.maxt - a.E) < a.E || 2 * tiles <= 3 * at2)) return false;
   const dim3 g(cols, a.maxt);
-  if (tiles <= at3) moe_ring_kernel<MODE, TC, 64, 64, 3><<<g, 256, 0, st>>>(a);
-  else moe_ring_kernel<MODE, TC, 64, 64, 2><<<g, 256, 0, st>>>(a);
+  if (tiles <= at3) tile_ring_kernel<MODE, TC, 64, 64, 3><<<g, 256, 0, st>>>(a);
+  else tile_ring_kernel<MODE, TC, 64, 64, 2><<<g, 256, 0, st>>>(a);
   return true;
 }
 
@@ -398,7 +450,7 @@ void launch_moe_gate_up_tile(const void* h, int64_t ldh, const void* wg, const v
     const bool ring = moe_ring_ok(a, ldh, (int64_t)maxt * tile_rows / top, F);
     const int bn = tile_rows == 128 && F >= 512 ? 256 : tile_rows;
     dim3 g((F + bn - 1) / bn, maxt);
-    if (ring && tile_rows == 128) moe_ring_kernel<GT_UP, bf16_t, 128, 128, 2><<<dim3((F + 127) / 128, maxt), 256, 0, st>>>(a);
+    if (ring && tile_rows == 128) tile_ring_kernel<GT_UP, bf16_t, 128, 128, 2><<<dim3((F + 127) / 128, maxt), 256, 0, st>>>(a);
     else if (ring && moe_ring64<GT_UP, bf16_t>(a, st)) {}
     else if (bn == 256) gemm_tile_kernel<GT_UP, bf16_t, 128, 256><<<g, 256, 0, st>>>(a);
     else if (tile_rows == 128) gemm_tile_kernel<GT_UP, bf16_t, 128, 128><<<g, 256, 0, st>>>(a);
@@ -408,7 +460,7 @@ void launch_moe_gate_up_tile(const void* h, int64_t ldh, const void* wg, const v
   }
   dim3 g((F + 63) / 64, maxt);
   const bool ring = moe_ring_ok(a, ldh, (int64_t)maxt * tile_rows / top, (int64_t)(ilv ? 2 : 1) * F);
-  if (ring && tile_rows == 128) moe_ring_kernel<GT_GATE_UP, bf16_t, 128, 64, 2><<<g, 256, 0, st>>>(a);
+  if (ring && tile_rows == 128) tile_ring_kernel<GT_GATE_UP, bf16_t, 128, 64, 2><<<g, 256, 0, st>>>(a);
   else if (ring && moe_ring64<GT_GATE_UP, bf16_t>(a, st)) {}
   else if (tile_rows == 128) gemm_tile_kernel<GT_GATE_UP, bf16_t, 128, 64><<<g, 256, 0, st>>>(a);
   else gemm_tile_kernel<GT_GATE_UP, bf16_t, 64, 64><<<g, 256, 0, st>>>(a);
@@ -428,7 +480,7 @@ void launch_moe_down_tile(const void* act, const void* wd, const void* meta, voi
   const int bn = tile_rows == 128 && N >= 512 ? 256 : tile_rows;
   dim3 g((N + bn - 1) / bn, maxt);
   const bool ring = moe_ring_ok(a, F, (int64_t)maxt * tile_rows, N);
-  if (ring && tile_rows == 128) moe_ring_kernel<GT_DOWN, float, 128, 128, 2><<<dim3((N + 127) / 128, maxt), 256, 0, st>>>(a);
+  if (ring && tile_rows == 128) tile_ring_kernel<GT_DOWN, float, 128, 128, 2><<<dim3((N + 127) / 128, maxt), 256, 0, st>>>(a);
   else if (ring && moe_ring64<GT_DOWN, float>(a, st)) {}
   else if (bn == 256) gemm_tile_kernel<GT_DOWN, float, 128, 256><<<g, 256, 0, st>>>(a);
   else if (tile_rows == 128) gemm_tile_kernel<GT_DOWN, float, 128, 128><<<g, 256, 0, st>>>(a);
