@@ -211,8 +211,8 @@ __global__ __launch_bounds__(256, BM * BN > 128 * 128 ? 2 : 1) void gemm_tile_ke
 // 1408 x 2048, 96 rows 360 -> 294, 66 rows 321 -> 277; over 108 random layers (8 - 128 experts, 9 - 130 rows each) 0.81 of the time, 1.08 at
 // worst. Batched and 32-bit-result products (PLAIN), whose K of 128 - 256 is on its way whole and whose bf16 results leave in 16-byte pieces
 // instead of two bytes a lane: 16 heads of 8261 x 256 x 128 45.5 -> 35.6 us, x 128 x 256 37.8 -> 28.4, one of 8261 x 4096 x 1024 in 32 bits 143 -> 112,
-// 64 x 2048 x 2048 23.2 -> 11.6, 8 x 2048 x 1024 12.2 -> 7.3. Four or six steps were slower everywhere (822 x 4 rows over 32 experts: 127 and 139 against 120). 128 rows: 128 x 128 tiles for one
-// matrix (64 and 256 columns 111 and 105 against 102 us).
+// 64 x 2048 x 2048 23.2 -> 11.6, 8 x 2048 x 1024 12.2 -> 7.3. Four or six steps were slower everywhere (822 x 4 rows over 32 experts: 127 and 139
+// against 120). 128 rows: 128 x 128 tiles for one matrix (64 and 256 columns 111 and 105 against 102 us).
 template <int MODE, typename TC, int BM, int BN, int NS>
 __global__ __launch_bounds__(256) void tile_ring_kernel(GemmTileArgs p) {
   constexpr int MB = BM / 32, NB = BN / 32;
