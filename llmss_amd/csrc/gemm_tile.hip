@@ -239,11 +239,14 @@ __global__ __launch_bounds__(256) void tile_ring_kernel(GemmTileArgs p) {
   }
 
   const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(A)), (short)0, 0x7fffffff, 0x00020000);
-  const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(p.B + (int64_t)e * p.sBb)), (short)0,
-                                                    0x7fffffff, 0x00020000);
+  // PLAIN: of B too from the tile's own first row on, so that 31 bits hold a tile's rows whatever the matrix's size
+  const int b0 = PLAIN ? n0 : 0;
+  const auto rb = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char*>(reinterpret_cast<const char*>(p.B + (int64_t)e * p.sBb + (int64_t)b0 * p.sBn)), (short)0, 0x7fffffff, 0x00020000);
   const auto rb2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>((DUAL ? p.B2 : p.B) + (int64_t)e * p.sBb)),
                                                      (short)0, 0x7fffffff, 0x00020000);
-  // wave w takes rows 8 (w + 4 i) .. + 7 of each operand; past the rows or columns: an offset that reads as zero
+  // wave w takes rows 8 (w + 4 i) .. + 7 of each operand; past the rows or columns, or past the last step: an offset that reads as zero (past
+  // both the two offsets wrap to the operand's first bytes, which are there and land where nobody reads)
   uint32_t va[AI], vb[BN / 32];
   const int sr0 = 8 * w + (lane >> 3), ch = ((lane & 7) ^ (sr0 & 7)) << 4;
 #pragma unroll
@@ -257,7 +260,7 @@ __global__ __launch_bounds__(256) void tile_ring_kernel(GemmTileArgs p) {
   }
 #pragma unroll
   for (int i = 0; i < BN / 32; ++i) {
-    const int n = n0 + sr0 + 32 * i, row = DUAL && p.ilv ? (n >> 4) * 32 + (n & 15) : n;
+    const int n = n0 + sr0 + 32 * i, row = DUAL && p.ilv ? (n >> 4) * 32 + (n & 15) : n - b0;
     vb[i] = n < p.N ? (uint32_t)(row * p.sBn * 2 + ch) : 0x80000000u;
   }
   const int nk = p.K / 64;
@@ -314,7 +317,7 @@ __global__ __launch_bounds__(256) void tile_ring_kernel(GemmTileArgs p) {
     slot = slot == NS - 1 ? 0 : slot + 1;
   }
 #undef MR_ISSUE
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (loads past the last step write zeros to LDS)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (loads past the last step write to LDS too)
   TC* C = (TC*)p.C;
   if constexpr (PLAIN) C += (int64_t)e * p.sCb;
   if constexpr (PLAIN && sizeof(TC) == 2) {
@@ -375,7 +378,7 @@ void launch_gemm_tile(const void* A, const void* B, void* C, int M, int N, int K
   a.bias = (const bf16_t*)bias;
   dim3 g((N + T - 1) / T, (M + T - 1) / T, batch);
   if (dc != 0 && dc != 1) throw std::runtime_error("gemm_tile: bad output dtype code");
-  // whole k-steps, rows of 16-byte alignment that fit 31 bits a tile: the ring
+  // whole k-steps, rows of 16-byte alignment of which a tile's 128, of either operand, fit 31 bits: the ring
   const bool ring = K > 0 && K % 64 == 0 && !((sAb | sAm | sBb | sBn) & 7) && !(((uintptr_t)A | (uintptr_t)B) & 15) && sAm >= 0 && sBn >= 0 &&
                     std::max(sAm, sBn) < (1 << 22) && K < (1 << 22);
   if (ring) {

@@ -27,3 +27,21 @@ def test_plain(M, N, K, H, dtype, pad, bias):
     assert ((got - want).abs() <= lim).all()
     C[1:M + 1, pad // 2:pad // 2 + H * N] = 7.0
     assert (C == 7.0).all()
+
+
+# a matrix of 2 GiB and one of 4 GiB, and a few rows more: columns whose rows lie where a 31- or 32-bit offset from its start ends
+@pytest.mark.parametrize("N,K", [(2 ** 18 + 3, 4096), (2 ** 19 + 70, 4096), (2 ** 14 + 66, 2 ** 16)])
+@pytest.mark.parametrize("M,dtype", [(3, torch.float32), (520, torch.bfloat16)])
+def test_plain_large_matrix(N, K, M, dtype):
+    from llmss_amd.ops import hip
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(M, K, generator=g, device="cuda", dtype=torch.bfloat16)
+    w = torch.empty(N, K, device="cuda", dtype=torch.bfloat16).normal_(0, K ** -0.5, generator=g)
+    y = torch.empty(M, N, dtype=dtype, device="cuda")
+    hip.gemm_any(x, w, y, M, N, K, 1, 0, K, 0, K, 1, 0, N)
+    edge = 2 ** 30 // K
+    cols = sorted({c for at in (0, edge, 2 * edge, N // 2, N - 4) for c in range(at - 70, at + 70) if 0 <= c < N})
+    wd, xd = w[cols].double(), x.double()
+    want, size = xd @ wd.t(), xd.abs() @ wd.abs().t()
+    lim = (K + 2) * 2.0 ** -24 * size + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23) * want.abs()
+    assert ((y[:, cols].double() - want).abs() <= lim).all()
