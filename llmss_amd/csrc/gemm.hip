@@ -2213,9 +2213,11 @@ int launch_tiled(const bf16_t* X, int64_t ldx, const void* W, int64_t ldw, const
   if ((tsel == 2 || tsel == 6) && ns > 4) ns = 4;
   if (f8 && tsel == 4) tsel = 1;
   if (tsel == 4) {
-    if (gemm_quad_ok(N, K, ldx, ldw, 256, Y, ldy, 2, g != 0))
+    const bool quad = gemm_quad_ok(N, K, ldx, ldw, 256, Y, ldy, 2, g != 0);
+    if (qe && !quad) throw std::runtime_error("gemm: the QKV epilogue of 256 x 256 tiles needs the four-wave kernel");
+    if (quad)
       launch_gemm_quad(0, X, ldx, (const bf16_t*)W, ldw, B, Y, ldy, M, N, K, act, g, g_big_group_m,
-                       tiles_of(M, N, 256, 256), PpGroup{}, st);
+                       tiles_of(M, N, 256, 256), PpGroup{}, st, qe);
     else
       gemm_pp_kernel<0><<<tiles_of(M, N, 256, 256), 512, 0, st>>>(X, ldx, (const bf16_t*)W, ldw, B, Y, ldy, M, N, K, act, g,
                                                                   g_big_group_m, K & 63 ? zero_page() : nullptr, PpGroup{});
@@ -2356,9 +2358,9 @@ static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int
 
 // QKV projection with the RoPE + paged-KV write in its LDS-staged epilogue (common.h QkvEpi, tuned kind 3).
 // Plan: the hints, else the tuned kind-3 entry, else the static tiled plan; a split plan runs as an in-launch
-// combine (the epilogue needs finished sums). Returns -1 when the shape / plan cannot take the epilogue
-// (stream / big-tile / stream-K plans, neox RoPE on tiles that are not head-aligned, workspace too small) -
-// the caller then runs the plain GEMM and the rope_cache kernel; 0 when launched.
+// combine (the epilogue needs finished sums), a plan of 256 x 256 tiles in the two launches that a product of its size is cut into. Returns -1
+// when the shape / plan cannot take the epilogue (stream / stream-K plans, neox RoPE on 256 x 256 tiles or on tiles that are not head-aligned,
+// heads that do not divide 256 columns, workspace too small) - the caller then runs the plain GEMM and the rope_cache kernel; 0 when launched.
 int launch_gemm_qkv(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, void* y, int64_t ldy,
                     int M, int N, int K, void* workspace, int64_t ws_bytes, int nt_hint, int split_hint,
                     const QkvEpi& qe, hipStream_t st) {
@@ -2387,8 +2389,8 @@ int launch_gemm_qkv(const void* x, int64_t ldx, const void* w, int64_t ldw, cons
     if ((qe.do_rope && qe.style != 1) || 256 % qe.D || !gemm_quad_ok(N, K, ldx, ldw, 256, y, ldy, 2, false)) return -1;
     const GemmCut cut = gemm_cut(M, N, K, false, 0);  // unsplit: the epilogue needs finished sums
     const int rows = cut.rows ? cut.rows : M, cols = cut.cols ? cut.cols : N;
-    launch_gemm_quad(0, (const bf16_t*)x, ldx, (const bf16_t*)w, ldw, (const bf16_t*)bias, (bf16_t*)y, ldy, rows, cols, K, 0, 0,
-                     g_big_group_m, tiles_of(rows, cols, 256, 256), PpGroup{}, st, &qe);
+    launch_tiled((const bf16_t*)x, ldx, w, ldw, (const bf16_t*)bias, (bf16_t*)y, ldy, rows, cols, K, 0, 0, 4, 1, workspace, ws_bytes, false, st,
+                 nullptr, &qe);
     if (rows == M && cols == N) return 0;
     QkvEpi re = qe;  // the rest: its own rows, or the heads from column `cols` on
     if (re.pos) re.pos += rows < M ? rows : 0;
