@@ -1893,10 +1893,11 @@ static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int
 // cuts, 257 - 10000 rows and whole steps of k, two launches take 0.886 of the time from K = 1024 on, 1.11 at worst. Below, a tile's start and end
 // are half of it, and what is promised up to there does not come: gated products 0.87 (0.98 at worst), others 0.954 where more than 6.5 % are
 // promised (95 products; 1.15 at worst, all of those at 6.5 - 10 %: 3764 x 5664 x 256 27 -> 31), 1.02 where less, so those stay whole.
-// The rest's tiles can be too few for the chip (69 x 2048: 32 of 64 x 128, each alone with all of K): K is split where that promises a tenth
-// of the rest's time, priced as in gemm_static_plan. 390 of 5246 random products; over 158 of them 0.982 of the whole product's time
-// (0.96 up to 3.4 MB of slabs, all but six of the 158 at most 1.01; at worst 1.05 with 28 MB, so those end at 24 MB): 8261 x 2048 x 4096
-// 122.8 -> 108.2 us (its rest 27.4 -> 12.7), x 2560 81.9 -> 73.0, 1240 x 13248 x 3392 110.8 -> 100.6, 909 x 20000 x 12160 464 -> 421.
+// The rest's tiles can be too few for the chip (69 x 2048: 32 of 64 x 128, each alone with all of K): K is split where that is priced a tenth
+// below the best of the tiles looked at before, as in gemm_static_plan, up to 24 MB of slabs. The cut may then lie elsewhere than without splits, but
+// not where that would leave up to 64 rows, whose price is too high (4106 x 15840 x 11520, ten rows left or 480 columns 1110 and 1180 us).
+// Over 552 random products that a split changes, 257 - 10000 rows, 0.953 of the time without, five above 1.01, 1.025 at worst (2579 x 7120 x 8576):
+// 8261 x 2048 x 4096 152 -> 132 us, x 2560 100 -> 91, 1240 x 13248 x 3392 133 -> 118.
 struct GemmCut {
   int rows, cols;  // of the first launch; 0: not cut
   int hint;        // plan of the second (0: the plan of its size)
@@ -1914,7 +1915,7 @@ static GemmCut gemm_cut(int M, int N, int K, bool glu, int64_t ws_bytes) {
   };
   GemmCut cut{0, 0, 0, 1};
   double best = (K < 1024 && !glu ? 0.935 : 0.97) * tiles_us(kTileCost[0], M, N);
-  auto consider = [&](int rows, int cols) {
+  auto consider = [&](int rows, int cols, bool splits) {
     if (rows <= 0 || cols <= 0 || (rows >= M && cols >= N)) return;
     const int last = (rows < M ? rows / 256 * ntn : ntm * (cols / 256)) % 256;
     if (last && last < 218) return;  // whole waves, the last of them at least 0.85 full
@@ -1924,7 +1925,7 @@ static GemmCut gemm_cut(int M, int N, int K, bool glu, int64_t ws_bytes) {
     for (const TileCost& c : kTileCost) {
       if (m <= 64) break;
       for (int s : {1, 2, 3, 4, 6, 8}) {
-        if (s > 1 && (c.tsel == 4 || K / s < 256 || (int64_t)s * m * n * 4 > std::min<int64_t>(ws_bytes, 24 << 20))) break;
+        if (s > 1 && (!splits || c.tsel == 4 || K / s < 256 || (int64_t)s * m * n * 4 > std::min<int64_t>(ws_bytes, 24 << 20))) break;
         const double t = tiles_us(c, m, n, s);
         if (!hint || t < (s > split ? 0.9 : 1.0) * rest) rest = t, hint = c.tsel << 8, split = s;
       }
@@ -1933,11 +1934,14 @@ static GemmCut gemm_cut(int M, int N, int K, bool glu, int64_t ws_bytes) {
     if (t < best) best = t, cut = GemmCut{rows < M ? rows : 0, cols < N ? cols : 0, hint, split};
   };
   const int waves = (int)std::min<int64_t>((int64_t)ntm * ntn / 256, 64);
-  for (int w = 1; w <= waves; ++w) {
-    consider(256 * w / ntn * 256, N);
-    consider(M, 256 * w / ntm * 256);
+  for (bool splits : {false, true}) {
+    for (int w = 1; w <= waves; ++w) {
+      consider(256 * w / ntn * 256, N, splits);
+      consider(M, 256 * w / ntm * 256, splits);
+    }
+    consider((ntm - 1) * 256, N, splits);
+    if (cut.rows && !cut.hint) break;
   }
-  consider((ntm - 1) * 256, N);
   return cut;
 }
 
