@@ -89,7 +89,8 @@ void launch_gemm_tile(const void* A, const void* B, void* C, int M, int N, int K
                       int64_t sBb, int64_t sBn, int64_t sCb, int64_t sCm, int dc, const void* bias, hipStream_t st);
 void launch_moe_gate_up_tile(const void* h, int64_t ldh, const void* wg, const void* wu, const void* meta,
                              const void* order, void* act, int E, int maxt, int top, int F, int K, float limit,
-                             float alpha, int tile_rows, const void* pw, int silu, int ilv, hipStream_t st);
+                             float alpha, int tile_rows, const void* pw, int silu, int ilv, bool use_ring, hipStream_t st);
+void moe_plan(int P, int E, int F, int N, int K, bool glu, int rows, bool big, int* rows_out, int* ring);
 void launch_moe_pp(int mode, const void* A, int64_t lda, const void* W, const void* meta, const void* order, void* C, int E,
                    int maxt, int top, int N, int K, int act, hipStream_t st);
 bool moe_pp_glu_ok(int64_t ldh, int maxt, int top, int F, int K);
@@ -100,7 +101,7 @@ void launch_moe_dec(int mode, const void* X, int64_t ldx, const void* W, const v
                     void* place, int T, const void* sX, const void* sW, void* sC, void* sD, int64_t sldd, int sN, int sK, int sE,
                     int sinter, float slimit, hipStream_t st);
 void launch_moe_down_tile(const void* act, const void* wd, const void* meta, void* y, int E, int maxt, int N, int F,
-                          int tile_rows, hipStream_t st);
+                          int tile_rows, bool use_ring, hipStream_t st);
 void launch_latent_norm_cache(const void* src, int64_t ld, int off, const void* w, float eps, void* cache,
                               const void* slots, int T_, int R, int rot, int rdims, const void* cs, void* qa,
                               const void* qsrc, int64_t ldq, int H, int qdim, int dt, int dq, hipStream_t st);
@@ -445,9 +446,14 @@ PYBIND11_MODULE(_C, m) {
   });
   m.def("moe_gate_up_tile", [](uintptr_t h, int64_t ldh, uintptr_t wg, uintptr_t wu, uintptr_t meta, uintptr_t order,
                                uintptr_t act, int E, int maxt, int top, int F, int K, float limit, float alpha,
-                               int tile_rows, uintptr_t pw, int silu, int ilv, uintptr_t st) {
+                               int tile_rows, uintptr_t pw, int silu, int ilv, bool use_ring, uintptr_t st) {
     launch_moe_gate_up_tile(CP(h), ldh, CP(wg), CP(wu), CP(meta), CP(order), P(act), E, maxt, top, F, K, limit, alpha,
-                            tile_rows, CP(pw), silu, ilv, S(st));
+                            tile_rows, CP(pw), silu, ilv, use_ring, S(st));
+  });
+  m.def("moe_plan", [](int P, int E, int F, int N, int K, bool glu, int rows, bool big) {  // rows of a tile, products through the ring
+    int r, ring;
+    moe_plan(P, E, F, N, K, glu, rows, big, &r, &ring);
+    return py::make_tuple(r, ring);
   });
   m.def("moe_pp", [](int mode, uintptr_t A, int64_t lda, uintptr_t W, uintptr_t meta, uintptr_t order, uintptr_t C, int E,
                      int maxt, int top, int N, int K, int act, uintptr_t st) {
@@ -466,8 +472,8 @@ PYBIND11_MODULE(_C, m) {
                    P(place), T, CP(sX), CP(sW), P(sC), P(sD), sldd, sN, sK, sE, sinter, slimit, S(st));
   });
   m.def("moe_down_tile", [](uintptr_t act, uintptr_t wd, uintptr_t meta, uintptr_t y, int E, int maxt, int N, int F,
-                            int tile_rows, uintptr_t st) {
-    launch_moe_down_tile(CP(act), CP(wd), CP(meta), P(y), E, maxt, N, F, tile_rows, S(st));
+                            int tile_rows, bool use_ring, uintptr_t st) {
+    launch_moe_down_tile(CP(act), CP(wd), CP(meta), P(y), E, maxt, N, F, tile_rows, use_ring, S(st));
   });
   m.def("latent_norm_cache", [](uintptr_t src, int64_t ld, int off, uintptr_t w, float eps, uintptr_t cache,
                                 uintptr_t slots, int T, int R, int rot, int rdims, uintptr_t cs, uintptr_t qa,

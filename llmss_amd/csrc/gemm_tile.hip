@@ -13,6 +13,8 @@
 // order[] / top, two weight matrices, output glu(gate, up) in bf16), UP (the same with one weight matrix, output
 // gelu(up), the error-function form) and DOWN (grouped: A = the activation rows,
 // fp32 output). The tile list and offsets are those moe_group writes (moe.hip).
+#include <cmath>
+
 #include "anytype.h"
 #include "gemm_quad.h"
 
@@ -410,28 +412,94 @@ static bool moe_ring_ok(const GemmTileArgs& a, int64_t lda, int64_t rows, int64_
 }
 
 // 64-row tiles: three steps deep where the list's tiles (a row tile an expert, or half of one beside the full ones) then still run at once,
-// else two. More tiles than that of few rows each are bound by the weights alone, and up to half a wave more would run after the others:
-// those stay on the kernel above, of which more workgroups share a CU (us of both products, there and here: 64 experts of 960 x 1280, 19 rows
-// each 105 and 124, of 896 x 768, 55 rows each 79 and 86; 128 of 512 x 2048, 16 rows each 172 and 191).
+// else two.
 template <int MODE, typename TC>
-static bool moe_ring64(const GemmTileArgs& a, hipStream_t st) {
+static void moe_ring64(const GemmTileArgs& a, hipStream_t st) {
   constexpr int slot = MODE == GT_GATE_UP ? 24 : 16;  // KB
-  constexpr int at3 = 256 * (160 / (3 * slot)), at2 = 256 * (160 / (2 * slot));
+  constexpr int at3 = 256 * (160 / (3 * slot));
   const int cols = (a.N + 63) / 64;
   const int64_t tiles = (int64_t)std::max(std::min(a.E, a.maxt), a.maxt - a.E / 2) * cols;
-  if (tiles > at2 && (2 * (a.maxt - a.E) < a.E || 2 * tiles <= 3 * at2)) return false;
   const dim3 g(cols, a.maxt);
   if (tiles <= at3) tile_ring_kernel<MODE, TC, 64, 64, 3><<<g, 256, 0, st>>>(a);
   else tile_ring_kernel<MODE, TC, 64, 64, 2><<<g, 256, 0, st>>>(a);
-  return true;
+}
+
+// Rows of a tile for a layer of experts (more than 8 pairs each) whose operands the ring kernel takes, and whether its products take that kernel
+// (bit 0: gate and up, bit 1: down; 128 rows: always). `rows`: what the rule without the ring says, 64 below 128 pairs an expert, 128 from there on,
+// 256 (gemm_quad.hip) where `big` and from 128 pairs on (gate and up in two matrices: 256). That stays unless another form is priced 1.12 times below,
+// and the kernel without the ring, for a product of 64 rows, unless the ring is priced 1.08 times below.
+// A product's price: `at_once` of its tiles share a CU, a step of 64 of k then taking `step` us and `more` for every tile beside the first, behind
+// `begin` a tile; and its weights at `rate`, the two joined as sides of a right triangle (neither hides the other). Beside the products a start, the
+// rows that are gathered, written and read, and the pairs' grouping. Experts get as many rows as if tokens chose at random. Constants fitted over two thirds
+// of 1020 random layers (2 - 200 experts of 64 - 3072 x 128 - 3072, 9 - 600 pairs each, gate and up together, apart or no gate, weights from
+// memory), 4 - 8 % off on average on the other third.
+// Against that rule, over 900 other layers, a third of them with uneven experts: 0.737 of the whole layer's time, five above 1.02, 1.09 at worst (198
+// experts of 192 x 384, uneven, 71 pairs each 50 -> 54 us). By tile counts alone instead of prices, 128 rows from 64 pairs an expert and 384 tiles on: 0.79 over
+// 1020, 54 above 1.02, 1.35 at worst (142 of 768 x 128, 70 pairs each 57 -> 77; now 64 rows, 53 there and here). us without and with: 64 of 896 x 768,
+// 55 pairs each 82 and 89 (stays); 12 of 2176 x 512, 123 each 65 -> 47; 64 of 1408 x 2048, 96 each 405 -> 373.
+struct MoeCost {  // us; bytes per us
+  int rows;
+  double start, rate, row_rate, pair;
+  struct {
+    double step, more, begin;
+    int at_once, bn;
+  } plain, glu;
+};
+static constexpr MoeCost kMoeCost[] = {
+    {64, 14.0, 5.25e6, 5.72e6, 0.243e-3, {0.894, 0.070, 0.0, 5, 64}, {0.999, 0.178, 0.90, 4, 64}},     // without the ring
+    {64, 14.2, 4.93e6, 5.11e6, 0.298e-3, {0.367, 0.213, 0.0, 5, 64}, {0.411, 0.372, 1.33, 3, 64}},     // with it
+    {128, 16.3, 5.87e6, 4.59e6, 0.545e-3, {0.936, 0.127, 2.03, 2, 128}, {0.720, 0.483, 0.55, 2, 64}},
+    {256, 9.67, 5.16e6, 12.7e6, 0.646e-3, {1.350, 0.0, 13.5, 1, 256}, {1.190, 0.0, 6.94, 1, 128}}};
+void moe_plan(int P, int E, int F, int N, int K, bool glu, int rows, bool big, int* rows_out, int* ring) {
+  auto row_tiles = [&](int r) {
+    const double mean = (double)P / E;
+    double t = 0;
+    for (double q : {-1.5, -0.9, -0.5, -0.15, 0.15, 0.5, 0.9, 1.5}) t += std::ceil(std::max(1.0, mean + q * std::sqrt(mean)) / r);
+    return t * E / 8;
+  };
+  auto us = [&](const MoeCost& c, bool up) {
+    const auto& m = up && glu ? c.glu : c.plain;
+    const int cols = up ? F : N, k = up ? K : F;
+    const double wgs = row_tiles(c.rows) * ((cols + m.bn - 1) / m.bn) / 256, nk = (k + 63) / 64;
+    const double full = std::floor(wgs / m.at_once), rest = wgs - full * m.at_once;
+    const double tiles = full * (nk * (m.step + m.more * (m.at_once - 1)) + m.begin) +
+                         (rest > 0 ? nk * (m.step + m.more * (std::max(1.0, rest) - 1)) + m.begin : 0.0);
+    return std::hypot(tiles, 2.0 * E * cols * k * (up && glu ? 2 : 1) / c.rate) + (double)P * (up ? 2.0 * F + 2.0 * K : 4.0 * N + 2.0 * F) / c.row_rate;
+  };
+  auto start = [&](const MoeCost& c) { return c.start + c.pair * P; };
+  constexpr double by_rows = 1.12, by_ring = 1.08;
+  double now = 0, best = 0;
+  int best_ring = 0, now_ring = 0;
+  for (int r : {64, 128, 256}) {
+    if (r == 256 && !big) continue;
+    double t, rule;  // of this form, and as the rule without the ring has it
+    int on = 0;
+    if (r == 64) {
+      t = rule = start(kMoeCost[0]);
+      const double extra = 0.5 * (start(kMoeCost[1]) - t);
+      for (bool up : {true, false}) {
+        const double a = us(kMoeCost[0], up), b = us(kMoeCost[1], up) + extra;
+        const bool take = b * by_ring < a;
+        rule += a, t += take ? b : a, on |= take ? (up ? 1 : 2) : 0;
+      }
+    } else {
+      const MoeCost& c = kMoeCost[r == 128 ? 2 : 3];
+      t = rule = start(c) + us(c, true) + us(c, false);
+      on = r == 128 ? 3 : 0;
+    }
+    if (r == rows) now = rule, now_ring = on;
+    if (best == 0 || t < best) best = t, *rows_out = r, best_ring = on;
+  }
+  *ring = best_ring;
+  if (*rows_out != rows && best * by_rows >= now) *rows_out = rows, *ring = now_ring;
 }
 
 // act[r, f] = glu(h[order[r] / top] . gate_e[f], h[..] . up_e[f]) over the tile list (bf16), or gelu(h[..] . up_e[f])
 // where there is no gate (wg null); tile_rows = the rows
-// per tile the list was built with (moe_group): 64 or 128
+// per tile the list was built with (moe_group): 64 or 128; use_ring: through the ring of k-steps where the operands allow it
 void launch_moe_gate_up_tile(const void* h, int64_t ldh, const void* wg, const void* wu, const void* meta,
                              const void* order, void* act, int E, int maxt, int top, int F, int K, float limit,
-                             float alpha, int tile_rows, const void* pw, int silu, int ilv, hipStream_t st) {
+                             float alpha, int tile_rows, const void* pw, int silu, int ilv, bool use_ring, hipStream_t st) {
   if (ilv && F % 16) throw std::runtime_error("moe_gate_up: gate and up in groups of 16 rows");
   if (tile_rows != 64 && tile_rows != 128) throw std::runtime_error("moe_gate_up: tile rows must be 64 or 128");
   if (maxt <= 0) return;
@@ -450,11 +518,11 @@ void launch_moe_gate_up_tile(const void* h, int64_t ldh, const void* wg, const v
   // workgroup per CU; at 128x64 two to three fit and hide each other's staging
   if (!wg) {
     a.B = (const bf16_t*)wu; a.B2 = nullptr;
-    const bool ring = moe_ring_ok(a, ldh, (int64_t)maxt * tile_rows / top, F);
+    const bool ring = use_ring && moe_ring_ok(a, ldh, (int64_t)maxt * tile_rows / top, F);
     const int bn = tile_rows == 128 && F >= 512 ? 256 : tile_rows;
     dim3 g((F + bn - 1) / bn, maxt);
     if (ring && tile_rows == 128) tile_ring_kernel<GT_UP, bf16_t, 128, 128, 2><<<dim3((F + 127) / 128, maxt), 256, 0, st>>>(a);
-    else if (ring && moe_ring64<GT_UP, bf16_t>(a, st)) {}
+    else if (ring) moe_ring64<GT_UP, bf16_t>(a, st);
     else if (bn == 256) gemm_tile_kernel<GT_UP, bf16_t, 128, 256><<<g, 256, 0, st>>>(a);
     else if (tile_rows == 128) gemm_tile_kernel<GT_UP, bf16_t, 128, 128><<<g, 256, 0, st>>>(a);
     else gemm_tile_kernel<GT_UP, bf16_t, 64, 64><<<g, 256, 0, st>>>(a);
@@ -462,9 +530,9 @@ void launch_moe_gate_up_tile(const void* h, int64_t ldh, const void* wg, const v
     return;
   }
   dim3 g((F + 63) / 64, maxt);
-  const bool ring = moe_ring_ok(a, ldh, (int64_t)maxt * tile_rows / top, (int64_t)(ilv ? 2 : 1) * F);
+  const bool ring = use_ring && moe_ring_ok(a, ldh, (int64_t)maxt * tile_rows / top, (int64_t)(ilv ? 2 : 1) * F);
   if (ring && tile_rows == 128) tile_ring_kernel<GT_GATE_UP, bf16_t, 128, 64, 2><<<g, 256, 0, st>>>(a);
-  else if (ring && moe_ring64<GT_GATE_UP, bf16_t>(a, st)) {}
+  else if (ring) moe_ring64<GT_GATE_UP, bf16_t>(a, st);
   else if (tile_rows == 128) gemm_tile_kernel<GT_GATE_UP, bf16_t, 128, 64><<<g, 256, 0, st>>>(a);
   else gemm_tile_kernel<GT_GATE_UP, bf16_t, 64, 64><<<g, 256, 0, st>>>(a);
   HIP_CHECK_LAUNCH();
@@ -472,7 +540,7 @@ void launch_moe_gate_up_tile(const void* h, int64_t ldh, const void* wg, const v
 
 // y[r, n] = act[r, :] . down_e[n, :] over the tile list (fp32)
 void launch_moe_down_tile(const void* act, const void* wd, const void* meta, void* y, int E, int maxt, int N, int F,
-                          int tile_rows, hipStream_t st) {
+                          int tile_rows, bool use_ring, hipStream_t st) {
   if (tile_rows != 64 && tile_rows != 128) throw std::runtime_error("moe_down: tile rows must be 64 or 128");
   if (maxt <= 0) return;
   if (maxt > 65535) throw std::runtime_error("moe_down: too many row tiles");
@@ -482,9 +550,9 @@ void launch_moe_down_tile(const void* act, const void* wd, const void* meta, voi
   a.meta = (const int*)meta; a.E = E; a.maxt = maxt; a.top = 1;
   const int bn = tile_rows == 128 && N >= 512 ? 256 : tile_rows;
   dim3 g((N + bn - 1) / bn, maxt);
-  const bool ring = moe_ring_ok(a, F, (int64_t)maxt * tile_rows, N);
+  const bool ring = use_ring && moe_ring_ok(a, F, (int64_t)maxt * tile_rows, N);
   if (ring && tile_rows == 128) tile_ring_kernel<GT_DOWN, float, 128, 128, 2><<<dim3((N + 127) / 128, maxt), 256, 0, st>>>(a);
-  else if (ring && moe_ring64<GT_DOWN, float>(a, st)) {}
+  else if (ring) moe_ring64<GT_DOWN, float>(a, st);
   else if (bn == 256) gemm_tile_kernel<GT_DOWN, float, 128, 256><<<g, 256, 0, st>>>(a);
   else if (tile_rows == 128) gemm_tile_kernel<GT_DOWN, float, 128, 128><<<g, 256, 0, st>>>(a);
   else gemm_tile_kernel<GT_DOWN, float, 64, 64><<<g, 256, 0, st>>>(a);

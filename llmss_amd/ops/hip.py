@@ -1128,13 +1128,8 @@ _MOE_PP = os.environ.get("LLMSS_MOE_PP", "1") != "0"  # 0: grouped products on t
 # 186 -> 163; no gate, 128 pairs 145 -> 105, 100 -> 72, 230 -> 174, 64 pairs 75 -> 105, 35 -> 68, 118 -> 164; two matrices, 128 pairs
 # 163 -> 124, 64 -> 68, 188 -> 178, 256 pairs 208 -> 206, 74 -> 71, 288 -> 183, 1024 pairs 605 -> 449, 166 -> 138, 739 -> 511.
 MOE_PP_ROWS_TWO, MOE_PP_ROWS = 256, 128
-# Beside the ring of k-steps, which takes whole steps of 64 (csrc/gemm_tile.hip), they are the faster ones from MOE_PP_ROWS pairs on in either form,
-# but up to 512 pairs only where their waves are filled: _moe_pp_fill (8 experts and more; fewer were not measured). us of both products, ring and 256-row tiles: 16 experts of 512 x 1024
-# (0.25 - 0.5 filled) 200 pairs 35 and 55, 400 pairs 51 and 59; 8 of 2048 x 2048 (0.38) 128 pairs 94 and 116, (0.75) 320 pairs 129 and
-# 118; 32 of 768 x 2048 (0.82) 128 pairs 131 and 108, without a gate (0.55) 98 and 112, in two matrices (0.82) 137 and 114; 64 of 1408 x 2048
-# (0.94) 128 pairs 368 and 322.
-MOE_PP_FILL = 0.65
-# And up to which those of 16 rows are, against the ring: at 8 pairs 0.8 - 0.98 of its time, at 12 0.85 - 0.99 for up to 32 experts but
+# (Whole steps of 64 of width: these lines are where csrc/gemm_tile.hip's moe_plan starts from.)
+# And up to which those of 16 rows are, against the ring of k-steps there: at 8 pairs 0.8 - 0.98 of its time, at 12 0.85 - 0.99 for up to 32 experts but
 # to 1.3 for 64 and 128 (128 of 576 x 640 73 -> 95).
 MOE_DEC_ROWS = 8
 MOE_DEC_PAIRS = 1024  # pairs (and experts) up to which that kernel finds every expert's rows itself, without a grouping launch
@@ -1142,13 +1137,9 @@ MOE_SHARED_ROWS = 64  # rows up to which it takes the shared expert along: two t
 MOE_GROUP_PAIRS = 4096  # pairs up to which one workgroup groups them: 4096 in 4.4 us (4.8 in two launches), 8192 in 6.5 (5.1)
 
 
-def _moe_pp_fill(P, E, up, N, K, F):
-    """How much of the waves of 256 x 256 tiles that both products of a layer take is filled (up: columns of the first product)."""
-    work = room = 0
-    for cols, k in ((up, K), (N, F)):
-        tiles = E * -(-P // (256 * E)) * -(-cols // 256)
-        work, room = work + tiles * k, room + -(-tiles // 256) * 256 * k
-    return work / room
+def _moe_plan(P, E, F, N, K, glu, rows, big):
+    """(rows of a tile, which products take the ring of k-steps), for operands in whole steps of 64 (csrc/gemm_tile.hip moe_plan)."""
+    return lib().moe_plan(P, E, F, N, K, glu, rows, big)
 
 
 def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=True, act="glu_clamp",
@@ -1193,26 +1184,19 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     P = T * top
     # (both forms below load the weights in pieces of 16 bytes; the tile kernel takes any place)
     aligned = not (h.data_ptr() | up.data_ptr() | down.data_ptr() | _ptr(gate)) & 15 and h.stride(0) % 8 == 0
-    # rows per tile of the grouped GEMMs: 128 where the experts get enough rows to fill big tiles (bf16 only). Whole k-steps go through the
-    # ring of csrc/gemm_tile.hip, whose big tiles pay from half as many rows on, but only where they still fill the chip (us of both products
-    # at 64 and 128 rows: 32 experts of 768 x 2048, 1.5 tiles per CU, 64 rows each 93 and 93, 103 each 120 and 102; 64 of 1408 x 2048, 96 each
-    # 355 and 293; 16 of 512 x 1024, 0.5 - 1 tiles per CU, 38 each 25 and 35, 188 each 36 and 43)
-    ring = h.dtype == torch.bfloat16 and aligned and K % 64 == 0 and F % 64 == 0
-    if ring:
-        rows = 128 if P >= 64 * E and (P // 128 + E // 2) * -(-F // (128 if act == "gelu" else 64)) >= 384 else 64
-    else:
-        rows = 128 if h.dtype == torch.bfloat16 and P >= 128 * E else 64
-    # experts with still more rows each: the dense GEMMs' 256 x 256 tiles; gate and up in one matrix (interleaved) or in two
-    if ring and E >= 8:
-        many = P >= MOE_PP_ROWS * E and (P >= 512 * E or _moe_pp_fill(P, E, F if act == "gelu" else 2 * F, N, K, F) >= MOE_PP_FILL)
-    else:
-        many = P >= (MOE_PP_ROWS if gate is None else MOE_PP_ROWS_TWO) * E
-    pp = (h.dtype == torch.bfloat16 and many
-          and min(F, N) >= 256 and F % 8 == 0 and K % 8 == 0 and aligned and _MOE_PP)
+    # rows per tile of the grouped GEMMs: 128 where the experts get enough rows to fill big tiles (bf16 only), with still more the dense GEMMs'
+    # 256 x 256 tiles; gate and up in one matrix (interleaved) or in two
+    rows, ring = 128 if h.dtype == torch.bfloat16 and P >= 128 * E else 64, 0
+    big = h.dtype == torch.bfloat16 and min(F, N) >= 256 and F % 8 == 0 and K % 8 == 0 and aligned and _MOE_PP
     if gate is not None:
-        pp = pp and lib().moe_pp_glu_ok(h.stride(0), -(-P // 256) + min(E, P), top, F, K)
+        big = big and lib().moe_pp_glu_ok(h.stride(0), -(-P // 256) + min(E, P), top, F, K)
     elif weight_input:
-        pp = False
+        big = False
+    if big and P >= (MOE_PP_ROWS if gate is None else MOE_PP_ROWS_TWO) * E:
+        rows = 256
+    if h.dtype == torch.bfloat16 and aligned and K % 64 == 0 and F % 64 == 0 and P > MOE_DEC_ROWS * E:
+        rows, ring = _moe_plan(P, E, F, N, K, act != "gelu", rows, big)
+    pp = rows == 256
     # and those with a few rows each: weights straight into the matrix instructions' operands
     dec = h.dtype == torch.bfloat16 and P <= MOE_DEC_ROWS * E and K % 32 == 0 and F % 32 == 0 and aligned and not pp
     own = dec and P <= MOE_DEC_PAIRS and E <= MOE_DEC_PAIRS  # (no grouping: results in the pairs' order)
@@ -1225,8 +1209,6 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
             gu = linear_f(h, sgu, h.dtype)
             shared = linear_f(glu_act(gu, Fs, "silu") if act == "silu" else glu_clamp(gu, Fs, slimit, alpha), sdown, h.dtype)
             gu = gu if D else None
-    if pp:
-        rows = 256
     if dec:
         rows = 16
     maxt = -(-P // rows) + min(E, P)
@@ -1277,8 +1259,8 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     elif h.dtype == torch.bfloat16:  # matrix cores (csrc/gemm_tile.hip)
         L.moe_gate_up_tile(h.data_ptr(), h.stride(0), up.data_ptr() if interleaved else _ptr(gate), up.data_ptr(),
                            meta.data_ptr(), order.data_ptr(), act_.data_ptr(), E, maxt, top, F, K, float(limit), float(alpha),
-                           rows, pw, silu, int(interleaved), st)
-        L.moe_down_tile(act_.data_ptr(), down.data_ptr(), meta.data_ptr(), y.data_ptr(), E, maxt, N, F, rows, st)
+                           rows, pw, silu, int(interleaved), bool(ring & 1), st)
+        L.moe_down_tile(act_.data_ptr(), down.data_ptr(), meta.data_ptr(), y.data_ptr(), E, maxt, N, F, rows, bool(ring & 2), st)
     else:
         L.moe_gate_up(h.data_ptr(), h.stride(0), _ptr(gate), up.data_ptr(), meta.data_ptr(), order.data_ptr(),
                       act_.data_ptr(), E, maxt, top, F, K, float(limit), float(alpha), dt, pw, silu, st)

@@ -147,6 +147,24 @@ def test_split_rests_cut_elsewhere_only_beside_more_than_64_rows(M, N, K, cut, s
     assert tuple(H.lib().gemm_cut(M, N, K, False)) == cut and H.lib().gemm_cut_split(M, N, K, False) == split
 
 
+@pytest.mark.parametrize("E,pairs,F,K,glu,rows,plan", [
+    (142, 70, 768, 128, True, 64, (64, (0, 2))),    # 57 us without the ring, 77 on its tiles of 128 rows
+    (36, 96, 1664, 256, True, 64, (64, (1, 2, 3))),  # 65, 70; 57 on those of 64
+    (64, 55, 896, 768, True, 64, (64, (0,))),       # 82; 89 on either
+    (61, 194, 896, 320, True, 256, (64, (0,))),     # 79, as on 256 rows; 92 on 128
+    (16, 38, 512, 1024, True, 64, (64, (3,))),      # 41; 30
+    (16, 188, 512, 1024, True, 256, (64, (1, 3))),  # 62; 42
+    (32, 64, 768, 2048, True, 64, (128, (3,))),     # 114; 90, 108 on 64 rows
+    (32, 103, 768, 2048, True, 64, (128, (3,))),    # 116; 99
+])
+def test_expert_layers_take_the_ring_where_it_is_the_faster_one(E, pairs, F, K, glu, rows, plan):
+    """Rows of a tile and the products that go through the ring of k-steps, at layers where both were measured (us)."""
+    from llmss_amd.ops import hip as H
+
+    got = H.lib().moe_plan(E * pairs, E, F, K, K, glu, rows, min(F, K) >= 256)
+    assert got[0] == plan[0] and got[1] in plan[1], got
+
+
 @pytest.mark.parametrize("block", [2, 16, 48])
 @pytest.mark.parametrize("group,head_dim,fp8,alone", [(1, 128, True, 800), (2, 128, True, 800), (1, 64, True, 800), (1, 64, False, 512),
                                                       (4, 128, True, 0), (1, 256, True, 0), (1, 128, False, 0), (2, 64, False, 0),
