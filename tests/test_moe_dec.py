@@ -5,11 +5,16 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# K of one step up to more than a wave's eight, F that is no multiple of 128; one row, an expert with more rows than a tile, one with none
-@pytest.mark.parametrize("E,top,W,F,T", [(4, 2, 32, 32, 1), (8, 2, 96, 160, 15), (5, 3, 1056, 96, 13), (40, 1, 2048, 768, 21)])
+# K of one step up to more than a wave's eight, F that is no multiple of 128; one row, an expert with more rows than a tile, one with none; in
+# whole lines, steps that do not divide evenly among a wave's four; without and with a tile list (so does a layer of many experts by itself)
+@pytest.mark.parametrize("E,top,W,F,T", [(4, 2, 32, 32, 1), (8, 2, 96, 160, 15), (5, 3, 1056, 96, 13), (40, 1, 2048, 768, 21), (16, 2, 1088, 704, 33),
+                                         (12, 2, 2304, 320, 9), (160, 8, 64, 64, 150)])
 @pytest.mark.parametrize("kind", ["silu", "weighted", "clamp", "interleaved", "gelu"])
-def test_moe_dec(E, top, W, F, T, kind, monkeypatch):
+@pytest.mark.parametrize("grouped", [False, True])
+def test_moe_dec(E, top, W, F, T, kind, grouped, monkeypatch):
     from llmss_amd.ops import hip, glu_interleave
+    if grouped:
+        monkeypatch.setattr(hip, "MOE_DEC_PAIRS", 0)
     g = torch.Generator().manual_seed(E + W + F)
     h = torch.randn(T, W + 8, generator=g).bfloat16().cuda()[:, :W]
     gate, up = ((torch.randn(E, F, W, generator=g) * W ** -0.5).bfloat16().cuda() for _ in range(2))
@@ -31,7 +36,7 @@ def test_moe_dec(E, top, W, F, T, kind, monkeypatch):
         y = hip.moe_experts(h, idx, w, None, glu_interleave(gate, up, 1).contiguous(), down, 0.0, 0.0, act=act, interleaved=True)
     else:
         y = hip.moe_experts(h, idx, w, None if kind == "gelu" else gate, up, down, 1.5, 1.702, act=act, weight_input=weighted)
-    assert calls.count("moe_dec") == 2
+    assert calls.count("moe_dec") == 2 and calls.count("moe_group") == (1 if grouped or T * top > 1024 else 0)
     want = torch.zeros(T, W, dtype=torch.float64, device="cuda")
     lim = torch.zeros_like(want)
     hd = h.double()
@@ -60,9 +65,11 @@ def test_moe_dec(E, top, W, F, T, kind, monkeypatch):
 
 
 # One look at the choices instead of a grouping launch, the shared expert in the same launches: experts of no, one, 16, 17, 32, 33 and all
-# rows (tiles past an expert's first), the largest number of pairs, a shared expert of another width, further columns behind it
+# rows (tiles past an expert's first), the largest number of pairs, a shared expert of another width, further columns behind it; both launches in
+# whole lines, several looks of a wave with a partial last one, up to 16 rows and more
 @pytest.mark.parametrize("E,top,W,F,Fs,D,T", [(4, 1, 64, 32, 64, 24, 1), (9, 3, 96, 96, 32, 0, 16), (8, 1, 160, 64, 96, 40, 33),
-                                              (16, 2, 256, 96, 160, 256, 64), (128, 16, 64, 32, 32, 7, 64)])
+                                              (16, 2, 256, 96, 160, 256, 64), (128, 16, 64, 32, 32, 7, 64),
+                                              (16, 2, 2048, 768, 1024, 40, 8), (16, 2, 1088, 1344, 1088, 24, 33), (8, 1, 2304, 1344, 320, 8, 40)])
 @pytest.mark.parametrize("kind", ["silu", "weighted", "clamp", "interleaved"])
 def test_moe_dec_own_rows(E, top, W, F, Fs, D, T, kind, monkeypatch):
     from llmss_amd.ops import glu_interleave, hip
