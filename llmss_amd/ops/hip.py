@@ -1128,7 +1128,8 @@ _MOE_PP = os.environ.get("LLMSS_MOE_PP", "1") != "0"  # 0: grouped products on t
 # 186 -> 163; no gate, 128 pairs 145 -> 105, 100 -> 72, 230 -> 174, 64 pairs 75 -> 105, 35 -> 68, 118 -> 164; two matrices, 128 pairs
 # 163 -> 124, 64 -> 68, 188 -> 178, 256 pairs 208 -> 206, 74 -> 71, 288 -> 183, 1024 pairs 605 -> 449, 166 -> 138, 739 -> 511.
 MOE_PP_ROWS_TWO, MOE_PP_ROWS = 256, 128
-# (Whole steps of 64 of width: these lines are where csrc/gemm_tile.hip's moe_plan starts from.)
+# (Whole steps of 64 of width: these lines are where csrc/gemm_tile.hip's moe_plan starts from. Layers of fewer than MOE_PP_FEW experts stay with them.)
+MOE_PP_FEW = 8
 # And up to which those of 16 rows are, against the ring of k-steps there: at 8 pairs 0.8 - 0.98 of its time, at 12 0.85 - 0.99 for up to 32 experts but
 # to 1.3 for 64 and 128 (128 of 576 x 640 73 -> 95).
 MOE_DEC_ROWS = 8
@@ -1194,7 +1195,7 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
         big = False
     if big and P >= (MOE_PP_ROWS if gate is None else MOE_PP_ROWS_TWO) * E:
         rows = 256
-    if h.dtype == torch.bfloat16 and aligned and K % 64 == 0 and F % 64 == 0 and P > MOE_DEC_ROWS * E:
+    if h.dtype == torch.bfloat16 and aligned and K % 64 == 0 and F % 64 == 0 and P > MOE_DEC_ROWS * E and (rows < 256 or E >= MOE_PP_FEW):
         rows, ring = _moe_plan(P, E, F, N, K, act != "gelu", rows, big)
     pp = rows == 256
     # and those with a few rows each: weights straight into the matrix instructions' operands
