@@ -210,8 +210,8 @@ __global__ __launch_bounds__(256, BM * BN > 128 * 128 ? 2 : 1) void gemm_tile_ke
 // two bytes lie on few memory channels, which all tiles would otherwise walk together (32 experts of 768 x 2048, 80 rows each: 100 -> 94 us of
 // both products; by row tile instead, tiles that share an expert's weights lose each other: 188 rows each 151 -> 158). us of both products
 // against the kernel above: 16 experts of 512 x 1024, 38 rows each 33.2 -> 24.6; 32 of 768 x 2048, 80 rows 120 -> 94, 103 rows 117 -> 99; 64 of
-// 1408 x 2048, 96 rows 360 -> 294, 66 rows 321 -> 277; over 108 random layers (8 - 128 experts, 9 - 130 rows each) 0.81 of the time, 1.08 at
-// worst. Batched and 32-bit-result products (PLAIN), whose K of 128 - 256 is on its way whole and whose bf16 results leave in 16-byte pieces
+// 1408 x 2048, 96 rows 360 -> 294, 66 rows 321 -> 277; but 89 against 82 for 64 of 896 x 768, 55 rows each: moe_plan below says
+// which layers come here. Batched and 32-bit-result products (PLAIN), whose K of 128 - 256 is on its way whole and whose bf16 results leave in 16-byte pieces
 // instead of two bytes a lane: 16 heads of 8261 x 256 x 128 45.5 -> 35.6 us, x 128 x 256 37.8 -> 28.4, one of 8261 x 4096 x 1024 in 32 bits 143 -> 112,
 // 64 x 2048 x 2048 23.2 -> 11.6, 8 x 2048 x 1024 12.2 -> 7.3. Four or six steps were slower everywhere (822 x 4 rows over 32 experts: 127 and 139
 // against 120). 128 rows: 128 x 128 tiles for one matrix (64 and 256 columns 111 and 105 against 102 us).
@@ -368,10 +368,23 @@ __global__ __launch_bounds__(256) void tile_ring_kernel(GemmTileArgs p) {
     }
 }
 
+static int plain_tile(int M, int N) { return M >= 512 && N >= 128 ? 128 : 64; }  // big tiles where there is enough work to fill the chip
+
+// Whether a batched or 32-bit-result product of whole k-steps takes the ring: not on 64 x 64 tiles that do not all run at once, three on a CU there,
+// where the kernel without it has more of them - up to half a wave too many, and with K up to 256 any number. Over 1900 products of 769 tiles and more
+// the ring took 1.04 - 1.25 of that kernel's time at K = 64 - 192, 1.01 - 1.05 up to 1152 tiles beyond, else 0.95 (tiles of 128 x 128: 0.83, 0.94 in 32
+// bits, hardly one slower). us without and with: 16 heads of 3680 x 40 x 128 in 32 bits 8.3 and 9.9, 8 of 383 x 2040 x 192 14.5 and 17.6, 40 of 8 x
+// 3936 x 64 10.3 and 14.3. With this line 0.80 over 4477 other products, 94 above 1.02, 1.12 at worst (64 of 7594 x 103 x 320 173 and 194).
+bool gemm_tile_rings(int M, int N, int K, int batch) {
+  const int T = plain_tile(M, N);
+  const int64_t tiles = (int64_t)((M + T - 1) / T) * ((N + T - 1) / T) * batch;
+  return K % 64 == 0 && (T == 128 || tiles <= 768 || (K > 256 && tiles > 1152));
+}
+
 void launch_gemm_tile(const void* A, const void* B, void* C, int M, int N, int K, int batch, int64_t sAb, int64_t sAm,
                       int64_t sBb, int64_t sBn, int64_t sCb, int64_t sCm, int dc, const void* bias, hipStream_t st) {
   if (M <= 0 || N <= 0 || batch <= 0) return;
-  const int T = (M >= 512 && N >= 128) ? 128 : 64;  // big tiles where there is enough work to fill the chip
+  const int T = plain_tile(M, N);
   if (batch > 65535 || (M + T - 1) / T > 65535) throw std::runtime_error("gemm_tile: grid too large");
   GemmTileArgs a{};
   a.A = (const bf16_t*)A; a.B = (const bf16_t*)B; a.C = C;
@@ -380,8 +393,8 @@ void launch_gemm_tile(const void* A, const void* B, void* C, int M, int N, int K
   a.bias = (const bf16_t*)bias;
   dim3 g((N + T - 1) / T, (M + T - 1) / T, batch);
   if (dc != 0 && dc != 1) throw std::runtime_error("gemm_tile: bad output dtype code");
-  // whole k-steps, rows of 16-byte alignment of which a tile's 128, of either operand, fit 31 bits: the ring
-  const bool ring = K > 0 && K % 64 == 0 && !((sAb | sAm | sBb | sBn) & 7) && !(((uintptr_t)A | (uintptr_t)B) & 15) && sAm >= 0 && sBn >= 0 &&
+  // whole k-steps, rows of 16-byte alignment of which a tile's 128, of either operand, fit 31 bits: the ring, where the size is one for it
+  const bool ring = gemm_tile_rings(M, N, K, batch) && K > 0 && !((sAb | sAm | sBb | sBn) & 7) && !(((uintptr_t)A | (uintptr_t)B) & 15) && sAm >= 0 && sBn >= 0 &&
                     std::max(sAm, sBn) < (1 << 22) && K < (1 << 22);
   if (ring) {
     a.wide = N % 8 == 0 && !((sCb | sCm) & 7) && !((uintptr_t)C & 15);

@@ -165,6 +165,21 @@ def test_expert_layers_take_the_ring_where_it_is_the_faster_one(E, pairs, F, K, 
     assert got[0] == plan[0] and got[1] in plan[1], got
 
 
+@pytest.mark.parametrize("M,N,K,batch,ring", [
+    (3680, 40, 128, 16, False),  # 8.3 us without the ring, 9.9 with it
+    (383, 2040, 192, 8, False),  # 14.5, 17.6
+    (8, 3936, 64, 40, False),    # 10.3, 14.3
+    (71, 1905, 320, 16, False),  # 14.6, 16.7: a wave and a quarter
+    (8261, 256, 128, 16, True),  # 45.5, 35.6
+    (64, 2048, 2048, 1, True),   # 23.2, 11.6
+    (64, 4096, 1024, 24, True), (64, 4096, 130, 1, False),
+])
+def test_batched_products_take_the_ring_where_it_is_the_faster_one(M, N, K, batch, ring):
+    from llmss_amd.ops import hip as H
+
+    assert H.lib().gemm_tile_rings(M, N, K, batch) == ring
+
+
 @pytest.mark.parametrize("block", [2, 16, 48])
 @pytest.mark.parametrize("group,head_dim,fp8,alone", [(1, 128, True, 800), (2, 128, True, 800), (1, 64, True, 800), (1, 64, False, 512),
                                                       (4, 128, True, 0), (1, 256, True, 0), (1, 128, False, 0), (2, 64, False, 0),

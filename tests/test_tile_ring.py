@@ -7,7 +7,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("M,N,K,H", [(1, 8, 64, 3), (63, 72, 128, 2), (65, 64, 192, 1), (511, 136, 64, 4), (512, 128, 128, 2), (513, 130, 64, 3),
-                                     (641, 200, 320, 2), (8, 2048, 1024, 1), (700, 1, 64, 1)])
+                                     (641, 200, 320, 2), (8, 2048, 1024, 1), (700, 1, 64, 1), (130, 1030, 64, 16),
+                                     (70, 72, 256, 193), (66, 520, 320, 43), (66, 520, 320, 64)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("pad,bias", [(0, False), (8, True), (3, True)])
 def test_plain(M, N, K, H, dtype, pad, bias):
