@@ -90,6 +90,7 @@ void launch_gemm_tile(const void* A, const void* B, void* C, int M, int N, int K
 void launch_moe_gate_up_tile(const void* h, int64_t ldh, const void* wg, const void* wu, const void* meta,
                              const void* order, void* act, int E, int maxt, int top, int F, int K, float limit,
                              float alpha, int tile_rows, const void* pw, int silu, int ilv, bool use_ring, hipStream_t st);
+bool moe_dec_own_rows(int T_, int top, int E, int F, int N, int K, bool glu, bool shared);
 bool gemm_tile_rings(int M, int N, int K, int batch);
 void moe_plan(int P, int E, int F, int N, int K, bool glu, int rows, bool big, int* rows_out, int* ring);
 void launch_moe_pp(int mode, const void* A, int64_t lda, const void* W, const void* meta, const void* order, void* C, int E,
@@ -451,6 +452,7 @@ PYBIND11_MODULE(_C, m) {
     launch_moe_gate_up_tile(CP(h), ldh, CP(wg), CP(wu), CP(meta), CP(order), P(act), E, maxt, top, F, K, limit, alpha,
                             tile_rows, CP(pw), silu, ilv, use_ring, S(st));
   });
+  m.def("moe_dec_own_rows", &moe_dec_own_rows);
   m.def("gemm_tile_rings", &gemm_tile_rings);
   m.def("moe_plan", [](int P, int E, int F, int N, int K, bool glu, int rows, bool big) {  // rows of a tile, products through the ring
     int r, ring;

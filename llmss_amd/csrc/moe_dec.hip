@@ -11,10 +11,14 @@
 // shared one) 53 -> 40 us, 5.4 TB/s, 105 MB of down rows 31.5 -> 25.8; reads alone, 210 MB, 36.9 and 32.5 us, half lines past the caches 38.3.
 //
 // Who chose whom: up to MD_PAIRS (token, expert) pairs a workgroup finds its expert's pairs itself, with one look at all choices, and the
-// rows of the results are the pairs' own numbers: no grouping launch before the products. Beyond that it reads moe.hip's tile list, 16 rows a tile. The shared expert's products, and
+// rows of the results are the pairs' own numbers: no grouping launch before the products. With fewer pairs than experts there is a workgroup row a
+// pair, and an expert's first pair has it: with one an expert, most of which found nobody, 60 experts of 192 x 832 took 20.9 us for 8
+// pairs, 14.7 with a grouping launch, and 384 of 2368 x 320 took 73 for 4, 33 with it. Beyond that, or where the workgroups that find nothing cost more than the launch, it reads moe.hip's tile list, 16 rows a tile. The shared expert's products, and
 // columns of further weights behind its gate and up rows, ride along as workgroups of their own, 32 rows each.
 // A layer's experts in a decode step, grouping and the shared expert's launches beside them before: 33 rows, 32 experts of 2048 x 768 and a
 // shared one of 1024 with 2048 further columns, 14 us less; 8 rows, 16 experts of 1024 x 512 and a shared one of 512, 11 us less.
+#include <cmath>
+
 #include "anytype.h"
 #include "gemm_quad.h"
 
@@ -157,8 +161,11 @@ __device__ __forceinline__ int2 md_extra(const MoeDecArgs& p, int j, int* cnt) {
   return found;
 }
 
-template <int MODE, bool LIST, bool LINES>
+// WHO: a tile's rows from moe.hip's tile list, or found here, a workgroup row an expert or (fewer of them) a pair
+enum { WHO_LIST, WHO_EXPERT, WHO_PAIR };
+template <int MODE, int WHO, bool LINES>
 __global__ __launch_bounds__(256, 4) void moe_dec_kernel(MoeDecArgs p) {
+  constexpr bool LIST = WHO == WHO_LIST;
   constexpr int BN = MODE == MD_GLU ? 16 : 32, G = LIST ? 1 : 2;
   __shared__ __attribute__((aligned(16))) float part[4][2][16 * G][20];  // (rows of 20: 16-byte places, spread over the banks)
   __shared__ int list[MD_ROWS], found[16];
@@ -195,12 +202,17 @@ __global__ __launch_bounds__(256, 4) void moe_dec_kernel(MoeDecArgs p) {
     } else {
       b -= sb;
       const int ct = (N + BN - 1) / BN;
-      int e = b / ct, tile = 0;
+      int e = b / ct, tile = 0, pair = -1;
       n0 = b % ct * BN;
-      if (e >= p.E) {
-        const int2 f = md_extra(p, e - p.E, reinterpret_cast<int*>(part));
+      const int firsts = WHO == WHO_PAIR ? p.P : p.E;
+      if (e >= firsts) {
+        const int2 f = md_extra(p, e - firsts, reinterpret_cast<int*>(part));
         if (f.x < 0) return;
         e = f.x, tile = f.y;
+      } else if constexpr (WHO == WHO_PAIR) {
+        pair = e;
+        e = p.idx[pair];
+        if ((unsigned)e >= (unsigned)p.E) return;
       }
       // the expert's pairs, by number: each wave counts those of its 64 numbers
       int v[MD_PAIRS / 256];
@@ -227,6 +239,7 @@ __global__ __launch_bounds__(256, 4) void moe_dec_kernel(MoeDecArgs p) {
         if (v[u] == e && r >= 0 && r < MD_ROWS) list[r] = threadIdx.x + 256 * u;
       }
       __syncthreads();
+      if (WHO == WHO_PAIR && pair >= 0 && list[0] != pair) return;  // (in the pairs' order: another workgroup has the expert)
       x = p.X;
       W += (int64_t)e * (inter ? 2 : 1) * N * K;
       if (W2) W2 += (int64_t)e * N * K;
@@ -312,18 +325,29 @@ __global__ __launch_bounds__(256, 4) void moe_dec_kernel(MoeDecArgs p) {
   }
 }
 
-template <bool LIST>
+template <int WHO>
 static void launch_moe_dec_t(int mode, bool lines, dim3 g, const MoeDecArgs& a, hipStream_t st) {
 #define MD_LAUNCH(M_)                                                       \
   do {                                                                      \
-    if (lines) moe_dec_kernel<M_, LIST, true><<<g, 256, 0, st>>>(a);        \
-    else moe_dec_kernel<M_, LIST, false><<<g, 256, 0, st>>>(a);             \
+    if (lines) moe_dec_kernel<M_, WHO, true><<<g, 256, 0, st>>>(a);        \
+    else moe_dec_kernel<M_, WHO, false><<<g, 256, 0, st>>>(a);             \
   } while (0)
   if (mode == MD_GLU) MD_LAUNCH(MD_GLU);
   else if (mode == MD_GELU) MD_LAUNCH(MD_GELU);
   else MD_LAUNCH(MD_DOWN);
 #undef MD_LAUNCH
   HIP_CHECK_LAUNCH();
+}
+
+// Whether workgroups find their experts' rows themselves (`shared`: the shared expert comes along). What that costs, us: workgroups for pairs
+// whose expert another one has (or experts that nobody chose, where pairs are more), 3.9 a thousand; each looks at all pairs; and the
+// weights arrive 1 % slower. It saves the grouping launch, and with the shared expert that one's four. Fitted over 4100 random layers (4 - 1024
+// experts, 1 - 64 rows, up to 8 pairs an expert), choices at random; over 2606 others 0.76 of the time with a grouping launch, 41 above 1.02, 1.18 at worst
+// (16 experts of 320 x 3072, 11 rows 31.9 and 37.8 us).
+bool moe_dec_own_rows(int T_, int top, int E, int F, int N, int K, bool glu, bool shared) {
+  const double P = (double)T_ * top, n = std::min<double>(E, P), found = E * (1.0 - std::pow(1.0 - (double)top / E, T_));
+  const double cols = (F + (glu ? 15 : 31)) / (glu ? 16 : 32) + (N + 31) / 32, weights = 2e-6 * found * F * (K * (glu ? 2.0 : 1.0) + N);
+  return 3.9e-3 * (n - found) * cols + 0.002 * P + 0.0095 * weights + 0.7e-6 * P * n * cols < (shared ? 14.6 : 3.3);
 }
 
 // mode 0: act [pairs, N] = glu(X W^T, X W2^T) (W2 null: gate and up rows of W [E, 2 N, K] in alternating groups of 16), 1: gelu(X W^T),
@@ -347,13 +371,13 @@ void launch_moe_dec(int mode, const void* X, int64_t ldx, const void* W, const v
   if (list) {
     if (maxt > 65535) throw std::runtime_error("moe_dec: too many row tiles");
     if (sW) throw std::runtime_error("moe_dec: no shared expert beside a tile list");
-    launch_moe_dec_t<true>(mode, K % 64 == 0, dim3((N + bn - 1) / bn, maxt), a, st);
+    launch_moe_dec_t<WHO_LIST>(mode, K % 64 == 0, dim3((N + bn - 1) / bn, maxt), a, st);
     return;
   }
   const int64_t P = (int64_t)T_ * top;
   if (P > MD_PAIRS || E <= 0 || E > MD_PAIRS || !idx || (mode != MD_DOWN && !place)) throw std::runtime_error("moe_dec: pairs");
   a.idx = (const int*)idx, a.place = (int*)place, a.P = (int)P, a.xt = (int)P / MD_ROWS;
-  int64_t wgs = (int64_t)(E + a.xt) * ((N + bn - 1) / bn);
+  int64_t wgs = (std::min<int64_t>(E, P) + a.xt) * ((N + bn - 1) / bn);
   if (sW) {
     if (mode == MD_GELU || sK % 32 || sK <= 0 || sE < 0 || (((uintptr_t)sW | (uintptr_t)sX) & 15) || !sC ||
         (mode == MD_GLU ? sN < 0 || sK != K || (sinter && (sN % 16 || sE)) || (sE && !sD) : sE != 0 || !sX))
@@ -363,5 +387,7 @@ void launch_moe_dec(int mode, const void* X, int64_t ldx, const void* W, const v
     wgs += (int64_t)((T_ + MD_ROWS - 1) / MD_ROWS) * (((mode == MD_GLU ? sN : N) + bn - 1) / bn + (sE + 31) / 32);
   }
   if (wgs > 0x7fffffff) throw std::runtime_error("moe_dec: too many workgroups");
-  launch_moe_dec_t<false>(mode, K % 64 == 0 && (!sW || sK % 64 == 0), dim3((unsigned)wgs), a, st);
+  const bool lines = K % 64 == 0 && (!sW || sK % 64 == 0);
+  if (P < E) launch_moe_dec_t<WHO_PAIR>(mode, lines, dim3((unsigned)wgs), a, st);
+  else launch_moe_dec_t<WHO_EXPERT>(mode, lines, dim3((unsigned)wgs), a, st);
 }

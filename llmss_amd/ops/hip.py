@@ -1133,13 +1133,18 @@ MOE_PP_FEW = 8
 # And up to which those of 16 rows are, against the ring of k-steps there: at 8 pairs 0.8 - 0.98 of its time, at 12 0.85 - 0.99 for up to 32 experts but
 # to 1.3 for 64 and 128 (128 of 576 x 640 73 -> 95).
 MOE_DEC_ROWS = 8
-MOE_DEC_PAIRS = 1024  # pairs (and experts) up to which that kernel finds every expert's rows itself, without a grouping launch
+MOE_DEC_PAIRS = 1024  # pairs (and experts) up to which that kernel can find every expert's rows itself, without a grouping launch
 MOE_SHARED_ROWS = 64  # rows up to which it takes the shared expert along: two tiles, each reading that expert's weights
 MOE_GROUP_PAIRS = 4096  # pairs up to which one workgroup groups them: 4096 in 4.4 us (4.8 in two launches), 8192 in 6.5 (5.1)
 
 
 def _moe_plan(P, E, F, N, K, glu, rows, big):
     """(rows of a tile, which products take the ring of k-steps), for operands in whole steps of 64 (csrc/gemm_tile.hip moe_plan)."""
+def _moe_own_rows(T, top, E, F, N, K, glu, shared):
+    """Whether workgroups of few-row experts find their rows themselves (csrc/moe_dec.hip moe_dec_own_rows)."""
+    return lib().moe_dec_own_rows(T, top, E, F, N, K, glu, shared)
+
+
     return lib().moe_plan(P, E, F, N, K, glu, rows, big)
 
 
@@ -1200,8 +1205,10 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     pp = rows == 256
     # and those with a few rows each: weights straight into the matrix instructions' operands
     dec = h.dtype == torch.bfloat16 and P <= MOE_DEC_ROWS * E and K % 32 == 0 and F % 32 == 0 and aligned and not pp
-    own = dec and P <= MOE_DEC_PAIRS and E <= MOE_DEC_PAIRS  # (no grouping: results in the pairs' order)
-    within = own and shared_mlp is not None and T <= MOE_SHARED_ROWS and Fs % 32 == 0 and not (sgu.data_ptr() | sdown.data_ptr()) & 15
+    within = shared_mlp is not None and T <= MOE_SHARED_ROWS and Fs % 32 == 0 and not (sgu.data_ptr() | sdown.data_ptr()) & 15
+    # (no grouping: results in the pairs' order)
+    own = dec and P <= MOE_DEC_PAIRS and E <= MOE_DEC_PAIRS and _moe_own_rows(T, top, E, F, N, K, act != "gelu", within)
+    within = own and within
     gu = None
     if shared_mlp is not None and not within:  # the shared expert on its own
         if sinter:

@@ -8,13 +8,12 @@ pytestmark = pytest.mark.gpu
 # K of one step up to more than a wave's eight, F that is no multiple of 128; one row, an expert with more rows than a tile, one with none; in
 # whole lines, steps that do not divide evenly among a wave's four; without and with a tile list (so does a layer of many experts by itself)
 @pytest.mark.parametrize("E,top,W,F,T", [(4, 2, 32, 32, 1), (8, 2, 96, 160, 15), (5, 3, 1056, 96, 13), (40, 1, 2048, 768, 21), (16, 2, 1088, 704, 33),
-                                         (12, 2, 2304, 320, 9), (160, 8, 64, 64, 150)])
+                                         (12, 2, 2304, 320, 9), (160, 8, 64, 64, 150), (1024, 8, 64, 64, 2), (200, 3, 96, 64, 64), (256, 1, 64, 32, 255)])
 @pytest.mark.parametrize("kind", ["silu", "weighted", "clamp", "interleaved", "gelu"])
 @pytest.mark.parametrize("grouped", [False, True])
 def test_moe_dec(E, top, W, F, T, kind, grouped, monkeypatch):
     from llmss_amd.ops import hip, glu_interleave
-    if grouped:
-        monkeypatch.setattr(hip, "MOE_DEC_PAIRS", 0)
+    monkeypatch.setattr(hip, "_moe_own_rows", lambda *a: not grouped)
     g = torch.Generator().manual_seed(E + W + F)
     h = torch.randn(T, W + 8, generator=g).bfloat16().cuda()[:, :W]
     gate, up = ((torch.randn(E, F, W, generator=g) * W ** -0.5).bfloat16().cuda() for _ in range(2))

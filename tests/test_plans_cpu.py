@@ -180,6 +180,18 @@ def test_batched_products_take_the_ring_where_it_is_the_faster_one(M, N, K, batc
     assert H.lib().gemm_tile_rings(M, N, K, batch) == ring
 
 
+@pytest.mark.parametrize("T,top,E,F,N,shared,own", [
+    (33, 4, 32, 768, 2048, True, True), (8, 2, 16, 512, 1024, True, True), (8, 8, 64, 64, 512, False, True),
+    (13, 4, 64, 576, 3392, False, False),     # 81 us with a grouping launch, 99 without
+    (55, 16, 512, 64, 2112, False, False),    # 135, 181
+    (17, 4, 160, 64, 3840, False, False),     # 37, 49
+])
+def test_few_row_experts_find_their_rows_where_that_is_the_faster_way(T, top, E, F, N, shared, own):
+    from llmss_amd.ops import hip as H
+
+    assert H._moe_own_rows(T, top, E, F, N, N, True, shared) == own
+
+
 @pytest.mark.parametrize("block", [2, 16, 48])
 @pytest.mark.parametrize("group,head_dim,fp8,alone", [(1, 128, True, 800), (2, 128, True, 800), (1, 64, True, 800), (1, 64, False, 512),
                                                       (4, 128, True, 0), (1, 256, True, 0), (1, 128, False, 0), (2, 64, False, 0),
