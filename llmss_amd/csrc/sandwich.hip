@@ -260,7 +260,9 @@ __device__ __forceinline__ float gelu_tanh_f(float z) {
 struct NoTail {
   static constexpr int kind = 0;
 };
-// the router of the next sublayer's experts, over h as moe_router (moe.hip) has it: the same sums in the same order
+// the router of the next sublayer's experts, over h as moe_router (moe.hip) has it: the same sums in the same order. Looks of 40 outputs; a second one
+// takes longer than a launch of its own, which spreads the outputs over the chip (64 outputs 1.03 - 1.05, 128 1.09 - 1.11 of the time of both),
+// so sandwich_add_norm (ops/hip.py) sends no more than 40. (With the loop over looks taken out, 32 outputs over 33 rows took 9.6 us in place of 9.3.)
 struct RouteTail {
   static constexpr int kind = 1;
   const bf16_t* wr;  // [E (+ 1), W]

@@ -38,7 +38,7 @@ def close(a, b, lim):
 
 # outputs: one, a look's 40 and more, the largest number; widths with idle threads, not in whole 512s; one row and the most
 @pytest.mark.parametrize("T,W,E,top,gate", [(1, 64, 1, 1, True), (33, 2048, 32, 4, False), (8, 1024, 16, 2, True), (256, 520, 41, 3, True),
-                                            (5, 1096, 128, 8, False)])
+                                            (5, 1096, 128, 8, False), (5, 1096, 40, 8, False), (4, 1032, 40, 8, True)])
 @pytest.mark.parametrize("kind", KINDS)
 def test_route(T, W, E, top, gate, kind, monkeypatch):
     from llmss_amd.ops import hip
@@ -48,7 +48,21 @@ def test_route(T, W, E, top, gate, kind, monkeypatch):
     x, wpost, wnext, add = rnd(T, W), rnd(W), rnd(W), rnd(W)
     route = ((rnd(E + int(gate), W) * W ** -0.5).bfloat16(), None if E == 32 else rnd(E), top, True, "sigmoid", rnd(E) if gate else None, gate)
     x1, x2 = x.clone(), x.clone()
-    h1, got = hip.sandwich_add_norm(x1, y, r, rb, wpost, 1e-5, add, wnext, torch.bfloat16, route=route)
+    lib, calls = hip.lib(), []
+
+    class Seen:
+        def __getattr__(self, name):
+            calls.append(name)
+            return getattr(lib, name)
+    with monkeypatch.context() as m:
+        m.setattr(hip, "lib", Seen)
+        hip.sandwich_add_norm(x.clone(), y, r, rb, wpost, 1e-5, add, wnext, torch.bfloat16, route=route)
+        assert calls.count("sandwich_tail") == (W >= 768 and E + gate <= 40)  # (narrow rows and many outputs: two launches are the faster ones)
+        m.setattr(hip, "TAIL_WIDTH", 0)
+        m.setattr(hip, "TAIL_OUTPUTS", 129)
+        calls.clear()
+        h1, got = hip.sandwich_add_norm(x1, y, r, rb, wpost, 1e-5, add, wnext, torch.bfloat16, route=route)
+        assert calls.count("sandwich_tail") == 1
     monkeypatch.setattr(hip, "TAIL_ROWS", -1)
     h2, _ = hip.sandwich_add_norm(x2, y, r, rb, wpost, 1e-5, add, wnext, torch.bfloat16, route=route)
     assert close(x1, x2, 2.0 ** -17) and close(h1, h2, 2.0 ** -7)
