@@ -1708,11 +1708,12 @@ static int tiles_of(int M, int N, int bm, int bn);
 // whichever is priced lower together with the closing op that reads the slabs. Constants fitted over two thirds of 850 (17 - 32 rows:
 // 800) random products with their add_norm behind them, N to 8192, K of 512 - 12800, weights not in the caches; the choice is 0.9 %
 // (0.5 %) above the best of all on the other third. Against the plans before (tiles one step deep from 33 rows on, below 3072 columns
-// without a look at the decode kernel, and K split by a rule of its length) 0.92 of the time (0.97 to 32 rows), 42 of the 850 more than 1.02,
-// at worst 1.14 (63 x 320 x 1536: 6.6 -> 7.5); above 12800 in K 0.91 over 41 products (1.08 at worst, 64 x 5712 x 25408; to 32 rows not
-// measured, so that those stay with the older price), above 8192 columns 1.01 over 19. us with the closing op: 64 x 2048 x 2048 10.3 -> 9.2,
-// x 4096 11.9 -> 11.2, 33 x 2048 x 4096 10.8 -> 10.0, 64 x 4096 x 4096 15.2 -> 14.8, x 11008 26.1 -> 25.3, 64 x 2640 x 4320 17.9 -> 15.3,
-// 48 x 1488 x 1920 12.0 -> 8.8.
+// without a look at the decode kernel, and K split by a rule of its length) 0.85 of the time over 1200 others, 43 of them more than 1.02,
+// 1.06 at worst (54 x 6480 x 10816: 45.9 -> 48.5); a margin of 4 % beside the older plan's price would leave 13 of those and take a fifth of the
+// gains back. Above 12800 in K 0.91 over 41 products (to 32 rows not measured, so that those stay with the older price), above 8192 columns
+// 1.01 over 19. us with the closing op: 64 x 2048 x 2048 11.5 -> 10.5, x 4096 13.2 -> 12.6, 33 x 2048 x 4096 12.2 -> 11.7, 64 x 4096 x 4096 17.8 ->
+// 16.9, 63 x 320 x 1536 11.9 -> 8.7. The layered models' closing products, 64 x 2048 x 5632 and the like, are not among them: linear_f (ops/hip.py)
+// takes the plan of the finished product and leaves its slabs unsummed; this price has add_norm behind it, not their closing ops.
 struct SlabCost {  // as DecCost; us of the closing op in start, slab: bytes of sums written and read per us
   double start, cu, x, wave, chip, spare, slab;
 };

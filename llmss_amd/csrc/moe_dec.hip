@@ -342,8 +342,8 @@ static void launch_moe_dec_t(int mode, bool lines, dim3 g, const MoeDecArgs& a, 
 // Whether workgroups find their experts' rows themselves (`shared`: the shared expert comes along). What that costs, us: workgroups for pairs
 // whose expert another one has (or experts that nobody chose, where pairs are more), 3.9 a thousand; each looks at all pairs; and the
 // weights arrive 1 % slower. It saves the grouping launch, and with the shared expert that one's four. Fitted over 4100 random layers (4 - 1024
-// experts, 1 - 64 rows, up to 8 pairs an expert), choices at random; over 2606 others 0.76 of the time with a grouping launch, 41 above 1.02, 1.18 at worst
-// (16 experts of 320 x 3072, 11 rows 31.9 and 37.8 us).
+// experts, 1 - 64 rows, up to 8 pairs an expert), choices at random; over 5200 others 0.76 of the time with a grouping launch, 90 above 1.02, 1.26 at worst
+// (8 experts of 1344 x 2304, four pairs 25.9 and 32.7 us).
 bool moe_dec_own_rows(int T_, int top, int E, int F, int N, int K, bool glu, bool shared) {
   const double P = (double)T_ * top, n = std::min<double>(E, P), found = E * (1.0 - std::pow(1.0 - (double)top / E, T_));
   const double cols = (F + (glu ? 15 : 31)) / (glu ? 16 : 32) + (N + 31) / 32, weights = 2e-6 * found * F * (K * (glu ? 2.0 : 1.0) + N);

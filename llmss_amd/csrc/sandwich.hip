@@ -282,7 +282,7 @@ struct SideTail : SideArgs {
 // The same for rows of up to 4096 and a norm of one part: a thread keeps NC times four columns of everything in registers, all loads are
 // issued before the first sum, and only two sums pass through LDS. The kernel above asks for the stream and the weights behind the
 // first sum, a round trip more. us, plain rows / gated / four experts' rows: 33 x 2048 5.0 / 5.3 / 5.5 -> 4.3 / 4.7 / 4.8, 8192 x 2048
-// 8192 x 1024 24.8 / 28.3 / 37.8 -> 20.6 / 24.5 / 34.1. NT: the stream, y and what is read with it past the caches' replacement.
+// (NT) 48.9 / 58.8 / 88 -> 41.4 / 54.4 / 72.6, 8192 x 1024 24.8 / 28.3 / 37.8 -> 20.6 / 24.5 / 34.1. NT: the stream, y and what is read with it past the caches' replacement.
 // With a tail, one launch against two, in a decode step (kernel times, us): the router of 17 outputs over 8 rows of 1024 11.0 -> 7.9, of 32
 // over 33 rows of 2048 13.8 -> 11.1, the token input of 32 numbers 17.1 -> 14.7 (each of 33 workgroups draws its 256 KB of weights through one
 // CU). A tail's kernel for every form of y at once, its loads behind a branch a column: 8.7, 11.3 and 16.2.
@@ -600,7 +600,8 @@ static void launch_sandwich_add_norm(void* x, const void* y, int64_t ldy, const 
   // 20.1, gated 30.9 -> 27.4, 8192 rows 48.9 -> 44.3 and 58.8 -> 59.6, past the caches 41.4 and 54.4)
   const bool rows = vec && groups == 1 && !ident && (W <= 1280 || (W <= 2048 && (T_ <= 1024 || ((y || ey) && T_ > 2048))) || (W <= 4096 && T_ <= 512));
   // a stream that the caches do not keep until the next closing op passes their replacement by, with what is read beside it: also four experts'
-  // rows, 8192 x 2048, 88 -> 72.6; but 8192 x 1024, 34 MB, 20.1 -> 22.7
+  // rows, 8192 x 2048, 88 -> 72.6; but 8192 x 1024, 34 MB, 20.1 -> 22.7. With the two products of a feed-forward behind it, rows of 1024 - 2048:
+  // streams of 48 - 200 MB 0.965 - 1.007 of the time, experts' 0.91 - 0.975, of 24 - 42 MB to 1.016
   const bool past = (y || ey) && (int64_t)T_ * W * 4 >= (48 << 20);
   if (slabs < 0 || (slabs && (!y || y2))) throw std::runtime_error("sandwich_add_norm: slabs of one product only");
   if (tail.kind) {

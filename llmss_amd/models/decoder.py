@@ -210,7 +210,7 @@ class DecoderLM:
     # ---------------------------------------------------------------------------- forward
     def _qkv_plan(self, M: int, N: int, K: int):
         """(nt_hint, split_hint) of the QKV product with RoPE and the cache write in its epilogue, None: two launches. Without a tuned
-        plan of either form: where the static plan of a finished product is the decode kernel's, unsplit. The two launches may
+        plan of either form: up to 64 rows where the static plan of a finished product is the decode kernel's, unsplit. The two launches may
         split K, whose slabs rope_cache sums on the way; over 175 random layers of 1 - 64 rows one launch takes 0.87 of their time, and 1.07
         at worst (us, two and one: 4800 x 1600, one row 8.9 and 6.3, 64 rows 13.4 and 9.7; 12288 x 4096 23.6 and 19.9, 28.7 and 24.1;
         6144 x 4096 14.6 and 11.7, 18.3 and 17.7; 3072 x 1024 6.8 and 4.8, 10.4 and 6.7; 15360 x 5120 31.2 and 27.5, 42.0 and 35.2; 10240 x
@@ -230,8 +230,8 @@ class DecoderLM:
     def _qkv_rope_cache(self, L, y, inp: StepInput, kc, vc):
         """QKV projection, RoPE and the paged KV write of the step's tokens -> the bf16 qkv rows.
 
-        Where the autotuner found it faster (a kind-3 plan for this M, ops/autotune.py tune_qkv_epilogue), or nothing is tuned and the
-        decode kernel's unsplit plan serves (:meth:`_qkv_plan`), this is ONE GEMM launch whose epilogue rotates q / k
+        Where the autotuner found it faster (a kind-3 plan for this M, ops/autotune.py tune_qkv_epilogue), or nothing is tuned and an
+        unsplit plan serves, the decode kernel's or from 128 rows on a prompt's tiles (:meth:`_qkv_plan`), this is ONE GEMM launch whose epilogue rotates q / k
         and stores k / v to the cache; otherwise the GEMM (split-K slabs allowed) followed by the rope_cache kernel, which sums
         the slabs itself."""
         cfg, p = self.cfg, self.plan

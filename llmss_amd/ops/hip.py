@@ -678,8 +678,9 @@ def linear_qkv(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv
                nt_hint=0, split_hint=0):
     """QKV projection whose GEMM epilogue applies RoPE and writes k / v into the paged cache (one launch
     instead of GEMM + rope_cache; same values). Returns the bf16 [T, N] qkv tensor, or None when this
-    weight / cache / plan cannot take the fused epilogue (packed or fp8 weights, fp8 KV rows, streaming or
-    big-tile plans, neox RoPE on tiles that are not head-aligned): the caller then runs linear + rope_cache."""
+    weight / cache / plan cannot take the fused epilogue (packed or fp8 weights, fp8 KV rows, streaming plans, on 256 x 256 tiles neox
+    RoPE and heads that do not divide 256 columns, on others neox RoPE where they do not hold whole heads): the caller then runs linear +
+    rope_cache. Prompts' rows may lie further apart than they are wide (QKV_PAD)."""
     if w.dim() != 2 or w.dtype != torch.bfloat16 or (k_cache is not None and k_cache.dtype != torch.bfloat16):
         return None
     M, K = x.shape
@@ -703,7 +704,8 @@ def linear_qkv(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv
         bs = k_cache.shape[2]
     ws = _GEMM_WS.get(64 << 20, x.device)
     # rows a multiple of 4 KB apart lie in few of the caches' channels, head by head, where attention reads them: prompts' rows are kept 256
-    # bytes further apart (3999 rows of 12288, 32 heads of 128: 176 -> 158 us of attention)
+    # bytes further apart (3999 rows of 12288, 32 heads of 128: 176 -> 158 us of attention; product and attention over eight layouts of heads of 64 -
+    # 256, 1 - 32 sequences, 128 - 8000 rows in all: 0.996 on average, 0.957 - 1.017)
     pad = QKV_PAD if M >= 128 and N * 2 % 4096 == 0 else 0
     y = torch.empty(M, N + pad, dtype=x.dtype, device=x.device)[:, :N]
     rc = lib().gemm_qkv(x.data_ptr(), x.stride(0), w.data_ptr(), K, _ptr(bias), y.data_ptr(), y.stride(0), M, N, K,
@@ -1138,13 +1140,13 @@ MOE_SHARED_ROWS = 64  # rows up to which it takes the shared expert along: two t
 MOE_GROUP_PAIRS = 4096  # pairs up to which one workgroup groups them: 4096 in 4.4 us (4.8 in two launches), 8192 in 6.5 (5.1)
 
 
-def _moe_plan(P, E, F, N, K, glu, rows, big):
-    """(rows of a tile, which products take the ring of k-steps), for operands in whole steps of 64 (csrc/gemm_tile.hip moe_plan)."""
 def _moe_own_rows(T, top, E, F, N, K, glu, shared):
     """Whether workgroups of few-row experts find their rows themselves (csrc/moe_dec.hip moe_dec_own_rows)."""
     return lib().moe_dec_own_rows(T, top, E, F, N, K, glu, shared)
 
 
+def _moe_plan(P, E, F, N, K, glu, rows, big):
+    """(rows of a tile, which products take the ring of k-steps), for operands in whole steps of 64 (csrc/gemm_tile.hip moe_plan)."""
     return lib().moe_plan(P, E, F, N, K, glu, rows, big)
 
 
@@ -1858,11 +1860,11 @@ def diff_combine(O, lam, eps, mult, heads, kv_heads, vdim, out_dtype):
 
 # ------------------- blocks normed on both sides / token input / windowed sigmoid attention with pooled blocks / SSD
 TAIL_ROWS = 256  # rows up to which the next router or the token input rides in the closing op's launch, a workgroup per row
-
-
 # And for the router outputs up to which (a look of the kernel's) and widths from which: 4 - 32 outputs over 1 - 255 rows, both launches against one, 1536 -
 # 2048 wide 0.76 - 0.87 of the time, 768 0.84 - 0.97, 512 0.92 - 1.06, 256 0.93 - 1.10 (experts' sums the slower ones). The token input: 0.82 - 0.98.
 TAIL_OUTPUTS, TAIL_WIDTH = 40, 768
+
+
 def sandwich_add_norm(x, y, r, rb, wpost, eps, add, wnext, out_dtype, groups=1, route=None, side=None):
     """``y``: rows in the storage type, a :class:`MoEPending` (combined while it is read), a ``PairPending`` (the results
     of two mixers, normed and joined while they are read) or a :class:`PartialSum` (summed while it is read). ``route``, ``side``: in the
