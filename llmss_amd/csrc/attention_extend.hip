@@ -29,6 +29,8 @@
 // the mask. Portions of 950 and 823 rows behind prefixes of as many, 32 heads of 128: 135 -> 94 us (413
 // TFLOP/s), 111 with one group; inside a step 104 -> 88 us with maxima by lane, the masks' positions where there is a mask and four sums a
 // group side by side.
+// Heads of 256 are held to the 256 registers at which two waves share a SIMD: left to itself the compiler took 266 with four sums side by side, one
+// wave, and 1.2 of the time of one sum after another (1.8 at worst; 4899 rows of 32 heads 413 -> 692 us). Held, 0.875 of it over 340 steps, 1.01 at worst.
 // SAME: keys and values are one tensor (latent attention, where both are the cached latent row and nkv = 1): the
 // tile is loaded and staged once and serves both products.
 #include "common.h"
@@ -44,7 +46,7 @@ constexpr float kLog2eX = 1.4426950408889634f;
 // quantisation launch. Only when a workgroup holds every head of its rows: one kv head (nkv = 1) whose whole query
 // group fits the slots of a wave (GE = G, a power of two <= 16) - Llama-2-70B at TP=8 (8 query heads per rank).
 template <int D, bool KV8, bool SAME, int NS>
-__global__ __launch_bounds__(256, NS) void attn_extend_kernel(
+__global__ __launch_bounds__(256, D == 256 ? 2 : NS) void attn_extend_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ kcv, const void* __restrict__ vcv,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ cu_q, const int* __restrict__ ctx_lens,
     bf16_t* __restrict__ out, int64_t out_stride, int nh, int nkv, int GE, int bs, float scale_log2,
