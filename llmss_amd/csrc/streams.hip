@@ -135,6 +135,7 @@ __global__ __launch_bounds__(256) void stream_rows_kernel(float* __restrict__ x,
   // read from something that is)
   const T* yp = y && !slabs ? y + (int64_t)t * ldy : w;
   const T* wp = w ? w : yp;
+  const int ys = y && !slabs ? 1 : 0, ws = w ? 1 : 0;  // (then its first numbers, over and over)
   float mx[S][S], ow[S], iw[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
@@ -148,8 +149,8 @@ __global__ __launch_bounds__(256) void stream_rows_kernel(float* __restrict__ x,
     const int at = min(4 * (int)(threadIdx.x + 256 * i), W - 4);
 #pragma unroll
     for (int s = 0; s < S; ++s) xs[s][i] = ld4(x + ((int64_t)s * T_ + t) * W + at);
-    if (yp) yr[i] = *reinterpret_cast<const Raw*>(yp + at);
-    if (wp) wr[i] = *reinterpret_cast<const Raw*>(wp + at);
+    if (yp) yr[i] = *reinterpret_cast<const Raw*>(yp + ys * at);
+    if (wp) wr[i] = *reinterpret_cast<const Raw*>(wp + ws * at);
     if (slabs) yv[i] = slab_sum<f32x4>((const float*)y + (int64_t)t * W + at, slabs, (int64_t)T_ * W);
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -222,7 +223,10 @@ __global__ __launch_bounds__(256) void stream_rows_kernel(float* __restrict__ x,
 template <typename T, typename TH, int S>
 void launch_stream_rows(float* x, const T* y, int64_t ldy, const float* mix, const float* outw, float c, const float* inw,
                         const T* w, float eps, int rms, TH* h, int64_t ldh, int T_, int W, int slabs, hipStream_t st) {
-  if (W <= 1024) stream_rows_kernel<T, TH, S, 1><<<T_, 256, 0, st>>>(x, y, ldy, mix, outw, c, inw, w, eps, rms, h, ldh, T_, W, slabs);
+  // (narrow rows: no more waves than they have columns for - with four of them always, those past the row load its last columns as well: 9373 rows of 128,
+  // four streams 21.0 -> 24.8 us against the loads under a condition, now 10.5; over 600 rows below 1024 0.92 of that time. Without a norm behind, the
+  // connections' numbers at the start cost 0.25 us of 2.5 - 3, as they stay)
+  if (W <= 1024) stream_rows_kernel<T, TH, S, 1><<<T_, (W / 4 + 63) / 64 * 64, 0, st>>>(x, y, ldy, mix, outw, c, inw, w, eps, rms, h, ldh, T_, W, slabs);
   else if (W <= 2048) stream_rows_kernel<T, TH, S, 2><<<T_, 256, 0, st>>>(x, y, ldy, mix, outw, c, inw, w, eps, rms, h, ldh, T_, W, slabs);
   else stream_rows_kernel<T, TH, S, 4><<<T_, 256, 0, st>>>(x, y, ldy, mix, outw, c, inw, w, eps, rms, h, ldh, T_, W, slabs);
 }

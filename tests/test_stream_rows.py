@@ -7,7 +7,7 @@ pytestmark = pytest.mark.gpu
 
 # widths: one access, edges of 1024, 2048 and 4096, beyond; more streams than the kernel takes; outputs in both types
 @pytest.mark.parametrize("S,T,W", [(1, 3, 4), (2, 5, 1020), (2, 1, 1024), (3, 7, 1028), (4, 2, 2048), (2, 3, 2052), (1, 2, 4096),
-                                   (2, 2, 4100), (5, 2, 256), (2, 3, 1022)])
+                                   (2, 2, 4100), (5, 2, 256), (2, 3, 1022), (2, 5, 256), (4, 3, 260), (1, 2, 508), (3, 2, 768)])
 @pytest.mark.parametrize("rms", [False, True])
 @pytest.mark.parametrize("dtype,out", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float32, torch.float32)])
 def test_stream_add_norm(S, T, W, rms, dtype, out):
