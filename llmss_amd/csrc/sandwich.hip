@@ -273,7 +273,9 @@ struct RouteTail {
   const float* zb;
   float* sg;
 };
-// the token input (D its numbers, NW at least W / 256), before `add` and the norm
+// the token input (D its numbers, NW at least W / 256), before `add` and the norm. Its weights are asked for under a condition that is the wave's: those
+// past a narrow row read again, rows of 256 took 10.4 us for the token input of 64 numbers alone, a kernel of its own before 7.6; now 8.2, and with the
+// closing op 0.82 - 0.98 of the two launches at 256 - 2048 (32 numbers 0.82 - 0.87)
 template <int D_, int NW_>
 struct SideTail : SideArgs {
   static constexpr int kind = 2, D = D_, NW = NW_;
@@ -351,6 +353,7 @@ __global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p, TAIL
   };
   auto load_proj = [&]() {
     if constexpr (SIDE) {
+      if (SW < 8 && __builtin_amdgcn_readfirstlane(wv) * 256 >= W) return;  // (a wave past a narrow row)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -373,7 +376,7 @@ __global__ __launch_bounds__(512) void sandwich_rows_kernel(SandwichArgs p, TAIL
       for (int r = 0; r < SR; ++r)
 #pragma unroll
         for (int k = 0; k < SW; ++k)
-          sgw[r][k] = *reinterpret_cast<const u16x4*>((const bf16_t*)a.wg + (int64_t)(wv * SR + r) * W + min(k * 256, W - 256) + lane * 4);
+          if (k * 256 < W) sgw[r][k] = *reinterpret_cast<const u16x4*>((const bf16_t*)a.wg + (int64_t)(wv * SR + r) * W + k * 256 + lane * 4);
       if constexpr (TAIL::D == 32) load_proj();  // (the deeper form's registers hold one of the two at a time)
       swn = ld4(a.wn + at[0]);
       id = id < 0 ? 0 : (id >= a.vocab ? a.vocab - 1 : id);
