@@ -48,7 +48,8 @@ int launch_gemm_qkv_args(const void* x, int64_t ldx, const void* w, int64_t ldw,
 int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_fp8, const void* w_scale,
                 const void* bias, void* y, int64_t ldy, int M, int N, int K, int act, bool glu, void* workspace,
                 int64_t ws_bytes, int nt_hint, int split_hint, bool partial_out, hipStream_t st);
-void gemm_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int* nt, int* splitk);
+void gemm_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int* nt, int* splitk, bool four = true);
+void gemm_closing_plan(int M, int N, int K, int* nt, int* splitk);
 void gemm_cut_of(int M, int N, int K, bool glu, int* rows, int* cols, int* split);
 void gemm_tuned_set(int M, int N, int K, bool glu, int kind, int nt_hint, int split);
 void gemm_tuned_clear();
@@ -365,6 +366,11 @@ PYBIND11_MODULE(_C, m) {
     return py::make_tuple(nt, s);
   }, pybind11::arg(), pybind11::arg(), pybind11::arg(), pybind11::arg(), pybind11::arg("glu") = false,
      pybind11::arg("slabs") = true);
+  m.def("gemm_closing_plan", [](int M, int N, int K) {
+    int nt, s;
+    gemm_closing_plan(M, N, K, &nt, &s);
+    return py::make_tuple(nt, s);
+  });
   m.def("gemm_cut", [](int M, int N, int K, bool glu) {  // rows or columns of the first of two launches, 0: one launch
     int rows, cols, split;
     gemm_cut_of(M, N, K, glu, &rows, &cols, &split);

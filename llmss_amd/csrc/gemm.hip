@@ -1418,6 +1418,11 @@ static int dec_split(int M, int N, int K, int split_hint, int64_t ws_bytes) {
   if ((int64_t)s * M * N * 4 > ws_bytes) s = 1;
   return s;
 }
+static constexpr int kFourHint = 2048;
+bool gemm_four_dims(int code, int* bm, int* bn);
+bool gemm_four_ok(int N, int K, int64_t ldx, int64_t ldw, const void* Y, int64_t ldy, bool glu);
+void launch_gemm_four(int code, const bf16_t* X, int64_t ldx, const bf16_t* W, int64_t ldw, const bf16_t* bias, bf16_t* Y, int64_t ldy, float* part,
+                      int M, int N, int K, int act, int glu, int split, int group_m, hipStream_t st, int* cnt, const QkvEpi* qe);
 bool gemm_mid_dims(int tsel, int* bm, int* bn, int* threads);
 void launch_gemm_mid(int tsel, int depth, bool wnt, const bf16_t* X, int64_t ldx, const bf16_t* W, int64_t ldw,
                      const bf16_t* bias, bf16_t* Y, int64_t ldy, float* part, int M, int N, int K, int act, int glu,
@@ -1664,7 +1669,10 @@ bool gemm_tuned_get(int M, int N, int K, bool glu, int kind, int* nt_hint, int* 
 // is nearly empty and where K is short (43776 x 8160 SwiGLU at 33 rows 182 -> 223 us on 128 columns, 178 on 96; 35616 x 384 at 45
 // rows 10.0 -> 13.9).
 //
-// M > 64: the cheapest of six tiles by a cost model. A wave of the chip takes (k-steps of 64) x us per step + 5 us, an unfilled
+// M > 64 and K in whole steps of 64: the cheapest of the four-wave tiles and of 256 x 256 tiles, cut or whole, by the prices below. 17 - 64 rows
+// of a finished product: those tiles where they are priced below 0.97 of the older rules, or 0.86 of the decode kernel.
+//
+// M > 64 otherwise: the cheapest of six tiles by a cost model. A wave of the chip takes (k-steps of 64) x us per step + 5 us, an unfilled
 // second workgroup per CU counts for less, a K split adds its slabs' write and read at 4.5 TB/s and a launch, and nothing
 // beats the operands' bytes at 4 TB/s. Steps measured at M = 80 - 6000 over the shapes above; the choice is 2.7 % above the
 // best of 60 plans on average, and 1.5 times faster than 128 x 128 tiles below 192 tiles of 256 x 256 (4096 x 4096: M = 500 56
@@ -1743,9 +1751,83 @@ static bool gemm_slab_plan(int M, int N, int K, int64_t ws_bytes, int* nt_hint, 
   return best > 0;
 }
 
+// The four-wave tiles (gemm_four.hip), from 17 rows on, by a price fitted to 60000 measurements of 14 tiles and splits of K over 7500 random
+// products (17 - 8300 rows, 256 - 24000 columns, K of 256 - 12000, with and without gate or activation, weights not in the caches). The
+// choice is 1.2 - 2 % above the best of all. Against the plans before, of the same products: 0.84 of the time at 33 - 48 rows, 0.80 to 64, 0.74
+// to 128, 0.75 to 512, 0.76 to 1024, 0.80 to 2048, 0.84 to 4096, 0.90 above; 17 - 32 rows, where the decode kernel is mostly the better one, 0.97.
+// One in a hundred takes more than 1.02 of it (one in twenty above 2048 rows); at worst 1.4 (22 x 5904 x 8448, 24 us and 34).
+// us of a launch; of a round of workgroups, and what a gate adds; per 64 of k with one
+// workgroup on a CU and with `slots` of them; how much less of that a round takes per CU left idle; the combine of split sums, once and per
+// slice and 128 x 128 tile; bytes per us.
+struct FourCost {
+  int code, bm, bn, slots;
+  double start, round, gate, alone, full, idle, sum, slice, chip;
+};
+static constexpr FourCost kFourFew[] = {  // up to 64 rows: weights are what there is to read
+    {0, 64, 64, 3, 0.00, 3.52, 0.29, 0.493, 1.411, 0.601, 1.29, 1.30, 5.36e6}, {1, 32, 64, 2, 2.16, 1.49, 0.09, 0.236, 0.512, 0.438, 1.19, 1.88, 4.10e6},
+    {8, 64, 32, 2, 0.82, 2.73, 0.00, 0.224, 0.458, 0.395, 1.25, 1.88, 4.05e6}, {10, 64, 128, 2, 0.12, 3.80, 0.82, 0.833, 1.807, 0.704, 1.74, 0.85, 9.91e6},
+    {13, 64, 64, 1, 0.38, 3.83, 0.31, 0.378, 0.371, 0.549, 1.33, 1.28, 13.0e6}, {12, 64, 128, 1, 0.00, 4.55, 0.79, 0.792, 0.744, 0.691, 1.79, 0.79, 4.78e6}};
+static constexpr FourCost kFourMid[] = {  // up to 128 rows
+    {0, 64, 64, 3, 2.78, 1.51, 0.31, 0.276, 0.766, 0.353, 1.42, 1.76, 17.1e6},  {1, 32, 64, 2, 1.90, 2.49, 0.09, 0.168, 0.294, 0.227, 1.39, 2.13, 3.22e6},
+    {2, 128, 64, 2, 0.88, 4.00, 0.77, 0.370, 0.876, 0.384, 1.92, 1.15, 3.63e6}, {3, 128, 128, 2, 3.70, 0.00, 1.96, 1.056, 1.918, 0.545, 1.98, 0.99, 3.61e6},
+    {4, 128, 128, 1, 0.00, 5.74, 1.80, 0.675, 0.820, 0.531, 2.09, 0.84, 4.01e6}, {6, 128, 192, 1, 0.00, 6.81, 2.39, 1.007, 1.207, 0.574, 2.16, 0.75, 4.19e6},
+    {8, 64, 32, 2, 1.91, 2.54, 0.00, 0.165, 0.267, 0.190, 1.46, 2.11, 3.13e6},  {10, 64, 128, 2, 0.98, 4.00, 0.72, 0.377, 0.887, 0.386, 1.89, 1.15, 3.57e6},
+    {11, 128, 64, 1, 0.86, 4.58, 0.78, 0.365, 0.426, 0.374, 1.96, 1.06, 3.84e6}, {12, 64, 128, 1, 0.79, 4.68, 0.72, 0.377, 0.445, 0.389, 1.93, 1.07, 3.64e6},
+    {13, 64, 64, 1, 1.17, 3.89, 0.27, 0.229, 0.231, 0.264, 1.56, 1.49, 3.46e6}};
+static constexpr FourCost kFourMany[] = {
+    {0, 64, 64, 3, 3.87, 0.63, 0.23, 0.235, 0.593, 0.231, 1.72, 2.22, 2.76e6},  {1, 32, 64, 2, 2.52, 2.10, 0.03, 0.157, 0.285, 0.178, 1.61, 1.80, 13.5e6},
+    {2, 128, 64, 2, 0.82, 4.36, 0.62, 0.300, 0.598, 0.257, 2.59, 1.42, 3.40e6}, {3, 128, 128, 2, 0.00, 4.75, 1.49, 0.689, 0.988, 0.342, 3.48, 1.11, 2.60e6},
+    {4, 128, 128, 1, 0.00, 6.29, 1.51, 0.446, 0.454, 0.316, 3.19, 0.94, 16.3e6}, {5, 192, 128, 1, 0.00, 7.53, 1.97, 0.602, 0.633, 0.318, 3.34, 0.84, 3.41e6},
+    {6, 128, 192, 1, 0.00, 7.62, 2.02, 0.617, 0.634, 0.332, 3.46, 0.81, 3.27e6}, {7, 256, 128, 1, 0.00, 8.12, 3.02, 0.781, 0.814, 0.297, 4.11, 0.82, 3.17e6},
+    {8, 64, 32, 2, 2.55, 1.96, 0.00, 0.162, 0.268, 0.180, 1.63, 2.06, 19.7e6},  {9, 192, 192, 1, 0.00, 8.76, 3.23, 0.855, 0.856, 0.286, 4.34, 0.77, 3.50e6},
+    {10, 64, 128, 2, 1.08, 4.24, 0.61, 0.302, 0.626, 0.236, 2.53, 1.32, 2.69e6}, {11, 128, 64, 1, 0.68, 5.01, 0.57, 0.292, 0.279, 0.225, 2.73, 1.14, 12.4e6},
+    {12, 64, 128, 1, 0.80, 4.87, 0.58, 0.311, 0.299, 0.272, 2.67, 1.06, 4.76e6}, {13, 64, 64, 1, 1.74, 3.34, 0.21, 0.208, 0.192, 0.174, 2.08, 1.58, 2.28e6}};
+static constexpr FourCost kQuadCost = {4, 256, 256, 1, 1.88, 8.24, 2.39, 1.335, 1.368, 0.261, 0, 0, 5.0e6};  // gemm_quad.hip
+static double four_us(const FourCost& c, int M, int N, int K, bool glu, int split) {
+  const int64_t wgs = (int64_t)tiles_of(M, N, c.bm, c.bn) * split, cap = 256 * c.slots, rest = wgs % cap;
+  const int per = (K / 64 + split - 1) / split, held = (int)((rest + 255) / 256);
+  const double round = c.round + (glu ? c.gate : 0.0);
+  double t = c.start + (double)(wgs / cap) * (per * c.full + round);
+  if (rest) {
+    const double step = c.slots > 1 ? c.alone + (c.full - c.alone) * (held - 1) / (c.slots - 1) : c.alone;
+    t += per * step * (1.0 - c.idle * (1.0 - (double)rest / (256 * held))) + round;
+  }
+  return std::max(t, c.start + (2.0 * N * K + 2.0 * M * K + 2.0 * M * (glu ? N / 2 : N)) / c.chip);
+}
+struct FourPlan {
+  int hint, split;  // hint 0: none
+  double us;
+};
+// slabs: split sums are left to the consumer
+static FourPlan gemm_four_plan(int M, int N, int K, bool glu, bool slabs, int64_t ws_bytes) {
+  FourPlan best{0, 1, 0.0};
+  if (M < 17 || N % 8 || K % 64) return best;
+  auto look = [&](const FourCost& c) {
+    if (glu && c.bn == 32) return;  // (a gate and its up lie in one wave)
+    const int64_t tiles = tiles_of(M, N, c.bm, c.bn);
+    for (int s : {1, 2, 3, 4, 6, 8}) {
+      if (s > 1 && (K / s < 256 || tiles * s > 1000 || (slabs ? (int64_t)s * M * N : tiles * s * c.bm * c.bn) * 4 > ws_bytes)) break;
+      if (s == 1 && slabs) continue;
+      double t = four_us(c, M, N, K, glu, s);
+      if (s > 1) t += slabs ? 8.0 * s * M * N / 4.5e6 : c.sum + c.slice * s * c.bm * c.bn / 16384;
+      if (!best.hint || t < best.us) best = FourPlan{(c.code | kFourHint | (s > 1 && !slabs ? 256 : 0)) << 8, s, t};
+    }
+  };
+  if (M <= 64) {
+    for (const FourCost& c : kFourFew)
+      if (M > 32 || c.bm == 32 || c.code == 8 || c.code == 13) look(c);
+  } else if (M <= 128) {
+    for (const FourCost& c : kFourMid) look(c);
+  } else {
+    for (const FourCost& c : kFourMany) look(c);
+  }
+  return best;
+}
+
 // slabs: the consumer sums split-K slabs itself and so gets the product in 32 bits. Where the older rules split K that stays so:
 // only split plans are looked at, their slabs costing a write and a read and no launch.
-static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t ws_bytes, int* nt_hint, int* split) {
+static double quad_us(int M, int N, int K, bool glu, int64_t ws_bytes);
+static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t ws_bytes, int* nt_hint, int* split, bool four = true) {
   if (N % 8 || K % 16) return;
   if (slabs) {
     int t = 0, s = 0;
@@ -1755,7 +1837,6 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
   }
   if (M <= 64) {
     if (slabs && M > 16 && gemm_slab_plan(M, N, K, ws_bytes, nt_hint, split)) return;
-    if (M > 32 && N < 3072) return;
     const double bytes = 2.0 * N * K, slab = 8.0 * M * N / 2.5e6;
     double older, faster = M <= 16 ? 1.25 : 1.15;
     if (M <= 16) {
@@ -1779,6 +1860,7 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
     double best = 0;
     int code = 0, sp = 1;
     for (int s = slabs ? 2 : 1; s <= (slabs ? 4 : 1); s *= 2) {
+      if (M > 32 && N < 3072) break;
       if (s > 1 && (K / s < 256 || (int64_t)s * M * N * 4 > ws_bytes)) break;
       for (int bn = 64; bn >= 16; bn -= 16) {
         if (glu && bn % 32) continue;
@@ -1796,9 +1878,18 @@ static void gemm_static_plan(int M, int N, int K, bool glu, bool slabs, int64_t 
         if (t < best) best = t, code = w.tsel;
       }
     }
-    if (!code || best * faster > older) return;
-    *nt_hint = code << 8;
-    *split = sp;
+    const bool dec = code && best * faster <= older;
+    if (dec) *nt_hint = code << 8, *split = sp;
+    if (!four || slabs) return;
+    const FourPlan p = gemm_four_plan(M, N, K, glu, false, ws_bytes);
+    if (p.hint && p.us < (dec ? 0.86 * best : 0.97 * older)) *nt_hint = p.hint, *split = p.split;
+    return;
+  }
+  const FourPlan p = gemm_four_plan(M, N, K, glu, slabs, ws_bytes);
+  if (p.hint) {
+    const bool quad = !slabs && quad_us(M, N, K, glu, ws_bytes) <= p.us;
+    *nt_hint = quad ? 4 << 8 : p.hint;
+    *split = quad ? 1 : p.split;
     return;
   }
   // two rows of 64 x 64 tiles, two to three workgroups per CU: the older rule's one launch of them is the faster one until K is long
@@ -1881,7 +1972,8 @@ static bool gemm_static_takes(bool w_fp8, const void* x, int64_t ldx, const void
 static void gemm_default_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int64_t ws_bytes, bool takes, int* nt_hint,
                               int* split) {
   if (*nt_hint || *split || gemm_tuned_get(M, N, K, glu, w_fp8 ? 1 : 0, nt_hint, split)) return;
-  if (takes) (w_fp8 ? gemm_static_plan_f8 : gemm_static_plan)(M, N, K, glu, slabs, ws_bytes, nt_hint, split);
+  if (takes && w_fp8) gemm_static_plan_f8(M, N, K, glu, slabs, ws_bytes, nt_hint, split);
+  else if (takes) gemm_static_plan(M, N, K, glu, slabs, ws_bytes, nt_hint, split);
 }
 static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint, int64_t ws_bytes);
 
@@ -1946,6 +2038,20 @@ static GemmCut gemm_cut(int M, int N, int K, bool glu, int64_t ws_bytes) {
   return cut;
 }
 
+// What the second launch runs with: four-wave tiles from 65 rows on, else the plan of its size (hint 0)
+static FourPlan gemm_rest_plan(const GemmCut& cut, int m, int n, int K, bool glu, int64_t ws_bytes) {
+  const FourPlan p = m > 64 ? gemm_four_plan(m, n, K, glu, false, ws_bytes) : FourPlan{0, 0, 0.0};
+  return p.hint ? p : FourPlan{cut.hint, cut.hint ? cut.split : 0, 8.0 + 2.0 * n * K / 4.5e6};
+}
+
+// 256 x 256 tiles, cut or whole
+static double quad_us(int M, int N, int K, bool glu, int64_t ws_bytes) {
+  const GemmCut cut = gemm_cut(M, N, K, glu, ws_bytes);
+  if (!cut.rows && !cut.cols) return four_us(kQuadCost, M, N, K, glu, 1);
+  const int rows = cut.rows ? cut.rows : M, cols = cut.cols ? cut.cols : N;
+  return four_us(kQuadCost, rows, cols, K, glu, 1) + gemm_rest_plan(cut, rows < M ? M - rows : M, cols < N ? N - cols : N, K, glu, ws_bytes).us;
+}
+
 int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_fp8, const void* w_scale,
                 const void* bias, void* y, int64_t ldy, int M, int N, int K, int act, bool glu, void* workspace,
                 int64_t ws_bytes, int nt_hint, int split_hint, bool partial_out, hipStream_t st) {
@@ -1958,14 +2064,16 @@ int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_f
     const GemmCut cut = gemm_cut(M, N, K, glu, ws_bytes);
     if (cut.rows) {
       launch_gemm(x, ldx, w, ldw, false, nullptr, bias, y, ldy, cut.rows, N, K, act, glu, workspace, ws_bytes, 4 << 8, 1, false, st);
+      const FourPlan rest = gemm_rest_plan(cut, M - cut.rows, N, K, glu, ws_bytes);
       return launch_gemm((const bf16_t*)x + cut.rows * ldx, ldx, w, ldw, false, nullptr, bias, (bf16_t*)y + cut.rows * ldy, ldy,
-                         M - cut.rows, N, K, act, glu, workspace, ws_bytes, cut.hint, cut.hint ? cut.split : 0, false, st);
+                         M - cut.rows, N, K, act, glu, workspace, ws_bytes, rest.hint, rest.split, false, st);
     }
     if (cut.cols) {
       launch_gemm(x, ldx, w, ldw, false, nullptr, bias, y, ldy, M, cut.cols, K, act, glu, workspace, ws_bytes, 4 << 8, 1, false, st);
+      const FourPlan rest = gemm_rest_plan(cut, M, N - cut.cols, K, glu, ws_bytes);
       return launch_gemm(x, ldx, (const bf16_t*)w + cut.cols * ldw, ldw, false, nullptr, bias ? (const bf16_t*)bias + cut.cols : nullptr,
-                         (bf16_t*)y + (glu ? cut.cols / 2 : cut.cols), ldy, M, N - cut.cols, K, act, glu, workspace, ws_bytes, cut.hint,
-                         cut.hint ? cut.split : 0, false, st);
+                         (bf16_t*)y + (glu ? cut.cols / 2 : cut.cols), ldy, M, N - cut.cols, K, act, glu, workspace, ws_bytes, rest.hint,
+                         rest.split, false, st);
     }
   }
   if (!y && (!partial_out || slabs_of_plan(M, N, K, w_fp8, glu, act, nt_hint, split_hint, ws_bytes) == 0))
@@ -2095,12 +2203,17 @@ static constexpr int kSlots = 4;
 static thread_local int g_ws_slot = 0;
 void gemm_set_slot(int s) { g_ws_slot = s & (kSlots - 1); }
 
-static int* sk_counters(int n) {
+// `capturing`: the stream of the launch; where it is being captured and the counters are not there yet, null is returned
+static int* sk_counters(int n, const hipStream_t* capturing = nullptr) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) throw std::runtime_error("gemm counters: bad device");
   std::lock_guard<std::mutex> lk(g_sk_mu);
   if (n <= g_sk_capacity[dev]) return g_sk_counters[dev] + (size_t)g_ws_slot * g_sk_capacity[dev];
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (capturing) {
+    (void)hipStreamIsCapturing(*capturing, &cs);
+    if (cs != hipStreamCaptureStatusNone) return nullptr;
+  }
   (void)hipStreamIsCapturing(nullptr, &cs);
   if (cs != hipStreamCaptureStatusNone) throw std::runtime_error("gemm counters must be allocated before capture");
   int cap = std::max(n, 1 << 16);
@@ -2204,6 +2317,24 @@ int launch_tiled(const bf16_t* X, int64_t ldx, const void* W, int64_t ldw, const
       splitk_reduce_kernel<<<rgrid, 256, 0, st>>>(part, s, M, N, B, Y, ldy, act, g);
       HIP_CHECK_LAUNCH();
     }
+    return 0;
+  }
+  if ((tsel & kFourHint) && (f8 || !gemm_four_ok(N, K, ldx, ldw, Y, ldy, g != 0))) tsel = split_hint = s = 0;
+  if (tsel & kFourHint) {  // tiles by four waves (gemm_four.hip)
+    int bm, bn;
+    if (!gemm_four_dims(tsel & 15, &bm, &bn)) throw std::runtime_error("gemm: no such tile");
+    const int nt = tiles_of(M, N, bm, bn);
+    s = std::max(1, split_hint);
+    int* cnt = (tsel & 256) && s > 1 && Y && (int64_t)nt * s * bm * bn * 4 <= ws_bytes ? sk_counters(nt, &st) : nullptr;
+    if (!cnt && (qe || (int64_t)s * M * N * 4 > ws_bytes)) s = 1;
+    const bool slabs = s > 1 && !cnt;
+    launch_gemm_four(tsel & 15, X, ldx, (const bf16_t*)W, ldw, B, Y, ldy, s > 1 ? (float*)workspace : nullptr, M, N, K, slabs ? 0 : act,
+                     slabs ? 0 : g, s, 4, st, cnt, qe);
+    if (!slabs || (partial_out && !g && act == 0)) return slabs ? s : 0;
+    const int nout = g ? N / 2 : N;
+    dim3 rgrid(std::min((nout + 255) / 256, 64), M);
+    splitk_reduce_kernel<<<rgrid, 256, 0, st>>>((float*)workspace, s, M, N, B, Y, ldy, act, g);
+    HIP_CHECK_LAUNCH();
     return 0;
   }
   if (f8 && (tsel & 15) >= 5) tsel = (tsel & ~15) | 1;  // 8-wave and mid tiles are bf16-only
@@ -2345,6 +2476,14 @@ static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int
       return s > 1 ? s : 0;
     }
     if ((tsel & 128) && !w_fp8 && (tsel & 15) < 5) return 0;  // stream-K combines in-kernel
+    if ((tsel & kFourHint) && w_fp8) tsel = split_hint = 0;
+    if (tsel & kFourHint) {
+      int bm, bn;
+      if (!gemm_four_dims(tsel & 15, &bm, &bn)) return 0;  // rejected at launch
+      s = std::max(1, split_hint);
+      if ((tsel & 256) && (int64_t)tiles_of(M, N, bm, bn) * s * bm * bn * 4 <= ws_bytes) return 0;  // combined in the launch
+      return s > 1 && (int64_t)s * M * N * 4 <= ws_bytes ? s : 0;
+    }
     if (w_fp8 && ((tsel & 15) == 4 || (tsel & 15) >= 5)) tsel = (tsel & ~15) | 1;
     if ((tsel & 256) && (tsel & 15) != 4) {  // split-K combined in-launch
       int s2 = split_hint, t2 = tsel;
@@ -2389,6 +2528,20 @@ int launch_gemm_qkv(const void* x, int64_t ldx, const void* w, int64_t ldw, cons
     return 0;
   }
   int tsel = nt_hint >> 8, s = split_hint;
+  if (tsel & kFourHint) {  // four-wave tiles; a plan that combines split sums in the launch brings no split along (gemm_plan)
+    int bm, bn;
+    if ((tsel & 256) && s <= 1) {
+      const FourPlan p = gemm_four_plan(M, N, K, false, false, ws_bytes);
+      tsel = p.hint >> 8, s = p.split;
+    }
+    if (!gemm_four_ok(N, K, ldx, ldw, y, ldy, false) || !gemm_four_dims(tsel & 15, &bm, &bn) || (s > 1 && !(tsel & 256)) ||
+        (qe.do_rope && qe.style == 0 && bn % qe.D))
+      return -1;
+    if (s > 1 && (int64_t)tiles_of(M, N, bm, bn) * s * bm * bn * 4 > ws_bytes) return -1;
+    launch_tiled((const bf16_t*)x, ldx, w, ldw, (const bf16_t*)bias, (bf16_t*)y, ldy, M, N, K, 0, 0, tsel, s, workspace, ws_bytes, false, st,
+                 nullptr, &qe);
+    return 0;
+  }
   gemm_tiled_plan(M, N, K, &tsel, &s, false);
   if (tsel == 4) {  // 256 x 256 tiles, and what they leave over as launch_gemm has it
     if ((qe.do_rope && qe.style != 1) || 256 % qe.D || !gemm_quad_ok(N, K, ldx, ldw, 256, y, ldy, 2, false)) return -1;
@@ -2406,12 +2559,13 @@ int launch_gemm_qkv(const void* x, int64_t ldx, const void* w, int64_t ldw, cons
     const bf16_t* rw = (const bf16_t*)w + (cols < N ? (int64_t)cols * ldw : 0);
     const bf16_t* rb = bias ? (const bf16_t*)bias + (cols < N ? cols : 0) : nullptr;
     const int m = rows < M ? M - rows : M, n = cols < N ? N - cols : N;
-    int nt = cut.hint, sp = 1;
+    const FourPlan rest = gemm_rest_plan(cut, m, n, K, false, ws_bytes);
+    int nt = rest.hint, sp = 1;
     if (!nt) {  // up to 64 rows: the decode kernel where its plan is unsplit, else 64 x 64 tiles
       gemm_static_plan(m, n, K, false, false, ws_bytes, &nt, &sp);
       if (!((nt >> 8) & kDecHint) || sp > 1) nt = 3 << 8;
     }
-    launch_tiled(rx, ldx, rw, ldw, rb, ry, ldy, m, n, K, 0, 0, nt >> 8, 1, workspace, ws_bytes, false, st, nullptr, &re);
+    launch_tiled(rx, ldx, rw, ldw, rb, ry, ldy, m, n, K, 0, 0, nt >> 8, rest.hint ? rest.split : 1, workspace, ws_bytes, false, st, nullptr, &re);
     return 0;
   }
   if ((tsel & 15) == 4 || (tsel & 128)) return -1;
@@ -2436,6 +2590,7 @@ int launch_gemm_qkv_args(const void* x, int64_t ldx, const void* w, int64_t ldw,
   return launch_gemm_qkv(x, ldx, w, ldw, bias, y, ldy, M, N, K, workspace, ws_bytes, nt_hint, split_hint, qe, st);
 }
 
+void gemm_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int* nt, int* splitk, bool four);
 void gemm_cut_of(int M, int N, int K, bool glu, int* rows, int* cols, int* split) {
   const GemmCut c = gemm_cut(M, N, K, glu, 64 << 20);
   *rows = c.rows;
@@ -2443,17 +2598,27 @@ void gemm_cut_of(int M, int N, int K, bool glu, int* rows, int* cols, int* split
   *split = c.split;
 }
 
+// The plan of a product whose result goes straight into an op that can sum its slabs: a split one, the slabs unsummed, where the older rules
+// split K of the finished product, so that it stays in 32 bits there; else split 1, and the product is finished by the plan of its size
+void gemm_closing_plan(int M, int N, int K, int* nt, int* splitk) {
+  gemm_plan(M, N, K, false, false, false, nt, splitk, false);
+  if (*splitk <= 1 || (M <= 32 && K > 5120)) return;  // (27 x 2048 x 5632: 8.4 us on 64 x 64 tiles in eight slabs, 10.2 here in four)
+  const FourPlan p = gemm_four_plan(M, N, K, false, true, 64 << 20);
+  if (p.hint) *nt = p.hint, *splitk = p.split;
+}
+
 // The plan of a product without hints. slabs: of one whose consumer sums split-K slabs itself
-void gemm_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int* nt, int* splitk) {
+void gemm_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int* nt, int* splitk, bool four) {
   *nt = *splitk = 0;
   const bool tuned = gemm_tuned_get(M, N, K, glu, w_fp8 ? 1 : 0, nt, splitk);
-  if (!tuned) (w_fp8 ? gemm_static_plan_f8 : gemm_static_plan)(M, N, K, glu, slabs && !glu, 64 << 20, nt, splitk);
+  if (!tuned && w_fp8) gemm_static_plan_f8(M, N, K, glu, slabs && !glu, 64 << 20, nt, splitk);
+  else if (!tuned) gemm_static_plan(M, N, K, glu, slabs && !glu, 64 << 20, nt, splitk, four);
   if (tuned || *nt) {
     if ((*nt >> 8) & kDecHint) {
       *splitk = ((*nt >> 8) & 256) ? 1 : dec_split(M, N, K, *splitk, INT64_MAX);
     } else if ((*nt >> 8) & (128 | 256)) {
       *splitk = 1;  // stream-K / split-K combine finish their tiles in-kernel: no partial slabs for the consumer
-    } else if (*nt >> 8) {  // tiled hint: the split the kernel will really use
+    } else if ((*nt >> 8) && !((*nt >> 8) & kFourHint)) {  // tiled hint: the split the kernel will really use
       int tsel = *nt >> 8;
       gemm_tiled_plan(M, N, K, &tsel, splitk, glu);
     }

@@ -225,7 +225,7 @@ class DecoderLM:
         nt, split = lib.gemm_plan(M, N, K, False, False, M > 64)
         if M > 64:
             return (nt, 1) if split <= 1 and nt >> 8 and M >= 128 else None
-        return (nt, split) if nt >> 8 & 1024 and split == 1 else None  # (the hint bit of csrc/gemm_dec.hip)
+        return (nt, split) if nt >> 8 & (1024 | 2048) and split == 1 else None  # (the hint bits of csrc/gemm_dec.hip, gemm_four.hip)
 
     def _qkv_rope_cache(self, L, y, inp: StepInput, kc, vc):
         """QKV projection, RoPE and the paged KV write of the step's tokens -> the bf16 qkv rows.

@@ -924,8 +924,8 @@ def linear_f(x, w, out_dtype, bias=None, act="none", closing=False):
         return torch.empty(0, N, dtype=out_dtype, device=x.device)
     if _mfma_ok(x, w, out_dtype):
         if closing and bias is None and M <= 64 and N <= 2048:
-            nt, split = lib().gemm_plan(M, N, K, False, False, False)
-            if split > 1:  # (the plan of the finished product, but for its sum)
+            nt, split = lib().gemm_closing_plan(M, N, K)
+            if split > 1:
                 return linear(x, w, nt_hint=nt, split_hint=split, partial_ok=True)
         return linear(x, w, bias, act)
     y = torch.empty(M, N, dtype=out_dtype, device=x.device)
