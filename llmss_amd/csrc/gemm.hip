@@ -1782,7 +1782,7 @@ static constexpr FourCost kFourMany[] = {
     {8, 64, 32, 2, 2.55, 1.96, 0.00, 0.162, 0.268, 0.180, 1.63, 2.06, 19.7e6},  {9, 192, 192, 1, 0.00, 8.76, 3.23, 0.855, 0.856, 0.286, 4.34, 0.77, 3.50e6},
     {10, 64, 128, 2, 1.08, 4.24, 0.61, 0.302, 0.626, 0.236, 2.53, 1.32, 2.69e6}, {11, 128, 64, 1, 0.68, 5.01, 0.57, 0.292, 0.279, 0.225, 2.73, 1.14, 12.4e6},
     {12, 64, 128, 1, 0.80, 4.87, 0.58, 0.311, 0.299, 0.272, 2.67, 1.06, 4.76e6}, {13, 64, 64, 1, 1.74, 3.34, 0.21, 0.208, 0.192, 0.174, 2.08, 1.58, 2.28e6}};
-static constexpr FourCost kQuadCost = {4, 256, 256, 1, 1.88, 8.24, 2.39, 1.335, 1.368, 0.261, 0, 0, 5.0e6};  // gemm_quad.hip
+static constexpr FourCost kQuadCost = {4, 256, 256, 1, 3.07, 5.70, 1.72, 1.465, 1.425, 0.317, 0, 0, 5.0e6};  // gemm_quad.hip
 static double four_us(const FourCost& c, int M, int N, int K, bool glu, int split) {
   const int64_t wgs = (int64_t)tiles_of(M, N, c.bm, c.bn) * split, cap = 256 * c.slots, rest = wgs % cap;
   const int per = (K / 64 + split - 1) / split, held = (int)((rest + 255) / 256);

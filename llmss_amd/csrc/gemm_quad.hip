@@ -8,8 +8,15 @@
 // costs is the loads and the epilogue:
 // - a step's loads are issued 1.5 (X) and 1 (W) steps before the barrier that waits for them, by count. With a step's distance of less than
 //   one (two buffers) it took 1.63 - 1.84 us; a ring of four 32-k buffers, with more distance but rows of 64 bytes, 1.6 - 1.75 us.
-// - 42 us a tile with stores of 64 bytes a row straight from the accumulators, 20 us through LDS with the activations' code
-//   unrolled (36 KB of it), 6 - 8 us as written below.
+// - the start of a tile and its end, 8.5 us of 53 at K = 2048 while each tile was a workgroup: 42 us a tile with stores of 64 bytes a row straight
+//   from the accumulators, 20 us through LDS with the activations' code unrolled (36 KB of it), 6 - 8 us through LDS as written at the end. So
+//   a workgroup now takes every 256th tile (RING): the ring of loads runs on into the next tile while the last steps of this one are
+//   multiplied, and the tile leaves straight from the accumulators in whole lines, without LDS (quad_store): 5.7 us a tile. The clock gives a
+//   part back: matrix units that are busy for more of the time run slower. us: 8192 x 10240 x 2048 248 -> 241, x 9472 243 -> 233, SwiGLU
+//   8192 x 11264 x 2048 297 -> 280, x 4096 105 -> 100, 8192 x 8192 x 768 97 -> 88, SwiGLU 8192 x 22016 x 4096 1047 -> 1017, 8192 x 5120 x 2048 143 -> 138;
+//   one tile a CU is as before (8192 x 2048 x 4096 100). Prompts of Babotar 5831 -> 5694, Fizelix 6963 -> 6823, Nolavik 5024 -> 4919.
+//   Products with an activation but no gate, whose code does not fit beside so many accumulators, and the query / key / value product with its
+//   rotation keep the way through LDS.
 // Against the ping-pong kernel of 8 waves (weights not in the caches, us): 8192 x 12288 x 4096 794 -> 715, 8192 x 4096 x 4096 232 -> 206,
 // 8192 x 4096 x 11008 540 -> 530, 8192 x 11264 x 2048 379 -> 330; SwiGLU 8192 x 22016 x 4096 1237 (1195 TFLOP/s).
 //
@@ -18,7 +25,71 @@
 // matrices, gate and up, the products scaled by the pair's weight first. GLU: W's rows are gate and up in alternating groups of 16.
 #include "gemm_quad.h"
 
+#include <algorithm>
 #include <type_traits>
+
+// The wave's 128 x 128 part of a finished tile, straight from the accumulators. A lane holds, of row 16 mt + li, sixteen bytes of neighbouring
+// columns (two tiles of eight: GLU, four gates and their four ups twice; fp32: one tile of four) - 64 bytes a row and instruction, and stores of
+// half lines take four times as long. So two such pieces change hands between lanes li and li ^ 8 (a rotation by eight within the row of
+// sixteen lanes): one instruction then writes rows 0 .. 7 of the sixteen in whole lines, another rows 8 .. 15.
+// Rows and columns past the last lie outside the descriptor, so that no branch stands between the stores.
+template <int GRP, int GLU>
+__device__ __forceinline__ void quad_store(const f32x4 (&acc)[8][8], const PpGroup& gr, const bf16_t* __restrict__ bias, bf16_t* __restrict__ Y,
+                                           int64_t ldy, int m0, int n0, int M, int N, int li, int g, const float (&sw)[8]) {
+  constexpr int ES = GRP == 2 ? 4 : 2, COLS = GRP == 2 ? 4 : GLU ? 1 : 2, RUN = GRP == 2 ? 32 : 64;  // runs of a line
+  const int nout = GLU ? N / 2 : N, o0 = GLU ? n0 / 2 : n0, up = li >> 3;
+  const uint32_t pitch = (uint32_t)ldy * ES;
+  const auto ry = uniform_rsrc((GRP == 2 ? reinterpret_cast<char*>(gr.Yf) : reinterpret_cast<char*>(Y)) + (int64_t)m0 * ldy * ES,
+                               (int64_t)max(min(M - m0, 128), 0) * pitch);
+#pragma unroll
+  for (int c = 0; c < COLS; ++c) {
+    float bs[2][GLU ? 16 : 8] = {};
+    if (GRP != 2 && bias) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          // (GLU: bias lies as W's rows, gates and ups in groups of 16)
+          const int n = GLU ? n0 + 64 * h + 32 * (g >> 1) + 8 * (g & 1) + i : n0 + 64 * c + 32 * h + 8 * g + i;
+          bs[h][i] = n < N ? bf2f(bias[n]) : 0.f;
+          if constexpr (GLU) bs[h][8 + i] = n < N ? bf2f(bias[n + 16]) : 0.f;
+        }
+    }
+    const int n = o0 + RUN * c + RUN / 2 * up + RUN / 8 * g;
+    const uint32_t at = (uint32_t)(li & 7) * pitch + (uint32_t)n * ES + (n < nout ? 0u : 0x80000000u);
+#pragma unroll
+    for (int mt = 0; mt < 8; ++mt) {
+      u32x4 a, b;
+      if constexpr (GRP == 2) {
+        a = __builtin_bit_cast(u32x4, acc[2 * c][mt]), b = __builtin_bit_cast(u32x4, acc[2 * c + 1][mt]);
+      } else {
+        u16x8 o[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            if constexpr (GLU) {
+              const int t = 4 * h + 2 * (i >> 2);
+              const float gv = acc[t][mt][i & 3], uv = acc[t + 1][mt][i & 3];
+              if constexpr (GRP == 3) o[h][i] = f2bf(glu_clamped_t(gv * sw[mt], uv * sw[mt], gr.limit, gr.alpha, gr.silu));
+              else o[h][i] = f2bf((GLU == 2 ? gelu_gate(gv + bs[h][i]) : silu(gv + bs[h][i])) * (uv + bs[h][8 + i]));
+            } else {
+              o[h][i] = f2bf(acc[4 * c + 2 * h + (i >> 2)][mt][i & 3] + bs[h][i]);
+            }
+          }
+        a = __builtin_bit_cast(u32x4, o[0]), b = __builtin_bit_cast(u32x4, o[1]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t x = a[i], y = b[i];
+        a[i] = __builtin_amdgcn_update_dpp(x, y, 0x128, 0xf, 0xc, false);  // lanes 8 .. 15: of b, from li - 8
+        b[i] = __builtin_amdgcn_update_dpp(y, x, 0x128, 0xf, 0x3, false);  // lanes 0 .. 7: of a, from li + 8
+      }
+      __builtin_amdgcn_raw_buffer_store_b128(a, ry, at + (uint32_t)(16 * mt) * pitch, 0, GRP == 2 ? 0 : 2);
+      __builtin_amdgcn_raw_buffer_store_b128(b, ry, at + (uint32_t)(16 * mt + 8) * pitch, 0, GRP == 2 ? 0 : 2);
+    }
+  }
+}
 
 // GLU 1: SiLU gates, 2: the tanh form of GELU, 8192 x 11264 x 2048 with its gate 323 us (the product alone 306, with a launch of its own for the
 // gate 356; 64 rows 15.5 and 17.3, one row 11.2 and 13.0)
@@ -28,7 +99,7 @@
 // looked up once a row and kept in the ring's fifth buffer.
 // Against the product and a rotation of its own, which reads and writes all of it again (us): 8192 x 12288 x 4096 676 -> 621, 3999 rows 343 ->
 // 315; 8192 x 4800 x 1600 without a rotation 159 -> 140.
-template <int GRP, int GLU, bool QKV = false>
+template <int GRP, int GLU, bool QKV = false, bool RING = false>
 __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restrict__ X, int64_t ldx,
                                                            const bf16_t* __restrict__ W, int64_t ldw,
                                                            const bf16_t* __restrict__ bias, bf16_t* __restrict__ Y,
@@ -43,56 +114,82 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
   const int li = lane & 15, g = lane >> 4;
   const int wr = w >> 1, wc = w & 1;
   const int ntn = (N + 255) / 256, ntm = (M + 255) / 256;
-  int m0, n0;
-  if constexpr (GRP != 0) {
-    const int nt = gr.meta[0];
-    if ((int)blockIdx.x >= nt * ntn) return;
-    const int id = xcd_remap(blockIdx.x, nt * ntn), ty = id / ntn;
-    const int e = gr.meta[1 + (gr.E + 1) + ty];
-    n0 = (id - ty * ntn) * 256;
-    m0 = gr.meta[1 + (gr.E + 1) + gr.maxt + ty];
-    M = gr.meta[1 + e + 1];
-    // (rows 16 .. 31 of every 32 of a tile are up rows: a load takes eight rows, so a wave's loads are all of one matrix)
-    if (GRP == 3 && (w & 2)) W = gr.Wu;
-    W += (int64_t)e * gr.sB;
-  } else {
-    const int tile = xcd_remap(blockIdx.x, ntn * ntm);
-    const int grp = tile / (group_m * ntn), gidx = tile - grp * (group_m * ntn);
-    const int gm = min(group_m, ntm - grp * group_m);
-    m0 = (grp * group_m + gidx % gm) * 256, n0 = (gidx / gm) * 256;
-  }
+  const int tiles = GRP != 0 ? __builtin_amdgcn_readfirstlane(gr.meta[0]) * ntn : ntn * ntm;
+  if ((int)blockIdx.x >= tiles) return;
   const int nk = K >> 6;
-  const uint64_t xbytes = (uint64_t)(M - m0) * (uint64_t)ldx * 2, wbytes = (uint64_t)(GRP == 3 ? (N - n0) / 2 : N - n0) * (uint64_t)ldw * 2;
-  const auto rx = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<char*>(reinterpret_cast<const char*>(X) + (GATHER ? 0 : (int64_t)m0 * ldx * 2)), (short)0,
-      (int)(GATHER || xbytes > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)xbytes), 0x00020000);
-  const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(W) + (int64_t)(GRP == 3 ? n0 / 2 : n0) * ldw * 2),
-                                                    (short)0, (int)(wbytes > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)wbytes),
-                                                    0x00020000);
+  if (GRP == 3 && (w & 2)) W = gr.Wu;
+  // tile b: its first row and column, the rows that there are, and where its operands lie (bytes that exist from there on)
+  struct Tile {
+    int m0, n0, M;
+    const char *x, *w;
+    uint32_t xb, wb;
+  };
+  auto place = [&](int b) {
+    Tile t;
+    const bf16_t* wt = W;
+    t.M = M;
+    if constexpr (GRP != 0) {
+      const int id = xcd_remap(b, tiles), ty = id / ntn;
+      const int e = __builtin_amdgcn_readfirstlane(gr.meta[1 + (gr.E + 1) + ty]);
+      t.n0 = (id - ty * ntn) * 256;
+      t.m0 = __builtin_amdgcn_readfirstlane(gr.meta[1 + (gr.E + 1) + gr.maxt + ty]);
+      t.M = __builtin_amdgcn_readfirstlane(gr.meta[1 + e + 1]);
+      wt += (int64_t)e * gr.sB;
+    } else {
+      const int tile = xcd_remap(b, tiles);
+      const int grp = tile / (group_m * ntn), gidx = tile - grp * (group_m * ntn);
+      const int gm = min(group_m, ntm - grp * group_m);
+      t.m0 = (grp * group_m + gidx % gm) * 256, t.n0 = (gidx / gm) * 256;
+    }
+    const uint64_t xb = GATHER ? ~0ull : (uint64_t)(t.M - t.m0) * (uint64_t)ldx * 2;
+    // (rows 16 .. 31 of every 32 of a tile are up rows: a load takes eight rows, so a wave's loads are all of one matrix)
+    const uint64_t wb = (uint64_t)(GRP == 3 ? (N - t.n0) / 2 : N - t.n0) * (uint64_t)ldw * 2;
+    t.x = reinterpret_cast<const char*>(X) + (GATHER ? 0 : (int64_t)t.m0 * ldx * 2);
+    t.w = reinterpret_cast<const char*>(wt) + (int64_t)(GRP == 3 ? t.n0 / 2 : t.n0) * ldw * 2;
+    t.xb = xb > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)xb;
+    t.wb = wb > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)wb;
+    return t;
+  };
+  int blk = blockIdx.x;
+  Tile cur = place(blk), next = cur;
+  if constexpr (RING) {
+    if (blk + (int)gridDim.x < tiles) next = place(blk + gridDim.x);
+    else next.xb = next.wb = 0;  // (nothing is in its range)
+  }
   // chunk c of row r lies at place c ^ key(r) of the row: the eight rows that a fragment read's eight lanes take fall on eight
   // different 16-byte columns of the banks
   auto xkey = [](int r) { return r & 7; };
-  auto wkey = [](int r) { return GLU ? r & 7 : (r & 3) | ((r >> 3) & 1) << 2; };
-  uint32_t vx[8], vw[8];
+  // (W's rows as they come, or so that a lane gets eight neighbouring columns in two tiles, below)
+  constexpr bool PLAIN = RING ? GRP == 2 : GLU != 0;
+  auto wkey = [](int r) { return PLAIN ? r & 7 : (r & 3) | ((r >> 3) & 1) << 2; };
+  uint32_t vx[8], vw[8], vn[8];
+  // rows of X that a lane loads (GATHER: by pair), and what its pairs weigh
+  auto pair_of = [&](const Tile& t, int i) { return GATHER ? gr.order[min(t.m0 + (i * 4 + w) * 8 + (lane >> 3), t.M - 1)] : 0; };
+  auto offset_of = [&](int pair, int i) {
+    const int row = (i * 4 + w) * 8 + (lane >> 3);
+    return (uint32_t)(GATHER ? pair / gr.top : row) * (uint32_t)(ldx * 2) + (uint32_t)(((lane & 7) ^ xkey(row)) << 4);
+  };
+  auto weight_of = [&](const Tile& t, int mt) { return gr.pw ? gr.pw[gr.order[min(t.m0 + wr * 128 + 16 * mt + li, t.M - 1)]] : 1.f; };
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int row = (i * 4 + w) * 8 + (lane >> 3);
-    int xr = row;
-    if constexpr (GATHER) xr = gr.order[min(m0 + row, M - 1)] / gr.top;
-    vx[i] = (uint32_t)xr * (uint32_t)(ldx * 2) + (uint32_t)(((lane & 7) ^ xkey(row)) << 4);
+    vx[i] = offset_of(pair_of(cur, i), i);
+    if constexpr (RING && GATHER) vn[i] = offset_of(pair_of(next, i), i);
     const int wrw = GRP == 3 ? (row >> 5) * 16 + (row & 15) : row;
     vw[i] = (uint32_t)wrw * (uint32_t)(ldw * 2) + (uint32_t)(((lane & 7) ^ wkey(row)) << 4);
   }
   // eight rows (1 KB) of step T_ of X or W into buffer B_
-#define Q_LOADX(I_, T_, B_)                                                                                           \
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (LDS_AS void*)(smem + (B_) + ((I_) * 4 + w) * 1024), 16, vx[I_], (uint32_t)((T_) * 128), 0, 0)
-#define Q_LOADW(I_, T_, B_)                                                                                           \
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (LDS_AS void*)(smem + (B_) + ((I_) * 4 + w) * 1024), 16, vw[I_], (uint32_t)((T_) * 128), 0, 0)
-  const int wrow = GLU ? li : 8 * (li >> 2) + (li & 3);
+#define Q_RSRC(P_, B_) __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(P_), (short)0, (int)(B_), 0x00020000)
+#define Q_LOAD(R_, V_, I_, T_, B_)                                                                                    \
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(R_, (LDS_AS void*)(smem + (B_) + ((I_) * 4 + w) * 1024), 16, (uint32_t)(V_), (uint32_t)((T_) * 128), 0, 0)
+  const int wrow = PLAIN ? li : (GLU ? 32 * (li >> 3) + 8 * ((li >> 2) & 1) + (li & 3) : 8 * (li >> 2) + (li & 3));
   const int xo = (wr * 128 + li) * 128 + ((g ^ xkey(li)) << 4);
   const int wo = (wc * 128 + wrow) * 128 + ((g ^ wkey(wrow)) << 4);
 #define Q_X(P_, T_) (*reinterpret_cast<const s16x8*>(smem + (P_) + (T_) * 2048))
-#define Q_W(P_, T_) (*reinterpret_cast<const s16x8*>(smem + (P_) + (GLU ? (T_) * 2048 : ((T_) >> 1) * 4096 + ((T_) & 1) * 512)))
+#define Q_W(P_, T_)                                \
+  (*reinterpret_cast<const s16x8*>(smem + (P_) + (PLAIN ? (T_) * 2048                                                        \
+                                                  : GLU ? ((T_) >> 2) * 8192 + (((T_) >> 1) & 1) * 512 + ((T_) & 1) * 2048  \
+                                                        : ((T_) >> 1) * 4096 + ((T_) & 1) * 512)))
   f32x4 acc[8][8];  // [W tile][X tile]
 #pragma unroll
   for (int a = 0; a < 8; ++a)
@@ -108,13 +205,16 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
     else                                                                                                                  \
       asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[NT_][MT_]) : "v"(W_[NT_]), "v"(X_[MT_]));                  \
   } while (0)
+  {
+    const auto rx = Q_RSRC(cur.x, cur.xb), rw = Q_RSRC(cur.w, cur.wb);
 #pragma unroll
-  for (int l = 0; l < 5; ++l) {
-    const int t = min(l >> 1, nk - 1);
+    for (int l = 0; l < 5; ++l) {
+      const int t = min(l >> 1, nk - 1);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (l & 1) Q_LOADW(i, t, l * BUF);
-      else Q_LOADX(i, t, l * BUF);
+      for (int i = 0; i < 8; ++i) {
+        if (l & 1) Q_LOAD(rw, vw[i], i, t, l * BUF);
+        else Q_LOAD(rx, vx[i], i, t, l * BUF);
+      }
     }
   }
   __builtin_amdgcn_s_waitcnt(0x4F78);  // vmcnt(24): the first step has landed
@@ -125,57 +225,95 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
     w0[q] = Q_W(BUF + wo, q);
     x0[q] = Q_X(xo, q);
   }
-  // One copy of the body: with separate last steps the compiler moves every accumulator between register files. The last steps
-  // load the last one again, and the very last reads fragments that nobody uses.
   int cx = 0;  // buffer of this step's X; its W lies in the next one
 #pragma unroll 1
-  for (int t = 0; t < nk; ++t) {
-    const int cw = cx == 4 * BUF ? 0 : cx + BUF;
-    const int nx = cw == 4 * BUF ? 0 : cw + BUF;
-    const int nw = nx == 4 * BUF ? 0 : nx + BUF;
-    const int xa = cx + (xo ^ 64), wa = cw + (wo ^ 64), xb = nx + xo, wb = nw + wo;
-    const int tw = min(t + 2, nk - 1), tx = min(t + 3, nk - 1);
+  for (;;) {
+    // One copy of the body: with separate last steps the compiler moves every accumulator between register files. The last steps load the
+    // next tile's first ones (RING; or the last one again), and the very last reads its fragments (or some that nobody uses).
+#pragma unroll 1
+    for (int t = 0; t < nk; ++t) {
+      const int cw = cx == 4 * BUF ? 0 : cx + BUF;
+      const int nx = cw == 4 * BUF ? 0 : cw + BUF;
+      const int nw = nx == 4 * BUF ? 0 : nx + BUF;
+      const int xa = cx + (xo ^ 64), wa = cw + (wo ^ 64), xb = nx + xo, wb = nw + wo;
+      const bool wn = RING && t + 2 >= nk, xn = RING && t + 3 >= nk;
+      const int tw = RING ? t + 2 - (wn ? nk : 0) : min(t + 2, nk - 1), tx = RING ? t + 3 - (xn ? nk : 0) : min(t + 3, nk - 1);
+      const auto rx = Q_RSRC(xn ? next.x : cur.x, xn ? next.xb : cur.xb), rw = Q_RSRC(wn ? next.w : cur.w, wn ? next.wb : cur.wb);
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      if (q < 8) {
-        w1[q] = Q_W(wa, q);
-        x1[q] = Q_X(xa, q);
+      for (int q = 0; q < 16; ++q) {
+        if (q < 8) {
+          w1[q] = Q_W(wa, q);
+          x1[q] = Q_X(xa, q);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) Q_MFMA(w0, x0, q >> 1, (q & 1) * 4 + e);
+        __builtin_amdgcn_sched_barrier(0);
       }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) Q_MFMA(w0, x0, q >> 1, (q & 1) * 4 + e);
+      __builtin_amdgcn_s_waitcnt(0x0078);  // vmcnt(8) lgkmcnt(0): this step is read, this wave's part of the next has landed
+      __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        if (q < 8) {
+          w0[q] = Q_W(wb, q);
+          x0[q] = Q_X(xb, q);
+          Q_LOAD(rw, vw[q], q, tw, cx);
+        } else {
+          Q_LOAD(rx, RING && GATHER && xn ? vn[q - 8] : vx[q - 8], q - 8, tx, cw);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) Q_MFMA(w1, x1, q >> 1, (q & 1) * 4 + e);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      cx = nx;
     }
-    __builtin_amdgcn_s_waitcnt(0x0078);  // vmcnt(8) lgkmcnt(0): this step is read, this wave's part of the next has landed
-    __builtin_amdgcn_s_barrier();
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products are written, which the compiler does not see
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!RING) {
+      break;
+    } else {
+      // (what the tile after the next needs of the lists is asked for before the stores, behind which it would wait)
+      Tile then = next;
+      if (blk + 2 * (int)gridDim.x < tiles) then = place(blk + 2 * gridDim.x);
+      else then.xb = then.wb = 0;
+      int pairs[8];
+      float sw[8];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      if (q < 8) {
-        w0[q] = Q_W(wb, q);
-        x0[q] = Q_X(xb, q);
-        Q_LOADW(q, tw, cx);
-      } else {
-        Q_LOADX(q - 8, tx, cw);
+      for (int i = 0; i < 8; ++i) {
+        if constexpr (GATHER) pairs[i] = pair_of(then, i);
+        if constexpr (GRP == 3) sw[i] = weight_of(cur, i);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      quad_store<GRP, GLU>(acc, gr, bias, Y, ldy, cur.m0 + wr * 128, cur.n0 + wc * 128, cur.M, N, li, g, sw);
+      blk += gridDim.x;
+      if (blk >= tiles) break;
+      cur = next, next = then;
+      if constexpr (GATHER) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) vx[i] = vn[i], vn[i] = offset_of(pairs[i], i);
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) Q_MFMA(w1, x1, q >> 1, (q & 1) * 4 + e);
+      for (int a = 0; a < 8; ++a)
+#pragma unroll
+        for (int b = 0; b < 8; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+      asm volatile("s_nop 7" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
     }
-    cx = nx;
   }
 #undef Q_MFMA
 #undef Q_X
 #undef Q_W
-#undef Q_LOADX
-#undef Q_LOADW
-  __builtin_amdgcn_s_waitcnt(0x0070);                    // no load of this wave is on its way into LDS any more,
-  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");     // the last products are written, which the compiler does not see,
-  __builtin_amdgcn_s_barrier();                          // and all waves are there
+#undef Q_LOAD
+#undef Q_RSRC
+  __builtin_amdgcn_s_waitcnt(0x0070);  // no load of this wave is on its way into LDS any more,
+  if constexpr (RING) return;
+  const int m0 = cur.m0, n0 = cur.n0;
+  M = cur.M;
+  __builtin_amdgcn_s_barrier();  // and all waves are there
   __builtin_amdgcn_sched_barrier(0);
-  // Out through LDS, 64 columns of the wave's 128 rows at a time as fp32: stored from the accumulators' own layout (16 rows of 64
-  // bytes an instruction) the stores alone took 42 us a tile. A lane holds, of row 16 mt + li, eight neighbouring columns in tiles
-  // 2 p and 2 p + 1 (GLU: four gates and their four ups). The bf16 stores bypass the caches' replacement, which keeps X and W of the tiles
-  // to come: 632 -> 606 us at 8192 x 12288 x 4096, 1.5 % of a prompt step.
+  // Out through LDS, 64 columns of the wave's 128 rows at a time as fp32. A lane holds, of row 16 mt + li, eight neighbouring columns in tiles
+  // 2 p and 2 p + 1. The bf16 stores bypass the caches' replacement, which keeps X and W of the tiles to come: 632 -> 606 us at 8192 x 12288 x
+  // 4096, 1.5 % of a prompt step.
   char* img = smem + w * BUF;
   if constexpr (QKV) {
     const int D = qe.D, nq = qe.nh * D, nqk = nq + qe.nkv * D, rh = qe.rot >> 1, nw0 = n0 + wc * 128, mw0 = m0 + wr * 128;
@@ -253,99 +391,40 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
     return;
   }
   auto flush = [&](int c0) {  // the image is columns c0 .. c0 + 63 of the output
-    if constexpr (GRP == 2) {
-      const int n = c0 + 4 * li;
-#pragma unroll 4
-      for (int i = 0; i < 32; ++i) {
-        const int r = 4 * i + g, m = m0 + wr * 128 + r;
-        const f32x4 v = *reinterpret_cast<const f32x4*>(img + r * 256 + ((li ^ (r & 15)) << 4));
-        if (m < M && n < N) *reinterpret_cast<f32x4*>(gr.Yf + (int64_t)m * ldy + n) = v;
-      }
-    } else {
-      const int j = lane & 7, n = c0 + 8 * j, nmax = GLU ? N / 2 : N;
-      float bl[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (!GLU && bias && n < nmax) {
+    const int j = lane & 7, n = c0 + 8 * j;
+    float bl[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (bias && n < N) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) bl[i] = bf2f(bias[n + i]);
-      }
-      auto row = [&](int i, float (&v)[8]) {
-        const int r = 8 * i + (lane >> 3);
+      for (int i = 0; i < 8; ++i) bl[i] = bf2f(bias[n + i]);
+    }
+    auto some = [&](auto kind) {
+#pragma unroll 2
+      for (int i = 0; i < 16; ++i) {
+        const int r = 8 * i + (lane >> 3), m = m0 + wr * 128 + r;
         const f32x4 lo = *reinterpret_cast<const f32x4*>(img + r * 256 + (((2 * j) ^ (r & 15)) << 4));
         const f32x4 hi = *reinterpret_cast<const f32x4*>(img + r * 256 + (((2 * j + 1) ^ (r & 15)) << 4));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v[e] = lo[e] + bl[e];
-          v[4 + e] = hi[e] + bl[4 + e];
-        }
-      };
-      auto out = [&](int i, const float (&v)[8]) {
-        const int m = m0 + wr * 128 + 8 * i + (lane >> 3);
         u16x8 o;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = f2bf(v[e]);
-        if (m < M && n < nmax) __builtin_nontemporal_store(o, reinterpret_cast<u16x8*>(Y + (int64_t)m * ldy + n));
-      };
-      auto some = [&](auto kind) {
-#pragma unroll 2
-        for (int i = 0; i < 16; ++i) {
-          float v[8];
-          row(i, v);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = apply_act(v[e], kind());
-          out(i, v);
+        for (int e = 0; e < 4; ++e) {
+          o[e] = f2bf(apply_act(lo[e] + bl[e], kind()));
+          o[4 + e] = f2bf(apply_act(hi[e] + bl[4 + e], kind()));
         }
-      };
-      // (a loop for each function: with the choice inside, the unrolled code does not fit the instruction cache)
-      if (GLU || act == ACT_NONE) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          float v[8];
-          row(i, v);
-          out(i, v);
-        }
-      } else if (act == ACT_GELU_TANH) {
-        some(std::integral_constant<int, ACT_GELU_TANH>());
-      } else if (act == ACT_GELU) {
-        some(std::integral_constant<int, ACT_GELU>());
-      } else if (act == ACT_RELU) {
-        some(std::integral_constant<int, ACT_RELU>());
-      } else {
-        some(std::integral_constant<int, ACT_RELU2>());
+        if (m < M && n < N) __builtin_nontemporal_store(o, reinterpret_cast<u16x8*>(Y + (int64_t)m * ldy + n));
       }
-    }
+    };
+    // (a loop for each function: with the choice inside, the unrolled code does not fit the instruction cache)
+    if (act == ACT_GELU_TANH) some(std::integral_constant<int, ACT_GELU_TANH>());
+    else if (act == ACT_GELU) some(std::integral_constant<int, ACT_GELU>());
+    else if (act == ACT_RELU) some(std::integral_constant<int, ACT_RELU>());
+    else some(std::integral_constant<int, ACT_RELU2>());
   };
-  float sw[8];
-  if constexpr (GRP == 3) {
-#pragma unroll
-    for (int mt = 0; mt < 8; ++mt) sw[mt] = gr.pw ? gr.pw[gr.order[min(m0 + wr * 128 + 16 * mt + li, M - 1)]] : 1.f;
-  }
   auto put = [&](int p, const f32x4 (&lo)[8], const f32x4 (&hi)[8]) {
-    if constexpr (GLU) {
-      const int n = n0 + wc * 128 + 32 * p + 4 * g;
-      float bg[4], bu[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        bg[i] = bias && n < N ? bf2f(bias[n + i]) : 0.f;
-        bu[i] = bias && n < N ? bf2f(bias[n + 16 + i]) : 0.f;
-      }
-#pragma unroll
-      for (int mt = 0; mt < 8; ++mt) {
-        f32x4 v;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if constexpr (GRP == 3) v[i] = glu_clamped_t(lo[mt][i] * sw[mt], hi[mt][i] * sw[mt], gr.limit, gr.alpha, gr.silu);
-          else v[i] = (GLU == 2 ? gelu_gate(lo[mt][i] + bg[i]) : silu(lo[mt][i] + bg[i])) * (hi[mt][i] + bu[i]);
-        }
-        *reinterpret_cast<f32x4*>(img + (16 * mt + li) * 256 + (((4 * p + g) ^ li) << 4)) = v;
-      }
-    } else {
-#pragma unroll
-      for (int mt = 0; mt < 8; ++mt) {
-        char* row = img + (16 * mt + li) * 256;
-        const int c = 8 * (p & 1) + 2 * g;
-        *reinterpret_cast<f32x4*>(row + ((c ^ li) << 4)) = lo[mt];
-        *reinterpret_cast<f32x4*>(row + (((c + 1) ^ li) << 4)) = hi[mt];
-      }
+    for (int mt = 0; mt < 8; ++mt) {
+      char* row = img + (16 * mt + li) * 256;
+      const int c = 8 * (p & 1) + 2 * g;
+      *reinterpret_cast<f32x4*>(row + ((c ^ li) << 4)) = lo[mt];
+      *reinterpret_cast<f32x4*>(row + (((c + 1) ^ li) << 4)) = hi[mt];
     }
   };
   // the image passes numbers between the lanes of this wave: its writes before the reads, and those before the next writes
@@ -355,35 +434,40 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
   };
   put(0, acc[0], acc[1]);
   put(1, acc[2], acc[3]);
-  if constexpr (!GLU) {
-    turn();
-    flush(n0 + wc * 128);
-    turn();
-  }
+  turn();
+  flush(n0 + wc * 128);
+  turn();
   put(2, acc[4], acc[5]);
   put(3, acc[6], acc[7]);
   turn();
-  flush(GLU ? n0 / 2 + wc * 64 : n0 + wc * 128 + 64);
+  flush(n0 + wc * 128 + 64);
 }
 
 // rows: of X that one descriptor covers; es: bytes of an output element
 bool gemm_quad_ok(int N, int K, int64_t ldx, int64_t ldw, int64_t rows, const void* Y, int64_t ldy, int es, bool glu) {
   return K % 64 == 0 && K >= 64 && (uint64_t)rows * (uint64_t)ldx * 2 < (1ull << 31) && (uint64_t)256 * (uint64_t)ldw * 2 < (1ull << 31) &&
-         ldx % 8 == 0 && ldw % 8 == 0 && N % (glu ? 32 : 8) == 0 && ((uintptr_t)Y & 15) == 0 && ldy * es % 16 == 0;
+         ldx % 8 == 0 && ldw % 8 == 0 && N % (glu ? 32 : 8) == 0 && ((uintptr_t)Y & 15) == 0 && ldy * es % 16 == 0 &&
+         (uint64_t)128 * (uint64_t)ldy * es < (1ull << 31);
 }
 
 void launch_gemm_quad(int grp, const bf16_t* X, int64_t ldx, const bf16_t* W, int64_t ldw, const bf16_t* bias, bf16_t* Y,
                       int64_t ldy, int M, int N, int K, int act, int glu, int group_m, unsigned nwg, const PpGroup& gr,
                       hipStream_t st, const QkvEpi* qe) {
-#define LAUNCH_Q(G_, U_) gemm_quad_kernel<G_, U_><<<nwg, 256, 0, st>>>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, act, group_m, gr, QkvEpi{})
-  if (qe) gemm_quad_kernel<0, 0, true><<<nwg, 256, 0, st>>>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, act, group_m, gr, *qe);
-  else if (grp == 2) LAUNCH_Q(2, 0);
-  else if (grp == 3) LAUNCH_Q(3, 1);
-  else if (grp == 1 && glu) LAUNCH_Q(1, 1);
-  else if (grp == 1) LAUNCH_Q(1, 0);
-  else if (glu && act == ACT_GELU_TANH) LAUNCH_Q(0, 2);
-  else if (glu) LAUNCH_Q(0, 1);
-  else LAUNCH_Q(0, 0);
+  // a workgroup per CU, each taking every 256th tile; rings of fewer than four steps do not reach into another tile
+  const unsigned ring = K >= 256 ? std::min(nwg, 256u) : nwg;
+  const bool lds = qe || (!glu && grp != 2 && act != ACT_NONE);
+#define LAUNCH_Q(G_, U_, Q_, R_) \
+  gemm_quad_kernel<G_, U_, Q_, R_><<<R_ ? ring : nwg, 256, 0, st>>>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, act, group_m, gr, qe ? *qe : QkvEpi{})
+  if (qe) LAUNCH_Q(0, 0, true, false);
+  else if (grp == 2) LAUNCH_Q(2, 0, false, true);
+  else if (grp == 3) LAUNCH_Q(3, 1, false, true);
+  else if (grp == 1 && glu) LAUNCH_Q(1, 1, false, true);
+  else if (grp == 1 && lds) LAUNCH_Q(1, 0, false, false);
+  else if (grp == 1) LAUNCH_Q(1, 0, false, true);
+  else if (glu && act == ACT_GELU_TANH) LAUNCH_Q(0, 2, false, true);
+  else if (glu) LAUNCH_Q(0, 1, false, true);
+  else if (lds) LAUNCH_Q(0, 0, false, false);
+  else LAUNCH_Q(0, 0, false, true);
 #undef LAUNCH_Q
   HIP_CHECK_LAUNCH();
 }
