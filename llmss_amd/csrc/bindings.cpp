@@ -122,7 +122,7 @@ bool moe_router_mfma_ok(int E, int gate, int K);
 void launch_moe_router_mfma(const void* h, int64_t ldh, const void* wr, const void* corr, void* idx, void* wts, int T_,
                             int E, int K, int top, int norm, int smax, const void* zb, void* sg, hipStream_t st);
 void launch_moe_group(const void* idx, int P, int E, int maxt, void* meta, void* order, void* place, int tile_rows,
-                      int blocks, hipStream_t st);
+                      int blocks, int tall, hipStream_t st);
 void launch_moe_gate_up(const void* h, int64_t ldh, const void* wg, const void* wu, const void* meta,
                         const void* order, void* act, int E, int maxt, int top, int F, int K, float limit,
                         float alpha, int dt, const void* pw, int silu, hipStream_t st);
@@ -517,7 +517,11 @@ PYBIND11_MODULE(_C, m) {
   });
   m.def("moe_group", [](uintptr_t idx, int Pn, int E, int maxt, uintptr_t meta, uintptr_t order, uintptr_t place,
                         int tile_rows, int blocks, uintptr_t st) {
-    launch_moe_group(CP(idx), Pn, E, maxt, P(meta), P(order), P(place), tile_rows, blocks, S(st));
+    launch_moe_group(CP(idx), Pn, E, maxt, P(meta), P(order), P(place), tile_rows, blocks, 0, S(st));
+  });
+  m.def("moe_group_tall", [](uintptr_t idx, int Pn, int E, int maxt, uintptr_t meta, uintptr_t order, uintptr_t place,
+                             int tile_rows, int blocks, uintptr_t st) {
+    launch_moe_group(CP(idx), Pn, E, maxt, P(meta), P(order), P(place), tile_rows, blocks, 1, S(st));
   });
   m.def("moe_gate_up", [](uintptr_t h, int64_t ldh, uintptr_t wg, uintptr_t wu, uintptr_t meta, uintptr_t order,
                           uintptr_t act, int E, int maxt, int top, int F, int K, float limit, float alpha, int dt,

@@ -28,19 +28,23 @@
 #include <algorithm>
 #include <type_traits>
 
-// The wave's 128 x 128 part of a finished tile, straight from the accumulators. A lane holds, of row 16 mt + li, sixteen bytes of neighbouring
+// The wave's 128 x 128 part of a finished tile (GRP: every other sixteen rows from m0 on; half: four of them), straight from the accumulators.
+// A lane holds, of row MS mt + li, sixteen bytes of neighbouring
 // columns (two tiles of eight: GLU, four gates and their four ups twice; fp32: one tile of four) - 64 bytes a row and instruction, and stores of
 // half lines take four times as long. So two such pieces change hands between lanes li and li ^ 8 (a rotation by eight within the row of
 // sixteen lanes): one instruction then writes rows 0 .. 7 of the sixteen in whole lines, another rows 8 .. 15.
-// Rows and columns past the last lie outside the descriptor, so that no branch stands between the stores.
-template <int GRP, int GLU>
+// Rows and columns past the last lie outside the descriptor, so that no branch stands between the stores. (A row's pitch is under 2^24 bytes,
+// gemm_quad_ok, so that 256 of them fit the offsets.)
+// All go past the caches: fp32 sums of 32768 pairs x 2048 (K = 768) 152 -> 131 us, which no cache would hold until they are read.
+template <int GRP, int GLU, int MS>
 __device__ __forceinline__ void quad_store(const f32x4 (&acc)[8][8], const PpGroup& gr, const bf16_t* __restrict__ bias, bf16_t* __restrict__ Y,
-                                           int64_t ldy, int m0, int n0, int M, int N, int li, int g, const float (&sw)[8]) {
+                                           int64_t ldy, int m0, int n0, int M, int N, int li, int g, const float (&sw)[8], bool half) {
   constexpr int ES = GRP == 2 ? 4 : 2, COLS = GRP == 2 ? 4 : GLU ? 1 : 2, RUN = GRP == 2 ? 32 : 64;  // runs of a line
   const int nout = GLU ? N / 2 : N, o0 = GLU ? n0 / 2 : n0, up = li >> 3;
   const uint32_t pitch = (uint32_t)ldy * ES;
+  const GluForm glu(gr.limit, gr.alpha, gr.silu);
   const auto ry = uniform_rsrc((GRP == 2 ? reinterpret_cast<char*>(gr.Yf) : reinterpret_cast<char*>(Y)) + (int64_t)m0 * ldy * ES,
-                               (int64_t)max(min(M - m0, 128), 0) * pitch);
+                               (int64_t)max(min(M - m0, 7 * MS + 16), 0) * pitch);
 #pragma unroll
   for (int c = 0; c < COLS; ++c) {
     float bs[2][GLU ? 16 : 8] = {};
@@ -56,9 +60,10 @@ __device__ __forceinline__ void quad_store(const f32x4 (&acc)[8][8], const PpGro
         }
     }
     const int n = o0 + RUN * c + RUN / 2 * up + RUN / 8 * g;
-    const uint32_t at = (uint32_t)(li & 7) * pitch + (uint32_t)n * ES + (n < nout ? 0u : 0x80000000u);
+    const uint32_t at = (uint32_t)(li & 7) * pitch + (uint32_t)n * ES;
 #pragma unroll
     for (int mt = 0; mt < 8; ++mt) {
+      if (GRP != 0 && mt == 4 && half) break;
       u32x4 a, b;
       if constexpr (GRP == 2) {
         a = __builtin_bit_cast(u32x4, acc[2 * c][mt]), b = __builtin_bit_cast(u32x4, acc[2 * c + 1][mt]);
@@ -71,8 +76,8 @@ __device__ __forceinline__ void quad_store(const f32x4 (&acc)[8][8], const PpGro
             if constexpr (GLU) {
               const int t = 4 * h + 2 * (i >> 2);
               const float gv = acc[t][mt][i & 3], uv = acc[t + 1][mt][i & 3];
-              if constexpr (GRP == 3) o[h][i] = f2bf(glu_clamped_t(gv * sw[mt], uv * sw[mt], gr.limit, gr.alpha, gr.silu));
-              else o[h][i] = f2bf((GLU == 2 ? gelu_gate(gv + bs[h][i]) : silu(gv + bs[h][i])) * (uv + bs[h][8 + i]));
+              if constexpr (GRP == 3) o[h][i] = f2bf(glu(gv * sw[mt], uv * sw[mt]));
+              else o[h][i] = f2bf((GLU == 2 ? gelu_gate_by(gv + bs[h][i]) : silu_gate_by(gv + bs[h][i])) * (uv + bs[h][8 + i]));
             } else {
               o[h][i] = f2bf(acc[4 * c + 2 * h + (i >> 2)][mt][i & 3] + bs[h][i]);
             }
@@ -85,8 +90,9 @@ __device__ __forceinline__ void quad_store(const f32x4 (&acc)[8][8], const PpGro
         a[i] = __builtin_amdgcn_update_dpp(x, y, 0x128, 0xf, 0xc, false);  // lanes 8 .. 15: of b, from li - 8
         b[i] = __builtin_amdgcn_update_dpp(y, x, 0x128, 0xf, 0x3, false);  // lanes 0 .. 7: of a, from li + 8
       }
-      __builtin_amdgcn_raw_buffer_store_b128(a, ry, at + (uint32_t)(16 * mt) * pitch, 0, GRP == 2 ? 0 : 2);
-      __builtin_amdgcn_raw_buffer_store_b128(b, ry, at + (uint32_t)(16 * mt + 8) * pitch, 0, GRP == 2 ? 0 : 2);
+      const uint32_t ra = n < nout ? at + (uint32_t)(MS * mt) * pitch : ~0u, rb = n < nout ? at + (uint32_t)(MS * mt + 8) * pitch : ~0u;
+      __builtin_amdgcn_raw_buffer_store_b128(a, ry, ra, 0, 2);
+      __builtin_amdgcn_raw_buffer_store_b128(b, ry, rb, 0, 2);
     }
   }
 }
@@ -107,7 +113,7 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
   static_assert(!QKV || (GRP == 0 && GLU == 0), "QKV: plain products");
   // a ring of five buffers, each 64 of k (128 bytes, a line) of 256 rows: X of step 0, W of step 0, X of step 1, ...
   constexpr int BUF = 32768, NB = 5, QA = 6;
-  constexpr bool GATHER = GRP == 1 || GRP == 3;
+  constexpr bool GATHER = GRP == 1 || GRP == 3, HALF = RING && GRP != 0;
   __shared__ __attribute__((aligned(16))) char smem[NB * BUF];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -118,26 +124,41 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
   if ((int)blockIdx.x >= tiles) return;
   const int nk = K >> 6;
   if (GRP == 3 && (w & 2)) W = gr.Wu;
-  // tile b: its first row and column, the rows that there are, and where its operands lie (bytes that exist from there on)
+  // Expert lists: first the tiles of more than 128 rows, tall of them, round by round, then the half tiles, whose upper products are left out.
+  // Workgroups that have one round less begin with those, two each, before the others get any. 32 experts of 2048 x 768, us: 1024 pairs each by
+  // chance, a rest of some rows for every other, first product 228 -> 201 (170 without rests: half tiles read weights that have left the caches,
+  // a step a microsecond), second 156 -> 130; 320 each 110 -> 91 and 55 -> 57; 16 of 1024 x 512 by about 900, 68 -> 45 and 43 -> 31.
+  const int G = gridDim.x, tall = HALF ? __builtin_amdgcn_readfirstlane(gr.meta[2 + gr.E + 2 * gr.maxt]) * ntn : tiles;
+  const int over = tall % G;  // workgroups that have a round more
+  const int rounds = tall / G + ((int)blockIdx.x < over);
+  // number i of this workgroup's tiles, or -1
+  auto tile_no = [&](int i) {
+    const int b = (int)blockIdx.x;
+    if (!RING) return i ? -1 : xcd_remap(b, tiles);
+    if (i < rounds) return xcd_remap(b + i * G, tall);
+    const int k = i - rounds, early = b >= over ? 2 : 0;
+    const int t = tall + (k < early ? b - over + k * (G - over) : 2 * (G - over) + b + (k - early) * G);
+    return t < tiles ? t : -1;
+  };
+  // tile id: its first row and column, the rows that there are, and where its operands lie (bytes that exist from there on)
   struct Tile {
     int m0, n0, M;
     const char *x, *w;
     uint32_t xb, wb;
   };
-  auto place = [&](int b) {
+  auto place = [&](int id) {
     Tile t;
     const bf16_t* wt = W;
     t.M = M;
     if constexpr (GRP != 0) {
-      const int id = xcd_remap(b, tiles), ty = id / ntn;
+      const int ty = id / ntn;
       const int e = __builtin_amdgcn_readfirstlane(gr.meta[1 + (gr.E + 1) + ty]);
       t.n0 = (id - ty * ntn) * 256;
       t.m0 = __builtin_amdgcn_readfirstlane(gr.meta[1 + (gr.E + 1) + gr.maxt + ty]);
       t.M = __builtin_amdgcn_readfirstlane(gr.meta[1 + e + 1]);
       wt += (int64_t)e * gr.sB;
     } else {
-      const int tile = xcd_remap(b, tiles);
-      const int grp = tile / (group_m * ntn), gidx = tile - grp * (group_m * ntn);
+      const int grp = id / (group_m * ntn), gidx = id - grp * (group_m * ntn);
       const int gm = min(group_m, ntm - grp * group_m);
       t.m0 = (grp * group_m + gidx % gm) * 256, t.n0 = (gidx / gm) * 256;
     }
@@ -150,10 +171,12 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
     t.wb = wb > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)wb;
     return t;
   };
-  int blk = blockIdx.x;
-  Tile cur = place(blk), next = cur;
+  int at = 0, ahead = RING ? tile_no(1) : -1;
+  const int first = tile_no(0);
+  if (first < 0) return;
+  Tile cur = place(first), next = cur;
   if constexpr (RING) {
-    if (blk + (int)gridDim.x < tiles) next = place(blk + gridDim.x);
+    if (ahead >= 0) next = place(ahead);
     else next.xb = next.wb = 0;  // (nothing is in its range)
   }
   // chunk c of row r lies at place c ^ key(r) of the row: the eight rows that a fragment read's eight lanes take fall on eight
@@ -169,7 +192,7 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
     const int row = (i * 4 + w) * 8 + (lane >> 3);
     return (uint32_t)(GATHER ? pair / gr.top : row) * (uint32_t)(ldx * 2) + (uint32_t)(((lane & 7) ^ xkey(row)) << 4);
   };
-  auto weight_of = [&](const Tile& t, int mt) { return gr.pw ? gr.pw[gr.order[min(t.m0 + wr * 128 + 16 * mt + li, t.M - 1)]] : 1.f; };
+  auto weight_of = [&](const Tile& t, int mt) { return gr.pw ? gr.pw[gr.order[min(t.m0 + 32 * mt + 16 * wr + li, t.M - 1)]] : 1.f; };
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int row = (i * 4 + w) * 8 + (lane >> 3);
@@ -183,9 +206,11 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
 #define Q_LOAD(R_, V_, I_, T_, B_)                                                                                    \
   __builtin_amdgcn_raw_ptr_buffer_load_lds(R_, (LDS_AS void*)(smem + (B_) + ((I_) * 4 + w) * 1024), 16, (uint32_t)(V_), (uint32_t)((T_) * 128), 0, 0)
   const int wrow = PLAIN ? li : (GLU ? 32 * (li >> 3) + 8 * ((li >> 2) & 1) + (li & 3) : 8 * (li >> 2) + (li & 3));
-  const int xo = (wr * 128 + li) * 128 + ((g ^ xkey(li)) << 4);
+  // (HALF: the waves' rows alternate by sixteens, so that a tile of up to 128 rows is the first half of both waves' products)
+  constexpr int XT = HALF ? 4096 : 2048;
+  const int xo = (wr * (HALF ? 16 : 128) + li) * 128 + ((g ^ xkey(li)) << 4);
   const int wo = (wc * 128 + wrow) * 128 + ((g ^ wkey(wrow)) << 4);
-#define Q_X(P_, T_) (*reinterpret_cast<const s16x8*>(smem + (P_) + (T_) * 2048))
+#define Q_X(P_, T_) (*reinterpret_cast<const s16x8*>(smem + (P_) + (T_) * XT))
 #define Q_W(P_, T_)                                \
   (*reinterpret_cast<const s16x8*>(smem + (P_) + (PLAIN ? (T_) * 2048                                                        \
                                                   : GLU ? ((T_) >> 2) * 8192 + (((T_) >> 1) & 1) * 512 + ((T_) & 1) * 2048  \
@@ -204,6 +229,30 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
       asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[NT_][MT_]) : "v"(W_[NT_]), "v"(X_[MT_]));                  \
     else                                                                                                                  \
       asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[NT_][MT_]) : "v"(W_[NT_]), "v"(X_[MT_]));                  \
+  } while (0)
+  // The products of W tiles NT_ and NT_ + 1 with X tiles 4 .. 7, which half tiles pass over. The branch stands inside, for the compiler moves and
+  // spills accumulators around one that it sees; one for eight products costs whole tiles 2 % (one for four 4 %).
+#define Q_UPPER8(C_, W_, X_, NT_)                                                                                         \
+  asm("s_cmp_lg_u32 %14, 0\n\ts_cbranch_scc0 1f\n\t"                                                                    \
+      "v_mfma_f32_16x16x32_bf16 %0, %8, %10, %0\n\tv_mfma_f32_16x16x32_bf16 %1, %8, %11, %1\n\t"                        \
+      "v_mfma_f32_16x16x32_bf16 %2, %8, %12, %2\n\tv_mfma_f32_16x16x32_bf16 %3, %8, %13, %3\n\t"                        \
+      "v_mfma_f32_16x16x32_bf16 %4, %9, %10, %4\n\tv_mfma_f32_16x16x32_bf16 %5, %9, %11, %5\n\t"                        \
+      "v_mfma_f32_16x16x32_bf16 %6, %9, %12, %6\n\tv_mfma_f32_16x16x32_bf16 %7, %9, %13, %7\n1:"                        \
+      : "+" C_(acc[NT_][4]), "+" C_(acc[NT_][5]), "+" C_(acc[NT_][6]), "+" C_(acc[NT_][7]), "+" C_(acc[NT_ + 1][4]),      \
+        "+" C_(acc[NT_ + 1][5]), "+" C_(acc[NT_ + 1][6]), "+" C_(acc[NT_ + 1][7])                                         \
+      : "v"(W_[NT_]), "v"(W_[NT_ + 1]), "v"(X_[4]), "v"(X_[5]), "v"(X_[6]), "v"(X_[7]), "s"(full)                         \
+      : "scc")
+  // A step's 64 products over its 16 places, four each (HALF: tiles 4 .. 7 of two W tiles in every fourth place).
+#define Q_FOUR(W_, X_, Q_)                                                                                    \
+  do {                                                                                                        \
+    const int nt = (Q_) >> 1;                                                                                 \
+    if (HALF && ((Q_) & 3) == 3) {                                                                            \
+      if (nt < QA) Q_UPPER8("a", W_, X_, nt - 1);                                                             \
+      else Q_UPPER8("v", W_, X_, nt - 1);                                                                     \
+    } else if (!HALF || ((Q_) & 3) != 2) {                                                                    \
+      const int n1 = HALF ? nt + ((Q_) & 1) : nt, m1 = HALF ? 0 : ((Q_) & 1) * 4;                             \
+      _Pragma("unroll") for (int e = 0; e < 4; ++e) Q_MFMA(W_, X_, n1, m1 + e);                               \
+    }                                                                                                         \
   } while (0)
   {
     const auto rx = Q_RSRC(cur.x, cur.xb), rw = Q_RSRC(cur.w, cur.wb);
@@ -230,6 +279,9 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
   for (;;) {
     // One copy of the body: with separate last steps the compiler moves every accumulator between register files. The last steps load the
     // next tile's first ones (RING; or the last one again), and the very last reads its fragments (or some that nobody uses).
+    // (the builtin is taken out as one of a uniform value, which then lies in a vector register)
+    int full = 1;
+    if constexpr (HALF) asm("s_nop 4\n\tv_readfirstlane_b32 %0, %1\n\ts_nop 4" : "=s"(full) : "v"((int)(cur.M - cur.m0 > 128)));
 #pragma unroll 1
     for (int t = 0; t < nk; ++t) {
       const int cw = cx == 4 * BUF ? 0 : cx + BUF;
@@ -245,8 +297,7 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
           w1[q] = Q_W(wa, q);
           x1[q] = Q_X(xa, q);
         }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) Q_MFMA(w0, x0, q >> 1, (q & 1) * 4 + e);
+        Q_FOUR(w0, x0, q);
         __builtin_amdgcn_sched_barrier(0);
       }
       __builtin_amdgcn_s_waitcnt(0x0078);  // vmcnt(8) lgkmcnt(0): this step is read, this wave's part of the next has landed
@@ -261,8 +312,7 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
         } else {
           Q_LOAD(rx, RING && GATHER && xn ? vn[q - 8] : vx[q - 8], q - 8, tx, cw);
         }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) Q_MFMA(w1, x1, q >> 1, (q & 1) * 4 + e);
+        Q_FOUR(w1, x1, q);
         __builtin_amdgcn_sched_barrier(0);
       }
       cx = nx;
@@ -274,7 +324,8 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
     } else {
       // (what the tile after the next needs of the lists is asked for before the stores, behind which it would wait)
       Tile then = next;
-      if (blk + 2 * (int)gridDim.x < tiles) then = place(blk + 2 * gridDim.x);
+      const int after = ahead < 0 ? -1 : tile_no(++at + 1);
+      if (after >= 0) then = place(after);
       else then.xb = then.wb = 0;
       int pairs[8];
       float sw[8];
@@ -284,9 +335,9 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
         if constexpr (GRP == 3) sw[i] = weight_of(cur, i);
       }
       __builtin_amdgcn_sched_barrier(0);
-      quad_store<GRP, GLU>(acc, gr, bias, Y, ldy, cur.m0 + wr * 128, cur.n0 + wc * 128, cur.M, N, li, g, sw);
-      blk += gridDim.x;
-      if (blk >= tiles) break;
+      quad_store<GRP, GLU, HALF ? 32 : 16>(acc, gr, bias, Y, ldy, cur.m0 + (HALF ? 16 : 128) * wr, cur.n0 + wc * 128, cur.M, N, li, g, sw, !full);
+      if (ahead < 0) break;
+      ahead = after;
       cur = next, next = then;
       if constexpr (GATHER) {
 #pragma unroll
@@ -301,6 +352,8 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
     }
   }
 #undef Q_MFMA
+#undef Q_FOUR
+#undef Q_UPPER8
 #undef Q_X
 #undef Q_W
 #undef Q_LOAD

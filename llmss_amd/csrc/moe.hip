@@ -480,15 +480,16 @@ void launch_moe_router_mfma(const void* h, int64_t ldh, const void* wr, const vo
 // ------------------------------------------------------------------------------------------------ grouping
 // meta = [ntiles | off[E + 1] | tile_expert[maxt] | tile_row0[maxt]], order [P], place [P].
 // One wave turns the experts' counts into their first rows (off, and `cur` in LDS for the caller's own use) and the list of tiles: a lane an
-// expert, sums over the lanes. meta null: only `cur`.
-__device__ __forceinline__ void group_scan(const int* cnt, int* cur, int E, int maxt, int tile_rows, int* meta) {
+// expert, sums over the lanes. meta null: only `cur`. tall: the list in two parts, first the tiles of more than half of their rows, whose number
+// lies behind the list, then the others (gemm_quad.hip).
+__device__ __forceinline__ void group_scan(const int* cnt, int* cur, int E, int maxt, int tile_rows, int* meta, int tall) {
   const int lane = threadIdx.x & 63;
   int* off = meta + 1;
   int* tile_e = meta + 1 + (E + 1);
   int* tile_r = tile_e + maxt;
   int o = 0, nt = 0;
   for (int e0 = 0; e0 < E; e0 += 64) {
-    const int e = e0 + lane, c = e < E ? cnt[e] : 0, t = (c + tile_rows - 1) / tile_rows;
+    const int e = e0 + lane, c = e < E ? cnt[e] : 0, t = (c + (tall ? tile_rows - tile_rows / 2 : tile_rows) - 1) / tile_rows;
     int so = c, st = t;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -510,6 +511,19 @@ __device__ __forceinline__ void group_scan(const int* cnt, int* cur, int E, int 
     o += __shfl(so, 63, 64);
     nt += __shfl(st, 63, 64);
   }
+  if (tall && meta) {
+    if (lane == 0) meta[2 + E + 2 * (int64_t)maxt] = nt < maxt ? nt : maxt;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane, c = e < E ? cnt[e] : 0, rest = c % tile_rows;
+      const uint64_t some = __ballot(rest > 0 && 2 * rest <= tile_rows);
+      const int at = nt + __popcll(some & ((1ull << lane) - 1));
+      if ((some >> lane & 1) && at < maxt) {
+        tile_e[at] = e;
+        tile_r[at] = off[e] + c - rest;
+      }
+      nt += __popcll(some);
+    }
+  }
   if (meta && lane == 0) {
     off[E] = o;
     meta[0] = nt < maxt ? nt : maxt;
@@ -520,7 +534,7 @@ __device__ __forceinline__ void group_scan(const int* cnt, int* cur, int E, int 
 // expert after the other, and the pairs read twice: 132 pairs of 32 experts 6.3 us, 2.7 here.)
 __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__ idx, int P, int E, int maxt,
                                                          int* __restrict__ meta, int* __restrict__ order,
-                                                         int* __restrict__ place, int tile_rows) {
+                                                         int* __restrict__ place, int tile_rows, int tall) {
   extern __shared__ int sm[];  // cnt[E], cur[E]
   int* cnt = sm;
   int* cur = sm + E;
@@ -539,7 +553,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
       if (e[u] < E) atomicAdd(&cnt[e[u]], 1);
   }
   __syncthreads();
-  if (threadIdx.x < 64) group_scan(cnt, cur, E, maxt, tile_rows, meta);
+  if (threadIdx.x < 64) group_scan(cnt, cur, E, maxt, tile_rows, meta, tall);
   __syncthreads();
   // rows within an expert take whatever order the atomics give: every pair's row is computed on its own, so the
   // values do not depend on where the row lands
@@ -581,7 +595,7 @@ __global__ __launch_bounds__(1024) void moe_count_kernel(const int* __restrict__
 
 __global__ __launch_bounds__(1024) void moe_place_kernel(const int* __restrict__ idx, int P, int E, int maxt,
                                                          const int* __restrict__ hist, int* __restrict__ meta,
-                                                         int* __restrict__ order, int* __restrict__ place, int tile_rows) {
+                                                         int* __restrict__ order, int* __restrict__ place, int tile_rows, int tall) {
   extern __shared__ int sm[];  // cnt[E], cur[E], before[E]
   int* cnt = sm;
   int* cur = sm + E;
@@ -597,7 +611,7 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(const int* __restrict__
     if (i < own) atomicAdd(&before[i % E], c);
   }
   __syncthreads();
-  if (threadIdx.x < 64) group_scan(cnt, cur, E, maxt, tile_rows, blockIdx.x == 0 ? meta : nullptr);
+  if (threadIdx.x < 64) group_scan(cnt, cur, E, maxt, tile_rows, blockIdx.x == 0 ? meta : nullptr, tall);
   __syncthreads();
   if (p >= P) return;
   int o = -1;
@@ -608,24 +622,25 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(const int* __restrict__
   place[p] = o;
 }
 
-// blocks > 1: workgroups of 1024 pairs, and `meta` has room for blocks * E counts behind its 2 + E + 2 * maxt numbers
+// blocks > 1: workgroups of 1024 pairs, and `meta` has room for blocks * E counts behind its 2 + E + 2 * maxt numbers (tall: one more, the
+// tiles of more than half of their rows, which stand first in the list)
 void launch_moe_group(const void* idx, int P, int E, int maxt, void* meta, void* order, void* place, int tile_rows, int blocks,
-                      hipStream_t st) {
+                      int tall, hipStream_t st) {
   if (P == 0) return;
   if (tile_rows <= 0) throw std::runtime_error("moe_group: tile rows");
   if (E > 4096) throw std::runtime_error("moe_group: more than 4096 experts");
   if (blocks > 1) {
     if (blocks != (P + 1023) / 1024 || (int64_t)blocks * E > 0x7fffffff) throw std::runtime_error("moe_group: workgroups of 1024 pairs");
-    int* hist = (int*)meta + 2 + E + 2 * (int64_t)maxt;
+    int* hist = (int*)meta + 2 + E + 2 * (int64_t)maxt + (tall ? 1 : 0);
     moe_count_kernel<<<blocks, 1024, E * sizeof(int), st>>>((const int*)idx, P, E, hist);
     HIP_CHECK_LAUNCH();
     moe_place_kernel<<<blocks, 1024, 3 * E * sizeof(int), st>>>((const int*)idx, P, E, maxt, hist, (int*)meta, (int*)order,
-                                                                (int*)place, tile_rows);
+                                                                (int*)place, tile_rows, tall);
     HIP_CHECK_LAUNCH();
     return;
   }
   moe_group_kernel<<<1, 1024, 2 * E * sizeof(int), st>>>((const int*)idx, P, E, maxt, (int*)meta, (int*)order,
-                                                          (int*)place, tile_rows);
+                                                          (int*)place, tile_rows, tall);
   HIP_CHECK_LAUNCH();
 }
 

@@ -1226,7 +1226,7 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     dev = h.device
     blocks = -(-P // 1024) if P > MOE_GROUP_PAIRS else 1  # (each leaves its counts behind meta)
     if not own:
-        meta = torch.empty(1 + (E + 1) + 2 * maxt + (blocks * E if blocks > 1 else 0), dtype=torch.int32, device=dev)
+        meta = torch.empty(1 + (E + 1) + 2 * maxt + int(pp) + (blocks * E if blocks > 1 else 0), dtype=torch.int32, device=dev)
         order = torch.empty(P, dtype=torch.int32, device=dev)
     place = torch.empty(P, dtype=torch.int32, device=dev)
     act_ = torch.empty(P, F, dtype=h.dtype, device=dev)
@@ -1237,7 +1237,7 @@ def moe_experts(h, idx, wts, gate, up, down, limit, alpha, shared=None, combine=
     L = lib()
     st = _stream()
     if not own:
-        L.moe_group(idx.data_ptr(), P, E, maxt, meta.data_ptr(), order.data_ptr(), place.data_ptr(), rows, blocks, st)
+        (L.moe_group_tall if pp else L.moe_group)(idx.data_ptr(), P, E, maxt, meta.data_ptr(), order.data_ptr(), place.data_ptr(), rows, blocks, st)
     if own:
         sact = None
         if within:

@@ -66,3 +66,60 @@ def test_many_tiles_of_experts_in_one_matrix(kind):
             want[r] += w[r, j].double()[:, None] * (v @ down[e].double().t())
     # the activations rounded to bf16 once (2^-9 of each, of random sign over F of them), sums in fp32, row by row
     assert ((y.double() - want).norm(dim=1) / want.norm(dim=1)).max().item() < 8e-3
+
+
+# experts with rests of half a tile and less, which come last and by halves: one row, a matrix instruction's sixteen, 127 - 129 and whole tiles; more
+# tiles than CUs in both products, fewer, and only halves
+@pytest.mark.parametrize("counts,F,N", [([1000, 128, 2300, 129, 16, 513, 640], 2048, 3080), ([127, 1, 1536, 17, 256 + 255, 0], 288, 264),
+                                        ([2048, 384 + 1, 256 + 31], 3072, 2048), ([100, 128, 90, 33, 64, 12, 128, 1], 640, 520)])
+@pytest.mark.parametrize("kind", ["two", "interleaved", "gelu"])
+def test_half_tiles_of_experts(counts, F, N, kind, monkeypatch):
+    from llmss_amd.ops import glu_interleave, hip
+    E, W, P = len(counts), 320, sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(P)
+    h = torch.randn(P, W, generator=g, device="cuda").bfloat16()
+    gate, up = ((torch.randn(E, F, W, generator=g, device="cuda") * W ** -0.5).bfloat16() for _ in range(2))
+    down = (torch.randn(E, N, F, generator=g, device="cuda") * F ** -0.5).bfloat16()
+    idx = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])[torch.randperm(P)].int()[:, None].cuda()
+    w = torch.rand(P, 1, generator=g, device="cuda")
+    for name in ("MOE_PP_ROWS", "MOE_PP_ROWS_TWO", "MOE_DEC_ROWS"):
+        monkeypatch.setattr(hip, name, 0)
+    monkeypatch.setattr(hip, "_moe_plan", lambda *a: (256, 0))
+    if kind == "gelu":
+        y = hip.moe_experts(h, idx, w, None, up, down, 0.0, 0.0, act="gelu")
+    elif kind == "two":
+        y = hip.moe_experts(h, idx, w, gate, up, down, 0.0, 0.0, act="silu")
+    else:
+        y = hip.moe_experts(h, idx, w, None, glu_interleave(gate, up, 1).contiguous(), down, 0.0, 0.0, act="silu", interleaved=True)
+    for e in range(E):
+        r = (idx[:, 0] == e).nonzero()[:, 0]
+        if not len(r):
+            continue
+        a, b = (h[r].double() @ m[e].double().t() for m in (gate, up))
+        v = torch.nn.functional.gelu(b) if kind == "gelu" else torch.nn.functional.silu(a) * b
+        want = w[r].double() * (v @ down[e].double().t())
+        # the activations rounded to bf16 once (2^-9 of each, of random sign over F of them), sums in fp32, row by row
+        assert ((y[r].double() - want).norm(dim=1) / want.norm(dim=1)).max().item() < 8e-3
+
+
+@pytest.mark.parametrize("P,blocks", [(700, 1), (9000, 1), (33044, 33)])
+@pytest.mark.parametrize("E,rows", [(1, 256), (64, 256), (130, 64)])
+def test_list_with_its_half_tiles_last(P, blocks, E, rows):
+    from llmss_amd.ops import hip
+    idx = torch.randint(0, E, (P,), generator=torch.Generator().manual_seed(P + E)).int()
+    maxt = -(-P // rows) + min(E, P)
+    meta = torch.full((3 + E + 2 * maxt + blocks * E,), -7, dtype=torch.int32, device="cuda")
+    order, place = (torch.full((P,), -7, dtype=torch.int32, device="cuda") for _ in range(2))
+    d = idx.cuda()
+    hip.lib().moe_group_tall(d.data_ptr(), P, E, maxt, meta.data_ptr(), order.data_ptr(), place.data_ptr(), rows, blocks,
+                             torch.cuda.current_stream().cuda_stream)
+    meta = meta.cpu()
+    off = [0] + torch.bincount(idx.long(), minlength=E).cumsum(0).tolist()
+    assert meta[1:E + 2].tolist() == off
+    tiles = [(e, r, 2 * (off[e + 1] - r) > rows) for e in range(E) for r in range(off[e], off[e + 1], rows)]
+    tiles = [t[:2] for t in tiles if t[2]] + [t[:2] for t in tiles if not t[2]]
+    tall = sum(2 * (off[e + 1] - r) > rows for e, r in tiles)
+    assert meta[0].item() == len(tiles) <= maxt and meta[2 + E + 2 * maxt].item() == tall
+    at = 2 + E
+    assert list(zip(meta[at:at + len(tiles)].tolist(), meta[at + maxt:at + maxt + len(tiles)].tolist())) == tiles
+    assert (order.cpu()[place.cpu().long()] == torch.arange(P)).all()
