@@ -18,6 +18,8 @@
 #include "anytype.h"
 #include "chunk_rows.h"
 
+#include <type_traits>
+
 // ------------------------------------------------------------------------------------------------ single rows
 struct DeltaStepArgs {
   const void* q;  // [T, ldq]: head group's query at q + (h / rep) * dim
@@ -207,6 +209,24 @@ __device__ __forceinline__ void split2(float x, bf16_t& hi, bf16_t& lo) {
   lo = f2bf(x - bf2f(hi));
 }
 
+// A lane's column of the state, rows r0 + 16 kt + i; zeros where there is none. (All loads first.)
+template <int N>
+__device__ __forceinline__ void load_state(f32x4 (&S)[N], bool cont, const float* sp, int r0, int dim, int vdim, int col) {
+#pragma unroll
+  for (int kt = 0; kt < N; ++kt) S[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (!cont) return;
+  const float* const p = sp + min(col, vdim - 1);
+#pragma unroll
+  for (int kt = 0; kt < N; ++kt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[kt][i] = p[(int64_t)min(r0 + 16 * kt + i, dim - 1) * vdim];
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int kt = 0; kt < N; ++kt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[kt][i] = r0 + 16 * kt + i < dim && col < vdim ? S[kt][i] : 0.f;
+}
+
 constexpr int prep_kq_bytes(int kt) {  // K and Q rows, or P (value, remainder) and the fp32 inverse
   return 2 * 64 * (16 * kt + 8) * 2 > 2 * 64 * 72 * 2 + 64 * 68 * 4 ? 2 * 64 * (16 * kt + 8) * 2 : 2 * 64 * 72 * 2 + 64 * 68 * 4;
 }
@@ -281,26 +301,37 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(DeltaChunkArgs A) {
   constexpr int CHK = DKP / 8, NK = C * CHK / 256;
   static_assert((C * CHK) % 256 == 0, "whole 16-byte pieces per thread");
   const u16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  // (all loads first, from the nearest place that is there: behind a condition each was waited for before the next, a memory's latency each)
+  u16x8 rk[NK], rq[NK];
+#pragma unroll
+  for (int j = 0; j < NK; ++j) {
+    const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 8;
+    const int64_t tt = t0 + j0 + min(r, nt - 1), at = (int64_t)gq * dim + (d < dim ? d : 0);
+    rk[j] = *reinterpret_cast<const u16x8*>(A.k + tt * A.ldk + at);
+    rq[j] = *reinterpret_cast<const u16x8*>(A.q + tt * A.ldq + at);
+  }
+  const int64_t tab = (int64_t)(t0 + j0 + min(lane, nt - 1)) * A.ldab + h;
+  const bf16_t ra = A.a[tab], rb = A.b[tab];
+  const float alog = A.A_log[h], dtb = A.dt_bias[h];
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int j = 0; j < NK; ++j) {
     const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 8;
     const bool in = r < nt && d < dim;
-    const int64_t tt = t0 + j0 + r;
-    *reinterpret_cast<u16x8*>(&Ks[r * LDK + d]) = in ? *reinterpret_cast<const u16x8*>(A.k + tt * A.ldk + (int64_t)gq * dim + d) : zero8;
-    *reinterpret_cast<u16x8*>(&Qs[r * LDK + d]) = in ? *reinterpret_cast<const u16x8*>(A.q + tt * A.ldq + (int64_t)gq * dim + d) : zero8;
+    *reinterpret_cast<u16x8*>(&Ks[r * LDK + d]) = in ? rk[j] : zero8;
+    *reinterpret_cast<u16x8*>(&Qs[r * LDK + d]) = in ? rq[j] : zero8;
   }
   if (w == 0) {  // the tokens' decays and write strengths
     const bool in = lane < nt;
-    const int64_t tt = (int64_t)(t0 + j0 + min(lane, nt - 1)) * A.ldab + h;
-    const float z = bf2f(A.a[tt]) + A.dt_bias[h];
-    float F = in ? -expf(A.A_log[h]) * (z > 20.f ? z : log1pf(expf(z))) : 0.f;
+    const float z = bf2f(ra) + dtb;
+    float F = in ? -expf(alog) * (z > 20.f ? z : log1pf(expf(z))) : 0.f;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const float x = __shfl_up(F, o, 64);
       if (lane >= o) F += x;
     }
     bs[lane] = F;
-    be[lane] = in ? 1.0f / (1.0f + expf(-bf2f(A.b[tt]))) : 0.f;
+    be[lane] = in ? 1.0f / (1.0f + expf(-bf2f(rb))) : 0.f;
   }
   __syncthreads();
   {  // norms: four neighbouring lanes per row
@@ -410,39 +441,31 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaChunkArgs A) {
   const bool cont = ctx > qlen;  // continues an earlier portion
   f32x4 S[KT];
   float* sp = A.S + (((int64_t)slot * H + h) * dim) * (int64_t)vdim;
-#pragma unroll
-  for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 16 * kt + 4 * g + i;
-      S[kt][i] = (cont && r < dim && col < vdim) ? sp[(int64_t)r * vdim + col] : 0.f;
-    }
+  load_state(S, cont, sp, 4 * g, dim, vdim, col);
   constexpr int CHK = DKP / 8, NK = C * CHK / 256;
   u16x8 rq[NK], rk[NK], rm[8];
-  bf16_t rv[16];
+  uint32_t rv[16];  // (words: two numbers to a register wait for both)
   f32x4 ra = {0.f, 0.f, 0.f, 0.f};
   const u16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-  auto fetch = [&](int j0) {
+  auto fetch = [&](int j0) {  // (as in delta_chunk32)
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
       const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 8;
-      const bool in = j0 + r < qlen && d < dim;
-      const int64_t tt = t0 + j0 + r;
-      rq[j] = in ? *reinterpret_cast<const u16x8*>(A.q + tt * A.ldq + (int64_t)gq * dim + d) : zero8;
-      rk[j] = in ? *reinterpret_cast<const u16x8*>(A.k + tt * A.ldk + (int64_t)gq * dim + d) : zero8;
+      const int64_t tt = t0 + min(j0 + r, qlen - 1), at = (int64_t)gq * dim + (d < dim ? d : 0);
+      rq[j] = *reinterpret_cast<const u16x8*>(A.q + tt * A.ldq + at);
+      rk[j] = *reinterpret_cast<const u16x8*>(A.k + tt * A.ldk + at);
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int c = tid + 256 * (j & 1), r = c >> 3, s0 = (c & 7) * 8;
-      rm[j] = j0 + r < qlen ? *reinterpret_cast<const u16x8*>(A.X + (j >> 1) * A.mat + ((int64_t)(t0 + j0 + r) * H + h) * 64 + s0)
-                            : zero8;
+      rm[j] = *reinterpret_cast<const u16x8*>(A.X + (j >> 1) * A.mat + ((int64_t)(t0 + min(j0 + r, qlen - 1)) * H + h) * 64 + s0);
     }
 #pragma unroll
     for (int j = 0; j < 16; ++j) {  // token 16 (j / 4) + 4 g + j % 4 at this lane's column
       const int r = j0 + 16 * (j >> 2) + 4 * g + (j & 3);
       rv[j] = A.v[(int64_t)(t0 + min(r, qlen - 1)) * A.ldv + (int64_t)h * vdim + colc];
     }
-    if (w == 0) ra = A.aux[(int64_t)(t0 + min(j0 + lane, qlen - 1)) * H + h];
+    ra = A.aux[(int64_t)(t0 + min(j0 + lane, qlen - 1)) * H + h];
   };
   fetch(0);
   for (int j0 = 0; j0 < qlen; j0 += C) {
@@ -451,18 +474,19 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaChunkArgs A) {
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
       const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 8;
-      *reinterpret_cast<u16x8*>(&Qs[r * LDK + d]) = rq[j];
-      *reinterpret_cast<u16x8*>(&Ks[r * LDK + d]) = rk[j];
+      const bool in = r < nt && d < dim;
+      *reinterpret_cast<u16x8*>(&Qs[r * LDK + d]) = in ? rq[j] : zero8;
+      *reinterpret_cast<u16x8*>(&Ks[r * LDK + d]) = in ? rk[j] : zero8;
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int c = tid + 256 * (j & 1);
-      *reinterpret_cast<u16x8*>(&Ms[(j >> 1) * C * LDP + (c >> 3) * LDP + (c & 7) * 8]) = rm[j];
+      *reinterpret_cast<u16x8*>(&Ms[(j >> 1) * C * LDP + (c >> 3) * LDP + (c & 7) * 8]) = (c >> 3) < nt ? rm[j] : zero8;
     }
     if (w == 0) ax[lane] = ra;
     f32x4 u[4];  // first V, then V - e^b K S_0
 #pragma unroll
-    for (int j = 0; j < 16; ++j) u[j >> 2][j & 3] = bf2f(rv[j]);
+    for (int j = 0; j < 16; ++j) u[j >> 2][j & 3] = bf2f((bf16_t)rv[j]);
     __syncthreads();
     if (j0 + C < qlen) fetch(j0 + C);
     // K S_0 and Q S_0 for this wave's columns
@@ -679,27 +703,24 @@ __device__ __forceinline__ f32x4 dot32(const f32x4* a, const float* bp) {
 }
 // A S: the state's tiles are the second operand as they stand
 template <int KT>
-__device__ __forceinline__ f32x4 dot32s(const float* ap, const f32x4* S) {
+__device__ __forceinline__ f32x4 dot32s(const f32x4 (&x)[KT], const f32x4 (&S)[KT]) {
   constexpr int N = KT < 4 ? 2 : 4;
   f32x4 c[N];
 #pragma unroll
   for (int n = 0; n < N; ++n) c[n] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int kt = 0; kt < KT; kt += N) {
-    f32x4 x[N];
-#pragma unroll
-    for (int n = 0; n < N; ++n) x[n] = ldv4(ap + 16 * (kt + n));
+  for (int kt = 0; kt < KT; kt += N)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int n = 0; n < N; ++n) c[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[n][i], S[kt + n][i], c[n], 0, 0, 0);
-  }
+      for (int n = 0; n < N; ++n) c[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[kt + n][i], S[kt + n][i], c[n], 0, 0, 0);
   return N == 4 ? (c[0] + c[1]) + (c[N - 2] + c[N - 1]) : c[0] + c[1];
 }
 
 // Workgroup (chunk of a portion, head, sequence), 4 waves. TP: storage of a and b. Bound by its chain of stages (rows, sums, products,
 // 64 steps of substitution), so by how many workgroups a CU holds: the queries stay in the registers of the wave whose rows they
-// are, and 54 KB of LDS let three in where keys and queries in LDS (86 KB) left room for one.
+// are, and 54 KB of LDS let three in where keys and queries in LDS (86 KB) left room for one. With all loads before the first use 80 -> 66 us
+// (8 x 1024 tokens, 16 heads of 128), delta_prep 75 -> 60, delta_chunk 133 -> 111 (7 x 1180).
 template <int KT, typename TP>
 __global__ __launch_bounds__(256, 3) void delta_prep32_kernel(DeltaChunk32Args A) {
   constexpr int C = 64, DKP = 16 * KT, LDK = DKP + 4, LDL = 64 + 4;
@@ -718,34 +739,42 @@ __global__ __launch_bounds__(256, 3) void delta_prep32_kernel(DeltaChunk32Args A
   const int nt = min(C, qlen - j0), dim = A.dim, H = A.H, gq = h / (H / A.G);
   constexpr int CHK = DKP / 4, NK = C * CHK / 256;
   static_assert((C * CHK) % 256 == 0, "whole 16-byte pieces per thread");
+  // (all loads first, as in delta_prep)
+  f32x4 rk[NK];
 #pragma unroll
   for (int j = 0; j < NK; ++j) {
     const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 4;
-    const bool in = r < nt && d < dim;
-    const int64_t tt = t0 + j0 + r;
-    *reinterpret_cast<f32x4*>(&Ks[r * LDK + d]) = in ? ldv4(A.k + tt * A.ldk + (int64_t)gq * dim + d) : f32x4{0.f, 0.f, 0.f, 0.f};
+    rk[j] = ldv4(A.k + (int64_t)(t0 + j0 + min(r, nt - 1)) * A.ldk + (int64_t)gq * dim + (d < dim ? d : 0));
   }
+  const int64_t tab = (int64_t)(t0 + j0 + min(lane, nt - 1)) * A.ldab + h;
+  const TP ra = ((const TP*)A.a)[tab], rb = ((const TP*)A.b)[tab];
+  const float alog = A.A_log[h], dtb = A.dt_bias[h];
   f32x4 q[KT];  // row 16 w + li, columns 16 kt + 4 g on
   {
-    const int r = 16 * w + li;
-    const float* qp = A.q + (int64_t)(t0 + j0 + min(r, nt - 1)) * A.ldq + (int64_t)gq * dim;
+    const float* qp = A.q + (int64_t)(t0 + j0 + min(16 * w + li, nt - 1)) * A.ldq + (int64_t)gq * dim;
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
-      q[kt] = r < nt && 16 * kt + 4 * g < dim ? ldv4(qp + 16 * kt + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int kt = 0; kt < KT; ++kt) q[kt] = ldv4(qp + (16 * kt + 4 * g < dim ? 16 * kt + 4 * g : 0));
   }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < NK; ++j) {
+    const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 4;
+    *reinterpret_cast<f32x4*>(&Ks[r * LDK + d]) = r < nt && d < dim ? rk[j] : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) q[kt] = 16 * w + li < nt && 16 * kt + 4 * g < dim ? q[kt] : f32x4{0.f, 0.f, 0.f, 0.f};
   if (w == 0) {  // the tokens' decays and write strengths
     const bool in = lane < nt;
-    const int64_t tt = (int64_t)(t0 + j0 + min(lane, nt - 1)) * A.ldab + h;
-    const float z = El<TP>::ld((const TP*)A.a + tt) + A.dt_bias[h];
+    const float z = El<TP>::ld(&ra) + dtb;
     // (a decay of zero: a sum this low vanishes over a single token, and differences of equal sums stay zero)
-    double F = in ? at_least((double)(-expf(A.A_log[h]) * (z > 20.f ? z : log1pf(expf(z)))), -1e8) : 0.0;
+    double F = in ? at_least((double)(-expf(alog) * (z > 20.f ? z : log1pf(expf(z)))), -1e8) : 0.0;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const double x = __shfl_up(F, o, 64);
       if (lane >= o) F += x;
     }
     bs[lane] = F;
-    be[lane] = in ? 1.0f / (1.0f + expf(-El<TP>::ld((const TP*)A.b + tt))) : 0.f;
+    be[lane] = in ? 1.0f / (1.0f + expf(-El<TP>::ld(&rb))) : 0.f;
   }
   __syncthreads();
   {  // norms: four neighbouring lanes per row
@@ -814,167 +843,252 @@ __global__ __launch_bounds__(256, 3) void delta_prep32_kernel(DeltaChunk32Args A
   }
 }
 
-// Workgroup (head, block of 64 value columns, sequence), 4 waves, the portion's chunks in order; layouts as in delta_chunk: a
-// register of an accumulator tile is the second operand of a 16x16x4 instruction over its rows 4 g + i, and the first operand's
-// matching numbers are four neighbours of a row in LDS. Blocks of 16 tokens past the portion's end are skipped.
-template <int KT>
-__global__ __launch_bounds__(256, KT <= 2 ? 2 : 1) void delta_chunk32_kernel(DeltaChunk32Args A) {
-  constexpr int C = 64, DKP = 16 * KT, LDK = DKP + 4, LDP = 64 + 4;
+// Workgroup (head, block of 64 value columns, sequence), the portion's chunks in order; layouts as in delta_chunk: a register of an
+// accumulator tile is the second operand of a 16x16x4 instruction over its rows 4 g + i, and the first operand's matching numbers are four
+// neighbours of a row in LDS. Blocks of 16 tokens past the portion's end are skipped.
+// Bound by the chain of a chunk's products, reads and barriers: of 14.3 us a chunk the fp32 matrix instructions took 6.2, now of 12.0 (8 x 1024
+// tokens, 16 heads of 128 x 128, 229 -> 192 us). NH = 2 (keys of more than 32): two waves a SIMD, 8 a workgroup; two share 16 columns, each with half of the state's rows (its part of K S and Q S over those; its rows of the update) and
+// two of the four blocks of tokens (0 and 3, 1 and 2: five products each with X and with P). Parts of sums, u and U change hands through LDS.
+template <int KT, int NH>
+__global__ __launch_bounds__(256 * NH, KT <= 2 ? 2 : 1) void delta_chunk32_kernel(DeltaChunk32Args A) {
+  constexpr int C = 64, DKP = 16 * KT, LDK = DKP + 4, LDP = 64 + 4, KO = KT / NH, TH = 256 * NH;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   float* Qs = reinterpret_cast<float*>(smem);
   float* Ks = Qs + C * LDK;
   float* Ms = Ks + C * LDK;                                // [2][64][LDP]: X, P
   f32x4* ax = reinterpret_cast<f32x4*>(Ms + 2 * C * LDP);  // [64]
+  f32x4* ex = ax + C;                                      // [8 waves][2][2][64 lanes] parts of K S and Q S (NH = 2)
+  f32x4* ux = ex + 8 * 4 * 64;                             // [4][4][64] u
+  f32x4* uX = ex;                                          // [4][4][64] U: the parts are read by then
   const int h = blockIdx.x, b = gridDim.z - 1 - blockIdx.z;
   const int dim = A.dim, vdim = A.vdim, H = A.H, gq = h / (H / A.G);
   const int t0 = A.cu[b], qlen = A.cu[b + 1] - t0, slot = A.sslots[b], ctx = A.ctx[b];
   if (qlen <= 0) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3, hf = wave >> 2;
   const int col = blockIdx.y * 64 + 16 * w + li, colc = min(col, vdim - 1);
   float* outp = A.out + (int64_t)t0 * H * vdim + (int64_t)h * vdim + col;
   if (slot < 0 || ctx <= 0) {
-    if (g == 0 && col < vdim)
+    if (g == 0 && col < vdim && hf == 0)
       for (int j = 0; j < qlen; ++j) outp[(int64_t)j * H * vdim] = 0.f;
     return;
   }
   const bool cont = ctx > qlen;  // continues an earlier portion
-  f32x4 S[KT];
+  constexpr int NO = 4 / NH;  // blocks of this wave: 0 and 3, 1 and 2
+  auto own = [&](int rt) { return NH == 1 || hf == ((rt ^ (rt >> 1)) & 1); };
+  auto block = [&](int n) { return NH == 1 ? n : n ? 3 - hf : hf; };
+  const int k0w = NH == 1 ? 0 : 16 * KO * hf;                                   // first of this wave's rows of the state
+  f32x4 S[KO];
   float* sp = A.S + (((int64_t)slot * H + h) * dim) * (int64_t)vdim;
-#pragma unroll
-  for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 16 * kt + 4 * g + i;
-      S[kt][i] = (cont && r < dim && col < vdim) ? sp[(int64_t)r * vdim + col] : 0.f;
-    }
-  constexpr int CHK = DKP / 4, NK = C * CHK / 256;
-  f32x4 rq[NK], rk[NK], rm[8];
-  float rv[16];
+  load_state(S, cont, sp, k0w + 4 * g, dim, vdim, col);
+  constexpr int CHK = DKP / 4, NK = C * CHK / TH, NM = 8 / NH;
+  f32x4 rq[NK], rk[NK], rm[NM];
+  f32x4 rv[NO];
   f32x4 ra = {0.f, 0.f, 0.f, 0.f};
   const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+  // (the portion's last row again and again past its end, a row's first piece past its last; what is not there becomes zero where it is
+  // staged: a zero put in here waits for the load)
   auto fetch = [&](int j0) {
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
-      const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 4;
-      const bool in = j0 + r < qlen && d < dim;
-      const int64_t tt = t0 + j0 + r;
-      rq[j] = in ? ldv4(A.q + tt * A.ldq + (int64_t)gq * dim + d) : zero4;
-      rk[j] = in ? ldv4(A.k + tt * A.ldk + (int64_t)gq * dim + d) : zero4;
+      const int c = tid + TH * j, r = c / CHK, d = (c % CHK) * 4;
+      const int64_t tt = t0 + min(j0 + r, qlen - 1), at = (int64_t)gq * dim + (d < dim ? d : 0);
+      rq[j] = ldv4(A.q + tt * A.ldq + at);
+      rk[j] = ldv4(A.k + tt * A.ldk + at);
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int c = tid + 256 * (j & 3), r = c >> 4, s0 = (c & 15) * 4;
-      rm[j] = j0 + r < qlen ? ldv4(A.X + (j >> 2) * A.mat + ((int64_t)(t0 + j0 + r) * H + h) * 64 + s0) : zero4;
+    for (int j = 0; j < NM; ++j) {
+      const int c = tid + TH * j, r = (c >> 4) & 63, s0 = (c & 15) * 4;
+      rm[j] = ldv4(A.X + (c >> 10) * A.mat + ((int64_t)(t0 + min(j0 + r, qlen - 1)) * H + h) * 64 + s0);
     }
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {  // token 16 (j / 4) + 4 g + j % 4 at this lane's column
-      const int r = j0 + 16 * (j >> 2) + 4 * g + (j & 3);
-      rv[j] = A.v[(int64_t)(t0 + min(r, qlen - 1)) * A.ldv + (int64_t)h * vdim + colc];
-      if (r >= qlen) rv[j] = 0.f;
-    }
-    if (w == 0) ra = A.aux[(int64_t)(t0 + min(j0 + lane, qlen - 1)) * H + h];
+    for (int n = 0; n < NO; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)  // this lane's column of the blocks' tokens
+        rv[n][i] = A.v[(int64_t)(t0 + min(j0 + 16 * block(n) + 4 * g + i, qlen - 1)) * A.ldv + (int64_t)h * vdim + colc];
+    ra = A.aux[(int64_t)(t0 + min(j0 + lane, qlen - 1)) * H + h];
   };
   fetch(0);
-  for (int j0 = 0; j0 < qlen; j0 += C) {
-    const int nt = min(C, qlen - j0), nb = (nt + 15) >> 4;
+  // A chunk; ALL: of 64 tokens, without a branch between its blocks, across which no read is moved ahead
+  auto chunk = [&](int j0, auto all_c) {
+    constexpr bool ALL = decltype(all_c)::value;
+    const int nt = ALL ? C : min(C, qlen - j0), nb = ALL ? 4 : (nt + 15) >> 4;
     __syncthreads();  // the previous chunk's readers are done
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
-      const int c = tid + 256 * j, r = c / CHK, d = (c % CHK) * 4;
-      *reinterpret_cast<f32x4*>(&Qs[r * LDK + d]) = rq[j];
-      *reinterpret_cast<f32x4*>(&Ks[r * LDK + d]) = rk[j];
+      const int c = tid + TH * j, r = c / CHK, d = (c % CHK) * 4;
+      const bool in = (ALL || r < nt) && d < dim;
+      *reinterpret_cast<f32x4*>(&Qs[r * LDK + d]) = in ? rq[j] : zero4;
+      *reinterpret_cast<f32x4*>(&Ks[r * LDK + d]) = in ? rk[j] : zero4;
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int c = tid + 256 * (j & 3);
-      *reinterpret_cast<f32x4*>(&Ms[(j >> 2) * C * LDP + (c >> 4) * LDP + (c & 15) * 4]) = rm[j];
+    for (int j = 0; j < NM; ++j) {
+      const int c = tid + TH * j, r = (c >> 4) & 63;
+      *reinterpret_cast<f32x4*>(&Ms[(c >> 10) * C * LDP + r * LDP + (c & 15) * 4]) = ALL || r < nt ? rm[j] : zero4;
     }
-    if (w == 0) ax[lane] = ra;
-    f32x4 u[4], o[4], U[4];  // u: first V, then V - e^b K S_0
+    if (wave == 0) ax[lane] = ra;
+    f32x4 v[NO], o[NO], ks[NO];  // of this wave's blocks: v first V, then V - e^b K S_0, then U
 #pragma unroll
-    for (int j = 0; j < 16; ++j) u[j >> 2][j & 3] = rv[j];
+    for (int n = 0; n < NO; ++n) {
+      o[n] = ks[n] = zero4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[n][i] = ALL || 16 * block(n) + 4 * g + i < nt ? rv[n][i] : 0.f;
+    }
     __syncthreads();
     if (j0 + C < qlen) fetch(j0 + C);
     const float a_all = ax[0][3];
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
-      o[rt] = U[rt] = zero4;
       if (rt >= nb) continue;
-      const f32x4 ksv = dot32s<KT>(&Ks[(16 * rt + li) * LDK + 4 * g], S);
-      o[rt] = dot32s<KT>(&Qs[(16 * rt + li) * LDK + 4 * g], S);
+      f32x4 xk[KO], xq[KO];  // (all of a block's reads before its products)
+#pragma unroll
+      for (int kt = 0; kt < KO; ++kt) {
+        xk[kt] = ldv4(&Ks[(16 * rt + li) * LDK + k0w + 4 * g + 16 * kt]);
+        xq[kt] = ldv4(&Qs[(16 * rt + li) * LDK + k0w + 4 * g + 16 * kt]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      const f32x4 kp = dot32s<KO>(xk, S), qp = dot32s<KO>(xq, S);
+      if constexpr (NH == 1) {
+        ks[rt] = kp, o[rt] = qp;
+      } else {  // one of two blocks is the other wave's
+        const int n = rt >> 1;
+        const bool mine = own(rt);
+        f32x4* const at = ex + ((wave * 2 + n) * 2) * 64 + lane;
+        if (rt & 1) {
+          const f32x4 kx = mine ? ks[n] : kp, qx = mine ? o[n] : qp;
+          at[0] = kx, at[64] = qx;
+          ks[n] = mine ? kp : ks[n], o[n] = mine ? qp : o[n];
+        } else {
+          ks[n] = kp, o[n] = qp;
+        }
+      }
+    }
+    if (NH == 2 && (nb & 1)) {  // (its second half was not taken)
+      const int n = nb >> 1;
+      if (!own(nb - 1)) ex[((wave * 2 + n) * 2) * 64 + lane] = ks[n], ex[((wave * 2 + n) * 2 + 1) * 64 + lane] = o[n];
+    }
+    if (NH == 2) __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NO; ++n) {
+      const int rt = block(n);
+      if (rt >= nb) {
+        ks[n] = o[n] = zero4;
+        continue;
+      }
+      if (NH == 2) {
+        ks[n] += ex[(((wave ^ 4) * 2 + n) * 2) * 64 + lane];
+        o[n] += ex[(((wave ^ 4) * 2 + n) * 2 + 1) * 64 + lane];
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const f32x4 x = ax[16 * rt + 4 * g + i];
-        u[rt][i] = fmaf(-x[0], ksv[i], u[rt][i]);
-        o[rt][i] *= x[1];
+        v[n][i] = fmaf(-x[0], ks[n][i], v[n][i]);
+        o[n][i] *= x[1];
       }
     }
-    int bad = contain(u, o, g);
+    f32x4 u[4];  // all blocks
+    auto gather = [&](f32x4* at) {
+      if constexpr (NH == 2) {
+#pragma unroll
+        for (int n = 0; n < NO; ++n) at[(w * 4 + block(n)) * 64 + lane] = v[n];
+        __syncthreads();
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) u[rt] = at[(w * 4 + rt) * 64 + lane];
+      } else {
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) u[rt] = v[rt];
+      }
+      const int bad = contain(u, g);
+      if (__builtin_expect(__any(bad < C), 0)) {
+#pragma unroll
+        for (int n = 0; n < NO; ++n) from_bad(o[n], bad, block(n), g);
+      }
+      return bad;
+    };
+    // y += M u of this wave's blocks, M lower triangular. Two blocks (h = 0: 0 and 3, 1: 1 and 2): the first block's first product, the second's
+    // first three, and one that is either's.
+    auto product = [&](const f32x4& x, const f32x4& y, f32x4 sum) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], y[i], sum, 0, 0, 0);
+      return sum;
+    };
+    auto lower = [&](const float* M, f32x4 (&y)[NO]) {
+      auto part = [&](int rt, int m) { return ldv4(M + (16 * rt + li) * LDP + 16 * m + 4 * g); };
+      if constexpr (NH == 2) {
+        const f32x4 x0 = part(hf, 0), x1 = part(3 - hf, 0), x2 = part(3 - hf, 1), x3 = part(3 - hf, 2), x4 = part(hf ? 1 : 3, hf ? 1 : 3);
+        const f32x4 ue = hf ? u[1] : u[3];
+        const f32x4 a = product(x0, u[0], zero4), f = product(x3, u[2], product(x2, u[1], product(x1, u[0], zero4)));
+        const f32x4 e = product(x4, ue, hf ? a : f);
+        y[0] += hf ? e : a;
+        y[1] += hf ? f : e;
+      } else {
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) {
+          if (rt >= nb) continue;
+          f32x4 sum = zero4;
+#pragma unroll
+          for (int m = 0; m <= rt; ++m) sum = product(part(rt, m), u[m], sum);
+          y[rt] += sum;
+        }
+      }
+    };
     // U = X u, O += P U
+    int bad = gather(ux);
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      if (rt >= nb) continue;
-#pragma unroll
-      for (int m = 0; m <= rt; ++m) {
-        const f32x4 x = ldv4(&Ms[(16 * rt + li) * LDP + 16 * m + 4 * g]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) U[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], u[m][i], U[rt], 0, 0, 0);
-      }
-    }
-    bad = min(bad, contain(U, o, g));
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      if (rt >= nb) continue;
-      f32x4 in = zero4;
-#pragma unroll
-      for (int m = 0; m <= rt; ++m) {
-        const f32x4 x = ldv4(&Ms[C * LDP + (16 * rt + li) * LDP + 16 * m + 4 * g]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) in = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], U[m][i], in, 0, 0, 0);
-      }
-      o[rt] += in;
-    }
+    for (int n = 0; n < NO; ++n) v[n] = zero4;
+    lower(Ms, v);
+    bad = min(bad, gather(uX));
+    lower(Ms + C * LDP, o);
     // the state: e^(b_C) S_0 + K^T (w U)
     const float keep = bad < C ? __uint_as_float(0x7fc00000u) : a_all;
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
+    for (int kt = 0; kt < KO; ++kt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) S[kt][i] *= keep;
+    f32x4 xs[KO], xw;
+    auto columns = [&](int m) {
+#pragma unroll
+      for (int kt = 0; kt < KO; ++kt) {
+        const float* p = &Ks[(16 * m + 4 * g) * LDK + k0w + 16 * kt + li];
+        xs[kt] = f32x4{p[0], p[LDK], p[2 * LDK], p[3 * LDK]};
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xw[i] = ax[16 * m + 4 * g + i][2];
+    };
+    columns(0);
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       if (m >= nb) continue;
-      f32x4 wu;
+      f32x4 x[KO];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) wu[i] = U[m][i] * ax[16 * m + 4 * g + i][2];
+      for (int kt = 0; kt < KO; ++kt) x[kt] = xs[kt];
+      const f32x4 wu = u[m] * xw;
+      if (m < 3) columns(m + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int k0 = 0; k0 < KT; k0 += 2) {
-        f32x4 x[2];
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int n = 0; n < 2; ++n) {
-          const float* p = &Ks[(16 * m + 4 * g) * LDK + 16 * (k0 + n) + li];
-          x[n] = f32x4{p[0], p[LDK], p[2 * LDK], p[3 * LDK]};
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int n = 0; n < 2; ++n) S[k0 + n] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[n][i], wu[i], S[k0 + n], 0, 0, 0);
-      }
+        for (int kt = 0; kt < KO; ++kt) S[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[kt][i], wu[i], S[kt], 0, 0, 0);
     }
     if (col < vdim) {
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt)
+      for (int n = 0; n < NO; ++n)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int t = 16 * rt + 4 * g + i;
-          if (t < nt) outp[(int64_t)(j0 + t) * H * vdim] = o[rt][i];
+          const int t = 16 * block(n) + 4 * g + i;
+          if (ALL || t < nt) outp[(int64_t)(j0 + t) * H * vdim] = o[n][i];
         }
     }
-  }
-  int r0 = 4 * g;
+  };
+  int j0 = 0;
+  if constexpr (NH == 2)
+    for (; j0 + C <= qlen; j0 += C) chunk(j0, std::true_type{});
+  for (; j0 < qlen; j0 += C) chunk(j0, std::false_type{});
+  int r0 = k0w + 4 * g;
   asm volatile("" : "+v"(r0));  // (the rows anew: which of them the state has would be kept in spilled registers through the loop)
   if (col < vdim) {
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
+    for (int kt = 0; kt < KO; ++kt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r = r0 + 16 * kt + i;
@@ -1000,22 +1114,23 @@ void launch_delta_chunk32(const void* q, const void* k, const void* v, int64_t l
                      (float*)work, (int64_t)T_ * H * 64, (f32x4*)aux, H, G, dim, vdim};
   dim3 g1((max_qlen + 63) / 64, H, B), g2(H, (vdim + 63) / 64, B);
   auto lds1 = [](int kt) { return (size_t)prep32_k_bytes(kt) + (size_t)4 * (64 * 68 + 3 * 64) + 8 * 64; };
-  auto lds2 = [](int kt) { return (size_t)4 * (2 * 64 * (16 * kt + 4) + 2 * 64 * 68) + (size_t)16 * 64; };
-#define LAUNCH_DC32(KT_)                                                                                             \
-  do {                                                                                                               \
-    static bool once = [] {                                                                                          \
-      for (const void* f : {(const void*)delta_prep32_kernel<KT_, bf16_t>, (const void*)delta_prep32_kernel<KT_, float>, \
-                            (const void*)delta_chunk32_kernel<KT_>})                                                 \
-        (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                        \
-      return true;                                                                                                   \
-    }();                                                                                                             \
-    (void)once;                                                                                                      \
-    DISPATCH_T(dp, TP, (delta_prep32_kernel<KT_, TP><<<g1, 256, lds1(KT_), st>>>(A)));                               \
-    delta_chunk32_kernel<KT_><<<g2, 256, lds2(KT_), st>>>(A);                                                        \
+  // (two halves: parts of sums, u and U besides)
+  auto lds2 = [](int kt, int nh) { return (size_t)4 * (2 * 64 * (16 * kt + 4) + 2 * 64 * 68) + (size_t)16 * 64 + (nh == 2 ? 16 * 64 * 48 : 0); };
+#define LAUNCH_DC32(KT_, NH_)                                                                                         \
+  do {                                                                                                                \
+    static bool once = [] {                                                                                           \
+      for (const void* f : {(const void*)delta_prep32_kernel<KT_, bf16_t>, (const void*)delta_prep32_kernel<KT_, float>,\
+                            (const void*)delta_chunk32_kernel<KT_, NH_>})                                             \
+        (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                         \
+      return true;                                                                                                    \
+    }();                                                                                                              \
+    (void)once;                                                                                                       \
+    DISPATCH_T(dp, TP, (delta_prep32_kernel<KT_, TP><<<g1, 256, lds1(KT_), st>>>(A)));                                \
+    delta_chunk32_kernel<KT_, NH_><<<g2, 256 * NH_, lds2(KT_, NH_), st>>>(A);                                         \
   } while (0)
-  if (dim <= 32) LAUNCH_DC32(2);
-  else if (dim <= 64) LAUNCH_DC32(4);
-  else LAUNCH_DC32(8);
+  if (dim <= 32) LAUNCH_DC32(2, 1);
+  else if (dim <= 64) LAUNCH_DC32(4, 2);
+  else LAUNCH_DC32(8, 2);
 #undef LAUNCH_DC32
   HIP_CHECK_LAUNCH();
 }
