@@ -238,7 +238,7 @@ __device__ __forceinline__ void linear_mend(const LinearArgs& A, int h, int b, i
 // activation comes first. The next chunk's rows are fetched into registers while this one is computed. KT: 16-row tiles of the
 // state (dim padded with zeros).
 template <int KT, int MODE>
-__global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chunk_kernel(LinearArgs A) {
+__global__ __launch_bounds__(256, KT <= 4 || (MODE == 2 && KT <= 8) ? 2 : 1) void linear_chunk_kernel(LinearArgs A) {
   using LT = typename std::conditional<MODE == 2, bf16_t, float>::type;
   constexpr int C = 64, DKP = 16 * KT, LDK = DKP + (MODE == 2 ? 8 : 4), LDP = 64 + 4;
   constexpr int NCH = KT < 4 ? 2 : 4;  // chains an fp32 product over the keys is summed in: shorter ones round less
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
   const int dim = A.dim, vdim = A.vdim, H = A.H, gq = h / (H / A.G);
   const int t0 = A.cu[b], qlen = A.cu[b + 1] - t0, slot = A.sslots[b], ctx = A.ctx[b];
   if (qlen <= 0) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, g = lane >> 4;
   const int col = blockIdx.y * 64 + 16 * w + li, colc = min(col, vdim - 1);
   float* outp = A.out + ((int64_t)t0 * H + h) * vdim + col;
   if (slot < 0 || ctx <= 0) {
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
   constexpr int CHK = DKP / 8, NK = C * CHK / 256;
   static_assert((C * CHK) % 256 == 0, "whole 16-byte pieces per thread");
   u16x8 rq[NK], rk[NK];
-  bf16_t rv[16], rd = 0;
+  uint32_t rv[16], rd = 0;  // (words: two numbers to a register wait for both)
   const u16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
   auto fetch = [&](int j0) {  // the portion's last row again and again past its end, a row's first piece past its last
 #pragma unroll
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
     }
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
-      const float x = j0 + 16 * (j >> 2) + 4 * g + (j & 3) < qlen ? bf2f(rv[j]) : 0.f;
+      const float x = j0 + 16 * (j >> 2) + 4 * g + (j & 3) < qlen ? bf2f((bf16_t)rv[j]) : 0.f;
       v[j >> 2][j & 3] = MODE == 0 && SILU ? lin_silu<bf16_t>(x) : x;
     }
   };
@@ -339,8 +339,16 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
   const bool alt = MODE == 0 && dec < 0.f;  // a negative factor: the sign alternates with the distance
   const float ea = MODE == 2 ? expf(dec) : 0.f, dtb = MODE == 2 ? A.dt_bias[h] : 0.f;
   fetch(0);
-  for (int j0 = 0; j0 < qlen; j0 += C) {
-    const int nt = min(C, qlen - j0);
+  // A chunk; ALL: of 64 tokens, without a branch between its blocks
+  auto chunk = [&](int j0, auto all_c) {
+    constexpr bool ALL = decltype(all_c)::value;
+    const int nt = ALL ? C : min(C, qlen - j0);
+    // (the places anew: those of all reads below, kept through the loop, leave no room for the next chunk's rows, and a number in scratch is waited
+    // for with every load that is on its way: state space, 64 heads of 128 x 64 over 8 x 1024 tokens, 193 -> 159 us; decay, 16 heads of 128 x 128,
+    // 243 -> 228)
+    int lo = lane;
+    asm volatile("" : "+v"(lo));
+    const int li = lo & 15, g = lo >> 4;
     __syncthreads();  // the previous chunk's readers are done
     f32x4 v[4];
     if (MODE != 2 && A.silu) stage_as(j0, v, std::true_type{});
@@ -350,7 +358,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
       double F;
       float e = in ? 1.0f : 0.f;
       if (MODE == 2) {
-        e = in ? lin_softplus(bf2f(rd) + dtb) : 0.f;
+        e = in ? lin_softplus(bf2f((bf16_t)rd) + dtb) : 0.f;
         F = in ? at_least((double)(-ea * e), -1e8) : 0.0;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -373,7 +381,7 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
     }
     __syncthreads();
     if (j0 + C < qlen) fetch(j0 + C);
-    const int nb = (nt + 15) >> 4;  // blocks of tokens
+    const int nb = ALL ? 4 : (nt + 15) >> 4;  // blocks of tokens
     // weighted scores: wave w owns the tokens 16 w .. 16 w + 15 (rows) and the keys up to them (columns)
     if (w < nb) {
       f32x4 p[4];
@@ -539,10 +547,13 @@ __global__ __launch_bounds__(256, MODE == 2 && KT <= 8 ? 2 : 1) void linear_chun
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int t = 16 * rt + 4 * g + i;
-          if (t < nt) outp[(int64_t)(j0 + t) * H * vdim] = MODE == 2 ? fmaf(dskip, v[rt][i], o[rt][i]) : o[rt][i];
+          if (ALL || t < nt) outp[(int64_t)(j0 + t) * H * vdim] = MODE == 2 ? fmaf(dskip, v[rt][i], o[rt][i]) : o[rt][i];
         }
     }
-  }
+  };
+  int j0 = 0;
+  for (; j0 + C <= qlen; j0 += C) chunk(j0, std::true_type{});
+  if (j0 < qlen) chunk(j0, std::false_type{});
   float z = 0.f;
 #pragma unroll
   for (int kt = 0; kt < KT; ++kt)
