@@ -478,7 +478,7 @@ void launch_pool_window_attn(const void* q, const void* kc, const void* vc, cons
 // step of single rows enough workgroups. The next tile's 16-byte chunks are fetched into registers while this one is
 // computed from LDS.
 template <int DK, int NVT, int NS>
-__global__ __launch_bounds__(256, 2) void pool_window_attn_mfma_kernel(
+__global__ __launch_bounds__(256, NS == 1 && NVT <= 8 ? 3 : 2) void pool_window_attn_mfma_kernel(
     const float* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
     const bf16_t* __restrict__ kp, const bf16_t* __restrict__ vp, const int* __restrict__ block_tables, int max_blocks,
     const int* __restrict__ cu_q, const int* __restrict__ ctx_lens, const float* __restrict__ pb,
@@ -500,7 +500,7 @@ __global__ __launch_bounds__(256, 2) void pool_window_attn_mfma_kernel(
   const int r0 = rb * rows_per_wg;
   if (r0 >= qlen || ctx_lens[b] <= 0) return;
   const int p0 = ctx_lens[b] - qlen;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15, g = lane >> 4;
   const int v0 = vch * VCH;
   const int64_t vrow = (int64_t)G * vdim;
@@ -554,17 +554,29 @@ __global__ __launch_bounds__(256, 2) void pool_window_attn_mfma_kernel(
   // The cache rows of a tile's 64 keys lie in LDS two tiles ahead: one look-up a thread and tile, its page number in flight behind the
   // tile that is being computed. Looked up where a row is read, with a branch between pages and pooled rows, a thread's eight rows
   // came one after the other, each behind its page number: 8 prompts of 1024 rows, 16 heads of 128 in groups of four, window 512 and
-  // blocks of 16, 197 -> 127 us, 33 single rows 10.8 -> 8.4 us. (Two slot groups a wave, for which the registers suffice: 126 us.)
+  // blocks of 16, 197 -> 127 us, 33 single rows 10.8 -> 8.4 us. (Two slot groups a wave, for which the registers suffice: 126 us.) The page
+  // number stays as it was read until the row is stored, the next tile is fetched without a condition, and what a row sees are three numbers
+  // of its own: with a branch for each weight, and waits for the fetch before the products, the same took 127 us against 112, and three
+  // workgroups a CU, for which the registers now suffice, take 98.
   __shared__ int64_t s_row[2][BKV];
   const int pool1 = max(pool, 1);
-  auto look_up = [&](int u0) -> int64_t {  // a pooled row (negative) or a page row
+  auto key_of = [&](int u0) {  // this lane's key of a tile: the position that it is, or that its block begins at
     const int u = min(u0 + lane, total - 1);
-    const bool pooled = u < nb;
-    const int j = pooled ? u * pool : jlo + (u - nb);
-    const int64_t page = bt[j / bs];
-    const int off = j % bs;
-    return pooled ? -1 - (page * per + off / pool1) : page * bs + off;
+    return u < nb ? u * pool : jlo + (u - nb);
   };
+  auto row_of = [&](int u0, int64_t page) -> int64_t {  // a pooled row (negative) or a page row
+    const int off = key_of(u0) % bs;
+    return min(u0 + lane, total - 1) < nb ? -1 - (page * per + off / pool1) : page * bs + off;
+  };
+  // What a row sees: pooled rows below seen, keys from from on, as many as count
+  int seen[NS], from[NS], count[NS];
+#pragma unroll
+  for (int n = 0; n < NS; ++n) {
+    const int out = window > 0 ? max(qpos[n] - window + 1, 0) : 0;  // positions before the row's window
+    seen[n] = min(nb > 0 ? out / pool1 : 0, min(nb, u_end));
+    from[n] = nb + max(out - jlo, 0);
+    count[n] = max(min(nb + qpos[n] - jlo + 1, u_end) - from[n], 0);
+  }
   auto load_tile = [&](const int64_t* rows) {
 #pragma unroll
     for (int j = 0; j < NCK; ++j) {
@@ -642,13 +654,7 @@ __global__ __launch_bounds__(256, 2) void pool_window_attn_mfma_kernel(
           float p = __builtin_amdgcn_rcpf(1.0f + e);
           if constexpr (!WHOLE) {
             const int u = u0 + kt * 16 + 4 * g + i;
-            bool vis = u < u_end;
-            if (u < nb) {
-              vis = vis && u * pool + pool - 1 <= qpos[n] - window;
-            } else {
-              const int j = jlo + (u - nb);
-              vis = vis && j <= qpos[n] && (window == 0 || qpos[n] - j < window);
-            }
+            const bool vis = u < seen[n] || (unsigned)(u - from[n]) < (unsigned)count[n];
             p = vis ? p : 0.f;
           }
           const bf16_t hi = f2bf(p);
@@ -686,18 +692,19 @@ __global__ __launch_bounds__(256, 2) void pool_window_attn_mfma_kernel(
     }
   };
   if (u_end > u_begin) {
-    if (w < 2) s_row[w][lane] = look_up(u_begin + w * BKV);
+    if (w < 2) s_row[w][lane] = row_of(u_begin + w * BKV, bt[key_of(u_begin + w * BKV) / bs]);
     __syncthreads();
     load_tile(s_row[0]);
   }
   for (int u0 = u_begin, k = 0; u0 < u_end; u0 += BKV, k ^= 1) {
     __syncthreads();  // every wave is done reading the previous tile, and its rows
     store_tile();
-    const int64_t ahead = look_up(u0 + 2 * BKV);
+    int page = 0;
+    if (w == 0) page = bt[key_of(u0 + 2 * BKV) / bs];
     __syncthreads();
-    if (u0 + BKV < u_end) load_tile(s_row[k ^ 1]);
+    load_tile(s_row[k ^ 1]);  // (behind the last tile its last row again and again)
     if (wave_rows) compute_tile(u0);
-    if (w == 0) s_row[k][lane] = ahead;
+    if (w == 0) s_row[k][lane] = row_of(u0 + 2 * BKV, page);
   }
 #pragma unroll
   for (int n = 0; n < NS; ++n) {
