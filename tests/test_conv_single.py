@@ -49,3 +49,39 @@ def test_single_rows(device, dtype, out_dtype, residual, bias, silu, C, taps):
             if slots[s] >= 0:
                 assert torch.equal(y[slots[s]].cpu().double(), past[s])
         assert torch.equal(y.cpu(), z.cpu()) and torch.equal(y[[1, 3]].cpu(), state[[1, 3]])
+
+
+# portions over strips of sixteen rows: strips within one, over its first rows, over a border, past the last row and with a padded sequence
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("residual,bias,silu", [(True, False, False), (False, True, True)])
+@pytest.mark.parametrize("C,taps", [(40, 4), (1032, 9), (12, 2), (70, 3)])
+def test_strips_of_portions(dtype, out_dtype, residual, bias, silu, C, taps):
+    gen = torch.Generator().manual_seed(C + taps)
+    lens, first, slots = [19, 100, 1, 16, 40, 35], [0, 7, 2, 0, 3, 0], [4, 0, 1, 2, -1, 5]
+    T, R = sum(lens), taps - 1
+    x = torch.randn(T, C, generator=gen).to(dtype)
+    w, b = (torch.randn(C, taps, generator=gen) * taps ** -0.5).to(dtype), torch.randn(C, generator=gen).to(dtype)
+    state = torch.randn(6, R, C, generator=gen)
+    want, size, t = torch.zeros(T, C, dtype=torch.float64), torch.zeros(T, C, dtype=torch.float64), 0
+    for n, p0, s in zip(lens, first, slots):
+        if s >= 0:
+            past = torch.zeros(R, C, dtype=torch.float64)
+            if p0:
+                past[max(R - p0, 0):] = state[s, max(R - p0, 0):].double()
+            full = torch.cat([past, x[t:t + n].double()])
+            for k in range(taps):
+                want[t:t + n] += full[k:k + n] * w[:, k].double()
+                size[t:t + n] += (full[k:k + n] * w[:, k].double()).abs()
+            want[t:t + n] += (x[t:t + n].double() if residual else 0) + (b.double() if bias else 0)
+        t += n
+    size += want.abs() + x.double().abs() + 1
+    want = want * torch.sigmoid(want) if silu else want
+    ctx = torch.tensor([n + p if s >= 0 else 0 for n, p, s in zip(lens, first, slots)], dtype=torch.int32)
+    got = ops.causal_conv(x.cuda(), w.cuda(), state.clone().cuda(), torch.tensor([0] + lens).cumsum(0).int().cuda(), ctx.cuda(),
+                          torch.tensor(slots, dtype=torch.int32).cuda(), residual, silu, out_dtype, bias=b.cuda() if bias else None)
+    # sums of up to 11 terms in fp32, 2^-24 of their absolute sum each; the activation's slope is under 1.1, its own error 8 units; bf16 results 2^-8
+    lim = size * 24 * 2.0 ** -24 + (want.abs() * 2.0 ** -8 if out_dtype == torch.bfloat16 else 0)
+    live = torch.cat([torch.full((n,), s >= 0) for n, s in zip(lens, slots)])
+    assert ((got.cpu().double() - want).abs() <= lim)[live].all()
+    assert (got.cpu()[~live] == 0).all()
