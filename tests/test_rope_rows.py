@@ -49,3 +49,40 @@ def test_rope_rows(T, H, G, dim, vdim, rot, off, dtype, form):
         live = slots >= 0
         full[slots[live]], flim[slots[live]] = w[live], lm[live] + rnd * w[live].abs()
         assert ((cache[:, 0].double() - full).abs() <= flim).all()
+
+
+# latent rows of more numbers than a wave asks for at once, of one and of a few; heads and pairs past whole rounds of three waves; rows that are not cached
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H,R,rot,rdims", [(3, 1, 1, 2, 2), (5, 7, 511, 64, 62), (70, 16, 513, 64, 64), (2, 130, 700, 34, 34), (4, 3, 192, 6, 0), (9, 1, 96, 0, 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_latent_rows_and_their_queries(T, H, R, rot, rdims, dtype):
+    from llmss_amd.ops import hip
+    g = torch.Generator().manual_seed(T + R)
+    qdim, n = 5, R + rot
+    src = torch.randn(T, n + H * (qdim + rot), generator=g).to(dtype)
+    w = torch.randn(R, generator=g).to(dtype)
+    cs = torch.randn(T, rdims // 2, 2, generator=g)
+    slots = torch.randperm(T + 3, generator=g)[:T]
+    slots[0] = -1
+    cache, qa = torch.full((T + 3, 1, n), 7.0, dtype=dtype).cuda(), torch.full((T, H, n), 7.0).cuda()
+    hip.latent_norm_cache(src.cuda(), 0, R, w.cuda(), 1e-6, cache, slots.cuda(), rot, cs.cuda() if rot else None, qa if rot else None, n, qdim)
+
+    def turn(x):  # [..., rot] of row t
+        x = x.double().clone()
+        c, s = (cs[:, :, k].double().view(T, *[1] * (x.dim() - 2), rdims // 2) for k in range(2))
+        a, b = x[..., 0:rdims:2].clone(), x[..., 1:rdims:2].clone()
+        x[..., 0:rdims:2], x[..., 1:rdims:2] = a * c - b * s, b * c + a * s
+        return x
+    x = src.double()
+    row = x[:, :R] / (x[:, :R].pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * w.double()
+    want = torch.full((T + 3, n), 7.0, dtype=torch.float64)
+    for t in range(1, T):
+        want[slots[t], :R] = row[t]
+        want[slots[t], R:] = turn(x[:, R:n])[t]
+    # fp32: a few units, the mean over R of them; a rotation's two products of up to 4 x 4; bf16 results 2^-9 of theirs
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    assert ((cache.cpu().double()[:, 0] - want).abs() <= want.abs() * (eps + 64 * 2.0 ** -24) + 32 * 2.0 ** -24).all()
+    if rot:
+        q = turn(x[:, n:].view(T, H, qdim + rot)[..., qdim:])
+        assert ((qa.cpu().double()[..., R:] - q).abs() <= 64 * 2.0 ** -24 + q.abs() * 2.0 ** -20).all()
+        assert (qa[..., :R] == 7.0).all()
