@@ -96,6 +96,7 @@ bool gemm_tile_rings(int M, int N, int K, int batch);
 void moe_plan(int P, int E, int F, int N, int K, bool glu, int rows, bool big, int* rows_out, int* ring);
 void launch_moe_pp(int mode, const void* A, int64_t lda, const void* W, const void* meta, const void* order, void* C, int E,
                    int maxt, int top, int N, int K, int act, hipStream_t st);
+bool moe_pp_quad(int mode, int64_t lda, int maxt, int top, int N, int K, const void* C);
 bool moe_pp_glu_ok(int64_t ldh, int maxt, int top, int F, int K);
 void launch_moe_pp_glu(const void* h, int64_t ldh, const void* Wg, const void* Wu, const void* meta, const void* order, void* act,
                        int E, int maxt, int top, int F, int K, float limit, float alpha, const void* pw, int silu, hipStream_t st);
@@ -469,6 +470,7 @@ PYBIND11_MODULE(_C, m) {
                      int maxt, int top, int N, int K, int act, uintptr_t st) {
     launch_moe_pp(mode, CP(A), lda, CP(W), CP(meta), CP(order), P(C), E, maxt, top, N, K, act, S(st));
   });
+  m.def("moe_pp_quad", [](int mode, int64_t lda, int maxt, int top, int N, int K) { return moe_pp_quad(mode, lda, maxt, top, N, K, nullptr); });
   m.def("moe_pp_glu_ok", &moe_pp_glu_ok);
   m.def("moe_pp_glu", [](uintptr_t h, int64_t ldh, uintptr_t Wg, uintptr_t Wu, uintptr_t meta, uintptr_t order, uintptr_t act,
                          int E, int maxt, int top, int F, int K, float limit, float alpha, uintptr_t pw, int silu, uintptr_t st) {

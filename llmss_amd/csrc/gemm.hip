@@ -2649,9 +2649,16 @@ void gemm_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int* nt, i
   }
 }
 
-// Grouped expert products on 256 x 256 tiles (gemm_quad.hip, else the ping-pong kernel), over a tile list of 256 rows per tile (moe_group): C = act(A[order / top]
-// W_e^T) in bf16 (mode 1), C = A W_e^T in fp32 (mode 2), or C [rows, N / 2] = silu(gate) * up in bf16 with W's rows gate and up
-// in alternating groups of 16 (mode 3). A [rows, K] with row stride lda, W [E, N, K].
+// Whether grouped products of launch_moe_pp's modes take the four-wave kernel
+bool moe_pp_quad(int mode, int64_t lda, int maxt, int top, int N, int K, const void* C) {
+  return gemm_quad_ok(N, K, lda, K, mode == 2 ? 256 : (int64_t)maxt * 256 / std::max(top, 1) + 1, C, mode == 3 ? N / 2 : N, mode == 2 ? 4 : 2,
+                      mode == 3, true);
+}
+
+// Grouped expert products on 256 x 256 tiles (gemm_quad.hip, else the ping-pong kernel), over a tile list of 256 rows per tile whose taller tiles
+// stand first, their number behind it (launch_moe_group with `tall`): C = act(A[order / top] W_e^T) in bf16 (mode 1), C = A W_e^T in fp32 (mode
+// 2), or C [rows, N / 2] = silu(gate) * up in bf16 with W's rows gate and up in alternating groups of 16 (mode 3). A [rows, K] with row stride
+// lda, W [E, N, K].
 void launch_moe_pp(int mode, const void* A, int64_t lda, const void* W, const void* meta, const void* order, void* C, int E,
                    int maxt, int top, int N, int K, int act, hipStream_t st) {
   if (maxt <= 0) return;
@@ -2665,8 +2672,7 @@ void launch_moe_pp(int mode, const void* A, int64_t lda, const void* W, const vo
   const char* z = K & 63 ? zero_page() : nullptr;
   const int glu = mode == 3;
   if (glu && N % 32) throw std::runtime_error("moe_pp: gate and up in groups of 16 rows");
-  if (gemm_quad_ok(N, K, lda, K, mode == 2 ? 256 : (int64_t)maxt * 256 / std::max(top, 1) + 1, C, glu ? N / 2 : N,
-                   mode == 2 ? 4 : 2, glu != 0)) {
+  if (moe_pp_quad(mode, lda, maxt, top, N, K, C)) {
     if (mode < 1 || mode > 3) throw std::runtime_error("moe_pp: mode");
     launch_gemm_quad(mode == 2 ? 2 : 1, (const bf16_t*)A, lda, (const bf16_t*)W, K, nullptr, (bf16_t*)C, glu ? N / 2 : N, 0, N, K,
                      glu ? 0 : act, glu, 1, (unsigned)nwg, gr, st);
@@ -2684,10 +2690,10 @@ void launch_moe_pp(int mode, const void* A, int64_t lda, const void* W, const vo
 
 // Whether moe_pp_glu takes a layer with gate and up matrices [E, F, K] of their own: h [rows, K] with row stride ldh.
 bool moe_pp_glu_ok(int64_t ldh, int maxt, int top, int F, int K) {
-  return gemm_quad_ok(2 * F, K, ldh, K, (int64_t)maxt * 256 / std::max(top, 1) + 1, nullptr, F, 2, true) && F % 16 == 0;
+  return gemm_quad_ok(2 * F, K, ldh, K, (int64_t)maxt * 256 / std::max(top, 1) + 1, nullptr, F, 2, true, true) && F % 16 == 0;
 }
 
-// act [pairs, F] = glu(pw h Wg_e^T, pw h Wu_e^T) in bf16 over a tile list of 256 rows per tile
+// act [pairs, F] = glu(pw h Wg_e^T, pw h Wu_e^T) in bf16 over launch_moe_pp's tile list
 void launch_moe_pp_glu(const void* h, int64_t ldh, const void* Wg, const void* Wu, const void* meta, const void* order, void* act,
                        int E, int maxt, int top, int F, int K, float limit, float alpha, const void* pw, int silu, hipStream_t st) {
   if (maxt <= 0) return;

@@ -59,7 +59,8 @@ struct GluForm {
   }
 };
 
-bool gemm_quad_ok(int N, int K, int64_t ldx, int64_t ldw, int64_t rows, const void* Y, int64_t ldy, int es, bool glu);
+bool gemm_quad_ok(int N, int K, int64_t ldx, int64_t ldw, int64_t rows, const void* Y, int64_t ldy, int es, bool glu,
+                  bool list = false);
 void launch_gemm_quad(int grp, const bf16_t* A, int64_t lda, const bf16_t* B, int64_t ldb, const bf16_t* bias, bf16_t* Y,
                       int64_t ldy, int M, int N, int K, int act, int glu, int group_m, unsigned nwg, const PpGroup& gr,
                       hipStream_t st, const QkvEpi* qe = nullptr);

@@ -33,8 +33,8 @@
 // columns (two tiles of eight: GLU, four gates and their four ups twice; fp32: one tile of four) - 64 bytes a row and instruction, and stores of
 // half lines take four times as long. So two such pieces change hands between lanes li and li ^ 8 (a rotation by eight within the row of
 // sixteen lanes): one instruction then writes rows 0 .. 7 of the sixteen in whole lines, another rows 8 .. 15.
-// Rows and columns past the last lie outside the descriptor, so that no branch stands between the stores. (A row's pitch is under 2^24 bytes,
-// gemm_quad_ok, so that 256 of them fit the offsets.)
+// Rows and columns past the last lie outside the descriptor, so that no branch stands between the stores. (gemm_quad_ok: the rows that a wave
+// reaches over, 240 where they alternate by sixteens and else 128, fit a descriptor of 31 bits.)
 // All go past the caches: fp32 sums of 32768 pairs x 2048 (K = 768) 152 -> 131 us, which no cache would hold until they are read.
 template <int GRP, int GLU, int MS>
 __device__ __forceinline__ void quad_store(const f32x4 (&acc)[8][8], const PpGroup& gr, const bf16_t* __restrict__ bias, bf16_t* __restrict__ Y,
@@ -496,11 +496,11 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
   flush(n0 + wc * 128 + 64);
 }
 
-// rows: of X that one descriptor covers; es: bytes of an output element
-bool gemm_quad_ok(int N, int K, int64_t ldx, int64_t ldw, int64_t rows, const void* Y, int64_t ldy, int es, bool glu) {
+// rows: of X that one descriptor covers; es: bytes of an output element; list: tiles of an expert list, whose waves' rows alternate (quad_store)
+bool gemm_quad_ok(int N, int K, int64_t ldx, int64_t ldw, int64_t rows, const void* Y, int64_t ldy, int es, bool glu, bool list) {
   return K % 64 == 0 && K >= 64 && (uint64_t)rows * (uint64_t)ldx * 2 < (1ull << 31) && (uint64_t)256 * (uint64_t)ldw * 2 < (1ull << 31) &&
          ldx % 8 == 0 && ldw % 8 == 0 && N % (glu ? 32 : 8) == 0 && ((uintptr_t)Y & 15) == 0 && ldy * es % 16 == 0 &&
-         (uint64_t)128 * (uint64_t)ldy * es < (1ull << 31);
+         (uint64_t)(list ? 240 : 128) * (uint64_t)ldy * es < (1ull << 31);
 }
 
 void launch_gemm_quad(int grp, const bf16_t* X, int64_t ldx, const bf16_t* W, int64_t ldw, const bf16_t* bias, bf16_t* Y,

@@ -229,3 +229,20 @@ def test_gated_products_of_few_rows_leave_the_older_kernels(M, N, K, code):
 
     nt, split = H.lib().gemm_plan(M, N, K, False, True, False)
     assert split == 1 and (code is None or (nt >> 8) & (1024 if code == 1024 else 15) == code), (hex(nt), split)
+
+
+@pytest.mark.parametrize("mode,es", [(1, 2), (2, 4), (3, 2), (0, 2)])
+def test_rows_of_expert_results_fit_the_descriptor_that_stores_them(mode, es):
+    """A wave of the four-wave kernel stores over 240 rows of an expert tile (csrc/gemm_quad.hip quad_store), every other sixteen, through one
+    descriptor of 31 bits: rows past its end would be dropped. Wider results than fit go to another kernel; mode 0: gate and up in two matrices."""
+    from llmss_amd.ops import hip as H
+
+    def takes(width):  # numbers of a result row
+        if mode == 0:
+            return H.lib().moe_pp_glu_ok(256, 3, 1, width, 256)
+        return H.lib().moe_pp_quad(mode, 256, 3, 1, width * (2 if mode == 3 else 1), 256)
+
+    last = (2 ** 31 - 1) // (240 * es) // 16 * 16
+    assert takes(2048) and takes(last) and 240 * last * es < 2 ** 31
+    for width in (last + 16, 2_300_000 * 4 // es, 2 ** 31 // (128 * es) - 16):
+        assert 240 * width * es >= 2 ** 31 and not takes(width)
