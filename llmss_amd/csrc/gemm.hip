@@ -2614,9 +2614,12 @@ void gemm_cut_of(int M, int N, int K, bool glu, int* rows, int* cols, int* split
 }
 
 // The plan of a product whose result goes straight into an op that can sum its slabs: a split one, the slabs unsummed, where the older rules
-// split K of the finished product, so that it stays in 32 bits there; else split 1, and the product is finished by the plan of its size
+// split K of the finished product, so that it stays in 32 bits there; else split 1, and the product is finished by the plan of its size. A tuned
+// plan stays as it is.
 void gemm_closing_plan(int M, int N, int K, int* nt, int* splitk) {
+  int tuned_nt, tuned_split;
   gemm_plan(M, N, K, false, false, false, nt, splitk, false);
+  if (gemm_tuned_get(M, N, K, false, 0, &tuned_nt, &tuned_split)) return;
   if (*splitk <= 1 || (M <= 32 && K > 5120)) return;  // (27 x 2048 x 5632: 8.4 us on 64 x 64 tiles in eight slabs, 10.2 here in four)
   const FourPlan p = gemm_four_plan(M, N, K, false, true, 64 << 20);
   if (p.hint) *nt = p.hint, *splitk = p.split;

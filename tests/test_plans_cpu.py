@@ -246,3 +246,18 @@ def test_rows_of_expert_results_fit_the_descriptor_that_stores_them(mode, es):
     assert takes(2048) and takes(last) and 240 * last * es < 2 ** 31
     for width in (last + 16, 2_300_000 * 4 // es, 2 ** 31 // (128 * es) - 16):
         assert 240 * width * es >= 2 ** 31 and not takes(width)
+
+
+@pytest.mark.parametrize("nt,split", [(0x1300, 3), (0x1300, 1), ((3 | 32 | 1024) << 8, 2)])
+def test_closing_products_keep_a_tuned_plan(nt, split):
+    """The plan that a tuner or a plan file has set for a size stands, split or not, also where the op behind sums the slabs."""
+    from llmss_amd.ops import hip as H
+
+    M, N, K = 40, 1024, 4096
+    static = tuple(H.lib().gemm_closing_plan(M, N, K))
+    H.lib().gemm_tuned_set(M, N, K, False, 0, nt, split)
+    try:
+        assert tuple(H.lib().gemm_closing_plan(M, N, K)) == (nt, split) != static
+    finally:
+        H.lib().gemm_tuned_clear()
+    assert tuple(H.lib().gemm_closing_plan(M, N, K)) == static
