@@ -742,33 +742,20 @@ __global__ __launch_bounds__(512, NT <= 16 ? 4 : 2) void token_side_rows_kernel(
   f32x4 acc[DT];
 #pragma unroll
   for (int k = 0; k < DT; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // (Loads several blocks at a time throughout, those past the wave's columns its last one again: one after the other, each behind its condition,
-  // a workgroup waited 40 times for memory: 8192 rows of 2048 59 -> 57 us.)
-  constexpr int U = DT == 2 ? 4 : 2;
-#pragma unroll 1
-  for (int k0 = 0; k0 < span; k0 += 32 * U) {
-    float v[U][8];
-    s16x8 b[U][DT];
+#pragma unroll 8
+  for (int k = c0 + 8 * g; k < c0 + span; k += 32) {
+    float v[8];
+    ldv<float, 4>(xr + k, v);
+    ldv<float, 4>(xr + k + 4, v + 4);
+    s16x8 b[DT], h, m, l;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = c0 + min(k0 + 32 * u, span - 32) + 8 * g;
-      ldv<float, 4>(xr + k, v[u]);
-      ldv<float, 4>(xr + k + 4, v[u] + 4);
+    for (int j = 0; j < DT; ++j) b[j] = *reinterpret_cast<const s16x8*>(wg + (int64_t)(16 * j + li) * W + k);
+    split(v, h, m, l);
 #pragma unroll
-      for (int j = 0; j < DT; ++j) b[u][j] = *reinterpret_cast<const s16x8*>(wg + (int64_t)(16 * j + li) * W + k);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (k0 + 32 * u >= span) continue;
-      s16x8 h, m, l;
-      split(v[u], h, m, l);
-#pragma unroll
-      for (int j = 0; j < DT; ++j) {
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l, b[u][j], acc[j], 0, 0, 0);
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(m, b[u][j], acc[j], 0, 0, 0);
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h, b[u][j], acc[j], 0, 0, 0);
-      }
+    for (int j = 0; j < DT; ++j) {
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l, b[j], acc[j], 0, 0, 0);
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(m, b[j], acc[j], 0, 0, 0);
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h, b[j], acc[j], 0, 0, 0);
     }
   }
 #pragma unroll
@@ -826,55 +813,40 @@ __global__ __launch_bounds__(512, NT <= 16 ? 4 : 2) void token_side_rows_kernel(
   const bool in = t0 + li < T_;
   const float* ar = p.add ? p.add + (int64_t)t * W : nullptr;
   ss = 0.f;
-  constexpr int UX = NT == 16 ? 2 : 4;  // (as the registers suffice)
 #pragma unroll
-  for (int c4 = 0; c4 < NT; c4 += UX) {
-    float xv[UX][4], wn[UX][4], a[UX][4];
+  for (int ct = 0; ct < NT; ++ct) {
+    if (16 * ct >= span) continue;
+    const int c = c0 + 16 * ct + 4 * g;
+    float xv[4], wn[4];
+    ldv<float, 4>(xr + c, xv);
+    ldv<float, 4>(s.wn + c, wn);
 #pragma unroll
-    for (int u = 0; u < UX; ++u) {
-      const int c = c0 + min(16 * (c4 + u), span - 16) + 4 * g;
-      ldv<float, 4>(xr + c, xv[u]);
-      ldv<float, 4>(s.wn + c, wn[u]);
-    }
+    for (int i = 0; i < 4; ++i) xv[i] = fmaf(y[ct][i] * inv, wn[i], xv[i]);
     if (ar) {
+      float a[4];
+      ldv<float, 4>(ar + c, a);
 #pragma unroll
-      for (int u = 0; u < UX; ++u) ldv<float, 4>(ar + c0 + min(16 * (c4 + u), span - 16) + 4 * g, a[u]);
+      for (int i = 0; i < 4; ++i) xv[i] += a[i];
     }
-    __builtin_amdgcn_sched_barrier(0);
+    if (in) stv<float, 4>(xr + c, xv);
 #pragma unroll
-    for (int u = 0; u < UX; ++u) {
-      const int ct = c4 + u;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) xv[u][i] = fmaf(y[ct][i] * inv, wn[u][i], xv[u][i]);
-      if (ar) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) xv[u][i] += a[u][i];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) y[ct][i] = xv[u][i];
-      if (16 * ct >= span) continue;
-      if (in) stv<float, 4>(xr + c0 + 16 * ct + 4 * g, xv[u]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ss = fmaf(xv[u][i], xv[u][i], ss);
+    for (int i = 0; i < 4; ++i) {
+      y[ct][i] = xv[i];
+      ss = fmaf(xv[i], xv[i], ss);
     }
   }
   if (!p.wnext) return;
   const float inv2 = row_inv(ss, red[1]);
   bf16_t* hr = (bf16_t*)p.h + (int64_t)t * p.ldh;
 #pragma unroll
-  for (int c4 = 0; c4 < NT; c4 += 8) {
-    float wn[8][4], o[4];
+  for (int ct = 0; ct < NT; ++ct) {
+    if (16 * ct >= span) continue;
+    const int c = c0 + 16 * ct + 4 * g;
+    float wn[4], o[4];
+    ldv<float, 4>(p.wnext + c, wn);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) ldv<float, 4>(p.wnext + c0 + min(16 * (c4 + u), span - 16) + 4 * g, wn[u]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int ct = c4 + u;
-      if (16 * ct >= span) continue;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = y[ct][i] * inv2 * wn[u][i];
-      if (in) stv<bf16_t, 4>(hr + c0 + 16 * ct + 4 * g, o);
-    }
+    for (int i = 0; i < 4; ++i) o[i] = y[ct][i] * inv2 * wn[i];
+    if (in) stv<bf16_t, 4>(hr + c, o);
   }
 }
 
