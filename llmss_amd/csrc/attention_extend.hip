@@ -222,8 +222,9 @@ __global__ __launch_bounds__(256, D == 256 ? 2 : NS) void attn_extend_kernel(
       if constexpr (PIPE) store_tile();
       else stage_direct(kv0, staged);
       __syncthreads();
-      // (behind the last tile its last key again and again)
-      if constexpr (PIPE) load_tile(kv0 + BKV, staged);
+      if constexpr (PIPE) {
+        if (kv0 + BKV < kv_stop) load_tile(kv0 + BKV, staged);
+      }
       if (kv0 > wave_qhi) continue;  // whole tile in this wave's causal future (barriers stay uniform)
       if (kv0 + BKV <= wave_klo) continue;  // whole tile older than this wave's windows
 
