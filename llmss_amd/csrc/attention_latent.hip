@@ -23,9 +23,12 @@
 // (2i, 2i + 1), i < rdims / 2, turned by cs[t, i] = (cos, sin) and the numbers from rdims on passed unchanged; and
 // every query head's rotated part - head h holds qdim plain numbers, then rot - is turned the same way into
 // qa[t, h, R : R + rot] (qa [T, H, R + rot] in its own type TQ). The queries are columns of src, or rows of their own (qsrc).
-// A token's first wave forms its row, the other three turn its queries, four pairs of each lane's in flight: by one wave, pair by pair, a step of 8
-// tokens took 5.5 us, and a decode step of Nolavik's latent layer 2 us more than now (answers 2727 -> 2697 us).
-template <typename T, typename TQ>
+// Few tokens wait for memory: a token's first wave forms its row, up to three others turn its queries, U pairs of each lane's in flight (one wave,
+// pair by pair: 8 tokens of Nolavik's latent layer 5.5 us and 2 us more a decode step, answers 2727 -> 2697 us). Many are bound by instructions, so
+// that nothing is asked for twice: V blocks of 64 cover a row, and from 4096 tokens on one wave does both, pair by pair. us, one
+// wave in loops, four waves and eight blocks whatever the sizes, now: 8192 rows of 64 with 8 heads' 16 pairs 6.4, 8.1, 6.4; of 64, four heads' 32 6.2, 8.2,
+// 6.1; 8260 of 192, 16 heads 14.4, 14.2, 13.0; 4095 and 4096 rows with four heads 4.5 either way, 1000 3.4, 3.3, 3.0; 64 rows of 192, 16 heads 4.4, 2.9, 2.8.
+template <typename T, typename TQ, int V, int U>
 __global__ __launch_bounds__(256) void latent_norm_cache_kernel(const T* __restrict__ src, int64_t lds_, int off,
                                                                const T* __restrict__ w, float eps,
                                                                T* __restrict__ cache, const int64_t* __restrict__ slots,
@@ -36,9 +39,9 @@ __global__ __launch_bounds__(256) void latent_norm_cache_kernel(const T* __restr
   const int t = blockIdx.x, lane = threadIdx.x & 63;
   const int half = rdims >> 1, rest = rot - rdims;
   const float* tab = cs + (int64_t)t * half * 2;
-  if (threadIdx.x >= 64) {  // (only where queries have a rotated part)
-    constexpr int U = 4;
-    const int first = threadIdx.x - 64, step = blockDim.x - 64, n = H * half;
+  const int own = blockDim.x > 64 ? 64 : 0;  // threads that turn no queries
+  if (rot && (int)threadIdx.x >= own) {
+    const int first = threadIdx.x - own, step = blockDim.x - own, n = H * half;
     const T* q = qsrc + (int64_t)t * ldq;
     TQ* dst = qa + (int64_t)t * H * (R + rot) + R;
     for (int e0 = first; e0 < n; e0 += U * step) {
@@ -63,12 +66,11 @@ __global__ __launch_bounds__(256) void latent_norm_cache_kernel(const T* __restr
       const int h = e / rest, i = rdims + e - h * rest;
       El<TQ>::st(dst + (int64_t)h * (R + rot) + i, El<T>::ld(q + (int64_t)h * (qdim + rot) + qdim + i));
     }
-    return;
+    if (own) return;
   }
   const int64_t slot = slots[t];
   if (slot < 0) return;
   const T* s = src + (int64_t)t * lds_ + off;
-  constexpr int V = 8;  // numbers of a row, and their weights, that a lane asks for at once; what is past them in a loop
   T x[V], wx[V];
   if (R > 0) {
 #pragma unroll
@@ -106,9 +108,25 @@ void launch_latent_norm_cache(const void* src, int64_t ld, int off, const void* 
   if (T_ == 0) return;
   if (rot < 0 || rdims < 0 || rdims > rot || (rdims & 1))
     throw std::runtime_error("latent_norm_cache: rotated dimensions must be even and fit the rotated part");
-  DISPATCH_T(dt, T, DISPATCH_T(rot ? dq : 1, TQ, (latent_norm_cache_kernel<T, TQ><<<T_, rot ? 256 : 64, 0, st>>>(
-      (const T*)src, ld, off, (const T*)w, eps, (T*)cache, (const int64_t*)slots, R, rot, rdims, (const float*)cs,
-      (TQ*)qa, (const T*)qsrc, ldq, H, qdim))));
+  const int turns = rot ? H * std::max(rdims / 2, rot - rdims) : 0;  // of a token's queries
+  const int threads = T_ >= 4096 ? 64 : 64 + 64 * std::min(3, (turns + 63) / 64);
+  const int deep = threads > 64 ? (turns + threads - 65) / (threads - 64) : 1;
+#define LATENT_NORM(V_, U_)                                                                                          \
+  DISPATCH_T(dt, T, DISPATCH_T(rot ? dq : 1, TQ, (latent_norm_cache_kernel<T, TQ, V_, U_><<<T_, threads, 0, st>>>(     \
+      (const T*)src, ld, off, (const T*)w, eps, (T*)cache, (const int64_t*)slots, R, rot, rdims, (const float*)cs,   \
+      (TQ*)qa, (const T*)qsrc, ldq, H, qdim))))
+#define LATENT_NORM_U(V_)                  \
+  do {                                     \
+    if (deep > 2) LATENT_NORM(V_, 4);      \
+    else if (deep > 1) LATENT_NORM(V_, 2); \
+    else LATENT_NORM(V_, 1);               \
+  } while (0)
+  if (R <= 64) LATENT_NORM_U(1);
+  else if (R <= 128) LATENT_NORM_U(2);
+  else if (R <= 256) LATENT_NORM_U(4);
+  else LATENT_NORM_U(8);
+#undef LATENT_NORM_U
+#undef LATENT_NORM
   HIP_CHECK_LAUNCH();
 }
 

@@ -51,9 +51,11 @@ def test_rope_rows(T, H, G, dim, vdim, rot, off, dtype, form):
         assert ((cache[:, 0].double() - full).abs() <= flim).all()
 
 
-# latent rows of more numbers than a wave asks for at once, of one and of a few; heads and pairs past whole rounds of three waves; rows that are not cached
+# latent rows of more numbers than a wave asks for at once, of one and of a few; heads and pairs past whole rounds of three waves, or turned by the
+# row's own wave (4096 rows on); rows that are not cached
 @pytest.mark.gpu
-@pytest.mark.parametrize("T,H,R,rot,rdims", [(3, 1, 1, 2, 2), (5, 7, 511, 64, 62), (70, 16, 513, 64, 64), (2, 130, 700, 34, 34), (4, 3, 192, 6, 0), (9, 1, 96, 0, 0)])
+@pytest.mark.parametrize("T,H,R,rot,rdims", [(3, 1, 1, 2, 2), (5, 7, 511, 64, 62), (70, 16, 513, 64, 64), (2, 130, 700, 34, 34), (4, 3, 192, 6, 0), (9, 1, 96, 0, 0),
+                                            (4096, 4, 64, 64, 64), (4097, 43, 130, 8, 6), (4095, 9, 257, 30, 28), (6, 4, 128, 66, 66), (4100, 5, 65, 20, 0), (4, 8, 64, 128, 128)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_latent_rows_and_their_queries(T, H, R, rot, rdims, dtype):
     from llmss_amd.ops import hip
