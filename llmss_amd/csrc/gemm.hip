@@ -1754,8 +1754,12 @@ static bool gemm_slab_plan(int M, int N, int K, int64_t ws_bytes, int* nt_hint, 
 // The four-wave tiles (gemm_four.hip), from 17 rows on, by a price fitted to 60000 measurements of 14 tiles and splits of K over 7500 random
 // products (17 - 8300 rows, 256 - 24000 columns, K of 256 - 12000, with and without gate or activation, weights not in the caches). The
 // choice is 1.2 - 2 % above the best of all. Against the plans before, of the same products: 0.84 of the time at 33 - 48 rows, 0.80 to 64, 0.74
-// to 128, 0.75 to 512, 0.76 to 1024, 0.80 to 2048, 0.84 to 4096, 0.90 above; 17 - 32 rows, where the decode kernel is mostly the better one, 0.97.
-// One in a hundred takes more than 1.02 of it (one in twenty above 2048 rows); at worst 1.4 (22 x 5904 x 8448, 24 us and 34).
+// to 128, 0.75 to 512, 0.76 to 1024, 0.80 to 2048, 0.84 to 4096, 0.90 above; 17 - 32 rows, where the decode kernel is mostly the better one, 0.95.
+// One in a hundred takes more than 1.02 of it (one in twenty above 2048 rows); at worst 1.23 (235 x 15360 x 6400 in slabs, 72 us and 88).
+// Up to 32 rows and to 128 the numbers come from 570 products of their own, K to 12800, every tile and split, plans near the best counting most: with
+// those of all rows a long K was left to too few workgroups. Over 570 others 2.8 and 1.2 % above the best (3.9 and 2.4 before), up to 1.03 and 1.05 of
+// the older plans (1.42 and 1.30); us, older plan, numbers of all rows, now: 25 x 5752 x 7104 22, 30, 21; 32 x 5528 x
+// 11328 32, 48, 32; 121 x 10016 x 7744 48, 57, 45; 122 x 9376 x 10816 gated 58, 75, 59; 66 x 10240 x 11392 gated 54, 70, 58.
 // us of a launch; of a round of workgroups, and what a gate adds; per 64 of k with one
 // workgroup on a CU and with `slots` of them; how much less of that a round takes per CU left idle; the combine of split sums, once and per
 // slice and 128 x 128 tile; bytes per us.
@@ -1763,17 +1767,20 @@ struct FourCost {
   int code, bm, bn, slots;
   double start, round, gate, alone, full, idle, sum, slice, chip;
 };
-static constexpr FourCost kFourFew[] = {  // up to 64 rows: weights are what there is to read
+static constexpr FourCost kFourFew[] = {  // up to 32 rows: weights are what there is to read
+    {1, 32, 64, 2, 1.25, 2.07, 0.18, 0.389, 0.834, 0.648, 1.22, 1.19, 5.50e6}, {8, 64, 32, 2, 0.69, 2.79, 0.30, 0.228, 0.442, 0.413, 1.28, 1.64, 4.64e6},
+    {13, 64, 64, 1, 0.18, 3.89, 0.40, 0.370, 0.352, 0.542, 1.45, 0.91, 10.8e6}};
+static constexpr FourCost kFourMore[] = {  // up to 64 rows
     {0, 64, 64, 3, 0.00, 3.52, 0.29, 0.493, 1.411, 0.601, 1.29, 1.30, 5.36e6}, {1, 32, 64, 2, 2.16, 1.49, 0.09, 0.236, 0.512, 0.438, 1.19, 1.88, 4.10e6},
     {8, 64, 32, 2, 0.82, 2.73, 0.00, 0.224, 0.458, 0.395, 1.25, 1.88, 4.05e6}, {10, 64, 128, 2, 0.12, 3.80, 0.82, 0.833, 1.807, 0.704, 1.74, 0.85, 9.91e6},
     {13, 64, 64, 1, 0.38, 3.83, 0.31, 0.378, 0.371, 0.549, 1.33, 1.28, 13.0e6}, {12, 64, 128, 1, 0.00, 4.55, 0.79, 0.792, 0.744, 0.691, 1.79, 0.79, 4.78e6}};
 static constexpr FourCost kFourMid[] = {  // up to 128 rows
-    {0, 64, 64, 3, 2.78, 1.51, 0.31, 0.276, 0.766, 0.353, 1.42, 1.76, 17.1e6},  {1, 32, 64, 2, 1.90, 2.49, 0.09, 0.168, 0.294, 0.227, 1.39, 2.13, 3.22e6},
-    {2, 128, 64, 2, 0.88, 4.00, 0.77, 0.370, 0.876, 0.384, 1.92, 1.15, 3.63e6}, {3, 128, 128, 2, 3.70, 0.00, 1.96, 1.056, 1.918, 0.545, 1.98, 0.99, 3.61e6},
-    {4, 128, 128, 1, 0.00, 5.74, 1.80, 0.675, 0.820, 0.531, 2.09, 0.84, 4.01e6}, {6, 128, 192, 1, 0.00, 6.81, 2.39, 1.007, 1.207, 0.574, 2.16, 0.75, 4.19e6},
-    {8, 64, 32, 2, 1.91, 2.54, 0.00, 0.165, 0.267, 0.190, 1.46, 2.11, 3.13e6},  {10, 64, 128, 2, 0.98, 4.00, 0.72, 0.377, 0.887, 0.386, 1.89, 1.15, 3.57e6},
-    {11, 128, 64, 1, 0.86, 4.58, 0.78, 0.365, 0.426, 0.374, 1.96, 1.06, 3.84e6}, {12, 64, 128, 1, 0.79, 4.68, 0.72, 0.377, 0.445, 0.389, 1.93, 1.07, 3.64e6},
-    {13, 64, 64, 1, 1.17, 3.89, 0.27, 0.229, 0.231, 0.264, 1.56, 1.49, 3.46e6}};
+    {0, 64, 64, 3, 1.10, 2.49, 0.32, 0.390, 1.010, 0.537, 1.41, 1.24, 18.1e6},  {1, 32, 64, 2, 1.33, 2.27, 0.07, 0.216, 0.428, 0.409, 1.31, 1.60, 3.32e6},
+    {2, 128, 64, 2, 0.00, 3.98, 0.78, 0.577, 1.235, 0.598, 2.02, 0.81, 3.91e6}, {3, 128, 128, 2, 0.00, 3.44, 1.87, 1.299, 2.318, 0.585, 2.30, 0.74, 3.92e6},
+    {4, 128, 128, 1, 0.00, 4.88, 1.73, 0.945, 0.891, 0.637, 2.16, 0.70, 4.96e6}, {6, 128, 192, 1, 0.02, 5.93, 2.29, 1.266, 1.277, 0.623, 2.34, 0.64, 4.10e6},
+    {8, 64, 32, 2, 1.12, 2.56, 0.07, 0.198, 0.370, 0.348, 1.37, 1.58, 2.52e6},  {10, 64, 128, 2, 0.51, 3.53, 0.74, 0.614, 1.263, 0.621, 1.97, 0.81, 4.45e6},
+    {11, 128, 64, 1, 0.00, 4.69, 0.75, 0.522, 0.455, 0.557, 1.96, 0.78, 3.70e6}, {12, 64, 128, 1, 0.00, 4.77, 0.67, 0.563, 0.483, 0.589, 1.92, 0.76, 3.73e6},
+    {13, 64, 64, 1, 0.37, 4.05, 0.24, 0.289, 0.258, 0.434, 1.35, 1.27, 3.59e6}};
 static constexpr FourCost kFourMany[] = {
     {0, 64, 64, 3, 3.87, 0.63, 0.23, 0.235, 0.593, 0.231, 1.72, 2.22, 2.76e6},  {1, 32, 64, 2, 2.52, 2.10, 0.03, 0.157, 0.285, 0.178, 1.61, 1.80, 13.5e6},
     {2, 128, 64, 2, 0.82, 4.36, 0.62, 0.300, 0.598, 0.257, 2.59, 1.42, 3.40e6}, {3, 128, 128, 2, 0.00, 4.75, 1.49, 0.689, 0.988, 0.342, 3.48, 1.11, 2.60e6},
@@ -1811,9 +1818,10 @@ static FourPlan gemm_four_price(int M, int N, int K, bool glu, bool slabs, int64
       if (!best.hint || t < best.us) best = FourPlan{(c.code | kFourHint | (s > 1 && !slabs ? 256 : 0)) << 8, s, t};
     }
   };
-  if (M <= 64) {
-    for (const FourCost& c : kFourFew)
-      if (M > 32 || c.bm == 32 || c.code == 8 || c.code == 13) look(c);
+  if (M <= 32) {
+    for (const FourCost& c : kFourFew) look(c);
+  } else if (M <= 64) {
+    for (const FourCost& c : kFourMore) look(c);
   } else if (M <= 128) {
     for (const FourCost& c : kFourMid) look(c);
   } else {

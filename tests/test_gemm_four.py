@@ -134,3 +134,12 @@ def test_closing_products_stay_in_32_bits(M, N, K):
     assert split > 1 or M <= 32  # (up to 32 rows the decode kernel's, unsplit)
     if split > 1:
         assert H.lib().gemm_partial_slabs(M, N, K, False, False, 0, nt, split, 64 << 20) == split
+
+
+@pytest.mark.parametrize("M,N,K,glu", [(32, 5528, 11328, False), (25, 5752, 7104, False), (28, 5760, 6976, False), (66, 10240, 11392, True),
+                                       (121, 10016, 7744, False), (80, 10568, 7744, False)])
+def test_long_products_of_few_tiles_split_k(M, N, K, glu):
+    """87 - 168 tiles with 100 - 180 steps of K each leave half of the CUs idle and took 1.2 - 1.5 times as long as with K split."""
+    nt, _ = H.lib().gemm_plan(M, N, K, False, glu, False)
+    bm, bn = TILES[nt >> 8 & 15]
+    assert nt >> 8 & FOUR and (nt >> 8 & COMBINE or -(-M // bm) * -(-N // bn) >= 192)
