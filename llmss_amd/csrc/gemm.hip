@@ -2001,23 +2001,20 @@ static void gemm_default_plan(int M, int N, int K, bool w_fp8, bool glu, bool sl
 static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int nt_hint, int split_hint, int64_t ws_bytes);
 
 // Where to cut a product of 256 x 256 tiles whose last wave is mostly empty in two launches: the tiles of whole waves, and the rows or
-// columns left over, which smaller tiles spread over the chip. Waves cost what gemm_static_plan has measured, but one that is at most
-// 0.8 full only 0.78 of it (0.6 - 0.94 over eleven shapes: the clock rises as tiles end); up to 64 rows left over read all weights at
-// 4.5 TB/s behind 8 us. us, one launch and two: 1773 x 12288 x 4096 172 -> 151 (predicted 174 and 155), SwiGLU x 22016 280 -> 266,
-// 8261 x 2048 x 2048 91 -> 61, 8261 x 6400 x 2048 190 -> 174, 3999 x 22016 x 4096 570 -> 551. Left whole, as predicted: 8192 x 5120 x 2048
-// (2.5 waves) 141 and 143, 8192 x 9472 x 2048 (4.6) 255 and 255, 5000 x 12288 x 4096 (3.75) 359 and 357. Over 3286 random products that it
-// cuts, 257 - 10000 rows and whole steps of k, two launches take 0.886 of the time from K = 1024 on, 1.11 at worst. Below, a tile's start and end
-// are half of it, and what is promised up to there does not come: gated products 0.87 (0.98 at worst), others 0.954 where more than 6.5 % are
-// promised (95 products; 1.15 at worst, all of those at 6.5 - 10 %: 3764 x 5664 x 256 27 -> 31), 1.02 where less, so those stay whole.
-// The rest's tiles can be too few for the chip (69 x 2048: 32 of 64 x 128, each alone with all of K): K is split where that is priced a tenth
-// below the best of the tiles looked at before, as in gemm_static_plan, up to 24 MB of slabs. The cut may then lie elsewhere than without splits, but
-// not where that would leave up to 64 rows, whose price is too high (4106 x 15840 x 11520, ten rows left or 480 columns 1110 and 1180 us).
-// Over 552 random products that a split changes, 257 - 10000 rows, 0.953 of the time without, five above 1.01, 1.025 at worst (2579 x 7120 x 8576):
-// 8261 x 2048 x 4096 152 -> 132 us, x 2560 100 -> 91, 1240 x 13248 x 3392 133 -> 118.
+// columns left over, which smaller tiles spread over the chip. What the launches run with is gemm_rest_plan's; where the cut lies is priced with
+// numbers of the kernels before them (kTileCost; waves that are at most 0.8 full cost only 0.78: the clock rises as tiles end; up to 64 rows left over
+// read all weights at 4.5 TB/s behind 8 us), and those places still hold: over 204 random products that it cuts, 257 - 10000 rows and whole steps of
+// k, two launches take 0.888 of the time of one, 1.03 at worst, two of them above 1.02 (K from 1024 on 0.869, 1.01 at worst; below 0.934). us, one
+// launch and two: 1773 x 12288 x 4096 186 and 157, SwiGLU x 22016 277 and 263, 8261 x 2048 x 2048 86 and 61, x 4096 163 and 108, 8261 x 6400 x 2048
+// 192 and 179, 3999 x 22016 x 4096 561 and 541. Left whole: 8192 x 5120 x 2048 (2.5 waves) 145, 8192 x 9472 x 2048 (4.6) 249, 5000 x 12288 x 4096
+// (3.75) 373.
+// Below K = 1024 a tile's start and end are half of it, and what is promised up to there does not come: ungated products are cut there where more than
+// 6.5 % are promised, others from 3 % on.
+// The rest's tiles can be too few for the chip (69 x 2048): a split of K, priced a tenth below the best of the tiles looked at before, up to 24 MB of
+// sums, lets the cut lie elsewhere, but not where that would leave up to 64 rows, whose price is too high (4106 x 15840 x 11520, ten rows left or 480
+// columns 1110 and 1180 us). 1240 x 13248 x 3392 140 us in one launch and 104 in two, 2579 x 7120 x 8576 335 and 262.
 struct GemmCut {
   int rows, cols;  // of the first launch; 0: not cut
-  int hint;        // plan of the second (0: the plan of its size)
-  int split;       // of its K
 };
 static GemmCut gemm_cut(int M, int N, int K, bool glu, int64_t ws_bytes) {
   const int ntm = (M + 255) / 256, ntn = (N + 255) / 256, nk = (K + 63) / 64;
@@ -2029,7 +2026,8 @@ static GemmCut gemm_cut(int M, int N, int K, bool glu, int64_t ws_bytes) {
     t = std::max(t, (2.0 * n * K + 2.0 * m * K + 2.0 * m * (glu ? n / 2 : n)) / 4.0e6);
     return split > 1 ? t + 4.0 + 8.0 * split * m * n / 4.5e6 : t;
   };
-  GemmCut cut{0, 0, 0, 1};
+  GemmCut cut{0, 0};
+  bool few = false;  // (up to 64 rows left over)
   double best = (K < 1024 && !glu ? 0.935 : 0.97) * tiles_us(kTileCost[0], M, N);
   auto consider = [&](int rows, int cols, bool splits) {
     if (rows <= 0 || cols <= 0 || (rows >= M && cols >= N)) return;
@@ -2037,17 +2035,17 @@ static GemmCut gemm_cut(int M, int N, int K, bool glu, int64_t ws_bytes) {
     if (last && last < 218) return;  // whole waves, the last of them at least 0.85 full
     const int m = rows < M ? M - rows : M, n = cols < N ? N - cols : N;
     double rest = 8.0 + 2.0 * n * K / 4.5e6;
-    int hint = 0, split = 1;
+    int split = 0;
     for (const TileCost& c : kTileCost) {
       if (m <= 64) break;
       for (int s : {1, 2, 3, 4, 6, 8}) {
         if (s > 1 && (!splits || c.tsel == 4 || K / s < 256 || (int64_t)s * m * n * 4 > std::min<int64_t>(ws_bytes, 24 << 20))) break;
         const double t = tiles_us(c, m, n, s);
-        if (!hint || t < (s > split ? 0.9 : 1.0) * rest) rest = t, hint = c.tsel << 8, split = s;
+        if (!split || t < (s > split ? 0.9 : 1.0) * rest) rest = t, split = s;
       }
     }
     const double t = tiles_us(kTileCost[0], std::min(rows, M), std::min(cols, N)) + rest;
-    if (t < best) best = t, cut = GemmCut{rows < M ? rows : 0, cols < N ? cols : 0, hint, split};
+    if (t < best) best = t, few = m <= 64, cut = GemmCut{rows < M ? rows : 0, cols < N ? cols : 0};
   };
   const int waves = (int)std::min<int64_t>((int64_t)ntm * ntn / 256, 64);
   for (bool splits : {false, true}) {
@@ -2056,15 +2054,15 @@ static GemmCut gemm_cut(int M, int N, int K, bool glu, int64_t ws_bytes) {
       consider(M, 256 * w / ntm * 256, splits);
     }
     consider((ntm - 1) * 256, N, splits);
-    if (cut.rows && !cut.hint) break;
+    if (cut.rows && few) break;
   }
   return cut;
 }
 
 // What the second launch runs with: four-wave tiles from 65 rows on, else the plan of its size (hint 0)
-static FourPlan gemm_rest_plan(const GemmCut& cut, int m, int n, int K, bool glu, int64_t ws_bytes) {
+static FourPlan gemm_rest_plan(int m, int n, int K, bool glu, int64_t ws_bytes) {
   const FourPlan p = m > 64 ? gemm_four_plan(m, n, K, glu, false, ws_bytes) : FourPlan{0, 0, 0.0};
-  return p.hint ? p : FourPlan{cut.hint, cut.hint ? cut.split : 0, 8.0 + 2.0 * n * K / 4.5e6};
+  return p.hint ? p : FourPlan{0, 0, 8.0 + 2.0 * n * K / 4.5e6};
 }
 
 // 256 x 256 tiles, cut or whole
@@ -2072,7 +2070,7 @@ static double quad_us(int M, int N, int K, bool glu, int64_t ws_bytes) {
   const GemmCut cut = gemm_cut(M, N, K, glu, ws_bytes);
   if (!cut.rows && !cut.cols) return four_us(kQuadCost, M, N, K, glu, 1);
   const int rows = cut.rows ? cut.rows : M, cols = cut.cols ? cut.cols : N;
-  return four_us(kQuadCost, rows, cols, K, glu, 1) + gemm_rest_plan(cut, rows < M ? M - rows : M, cols < N ? N - cols : N, K, glu, ws_bytes).us;
+  return four_us(kQuadCost, rows, cols, K, glu, 1) + gemm_rest_plan(rows < M ? M - rows : M, cols < N ? N - cols : N, K, glu, ws_bytes).us;
 }
 
 int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_fp8, const void* w_scale,
@@ -2087,13 +2085,13 @@ int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_f
     const GemmCut cut = gemm_cut(M, N, K, glu, ws_bytes);
     if (cut.rows) {
       launch_gemm(x, ldx, w, ldw, false, nullptr, bias, y, ldy, cut.rows, N, K, act, glu, workspace, ws_bytes, 4 << 8, 1, false, st);
-      const FourPlan rest = gemm_rest_plan(cut, M - cut.rows, N, K, glu, ws_bytes);
+      const FourPlan rest = gemm_rest_plan(M - cut.rows, N, K, glu, ws_bytes);
       return launch_gemm((const bf16_t*)x + cut.rows * ldx, ldx, w, ldw, false, nullptr, bias, (bf16_t*)y + cut.rows * ldy, ldy,
                          M - cut.rows, N, K, act, glu, workspace, ws_bytes, rest.hint, rest.split, false, st);
     }
     if (cut.cols) {
       launch_gemm(x, ldx, w, ldw, false, nullptr, bias, y, ldy, M, cut.cols, K, act, glu, workspace, ws_bytes, 4 << 8, 1, false, st);
-      const FourPlan rest = gemm_rest_plan(cut, M, N - cut.cols, K, glu, ws_bytes);
+      const FourPlan rest = gemm_rest_plan(M, N - cut.cols, K, glu, ws_bytes);
       return launch_gemm(x, ldx, (const bf16_t*)w + cut.cols * ldw, ldw, false, nullptr, bias ? (const bf16_t*)bias + cut.cols : nullptr,
                          (bf16_t*)y + (glu ? cut.cols / 2 : cut.cols), ldy, M, N - cut.cols, K, act, glu, workspace, ws_bytes, rest.hint,
                          rest.split, false, st);
@@ -2582,7 +2580,7 @@ int launch_gemm_qkv(const void* x, int64_t ldx, const void* w, int64_t ldw, cons
     const bf16_t* rw = (const bf16_t*)w + (cols < N ? (int64_t)cols * ldw : 0);
     const bf16_t* rb = bias ? (const bf16_t*)bias + (cols < N ? cols : 0) : nullptr;
     const int m = rows < M ? M - rows : M, n = cols < N ? N - cols : N;
-    const FourPlan rest = gemm_rest_plan(cut, m, n, K, false, ws_bytes);
+    const FourPlan rest = gemm_rest_plan(m, n, K, false, ws_bytes);
     int nt = rest.hint, sp = 1;
     if (!nt) {  // up to 64 rows: the decode kernel where its plan is unsplit, else 64 x 64 tiles
       gemm_static_plan(m, n, K, false, false, ws_bytes, &nt, &sp);
@@ -2618,7 +2616,7 @@ void gemm_cut_of(int M, int N, int K, bool glu, int* rows, int* cols, int* split
   const GemmCut c = gemm_cut(M, N, K, glu, 64 << 20);
   *rows = c.rows;
   *cols = c.cols;
-  *split = c.split;
+  *split = c.rows || c.cols ? std::max(1, gemm_rest_plan(c.rows ? M - c.rows : M, c.cols ? N - c.cols : N, K, glu, 64 << 20).split) : 1;
 }
 
 // The plan of a product whose result goes straight into an op that can sum its slabs: a split one, the slabs unsummed, where the older rules

@@ -352,7 +352,7 @@ def test_gemm_mid_k_tail_reads_nothing_past_the_operands(tile):
 
 @pytest.mark.parametrize("M,N,K,glu,act", [(1773, 12288, 256, False, "none"), (1773, 22016, 1024, True, "none"), (8261, 2048, 512, False, "gelu_tanh"),
                                            (8193, 2048, 1024, False, "relu"), (8261, 6400, 1024, False, "none"), (8261, 2048, 1024, True, "none"),
-                                           (8256, 2056, 2048, False, "none")])
+                                           (8256, 2056, 2048, False, "none"), (964, 16576, 2112, True, "none"), (3558, 9344, 3008, False, "none")])
 def test_products_cut_in_two_launches(M, N, K, glu, act):
     """Products of 256 x 256 tiles whose last wave is nearly empty: whole waves and what is left over, by rows or columns, with bias
     and activation on either side, into strided rows; what lies around the output stays as it is."""
@@ -370,10 +370,10 @@ def test_products_cut_in_two_launches(M, N, K, glu, act):
 
 
 @pytest.mark.parametrize("M,N,K,glu,act,bias", [(8261, 2048, 2048, False, "gelu", True), (1240, 13248, 3392, False, "none", True),
-                                                (964, 16576, 2112, True, "none", True), (3558, 9344, 3008, False, "none", False)])
+                                                (803, 16512, 3200, True, "none", True), (8261, 2048, 4096, False, "none", False)])
 def test_rest_of_a_cut_product_splits_k(M, N, K, glu, act, bias):
-    """The rest of a product that is cut in two launches, with few tiles: K split in slabs of 32-bit sums, bias, activation and gate after
-    their sum; strided rows, what lies around them stays. Each side's error is a rounding of the result in bf16 and of 32-bit sums."""
+    """The rest of a product that is cut in two launches, with few tiles: the second launch's K split, its 32-bit sums combined there, bias,
+    activation and gate after their sum; strided rows, what lies around them stays. Each side's error is a rounding of the result in bf16 and of 32-bit sums."""
     torch.manual_seed(0)
     x, w, b = rnd(M, K + 8)[:, :K], rnd(N, K, scale=K ** -0.5), rnd(N, scale=0.1) if bias else None
     n = N // 2 if glu else N

@@ -138,10 +138,11 @@ def test_products_are_cut_where_the_last_wave_of_tiles_is_nearly_empty(M, N, K, 
 
 
 @pytest.mark.parametrize("M,N,K,cut,split", [(4106, 15840, 11520, (4096, 0), 1), (6662, 7264, 8448, (6656, 0), 1), (6161, 15888, 10688, (6144, 0), 1),
-                                             (8261, 2048, 4096, (8192, 0), 4), (4317, 3952, 9216, (0, 3840), 3), (6851, 2336, 8704, (0, 2304), 2)])
+                                             (8261, 2048, 4096, (8192, 0), 4), (4317, 3952, 9216, (0, 3840), 3), (6851, 2336, 8704, (0, 2304), 4)])
 def test_split_rests_cut_elsewhere_only_beside_more_than_64_rows(M, N, K, cut, split):
-    """The rest of a cut product may split K, and the product be cut where that pays; but up to 64 rows left over, which are priced
-    above what they take, stay where they are (1110 us against 1180 for the first, 631 and 660, 1858 and 1907)."""
+    """The rest of a cut product may split K (``split``: of the launch that it gets, by the plan of its size), and the product be cut where that
+    pays; but up to 64 rows left over, which are priced above what they take, stay where they are (1110 us against 1180 for the first, 631 and
+    660, 1858 and 1907)."""
     from llmss_amd.ops import hip as H
 
     assert tuple(H.lib().gemm_cut(M, N, K, False)) == cut and H.lib().gemm_cut_split(M, N, K, False) == split
