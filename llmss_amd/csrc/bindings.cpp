@@ -51,6 +51,7 @@ int launch_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, bool w_f
 void gemm_plan(int M, int N, int K, bool w_fp8, bool glu, bool slabs, int* nt, int* splitk, bool four = true);
 void gemm_closing_plan(int M, int N, int K, int* nt, int* splitk);
 void gemm_cut_of(int M, int N, int K, bool glu, int* rows, int* cols, int* split);
+int64_t gemm_priced();
 void gemm_tuned_set(int M, int N, int K, bool glu, int kind, int nt_hint, int split);
 void gemm_tuned_clear();
 void gemm_reserve_streamk(int n);
@@ -372,6 +373,7 @@ PYBIND11_MODULE(_C, m) {
     gemm_closing_plan(M, N, K, &nt, &s);
     return py::make_tuple(nt, s);
   });
+  m.def("gemm_priced", &gemm_priced);  // plans and cuts that this thread has priced, and not found among its last ones
   m.def("gemm_cut", [](int M, int N, int K, bool glu) {  // rows or columns of the first of two launches, 0: one launch
     int rows, cols, split;
     gemm_cut_of(M, N, K, glu, &rows, &cols, &split);

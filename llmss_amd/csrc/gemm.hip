@@ -1830,21 +1830,41 @@ static FourPlan gemm_four_price(int M, int N, int K, bool glu, bool slabs, int64
   return best;
 }
 
-// slabs: split sums are left to the consumer. A thread keeps its last prices by size (they depend on nothing else): 40 - 84 of them take 0.5 - 0.9 us,
-// more than the launch that they are for leaves where a step of few rows waits for the host.
-static FourPlan gemm_four_plan(int M, int N, int K, bool glu, bool slabs, int64_t ws_bytes) {
-  if (M < 17 || N % 8 || K % 64) return FourPlan{0, 1, 0.0};
-  struct Kept {
+// A thread's last answers by size, which depend on nothing else: 64 sets of four, of which the oldest makes room. 40 - 84 prices take 0.5 - 0.9 us and a
+// cut 1 - 3, and a product is planned two or three times, more than the launch that it is for leaves where a step of few rows waits for the host.
+// (64 single places, by the exclusive or of three products: two sizes met at every number of rows or at none, GPT-2 XL's 4800 x 1600 and 6400 x 1600 at
+// every one, so that its four sizes in turn took 0.77 us a plan, now 0.32; 8260 x 10240 x 2048 with its cut 2.7, now 0.41.)
+static thread_local int64_t g_priced = 0;
+int64_t gemm_priced() { return g_priced; }
+template <typename V>
+struct BySize {
+  struct Entry {
     int M, N, K, kind;
     int64_t ws;
-    FourPlan plan;
+    V value;
   };
-  static thread_local Kept kept[64] = {};
-  const int kind = glu | slabs << 1;
-  Kept& p = kept[((uint32_t)M * 0x9e3779b1u ^ (uint32_t)N * 0x85ebca6bu ^ (uint32_t)K * 0xc2b2ae35u ^ (uint32_t)kind << 26) >> 26];
-  if (p.M != M || p.N != N || p.K != K || p.kind != kind || p.ws != ws_bytes)
-    p = Kept{M, N, K, kind, ws_bytes, gemm_four_price(M, N, K, glu, slabs, ws_bytes)};
-  return p.plan;
+  Entry of[64][4] = {};
+  uint8_t oldest[64] = {};
+  template <typename F>
+  V get(int M, int N, int K, int kind, int64_t ws, F make) {
+    uint32_t h = (uint32_t)M * 0x9e3779b1u;
+    h = (h ^ h >> 15 ^ (uint32_t)N) * 0x85ebca6bu;
+    h = (h ^ h >> 15 ^ (uint32_t)K << 2 ^ (uint32_t)kind) * 0xc2b2ae35u;
+    h >>= 26;
+    for (const Entry& e : of[h])
+      if (e.M == M && e.N == N && e.K == K && e.kind == kind && e.ws == ws) return e.value;
+    ++g_priced;
+    const V value = make();
+    of[h][oldest[h]++ & 3] = Entry{M, N, K, kind, ws, value};
+    return value;
+  }
+};
+
+// slabs: split sums are left to the consumer
+static FourPlan gemm_four_plan(int M, int N, int K, bool glu, bool slabs, int64_t ws_bytes) {
+  if (M < 17 || N % 8 || K % 64) return FourPlan{0, 1, 0.0};
+  static thread_local BySize<FourPlan> kept;
+  return kept.get(M, N, K, glu | slabs << 1, ws_bytes, [&] { return gemm_four_price(M, N, K, glu, slabs, ws_bytes); });
 }
 
 // slabs: the consumer sums split-K slabs itself and so gets the product in 32 bits. Where the older rules split K that stays so:
@@ -2016,7 +2036,7 @@ static int slabs_of_plan(int M, int N, int K, bool w_fp8, bool glu, int act, int
 struct GemmCut {
   int rows, cols;  // of the first launch; 0: not cut
 };
-static GemmCut gemm_cut(int M, int N, int K, bool glu, int64_t ws_bytes) {
+static GemmCut gemm_cut_place(int M, int N, int K, bool glu, int64_t ws_bytes) {
   const int ntm = (M + 255) / 256, ntn = (N + 255) / 256, nk = (K + 63) / 64;
   auto tiles_us = [&](const TileCost& c, int m, int n, int split = 1) {
     const int slots = 256 * c.per_cu, wgs = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn) * split, rest = wgs % slots;
@@ -2057,6 +2077,11 @@ static GemmCut gemm_cut(int M, int N, int K, bool glu, int64_t ws_bytes) {
     if (cut.rows && few) break;
   }
   return cut;
+}
+
+static GemmCut gemm_cut(int M, int N, int K, bool glu, int64_t ws_bytes) {
+  static thread_local BySize<GemmCut> kept;
+  return kept.get(M, N, K, glu, ws_bytes, [&] { return gemm_cut_place(M, N, K, glu, ws_bytes); });
 }
 
 // What the second launch runs with: four-wave tiles from 65 rows on, else the plan of its size (hint 0)

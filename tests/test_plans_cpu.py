@@ -262,3 +262,24 @@ def test_closing_products_keep_a_tuned_plan(nt, split):
     finally:
         H.lib().gemm_tuned_clear()
     assert tuple(H.lib().gemm_closing_plan(M, N, K)) == static
+
+
+@pytest.mark.parametrize("sizes", [[(4800, 1600), (1600, 1600), (6400, 1600), (1600, 6400)], [(12288, 4096), (4096, 4096), (22016, 4096), (4096, 11008)],
+                                   [(10240, 2048), (2048, 4096), (11264, 2048), (2048, 5632), (2048, 2048), (4352, 2048)]])
+def test_prices_of_a_model_are_kept_at_every_number_of_rows(sizes):
+    """A step plans every size several times, layer by layer: none may take another's place, whatever the number of rows."""
+    from llmss_amd.ops import hip as H
+
+    L = H.lib()
+
+    def walk(M):
+        for N, K in sizes:
+            L.gemm_plan(M, N, K, False, False, False)
+            L.gemm_plan(M, N, K, False, False, True)
+            L.gemm_plan(M, N, K, False, True, False)
+
+    for M in list(range(17, 1100)) + list(range(1101, 9000, 97)):
+        walk(M)
+        before = L.gemm_priced()
+        walk(M)
+        assert L.gemm_priced() == before, M
