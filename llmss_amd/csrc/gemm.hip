@@ -2249,25 +2249,33 @@ static constexpr int kSlots = 4;
 static thread_local int g_ws_slot = 0;
 void gemm_set_slot(int s) { g_ws_slot = s & (kSlots - 1); }
 
-// `capturing`: the stream of the launch; where it is being captured and the counters are not there yet, null is returned
-static int* sk_counters(int n, const hipStream_t* capturing = nullptr) {
+// `on`: the stream of a launch by its own rules. Where it is being captured and the counters are not there yet, null is returned; else they are made
+// on it, so that another thread's capture is not disturbed (an allocation under the strict mode, or a wait for the device, would end it).
+static int* sk_counters(int n, const hipStream_t* on = nullptr) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) throw std::runtime_error("gemm counters: bad device");
   std::lock_guard<std::mutex> lk(g_sk_mu);
   if (n <= g_sk_capacity[dev]) return g_sk_counters[dev] + (size_t)g_ws_slot * g_sk_capacity[dev];
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (capturing) {
-    (void)hipStreamIsCapturing(*capturing, &cs);
-    if (cs != hipStreamCaptureStatusNone) return nullptr;
-  }
-  (void)hipStreamIsCapturing(nullptr, &cs);
-  if (cs != hipStreamCaptureStatusNone) throw std::runtime_error("gemm counters must be allocated before capture");
   int cap = std::max(n, 1 << 16);
   int* p = nullptr;
   const size_t bytes = (size_t)cap * kSlots * sizeof(int);
-  if (hipMalloc(&p, bytes) != hipSuccess) throw std::runtime_error("gemm counters: hipMalloc");
-  if (hipMemset(p, 0, bytes) != hipSuccess) throw std::runtime_error("gemm counters: memset");
-  (void)hipDeviceSynchronize();
+  if (on) {
+    (void)hipStreamIsCapturing(*on, &cs);
+    if (cs != hipStreamCaptureStatusNone) return nullptr;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const bool made = hipMalloc(&p, bytes) == hipSuccess && hipMemsetAsync(p, 0, bytes, *on) == hipSuccess &&
+                      hipStreamSynchronize(*on) == hipSuccess;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!made) throw std::runtime_error("gemm counters: not allocated");
+  } else {
+    (void)hipStreamIsCapturing(nullptr, &cs);
+    if (cs != hipStreamCaptureStatusNone) throw std::runtime_error("gemm counters must be allocated before capture");
+    if (hipMalloc(&p, bytes) != hipSuccess) throw std::runtime_error("gemm counters: hipMalloc");
+    if (hipMemset(p, 0, bytes) != hipSuccess) throw std::runtime_error("gemm counters: memset");
+    (void)hipDeviceSynchronize();
+  }
   g_sk_counters[dev] = p;  // the old (smaller) buffer is left to the process: launches may still reference it
   g_sk_capacity[dev] = cap;
   return p + (size_t)g_ws_slot * cap;

@@ -96,7 +96,7 @@ def test_rotation_and_cache_write(code, style, D, rot):
 
 @gpu
 @pytest.mark.parametrize("M,N,K", [(40, 384, 1920), (200, 1024, 8192)])
-def test_first_use_under_capture(M, N, K):
+def test_replays_among_eager_launches(M, N, K):
     """A plan that combines split sums in the launch, replayed among eager launches of the same product."""
     assert H.lib().gemm_plan(M, N, K, False, False, False)[0] >> 8 & (FOUR | COMBINE) == FOUR | COMBINE
     x, w = rand(10, M, K), rand(11, N, K) * K ** -0.5
