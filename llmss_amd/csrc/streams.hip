@@ -324,7 +324,10 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(const TI* __restrict__
 // channels of them (four: 16-byte reads of fp32 rows), so an input is read once (plus the rows before the strip)
 // instead of once per tap. The rows are loaded up front, all loads in flight together; the strip's place in its
 // sequence is found once and walked from there (looked up again where a sequence ends). Taps are added in the order
-// of the kernel above: the same numbers bit for bit. RMAX: the most rows back that a tap may reach (taps - 1).
+// of the kernel above: the same numbers bit for bit. RMAX: the most rows back that a tap may reach (taps - 1). WITHIN: strips within one portion
+// have a form of their own: bf16 rows, taps = RMAX + 1, portions of 32 rows and more on average. It takes up to 18 more registers (nine taps: three
+// waves a SIMD for four), which six to eight taps and short portions would pay for nothing: 6000 rows of 4096, seven taps, 47 us and 50 with it, 400
+// portions of 20 rows, nine taps, 75 and 80. Over 48 sizes each, of portions of 24 rows 0.994 of the time with it, of 40 0.987, of 64 0.968, of 200 0.962.
 #define CONV_STRIP 16
 template <typename T, int CH>
 __device__ __forceinline__ void conv_ld(const T* p, float* v) {
@@ -383,7 +386,7 @@ __device__ __forceinline__ void conv_st(T* p, const float* v) {
   }
 }
 
-template <typename TI, typename TW, typename TO, int RMAX, int CH>
+template <typename TI, typename TW, typename TO, int RMAX, int CH, bool WITHIN>
 __global__ __launch_bounds__(256) void causal_conv_strip_kernel(const TI* __restrict__ in, int64_t ldi,
                                                                 const TW* __restrict__ w,
                                                                 const float* __restrict__ state,
@@ -418,8 +421,9 @@ __global__ __launch_bounds__(256) void causal_conv_strip_kernel(const TI* __rest
   }
   RowSeq r = row_seq(cu, ctx, B, t0);
   // A strip within one portion, with all that it reaches back to: most of a prompt's, and then without a question for each row and tap. Rows of
-  // 4096 in bf16 45 -> 39 us (8260 rows), out in fp32 63 -> 58 (8192); of 2048 in fp32 25 and 27, which stay with the questions.
-  if (sizeof(TI) == 2 && R == RMAX && r.j >= RMAX && r.pos >= r.j && r.j + CONV_STRIP <= r.qlen) {
+  // 4096 in bf16 45 -> 39 us (8260 rows); of 2048 in fp32 25 and 27, which stay with the questions. 1000 and 8000 rows of 256 - 8192, two to nine taps, 0.86 -
+  // 0.99.
+  if (WITHIN && r.j >= RMAX && r.pos >= r.j && r.j + CONV_STRIP <= r.qlen) {
     float v[RMAX + 1][CH];  // [d]: the input d rows back
 #pragma unroll
     for (int d = 1; d <= RMAX; ++d) conv_of<TI, CH>(xr[RMAX - d], v[d]);
@@ -601,10 +605,16 @@ static void causal_conv_t(const void* in, int64_t ldi, const void* w, void* stat
   if (!single && T_ >= 256 && T_ >= 8 * B && taps <= 9) {  // portions of eight rows and more on average
     const auto al16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
     const bool four = C % 4 == 0 && ldi % 4 == 0 && ldo % 4 == 0 && al16(in) && al16(out) && al16(state);
-#define LAUNCH_STRIP(RMAX_, CH_)                                                                                    \
-  causal_conv_strip_kernel<TI, TW, TO, RMAX_, CH_><<<g, 256, 0, st>>>(                                              \
+    const bool within = sizeof(TI) == 2 && T_ >= 32 * B;
+#define LAUNCH_STRIP1(RMAX_, CH_, WITHIN_)                                                                          \
+  causal_conv_strip_kernel<TI, TW, TO, RMAX_, CH_, WITHIN_><<<g, 256, 0, st>>>(                                     \
       (const TI*)in, ldi, (const TW*)w, (const float*)state, (const int*)cu, (const int*)ctx, (const int*)sslots,   \
       (TO*)out, ldo, B, C, taps, res, silu, T_, (const TW*)bias)
+#define LAUNCH_STRIP(RMAX_, CH_)                                                                                    \
+  do {                                                                                                              \
+    if (within && taps == RMAX_ + 1) LAUNCH_STRIP1(RMAX_, CH_, (sizeof(TI) == 2));                                  \
+    else LAUNCH_STRIP1(RMAX_, CH_, false);                                                                          \
+  } while (0)
     if (four) {
       dim3 g((T_ + CONV_STRIP - 1) / CONV_STRIP, (C / 4 + 255) / 256);
       if (taps <= 2) LAUNCH_STRIP(1, 4);
@@ -617,6 +627,7 @@ static void causal_conv_t(const void* in, int64_t ldi, const void* w, void* stat
       else LAUNCH_STRIP(8, 1);
     }
 #undef LAUNCH_STRIP
+#undef LAUNCH_STRIP1
   } else {
     dim3 g(T_, (C + 256 * CONV_CPT - 1) / (256 * CONV_CPT));
     causal_conv_kernel<TI, TW, TO><<<g, 256, 0, st>>>((const TI*)in, ldi, (const TW*)w, (float*)state,

@@ -55,10 +55,12 @@ def test_single_rows(device, dtype, out_dtype, residual, bias, silu, C, taps):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,out_dtype", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("residual,bias,silu", [(True, False, False), (False, True, True)])
-@pytest.mark.parametrize("C,taps", [(40, 4), (1032, 9), (12, 2), (70, 3)])
-def test_strips_of_portions(dtype, out_dtype, residual, bias, silu, C, taps):
+@pytest.mark.parametrize("C,taps", [(40, 4), (1032, 9), (12, 2), (70, 3), (12, 5), (40, 7), (70, 4)])
+# strips from 256 rows on; that for strips within one portion in bf16, of 2, 4, 5 and 9 taps
+@pytest.mark.parametrize("lens", [[19, 100, 1, 16, 40, 35], [59, 100, 1, 26, 40, 35], [119, 300, 1, 16, 40, 35], [32, 200, 1, 16, 96, 39]])
+def test_strips_of_portions(dtype, out_dtype, residual, bias, silu, C, taps, lens):
     gen = torch.Generator().manual_seed(C + taps)
-    lens, first, slots = [19, 100, 1, 16, 40, 35], [0, 7, 2, 0, 3, 0], [4, 0, 1, 2, -1, 5]
+    first, slots = [0, 7, 2, 0, 3, 0], [4, 0, 1, 2, -1, 5]
     T, R = sum(lens), taps - 1
     x = torch.randn(T, C, generator=gen).to(dtype)
     w, b = (torch.randn(C, taps, generator=gen) * taps ** -0.5).to(dtype), torch.randn(C, generator=gen).to(dtype)
