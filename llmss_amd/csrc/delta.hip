@@ -849,7 +849,11 @@ __global__ __launch_bounds__(256, 3) void delta_prep32_kernel(DeltaChunk32Args A
 // Bound by the chain of a chunk's products, reads and barriers: of 14.3 us a chunk the fp32 matrix instructions took 6.2, now of 12.0 (8 x 1024
 // tokens, 16 heads of 128 x 128, 229 -> 192 us). NH = 2 (keys of more than 32): two waves a SIMD, 8 a workgroup; two share 16 columns, each with half of the state's rows (its part of K S and Q S over those; its rows of the update) and
 // two of the four blocks of tokens (0 and 3, 1 and 2: five products each with X and with P). Parts of sums, u and U change hands through LDS.
-template <int KT, int NH>
+// ANEW: every chunk forms its places anew. Kept through the loop they take what registers are left, and at keys of up to 32 and beyond 64 six and nine
+// of them in scratch. A long chain of chunks is still the faster one with them kept (us, kept and anew: one portion of 4096, 8 heads, keys of 32 384
+// and 412, of 128 681 and 707; 16 of 256, 32 x 128 82.8 and 83.4), portions of one or two are not (64 of 64, 16 heads of 32 x 128 97 and 90, of 128
+// x 128 172 and 166; 100 of 40, 32 x 256 178 and 165; 64 of 24, 128 x 128 125 and 120); keys of 64, with none in scratch, 1 % slower anew.
+template <int KT, int NH, bool ANEW>
 __global__ __launch_bounds__(256 * NH, KT <= 2 ? 2 : 1) void delta_chunk32_kernel(DeltaChunk32Args A) {
   constexpr int C = 64, DKP = 16 * KT, LDK = DKP + 4, LDP = 64 + 4, KO = KT / NH, TH = 256 * NH;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -864,7 +868,7 @@ __global__ __launch_bounds__(256 * NH, KT <= 2 ? 2 : 1) void delta_chunk32_kerne
   const int dim = A.dim, vdim = A.vdim, H = A.H, gq = h / (H / A.G);
   const int t0 = A.cu[b], qlen = A.cu[b + 1] - t0, slot = A.sslots[b], ctx = A.ctx[b];
   if (qlen <= 0) return;
-  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
+  int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3, hf = wave >> 2;
   const int col = blockIdx.y * 64 + 16 * w + li, colc = min(col, vdim - 1);
   float* outp = A.out + (int64_t)t0 * H * vdim + (int64_t)h * vdim + col;
@@ -913,6 +917,11 @@ __global__ __launch_bounds__(256 * NH, KT <= 2 ? 2 : 1) void delta_chunk32_kerne
   auto chunk = [&](int j0, auto all_c) {
     constexpr bool ALL = decltype(all_c)::value;
     const int nt = ALL ? C : min(C, qlen - j0), nb = ALL ? 4 : (nt + 15) >> 4;
+    if constexpr (ANEW) {
+      tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));
+      lane = tid & 63, li = lane & 15, g = lane >> 4;
+    }
     __syncthreads();  // the previous chunk's readers are done
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
@@ -1120,13 +1129,14 @@ void launch_delta_chunk32(const void* q, const void* k, const void* v, int64_t l
   do {                                                                                                                \
     static bool once = [] {                                                                                           \
       for (const void* f : {(const void*)delta_prep32_kernel<KT_, bf16_t>, (const void*)delta_prep32_kernel<KT_, float>,\
-                            (const void*)delta_chunk32_kernel<KT_, NH_>})                                             \
+                            (const void*)delta_chunk32_kernel<KT_, NH_, false>, (const void*)delta_chunk32_kernel<KT_, NH_, KT_ != 4>}) \
         (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                         \
       return true;                                                                                                    \
     }();                                                                                                              \
     (void)once;                                                                                                       \
     DISPATCH_T(dp, TP, (delta_prep32_kernel<KT_, TP><<<g1, 256, lds1(KT_), st>>>(A)));                                \
-    delta_chunk32_kernel<KT_, NH_><<<g2, 256 * NH_, lds2(KT_, NH_), st>>>(A);                                         \
+    if (max_qlen <= 128) delta_chunk32_kernel<KT_, NH_, KT_ != 4><<<g2, 256 * NH_, lds2(KT_, NH_), st>>>(A);          \
+    else delta_chunk32_kernel<KT_, NH_, false><<<g2, 256 * NH_, lds2(KT_, NH_), st>>>(A);                             \
   } while (0)
   if (dim <= 32) LAUNCH_DC32(2, 1);
   else if (dim <= 64) LAUNCH_DC32(4, 2);

@@ -72,6 +72,7 @@ def test_rows32_one_key_written_again():
 # a last chunk of one, two, three and four blocks of sixteen tokens, alone and behind a whole chunk, whose results and sums two waves share
 @pytest.mark.gpu
 @pytest.mark.parametrize("dim,vdim", [(32, 64), (64, 100), (100, 64), (128, 16)])
-@pytest.mark.parametrize("lens,starts", [([16, 17, 32, 33, 48, 49], [0, 3, 0, 0, 70, 1]), ([81, 64, 112, 127], [0, 0, 9, 64])])
+@pytest.mark.parametrize("lens,starts", [([16, 17, 32, 33, 48, 49], [0, 3, 0, 0, 70, 1]), ([81, 64, 112, 127], [0, 0, 9, 64]),
+                                         ([145, 128, 16, 161], [0, 0, 9, 64]), ([129, 191], [5, 0])])  # (beyond 128 rows: places kept)
 def test_rows32_blocks_of_the_last_chunk(dim, vdim, lens, starts):
     run(lens, starts, 0, 2, 1, dim, vdim, torch.bfloat16)
