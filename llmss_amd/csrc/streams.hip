@@ -325,9 +325,10 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(const TI* __restrict__
 // instead of once per tap. The rows are loaded up front, all loads in flight together; the strip's place in its
 // sequence is found once and walked from there (looked up again where a sequence ends). Taps are added in the order
 // of the kernel above: the same numbers bit for bit. RMAX: the most rows back that a tap may reach (taps - 1). WITHIN: strips within one portion
-// have a form of their own: bf16 rows, taps = RMAX + 1, portions of 32 rows and more on average. It takes up to 18 more registers (nine taps: three
+// have a form of their own: bf16 rows, taps = RMAX + 1, portions of 24 rows and more on average. It takes up to 18 more registers (nine taps: three
 // waves a SIMD for four), which six to eight taps and short portions would pay for nothing: 6000 rows of 4096, seven taps, 47 us and 50 with it, 400
-// portions of 20 rows, nine taps, 75 and 80. Over 48 sizes each, of portions of 24 rows 0.994 of the time with it, of 40 0.987, of 64 0.968, of 200 0.962.
+// portions of 20 rows, nine taps, 75 and 80. Over 48 sizes each, of portions of 24 rows 0.994 of the time with it (64 of 24, four taps, 6144
+// wide 24.1 and 23.4), of 40 0.987, of 64 0.968, of 200 0.962.
 #define CONV_STRIP 16
 template <typename T, int CH>
 __device__ __forceinline__ void conv_ld(const T* p, float* v) {
@@ -605,7 +606,7 @@ static void causal_conv_t(const void* in, int64_t ldi, const void* w, void* stat
   if (!single && T_ >= 256 && T_ >= 8 * B && taps <= 9) {  // portions of eight rows and more on average
     const auto al16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
     const bool four = C % 4 == 0 && ldi % 4 == 0 && ldo % 4 == 0 && al16(in) && al16(out) && al16(state);
-    const bool within = sizeof(TI) == 2 && T_ >= 32 * B;
+    const bool within = sizeof(TI) == 2 && T_ >= 24 * B;
 #define LAUNCH_STRIP1(RMAX_, CH_, WITHIN_)                                                                          \
   causal_conv_strip_kernel<TI, TW, TO, RMAX_, CH_, WITHIN_><<<g, 256, 0, st>>>(                                     \
       (const TI*)in, ldi, (const TW*)w, (const float*)state, (const int*)cu, (const int*)ctx, (const int*)sslots,   \
