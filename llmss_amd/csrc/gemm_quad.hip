@@ -35,8 +35,9 @@
 // sixteen lanes): one instruction then writes rows 0 .. 7 of the sixteen in whole lines, another rows 8 .. 15.
 // Rows and columns past the last lie outside the descriptor, so that no branch stands between the stores. (gemm_quad_ok: the rows that a wave
 // reaches over, 240 where they alternate by sixteens and else 128, fit a descriptor of 31 bits.)
-// All go past the caches: fp32 sums of 32768 pairs x 2048 (K = 768) 152 -> 131 us, which no cache would hold until they are read.
-template <int GRP, int GLU, int MS>
+// PAST: past the caches, as bf16 results (65536 pairs x 768 390 -> 367 us with all of their product) and fp32 sums that these would not hold until they
+// are read: of 32768 pairs x 2048 (K = 768) 152 -> 131 us. Up to 128 MB are in them when the combining launch reads them (launch_gemm_quad).
+template <int GRP, int GLU, int MS, bool PAST>
 __device__ __forceinline__ void quad_store(const f32x4 (&acc)[8][8], const PpGroup& gr, const bf16_t* __restrict__ bias, bf16_t* __restrict__ Y,
                                            int64_t ldy, int m0, int n0, int M, int N, int li, int g, const float (&sw)[8], bool half) {
   constexpr int ES = GRP == 2 ? 4 : 2, COLS = GRP == 2 ? 4 : GLU ? 1 : 2, RUN = GRP == 2 ? 32 : 64;  // runs of a line
@@ -91,8 +92,8 @@ __device__ __forceinline__ void quad_store(const f32x4 (&acc)[8][8], const PpGro
         b[i] = __builtin_amdgcn_update_dpp(y, x, 0x128, 0xf, 0x3, false);  // lanes 0 .. 7: of a, from li + 8
       }
       const uint32_t ra = n < nout ? at + (uint32_t)(MS * mt) * pitch : ~0u, rb = n < nout ? at + (uint32_t)(MS * mt + 8) * pitch : ~0u;
-      __builtin_amdgcn_raw_buffer_store_b128(a, ry, ra, 0, 2);
-      __builtin_amdgcn_raw_buffer_store_b128(b, ry, rb, 0, 2);
+      __builtin_amdgcn_raw_buffer_store_b128(a, ry, ra, 0, PAST ? 2 : 0);
+      __builtin_amdgcn_raw_buffer_store_b128(b, ry, rb, 0, PAST ? 2 : 0);
     }
   }
 }
@@ -105,7 +106,7 @@ __device__ __forceinline__ void quad_store(const f32x4 (&acc)[8][8], const PpGro
 // looked up once a row and kept in the ring's fifth buffer.
 // Against the product and a rotation of its own, which reads and writes all of it again (us): 8192 x 12288 x 4096 676 -> 621, 3999 rows 343 ->
 // 315; 8192 x 4800 x 1600 without a rotation 159 -> 140.
-template <int GRP, int GLU, bool QKV = false, bool RING = false>
+template <int GRP, int GLU, bool QKV = false, bool RING = false, bool PAST = true>
 __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restrict__ X, int64_t ldx,
                                                            const bf16_t* __restrict__ W, int64_t ldw,
                                                            const bf16_t* __restrict__ bias, bf16_t* __restrict__ Y,
@@ -335,7 +336,7 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(const bf16_t* __restr
         if constexpr (GRP == 3) sw[i] = weight_of(cur, i);
       }
       __builtin_amdgcn_sched_barrier(0);
-      quad_store<GRP, GLU, HALF ? 32 : 16>(acc, gr, bias, Y, ldy, cur.m0 + (HALF ? 16 : 128) * wr, cur.n0 + wc * 128, cur.M, N, li, g, sw, !full);
+      quad_store<GRP, GLU, HALF ? 32 : 16, PAST>(acc, gr, bias, Y, ldy, cur.m0 + (HALF ? 16 : 128) * wr, cur.n0 + wc * 128, cur.M, N, li, g, sw, !full);
       if (ahead < 0) break;
       ahead = after;
       cur = next, next = then;
@@ -509,10 +510,17 @@ void launch_gemm_quad(int grp, const bf16_t* X, int64_t ldx, const bf16_t* W, in
   // a workgroup per CU, each taking every 256th tile; rings of fewer than four steps do not reach into another tile
   const unsigned ring = K >= 256 ? std::min(nwg, 256u) : nwg;
   const bool lds = qe || (!glu && grp != 2 && act != ACT_NONE);
-#define LAUNCH_Q(G_, U_, Q_, R_) \
-  gemm_quad_kernel<G_, U_, Q_, R_><<<R_ ? ring : nwg, 256, 0, st>>>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, act, group_m, gr, qe ? *qe : QkvEpi{})
+  // fp32 sums of up to 128 MB stay in the caches. us, three launches, past them and in them: 5554 pairs x 2048 (45 MB), 8 experts of 1024, 124 and 118;
+  // 11108 x 2048 (91 MB), 16 of 768, 204 and 195; 22216 x 1024, 128 of 256, 128 and 117; 32768 x 1024 (134 MB), 32 of 512, 205 and 196; 16384 x 2048,
+  // 8 of 1024, 302 and 305; 22216 x 2048 (182 MB), 64 of 768, 400 and 420; 65536 x 1024, 128 of 256, 284 and 295. (A list of P pairs has room for
+  // ceil(P / 256) + E tiles.)
+  const bool past = (int64_t)std::max(gr.maxt - gr.E, 1) * 256 * ldy * 4 > (128 << 20);
+#define LAUNCH_P(G_, U_, Q_, R_, P_) \
+  gemm_quad_kernel<G_, U_, Q_, R_, P_><<<R_ ? ring : nwg, 256, 0, st>>>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, act, group_m, gr, qe ? *qe : QkvEpi{})
+#define LAUNCH_Q(G_, U_, Q_, R_) LAUNCH_P(G_, U_, Q_, R_, true)
   if (qe) LAUNCH_Q(0, 0, true, false);
-  else if (grp == 2) LAUNCH_Q(2, 0, false, true);
+  else if (grp == 2 && past) LAUNCH_Q(2, 0, false, true);
+  else if (grp == 2) LAUNCH_P(2, 0, false, true, false);
   else if (grp == 3) LAUNCH_Q(3, 1, false, true);
   else if (grp == 1 && glu) LAUNCH_Q(1, 1, false, true);
   else if (grp == 1 && lds) LAUNCH_Q(1, 0, false, false);
@@ -522,5 +530,6 @@ void launch_gemm_quad(int grp, const bf16_t* X, int64_t ldx, const bf16_t* W, in
   else if (lds) LAUNCH_Q(0, 0, false, false);
   else LAUNCH_Q(0, 0, false, true);
 #undef LAUNCH_Q
+#undef LAUNCH_P
   HIP_CHECK_LAUNCH();
 }

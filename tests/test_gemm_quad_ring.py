@@ -71,7 +71,8 @@ def test_many_tiles_of_experts_in_one_matrix(kind):
 # experts with rests of half a tile and less, which come last and by halves: one row, a matrix instruction's sixteen, 127 - 129 and whole tiles; more
 # tiles than CUs in both products, fewer, and only halves
 @pytest.mark.parametrize("counts,F,N", [([1000, 128, 2300, 129, 16, 513, 640], 2048, 3080), ([127, 1, 1536, 17, 256 + 255, 0], 288, 264),
-                                        ([2048, 384 + 1, 256 + 31], 3072, 2048), ([100, 128, 90, 33, 64, 12, 128, 1], 640, 520)])
+                                        ([2048, 384 + 1, 256 + 31], 3072, 2048), ([100, 128, 90, 33, 64, 12, 128, 1], 640, 520),
+                                        ([1000, 900, 128, 17, 2], 320, 16640)])  # (sums of 136 MB, past the caches)
 @pytest.mark.parametrize("kind", ["two", "interleaved", "gelu"])
 def test_half_tiles_of_experts(counts, F, N, kind, monkeypatch):
     from llmss_amd.ops import glu_interleave, hip
