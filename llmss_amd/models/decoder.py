@@ -210,12 +210,13 @@ class DecoderLM:
     # ---------------------------------------------------------------------------- forward
     def _qkv_plan(self, M: int, N: int, K: int):
         """(nt_hint, split_hint) of the QKV product with RoPE and the cache write in its epilogue, None: two launches. Without a tuned
-        plan of either form: up to 64 rows where the static plan of a finished product is the decode kernel's, unsplit. The two launches may
-        split K, whose slabs rope_cache sums on the way; over 175 random layers of 1 - 64 rows one launch takes 0.87 of their time, and 1.07
-        at worst (us, two and one: 4800 x 1600, one row 8.9 and 6.3, 64 rows 13.4 and 9.7; 12288 x 4096 23.6 and 19.9, 28.7 and 24.1;
-        6144 x 4096 14.6 and 11.7, 18.3 and 17.7; 3072 x 1024 6.8 and 4.8, 10.4 and 6.7; 15360 x 5120 31.2 and 27.5, 42.0 and 35.2; 10240 x
-        8192 32.2 and 32.6, 16 rows 34.3 and 32.6; 1536 x 5040, 15 rows 11.9 and 12.7). Prompts: where the two launches would not split K
-        either and from 128 rows on (66 rows of 12288 x 4096 39.2 and 39.5; 256 rows of 12288 x 4096: 47.5 in two with K split, 62.9 in one without). 12288 x 4096, 1024 rows 109 and 100,
+        plan of either form: up to 64 rows where the static plan of a finished product is the decode kernel's, unsplit, or, from 17 rows on, the
+        four-wave tiles', unsplit or combined in the launch. The two launches may split K, whose slabs rope_cache sums on the way; one launch by
+        the decode kernel takes 0.87 of their time over 175 random layers of 1 - 64 rows, 1.07 at worst (us, two and one: 4800 x 1600, one row 8.9 and
+        6.3; 12288 x 4096 23.6 and 19.9; 6144 x 4096 14.6 and 11.7; 3072 x 1024 6.8 and 4.8; 15360 x 5120 31.2 and 27.5; 10240 x 8192 32.2 and
+        32.6; 1536 x 5040, 15 rows 11.9 and 12.7), by the four-wave tiles 0.87 over 516 of 17 - 64 rows, 21 of them above 1.02, 1.13 at worst
+        (64 rows, 2560 x 1472 10.4 and 7.7, 1280 x 8192 13.6 and 11.7, 1920 x 5120 13.5 and 11.3, 10240 x 8192 43.8 and 41.5; 24 rows, 1536 x 4096
+        8.8 and 9.2; 48 rows, 6144 x 4096 17.5 and 19.3, x 5248 20.7 and 23.3). Prompts: where the two launches would not split K either and from 128 rows on (66 rows of 12288 x 4096 39.2 and 39.5; 256 rows of 12288 x 4096: 47.5 in two with K split, 62.9 in one without). 12288 x 4096, 1024 rows 109 and 100,
         1773 rows 192 and 177, 8192 rows 676 and 621; 4800 x 1600, 512 rows 32.6 and 25.5, 2048 rows 49 and 42, 8192 rows 159 and 140."""
         lib = _hip_ops().lib()
         if lib.gemm_tuned_get(M, N, K, False, 3) is not None:
